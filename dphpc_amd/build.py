@@ -2,6 +2,7 @@
 import os
 import shutil
 import subprocess
+import tempfile
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG, "csrc")
@@ -13,7 +14,6 @@ HIPCC_FLAGS = [
     "-O3",
     "-std=c++17",
     "-fPIC",
-    "-shared",
     "-ffp-contract=off",          # FMAs are written explicitly; the exact kernel needs mul and add apart
     "-fno-gpu-rdc",
     "-Wall",
@@ -31,17 +31,27 @@ def hipcc():
 
 
 def sources():
-    return [os.path.join(CSRC, "sddmm_amd.hip")]
+    return sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".hip"))
 
 
 def build_library(verbose=False, extra_flags=(), out=None):
-    """(Re)build dphpc_amd/lib/libsddmm_amd.so; returns its path."""
+    """(Re)build dphpc_amd/lib/libsddmm_amd.so; returns its path.  The translation units are compiled side by side."""
     os.makedirs(LIB_DIR, exist_ok=True)
-    cmd = [hipcc()] + HIPCC_FLAGS + list(extra_flags) + ["-o", out or LIB_PATH] + sources()
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    subprocess.check_call(cmd)
-    return LIB_PATH
+    out = out or LIB_PATH
+    with tempfile.TemporaryDirectory() as tmp:
+        jobs, objects = [], []
+        for src in sources():
+            obj = os.path.join(tmp, os.path.basename(src) + ".o")
+            cmd = [hipcc()] + HIPCC_FLAGS + list(extra_flags) + ["-c", "-o", obj, src]
+            if verbose:
+                print(" ".join(cmd), flush=True)
+            jobs.append((cmd, subprocess.Popen(cmd)))
+            objects.append(obj)
+        failed = [cmd for cmd, job in jobs if job.wait() != 0]
+        if failed:
+            raise subprocess.CalledProcessError(1, failed[0])
+        subprocess.check_call([hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", out] + objects)
+    return out
 
 
 if __name__ == "__main__":

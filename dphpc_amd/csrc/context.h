@@ -1,0 +1,296 @@
+// The context behind sddmm_ctx, error and launch macros, and the dispatch over row layouts: what the
+// planning code (sddmm_amd.hip) and the launchers (launch_*.hip) share.
+#pragma once
+#include "../../include/sddmm_amd.h"
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstdarg>
+#include <cstdio>
+#include <climits>
+#include <cstdlib>
+#include <cstring>
+#include <new>
+#include <vector>
+
+#include "kernels_gather.h"
+#include "kernels_plan.h"
+#include "kernels_tile.h"
+
+using namespace sddmm;
+
+// ---------------------------------------------------------------------------
+struct sddmm_ctx {
+    int device = 0;
+    hipStream_t stream = nullptr;      // where work is enqueued: own_stream unless the caller lent one
+    hipStream_t own_stream = nullptr;
+    bool lent_stream = false;
+    bool oversize = false;             // a launch was skipped because its grid does not fit one dispatch
+    hipEvent_t ev0 = nullptr, ev1 = nullptr;
+
+    char err[512] = {0};
+
+    // dense operands
+    int M = 0, N = 0, K = 0, dtype = SDDMM_F32;
+    bool have_dense = false;
+    void *dA = nullptr, *dB = nullptr;
+    bool own_dense = false;
+
+    // sparse operand
+    bool have_sparse = false, have_rowptr = false, own_sparse = false, from_coo = false;
+    int sM = 0, sN = 0;
+    int64_t nnz = 0;
+    int32_t *d_rowptr = nullptr, *d_col = nullptr, *d_rowidx = nullptr;
+    float *d_sval = nullptr, *dP = nullptr;
+    bool own_rowptr = false, own_rowidx = false;
+
+    // plan
+    bool planned = false;
+    int strategy = SDDMM_AUTO;       // resolved
+    int requested = SDDMM_AUTO;
+    DevCounters *d_pc = nullptr;     // device counters
+    DevCounters raw{};               // host copy of the device block
+    DevCounters *h_pc = nullptr;     // pinned landing place of the read-back (no staging copy)
+    PlanCounters pc{};               // its summary
+    sddmm_stats stats{};
+    // AUTO: rows shorter than ts go to the many-rows-per-wave kernel, the others
+    // become wave-per-segment items of at most seg entries
+    int ts = 0, seg = 0, rpw = 64;
+    RowItem *d_items = nullptr;
+    int64_t n_items = 0, items_cap = 0;
+    unsigned int *d_block_sums = nullptr;
+    int64_t block_sums_cap = 0;
+    int64_t rows_short = 0;
+    int launches = 0;
+    // dense-tile (MFMA) path
+    unsigned int *d_strip_ntiles = nullptr, *d_strip_off = nullptr;
+    int64_t strips_cap = 0;
+    TileDesc *d_tiles = nullptr;
+    int64_t n_tiles = 0, tiles_cap = 0, nnz_tiles = 0;
+    int tile_steps = 0;
+    bool tiles_active = false;       // d_tiles describes the current pattern
+    int32_t *d_win_order = nullptr;  // order in which the launch takes the windows (null: storage order)
+    unsigned int *d_win_bins = nullptr;
+    int64_t win_order_cap = 0;
+    bool use_win_order = false;
+    TileWindow *d_windows = nullptr; // one record per TILE_WINDOW consecutive descriptors
+    int64_t n_windows = 0, windows_cap = 0;
+    bool use_windows = false;        // tile kernels take windows as batches (else they walk them tile by tile)
+    int64_t n_tiles_natural = 0;     // descriptors: 16-row strips first, then union strips, then gathered strips
+    int64_t n_tiles_lead = 0;        // empty descriptors that fill the last window before the gathered strips
+    int64_t n_win_single = 0;        // windows taken one per wavefront; the rest (gathered pairs) two per wavefront
+    int64_t n_tile_units = 0;        // wavefronts of a tile launch
+    int64_t n_tiles_union = 0, nnz_tiles_union = 0;
+    unsigned int *d_ustrip_ntiles = nullptr, *d_ustrip_off = nullptr;
+    int64_t ustrips_cap = 0;
+    int32_t *d_tile_cols = nullptr;  // 16 B rows per descriptor
+    bool union_counted = false;
+    // gathered strips: candidate rows, sorted by first column, 16 per strip
+    unsigned long long *d_cand_keys = nullptr, *d_sorted_keys = nullptr;   // (first column << 32) | row
+    int32_t *d_vrows = nullptr;
+    void *d_sort_tmp = nullptr;
+    size_t sort_tmp_bytes = 0;
+    int64_t cand_cap = 0, vstrips_cap = 0, n_cand = 0, n_vstrips = 0;
+    unsigned int *d_vstrip_ntiles = nullptr, *d_vstrip_off = nullptr;
+    // row ownership (one byte per row: 0 row kernels, 1 dense tiles, 2 row panels, 3 gathered strips, 4 union strips)
+    unsigned char *d_owner = nullptr;
+    int64_t owner_cap = 0;
+    // every work array of the plan whose size follows from the number of rows lives in one
+    // allocation (a first plan then pays for one hipMalloc instead of a dozen)
+    char *d_arena = nullptr;
+    int64_t arena_rows = -1;
+    bool owner_active = false;
+    // row-panel path
+    unsigned int *d_panel_counts = nullptr, *d_panel_off = nullptr;
+    int64_t panels_cap = 0;
+    int2 *d_short_list = nullptr;    // {position, row} of the entries of the short rows nobody owns
+    int64_t n_short_list = 0, short_list_cap = 0;
+    ScanJobs scan_jobs{};            // short scans waiting for the next read-back of the counters
+    int n_scan_jobs = 0;
+    bool use_short_list = false;
+    unsigned int *d_short_sums = nullptr;   // arena view: entries of short rows per block of the row scan
+    RowItem *d_panel_items = nullptr;
+    int64_t n_panel_items = 0, panel_items_cap = 0, n_panels = 0, nnz_panels = 0;
+    bool panel_mfma = false;         // panels run on k_panel_mfma (else on k_panel)
+    bool panels_flagged = false;     // the panel detector ran in this plan
+    // fused SDDMM + SpMM: items covering every non-empty row, output M x K
+    RowItem *d_fused_items = nullptr;
+    int64_t n_fused_items = 0, fused_items_cap = 0;
+    bool fused_items_valid = false;
+    bool fused_items_panels = false; // the fused items leave out the rows that the panel kernel owns
+    double fused_short_avg = 0.0;    // entries per non-empty row of at most FUSED_ROW_MAX entries (panel rows apart)
+    float *dO = nullptr;
+    size_t o_cap = 0;
+    bool have_fused = false;
+};
+
+inline int fail(sddmm_ctx *c, int code, const char *fmt, ...) {
+    if (c) {
+        va_list ap;
+        va_start(ap, fmt);
+        vsnprintf(c->err, sizeof(c->err), fmt, ap);
+        va_end(ap);
+    }
+    return code;
+}
+
+#define HIP_TRY(c, call)                                                                         \
+    do {                                                                                         \
+        hipError_t e_ = (call);                                                                  \
+        if (e_ != hipSuccess)                                                                    \
+            return fail((c), SDDMM_ERR_HIP, "%s failed: %s (%s:%d)", #call, hipGetErrorString(e_), \
+                        __FILE__, __LINE__);                                                     \
+    } while (0)
+
+#define ALLOC_TRY(c, ptr, bytes)                                                                 \
+    do {                                                                                         \
+        hipError_t e_ = hipMalloc((void **)&(ptr), (bytes) ? (bytes) : 16);                      \
+        if (e_ != hipSuccess) {                                                                  \
+            (ptr) = nullptr;                                                                     \
+            return fail((c), SDDMM_ERR_ALLOC, "hipMalloc(%zu bytes) failed: %s", (size_t)(bytes), \
+                        hipGetErrorString(e_));                                                  \
+        }                                                                                        \
+    } while (0)
+
+// A dispatch packet counts the work-items of a grid dimension in 32 bits: a launch of 2^32
+// threads or more would run only part of its grid, without any error.  Such a launch is not
+// made; launch_status() turns the skipped launch into an error of the entry point.
+#define SDDMM_LAUNCH(c, kernel, grid, block, ...)                                                        \
+    do {                                                                                                 \
+        const int64_t g_ = (int64_t)(grid);                                                              \
+        const int b_ = (int)(block);                                                                     \
+        if (g_ * b_ >= ((int64_t)1 << 32)) (c)->oversize = true;                                         \
+        else hipLaunchKernelGGL(kernel, dim3((unsigned)g_), dim3((unsigned)b_), 0, (c)->stream, __VA_ARGS__); \
+    } while (0)
+
+inline int launch_status(sddmm_ctx *c) {
+    if (!c->oversize) return SDDMM_OK;
+    c->oversize = false;
+    return fail(c, SDDMM_ERR_UNSUPPORTED,
+                "a kernel of this strategy needs 2^32 threads or more in one launch for this matrix "
+                "(one wavefront per row or per work item): use SDDMM_AUTO or SDDMM_FLAT");
+}
+
+// after a group of launches: a failed launch, or one that was not made
+#define LAUNCH_CHECK(c)                                \
+    do {                                               \
+        HIP_TRY(c, hipGetLastError());                 \
+        const int ls_ = launch_status(c);              \
+        if (ls_) return ls_;                           \
+    } while (0)
+
+inline size_t elem_size(int dtype) { return dtype == SDDMM_F32 ? 4 : 2; }
+
+inline int env_int(const char *name, int fallback) {
+    const char *e = getenv(name);
+    return e && *e ? atoi(e) : fallback;
+}
+
+// ---- kernel dispatch over the (unit type, lanes per entry, units per lane) layouts ----
+struct Shape {
+    int unit;    // 0: fp32 x4, 1: fp32 x1, 2: bf16 x8, 3: fp16 x8
+    int KU;      // units per row
+    int LPN;     // lanes per entry (0: row too long for the register layout)
+    int UPL;     // units per lane
+    bool fullk;  // KU == LPN*UPL
+    bool wide;   // operands of 4 GiB or more: 64-bit byte offsets
+};
+
+inline int pow2ceil(int x) {
+    int l = 1;
+    while (l < x) l <<= 1;
+    return l;
+}
+
+inline Shape shape_of(const sddmm_ctx *c) {
+    Shape s{};
+    size_t unit_bytes;
+    if (c->dtype == SDDMM_BF16 || c->dtype == SDDMM_F16) { s.unit = c->dtype == SDDMM_BF16 ? 2 : 3; s.KU = c->K / 8; unit_bytes = 16; }
+    else if (c->K % 4 == 0) { s.unit = 0; s.KU = c->K / 4; unit_bytes = 16; }
+    else { s.unit = 1; s.KU = c->K; unit_bytes = 4; }
+    if (s.unit == 1) {
+        // 4-byte units: 16 lanes cover 64 contiguous bytes
+        if (s.KU <= 4) { s.LPN = 4; s.UPL = 1; }
+        else if (s.KU <= 16) { s.LPN = 16; s.UPL = 1; }
+        else if (s.KU <= 64) { s.LPN = 16; s.UPL = 4; }
+        else if (s.KU <= 128) { s.LPN = 16; s.UPL = 8; }
+        else { s.LPN = 0; s.UPL = 0; }
+    } else {
+        // 16-byte units: 8 lanes cover one whole 128-byte cache line per load
+        // instruction (measured faster than 4 lanes x 64 bytes: half the lines per
+        // instruction for the same bytes)
+        if (s.KU <= 8) { s.LPN = pow2ceil(s.KU); s.UPL = 1; }
+        else if (s.KU <= 64) { s.LPN = 8; s.UPL = pow2ceil((s.KU + 7) / 8); }
+        else if (s.KU <= 128) { s.LPN = 16; s.UPL = 8; }
+        else { s.LPN = 0; s.UPL = 0; }
+    }
+    s.fullk = s.LPN > 0 && s.KU == s.LPN * s.UPL;
+    const size_t rows = (size_t)std::max(c->M, c->N);
+    s.wide = rows * (size_t)s.KU * unit_bytes >= ((size_t)1 << 32);
+    return s;
+}
+
+// Calls f(Layout<...>{}) for the layout matching s.
+template <class U, int LPN, int UPL, class F>
+void with_mask_width(const Shape &s, F &&f) {
+    if (s.wide) f(Layout<U, LPN, UPL, false, true>{});
+    else if (s.fullk && U::ELEMS > 1) f(Layout<U, LPN, UPL, true, false>{});
+    else f(Layout<U, LPN, UPL, false, false>{});
+}
+
+template <class U, class F>
+void with_layout16(const Shape &s, F &&f) {
+    if (s.LPN == 0) { f(Layout<U, 0, 1, false, true>{}); return; }
+    if (s.LPN == 1) with_mask_width<U, 1, 1>(s, f);
+    else if (s.LPN == 2) with_mask_width<U, 2, 1>(s, f);
+    else if (s.LPN == 4) with_mask_width<U, 4, 1>(s, f);
+    else if (s.LPN == 16) with_mask_width<U, 16, 8>(s, f);
+    else if (s.UPL == 1) with_mask_width<U, 8, 1>(s, f);
+    else if (s.UPL == 2) with_mask_width<U, 8, 2>(s, f);
+    else if (s.UPL == 4) with_mask_width<U, 8, 4>(s, f);
+    else with_mask_width<U, 8, 8>(s, f);
+}
+
+template <class F>
+void with_layout(const Shape &s, F &&f) {
+    if (s.unit == 0) with_layout16<UnitF32x4>(s, f);
+    else if (s.unit == 2) with_layout16<UnitBF16x8>(s, f);
+    else if (s.unit == 3) with_layout16<UnitF16x8>(s, f);
+    else if (s.LPN == 0) f(Layout<UnitF32x1, 0, 1, false, true>{});
+    else if (s.LPN == 4) with_mask_width<UnitF32x1, 4, 1>(s, f);
+    else if (s.UPL == 1) with_mask_width<UnitF32x1, 16, 1>(s, f);
+    else if (s.UPL == 4) with_mask_width<UnitF32x1, 16, 4>(s, f);
+    else with_mask_width<UnitF32x1, 16, 8>(s, f);
+}
+
+// wavefronts of the short-row part of the AUTO launches: 64 entries of the entry list each, or
+// rpw consecutive rows each
+inline int64_t short_row_waves(const sddmm_ctx *c) {
+    if (c->rows_short <= 0) return 0;
+    if (c->use_short_list) return (c->n_short_list + WAVE - 1) / WAVE;
+    return ((int64_t)c->sM + c->rpw - 1) / c->rpw;
+}
+
+// Row-panel detector (8 consecutive rows, 8-aligned, same column list).  Two
+// kernels can run the panels: the MFMA one (row size a multiple of 64 bytes, up to
+// 1 KiB) and the VALU one (8-lanes-per-entry layouts whose 8 A rows fit in
+// registers: fp32 K = 32 or 64, bf16 / fp16 K = 64, 32-bit offsets); the VALU kernel has
+// the per-entry arithmetic of the gather kernels, the MFMA kernel is faster.
+inline int panel_mfma_steps(const sddmm_ctx *c) {
+    const size_t row_bytes = (size_t)c->K * elem_size(c->dtype);
+    if (row_bytes % 64) return 0;
+    const int steps = (int)(row_bytes / 64);
+    return (steps == 1 || steps == 2 || steps == 4 || steps == 8 || steps == 16) ? steps : 0;
+}
+
+// ---- launchers, one translation unit per family of kernels ----
+void launch_flat(sddmm_ctx *c);                                                  // launch_flat.hip
+void launch_row_wave(sddmm_ctx *c, const RowItem *items, int64_t n_items);       // launch_rows.hip
+void launch_short_rows(sddmm_ctx *c, int ts, int rpw);
+void launch_auto(sddmm_ctx *c);
+bool launch_auto_with_tiles(sddmm_ctx *c);                                       // launch_tiles.hip
+void launch_tiles(sddmm_ctx *c);
+void launch_panels(sddmm_ctx *c);                                                // launch_panels.hip
+void launch_panels_fused(sddmm_ctx *c);
+int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner);           // launch_fused.hip: number of launches

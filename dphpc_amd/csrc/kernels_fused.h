@@ -21,8 +21,6 @@
 
 namespace sddmm {
 
-constexpr int FUSED_ROW_MAX = 64;   // rows up to this length: one row per lane group
-
 template <class L>
 __global__ __launch_bounds__(BLOCK) void k_fusedmm(const void *__restrict__ A, const void *__restrict__ B, int KU,
                                                    const int32_t *__restrict__ rowptr,

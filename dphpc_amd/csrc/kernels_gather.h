@@ -25,6 +25,7 @@ namespace sddmm {
 
 constexpr int BLOCK = 256;                 // 4 wavefronts
 constexpr int WAVES_PER_BLOCK = BLOCK / WAVE;
+constexpr int FUSED_ROW_MAX = 64;          // fused SDDMM + SpMM: rows up to this length take one lane group each
 
 // Byte offset of a row: 32-bit when the whole operand is below 4 GiB (one VALU
 // multiply, scalar base + 32-bit vector offset addressing), 64-bit otherwise.

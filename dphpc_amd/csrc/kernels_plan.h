@@ -79,7 +79,7 @@ __device__ __forceinline__ unsigned int wave_max_u32(unsigned int v) {
 // runtime is a launch of its own for every region): the row-ownership bytes and every
 // counter except what validation measured (non-empty rows, longest row).  rows_only: just
 // the row classes and the item total, for the second count after the gathered strips.
-__global__ __launch_bounds__(256) void k_plan_reset(unsigned char *__restrict__ owner, int64_t owner_bytes,
+static __global__ __launch_bounds__(256) void k_plan_reset(unsigned char *__restrict__ owner, int64_t owner_bytes,
                                                     DevCounters *pc, int rows_only) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (!rows_only) {
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(256) void k_plan_reset(unsigned char *__restrict__ 
 
 // rowptr[0]==0, rowptr[M]==nnz, non-decreasing; also counts non-empty rows and the
 // longest row.  One lane per row, one set of atomics per workgroup.
-__global__ __launch_bounds__(256) void k_check_rowptr(const int32_t *__restrict__ rowptr, int M,
+static __global__ __launch_bounds__(256) void k_check_rowptr(const int32_t *__restrict__ rowptr, int M,
                                                       int64_t nnz, DevCounters *pc) {
     __shared__ unsigned int sh_ne, sh_mx, sh_bad;
     if (threadIdx.x == 0) { sh_ne = 0; sh_mx = 0; sh_bad = 0; }
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256) void k_check_rowptr(const int32_t *__restrict_
 }
 
 // every column index in [0,N)
-__global__ __launch_bounds__(256) void k_check_index(const int32_t *__restrict__ idx, int64_t n,
+static __global__ __launch_bounds__(256) void k_check_index(const int32_t *__restrict__ idx, int64_t n,
                                                      int bound, DevCounters *pc) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     unsigned int bad = 0;
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(256) void k_check_index(const int32_t *__restrict__
 // takes 64 rows: short rows are written by their own lane, long ones by the
 // whole wavefront.  Positions outside [0, limit) are never written, whatever the
 // row pointer holds (it may come unvalidated from the caller).
-__global__ __launch_bounds__(256) void k_expand_rows(const int32_t *__restrict__ rowptr, int M,
+static __global__ __launch_bounds__(256) void k_expand_rows(const int32_t *__restrict__ rowptr, int M,
                                                      int32_t *__restrict__ rowidx, int64_t limit) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = lane_id();
@@ -176,7 +176,7 @@ __global__ __launch_bounds__(256) void k_expand_rows(const int32_t *__restrict__
 }
 
 // COO rows non-decreasing?  (one lane per entry)
-__global__ __launch_bounds__(256) void k_check_coo_sorted(const int32_t *__restrict__ row, int64_t nnz,
+static __global__ __launch_bounds__(256) void k_check_coo_sorted(const int32_t *__restrict__ row, int64_t nnz,
                                                           DevCounters *pc) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     unsigned int uns = 0;
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(256) void k_check_coo_sorted(const int32_t *__restr
 }
 
 // sorted COO row array -> rowptr.  Entry n closes every row in (row[n-1], row[n]].
-__global__ __launch_bounds__(256) void k_rowptr_from_sorted_coo(const int32_t *__restrict__ row,
+static __global__ __launch_bounds__(256) void k_rowptr_from_sorted_coo(const int32_t *__restrict__ row,
                                                                 int64_t nnz, int M,
                                                                 int32_t *__restrict__ rowptr) {
     const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -250,7 +250,7 @@ __device__ __forceinline__ unsigned int block_exclusive_scan(unsigned int v, uns
 }
 
 // pass 1: items per block of SCAN_TILE rows, plus the row statistics
-__global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int32_t *__restrict__ rowptr,
+static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int32_t *__restrict__ rowptr,
                                                                const unsigned char *__restrict__ owner, int M,
                                                                int ts, int seg, unsigned int *__restrict__ block_sums,
                                                                DevCounters *pc, int only,
@@ -291,7 +291,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int32_t *__
 }
 
 // pass 2: exclusive scan of the block sums in place (one workgroup), total -> *total_out
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_block_sums(unsigned int *__restrict__ block_sums, int n,
+static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_block_sums(unsigned int *__restrict__ block_sums, int n,
                                                                 unsigned long long *__restrict__ total_out) {
     unsigned int carry = 0;
     for (int base = 0; base < n; base += SCAN_BLOCK) {
@@ -308,7 +308,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_block_sums(unsigned int *__
 // the whole exclusive scan of a short array in one workgroup (one launch instead of three)
 constexpr int SCAN_SMALL_ITEMS = 8;
 constexpr int SCAN_SMALL_MAX = 16384;
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_small(const unsigned int *__restrict__ in, int n,
+static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_small(const unsigned int *__restrict__ in, int n,
                                                            unsigned int *__restrict__ out,
                                                            unsigned long long *__restrict__ total_out) {
     unsigned int carry = 0;
@@ -343,7 +343,7 @@ struct ScanJob {
     int pad;
 };
 struct ScanJobs { ScanJob job[SCAN_JOBS_MAX]; };
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_jobs(ScanJobs jobs) {
+static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_jobs(ScanJobs jobs) {
     const ScanJob jb = jobs.job[blockIdx.x];
     unsigned int carry = 0;
     for (int base = 0; base < jb.n; base += SCAN_BLOCK * SCAN_SMALL_ITEMS) {
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_jobs(ScanJobs jobs) {
 // have fewer than ts entries and no owner, in storage order.  The kernels take it 64 entries
 // per wavefront, whatever the lengths of the rows (block_offsets: exclusive scan of the
 // short_sums of k_classify_count).
-__global__ __launch_bounds__(SCAN_BLOCK) void k_short_list_write(const int32_t *__restrict__ rowptr,
+static __global__ __launch_bounds__(SCAN_BLOCK) void k_short_list_write(const int32_t *__restrict__ rowptr,
                                                                  const unsigned char *__restrict__ owner, int M,
                                                                  int ts, const unsigned int *__restrict__ block_offsets,
                                                                  int2 *__restrict__ list) {
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_short_list_write(const int32_t *
 }
 
 // pass 3: write the items
-__global__ __launch_bounds__(SCAN_BLOCK) void k_classify_write(const int32_t *__restrict__ rowptr,
+static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_write(const int32_t *__restrict__ rowptr,
                                                                const unsigned char *__restrict__ owner, int M,
                                                                int ts, int seg,
                                                                const unsigned int *__restrict__ block_offsets,
@@ -428,7 +428,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_write(const int32_t *__
 // exist, are not owned by the dense-tile path, have the same length >= min_len and
 // the same column list.  One wavefront per panel; lanes stride over the list.
 // counts[p] = work items of the panel (ceil(len/pseg)) or 0; owner = 2 on its rows when taken.
-__global__ __launch_bounds__(256) void k_panel_flags(const int32_t *__restrict__ rowptr,
+static __global__ __launch_bounds__(256) void k_panel_flags(const int32_t *__restrict__ rowptr,
                                                      const int32_t *__restrict__ col, int M, int64_t n_panels,
                                                      int min_len, int pseg, unsigned char *__restrict__ owner,
                                                      unsigned int *__restrict__ counts, DevCounters *pc) {
@@ -470,7 +470,7 @@ __global__ __launch_bounds__(256) void k_panel_flags(const int32_t *__restrict__
 }
 
 // items of the taken panels: {first row, [start,end) inside the shared list}
-__global__ __launch_bounds__(256) void k_panel_items(const int32_t *__restrict__ rowptr, int64_t n_panels, int pseg,
+static __global__ __launch_bounds__(256) void k_panel_items(const int32_t *__restrict__ rowptr, int64_t n_panels, int pseg,
                                                      const unsigned int *__restrict__ counts,
                                                      const unsigned int *__restrict__ offsets,
                                                      RowItem *__restrict__ items) {

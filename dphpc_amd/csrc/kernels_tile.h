@@ -262,7 +262,7 @@ __device__ __forceinline__ void strip_bounds(const int32_t *__restrict__ col, in
 
 // pass 1: strip_ntiles[s] = number of tiles of a strip that goes to the tile path
 // (sorted rows, at least min_fill entries per tile on average), else 0.
-__global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_strip_count(
+static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_strip_count(
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int M, int64_t n_strips, int min_fill,
     unsigned int *__restrict__ strip_ntiles, unsigned char *__restrict__ owner, DevCounters *pc) {
     __shared__ unsigned int bm_all[STRIPS_PER_BLOCK][STRIP_BM_WORDS];
@@ -343,7 +343,7 @@ __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_strip_count(
 // column of every descriptor, in increasing tile column.  Descriptors of a strip
 // that needs the merging walk are written completely here (pad[0] = 1); the others
 // get their per-row fields from k_tile_rows.
-__global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_strip_tiles(
+static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_strip_tiles(
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int M, int64_t n_strips,
     const unsigned int *__restrict__ strip_ntiles, const unsigned int *__restrict__ strip_off,
     TileDesc *__restrict__ tiles, int32_t *__restrict__ tile_cols) {
@@ -415,7 +415,7 @@ constexpr int UNION_BM_WORDS = 4096;          // a column span of 131072 per str
 
 __device__ __forceinline__ int max16(int v) { return -min16(-v); }
 
-__global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_union_count(
+static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_union_count(
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int M, int64_t n_strips, int min_fill,
     unsigned char *__restrict__ owner, unsigned int *__restrict__ ustrip_ntiles, DevCounters *pc) {
     __shared__ unsigned int bm_all[STRIPS_PER_BLOCK][UNION_BM_WORDS];
@@ -464,7 +464,7 @@ __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_union_count(
 }
 
 // descriptors of the union strips: header and the 16 union columns of every tile
-__global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_union_tiles(
+static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_union_tiles(
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int M, int64_t n_strips,
     const unsigned int *__restrict__ ustrip_ntiles, const unsigned int *__restrict__ ustrip_off,
     TileDesc *__restrict__ tiles, int32_t *__restrict__ tile_cols) {
@@ -527,7 +527,7 @@ __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_union_tiles(
 constexpr int GATHERED_BASE = 1 << 30;
 constexpr int TILE_WINDOW = 4;                  // descriptors per window (what a wavefront of the tile kernels takes)
 
-__global__ __launch_bounds__(256) void k_gather_candidates(const int32_t *__restrict__ rowptr,
+static __global__ __launch_bounds__(256) void k_gather_candidates(const int32_t *__restrict__ rowptr,
                                                            const int32_t *__restrict__ col, int M,
                                                            const unsigned char *__restrict__ owner, int min_len,
                                                            unsigned long long *__restrict__ keys,
@@ -565,7 +565,7 @@ __global__ __launch_bounds__(256) void k_gather_candidates(const int32_t *__rest
 #define SDDMM_RANK_SORT_SPLIT 32
 #endif
 constexpr int RANK_SORT_MAX = 8192, RANK_SORT_BLOCK = 256, RANK_SORT_SPLIT = SDDMM_RANK_SORT_SPLIT;
-__global__ __launch_bounds__(RANK_SORT_BLOCK) void k_rank_sort(const unsigned long long *__restrict__ in,
+static __global__ __launch_bounds__(RANK_SORT_BLOCK) void k_rank_sort(const unsigned long long *__restrict__ in,
                                                                unsigned long long *__restrict__ out, int n) {
     __shared__ unsigned long long v[RANK_SORT_MAX];
     for (int i = (int)threadIdx.x; i < n; i += RANK_SORT_BLOCK) v[i] = in[i];
@@ -650,7 +650,7 @@ __device__ __forceinline__ bool gathered_mark(const int32_t *__restrict__ col, c
 
 // pass 1 of the gathered strips: descriptors per strip of the pair (0: not taken; the same for
 // both strips), the strips' row table, ownership of the rows of a taken pair.
-__global__ __launch_bounds__(GATHERED_BLOCK) void k_gathered_count(
+static __global__ __launch_bounds__(GATHERED_BLOCK) void k_gathered_count(
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col,
     const unsigned long long *__restrict__ sorted_keys,
     int64_t n_cand, int64_t n_vpairs, int min_fill, unsigned int *__restrict__ vstrip_ntiles,
@@ -706,7 +706,7 @@ __device__ __forceinline__ void write_empty_desc(TileDesc *__restrict__ tiles, i
 // (descriptor 8k + 4h + j of the pair: strip h, the (4k+j)-th tile column).  `tiles` / `tile_cols`
 // point at the first gathered descriptor; the `lead` descriptors before it (fewer than
 // TILE_WINDOW) fill the last window of the strips that precede the gathered ones.
-__global__ __launch_bounds__(GATHERED_BLOCK) void k_gathered_tiles(
+static __global__ __launch_bounds__(GATHERED_BLOCK) void k_gathered_tiles(
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col,
     const unsigned long long *__restrict__ sorted_keys,
     int64_t n_cand, int64_t n_vpairs, const unsigned int *__restrict__ vstrip_ntiles,
@@ -768,7 +768,7 @@ __global__ __launch_bounds__(GATHERED_BLOCK) void k_gathered_tiles(
 // at or after the tile's first column, and the mask of the tile's columns present.
 // Bit n of the mask stands for the n-th of the tile's 16 columns; a row's entries
 // inside a tile are consecutive in CSR, in the order of the tile's columns.
-__global__ __launch_bounds__(256) void k_tile_rows(const int32_t *__restrict__ rowptr,
+static __global__ __launch_bounds__(256) void k_tile_rows(const int32_t *__restrict__ rowptr,
                                                    const int32_t *__restrict__ col, int M,
                                                    const int32_t *__restrict__ vrows,
                                                    const int32_t *__restrict__ tile_cols,
@@ -823,7 +823,7 @@ __global__ __launch_bounds__(256) void k_tile_rows(const int32_t *__restrict__ r
 }
 
 // generic exclusive scan of n unsigned ints: block sums, then apply
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_sums(const unsigned int *__restrict__ in, int64_t n,
+static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_sums(const unsigned int *__restrict__ in, int64_t n,
                                                           unsigned int *__restrict__ block_sums) {
     const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
     unsigned int mine = 0;
@@ -832,7 +832,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_sums(const unsigned int *__
     (void)block_exclusive_scan(mine, &total);
     if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
 }
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_apply(const unsigned int *__restrict__ in, int64_t n,
+static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_apply(const unsigned int *__restrict__ in, int64_t n,
                                                            const unsigned int *__restrict__ block_offsets,
                                                            unsigned int *__restrict__ out) {
     const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
@@ -1026,7 +1026,7 @@ struct alignas(16) TileWindow {               // lane l < 48 loads dword l
 static_assert(sizeof(TileWindow) == 192, "TileWindow layout");
 
 // plan: one thread per (window, strip row)
-__global__ __launch_bounds__(256) void k_tile_windows(const int32_t *__restrict__ vrows, int M, int64_t nnz,
+static __global__ __launch_bounds__(256) void k_tile_windows(const int32_t *__restrict__ vrows, int M, int64_t nnz,
                                                       const TileDesc *__restrict__ tiles, int64_t n_tiles,
                                                       int64_t union_lo, int64_t union_hi, int64_t gathered_lo,
                                                       TileWindow *__restrict__ win, int64_t n_win) {
@@ -1603,14 +1603,14 @@ __device__ __forceinline__ int window_bin(const TileDesc *__restrict__ tiles, in
     const int fine = (int)(tj * (CB * WINDOW_SLICES) / tile_col_span);               // cb * WINDOW_SLICES + slice
     return rb * (CB * WINDOW_SLICES) + fine;
 }
-__global__ __launch_bounds__(256) void k_window_histogram(const TileDesc *__restrict__ tiles, int64_t n_win,
+static __global__ __launch_bounds__(256) void k_window_histogram(const TileDesc *__restrict__ tiles, int64_t n_win,
                                                           int64_t strip_span, int64_t tile_col_span, int RB, int CB,
                                                           unsigned int *__restrict__ bins) {
     const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (w < n_win) atomicAdd(&bins[window_bin(tiles, w, strip_span, tile_col_span, RB, CB)], 1u);
 }
 // one workgroup of WINDOW_BINS threads: counts -> start positions (also the scatter's cursors)
-__global__ __launch_bounds__(WINDOW_BINS) void k_window_offsets(unsigned int *__restrict__ bins) {
+static __global__ __launch_bounds__(WINDOW_BINS) void k_window_offsets(unsigned int *__restrict__ bins) {
     __shared__ unsigned int v[WINDOW_BINS];
     v[threadIdx.x] = bins[threadIdx.x];
     __syncthreads();
@@ -1618,7 +1618,7 @@ __global__ __launch_bounds__(WINDOW_BINS) void k_window_offsets(unsigned int *__
     for (int i = 0; i < (int)threadIdx.x; ++i) before += v[i];
     bins[threadIdx.x] = before;
 }
-__global__ __launch_bounds__(256) void k_window_scatter(const TileDesc *__restrict__ tiles, int64_t n_win,
+static __global__ __launch_bounds__(256) void k_window_scatter(const TileDesc *__restrict__ tiles, int64_t n_win,
                                                         int64_t strip_span, int64_t tile_col_span, int RB, int CB,
                                                         unsigned int *__restrict__ cursors, int32_t *__restrict__ order) {
     const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;

@@ -1,0 +1,47 @@
+// Launches of the gather kernels of the fused SDDMM + SpMM.
+#include "context.h"
+#include "kernels_fused.h"
+
+// Rows of at most FUSED_ROW_MAX entries, then the work items of the longer ones; 0: no kernel for this row layout.
+int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
+    const Shape s = shape_of(c);
+    // Short rows of fewer entries, on average, than half of what a lane group takes per step (a power-law
+    // graph: 3.5 against 8 lanes per entry at 128-byte rows): one row per lane group would idle most of its
+    // steps (20 % of them useful there), so the wavefronts deal whole rows out to their groups by entry
+    // count instead (576 -> 369 us for those rows).  With longer rows, or 4 lanes per entry, the extra
+    // gathers of the A rows and the longer walks cost more than the idle steps (mixed-density shape, 12.5
+    // entries per short row: 33 -> 65 us; power-law with 64-byte rows: 396 -> 432 us).
+    const int balanced_env = env_int("SDDMM_FUSED_BALANCED", -1);
+    const bool balanced = balanced_env >= 0 ? balanced_env != 0
+                                            : (c->fused_short_avg > 0.0 && 2.0 * c->fused_short_avg < (double)s.LPN);
+    int launches = 0;
+    with_layout(s, [&](auto L) {
+        using LT = decltype(L);
+        if constexpr (!LT::LONG && LT::LPN <= 8 && LT::U::ELEMS > 1 && LT::UPL * LT::U::ELEMS <= 32) {
+            const int64_t rows_per_wave = WAVE / LT::LPN;
+            const int64_t waves = ((int64_t)c->sM + rows_per_wave - 1) / rows_per_wave;
+            const int64_t rblocks = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+            if (balanced) {
+                const int64_t bwaves = ((int64_t)c->sM + WAVE - 1) / WAVE;
+                const int64_t bblocks = (bwaves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+                SDDMM_LAUNCH(c, (k_fusedmm_rows_balanced<LT>), xcd_grid(bblocks), BLOCK,
+                                   (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr, c->d_col, c->d_sval,
+                                   c->dP, c->dO, c->sM, FUSED_ROW_MAX, bblocks, panel_owner);
+            } else {
+                SDDMM_LAUNCH(c, (k_fusedmm_rows<LT>), xcd_grid(rblocks), BLOCK,
+                                   (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr, c->d_col, c->d_sval,
+                                   c->dP, c->dO, c->sM, FUSED_ROW_MAX, rblocks, panel_owner);
+            }
+            ++launches;
+            if (c->n_fused_items > 0) {
+                const int64_t nblocks = (c->n_fused_items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+                SDDMM_LAUNCH(c, (k_fusedmm<LT>), xcd_grid(nblocks), BLOCK,
+                                   (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr, c->d_col,
+                                   c->d_sval, c->dP, c->dO, (const RowItem *)c->d_fused_items, c->n_fused_items,
+                                   nblocks);
+                ++launches;
+            }
+        }
+    });
+    return launches;
+}

@@ -1,191 +1,12 @@
-// C ABI of the gfx950 SDDMM engine: context, operand upload, plan, launch.
+// C ABI of the gfx950 SDDMM engine: context, operand upload, plan, run.
 // See include/sddmm_amd.h for the contract of every entry point.
-#include "../../include/sddmm_amd.h"
+#include "context.h"
 
-#include <hip/hip_runtime.h>
-
-#include <cstring>
+#include <mutex>
 
 #include <rocprim/device/device_radix_sort.hpp>
 
-#include <algorithm>
-#include <cstdarg>
-#include <cstdio>
-#include <climits>
-#include <cstdlib>
-#include <cstring>
-#include <mutex>
-#include <new>
-#include <vector>
-
-#include "kernels_fused.h"
-#include "kernels_gather.h"
-#include "kernels_plan.h"
-#include "kernels_tile.h"
-
-using namespace sddmm;
-
-// ---------------------------------------------------------------------------
-struct sddmm_ctx {
-    int device = 0;
-    hipStream_t stream = nullptr;      // where work is enqueued: own_stream unless the caller lent one
-    hipStream_t own_stream = nullptr;
-    bool lent_stream = false;
-    bool oversize = false;             // a launch was skipped because its grid does not fit one dispatch
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
-
-    char err[512] = {0};
-
-    // dense operands
-    int M = 0, N = 0, K = 0, dtype = SDDMM_F32;
-    bool have_dense = false;
-    void *dA = nullptr, *dB = nullptr;
-    bool own_dense = false;
-
-    // sparse operand
-    bool have_sparse = false, have_rowptr = false, own_sparse = false, from_coo = false;
-    int sM = 0, sN = 0;
-    int64_t nnz = 0;
-    int32_t *d_rowptr = nullptr, *d_col = nullptr, *d_rowidx = nullptr;
-    float *d_sval = nullptr, *dP = nullptr;
-    bool own_rowptr = false, own_rowidx = false;
-
-    // plan
-    bool planned = false;
-    int strategy = SDDMM_AUTO;       // resolved
-    int requested = SDDMM_AUTO;
-    DevCounters *d_pc = nullptr;     // device counters
-    DevCounters raw{};               // host copy of the device block
-    DevCounters *h_pc = nullptr;     // pinned landing place of the read-back (no staging copy)
-    PlanCounters pc{};               // its summary
-    sddmm_stats stats{};
-    // AUTO: rows shorter than ts go to the many-rows-per-wave kernel, the others
-    // become wave-per-segment items of at most seg entries
-    int ts = 0, seg = 0, rpw = 64;
-    RowItem *d_items = nullptr;
-    int64_t n_items = 0, items_cap = 0;
-    unsigned int *d_block_sums = nullptr;
-    int64_t block_sums_cap = 0;
-    int64_t rows_short = 0;
-    int launches = 0;
-    // dense-tile (MFMA) path
-    unsigned int *d_strip_ntiles = nullptr, *d_strip_off = nullptr;
-    int64_t strips_cap = 0;
-    TileDesc *d_tiles = nullptr;
-    int64_t n_tiles = 0, tiles_cap = 0, nnz_tiles = 0;
-    int tile_steps = 0;
-    bool tiles_active = false;       // d_tiles describes the current pattern
-    int32_t *d_win_order = nullptr;  // order in which the launch takes the windows (null: storage order)
-    unsigned int *d_win_bins = nullptr;
-    int64_t win_order_cap = 0;
-    bool use_win_order = false;
-    TileWindow *d_windows = nullptr; // one record per TILE_WINDOW consecutive descriptors
-    int64_t n_windows = 0, windows_cap = 0;
-    bool use_windows = false;        // tile kernels take windows as batches (else they walk them tile by tile)
-    int64_t n_tiles_natural = 0;     // descriptors: 16-row strips first, then union strips, then gathered strips
-    int64_t n_tiles_lead = 0;        // empty descriptors that fill the last window before the gathered strips
-    int64_t n_win_single = 0;        // windows taken one per wavefront; the rest (gathered pairs) two per wavefront
-    int64_t n_tile_units = 0;        // wavefronts of a tile launch
-    int64_t n_tiles_union = 0, nnz_tiles_union = 0;
-    unsigned int *d_ustrip_ntiles = nullptr, *d_ustrip_off = nullptr;
-    int64_t ustrips_cap = 0;
-    int32_t *d_tile_cols = nullptr;  // 16 B rows per descriptor
-    bool union_counted = false;
-    // gathered strips: candidate rows, sorted by first column, 16 per strip
-    unsigned long long *d_cand_keys = nullptr, *d_sorted_keys = nullptr;   // (first column << 32) | row
-    int32_t *d_vrows = nullptr;
-    void *d_sort_tmp = nullptr;
-    size_t sort_tmp_bytes = 0;
-    int64_t cand_cap = 0, vstrips_cap = 0, n_cand = 0, n_vstrips = 0;
-    unsigned int *d_vstrip_ntiles = nullptr, *d_vstrip_off = nullptr;
-    // row ownership (one byte per row: 0 row kernels, 1 dense tiles, 2 row panels, 3 gathered strips, 4 union strips)
-    unsigned char *d_owner = nullptr;
-    int64_t owner_cap = 0;
-    // every work array of the plan whose size follows from the number of rows lives in one
-    // allocation (a first plan then pays for one hipMalloc instead of a dozen)
-    char *d_arena = nullptr;
-    int64_t arena_rows = -1;
-    bool owner_active = false;
-    // row-panel path
-    unsigned int *d_panel_counts = nullptr, *d_panel_off = nullptr;
-    int64_t panels_cap = 0;
-    int2 *d_short_list = nullptr;    // {position, row} of the entries of the short rows nobody owns
-    int64_t n_short_list = 0, short_list_cap = 0;
-    ScanJobs scan_jobs{};            // short scans waiting for the next read-back of the counters
-    int n_scan_jobs = 0;
-    bool use_short_list = false;
-    unsigned int *d_short_sums = nullptr;   // arena view: entries of short rows per block of the row scan
-    RowItem *d_panel_items = nullptr;
-    int64_t n_panel_items = 0, panel_items_cap = 0, n_panels = 0, nnz_panels = 0;
-    bool panel_mfma = false;         // panels run on k_panel_mfma (else on k_panel)
-    bool panels_flagged = false;     // the panel detector ran in this plan
-    // fused SDDMM + SpMM: items covering every non-empty row, output M x K
-    RowItem *d_fused_items = nullptr;
-    int64_t n_fused_items = 0, fused_items_cap = 0;
-    bool fused_items_valid = false;
-    bool fused_items_panels = false; // the fused items leave out the rows that the panel kernel owns
-    double fused_short_avg = 0.0;    // entries per non-empty row of at most FUSED_ROW_MAX entries (panel rows apart)
-    float *dO = nullptr;
-    size_t o_cap = 0;
-    bool have_fused = false;
-};
-
 namespace {
-
-int fail(sddmm_ctx *c, int code, const char *fmt, ...) {
-    if (c) {
-        va_list ap;
-        va_start(ap, fmt);
-        vsnprintf(c->err, sizeof(c->err), fmt, ap);
-        va_end(ap);
-    }
-    return code;
-}
-
-#define HIP_TRY(c, call)                                                                         \
-    do {                                                                                         \
-        hipError_t e_ = (call);                                                                  \
-        if (e_ != hipSuccess)                                                                    \
-            return fail((c), SDDMM_ERR_HIP, "%s failed: %s (%s:%d)", #call, hipGetErrorString(e_), \
-                        __FILE__, __LINE__);                                                     \
-    } while (0)
-
-#define ALLOC_TRY(c, ptr, bytes)                                                                 \
-    do {                                                                                         \
-        hipError_t e_ = hipMalloc((void **)&(ptr), (bytes) ? (bytes) : 16);                      \
-        if (e_ != hipSuccess) {                                                                  \
-            (ptr) = nullptr;                                                                     \
-            return fail((c), SDDMM_ERR_ALLOC, "hipMalloc(%zu bytes) failed: %s", (size_t)(bytes), \
-                        hipGetErrorString(e_));                                                  \
-        }                                                                                        \
-    } while (0)
-
-// A dispatch packet counts the work-items of a grid dimension in 32 bits: a launch of 2^32
-// threads or more would run only part of its grid, without any error.  Such a launch is not
-// made; launch_status() turns the skipped launch into an error of the entry point.
-#define SDDMM_LAUNCH(c, kernel, grid, block, ...)                                                        \
-    do {                                                                                                 \
-        const int64_t g_ = (int64_t)(grid);                                                              \
-        const int b_ = (int)(block);                                                                     \
-        if (g_ * b_ >= ((int64_t)1 << 32)) (c)->oversize = true;                                         \
-        else hipLaunchKernelGGL(kernel, dim3((unsigned)g_), dim3((unsigned)b_), 0, (c)->stream, __VA_ARGS__); \
-    } while (0)
-
-int launch_status(sddmm_ctx *c) {
-    if (!c->oversize) return SDDMM_OK;
-    c->oversize = false;
-    return fail(c, SDDMM_ERR_UNSUPPORTED,
-                "a kernel of this strategy needs 2^32 threads or more in one launch for this matrix "
-                "(one wavefront per row or per work item): use SDDMM_AUTO or SDDMM_FLAT");
-}
-
-// after a group of launches: a failed launch, or one that was not made
-#define LAUNCH_CHECK(c)                                \
-    do {                                               \
-        HIP_TRY(c, hipGetLastError());                 \
-        const int ls_ = launch_status(c);              \
-        if (ls_) return ls_;                           \
-    } while (0)
 
 template <class T>
 void dfree(T *&p) {
@@ -305,8 +126,6 @@ void release_sparse(sddmm_ctx *c) {
     c->nnz = 0;
 }
 
-size_t elem_size(int dtype) { return dtype == SDDMM_F32 ? 4 : 2; }
-
 int grid_for(int64_t n, int block) { return (int)std::max<int64_t>(1, (n + block - 1) / block); }
 int grid_capped(int64_t n, int block, int cap = 16384) {
     return (int)std::min<int64_t>(cap, std::max<int64_t>(1, (n + block - 1) / block));
@@ -343,197 +162,12 @@ int fetch_counters(sddmm_ctx *c) {
     return SDDMM_OK;
 }
 
-// ---- kernel dispatch over the (unit type, lanes per entry, units per lane) layouts ----
-struct Shape {
-    int unit;    // 0: fp32 x4, 1: fp32 x1, 2: bf16 x8, 3: fp16 x8
-    int KU;      // units per row
-    int LPN;     // lanes per entry (0: row too long for the register layout)
-    int UPL;     // units per lane
-    bool fullk;  // KU == LPN*UPL
-    bool wide;   // operands of 4 GiB or more: 64-bit byte offsets
-};
-
-int pow2ceil(int x) {
-    int l = 1;
-    while (l < x) l <<= 1;
-    return l;
-}
-
-Shape shape_of(const sddmm_ctx *c) {
-    Shape s{};
-    size_t unit_bytes;
-    if (c->dtype == SDDMM_BF16 || c->dtype == SDDMM_F16) { s.unit = c->dtype == SDDMM_BF16 ? 2 : 3; s.KU = c->K / 8; unit_bytes = 16; }
-    else if (c->K % 4 == 0) { s.unit = 0; s.KU = c->K / 4; unit_bytes = 16; }
-    else { s.unit = 1; s.KU = c->K; unit_bytes = 4; }
-    if (s.unit == 1) {
-        // 4-byte units: 16 lanes cover 64 contiguous bytes
-        if (s.KU <= 4) { s.LPN = 4; s.UPL = 1; }
-        else if (s.KU <= 16) { s.LPN = 16; s.UPL = 1; }
-        else if (s.KU <= 64) { s.LPN = 16; s.UPL = 4; }
-        else if (s.KU <= 128) { s.LPN = 16; s.UPL = 8; }
-        else { s.LPN = 0; s.UPL = 0; }
-    } else {
-        // 16-byte units: 8 lanes cover one whole 128-byte cache line per load
-        // instruction (measured faster than 4 lanes x 64 bytes: half the lines per
-        // instruction for the same bytes)
-        if (s.KU <= 8) { s.LPN = pow2ceil(s.KU); s.UPL = 1; }
-        else if (s.KU <= 64) { s.LPN = 8; s.UPL = pow2ceil((s.KU + 7) / 8); }
-        else if (s.KU <= 128) { s.LPN = 16; s.UPL = 8; }
-        else { s.LPN = 0; s.UPL = 0; }
-    }
-    s.fullk = s.LPN > 0 && s.KU == s.LPN * s.UPL;
-    const size_t rows = (size_t)std::max(c->M, c->N);
-    s.wide = rows * (size_t)s.KU * unit_bytes >= ((size_t)1 << 32);
-    return s;
-}
-
-// Calls f(Layout<...>{}) for the layout matching s.
-template <class U, int LPN, int UPL, class F>
-void with_mask_width(const Shape &s, F &&f) {
-    if (s.wide) f(Layout<U, LPN, UPL, false, true>{});
-    else if (s.fullk && U::ELEMS > 1) f(Layout<U, LPN, UPL, true, false>{});
-    else f(Layout<U, LPN, UPL, false, false>{});
-}
-
-template <class U, class F>
-void with_layout16(const Shape &s, F &&f) {
-    if (s.LPN == 0) { f(Layout<U, 0, 1, false, true>{}); return; }
-    if (s.LPN == 1) with_mask_width<U, 1, 1>(s, f);
-    else if (s.LPN == 2) with_mask_width<U, 2, 1>(s, f);
-    else if (s.LPN == 4) with_mask_width<U, 4, 1>(s, f);
-    else if (s.LPN == 16) with_mask_width<U, 16, 8>(s, f);
-    else if (s.UPL == 1) with_mask_width<U, 8, 1>(s, f);
-    else if (s.UPL == 2) with_mask_width<U, 8, 2>(s, f);
-    else if (s.UPL == 4) with_mask_width<U, 8, 4>(s, f);
-    else with_mask_width<U, 8, 8>(s, f);
-}
-
-template <class F>
-void with_layout(const Shape &s, F &&f) {
-    if (s.unit == 0) with_layout16<UnitF32x4>(s, f);
-    else if (s.unit == 2) with_layout16<UnitBF16x8>(s, f);
-    else if (s.unit == 3) with_layout16<UnitF16x8>(s, f);
-    else if (s.LPN == 0) f(Layout<UnitF32x1, 0, 1, false, true>{});
-    else if (s.LPN == 4) with_mask_width<UnitF32x1, 4, 1>(s, f);
-    else if (s.UPL == 1) with_mask_width<UnitF32x1, 16, 1>(s, f);
-    else if (s.UPL == 4) with_mask_width<UnitF32x1, 16, 4>(s, f);
-    else with_mask_width<UnitF32x1, 16, 8>(s, f);
-}
-
-void launch_flat(sddmm_ctx *c) {
-    const Shape s = shape_of(c);
-    const int64_t chunks = (c->nnz + WAVE - 1) / WAVE;
-    const int cpw = (int)std::min<int64_t>(8, std::max<int64_t>(1, chunks / (WAVES_PER_BLOCK * 4096)));
-    const int64_t waves = (chunks + cpw - 1) / cpw;
-    const int64_t nblocks = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    with_layout(s, [&](auto L) {
-        using LT = decltype(L);
-        SDDMM_LAUNCH(c, (k_flat<LT>), xcd_grid(nblocks), BLOCK,
-                           (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowidx, c->d_col, c->d_sval, c->dP,
-                           c->nnz, cpw, nblocks);
-    });
-}
-
-void launch_row_wave(sddmm_ctx *c, const RowItem *items, int64_t n_items) {
-    const Shape s = shape_of(c);
-    const int64_t nblocks = (n_items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    with_layout(s, [&](auto L) {
-        using LT = decltype(L);
-        SDDMM_LAUNCH(c, (k_row_wave<LT>), xcd_grid(nblocks), BLOCK,
-                           (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr, c->d_col, c->d_sval, c->dP,
-                           items, n_items, nblocks);
-    });
-}
-
 // rows per wavefront of the many-rows body: about 256 short entries per wave, so
 // that small matrices still produce enough waves to fill the chip
 int rows_per_wave(double avg_short_len) {
     int rpw = 64;
     while (rpw > 8 && rpw * std::max(avg_short_len, 1.0) > 384.0) rpw >>= 1;
     return rpw;
-}
-
-void launch_short_rows(sddmm_ctx *c, int ts, int rpw) {
-    const Shape s = shape_of(c);
-    const int64_t waves = ((int64_t)c->sM + rpw - 1) / rpw;
-    const int64_t nblocks = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    with_layout(s, [&](auto L) {
-        using LT = decltype(L);
-        SDDMM_LAUNCH(c, (k_short_rows<LT>), xcd_grid(nblocks), BLOCK,
-                           (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr, c->d_col, c->d_sval, c->dP,
-                           c->sM, ts, rpw, nblocks);
-    });
-}
-
-int env_int(const char *name, int fallback) {
-    const char *e = getenv(name);
-    return e && *e ? atoi(e) : fallback;
-}
-
-// wavefronts of the short-row part of the AUTO launches: 64 entries of the entry list each, or
-// rpw consecutive rows each
-int64_t short_row_waves(const sddmm_ctx *c) {
-    if (c->rows_short <= 0) return 0;
-    if (c->use_short_list) return (c->n_short_list + WAVE - 1) / WAVE;
-    return ((int64_t)c->sM + c->rpw - 1) / c->rpw;
-}
-
-// Tiles and rows in one launch (k_auto_tiles); measured faster than two launches at
-// every row size the tile path takes (mixed-density shape: 23 -> 20 us at 128-byte
-// rows, 107 -> 92 us at 1 KiB rows).  Returns false when the layout has no fused
-// kernel; the caller then launches the two kernels in turn.
-bool launch_auto_with_tiles(sddmm_ctx *c) {
-    const Shape s = shape_of(c);
-    if (c->tile_steps < 1 || c->tile_steps > env_int("SDDMM_FUSE_STEPS", 16) || !s.fullk || s.wide || s.unit == 1 || s.KU != 4 * c->tile_steps)
-        return false;
-    const int64_t waves = short_row_waves(c);
-    const int64_t short_blocks = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    const int64_t item_blocks = (c->n_items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    const int64_t tile_blocks = (c->n_tile_units + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    const int64_t nblocks = short_blocks + item_blocks + tile_blocks;
-    // Order of the blocks on every XCD.  Rows of up to 256 bytes: the tile windows (the wavefronts that
-    // live longest) start first, then the items, then the chunks of the entry list -- measured
-    // 14.7 -> 13.5 us on the mixed-density shape at 128 bytes, 21.3 -> 21.1 us (cold 29.7 -> 27.8) at
-    // 256; at 1 KiB, where the gathers of the short rows are the longer half, the even deal is 3 % faster.
-    const int longest_first = env_int("SDDMM_LONGEST_FIRST", c->tile_steps <= 4 ? 1 : 0);
-    auto eighth = [](int64_t n) { return (n + NUM_XCD - 1) / NUM_XCD; };
-    const int64_t grid = longest_first ? NUM_XCD * (eighth(short_blocks) + eighth(item_blocks) + eighth(tile_blocks))
-                                       : xcd_grid(nblocks);
-    bool launched = false;
-    with_layout(s, [&](auto L) {
-        using LT = decltype(L);
-        constexpr int KU_ = LT::LPN * LT::UPL;
-        if constexpr (!LT::LONG && LT::FULLK && !LT::WIDE && LT::U::ELEMS > 1 && (KU_ == 4 || KU_ == 8 || KU_ == 16 || KU_ == 32 || KU_ == 64)) {
-            SDDMM_LAUNCH(c, (k_auto_tiles<LT, KU_ / 4>), grid, BLOCK,
-                               (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr,
-                               (const unsigned char *)(c->owner_active ? c->d_owner : nullptr), c->d_col, c->d_sval,
-                               c->dP, c->sM, c->N, c->ts, c->rpw, short_blocks, c->d_items, c->n_items,
-                               (const int32_t *)c->d_vrows, (const int32_t *)c->d_tile_cols,
-                               (const TileDesc *)c->d_tiles, c->n_tiles,
-                               (const TileWindow *)(c->use_windows ? c->d_windows : nullptr), c->n_windows, c->nnz,
-                               tile_blocks, nblocks, (const int2 *)(c->use_short_list ? c->d_short_list : nullptr),
-                               c->n_short_list, longest_first,
-                               (const int32_t *)(c->use_win_order ? c->d_win_order : nullptr), c->n_win_single);
-            launched = true;
-        }
-    });
-    return launched;
-}
-
-void launch_auto(sddmm_ctx *c) {
-    const Shape s = shape_of(c);
-    const int64_t waves = short_row_waves(c);
-    const int64_t short_blocks = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    const int64_t item_blocks = (c->n_items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    const int64_t nblocks = short_blocks + item_blocks;
-    with_layout(s, [&](auto L) {
-        using LT = decltype(L);
-        SDDMM_LAUNCH(c, (k_auto<LT>), xcd_grid(nblocks), BLOCK,
-                           (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr,
-                           (const unsigned char *)(c->owner_active ? c->d_owner : nullptr), c->d_col, c->d_sval,
-                           c->dP, c->sM, c->ts, c->rpw, short_blocks, c->d_items, c->n_items, nblocks,
-                           (const int2 *)(c->use_short_list ? c->d_short_list : nullptr), c->n_short_list);
-    });
 }
 
 // Row classifier: statistics, then the item list of the wave-per-segment kernel.
@@ -897,17 +531,6 @@ int plan_tiles_fill(sddmm_ctx *c) {
     return SDDMM_OK;
 }
 
-// Row-panel detector (8 consecutive rows, 8-aligned, same column list).  Two
-// kernels can run the panels: the MFMA one (row size a multiple of 64 bytes, up to
-// 1 KiB) and the VALU one (8-lanes-per-entry layouts whose 8 A rows fit in
-// registers: fp32 K = 32 or 64, bf16 / fp16 K = 64, 32-bit offsets); the VALU kernel has
-// the per-entry arithmetic of the gather kernels, the MFMA kernel is faster.
-int panel_mfma_steps(const sddmm_ctx *c) {
-    const size_t row_bytes = (size_t)c->K * elem_size(c->dtype);
-    if (row_bytes % 64) return 0;
-    const int steps = (int)(row_bytes / 64);
-    return (steps == 1 || steps == 2 || steps == 4 || steps == 8 || steps == 16) ? steps : 0;
-}
 bool panel_valu_applicable(const sddmm_ctx *c) {
     const Shape s = shape_of(c);
     if (s.unit == 1 || s.LPN != 8 || !s.fullk || s.wide) return false;
@@ -948,99 +571,6 @@ int plan_panels_items(sddmm_ctx *c, int pseg) {
                        c->d_panel_items);
     LAUNCH_CHECK(c);
     return SDDMM_OK;
-}
-
-template <class U, int UPL>
-void launch_panel_t(sddmm_ctx *c, int KU) {
-    using LT = Layout<U, 8, UPL, true, false>;
-    const int64_t nblocks = (c->n_panel_items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    SDDMM_LAUNCH(c, (k_panel<LT>), xcd_grid(nblocks), BLOCK,
-                       (const void *)c->dA, (const void *)c->dB, KU, c->d_rowptr, c->d_col, c->d_sval, c->dP,
-                       (const RowItem *)c->d_panel_items, c->n_panel_items, nblocks);
-}
-template <class U>
-void launch_panel_u(sddmm_ctx *c, const Shape &s) {
-    if (s.UPL == 1) launch_panel_t<U, 1>(c, s.KU);
-    else launch_panel_t<U, 2>(c, s.KU);
-}
-template <int DT, int STEPS>
-void launch_panel_mfma_t(sddmm_ctx *c) {
-    constexpr int PW = panel_mfma_waves(STEPS);
-    const int64_t nblocks = (c->n_panel_items + PW - 1) / PW;
-    SDDMM_LAUNCH(c, (k_panel_mfma<DT, STEPS>), xcd_grid(nblocks), PW * WAVE,
-                       (const void *)c->dA, (const void *)c->dB, c->d_rowptr, c->d_col, (const float *)c->d_sval,
-                       c->dP, (const RowItem *)c->d_panel_items, c->n_panel_items, nblocks, (float *)nullptr);
-}
-// the panels of the fused SDDMM+SpMM: P and the panels' part of O
-template <int DT, int STEPS>
-void launch_panel_fused_t(sddmm_ctx *c) {
-    constexpr int PW = panel_mfma_waves(STEPS);
-    const int64_t nblocks = (c->n_panel_items + PW - 1) / PW;
-    SDDMM_LAUNCH(c, (k_panel_mfma<DT, STEPS, true>), xcd_grid(nblocks), PW * WAVE,
-                       (const void *)c->dA, (const void *)c->dB, c->d_rowptr, c->d_col, (const float *)c->d_sval,
-                       c->dP, (const RowItem *)c->d_panel_items, c->n_panel_items, nblocks, c->dO);
-}
-template <int DT>
-void launch_panel_mfma_steps(sddmm_ctx *c) {
-    switch (panel_mfma_steps(c)) {
-        case 1: launch_panel_mfma_t<DT, 1>(c); break;
-        case 2: launch_panel_mfma_t<DT, 2>(c); break;
-        case 4: launch_panel_mfma_t<DT, 4>(c); break;
-        case 8: launch_panel_mfma_t<DT, 8>(c); break;
-        default: launch_panel_mfma_t<DT, 16>(c); break;
-    }
-}
-
-void launch_panels(sddmm_ctx *c) {
-    if (c->panel_mfma) {
-        if (c->dtype == SDDMM_BF16) launch_panel_mfma_steps<DT_BF16>(c);
-        else if (c->dtype == SDDMM_F16) launch_panel_mfma_steps<DT_F16>(c);
-        else launch_panel_mfma_steps<DT_F32>(c);
-        return;
-    }
-    const Shape s = shape_of(c);
-    if (s.unit == 0) launch_panel_u<UnitF32x4>(c, s);
-    else if (s.unit == 2) launch_panel_t<UnitBF16x8, 1>(c, s.KU);
-    else launch_panel_t<UnitF16x8, 1>(c, s.KU);
-}
-
-template <int DT, int STEPS>
-void launch_tile_t(sddmm_ctx *c) {
-    // Well-filled tiles (walked from the descriptors' masks) of rows of 256 bytes and more, fewer
-    // windows than keep the chip busy on their own: one workgroup per window, K in four parts.
-    if constexpr (STEPS % KSPLIT == 0) {
-        if (!c->use_windows && c->n_windows <= (int64_t)env_int("SDDMM_KSPLIT_MAX", 32768) && env_int("SDDMM_KSPLIT", 1) != 0) {
-            const int64_t nb = c->n_windows;
-            SDDMM_LAUNCH(c, (k_tile_ksplit<DT, STEPS>), xcd_grid(nb), BLOCK,
-                               (const void *)c->dA, (const void *)c->dB, c->M, c->N, (const int32_t *)c->d_vrows,
-                               (const int32_t *)c->d_tile_cols, (const TileDesc *)c->d_tiles, c->n_tiles,
-                               (const float *)c->d_sval, c->dP, nb,
-                               (const int32_t *)(c->use_win_order ? c->d_win_order : nullptr));
-            return;
-        }
-    }
-    const int64_t nblocks = (c->n_tile_units + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    SDDMM_LAUNCH(c, (k_tile<DT, STEPS>), xcd_grid(nblocks), BLOCK,
-                       (const void *)c->dA, (const void *)c->dB, c->M, c->N, (const int32_t *)c->d_vrows,
-                       (const int32_t *)c->d_tile_cols, (const TileDesc *)c->d_tiles, c->n_tiles,
-                       (const TileWindow *)(c->use_windows ? c->d_windows : nullptr), c->n_windows,
-                       (const int32_t *)c->d_col, (const float *)c->d_sval, c->dP, c->nnz, nblocks,
-                       (const int32_t *)(c->use_win_order ? c->d_win_order : nullptr), c->n_win_single);
-}
-template <int DT>
-void launch_tile_steps(sddmm_ctx *c) {
-    switch (c->tile_steps) {
-        case 1: launch_tile_t<DT, 1>(c); break;
-        case 2: launch_tile_t<DT, 2>(c); break;
-        case 4: launch_tile_t<DT, 4>(c); break;
-        case 8: launch_tile_t<DT, 8>(c); break;
-        default: launch_tile_t<DT, 16>(c); break;
-    }
-}
-void launch_tiles(sddmm_ctx *c) {
-    if (c->dtype == SDDMM_BF16) launch_tile_steps<DT_BF16>(c);
-    else if (c->dtype == SDDMM_F16) launch_tile_steps<DT_F16>(c);
-    else launch_tile_steps<DT_F32>(c);
 }
 
 int ensure_rowidx(sddmm_ctx *c) {
@@ -1694,6 +1224,7 @@ int sddmm_run_fused(sddmm_ctx *c) {
     HIP_TRY(c, hipEventRecord(c->ev0, c->stream));
     // (when the panels own every row that has entries, O is complete after a memset and the panel kernel;
     // otherwise the kernel of the short rows, first in the stream, writes every row of O below sM, zeros
+
     // for the rows that the kernels after it add to, and only the rows of A beyond S are cleared here)
     const bool others = c->sM > 0 && c->nnz > 0 && (!panels || c->n_tiles > 0 || c->rows_short > 0 || c->n_items > 0);
     if (o_bytes) {
@@ -1701,62 +1232,13 @@ int sddmm_run_fused(sddmm_ctx *c) {
         if (written < o_bytes) HIP_TRY(c, hipMemsetAsync((char *)c->dO + written, 0, o_bytes - written, c->stream));
     }
     int launches = 0;
-    bool rows_written = false;
-    // Short rows of fewer entries, on average, than half of what a lane group takes per step (a power-law
-    // graph: 3.5 against 8 lanes per entry at 128-byte rows): one row per lane group would idle most of its
-    // steps (20 % of them useful there), so the wavefronts deal whole rows out to their groups by entry
-    // count instead (576 -> 369 us for those rows).  With longer rows, or 4 lanes per entry, the extra
-    // gathers of the A rows and the longer walks cost more than the idle steps (mixed-density shape, 12.5
-    // entries per short row: 33 -> 65 us; power-law with 64-byte rows: 396 -> 432 us).
-    const int balanced_env = env_int("SDDMM_FUSED_BALANCED", -1);
-    const bool balanced = balanced_env >= 0 ? balanced_env != 0
-                                            : (c->fused_short_avg > 0.0 && 2.0 * c->fused_short_avg < (double)s.LPN);
     if (c->sM > 0 && c->nnz > 0) {
-        with_layout(s, [&](auto L) {
-            using LT = decltype(L);
-            if (!others) return;
-            if constexpr (!LT::LONG && LT::LPN <= 8 && LT::U::ELEMS > 1 && LT::UPL * LT::U::ELEMS <= 32) {
-                const int64_t rows_per_wave = WAVE / LT::LPN;
-                const int64_t waves = ((int64_t)c->sM + rows_per_wave - 1) / rows_per_wave;
-                const int64_t rblocks = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-                if (balanced) {
-                    const int64_t bwaves = ((int64_t)c->sM + WAVE - 1) / WAVE;
-                    const int64_t bblocks = (bwaves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-                    SDDMM_LAUNCH(c, (k_fusedmm_rows_balanced<LT>), xcd_grid(bblocks), BLOCK,
-                                       (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr, c->d_col, c->d_sval,
-                                       c->dP, c->dO, c->sM, FUSED_ROW_MAX, bblocks, panel_owner);
-                } else {
-                    SDDMM_LAUNCH(c, (k_fusedmm_rows<LT>), xcd_grid(rblocks), BLOCK,
-                                       (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr, c->d_col, c->d_sval,
-                                       c->dP, c->dO, c->sM, FUSED_ROW_MAX, rblocks, panel_owner);
-                }
-                ++launches;
-                rows_written = true;
-                if (c->n_fused_items > 0) {
-                    const int64_t nblocks = (c->n_fused_items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-                    SDDMM_LAUNCH(c, (k_fusedmm<LT>), xcd_grid(nblocks), BLOCK,
-                                       (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr, c->d_col,
-                                       c->d_sval, c->dP, c->dO, (const RowItem *)c->d_fused_items, c->n_fused_items,
-                                       nblocks);
-                    ++launches;
-                }
-            }
-        });
-        if (others && !rows_written) return fail(c, SDDMM_ERR_UNSUPPORTED, "internal: no fused kernel for this row layout");
+        if (others) {
+            launches = launch_fused_rows(c, panel_owner);
+            if (launches == 0) return fail(c, SDDMM_ERR_UNSUPPORTED, "internal: no fused kernel for this row layout");
+        }
         if (panels) {
-            if (c->dtype == SDDMM_F32) {
-                if (c->K == 32) launch_panel_fused_t<DT_F32, 2>(c);
-                else if (c->K == 64) launch_panel_fused_t<DT_F32, 4>(c);
-                else launch_panel_fused_t<DT_F32, 8>(c);
-            } else if (c->dtype == SDDMM_BF16) {
-                if (c->K == 32) launch_panel_fused_t<DT_BF16, 1>(c);
-                else if (c->K == 64) launch_panel_fused_t<DT_BF16, 2>(c);
-                else launch_panel_fused_t<DT_BF16, 4>(c);
-            } else {
-                if (c->K == 32) launch_panel_fused_t<DT_F16, 1>(c);
-                else if (c->K == 64) launch_panel_fused_t<DT_F16, 2>(c);
-                else launch_panel_fused_t<DT_F16, 4>(c);
-            }
+            launch_panels_fused(c);
             ++launches;
         }
         LAUNCH_CHECK(c);
