@@ -114,6 +114,10 @@ struct sddmm_ctx {
     int64_t n_panel_items = 0, panel_items_cap = 0, n_panels = 0, nnz_panels = 0;
     bool panel_mfma = false;         // panels run on k_panel_mfma (else on k_panel)
     bool panels_flagged = false;     // the panel detector ran in this plan
+    // FLAT in slices of K (kernels_flat.h): partial products of a range of entries, [slice][entry]
+    float *d_part = nullptr;
+    int64_t part_floats = 0;
+    bool use_slices = false;         // set by a plan of SDDMM_AUTO
     // fused SDDMM + SpMM: items covering every non-empty row, output M x K
     RowItem *d_fused_items = nullptr;
     int64_t n_fused_items = 0, fused_items_cap = 0;
@@ -286,6 +290,9 @@ inline int panel_mfma_steps(const sddmm_ctx *c) {
 
 // ---- launchers, one translation unit per family of kernels ----
 void launch_flat(sddmm_ctx *c);                                                  // launch_flat.hip
+bool slices_pay(const sddmm_ctx *c, double entries_per_row);
+int64_t slice_workspace_floats(const sddmm_ctx *c);
+int launch_flat_sliced(sddmm_ctx *c);                                            // number of launches
 void launch_row_wave(sddmm_ctx *c, const RowItem *items, int64_t n_items);       // launch_rows.hip
 void launch_short_rows(sddmm_ctx *c, int ts, int rpw);
 void launch_auto(sddmm_ctx *c);

@@ -91,6 +91,11 @@ __device__ __forceinline__ void st_stream(T *p, T v) {
 #endif
 }
 
+// four consecutive values of an array that is only 4-byte aligned, as one access
+struct __attribute__((packed, aligned(4))) I4u { int x, y, z, w; };
+struct __attribute__((packed, aligned(4))) F4u { float x, y, z, w; };
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
+
 // One work item of the wave-per-segment kernel: entries [start,end) of one row.
 struct RowItem {
     int32_t row;

@@ -61,9 +61,6 @@ __device__ __forceinline__ int sum16(int v) {
 // row's first position and column mask in the tile (mask 0: row absent).  The walk
 // stops early when on_tile returns false (it must return the same in all 16 lanes).
 // Returns false in a lane whose row is not strictly increasing in column.
-struct __attribute__((packed, aligned(4))) I4u { int x, y, z, w; };
-struct __attribute__((packed, aligned(4))) F4u { float x, y, z, w; };
-
 template <class F>
 __device__ __forceinline__ bool walk_strip(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int M,
                                            int64_t strip, int sub, F &&on_tile) {
@@ -849,7 +846,6 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_apply(const unsigned
 // ---- the MFMA kernel ------------------------------------------------------------
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
 
 // One wavefront computes `tiles_per_wave` consecutive tiles.  Operand layout of
 // both MFMA shapes used: lane l supplies row (l & 15) of its operand and the k

@@ -1,5 +1,6 @@
-// Launch of the flat gather kernel.
+// Launches of the flat gather kernel and of its variant in slices of K.
 #include "context.h"
+#include "kernels_flat.h"
 
 void launch_flat(sddmm_ctx *c) {
     const Shape s = shape_of(c);
@@ -13,4 +14,82 @@ void launch_flat(sddmm_ctx *c) {
                            (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowidx, c->d_col, c->d_sval, c->dP,
                            c->nnz, cpw, nblocks);
     });
+}
+
+namespace {
+
+constexpr int64_t SLICE_WORKSPACE = (int64_t)1 << 26;      // floats: the partial products stay in the last-level cache
+
+// slices (lines) that the longest row touches: rows start anywhere in a line that B's address and the
+// row length lead to
+int slices_of(uint64_t b_address, int64_t row_bytes) {
+    int64_t most = 0;
+    for (int i = 0; i < 32; ++i) most = std::max(most, (int64_t)((b_address + (uint64_t)i * (uint64_t)row_bytes) % SLICE_BYTES));
+    return (int)((row_bytes + most + SLICE_BYTES - 1) / SLICE_BYTES);
+}
+
+template <class U, bool MISALIGNED, bool UNALIGNED, bool WIDE>
+int launch_slices_t(sddmm_ctx *c, int slices) {
+    const int row_bytes = c->K * (int)elem_size(c->dtype);
+    const int64_t most = c->part_floats / slices / SLICE_ENTRIES * SLICE_ENTRIES;      // entries the workspace holds
+    int launches = 0;
+    for (int64_t e0 = 0; e0 < c->nnz; e0 += most) {
+        const int64_t n = std::min(most, c->nnz - e0);
+        const int64_t stride = (n + WAVE - 1) / WAVE * WAVE;
+        const int64_t waves = (n + SLICE_ENTRIES - 1) / SLICE_ENTRIES;
+        const int64_t per_slice = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK, nblocks = per_slice * slices;
+        SDDMM_LAUNCH(c, (k_slice_dots<U, MISALIGNED, UNALIGNED, WIDE>), xcd_grid(nblocks), BLOCK, (const void *)c->dA,
+                     (const void *)c->dB, row_bytes, (const int32_t *)c->d_rowidx + e0, (const int32_t *)c->d_col + e0,
+                     c->d_part, n, stride, per_slice, nblocks);
+        SDDMM_LAUNCH(c, k_slice_sum, (n + 4 * BLOCK - 1) / (4 * BLOCK), BLOCK, (const float *)c->d_part, slices, stride,
+                     (const float *)c->d_sval + e0, c->dP + e0, n);
+        launches += 2;
+    }
+    return launches;
+}
+
+template <class U>
+int launch_slices_u(sddmm_ctx *c) {
+    const int64_t row_bytes = (int64_t)c->K * (int64_t)elem_size(c->dtype);
+    const int slices = slices_of((uint64_t)(uintptr_t)c->dB, row_bytes);
+    const bool wide = (size_t)std::max(c->M, c->N) * (size_t)row_bytes >= ((size_t)1 << 32);
+    if constexpr (U::DT == DT_F32) {
+        if (row_bytes % 16)
+            return wide ? launch_slices_t<U, true, true, true>(c, slices) : launch_slices_t<U, true, true, false>(c, slices);
+    }
+    if (wide) return launch_slices_t<U, true, false, true>(c, slices);
+    if (row_bytes % SLICE_BYTES || (uintptr_t)c->dB % SLICE_BYTES) return launch_slices_t<U, true, false, false>(c, slices);
+    return launch_slices_t<U, false, false, false>(c, slices);
+}
+
+}  // namespace
+
+// Measured on uniform random matrices of about 1 M entries, N = 1 000 .. 100 000, K = 64 .. 1 000 in fp32, 6 .. 60 entries
+// per row, against the better of k_flat and k_auto.  Slices gain where B exceeds the L2s (1.2 .. 2.2 times from 8 MB on;
+// 0.6 .. 1.1 times below 5 MB), as long as one slice of it comes near to fitting (N = 65 536 is 8 MB: 1.2; 100 000: 1.0) and
+// rows are several lines (256 bytes: 0.8 .. 1.1; 400 bytes: 1.0 .. 1.3).  Very short rows have their A rows gathered
+// per entry, which only pays while the slice fits (6 entries per row: 1.2 at N = 20 000, 0.8 .. 1.1 at 40 000).  Rows
+// beyond the register layout of the gather kernels (2 KB) gain everywhere: 1.3 times at the least.
+bool slices_pay(const sddmm_ctx *c, double entries_per_row) {
+    const int64_t row_bytes = (int64_t)c->K * (int64_t)elem_size(c->dtype);
+    const int mode = env_int("SDDMM_SLICES", -1);                   // -1: decide here, 0: never, 1: wherever the kernel can
+    if (mode >= 0) return mode != 0 && row_bytes > SLICE_BYTES && row_bytes < (1 << 30);
+    if (row_bytes > 2048) return row_bytes < (1 << 30);
+    const int64_t MB = 1 << 20;
+    return row_bytes >= 400 && (int64_t)c->N * row_bytes >= 8 * MB &&
+           (int64_t)c->N * SLICE_BYTES <= (entries_per_row >= 12.0 ? 8 * MB : 3 * MB);
+}
+
+// The partial products of all entries where they fit SLICE_WORKSPACE, of a range of entries at a time otherwise.
+int64_t slice_workspace_floats(const sddmm_ctx *c) {
+    const int64_t slices = ((int64_t)c->K * (int64_t)elem_size(c->dtype) + SLICE_BYTES - 1) / SLICE_BYTES + 1;   // whatever B's address
+    const int64_t all = (c->nnz + SLICE_ENTRIES - 1) / SLICE_ENTRIES * SLICE_ENTRIES * slices;
+    const int64_t cap = std::max((int64_t)env_int("SDDMM_SLICE_WORKSPACE", (int)SLICE_WORKSPACE), SLICE_ENTRIES * slices);
+    return std::min(all, cap);
+}
+
+int launch_flat_sliced(sddmm_ctx *c) {
+    if (c->dtype == SDDMM_BF16) return launch_slices_u<UnitBF16x8>(c);
+    if (c->dtype == SDDMM_F16) return launch_slices_u<UnitF16x8>(c);
+    return launch_slices_u<UnitF32x4>(c);
 }

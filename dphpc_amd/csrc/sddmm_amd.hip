@@ -584,6 +584,23 @@ int ensure_rowidx(sddmm_ctx *c) {
     return SDDMM_OK;
 }
 
+// Room for the partial products of the slices of K; false when the device does not have it (the launch
+// then takes the plain flat kernel).  Kept until the context goes.
+bool ensure_slice_workspace(sddmm_ctx *c) {
+    const int64_t need = slice_workspace_floats(c);
+    if (need <= c->part_floats) return true;
+    dfree(c->d_part);
+    c->part_floats = 0;
+    void *p = nullptr;
+    if (hipMalloc(&p, (size_t)need * sizeof(float)) != hipSuccess || !p) {
+        (void)hipGetLastError();                           // the failed allocation is not an error of the plan
+        return false;
+    }
+    c->d_part = static_cast<float *>(p);
+    c->part_floats = need;
+    return true;
+}
+
 // Validate the device-resident CSR and gather row statistics.
 int validate_csr(sddmm_ctx *c) {
     HIP_TRY(c, hipMemsetAsync(c->d_pc, 0, sizeof(DevCounters), c->stream));
@@ -636,7 +653,10 @@ int enqueue_run(sddmm_ctx *c) {
             if (rows && !fused) { launch_auto(c); ++c->launches; }
             break;
         }
-        case SDDMM_FLAT: launch_flat(c); break;
+        case SDDMM_FLAT:
+            if (c->use_slices) c->launches = launch_flat_sliced(c);
+            else launch_flat(c);
+            break;
         case SDDMM_ROW_WAVE: launch_row_wave(c, nullptr, c->sM); break;
         case SDDMM_SHORT_ROWS:
             launch_short_rows(c, INT32_MAX, rows_per_wave(c->sM ? (double)c->nnz / c->sM : 0.0));
@@ -664,6 +684,7 @@ int do_plan(sddmm_ctx *c, int strategy) {
     // previous one looking valid (its items exclude rows that tiles and panels owned)
     c->planned = false;
     c->n_scan_jobs = 0;
+    c->use_slices = false;
     c->fused_items_valid = false;    // they leave out the rows of this plan's panels
     int resolved = strategy;
     const bool csr_ok = c->have_rowptr;
@@ -751,14 +772,16 @@ int do_plan(sddmm_ctx *c, int strategy) {
             // kernel (row index per entry, perfectly balanced) measured 6 % faster there than
             // the row split (power-law shape, K=32: 634 us against 672 us).
             const double avg_len = c->pc.rows_nonempty ? (double)c->nnz / (double)c->pc.rows_nonempty : 0.0;
-            const bool flat = resolved == SDDMM_AUTO && c->n_tiles == 0 && c->n_panel_items == 0 &&
-                              avg_len < (double)env_int("SDDMM_FLAT_AVG", 32);
+            const bool only_rows = resolved == SDDMM_AUTO && c->n_tiles == 0 && c->n_panel_items == 0;
+            const bool sliced = only_rows && slices_pay(c, avg_len) && ensure_slice_workspace(c);
+            const bool flat = only_rows && (sliced || avg_len < (double)env_int("SDDMM_FLAT_AVG", 32));
             rc = classify_rows_items(c, !flat);      // (the flat kernel has no use for the entry list of the short rows)
             if (rc) return rc;
             if (flat) {
                 rc = ensure_rowidx(c);
                 if (rc) return rc;
                 resolved = SDDMM_FLAT;
+                c->use_slices = sliced;
             }
             break;
         }
@@ -766,6 +789,8 @@ int do_plan(sddmm_ctx *c, int strategy) {
         case SDDMM_EXACT: {
             int rc = ensure_rowidx(c);
             if (rc) return rc;
+            // (asked for by name, FLAT stays the plain kernel; AUTO on unsorted entries gets here too)
+            if (strategy == SDDMM_AUTO) c->use_slices = c->nnz > 0 && slices_pay(c, 1.0) && ensure_slice_workspace(c);
             break;
         }
         case SDDMM_ROW_WAVE:
@@ -872,6 +897,7 @@ void sddmm_destroy(sddmm_ctx *c) {
     release_dense(c);
     release_sparse(c);
     dfree(c->dO);
+    dfree(c->d_part);
     dfree(c->d_pc);
     if (c->h_pc) (void)hipHostFree(c->h_pc);
     if (c->ev0) (void)hipEventDestroy(c->ev0);

@@ -1,0 +1,139 @@
+"""The flat kernel in slices of K (rows of more than 128 bytes), forced on wherever it can run:
+edges of lines, units, chunks and staged rows, against the oracle.  All GPU.
+
+Same bar as test_gpu_parity.py.  B and A rows without entries hold NaN: every lane that
+reads outside its entry's row (windows are moved down to lines) must leave the sum alone.
+"""
+import numpy as np
+import pytest
+
+from dphpc_amd import capi
+from oracle import oracle as O
+from test_gpu_device_pointers import Hip
+
+pytestmark = pytest.mark.gpu
+f32 = np.float32
+
+
+def _case(seed, M, N, K, dtype, nnz=None, density=0.3):
+    rng = np.random.default_rng(seed)
+    mask = rng.random((M, N)) < density
+    mask[:, ::2] = False                                  # every other B row is nobody's
+    mask[1::5] = False                                    # and every fifth A row
+    r, c = np.nonzero(mask)
+    if nnz is not None:
+        assert len(r) >= nnz
+        r, c = r[:nnz], c[:nnz]
+    A = rng.uniform(-1, 1, (M, K)).astype(f32)
+    B = rng.uniform(-1, 1, (N, K)).astype(f32)
+    if dtype == capi.BF16:
+        A, B = capi.from_bf16(capi.to_bf16(A)), capi.from_bf16(capi.to_bf16(B))
+    elif dtype == capi.F16:
+        A, B = capi.from_f16(capi.to_f16(A)), capi.from_f16(capi.to_f16(B))
+    B[np.setdiff1d(np.arange(N), c)] = np.nan
+    A[np.setdiff1d(np.arange(M), r)] = np.nan
+    return r.astype(np.int32), c.astype(np.int32), rng.uniform(-1, 1, len(r)).astype(f32), A, B
+
+
+def _bits(x, dtype):
+    return x if dtype == capi.F32 else capi.to_bf16(x) if dtype == capi.BF16 else capi.to_f16(x)
+
+
+def _check(got, r, c, v, A, B, what):
+    M = A.shape[0]
+    rowptr, col, val = O.csr_from_triplets(M, r, c, v)
+    order = np.lexsort((c, r))
+    ref = O.sddmm_csr(rowptr, col, val, A, B, threads=0)
+    _, mag = O.sddmm_csr_f64(rowptr, col, val, A, B)
+    ok, worst, i = O.check_values(got[order], ref, mag=mag)
+    assert ok, "%s: entry %d got %r ref %r (%.2f x tolerance)" % (what, i, got[order][i], ref[i], worst)
+
+
+@pytest.fixture(autouse=True)
+def _no_tiles(monkeypatch):
+    """These patterns are dense enough for the matrix cores: keep every row on the gather kernels."""
+    for name, value in (("SDDMM_TILE_FILL", "100000"), ("SDDMM_UNION", "0"), ("SDDMM_GATHERED", "0")):
+        monkeypatch.setenv(name, value)
+
+
+SHAPES = [(capi.F32, K) for K in (33, 36, 63, 64, 65, 94, 100, 127, 128, 131, 250, 513, 1000, 1001)] + \
+         [(capi.BF16, K) for K in (72, 128, 136, 1032)] + [(capi.F16, K) for K in (72, 128, 2000)]
+
+
+@pytest.mark.parametrize("dtype,K", SHAPES)
+def test_slices_any_row_length(engine_factory, monkeypatch, dtype, K):
+    monkeypatch.setenv("SDDMM_SLICES", "1")
+    # rows of many entries (A staged in LDS), rows of one or two (A gathered), a bit of both
+    for seed, M, N, density in ((1, 60, 150, 0.6), (2, 700, 61, 0.04), (3, 150, 90, 0.3)):
+        r, c, v, A, B = _case(K + seed, M, N, K, dtype, density=density)
+        print("slices", dtype, K, M, N, len(r), flush=True)
+        rowptr, col, val = O.csr_from_triplets(M, r, c, v)
+        with engine_factory() as e:
+            e.set_dense(_bits(A, dtype), _bits(B, dtype), dtype)
+            e.set_csr(M, N, rowptr, col, val)
+            e.plan(capi.AUTO)
+            e.run()
+            assert e.stats().kernels_launched == 2
+            _check(e.values(), r, c, v, A, B, "K=%d sorted" % K)
+            perm = np.random.default_rng(seed).permutation(len(r))
+            e.set_coo(M, N, r[perm], c[perm], v[perm])
+            e.plan(capi.AUTO)
+            e.run()
+            assert e.stats().kernels_launched == 2
+            _check(e.values(), r[perm], c[perm], v[perm], A, B, "K=%d unsorted" % K)
+
+
+@pytest.mark.parametrize("nnz", [1, 63, 64, 65, 255, 256, 257, 1023, 1025, 2050])
+def test_slices_entry_counts_and_ranges(engine_factory, monkeypatch, nnz):
+    """Remainders of chunks, wavefronts and workgroups; and a workspace that holds a few hundred entries."""
+    monkeypatch.setenv("SDDMM_SLICES", "1")
+    K = 100
+    r, c, v, A, B = _case(nnz, 90, 120, K, capi.F32, nnz=nnz, density=0.7)
+    rowptr, col, val = O.csr_from_triplets(90, r, c, v)
+    for workspace in (None, "1", "3000"):
+        if workspace:
+            monkeypatch.setenv("SDDMM_SLICE_WORKSPACE", workspace)
+        print("slices nnz", nnz, workspace, flush=True)
+        with engine_factory() as e:
+            e.set_dense(A, B)
+            e.set_csr(90, 120, rowptr, col, val)
+            e.plan(capi.AUTO)
+            e.run()
+            _check(e.values(), r, c, v, A, B, "nnz=%d workspace=%s" % (nnz, workspace))
+
+
+@pytest.mark.parametrize("K", [64, 100, 301])
+def test_slices_follow_the_address_of_b(engine_factory, monkeypatch, K):
+    """New A and B at another alignment keep the plan: the lines of a row follow the new address."""
+    monkeypatch.setenv("SDDMM_SLICES", "1")
+    r, c, v, A, B = _case(K, 80, 110, K, capi.F32)
+    rowptr, col, val = O.csr_from_triplets(80, r, c, v)
+    hip = Hip()
+    e = engine_factory()                                   # creates the context (and selects the device) first
+    try:
+        for shift in (0, 4, 20, 28):                       # floats: 16-byte steps inside a 128-byte line
+            lead = np.zeros(shift, f32)
+            dA, dB = hip.upload(np.concatenate([lead, A.ravel()])), hip.upload(np.concatenate([lead, B.ravel()]))
+            e._chk(e.L.sddmm_set_dense_device(e.h, 80, 110, K, dA.value + 4 * shift, dB.value + 4 * shift, capi.F32))
+            if shift == 0:
+                e.set_csr(80, 110, rowptr, col, val)
+                e.plan(capi.AUTO)
+            e.run()
+            _check(e.values(), r, c, v, A, B, "K=%d shift=%d" % (K, shift))
+    finally:
+        e.close()                                          # the context goes first, the borrowed buffers after it
+        hip.free_all()
+
+
+def test_rows_beyond_the_register_layout_take_slices(engine_factory):
+    """The rule itself: rows of more than 2 KB take slices under AUTO; FLAT by name stays one plain kernel."""
+    r, c, v, A, B = _case(5, 70, 90, 515, capi.F32)
+    rowptr, col, val = O.csr_from_triplets(70, r, c, v)
+    with engine_factory() as e:
+        e.set_dense(A, B)
+        e.set_csr(70, 90, rowptr, col, val)
+        for strategy, launches in ((capi.AUTO, 2), (capi.FLAT, 1)):
+            e.plan(strategy)
+            e.run()
+            assert e.stats().strategy_used == capi.FLAT and e.stats().kernels_launched == launches
+            _check(e.values(), r, c, v, A, B, capi.STRATEGY_NAMES[strategy])
