@@ -193,12 +193,14 @@ inline int env_int(const char *name, int fallback) {
 
 // ---- kernel dispatch over the (unit type, lanes per entry, units per lane) layouts ----
 struct Shape {
-    int unit;    // 0: fp32 x4, 1: fp32 x1, 2: bf16 x8, 3: fp16 x8
+    int unit;    // 0: fp32 x4, 1: fp32 x1 (K < 4), 2: bf16 x8, 3: fp16 x8, 4: fp32 x4 in rows of no whole number of units
     int KU;      // units per row
+    int len;     // length of a row as the kernels take it: KU, or K where rows hold no whole number of units
     int LPN;     // lanes per entry (0: row too long for the register layout)
     int UPL;     // units per lane
     bool fullk;  // KU == LPN*UPL
     bool wide;   // operands of 4 GiB or more: 64-bit byte offsets
+    bool whole() const { return unit == 0 || unit == 2 || unit == 3; }     // 16-byte units only
 };
 
 inline int pow2ceil(int x) {
@@ -209,29 +211,30 @@ inline int pow2ceil(int x) {
 
 inline Shape shape_of(const sddmm_ctx *c) {
     Shape s{};
-    size_t unit_bytes;
-    if (c->dtype == SDDMM_BF16 || c->dtype == SDDMM_F16) { s.unit = c->dtype == SDDMM_BF16 ? 2 : 3; s.KU = c->K / 8; unit_bytes = 16; }
-    else if (c->K % 4 == 0) { s.unit = 0; s.KU = c->K / 4; unit_bytes = 16; }
-    else { s.unit = 1; s.KU = c->K; unit_bytes = 4; }
+    if (c->dtype == SDDMM_BF16 || c->dtype == SDDMM_F16) { s.unit = c->dtype == SDDMM_BF16 ? 2 : 3; s.KU = s.len = c->K / 8; }
+    else if (c->K % 4 == 0) { s.unit = 0; s.KU = s.len = c->K / 4; }
+    else if (c->K > 4) { s.unit = 4; s.KU = (c->K + 3) / 4; s.len = c->K; }
+    else { s.unit = 1; s.KU = s.len = c->K; }
     if (s.unit == 1) {
-        // 4-byte units: 16 lanes cover 64 contiguous bytes
-        if (s.KU <= 4) { s.LPN = 4; s.UPL = 1; }
-        else if (s.KU <= 16) { s.LPN = 16; s.UPL = 1; }
-        else if (s.KU <= 64) { s.LPN = 16; s.UPL = 4; }
-        else if (s.KU <= 128) { s.LPN = 16; s.UPL = 8; }
-        else { s.LPN = 0; s.UPL = 0; }
+        s.LPN = 4; s.UPL = 1;
     } else {
         // 16-byte units: 8 lanes cover one whole 128-byte cache line per load
         // instruction (measured faster than 4 lanes x 64 bytes: half the lines per
         // instruction for the same bytes)
         if (s.KU <= 8) { s.LPN = pow2ceil(s.KU); s.UPL = 1; }
-        else if (s.KU <= 64) { s.LPN = 8; s.UPL = pow2ceil((s.KU + 7) / 8); }
+        else if (s.KU <= 64) {
+            // units per lane: as few as hold the row, of those that have a kernel (a lane without a unit
+            // of its own loads another one again: K = 96 31.9 us with four per lane, 25.5 with three)
+            s.LPN = 8;
+            const int upl = (s.KU + 7) / 8;
+            s.UPL = upl <= 4 ? upl : upl <= 6 ? 6 : 8;
+        }
         else if (s.KU <= 128) { s.LPN = 16; s.UPL = 8; }
         else { s.LPN = 0; s.UPL = 0; }
     }
     s.fullk = s.LPN > 0 && s.KU == s.LPN * s.UPL;
     const size_t rows = (size_t)std::max(c->M, c->N);
-    s.wide = rows * (size_t)s.KU * unit_bytes >= ((size_t)1 << 32);
+    s.wide = rows * (size_t)c->K * elem_size(c->dtype) >= ((size_t)1 << 32);
     return s;
 }
 
@@ -239,7 +242,7 @@ inline Shape shape_of(const sddmm_ctx *c) {
 template <class U, int LPN, int UPL, class F>
 void with_mask_width(const Shape &s, F &&f) {
     if (s.wide) f(Layout<U, LPN, UPL, false, true>{});
-    else if (s.fullk && U::ELEMS > 1) f(Layout<U, LPN, UPL, true, false>{});
+    else if (s.fullk && U::WHOLE && U::ELEMS > 1 && UPL != 3 && UPL != 6) f(Layout<U, LPN, UPL, true, false>{});
     else f(Layout<U, LPN, UPL, false, false>{});
 }
 
@@ -252,7 +255,9 @@ void with_layout16(const Shape &s, F &&f) {
     else if (s.LPN == 16) with_mask_width<U, 16, 8>(s, f);
     else if (s.UPL == 1) with_mask_width<U, 8, 1>(s, f);
     else if (s.UPL == 2) with_mask_width<U, 8, 2>(s, f);
+    else if (s.UPL == 3) with_mask_width<U, 8, 3>(s, f);
     else if (s.UPL == 4) with_mask_width<U, 8, 4>(s, f);
+    else if (s.UPL == 6) with_mask_width<U, 8, 6>(s, f);
     else with_mask_width<U, 8, 8>(s, f);
 }
 
@@ -261,11 +266,8 @@ void with_layout(const Shape &s, F &&f) {
     if (s.unit == 0) with_layout16<UnitF32x4>(s, f);
     else if (s.unit == 2) with_layout16<UnitBF16x8>(s, f);
     else if (s.unit == 3) with_layout16<UnitF16x8>(s, f);
-    else if (s.LPN == 0) f(Layout<UnitF32x1, 0, 1, false, true>{});
-    else if (s.LPN == 4) with_mask_width<UnitF32x1, 4, 1>(s, f);
-    else if (s.UPL == 1) with_mask_width<UnitF32x1, 16, 1>(s, f);
-    else if (s.UPL == 4) with_mask_width<UnitF32x1, 16, 4>(s, f);
-    else with_mask_width<UnitF32x1, 16, 8>(s, f);
+    else if (s.unit == 4) with_layout16<UnitF32x4u>(s, f);
+    else with_mask_width<UnitF32x1, 4, 1>(s, f);
 }
 
 // wavefronts of the short-row part of the AUTO launches: 64 entries of the entry list each, or
@@ -295,7 +297,7 @@ int64_t slice_workspace_floats(const sddmm_ctx *c);
 int launch_flat_sliced(sddmm_ctx *c);                                            // number of launches
 void launch_row_wave(sddmm_ctx *c, const RowItem *items, int64_t n_items);       // launch_rows.hip
 void launch_short_rows(sddmm_ctx *c, int ts, int rpw);
-void launch_auto(sddmm_ctx *c);
+void launch_auto(sddmm_ctx *c);                                                  // launch_auto.hip
 bool launch_auto_with_tiles(sddmm_ctx *c);                                       // launch_tiles.hip
 void launch_tiles(sddmm_ctx *c);
 void launch_panels(sddmm_ctx *c);                                                // launch_panels.hip

@@ -108,12 +108,26 @@ struct RowItem {
 // A "unit" is what one lane loads per step along K: 16 bytes where alignment
 // allows (4 fp32, 8 bf16 or 8 fp16), one fp32 otherwise.  dot() extends an fp32
 // accumulator with fused multiply-adds in element order.
+// The kernels take the length of a row as a number of units, or of elements where rows hold no
+// whole number of units (fp32, K % 4 != 0: rows are 4-byte aligned, which is all that 16-byte
+// global loads need).  The last unit of such a row then ends with the row; its first elements
+// are the unit's before it, and trim() zeroes them.
 // element types of A and B as template arguments of the kernels
 constexpr int DT_F32 = 0, DT_BF16 = 1, DT_F16 = 2;
 
-struct UnitF32x4 {
+template <class T_>
+struct WholeUnits {
+    using T = T_;
+    static constexpr bool WHOLE = true;
+    static __device__ __forceinline__ int units(int len) { return len; }
+    static __device__ __forceinline__ uint32_t row_bytes(int len) { return (uint32_t)len * (uint32_t)sizeof(T); }
+    static __device__ __forceinline__ uint32_t unit_off(int u, int) { return (uint32_t)u * (uint32_t)sizeof(T); }
+    static __device__ __forceinline__ T load(const char *p) { return *reinterpret_cast<const T *>(p); }
+    static __device__ __forceinline__ T trim(const T &v, int, int) { return v; }
+};
+
+struct UnitF32x4 : WholeUnits<float4> {
     static constexpr int DT = DT_F32;
-    using T = float4;
     static constexpr int ELEMS = 4;
     static __device__ __forceinline__ T zero() { return make_float4(0.f, 0.f, 0.f, 0.f); }
     static __device__ __forceinline__ float dot(const T &a, const T &b, float acc) {
@@ -131,18 +145,33 @@ struct UnitF32x4 {
         acc[3] = __builtin_fmaf(p, b.w, acc[3]);
     }
 };
-struct UnitF32x1 {
+struct UnitF32x4u : UnitF32x4 {
+    static constexpr bool WHOLE = false;
+    static __device__ __forceinline__ int units(int len) { return (len + 3) >> 2; }
+    static __device__ __forceinline__ uint32_t row_bytes(int len) { return (uint32_t)len * 4u; }
+    static __device__ __forceinline__ uint32_t unit_off(int u, int len) {
+        const uint32_t at = (uint32_t)u * 16u, top = (uint32_t)len * 4u - 16u;
+        return at < top ? at : top;
+    }
+    static __device__ __forceinline__ T load(const char *p) {
+        return __builtin_bit_cast(T, *reinterpret_cast<const F4u *>(p));
+    }
+    static __device__ __forceinline__ T trim(const T &v, int u, int len) {
+        const int n = units(len), cut = u == n - 1 ? 4 * n - len : 0;
+        return make_float4(cut > 0 ? 0.f : v.x, cut > 1 ? 0.f : v.y, cut > 2 ? 0.f : v.z, v.w);
+    }
+};
+struct UnitF32x1 : WholeUnits<float> {           // rows of fewer than four elements
     static constexpr int DT = DT_F32;
-    using T = float;
     static constexpr int ELEMS = 1;
     static __device__ __forceinline__ T zero() { return 0.f; }
     static __device__ __forceinline__ float dot(const T &a, const T &b, float acc) {
         return __builtin_fmaf(a, b, acc);
     }
 };
-struct UnitBF16x8 {
+struct UnitBF16x8 : WholeUnits<uint4> {
     static constexpr int DT = DT_BF16;
-    using T = uint4;  // 8 bfloat16, two per 32-bit word, low half first
+    // 8 bfloat16, two per 32-bit word, low half first
     static constexpr int ELEMS = 8;
     static __device__ __forceinline__ T zero() { return make_uint4(0u, 0u, 0u, 0u); }
     static __device__ __forceinline__ float lo(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
@@ -167,9 +196,9 @@ struct UnitBF16x8 {
 };
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-struct UnitF16x8 {
+struct UnitF16x8 : WholeUnits<uint4> {
     static constexpr int DT = DT_F16;
-    using T = uint4;  // 8 IEEE half floats, two per 32-bit word, low half first
+    // 8 IEEE half floats, two per 32-bit word, low half first
     static constexpr int ELEMS = 8;
     static __device__ __forceinline__ T zero() { return make_uint4(0u, 0u, 0u, 0u); }
     // v_dot2c_f32_f16: acc + a.lo*b.lo + a.hi*b.hi with fp32 accumulation (products of

@@ -4,7 +4,7 @@
 // consecutive stored entries.  Lane l loads the column index / S value of entry
 // l of the chunk and finally stores its P value: plain coalesced 64-wide
 // accesses.  For the dot products the 64 lanes are cut into G = 64/LPN groups of
-// LPN lanes.  A row of K elements is KU units of 16 bytes; lane j of a group owns
+// LPN lanes.  A row of K elements is KU units of 16 bytes (device_utils.h); lane j of a group owns
 // units j, j+LPN, j+2*LPN, ... (UPL of them), so every load instruction has LPN
 // neighbouring lanes reading LPN*16 contiguous bytes of one row: at K=32 fp32,
 // LPN=8 and UPL=1, 8 lanes read one whole 128-byte B row (one cache line) per
@@ -38,6 +38,11 @@ __device__ __forceinline__ T load_at(const void *__restrict__ base, O byte_off) 
     return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + byte_off);
 }
 
+template <class U, class O>
+__device__ __forceinline__ typename U::T load_unit(const void *__restrict__ base, O byte_off) {
+    return U::load(reinterpret_cast<const char *>(base) + byte_off);
+}
+
 template <class O>
 __device__ __forceinline__ O shfl_off(O v, int src) {
     if constexpr (sizeof(O) == 4) return (O)__shfl((int)v, src, WAVE);
@@ -66,14 +71,19 @@ struct Chunk {
 
     struct Areg { T u[UPL]; };
 
-    static __device__ __forceinline__ bool unit_on(int j, int i, int KU) { return FULLK || (j + i * LPN) < KU; }
+    static __device__ __forceinline__ bool unit_on(int j, int i, int KU) { return FULLK || (j + i * LPN) < U::units(KU); }
+    // (the last unit of a row is among the upper half of a lane's units)
+    static __device__ __forceinline__ T trim(const T &v, int j, int i, int KU) {
+        if constexpr (U::WHOLE) return v;
+        else return 2 * i + 2 > UPL ? U::trim(v, j + i * LPN, KU) : v;
+    }
 
     static __device__ __forceinline__ Areg load_a(const void *__restrict__ A, O row_off, int j, int KU) {
         Areg a;
 #pragma unroll
         for (int i = 0; i < UPL; ++i) {
             const int u = unit_on(j, i, KU) ? j + i * LPN : 0;
-            a.u[i] = load_at<T, O>(A, row_off + (O)(u * (int)sizeof(T)));
+            a.u[i] = trim(load_unit<U, O>(A, row_off + (O)U::unit_off(u, KU)), j, i, KU);
         }
         return a;
     }
@@ -94,8 +104,8 @@ struct Chunk {
 #pragma unroll
             for (int i = 0; i < UPL; ++i) {
                 const int u = unit_on(j, i, KU) ? j + i * LPN : 0;
-                bf[s][i] = load_at<T, O>(B, bo + (O)(u * (int)sizeof(T)));
-                if constexpr (WITH_ROWS) af[s][i] = load_at<T, O>(A, ao + (O)(u * (int)sizeof(T)));
+                bf[s][i] = load_unit<U, O>(B, bo + (O)U::unit_off(u, KU));
+                if constexpr (WITH_ROWS) af[s][i] = load_unit<U, O>(A, ao + (O)U::unit_off(u, KU));
             }
         }
         after_issue();
@@ -105,8 +115,9 @@ struct Chunk {
 #pragma unroll
             for (int i = 0; i < UPL; ++i) {
                 float q;
-                if constexpr (WITH_ROWS) q = U::dot(af[s][i], bf[s][i], p);
-                else q = U::dot(a.u[i], bf[s][i], p);
+                const T b = trim(bf[s][i], j, i, KU);
+                if constexpr (WITH_ROWS) q = U::dot(trim(af[s][i], j, i, KU), b, p);
+                else q = U::dot(a.u[i], b, p);
                 p = unit_on(j, i, KU) ? q : p;
             }
             p = group_sum<LPN>(p);
@@ -142,17 +153,18 @@ struct Chunk {
 // K too long for the register layout (more than 64 units per row): one entry per
 // step, all 64 lanes stride over the row.
 template <class U>
-__device__ __forceinline__ float chunk_long(const typename U::T *__restrict__ A,
-                                            const typename U::T *__restrict__ B, int KU, int c, int r,
+__device__ __forceinline__ float chunk_long(const void *__restrict__ A, const void *__restrict__ B, int KU, int c, int r,
                                             int count, int lane) {
     float out = 0.f;
+    const int units = U::units(KU);
+    const uint64_t rb = U::row_bytes(KU);
     for (int t = 0; t < count; ++t) {
-        const int cc = __shfl(c, t, WAVE);
-        const int rr = __shfl(r, t, WAVE);
-        const typename U::T *__restrict__ Ar = A + (int64_t)rr * KU;
-        const typename U::T *__restrict__ Br = B + (int64_t)cc * KU;
+        const uint64_t bo = (uint64_t)(uint32_t)__shfl(c, t, WAVE) * rb, ao = (uint64_t)(uint32_t)__shfl(r, t, WAVE) * rb;
         float p = 0.f;
-        for (int u = lane; u < KU; u += WAVE) p = U::dot(Ar[u], Br[u], p);
+        for (int u = lane; u < units; u += WAVE) {
+            const uint64_t at = U::unit_off(u, KU);
+            p = U::dot(U::trim(load_unit<U, uint64_t>(A, ao + at), u, KU), U::trim(load_unit<U, uint64_t>(B, bo + at), u, KU), p);
+        }
         p = group_sum<WAVE>(p);
         if (lane == t) out = p;
     }
@@ -180,7 +192,6 @@ __global__ __launch_bounds__(BLOCK) void k_flat(const void *__restrict__ A, cons
                                                 float *__restrict__ P, int64_t nnz,
                                                 int chunks_per_wave, int64_t nblocks) {
     using U = typename L::U;
-    using T = typename U::T;
     const int64_t blk = xcd_remap(blockIdx.x, nblocks);
     if (blk < 0) return;
     const int lane = lane_id();
@@ -210,11 +221,11 @@ __global__ __launch_bounds__(BLOCK) void k_flat(const void *__restrict__ A, cons
         float res;
         if constexpr (L::LONG) {
             prefetch();
-            res = chunk_long<U>((const T *)A, (const T *)B, KU, c, r, count, lane);
+            res = chunk_long<U>(A, B, KU, c, r, count, lane);
         } else {
             using C = Chunk<U, L::LPN, L::UPL, L::FULLK, true, L::WIDE>;
             using O = typename C::O;
-            const O rb = (O)KU * (O)sizeof(T);
+            const O rb = (O)U::row_bytes(KU);
             typename C::Areg none;
             res = C::run(A, B, KU, none, (O)c * rb, (O)r * rb, count, lane, prefetch);
         }
@@ -233,7 +244,6 @@ __device__ __forceinline__ void row_segment_body(const void *__restrict__ A, con
                                                  const int32_t *__restrict__ col, const float *__restrict__ sval,
                                                  float *__restrict__ P, int row, int start, int end, int lane) {
     using U = typename L::U;
-    using T = typename U::T;
     if (start >= end) return;
     if constexpr (L::LONG) {
         for (int base = start; base < end; base += WAVE) {
@@ -242,13 +252,13 @@ __device__ __forceinline__ void row_segment_body(const void *__restrict__ A, con
             const int c = valid ? ld_stream(col + n) : 0;
             const float s = valid ? ld_stream(sval + n) : 0.f;
             const int left = end - base;
-            const float res = chunk_long<U>((const T *)A, (const T *)B, KU, c, row, left < WAVE ? left : WAVE, lane);
+            const float res = chunk_long<U>(A, B, KU, c, row, left < WAVE ? left : WAVE, lane);
             if (valid) st_stream(P + n, res * s);
         }
     } else {
         using C = Chunk<U, L::LPN, L::UPL, L::FULLK, false, L::WIDE>;
         using O = typename C::O;
-        const O rb = (O)KU * (O)sizeof(T);
+        const O rb = (O)U::row_bytes(KU);
         const typename C::Areg a = C::load_a(A, (O)row * rb, lane & (L::LPN - 1), KU);
         // Index loads are unconditional (clamped to the last entry of the range): lanes
         // past the end then hold a valid column whose result is never stored, and the
@@ -287,7 +297,6 @@ __device__ __forceinline__ void short_rows_body(const void *__restrict__ A, cons
                                                 const int32_t *__restrict__ col, const float *__restrict__ sval,
                                                 float *__restrict__ P, int M, int ts, int64_t r0, int rpw, int lane) {
     using U = typename L::U;
-    using T = typename U::T;
     int rs = 0, len = 0;
     if (lane < rpw && r0 + lane < M) {
         rs = rowptr[r0 + lane];
@@ -333,11 +342,11 @@ __device__ __forceinline__ void short_rows_body(const void *__restrict__ A, cons
         float res;
         if constexpr (L::LONG) {
             prefetch();
-            res = chunk_long<U>((const T *)A, (const T *)B, KU, c, row, count, lane);
+            res = chunk_long<U>(A, B, KU, c, row, count, lane);
         } else {
             using C = Chunk<U, L::LPN, L::UPL, L::FULLK, true, L::WIDE>;
             using O = typename C::O;
-            const O rb = (O)KU * (O)sizeof(T);
+            const O rb = (O)U::row_bytes(KU);
             typename C::Areg none;
             res = C::run(A, B, KU, none, (O)c * rb, (O)row * rb, count, lane, prefetch);
         }
@@ -357,7 +366,6 @@ __device__ __forceinline__ void entry_list_body(const void *__restrict__ A, cons
                                                 const int32_t *__restrict__ col, const float *__restrict__ sval,
                                                 float *__restrict__ P, int64_t chunk, int lane) {
     using U = typename L::U;
-    using T = typename U::T;
     const int64_t base = chunk * WAVE;
     if (base >= n_list) return;
     const int64_t left = n_list - base;
@@ -368,11 +376,11 @@ __device__ __forceinline__ void entry_list_body(const void *__restrict__ A, cons
     const float s = ld_stream(sval + pr.x);
     float res;
     if constexpr (L::LONG) {
-        res = chunk_long<U>((const T *)A, (const T *)B, KU, c, pr.y, count, lane);
+        res = chunk_long<U>(A, B, KU, c, pr.y, count, lane);
     } else {
         using C = Chunk<U, L::LPN, L::UPL, L::FULLK, true, L::WIDE>;
         using O = typename C::O;
-        const O rb = (O)KU * (O)sizeof(T);
+        const O rb = (O)U::row_bytes(KU);
         typename C::Areg none;
         res = C::run(A, B, KU, none, (O)c * rb, (O)pr.y * rb, count, lane, []() {});
     }
@@ -508,7 +516,7 @@ __global__ __launch_bounds__(BLOCK, SDDMM_PANEL_OCC) void k_panel(const void *__
     if (start >= end) return;
     const int lane = lane_id();
     const int g = lane >> 3, j = lane & 7;
-    const O rb = (O)KU * (O)sizeof(T);
+    const O rb = (O)U::row_bytes(KU);
     // units of the 8 A rows
     T a[PANEL_ROWS][UPL];
 #pragma unroll

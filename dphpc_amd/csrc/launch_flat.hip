@@ -11,7 +11,7 @@ void launch_flat(sddmm_ctx *c) {
     with_layout(s, [&](auto L) {
         using LT = decltype(L);
         SDDMM_LAUNCH(c, (k_flat<LT>), xcd_grid(nblocks), BLOCK,
-                           (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowidx, c->d_col, c->d_sval, c->dP,
+                           (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowidx, c->d_col, c->d_sval, c->dP,
                            c->nnz, cpw, nblocks);
     });
 }

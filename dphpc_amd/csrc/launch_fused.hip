@@ -17,7 +17,7 @@ int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
     int launches = 0;
     with_layout(s, [&](auto L) {
         using LT = decltype(L);
-        if constexpr (!LT::LONG && LT::LPN <= 8 && LT::U::ELEMS > 1 && LT::UPL * LT::U::ELEMS <= 32) {
+        if constexpr (!LT::LONG && LT::LPN <= 8 && LT::U::ELEMS > 1 && LT::U::WHOLE && LT::UPL * LT::U::ELEMS <= 32) {
             const int64_t rows_per_wave = WAVE / LT::LPN;
             const int64_t waves = ((int64_t)c->sM + rows_per_wave - 1) / rows_per_wave;
             const int64_t rblocks = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
@@ -25,18 +25,18 @@ int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
                 const int64_t bwaves = ((int64_t)c->sM + WAVE - 1) / WAVE;
                 const int64_t bblocks = (bwaves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
                 SDDMM_LAUNCH(c, (k_fusedmm_rows_balanced<LT>), xcd_grid(bblocks), BLOCK,
-                                   (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr, c->d_col, c->d_sval,
+                                   (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col, c->d_sval,
                                    c->dP, c->dO, c->sM, FUSED_ROW_MAX, bblocks, panel_owner);
             } else {
                 SDDMM_LAUNCH(c, (k_fusedmm_rows<LT>), xcd_grid(rblocks), BLOCK,
-                                   (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr, c->d_col, c->d_sval,
+                                   (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col, c->d_sval,
                                    c->dP, c->dO, c->sM, FUSED_ROW_MAX, rblocks, panel_owner);
             }
             ++launches;
             if (c->n_fused_items > 0) {
                 const int64_t nblocks = (c->n_fused_items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
                 SDDMM_LAUNCH(c, (k_fusedmm<LT>), xcd_grid(nblocks), BLOCK,
-                                   (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr, c->d_col,
+                                   (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col,
                                    c->d_sval, c->dP, c->dO, (const RowItem *)c->d_fused_items, c->n_fused_items,
                                    nblocks);
                 ++launches;

@@ -7,7 +7,7 @@ void launch_row_wave(sddmm_ctx *c, const RowItem *items, int64_t n_items) {
     with_layout(s, [&](auto L) {
         using LT = decltype(L);
         SDDMM_LAUNCH(c, (k_row_wave<LT>), xcd_grid(nblocks), BLOCK,
-                           (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr, c->d_col, c->d_sval, c->dP,
+                           (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col, c->d_sval, c->dP,
                            items, n_items, nblocks);
     });
 }
@@ -19,23 +19,7 @@ void launch_short_rows(sddmm_ctx *c, int ts, int rpw) {
     with_layout(s, [&](auto L) {
         using LT = decltype(L);
         SDDMM_LAUNCH(c, (k_short_rows<LT>), xcd_grid(nblocks), BLOCK,
-                           (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr, c->d_col, c->d_sval, c->dP,
+                           (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col, c->d_sval, c->dP,
                            c->sM, ts, rpw, nblocks);
-    });
-}
-
-void launch_auto(sddmm_ctx *c) {
-    const Shape s = shape_of(c);
-    const int64_t waves = short_row_waves(c);
-    const int64_t short_blocks = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    const int64_t item_blocks = (c->n_items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    const int64_t nblocks = short_blocks + item_blocks;
-    with_layout(s, [&](auto L) {
-        using LT = decltype(L);
-        SDDMM_LAUNCH(c, (k_auto<LT>), xcd_grid(nblocks), BLOCK,
-                           (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr,
-                           (const unsigned char *)(c->owner_active ? c->d_owner : nullptr), c->d_col, c->d_sval,
-                           c->dP, c->sM, c->ts, c->rpw, short_blocks, c->d_items, c->n_items, nblocks,
-                           (const int2 *)(c->use_short_list ? c->d_short_list : nullptr), c->n_short_list);
     });
 }

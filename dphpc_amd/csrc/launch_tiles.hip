@@ -7,7 +7,7 @@
 // kernel; the caller then launches the two kernels in turn.
 bool launch_auto_with_tiles(sddmm_ctx *c) {
     const Shape s = shape_of(c);
-    if (c->tile_steps < 1 || c->tile_steps > env_int("SDDMM_FUSE_STEPS", 16) || !s.fullk || s.wide || s.unit == 1 || s.KU != 4 * c->tile_steps)
+    if (c->tile_steps < 1 || c->tile_steps > env_int("SDDMM_FUSE_STEPS", 16) || !s.fullk || s.wide || !s.whole() || s.KU != 4 * c->tile_steps)
         return false;
     const int64_t waves = short_row_waves(c);
     const int64_t short_blocks = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
@@ -26,9 +26,9 @@ bool launch_auto_with_tiles(sddmm_ctx *c) {
     with_layout(s, [&](auto L) {
         using LT = decltype(L);
         constexpr int KU_ = LT::LPN * LT::UPL;
-        if constexpr (!LT::LONG && LT::FULLK && !LT::WIDE && LT::U::ELEMS > 1 && (KU_ == 4 || KU_ == 8 || KU_ == 16 || KU_ == 32 || KU_ == 64)) {
+        if constexpr (!LT::LONG && LT::FULLK && !LT::WIDE && LT::U::ELEMS > 1 && LT::U::WHOLE && (KU_ == 4 || KU_ == 8 || KU_ == 16 || KU_ == 32 || KU_ == 64)) {
             SDDMM_LAUNCH(c, (k_auto_tiles<LT, KU_ / 4>), grid, BLOCK,
-                               (const void *)c->dA, (const void *)c->dB, s.KU, c->d_rowptr,
+                               (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr,
                                (const unsigned char *)(c->owner_active ? c->d_owner : nullptr), c->d_col, c->d_sval,
                                c->dP, c->sM, c->N, c->ts, c->rpw, short_blocks, c->d_items, c->n_items,
                                (const int32_t *)c->d_vrows, (const int32_t *)c->d_tile_cols,

@@ -533,7 +533,7 @@ int plan_tiles_fill(sddmm_ctx *c) {
 
 bool panel_valu_applicable(const sddmm_ctx *c) {
     const Shape s = shape_of(c);
-    if (s.unit == 1 || s.LPN != 8 || !s.fullk || s.wide) return false;
+    if (!s.whole() || s.LPN != 8 || !s.fullk || s.wide) return false;
     return s.unit == 0 ? s.UPL <= 2 : s.UPL == 1;
 }
 
@@ -1223,7 +1223,7 @@ int sddmm_run_fused(sddmm_ctx *c) {
     if (rc) return rc;
     const Shape s = shape_of(c);
     // 16-byte units, at most 8 lanes per entry and 32 fp32 accumulators of the output row per lane
-    if (s.unit == 1 || s.LPN == 0 || s.LPN > 8 || c->K > 256)
+    if (!s.whole() || s.LPN == 0 || s.LPN > 8 || c->K > 256)
         return fail(c, SDDMM_ERR_UNSUPPORTED,
                     "the fused SDDMM+SpMM needs K <= 256, a multiple of 4 (fp32) or 8 (bf16, fp16)");
     if (!c->have_rowptr) return fail(c, SDDMM_ERR_UNSUPPORTED, "the fused SDDMM+SpMM needs row-sorted entries");

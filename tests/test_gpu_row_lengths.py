@@ -1,9 +1,12 @@
-"""The flat kernel in slices of K (rows of more than 128 bytes), forced on wherever it can run:
+"""Row lengths that are no power of two: the flat kernel in slices of K (rows of more than 128 bytes),
+forced on wherever it can run, and the gather kernels on rows of no whole number of 16-byte units:
 edges of lines, units, chunks and staged rows, against the oracle.  All GPU.
 
 Same bar as test_gpu_parity.py.  B and A rows without entries hold NaN: every lane that
 reads outside its entry's row (windows are moved down to lines) must leave the sum alone.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -137,3 +140,54 @@ def test_rows_beyond_the_register_layout_take_slices(engine_factory):
             e.run()
             assert e.stats().strategy_used == capi.FLAT and e.stats().kernels_launched == launches
             _check(e.values(), r, c, v, A, B, capi.STRATEGY_NAMES[strategy])
+
+
+@pytest.mark.parametrize("K", [5, 6, 7, 9, 17, 30, 35, 62, 65, 97, 127, 129, 161, 193, 255, 257, 510, 511])
+def test_rows_of_no_whole_number_of_units(engine_factory, monkeypatch, K):
+    """K % 4 != 0 in the gather kernels: the last unit of a row ends with the row and overlaps the one before."""
+    monkeypatch.setenv("SDDMM_SLICES", "0")
+    for seed, M, N, density in ((1, 60, 150, 0.6), (2, 700, 61, 0.04)):
+        r, c, v, A, B = _case(K + seed, M, N, K, capi.F32, density=density)
+        print("unaligned", K, M, N, len(r), flush=True)
+        rowptr, col, val = O.csr_from_triplets(M, r, c, v)
+        with engine_factory() as e:
+            e.set_dense(A, B)
+            for strategy in (capi.FLAT, capi.ROW_WAVE, capi.SHORT_ROWS, capi.AUTO):
+                e.set_csr(M, N, rowptr, col, val)         # clears P
+                e.plan(strategy)
+                e.run()
+                _check(e.values(), r, c, v, A, B, "K=%d %s" % (K, capi.STRATEGY_NAMES[strategy]))
+
+
+@pytest.mark.parametrize("slices", ["0", "1"])
+@pytest.mark.parametrize("K", [131, 132])
+def test_operand_beyond_4gib(engine_factory, monkeypatch, K, slices):
+    """64-bit row offsets, with rows of no whole number of units and with slices of K."""
+    monkeypatch.setenv("SDDMM_SLICES", slices)
+    M, N = 40, (1 << 32) // (4 * K) + 100
+    rng = np.random.default_rng(K)
+    hot = np.unique(np.concatenate([np.arange(30), np.arange(N - 130, N), rng.integers(0, N, 100)]))
+    B = rng.uniform(-1, 1, (len(hot), K)).astype(f32)
+    A = rng.uniform(-1, 1, (M, K)).astype(f32)
+    r, c = np.nonzero(rng.random((M, len(hot))) < 0.4)
+    r, c = r.astype(np.int32), c.astype(np.int32)
+    v = rng.uniform(-1, 1, len(r)).astype(f32)
+    rowptr, col, val = O.csr_from_triplets(M, r, c, v)    # columns among the rows that are filled in
+    print("wide", K, slices, "%.2f GiB" % (N * K * 4 / 2 ** 30), flush=True)
+    hip = Hip()
+    e = engine_factory()
+    try:
+        dA, dB = hip.upload(A), C.c_void_p()
+        assert hip.h.hipMalloc(C.byref(dB), N * K * 4) == 0
+        hip.live.append(dB)
+        for i, n in enumerate(hot):
+            assert hip.h.hipMemcpy(C.c_void_p(dB.value + int(n) * K * 4), B[i].ctypes.data_as(C.c_void_p), K * 4, 1) == 0
+        e._chk(e.L.sddmm_set_dense_device(e.h, M, N, K, dA, dB, capi.F32))
+        for strategy in (capi.AUTO, capi.FLAT, capi.ROW_WAVE):
+            e.set_csr(M, N, rowptr, hot[col].astype(np.int32), val)
+            e.plan(strategy)
+            e.run()
+            _check(e.values(), r, c, v, A, B, "K=%d %s" % (K, capi.STRATEGY_NAMES[strategy]))
+    finally:
+        e.close()
+        hip.free_all()
