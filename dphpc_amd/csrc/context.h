@@ -118,6 +118,14 @@ struct sddmm_ctx {
     float *d_part = nullptr;
     int64_t part_floats = 0;
     bool use_slices = false;         // set by a plan of SDDMM_AUTO
+    // FLAT with the long rows cut into column blocks (k_flat_blocks)
+    char *d_blocks = nullptr;        // one allocation: lists and scans of the plan, item counts, items
+    size_t blocks_bytes = 0;
+    RowItem *d_block_segments = nullptr, *d_block_gaps = nullptr;
+    unsigned long long *d_block_totals = nullptr;
+    int64_t block_segments_max = 0, block_gaps_max = 0;
+    bool use_blocks = false;         // set by a plan of SDDMM_AUTO
+    unsigned int *d_long_sums = nullptr;    // arena view: long rows per block of the row scan
     // fused SDDMM + SpMM: items covering every non-empty row, output M x K
     RowItem *d_fused_items = nullptr;
     int64_t n_fused_items = 0, fused_items_cap = 0;
@@ -292,6 +300,8 @@ inline int panel_mfma_steps(const sddmm_ctx *c) {
 
 // ---- launchers, one translation unit per family of kernels ----
 void launch_flat(sddmm_ctx *c);                                                  // launch_flat.hip
+void launch_flat_blocks(sddmm_ctx *c);
+bool blocks_pay(const sddmm_ctx *c);
 bool slices_pay(const sddmm_ctx *c, double entries_per_row);
 int64_t slice_workspace_floats(const sddmm_ctx *c);
 int launch_flat_sliced(sddmm_ctx *c);                                            // number of launches

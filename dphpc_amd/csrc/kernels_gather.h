@@ -184,22 +184,13 @@ struct Layout {
 // row array, or the expansion of rowptr built by the plan).  Perfectly balanced
 // whatever the row lengths are; A units are gathered per entry like B units
 // (L1/L2 hits while the row does not change).
+// entries [base, stop) on the calling wavefront
 template <class L>
-__global__ __launch_bounds__(BLOCK) void k_flat(const void *__restrict__ A, const void *__restrict__ B, int KU,
-                                                const int32_t *__restrict__ rowidx,
-                                                const int32_t *__restrict__ col,
-                                                const float *__restrict__ sval,
-                                                float *__restrict__ P, int64_t nnz,
-                                                int chunks_per_wave, int64_t nblocks) {
+__device__ __forceinline__ void flat_body(const void *__restrict__ A, const void *__restrict__ B, int KU,
+                                          const int32_t *__restrict__ rowidx, const int32_t *__restrict__ col,
+                                          const float *__restrict__ sval, float *__restrict__ P, int64_t base,
+                                          int64_t stop, int lane) {
     using U = typename L::U;
-    const int64_t blk = xcd_remap(blockIdx.x, nblocks);
-    if (blk < 0) return;
-    const int lane = lane_id();
-    const int64_t wave = blk * WAVES_PER_BLOCK + wave_in_block();
-    int64_t base = wave * (int64_t)chunks_per_wave * WAVE;
-    if (base >= nnz) return;
-    int64_t stop = base + (int64_t)chunks_per_wave * WAVE;
-    stop = stop < nnz ? stop : nnz;
     // Index loads are unconditional (clamped to the last entry of the range): lanes
     // past the end then hold a valid row/column whose result is never stored, and
     // the loads need no branch, which keeps the wait counts of the gathers exact.
@@ -232,6 +223,21 @@ __global__ __launch_bounds__(BLOCK) void k_flat(const void *__restrict__ A, cons
         if (valid) st_stream(P + n, res * s);
         c = cn; r = rn; s = sn;
     }
+}
+
+template <class L>
+__global__ __launch_bounds__(BLOCK) void k_flat(const void *__restrict__ A, const void *__restrict__ B, int KU,
+                                                const int32_t *__restrict__ rowidx,
+                                                const int32_t *__restrict__ col,
+                                                const float *__restrict__ sval,
+                                                float *__restrict__ P, int64_t nnz,
+                                                int chunks_per_wave, int64_t nblocks) {
+    const int64_t blk = xcd_remap(blockIdx.x, nblocks);
+    if (blk < 0) return;
+    const int64_t base = (blk * WAVES_PER_BLOCK + wave_in_block()) * (int64_t)chunks_per_wave * WAVE;
+    if (base >= nnz) return;
+    const int64_t stop = base + (int64_t)chunks_per_wave * WAVE;
+    flat_body<L>(A, B, KU, rowidx, col, sval, P, base, stop < nnz ? stop : nnz, lane_id());
 }
 
 // ---------------------------------------------------------------------------
@@ -385,6 +391,44 @@ __device__ __forceinline__ void entry_list_body(const void *__restrict__ A, cons
         res = C::run(A, B, KU, none, (O)c * rb, (O)pr.y * rb, count, lane, []() {});
     }
     if (valid) st_stream(P + pr.x, res * s);
+}
+
+// ---------------------------------------------------------------------------
+// FLAT with the long rows cut into column blocks.  The lines of B that a flat launch gathers come from
+// the last-level cache (7.3 TB/s, the bound on a graph: 633 us for 36 M entries over 333 MB of B), since
+// every XCD touches all of B.  Much of a power-law graph lies in rows of hundreds of entries: their
+// segments of one column block each are taken block by block, an XCD two of the COL_BLOCKS blocks, so
+// that its L2 sees an eighth of B from them (two thirds of the entries: 518 us).  A segment is a work
+// item of one row, its A row stays in registers.  The entries between the long rows are taken 64 at a
+// time in storage order (64: 524 us, 256: 538, 512: 541), after the segments on every XCD (before
+// them: the same; dealt out evenly: 542 us).
+// totals[0], totals[1]: work items of either kind (the grid is sized for an upper bound)
+template <class L>
+__global__ __launch_bounds__(BLOCK) void k_flat_blocks(const void *__restrict__ A, const void *__restrict__ B, int KU,
+                                                       const int32_t *__restrict__ rowidx,
+                                                       const int32_t *__restrict__ col,
+                                                       const float *__restrict__ sval, float *__restrict__ P,
+                                                       const RowItem *__restrict__ segments,
+                                                       const RowItem *__restrict__ gaps,
+                                                       const unsigned long long *__restrict__ totals) {
+    const int64_t n_seg = (int64_t)totals[0], n_gap = (int64_t)totals[1];
+    const int64_t sb = (n_seg + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK, gb = (n_gap + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+    // every XCD its contiguous eighth of each kind
+    const int x = (int)(blockIdx.x % NUM_XCD);
+    int64_t j = blockIdx.x / NUM_XCD;
+    const int64_t s_lo = x * sb / NUM_XCD, s_n = (x + 1) * sb / NUM_XCD - s_lo;
+    const int64_t g_lo = x * gb / NUM_XCD, g_n = (x + 1) * gb / NUM_XCD - g_lo;
+    const bool segment = j < s_n;
+    if (!segment) j -= s_n;
+    if (!segment && j >= g_n) return;
+    const int64_t w = (segment ? s_lo + j : g_lo + j) * WAVES_PER_BLOCK + wave_in_block();
+    if (w >= (segment ? n_seg : n_gap)) return;
+    const RowItem it = segment ? segments[w] : gaps[w];
+    const int row = __builtin_amdgcn_readfirstlane(it.row);
+    const int start = __builtin_amdgcn_readfirstlane(it.start);
+    const int end = __builtin_amdgcn_readfirstlane(it.end);
+    if (segment) row_segment_body<L>(A, B, KU, col, sval, P, row, start, end, lane_id());
+    else flat_body<L>(A, B, KU, rowidx, col, sval, P, start, end, lane_id());
 }
 
 // ---------------------------------------------------------------------------

@@ -36,6 +36,7 @@ struct DevCounters {
     unsigned long long n_items, tiles_scanned, panel_items;          // scan totals, one writer each
     unsigned long long n_candidates;                                 // rows offered to the gathered strips
     unsigned long long utiles_scanned, short_scanned;                // scan totals: union strips, entries of the short rows
+    unsigned long long long_scanned;                                 // scan total: rows of more than one item
     unsigned int max_len[SPREAD];
     unsigned long long k[K_KINDS][SPREAD];
 };
@@ -95,6 +96,7 @@ static __global__ __launch_bounds__(256) void k_plan_reset(unsigned char *__rest
         if (threadIdx.x == 0) {
             pc->n_items = 0ull;
             pc->short_scanned = 0ull;
+            pc->long_scanned = 0ull;
             if (!rows_only) {
                 pc->tiles_scanned = 0ull; pc->panel_items = 0ull; pc->n_candidates = 0ull; pc->utiles_scanned = 0ull;
             }
@@ -254,7 +256,8 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int3
                                                                const unsigned char *__restrict__ owner, int M,
                                                                int ts, int seg, unsigned int *__restrict__ block_sums,
                                                                DevCounters *pc, int only,
-                                                               unsigned int *__restrict__ short_sums) {
+                                                               unsigned int *__restrict__ short_sums,
+                                                               unsigned int *__restrict__ long_sums) {
     const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
     unsigned int items = 0;
     unsigned long long r_short = 0, r_med = 0, r_long = 0, n_short = 0, n_med = 0, n_long = 0;
@@ -288,6 +291,8 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int3
     if (threadIdx.x < 6) spread_add(pc, K_ROWS_SHORT + (int)threadIdx.x, sh[threadIdx.x]);
     // entries of this block's short rows, for the entry list (k_short_list_write)
     if (short_sums && threadIdx.x == 0) short_sums[blockIdx.x] = (unsigned int)sh[3];
+    // and its rows of more than one item, for the list of the long rows (k_long_rows)
+    if (long_sums && threadIdx.x == 0) long_sums[blockIdx.x] = (unsigned int)sh[2];
 }
 
 // pass 2: exclusive scan of the block sums in place (one workgroup), total -> *total_out
@@ -490,6 +495,106 @@ static __global__ __launch_bounds__(256) void k_panel_items(const int32_t *__res
         // start reading the column list without first waiting for a row pointer
         items[at++] = RowItem{row0, a, b, rs0};
     }
+}
+
+// ---------------------------------------------------------------------------
+// Column blocks for the long rows of a flat matrix (kernels_flat.h, k_flat_blocks).
+//
+// Rows of more than `seg` entries, in row order (block_offsets: exclusive scan of the long_sums of
+// k_classify_count).
+static __global__ __launch_bounds__(SCAN_BLOCK) void k_long_rows(const int32_t *__restrict__ rowptr, int M, int seg,
+                                                                 const unsigned int *__restrict__ block_offsets,
+                                                                 int32_t *__restrict__ long_rows) {
+    const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
+    unsigned int mine = 0, is_long = 0;
+    for (int q = 0; q < SCAN_ITEMS; ++q) {
+        const int64_t i = base + q;
+        const bool l = i < M && rowptr[i + 1] - rowptr[i] > seg;
+        is_long |= (l ? 1u : 0u) << q;
+        mine += l ? 1u : 0u;
+    }
+    unsigned int total;
+    unsigned int at = block_offsets[blockIdx.x] + block_exclusive_scan(mine, &total);
+    for (int q = 0; q < SCAN_ITEMS; ++q)
+        if ((is_long >> q) & 1u) long_rows[at++] = (int32_t)(base + q);
+}
+
+// 16 lanes per long row: lane b finds where the row's columns of block b start (columns ascend inside a
+// row: its entries of a block are consecutive; in a row that is not sorted the cuts fall anywhere, every
+// entry still lands in exactly one segment).  Segment (b, i): block b of long row i, block-major.
+constexpr int COL_BLOCKS = 16;
+static __global__ __launch_bounds__(256) void k_long_segments(const int32_t *__restrict__ rowptr,
+                                                              const int32_t *__restrict__ col, int N,
+                                                              const int32_t *__restrict__ long_rows, int n_long, int piece,
+                                                              int32_t *__restrict__ seg_start,
+                                                              unsigned int *__restrict__ seg_items) {
+    const int64_t slot = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = (int)(slot / COL_BLOCKS), b = (int)(slot % COL_BLOCKS);
+    const bool on = i < n_long;
+    int lo = 0, end = 0;
+    if (on) {
+        const int row = long_rows[i];
+        lo = rowptr[row];
+        end = rowptr[row + 1];
+        const int first = (int)((int64_t)N * b / COL_BLOCKS);
+        int hi = end;
+        if (b == 0) hi = lo;
+        while (lo < hi) {
+            const int mid = lo + ((hi - lo) >> 1);
+            if (col[mid] < first) lo = mid + 1; else hi = mid;
+        }
+    }
+    // the cuts of a row must ascend whatever its columns do: running maximum over the 16 lanes
+#pragma unroll
+    for (int o = 1; o < COL_BLOCKS; o <<= 1) {
+        const int up = __shfl_up(lo, o, WAVE);
+        if (b >= o) lo = up > lo ? up : lo;
+    }
+    int next = __shfl_down(lo, 1, WAVE);
+    if (b == COL_BLOCKS - 1) next = end;
+    if (!on) return;
+    const int len = next - lo;
+    seg_start[(int64_t)b * n_long + i] = lo;
+    seg_items[(int64_t)b * n_long + i] = (unsigned int)((len + piece - 1) / piece);
+}
+
+// the entries between long rows: gap i lies before long row i, the last one after all of them
+static __global__ __launch_bounds__(256) void k_long_gaps(const int32_t *__restrict__ rowptr,
+                                                          const int32_t *__restrict__ long_rows, int n_long, int nnz,
+                                                          int piece, int32_t *__restrict__ gap_start,
+                                                          unsigned int *__restrict__ gap_items) {
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (i > n_long) return;
+    const int start = i == 0 ? 0 : rowptr[long_rows[i - 1] + 1];
+    const int end = i == n_long ? nnz : rowptr[long_rows[i]];
+    gap_start[i] = start;
+    gap_items[i] = (unsigned int)((end - start + piece - 1) / piece);
+}
+
+// One thread per work item: its range by bisection over the exclusive scan of the ranges' item counts.
+// Ranges are the segments of the long rows or the gaps between those rows (items of no row).
+static __global__ __launch_bounds__(256) void k_range_items(const int32_t *__restrict__ rowptr,
+                                                            const int32_t *__restrict__ long_rows, int n_long, int nnz,
+                                                            int gaps, int piece, const int32_t *__restrict__ start,
+                                                            const unsigned int *__restrict__ offsets, int n_ranges,
+                                                            const unsigned long long *__restrict__ total,
+                                                            RowItem *__restrict__ items) {
+    const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (w >= (int64_t)*total) return;
+    int lo = 0, hi = n_ranges;                              // last range whose offset does not exceed w
+    while (hi - lo > 1) {
+        const int mid = lo + ((hi - lo) >> 1);
+        if ((int64_t)offsets[mid] <= w) lo = mid; else hi = mid;
+    }
+    int row = -1, end;
+    if (gaps) {
+        end = lo == n_long ? nnz : rowptr[long_rows[lo]];
+    } else {
+        row = long_rows[lo % n_long];
+        end = lo + n_long < n_ranges ? start[lo + n_long] : rowptr[row + 1];
+    }
+    const int a = start[lo] + (int)(w - (int64_t)offsets[lo]) * piece;
+    items[w] = RowItem{row, a, a + piece < end ? a + piece : end, 0};
 }
 
 }  // namespace sddmm

@@ -16,6 +16,35 @@ void launch_flat(sddmm_ctx *c) {
     });
 }
 
+void launch_flat_blocks(sddmm_ctx *c) {
+    const Shape s = shape_of(c);
+    auto eighth = [](int64_t items) {                      // workgroups per XCD, rounded up twice
+        const int64_t blocks = (items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+        return (blocks + NUM_XCD - 1) / NUM_XCD;
+    };
+    const int64_t grid = NUM_XCD * (eighth(c->block_segments_max) + eighth(c->block_gaps_max));
+    with_layout(s, [&](auto L) {
+        using LT = decltype(L);
+        if constexpr (!LT::LONG)
+            SDDMM_LAUNCH(c, (k_flat_blocks<LT>), grid, BLOCK, (const void *)c->dA, (const void *)c->dB, s.len,
+                         (const int32_t *)c->d_rowidx, (const int32_t *)c->d_col, (const float *)c->d_sval, c->dP,
+                         (const RowItem *)c->d_block_segments, (const RowItem *)c->d_block_gaps,
+                         (const unsigned long long *)c->d_block_totals);
+    });
+}
+
+// Measured on power-law graphs (rows of Zipf lengths, half to two thirds of the entries in rows of more than 256) of
+// 20 000 to 2.6 M vertices, K = 16 .. 250: 1.1 .. 1.4 times k_flat from 12 MB of B on; where B nearly fits the L2s
+// (60 000 vertices, 128-byte rows, 7.7 MB: 0.81 times) or the launch is short (500 k entries over 25 MB: 0.97) the
+// extra wavefronts cost more than the lines they save.
+bool blocks_pay(const sddmm_ctx *c) {
+    const int mode = env_int("SDDMM_COLUMN_BLOCKS", -1);            // -1: decide here, 0: never, 1: wherever there are long rows
+    if (shape_of(c).LPN == 0 || c->pc.rows_long == 0) return false;
+    if (mode >= 0) return mode != 0;
+    const double b_bytes = (double)c->N * (double)c->K * (double)elem_size(c->dtype);
+    return b_bytes >= 12.0 * (1 << 20) && c->nnz >= (1 << 20) && (double)c->pc.nnz_long >= 0.25 * (double)c->nnz;
+}
+
 namespace {
 
 constexpr int64_t SLICE_WORKSPACE = (int64_t)1 << 26;      // floats: the partial products stay in the last-level cache

@@ -23,7 +23,7 @@ void release_arena(sddmm_ctx *c) {
     c->d_panel_counts = c->d_panel_off = c->d_vstrip_ntiles = c->d_vstrip_off = nullptr;
     c->d_cand_keys = c->d_sorted_keys = nullptr;
     c->d_vrows = nullptr;
-    c->d_block_sums = c->d_short_sums = nullptr;
+    c->d_block_sums = c->d_short_sums = c->d_long_sums = nullptr;
     c->owner_cap = c->strips_cap = c->ustrips_cap = c->panels_cap = c->cand_cap = c->vstrips_cap = 0;
     c->block_sums_cap = 0;
 }
@@ -32,7 +32,7 @@ int ensure_arena(sddmm_ctx *c) {
     const int64_t M = c->sM;
     if (c->d_arena && c->arena_rows == M) return SDDMM_OK;
     release_arena(c);
-    const int64_t n_strips = (M + 15) / 16, n_panels = M / 8 + 1, n_sums = M / 1024 + 2;
+    const int64_t n_strips = (M + 15) / 16, n_panels = M / 8 + 1, n_sums = M / 256 + 8;
     size_t at = 0;
     auto take = [&](size_t bytes) {
         const size_t here = at;
@@ -47,7 +47,7 @@ int ensure_arena(sddmm_ctx *c) {
     const size_t o_vrows = take((size_t)(n_strips + 2) * 16 * 4);
     const size_t o_panel_n = take((size_t)n_panels * 4), o_panel_o = take((size_t)n_panels * 4);
     const size_t o_keys = take((size_t)(M + 1) * 8), o_sorted = take((size_t)(M + 1) * 8);
-    const size_t o_sums = take((size_t)n_sums * 4), o_short_sums = take((size_t)n_sums * 4);
+    const size_t o_sums = take((size_t)n_sums * 4), o_short_sums = take((size_t)n_sums * 4), o_long_sums = take((size_t)n_sums * 4);
     ALLOC_TRY(c, c->d_arena, at);
     char *b = c->d_arena;
     c->d_owner = (unsigned char *)(b + o_owner);
@@ -59,6 +59,7 @@ int ensure_arena(sddmm_ctx *c) {
     c->d_cand_keys = (unsigned long long *)(b + o_keys); c->d_sorted_keys = (unsigned long long *)(b + o_sorted);
     c->d_block_sums = (unsigned int *)(b + o_sums);
     c->d_short_sums = (unsigned int *)(b + o_short_sums);
+    c->d_long_sums = (unsigned int *)(b + o_long_sums);
     c->owner_cap = M + 64;
     c->strips_cap = c->ustrips_cap = n_strips;
     c->vstrips_cap = n_strips + 2;
@@ -185,25 +186,29 @@ int classify_rows_count(sddmm_ctx *c, bool again = false) {
     if (nb > 0) {
         const unsigned char *owner = c->owner_active ? c->d_owner : nullptr;
         SDDMM_LAUNCH(c, k_classify_count, nb, SCAN_BLOCK, c->d_rowptr, owner,
-                           c->sM, c->ts, c->seg, c->d_block_sums, c->d_pc, 0, c->d_short_sums);
+                           c->sM, c->ts, c->seg, c->d_block_sums, c->d_pc, 0, c->d_short_sums, c->d_long_sums);
         LAUNCH_CHECK(c);
         if (nb <= SCAN_SMALL_MAX) {
             int rc = queue_scan(c, c->d_block_sums, c->d_block_sums, nb, &c->d_pc->n_items);
             if (rc) return rc;
             rc = queue_scan(c, c->d_short_sums, c->d_short_sums, nb, &c->d_pc->short_scanned);
             if (rc) return rc;
+            rc = queue_scan(c, c->d_long_sums, c->d_long_sums, nb, &c->d_pc->long_scanned);
+            if (rc) return rc;
         } else {
             SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, c->d_block_sums, (int)nb,
                                &c->d_pc->n_items);
             SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, c->d_short_sums, (int)nb,
                                &c->d_pc->short_scanned);
+            SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, c->d_long_sums, (int)nb,
+                               &c->d_pc->long_scanned);
             LAUNCH_CHECK(c);
         }
     }
     return SDDMM_OK;
 }
 // ... and the items, once the counters are on the host (nothing may use the block sums in between)
-int classify_rows_items(sddmm_ctx *c, bool with_short_list = true) {
+int classify_rows_items(sddmm_ctx *c) {
     const int64_t nb = ((int64_t)c->sM + SCAN_TILE - 1) / SCAN_TILE;
     c->n_items = (int64_t)c->pc.n_items;
     c->rows_short = (int64_t)c->pc.rows_short;
@@ -222,7 +227,7 @@ int classify_rows_items(sddmm_ctx *c, bool with_short_list = true) {
     }
     // the entries of the short rows as a list, taken 64 at a time (entry_list_body)
     c->n_short_list = 0;
-    c->use_short_list = with_short_list && env_int("SDDMM_SHORT_LIST", 1) != 0 && c->rows_short > 0;
+    c->use_short_list = env_int("SDDMM_SHORT_LIST", 1) != 0 && c->rows_short > 0;
     if (c->use_short_list) {
         c->n_short_list = (int64_t)c->pc.nnz_short;
         if ((int64_t)c->raw.short_scanned != c->n_short_list)
@@ -584,6 +589,69 @@ int ensure_rowidx(sddmm_ctx *c) {
     return SDDMM_OK;
 }
 
+// Work items of k_flat_blocks: the segments of the long rows (more than `seg` entries) block by block, and
+// the entries between those rows.  Nothing is read back: the arrays are sized for the most items there
+// can be, the launch reads the true numbers.  Leaves use_blocks false when the device has no room.
+int plan_blocks(sddmm_ctx *c) {
+    const int64_t n_long = (int64_t)c->pc.rows_long, nb = ((int64_t)c->sM + SCAN_TILE - 1) / SCAN_TILE;
+    if ((int64_t)c->raw.long_scanned != n_long)
+        return fail(c, SDDMM_ERR_HIP, "internal: scan of the long rows disagrees with their number");
+    const int64_t n_seg = n_long * COL_BLOCKS, n_gap = n_long + 1;
+    const int64_t piece = c->seg, gap_piece = WAVE;
+    c->block_segments_max = (int64_t)c->pc.nnz_long / piece + n_seg;
+    c->block_gaps_max = (c->nnz - (int64_t)c->pc.nnz_long) / gap_piece + n_gap;
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        const size_t here = at;
+        at += (bytes + 255) & ~(size_t)255;
+        return here;
+    };
+    const size_t o_totals = take(16), o_rows = take((size_t)n_long * 4);
+    const size_t o_seg[3] = {take((size_t)n_seg * 4), take((size_t)n_seg * 4), take((size_t)n_seg * 4)};
+    const size_t o_gap[3] = {take((size_t)n_gap * 4), take((size_t)n_gap * 4), take((size_t)n_gap * 4)};
+    const size_t o_segments = take((size_t)c->block_segments_max * sizeof(RowItem));
+    const size_t o_gaps = take((size_t)c->block_gaps_max * sizeof(RowItem));
+    if (at > c->blocks_bytes) {
+        dfree(c->d_blocks);
+        c->blocks_bytes = 0;
+        void *p = nullptr;
+        if (hipMalloc(&p, at) != hipSuccess || !p) {
+            (void)hipGetLastError();                       // the failed allocation is not an error of the plan
+            return SDDMM_OK;
+        }
+        c->d_blocks = static_cast<char *>(p);
+        c->blocks_bytes = at;
+    }
+    char *b = c->d_blocks;
+    c->d_block_totals = (unsigned long long *)(b + o_totals);
+    c->d_block_segments = (RowItem *)(b + o_segments);
+    c->d_block_gaps = (RowItem *)(b + o_gaps);
+    int32_t *rows = (int32_t *)(b + o_rows), *seg_start = (int32_t *)(b + o_seg[0]), *gap_start = (int32_t *)(b + o_gap[0]);
+    unsigned int *seg_items = (unsigned int *)(b + o_seg[1]), *seg_off = (unsigned int *)(b + o_seg[2]);
+    unsigned int *gap_items = (unsigned int *)(b + o_gap[1]), *gap_off = (unsigned int *)(b + o_gap[2]);
+    SDDMM_LAUNCH(c, k_long_rows, nb, SCAN_BLOCK, c->d_rowptr, c->sM, c->seg, (const unsigned int *)c->d_long_sums, rows);
+    SDDMM_LAUNCH(c, k_long_segments, grid_for(n_seg, 256), 256, c->d_rowptr, c->d_col, c->sN, (const int32_t *)rows,
+                 (int)n_long, (int)piece, seg_start, seg_items);
+    SDDMM_LAUNCH(c, k_long_gaps, grid_for(n_gap, 256), 256, c->d_rowptr, (const int32_t *)rows, (int)n_long, (int)c->nnz,
+                 (int)gap_piece, gap_start, gap_items);
+    LAUNCH_CHECK(c);
+    int rc = device_scan(c, seg_items, seg_off, n_seg, c->d_block_totals);
+    if (rc) return rc;
+    rc = device_scan(c, gap_items, gap_off, n_gap, c->d_block_totals + 1);
+    if (rc) return rc;
+    rc = flush_scans(c);
+    if (rc) return rc;
+    SDDMM_LAUNCH(c, k_range_items, grid_for(c->block_segments_max, 256), 256, c->d_rowptr, (const int32_t *)rows, (int)n_long,
+                 (int)c->nnz, 0, (int)piece, (const int32_t *)seg_start, (const unsigned int *)seg_off, (int)n_seg,
+                 (const unsigned long long *)c->d_block_totals, c->d_block_segments);
+    SDDMM_LAUNCH(c, k_range_items, grid_for(c->block_gaps_max, 256), 256, c->d_rowptr, (const int32_t *)rows, (int)n_long,
+                 (int)c->nnz, 1, (int)gap_piece, (const int32_t *)gap_start, (const unsigned int *)gap_off, (int)n_gap,
+                 (const unsigned long long *)(c->d_block_totals + 1), c->d_block_gaps);
+    LAUNCH_CHECK(c);
+    c->use_blocks = true;
+    return SDDMM_OK;
+}
+
 // Room for the partial products of the slices of K; false when the device does not have it (the launch
 // then takes the plain flat kernel).  Kept until the context goes.
 bool ensure_slice_workspace(sddmm_ctx *c) {
@@ -655,6 +723,7 @@ int enqueue_run(sddmm_ctx *c) {
         }
         case SDDMM_FLAT:
             if (c->use_slices) c->launches = launch_flat_sliced(c);
+            else if (c->use_blocks) launch_flat_blocks(c);
             else launch_flat(c);
             break;
         case SDDMM_ROW_WAVE: launch_row_wave(c, nullptr, c->sM); break;
@@ -684,7 +753,7 @@ int do_plan(sddmm_ctx *c, int strategy) {
     // previous one looking valid (its items exclude rows that tiles and panels owned)
     c->planned = false;
     c->n_scan_jobs = 0;
-    c->use_slices = false;
+    c->use_slices = c->use_blocks = false;
     c->fused_items_valid = false;    // they leave out the rows of this plan's panels
     int resolved = strategy;
     const bool csr_ok = c->have_rowptr;
@@ -775,13 +844,20 @@ int do_plan(sddmm_ctx *c, int strategy) {
             const bool only_rows = resolved == SDDMM_AUTO && c->n_tiles == 0 && c->n_panel_items == 0;
             const bool sliced = only_rows && slices_pay(c, avg_len) && ensure_slice_workspace(c);
             const bool flat = only_rows && (sliced || avg_len < (double)env_int("SDDMM_FLAT_AVG", 32));
-            rc = classify_rows_items(c, !flat);      // (the flat kernel has no use for the entry list of the short rows)
-            if (rc) return rc;
-            if (flat) {
+            if (flat) {                              // (which has no use for items, or for the entry list of the short rows)
+                c->n_items = c->n_short_list = c->rows_short = 0;
+                c->use_short_list = false;
                 rc = ensure_rowidx(c);
                 if (rc) return rc;
                 resolved = SDDMM_FLAT;
                 c->use_slices = sliced;
+                if (!sliced && blocks_pay(c)) {
+                    rc = plan_blocks(c);
+                    if (rc) return rc;
+                }
+            } else {
+                rc = classify_rows_items(c);
+                if (rc) return rc;
             }
             break;
         }
@@ -898,6 +974,7 @@ void sddmm_destroy(sddmm_ctx *c) {
     release_sparse(c);
     dfree(c->dO);
     dfree(c->d_part);
+    dfree(c->d_blocks);
     dfree(c->d_pc);
     if (c->h_pc) (void)hipHostFree(c->h_pc);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
@@ -1171,7 +1248,7 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
             HIP_TRY(c, hipMemsetAsync(&c->d_pc->n_items, 0, sizeof(unsigned long long), c->stream));
             SDDMM_LAUNCH(c, k_classify_count, nb, SCAN_BLOCK, c->d_rowptr,
                                panel_owner, c->sM, FUSED_ROW_MAX + 1, seg, c->d_block_sums, c->d_pc, 2,
-                               (unsigned int *)nullptr);
+                               (unsigned int *)nullptr, (unsigned int *)nullptr);
             SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, c->d_block_sums, (int)nb,
                                &c->d_pc->n_items);
             LAUNCH_CHECK(c);

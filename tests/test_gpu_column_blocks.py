@@ -1,0 +1,72 @@
+"""The flat kernel with the long rows cut into column blocks, forced on (small matrices): row lengths around
+the length that makes a row long, around whole pieces, long rows at either end and next to each other,
+columns in one block only, unsorted rows; against the oracle.  All GPU.  Same bar as test_gpu_parity.py."""
+import numpy as np
+import pytest
+
+from dphpc_amd import capi
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+f32 = np.float32
+
+
+def _check(e, M, N, rowptr, col, val, A, B, dtype, what):
+    e.set_dense(A if dtype == capi.F32 else capi.to_f16(A), B if dtype == capi.F32 else capi.to_f16(B), dtype)
+    e.set_csr(M, N, rowptr, col, val)
+    e.plan(capi.AUTO)
+    assert e.stats().strategy_used == capi.FLAT, what
+    e.run()
+    ref = O.sddmm_csr(rowptr, col, val, A, B, threads=0)
+    _, mag = O.sddmm_csr_f64(rowptr, col, val, A, B)
+    got = e.values()
+    ok, worst, i = O.check_values(got, ref, mag=mag)
+    assert ok, "%s: entry %d got %r ref %r (%.2f x tolerance)" % (what, i, got[i], ref[i], worst)
+    # the same arithmetic per entry as the plain flat kernel
+    e.set_csr(M, N, rowptr, col, val)
+    e.plan(capi.FLAT)
+    e.run()
+    np.testing.assert_array_equal(e.values(), got)
+
+
+def _matrix(rng, lens, N, kind="spread"):
+    M = len(lens)
+    cols = []
+    for l in lens:
+        if kind == "one block":
+            c = np.sort(rng.choice(N // 16, size=min(int(l), N // 16), replace=False)) + N // 16 * 5
+        else:
+            c = np.sort(rng.choice(N, size=int(l), replace=False))
+        if kind == "unsorted":
+            c = rng.permutation(c)
+        cols.append(c)
+    rowptr = np.concatenate([[0], np.cumsum([len(c) for c in cols])]).astype(np.int32)
+    return M, rowptr, np.concatenate(cols).astype(np.int32), rng.uniform(-1, 1, rowptr[-1]).astype(f32)
+
+
+@pytest.mark.parametrize("K,dtype", [(7, capi.F32), (32, capi.F32), (64, capi.F16), (100, capi.F32)])
+@pytest.mark.parametrize("kind", ["spread", "one block", "unsorted"])
+def test_column_blocks(engine_factory, monkeypatch, K, dtype, kind):
+    monkeypatch.setenv("SDDMM_COLUMN_BLOCKS", "1")
+    monkeypatch.setenv("SDDMM_SLICES", "0")
+    N = 8 * 16 * 300 if kind == "one block" else 7001
+    rng = np.random.default_rng(K)
+    short = rng.integers(0, 9, 3000)
+    patterns = {
+        "edges": np.concatenate([[257, 256, 255], short[:1500], [512, 513, 4096, 1000], short[1500:], [300]]),
+        "one long row": np.concatenate([short, [2000]]),
+        "only at the start": np.concatenate([[258], short]),
+        "scattered": np.concatenate([np.append(short[k * 60:(k + 1) * 60], 257 + 13 * k) for k in range(40)]),
+    }
+    A_all = rng.uniform(-1, 1, (4000, K)).astype(f32)
+    B = rng.uniform(-1, 1, (N, K)).astype(f32)
+    if dtype == capi.F16:
+        A_all, B = capi.from_f16(capi.to_f16(A_all)), capi.from_f16(capi.to_f16(B))
+    with engine_factory() as e:
+        for name, lens in patterns.items():
+            print("blocks", K, kind, name, flush=True)
+            M, rowptr, col, val = _matrix(rng, lens, N, kind)
+            _check(e, M, N, rowptr, col, val, A_all[:M], B, dtype, "%s %s K=%d" % (kind, name, K))
+        # a pattern without a long row after one with: the plain kernel again
+        M, rowptr, col, val = _matrix(rng, short, N, kind)
+        _check(e, M, N, rowptr, col, val, A_all[:M], B, dtype, "no long row")
