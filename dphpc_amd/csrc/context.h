@@ -126,6 +126,14 @@ struct sddmm_ctx {
     int64_t block_segments_max = 0, block_gaps_max = 0;
     bool use_blocks = false;         // set by a plan of SDDMM_AUTO
     unsigned int *d_long_sums = nullptr;    // arena view: long rows per block of the row scan
+    // entries that came in no order, sorted by row and column block: row and column of each, the place every entry
+    // went to, and the dot products in that order
+    int32_t *d_order = nullptr;      // one allocation, kept until the sparse operand goes
+    int32_t *d_order_row = nullptr, *d_order_col = nullptr, *d_order_place = nullptr;
+    float *d_order_dots = nullptr;
+    int64_t order_cap = 0;
+    int64_t coo_jumps = 0;           // entries that share neither row nor column with the one before them
+    bool use_order = false;          // set by a plan of SDDMM_AUTO
     // fused SDDMM + SpMM: items covering every non-empty row, output M x K
     RowItem *d_fused_items = nullptr;
     int64_t n_fused_items = 0, fused_items_cap = 0;
@@ -191,6 +199,10 @@ inline int launch_status(sddmm_ctx *c) {
         const int ls_ = launch_status(c);              \
         if (ls_) return ls_;                           \
     } while (0)
+
+// the entries as the flat kernels take them: in the caller's order, or sorted by the plan
+inline const int32_t *entry_rows(const sddmm_ctx *c) { return c->use_order ? c->d_order_row : c->d_rowidx; }
+inline const int32_t *entry_cols(const sddmm_ctx *c) { return c->use_order ? c->d_order_col : c->d_col; }
 
 inline size_t elem_size(int dtype) { return dtype == SDDMM_F32 ? 4 : 2; }
 
@@ -301,7 +313,9 @@ inline int panel_mfma_steps(const sddmm_ctx *c) {
 // ---- launchers, one translation unit per family of kernels ----
 void launch_flat(sddmm_ctx *c);                                                  // launch_flat.hip
 void launch_flat_blocks(sddmm_ctx *c);
+void launch_unsort(sddmm_ctx *c);
 bool blocks_pay(const sddmm_ctx *c);
+bool order_pays(const sddmm_ctx *c);
 bool slices_pay(const sddmm_ctx *c, double entries_per_row);
 int64_t slice_workspace_floats(const sddmm_ctx *c);
 int launch_flat_sliced(sddmm_ctx *c);                                            // number of launches

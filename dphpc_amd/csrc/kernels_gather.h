@@ -185,7 +185,8 @@ struct Layout {
 // whatever the row lengths are; A units are gathered per entry like B units
 // (L1/L2 hits while the row does not change).
 // entries [base, stop) on the calling wavefront
-template <class L>
+// SCALED false: the dot products alone, without S
+template <class L, bool SCALED = true>
 __device__ __forceinline__ void flat_body(const void *__restrict__ A, const void *__restrict__ B, int KU,
                                           const int32_t *__restrict__ rowidx, const int32_t *__restrict__ col,
                                           const float *__restrict__ sval, float *__restrict__ P, int64_t base,
@@ -197,17 +198,19 @@ __device__ __forceinline__ void flat_body(const void *__restrict__ A, const void
     const int64_t last = stop - 1;
     const int64_t n0 = base + lane < last ? base + lane : last;
     int c = ld_stream(col + n0), r = ld_stream(rowidx + n0);
-    float s = ld_stream(sval + n0);
+    float s = 1.f;
+    if constexpr (SCALED) s = ld_stream(sval + n0);
     for (; base < stop; base += WAVE) {
         const int64_t n = base + lane;
         const bool valid = n < stop;
         const int64_t left = stop - base;
         const int count = left < WAVE ? (int)left : WAVE;
         int cn = 0, rn = 0;
-        float sn = 0.f;
+        float sn = 1.f;
         auto prefetch = [&]() {
             const int64_t pn = n + WAVE < last ? n + WAVE : last;
-            cn = ld_stream(col + pn); rn = ld_stream(rowidx + pn); sn = ld_stream(sval + pn);
+            cn = ld_stream(col + pn); rn = ld_stream(rowidx + pn);
+            if constexpr (SCALED) sn = ld_stream(sval + pn);
         };
         float res;
         if constexpr (L::LONG) {
@@ -220,7 +223,7 @@ __device__ __forceinline__ void flat_body(const void *__restrict__ A, const void
             typename C::Areg none;
             res = C::run(A, B, KU, none, (O)c * rb, (O)r * rb, count, lane, prefetch);
         }
-        if (valid) st_stream(P + n, res * s);
+        if (valid) st_stream(P + n, SCALED ? res * s : res);
         c = cn; r = rn; s = sn;
     }
 }
@@ -245,11 +248,12 @@ __global__ __launch_bounds__(BLOCK) void k_flat(const void *__restrict__ A, cons
 
 // One wavefront, one work item = entries [start,end) of `row`.  The lane's units
 // of the A row stay in registers for the whole segment; no row index is read.
-template <class L>
+template <class L, bool SCALED = true>
 __device__ __forceinline__ void row_segment_body(const void *__restrict__ A, const void *__restrict__ B, int KU,
                                                  const int32_t *__restrict__ col, const float *__restrict__ sval,
                                                  float *__restrict__ P, int row, int start, int end, int lane) {
     using U = typename L::U;
+    static_assert(!L::LONG || SCALED, "dot products alone: rows in the register layout only");
     if (start >= end) return;
     if constexpr (L::LONG) {
         for (int base = start; base < end; base += WAVE) {
@@ -272,19 +276,21 @@ __device__ __forceinline__ void row_segment_body(const void *__restrict__ A, con
         const int last = end - 1;
         const int n0 = start + lane < last ? start + lane : last;
         int c = ld_stream(col + n0);
-        float s = ld_stream(sval + n0);
+        float s = 1.f;
+        if constexpr (SCALED) s = ld_stream(sval + n0);
         for (int base = start; base < end; base += WAVE) {
             const int n = base + lane;
             const bool valid = n < end;
             const int left = end - base;
             int cn = 0;
-            float sn = 0.f;
+            float sn = 1.f;
             auto prefetch = [&]() {
                 const int pn = n + WAVE < last ? n + WAVE : last;
-                cn = ld_stream(col + pn); sn = ld_stream(sval + pn);
+                cn = ld_stream(col + pn);
+                if constexpr (SCALED) sn = ld_stream(sval + pn);
             };
             const float res = C::run(A, B, KU, a, (O)c * rb, (O)0, left < WAVE ? left : WAVE, lane, prefetch);
-            if (valid) st_stream(P + n, res * s);
+            if (valid) st_stream(P + n, SCALED ? res * s : res);
             c = cn; s = sn;
         }
     }
@@ -403,7 +409,8 @@ __device__ __forceinline__ void entry_list_body(const void *__restrict__ A, cons
 // time in storage order (64: 524 us, 256: 538, 512: 541), after the segments on every XCD (before
 // them: the same; dealt out evenly: 542 us).
 // totals[0], totals[1]: work items of either kind (the grid is sized for an upper bound)
-template <class L>
+//
+template <class L, bool SCALED>
 __global__ __launch_bounds__(BLOCK) void k_flat_blocks(const void *__restrict__ A, const void *__restrict__ B, int KU,
                                                        const int32_t *__restrict__ rowidx,
                                                        const int32_t *__restrict__ col,
@@ -427,8 +434,8 @@ __global__ __launch_bounds__(BLOCK) void k_flat_blocks(const void *__restrict__ 
     const int row = __builtin_amdgcn_readfirstlane(it.row);
     const int start = __builtin_amdgcn_readfirstlane(it.start);
     const int end = __builtin_amdgcn_readfirstlane(it.end);
-    if (segment) row_segment_body<L>(A, B, KU, col, sval, P, row, start, end, lane_id());
-    else flat_body<L>(A, B, KU, rowidx, col, sval, P, start, end, lane_id());
+    if (segment) row_segment_body<L, SCALED>(A, B, KU, col, sval, P, row, start, end, lane_id());
+    else flat_body<L, SCALED>(A, B, KU, rowidx, col, sval, P, start, end, lane_id());
 }
 
 // ---------------------------------------------------------------------------

@@ -25,12 +25,21 @@ void launch_flat_blocks(sddmm_ctx *c) {
     const int64_t grid = NUM_XCD * (eighth(c->block_segments_max) + eighth(c->block_gaps_max));
     with_layout(s, [&](auto L) {
         using LT = decltype(L);
-        if constexpr (!LT::LONG)
-            SDDMM_LAUNCH(c, (k_flat_blocks<LT>), grid, BLOCK, (const void *)c->dA, (const void *)c->dB, s.len,
-                         (const int32_t *)c->d_rowidx, (const int32_t *)c->d_col, (const float *)c->d_sval, c->dP,
-                         (const RowItem *)c->d_block_segments, (const RowItem *)c->d_block_gaps,
-                         (const unsigned long long *)c->d_block_totals);
+        if constexpr (!LT::LONG) {
+            auto launch = [&](auto kernel, float *out) {
+                SDDMM_LAUNCH(c, kernel, grid, BLOCK, (const void *)c->dA, (const void *)c->dB, s.len, entry_rows(c),
+                             entry_cols(c), (const float *)c->d_sval, out, (const RowItem *)c->d_block_segments,
+                             (const RowItem *)c->d_block_gaps, (const unsigned long long *)c->d_block_totals);
+            };
+            if (c->use_order) launch(k_flat_blocks<LT, false>, c->d_order_dots);
+            else launch(k_flat_blocks<LT, true>, c->dP);
+        }
     });
+}
+
+void launch_unsort(sddmm_ctx *c) {
+    SDDMM_LAUNCH(c, k_unsort, (c->nnz + 4 * BLOCK - 1) / (4 * BLOCK), BLOCK, (const float *)c->d_order_dots,
+                 (const int32_t *)c->d_order_place, (const float *)c->d_sval, c->dP, c->nnz);
 }
 
 // Measured on power-law graphs (rows of Zipf lengths, half to two thirds of the entries in rows of more than 256) of
@@ -43,6 +52,22 @@ bool blocks_pay(const sddmm_ctx *c) {
     if (mode >= 0) return mode != 0;
     const double b_bytes = (double)c->N * (double)c->K * (double)elem_size(c->dtype);
     return b_bytes >= 12.0 * (1 << 20) && c->nnz >= (1 << 20) && (double)c->pc.nnz_long >= 0.25 * (double)c->nnz;
+}
+
+// Entries in no order, sorted by the plan (k_unsort).  Measured on shuffled uniform, power-law, banded and tiled
+// matrices of 0.1 .. 6.5 M entries, K = 32 .. 400: 1.03 .. 2.1 times the plain kernel from 192-byte rows, 1.5 MB of A
+// and 150 MB of gathered B rows on, up to 3.5 times where the sorted entries can go in slices of K.  Below:
+// 128-byte rows 0.5 .. 1.2 times (k_unsort costs what the A rows save), 0.9 MB of A 0.87 .. 0.94 (A is found in the
+// L2s in any order), 100 MB gathered 0.7 .. 1.05.  Rows of one entry have nothing to share (0.9 .. 1.15).  Entries
+// that arrive grouped, by column (0.65 .. 0.95 times) or in runs of sorted rows (0.8 .. 1.2), keep their order: most
+// of them share a row or a column with the entry before.  The plan takes 0.2 ms for 1.2 M entries.
+bool order_pays(const sddmm_ctx *c) {
+    const int mode = env_int("SDDMM_ORDER", -1);                    // -1: decide here, 0: never, 1: wherever a kernel can
+    if (shape_of(c).LPN == 0 && !slices_pay(c, 1.0)) return false;  // (no kernel takes the order)
+    if (mode >= 0) return mode != 0;
+    const int64_t row_bytes = (int64_t)c->K * (int64_t)elem_size(c->dtype);
+    return 2 * c->coo_jumps >= c->nnz && c->nnz >= 2 * (int64_t)c->sM && row_bytes >= 192 &&
+           (int64_t)c->sM * row_bytes >= 1500 * 1000 && c->nnz * row_bytes >= (int64_t)150 * 1000 * 1000;
 }
 
 namespace {
@@ -68,10 +93,11 @@ int launch_slices_t(sddmm_ctx *c, int slices) {
         const int64_t waves = (n + SLICE_ENTRIES - 1) / SLICE_ENTRIES;
         const int64_t per_slice = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK, nblocks = per_slice * slices;
         SDDMM_LAUNCH(c, (k_slice_dots<U, MISALIGNED, UNALIGNED, WIDE>), xcd_grid(nblocks), BLOCK, (const void *)c->dA,
-                     (const void *)c->dB, row_bytes, (const int32_t *)c->d_rowidx + e0, (const int32_t *)c->d_col + e0,
+                     (const void *)c->dB, row_bytes, entry_rows(c) + e0, entry_cols(c) + e0,
                      c->d_part, n, stride, per_slice, nblocks);
         SDDMM_LAUNCH(c, k_slice_sum, (n + 4 * BLOCK - 1) / (4 * BLOCK), BLOCK, (const float *)c->d_part, slices, stride,
-                     (const float *)c->d_sval + e0, c->dP + e0, n);
+                     (const float *)(c->use_order ? nullptr : c->d_sval + e0),
+                     c->use_order ? c->d_order_dots + e0 : c->dP + e0, n);
         launches += 2;
     }
     return launches;

@@ -110,6 +110,11 @@ void release_sparse(sddmm_ctx *c) {
     dfree(c->d_short_list);
     c->short_list_cap = c->n_short_list = 0;
     c->use_short_list = false;
+    dfree(c->d_order);
+    c->d_order_row = c->d_order_col = c->d_order_place = nullptr;
+    c->d_order_dots = nullptr;
+    c->order_cap = 0;
+    c->use_order = false;
     dfree(c->d_fused_items);
     c->n_fused_items = c->fused_items_cap = 0;
     c->fused_items_valid = c->have_fused = false;
@@ -592,14 +597,17 @@ int ensure_rowidx(sddmm_ctx *c) {
 // Work items of k_flat_blocks: the segments of the long rows (more than `seg` entries) block by block, and
 // the entries between those rows.  Nothing is read back: the arrays are sized for the most items there
 // can be, the launch reads the true numbers.  Leaves use_blocks false when the device has no room.
-int plan_blocks(sddmm_ctx *c) {
-    const int64_t n_long = (int64_t)c->pc.rows_long, nb = ((int64_t)c->sM + SCAN_TILE - 1) / SCAN_TILE;
-    if ((int64_t)c->raw.long_scanned != n_long)
+// cut_long_rows false: the entries 64 at a time and nothing else (the way to take a sorted order whose long rows
+// need no cutting).
+int plan_blocks(sddmm_ctx *c, bool cut_long_rows) {
+    const int64_t n_long = cut_long_rows ? (int64_t)c->pc.rows_long : 0, nb = ((int64_t)c->sM + SCAN_TILE - 1) / SCAN_TILE;
+    const int64_t nnz_long = cut_long_rows ? (int64_t)c->pc.nnz_long : 0;
+    if (cut_long_rows && (int64_t)c->raw.long_scanned != n_long)
         return fail(c, SDDMM_ERR_HIP, "internal: scan of the long rows disagrees with their number");
     const int64_t n_seg = n_long * COL_BLOCKS, n_gap = n_long + 1;
     const int64_t piece = c->seg, gap_piece = WAVE;
-    c->block_segments_max = (int64_t)c->pc.nnz_long / piece + n_seg;
-    c->block_gaps_max = (c->nnz - (int64_t)c->pc.nnz_long) / gap_piece + n_gap;
+    c->block_segments_max = nnz_long / piece + n_seg;
+    c->block_gaps_max = (c->nnz - nnz_long) / gap_piece + n_gap;
     size_t at = 0;
     auto take = [&](size_t bytes) {
         const size_t here = at;
@@ -629,9 +637,11 @@ int plan_blocks(sddmm_ctx *c) {
     int32_t *rows = (int32_t *)(b + o_rows), *seg_start = (int32_t *)(b + o_seg[0]), *gap_start = (int32_t *)(b + o_gap[0]);
     unsigned int *seg_items = (unsigned int *)(b + o_seg[1]), *seg_off = (unsigned int *)(b + o_seg[2]);
     unsigned int *gap_items = (unsigned int *)(b + o_gap[1]), *gap_off = (unsigned int *)(b + o_gap[2]);
-    SDDMM_LAUNCH(c, k_long_rows, nb, SCAN_BLOCK, c->d_rowptr, c->sM, c->seg, (const unsigned int *)c->d_long_sums, rows);
-    SDDMM_LAUNCH(c, k_long_segments, grid_for(n_seg, 256), 256, c->d_rowptr, c->d_col, c->sN, (const int32_t *)rows,
-                 (int)n_long, (int)piece, seg_start, seg_items);
+    if (n_long > 0) {
+        SDDMM_LAUNCH(c, k_long_rows, nb, SCAN_BLOCK, c->d_rowptr, c->sM, c->seg, (const unsigned int *)c->d_long_sums, rows);
+        SDDMM_LAUNCH(c, k_long_segments, grid_for(n_seg, 256), 256, c->d_rowptr, entry_cols(c), c->sN, (const int32_t *)rows,
+                     (int)n_long, (int)piece, seg_start, seg_items);
+    }
     SDDMM_LAUNCH(c, k_long_gaps, grid_for(n_gap, 256), 256, c->d_rowptr, (const int32_t *)rows, (int)n_long, (int)c->nnz,
                  (int)gap_piece, gap_start, gap_items);
     LAUNCH_CHECK(c);
@@ -641,9 +651,10 @@ int plan_blocks(sddmm_ctx *c) {
     if (rc) return rc;
     rc = flush_scans(c);
     if (rc) return rc;
-    SDDMM_LAUNCH(c, k_range_items, grid_for(c->block_segments_max, 256), 256, c->d_rowptr, (const int32_t *)rows, (int)n_long,
-                 (int)c->nnz, 0, (int)piece, (const int32_t *)seg_start, (const unsigned int *)seg_off, (int)n_seg,
-                 (const unsigned long long *)c->d_block_totals, c->d_block_segments);
+    if (n_long > 0)
+        SDDMM_LAUNCH(c, k_range_items, grid_for(c->block_segments_max, 256), 256, c->d_rowptr, (const int32_t *)rows, (int)n_long,
+                     (int)c->nnz, 0, (int)piece, (const int32_t *)seg_start, (const unsigned int *)seg_off, (int)n_seg,
+                     (const unsigned long long *)c->d_block_totals, c->d_block_segments);
     SDDMM_LAUNCH(c, k_range_items, grid_for(c->block_gaps_max, 256), 256, c->d_rowptr, (const int32_t *)rows, (int)n_long,
                  (int)c->nnz, 1, (int)gap_piece, (const int32_t *)gap_start, (const unsigned int *)gap_off, (int)n_gap,
                  (const unsigned long long *)(c->d_block_totals + 1), c->d_block_gaps);
@@ -667,6 +678,93 @@ bool ensure_slice_workspace(sddmm_ctx *c) {
     c->d_part = static_cast<float *>(p);
     c->part_floats = need;
     return true;
+}
+
+// Entries in no order: sort them by row and column block and plan the flat launch over that order.  Leaves use_order
+// false when the device has no room.
+template <class Key>
+int sort_order(sddmm_ctx *c, bool *done) {
+    const size_t n = (size_t)c->nnz;
+    int bits = 1;
+    while (bits < 36 && ((int64_t)c->sM * COL_BLOCKS - 1) >> bits) ++bits;
+    // (the first buffers of either array hold the unsorted ones)
+    size_t at = 0, need = 0;
+    auto take = [&](size_t bytes) {
+        const size_t here = at;
+        at += (bytes + 255) & ~(size_t)255;
+        return here;
+    };
+    HIP_TRY(c, rocprim::radix_sort_pairs(nullptr, need, (Key *)nullptr, (Key *)nullptr, (int32_t *)nullptr, (int32_t *)nullptr, n,
+                                         0, bits, c->stream));
+    const size_t o_keys = take(n * sizeof(Key)), o_sorted = take(n * sizeof(Key)), o_from = take(n * 4), o_at = take(n * 4), o_tmp = take(need);
+    if (at > c->sort_tmp_bytes) {
+        dfree(c->d_sort_tmp);
+        c->sort_tmp_bytes = 0;
+        if (hipMalloc(&c->d_sort_tmp, at) != hipSuccess) {
+            (void)hipGetLastError();                       // the failed allocation is not an error of the plan
+            c->d_sort_tmp = nullptr;
+            return SDDMM_OK;
+        }
+        c->sort_tmp_bytes = at;
+    }
+    if (c->nnz > c->order_cap) {
+        const size_t column = (n * 4 + 255) & ~(size_t)255;
+        dfree(c->d_order);
+        c->order_cap = 0;
+        if (hipMalloc((void **)&c->d_order, 4 * column) != hipSuccess) {
+            (void)hipGetLastError();
+            c->d_order = nullptr;
+            return SDDMM_OK;
+        }
+        c->order_cap = c->nnz;
+        c->d_order_row = c->d_order;
+        c->d_order_col = c->d_order + column / 4;
+        c->d_order_place = c->d_order + 2 * (column / 4);
+        c->d_order_dots = (float *)(c->d_order + 3 * (column / 4));
+    }
+    char *b = (char *)c->d_sort_tmp;
+    Key *keys = (Key *)(b + o_keys), *sorted = (Key *)(b + o_sorted);
+    int32_t *from = (int32_t *)(b + o_from), *sorted_from = (int32_t *)(b + o_at);
+    const int64_t grid = (c->nnz + 255) / 256;
+    SDDMM_LAUNCH(c, k_order_keys<Key>, grid, 256, (const int32_t *)c->d_rowidx, (const int32_t *)c->d_col, c->nnz, c->sN, keys, from);
+    LAUNCH_CHECK(c);
+    HIP_TRY(c, rocprim::radix_sort_pairs(b + o_tmp, need, keys, sorted, from, sorted_from, n, 0, bits, c->stream));
+    SDDMM_LAUNCH(c, k_order_entries<Key>, grid, 256, (const Key *)sorted, (const int32_t *)sorted_from,
+                 (const int32_t *)c->d_col, c->nnz, c->d_order_row, c->d_order_col, c->d_order_place);
+    SDDMM_LAUNCH(c, k_rowptr_from_sorted_coo, grid_for(c->nnz + 1, 256), 256, (const int32_t *)c->d_order_row, c->nnz, c->sM,
+                 c->d_rowptr);
+    LAUNCH_CHECK(c);
+    *done = true;
+    return SDDMM_OK;
+}
+
+int plan_order(sddmm_ctx *c) {
+    bool done = false;
+    int rc = (int64_t)c->sM * COL_BLOCKS <= ((int64_t)1 << 32) ? sort_order<uint32_t>(c, &done) : sort_order<uint64_t>(c, &done);
+    if (rc || !done) return rc;
+    rc = begin_ownership(c);
+    if (rc) return rc;
+    // row statistics of the sorted entries; no row has another owner
+    c->ts = std::max(1, env_int("SDDMM_TS", 24));
+    c->seg = std::max(WAVE, env_int("SDDMM_SEG", 256));
+    HIP_TRY(c, hipMemsetAsync(&c->d_pc->k[K_ROWS_NONEMPTY][0], 0, sizeof(unsigned long long) * SPREAD, c->stream));
+    SDDMM_LAUNCH(c, k_check_rowptr, grid_for(c->sM, 256), 256, (const int32_t *)c->d_rowptr, c->sM, c->nnz, c->d_pc);
+    LAUNCH_CHECK(c);
+    rc = classify_rows_count(c);
+    if (rc) return rc;
+    rc = fetch_counters(c);
+    if (rc) return rc;
+    if (c->pc.bad_pattern) return fail(c, SDDMM_ERR_HIP, "internal: row pointer built from sorted entries is inconsistent");
+    const double avg_len = c->pc.rows_nonempty ? (double)c->nnz / (double)c->pc.rows_nonempty : 0.0;
+    c->pc.rows_nonempty = 0;                               // (reported as unknown without a row pointer of the caller's order)
+    c->use_order = true;
+    c->use_slices = slices_pay(c, avg_len) && ensure_slice_workspace(c);
+    if (!c->use_slices) {
+        rc = plan_blocks(c, blocks_pay(c));
+        if (rc) return rc;
+        c->use_order = c->use_blocks;
+    }
+    return SDDMM_OK;
 }
 
 // Validate the device-resident CSR and gather row statistics.
@@ -725,6 +823,7 @@ int enqueue_run(sddmm_ctx *c) {
             if (c->use_slices) c->launches = launch_flat_sliced(c);
             else if (c->use_blocks) launch_flat_blocks(c);
             else launch_flat(c);
+            if (c->use_order) { launch_unsort(c); ++c->launches; }
             break;
         case SDDMM_ROW_WAVE: launch_row_wave(c, nullptr, c->sM); break;
         case SDDMM_SHORT_ROWS:
@@ -753,7 +852,7 @@ int do_plan(sddmm_ctx *c, int strategy) {
     // previous one looking valid (its items exclude rows that tiles and panels owned)
     c->planned = false;
     c->n_scan_jobs = 0;
-    c->use_slices = c->use_blocks = false;
+    c->use_slices = c->use_blocks = c->use_order = false;
     c->fused_items_valid = false;    // they leave out the rows of this plan's panels
     int resolved = strategy;
     const bool csr_ok = c->have_rowptr;
@@ -852,7 +951,7 @@ int do_plan(sddmm_ctx *c, int strategy) {
                 resolved = SDDMM_FLAT;
                 c->use_slices = sliced;
                 if (!sliced && blocks_pay(c)) {
-                    rc = plan_blocks(c);
+                    rc = plan_blocks(c, true);
                     if (rc) return rc;
                 }
             } else {
@@ -866,7 +965,11 @@ int do_plan(sddmm_ctx *c, int strategy) {
             int rc = ensure_rowidx(c);
             if (rc) return rc;
             // (asked for by name, FLAT stays the plain kernel; AUTO on unsorted entries gets here too)
-            if (strategy == SDDMM_AUTO) c->use_slices = c->nnz > 0 && slices_pay(c, 1.0) && ensure_slice_workspace(c);
+            if (strategy == SDDMM_AUTO && c->nnz > 0) {
+                if (order_pays(c)) rc = plan_order(c);
+                if (rc) return rc;
+                if (!c->use_blocks && !c->use_slices) c->use_slices = slices_pay(c, 1.0) && ensure_slice_workspace(c);
+            }
             break;
         }
         case SDDMM_ROW_WAVE:
@@ -1105,7 +1208,8 @@ static int set_coo_common(sddmm_ctx *c, int M, int N, int64_t nnz, const int32_t
         const int g = grid_capped(nnz, 256);
         SDDMM_LAUNCH(c, k_check_index, g, 256, c->d_rowidx, nnz, M, c->d_pc);
         SDDMM_LAUNCH(c, k_check_index, g, 256, c->d_col, nnz, N, c->d_pc);
-        SDDMM_LAUNCH(c, k_check_coo_sorted, g, 256, c->d_rowidx, nnz, c->d_pc);
+        SDDMM_LAUNCH(c, k_check_coo_sorted, grid_capped(nnz, 256, 1024), 256, (const int32_t *)c->d_rowidx,
+                           (const int32_t *)c->d_col, nnz, c->d_pc);
         LAUNCH_CHECK(c);
     }
     rc = fetch_counters(c);
@@ -1115,6 +1219,7 @@ static int set_coo_common(sddmm_ctx *c, int M, int N, int64_t nnz, const int32_t
         return fail(c, SDDMM_ERR_PATTERN, "COO row or column index out of range");
     }
     const bool sorted = c->pc.coo_unsorted == 0;
+    c->coo_jumps = (int64_t)c->pc.coo_jumps;
     if (sorted) {
         SDDMM_LAUNCH(c, k_rowptr_from_sorted_coo, grid_for(nnz + 1, 256), 256,
                            c->d_rowidx, nnz, M, c->d_rowptr);
