@@ -32,7 +32,8 @@ int ensure_arena(sddmm_ctx *c) {
     const int64_t M = c->sM;
     if (c->d_arena && c->arena_rows == M) return SDDMM_OK;
     release_arena(c);
-    const int64_t n_strips = (M + 15) / 16, n_panels = M / 8 + 1, n_sums = M / 256 + 8;
+    const int64_t n_strips = (M + 15) / 16, n_panels = M / 8 + 1;
+    const int64_t n_sums = M * COL_BLOCKS / SCAN_TILE + 8;  // the longest scan: a count per row and column block
     size_t at = 0;
     auto take = [&](size_t bytes) {
         const size_t here = at;

@@ -77,6 +77,23 @@ def test_sorted_order(engine_factory, monkeypatch, K, dtype, blocks):
                     np.testing.assert_array_equal(e.values(), got)
 
 
+def test_every_row_long(engine_factory, monkeypatch):
+    """More column blocks of long rows than a scan in one workgroup takes, in a matrix of few rows."""
+    monkeypatch.setenv("SDDMM_ORDER", "1")
+    monkeypatch.setenv("SDDMM_COLUMN_BLOCKS", "1")
+    rng = np.random.default_rng(5)
+    M, N, K = 1100, 5000, 8
+    A, B = _operands(rng, M, N, K, capi.F32)
+    r, c, v = _entries(rng, M, N, [300] * M)
+    with engine_factory() as e:
+        e.set_dense(A, B)
+        e.set_coo(M, N, r, c, v)
+        e.plan(capi.AUTO)
+        e.run()
+        assert e.stats().kernels_launched == 2
+        _check(e.values(), r, c, v, A, B, "every row long")
+
+
 def test_sorted_order_in_ranges_of_the_slice_workspace(engine_factory, monkeypatch):
     monkeypatch.setenv("SDDMM_ORDER", "1")
     monkeypatch.setenv("SDDMM_SLICES", "1")
