@@ -140,6 +140,7 @@ struct sddmm_ctx {
     bool fused_items_valid = false;
     bool fused_items_panels = false; // the fused items leave out the rows that the panel kernel owns
     double fused_short_avg = 0.0;    // entries per non-empty row of at most FUSED_ROW_MAX entries (panel rows apart)
+    int fused_row_max = FUSED_ROW_MAX;   // rows beyond it are work items of their own
     float *dO = nullptr;
     size_t o_cap = 0;
     bool have_fused = false;

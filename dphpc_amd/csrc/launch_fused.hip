@@ -2,18 +2,21 @@
 #include "context.h"
 #include "kernels_fused.h"
 
-// Rows of at most FUSED_ROW_MAX entries, then the work items of the longer ones; 0: no kernel for this row layout.
+// Rows of at most fused_row_max entries, then the work items of the longer ones; 0: no kernel for this row layout.
 int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
     const Shape s = shape_of(c);
     // Short rows of fewer entries, on average, than half of what a lane group takes per step (a power-law
-    // graph: 3.5 against 8 lanes per entry at 128-byte rows): one row per lane group would idle most of its
-    // steps (20 % of them useful there), so the wavefronts deal whole rows out to their groups by entry
-    // count instead (576 -> 369 us for those rows).  With longer rows, or 4 lanes per entry, the extra
-    // gathers of the A rows and the longer walks cost more than the idle steps (mixed-density shape, 12.5
-    // entries per short row: 33 -> 65 us; power-law with 64-byte rows: 396 -> 432 us).
+    // graph: 2.8 against 8 lanes per entry) leave most lanes of a group idle in one row per lane group: the
+    // wavefronts deal whole rows out to their groups by entry count instead.  That takes 64 rows per wavefront,
+    // so it needs enough rows to fill the chip: graphs of 2.6 M rows, 128 bytes 944 -> 787 us, 1 M rows,
+    // 256 bytes 442 -> 414 us, 500 k rows 147 -> 132 us; 200 k rows 86 -> 86 us (128 bytes), 215 -> 235 us
+    // (512 bytes); 50 k rows 40 -> 44 us, 8 k rows 14.5 -> 20 us.  With longer rows, or fewer lanes per entry,
+    // the extra gathers of the A rows and the longer walks cost more than the idle lanes (12.5 entries per
+    // short row: 33 -> 65 us; 1 M rows of 64 bytes 206 -> 239 us).
     const int balanced_env = env_int("SDDMM_FUSED_BALANCED", -1);
     const bool balanced = balanced_env >= 0 ? balanced_env != 0
-                                            : (c->fused_short_avg > 0.0 && 2.0 * c->fused_short_avg < (double)s.LPN);
+                                            : (c->sM >= 400000 && c->fused_short_avg > 0.0 &&
+                                               2.0 * c->fused_short_avg < (double)s.LPN);
     int launches = 0;
     with_layout(s, [&](auto L) {
         using LT = decltype(L);
@@ -26,11 +29,11 @@ int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
                 const int64_t bblocks = (bwaves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
                 SDDMM_LAUNCH(c, (k_fusedmm_rows_balanced<LT>), xcd_grid(bblocks), BLOCK,
                                    (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col, c->d_sval,
-                                   c->dP, c->dO, c->sM, FUSED_ROW_MAX, bblocks, panel_owner);
+                                   c->dP, c->dO, c->sM, c->fused_row_max, bblocks, panel_owner);
             } else {
                 SDDMM_LAUNCH(c, (k_fusedmm_rows<LT>), xcd_grid(rblocks), BLOCK,
                                    (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col, c->d_sval,
-                                   c->dP, c->dO, c->sM, FUSED_ROW_MAX, rblocks, panel_owner);
+                                   c->dP, c->dO, c->sM, c->fused_row_max, rblocks, panel_owner);
             }
             ++launches;
             if (c->n_fused_items > 0) {

@@ -1334,14 +1334,15 @@ int sddmm_run(sddmm_ctx *c) {
     return SDDMM_OK;
 }
 
-// items of the fused kernel: the rows of more than FUSED_ROW_MAX entries, cut into segments of
-// SDDMM_FUSED_SEG entries (default 2048, shortened below when there are few items; a knob of its own,
+// items of the fused kernel: the rows of more than fused_row_max entries, cut into segments of
+// SDDMM_FUSED_SEG entries (default 1024, shortened below when there are few entries; a knob of its own,
 // apart from SDDMM_SEG of the plain SDDMM, because the pieces of a row add to O atomically: the segment
 // length decides which rows are summed in an order that may differ from run to run)
 static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
     if (c->fused_items_valid && c->fused_items_panels == (panel_owner != nullptr)) return SDDMM_OK;
-    int seg = std::max(WAVE, env_int("SDDMM_FUSED_SEG", 2048));
+    int seg = std::max(WAVE, env_int("SDDMM_FUSED_SEG", 1024));
     const int64_t nb = ((int64_t)c->sM + SCAN_TILE - 1) / SCAN_TILE;
+    int row_max = FUSED_ROW_MAX;
     const int arc = ensure_arena(c);
     if (arc) return arc;
     ARENA_HOLDS(c, nb, c->block_sums_cap, "block sums");
@@ -1353,7 +1354,7 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
                                       sizeof(unsigned long long) * SPREAD * (K_NNZ_LONG - K_ROWS_SHORT + 1), c->stream));
             HIP_TRY(c, hipMemsetAsync(&c->d_pc->n_items, 0, sizeof(unsigned long long), c->stream));
             SDDMM_LAUNCH(c, k_classify_count, nb, SCAN_BLOCK, c->d_rowptr,
-                               panel_owner, c->sM, FUSED_ROW_MAX + 1, seg, c->d_block_sums, c->d_pc, 2,
+                               panel_owner, c->sM, row_max + 1, seg, c->d_block_sums, c->d_pc, 2,
                                (unsigned int *)nullptr, (unsigned int *)nullptr);
             SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, c->d_block_sums, (int)nb,
                                &c->d_pc->n_items);
@@ -1364,23 +1365,30 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
         };
         int rc = count();
         if (rc) return rc;
-        // Few long rows: one wavefront per row walks its chunks one after the other and the launch
-        // waits for them (3 000 rows of 554 entries: 50 us as single items, 42 us in pieces of 256,
-        // the pieces of a row adding to O atomically).  With enough items to fill the chip several
-        // times the long segments stay: there the atomic adds cost more than they return.
         const PlanCounters first = summarize(tmp);
         const int64_t item_entries = (int64_t)(first.nnz_medium + first.nnz_long);
         c->fused_short_avg = first.rows_short ? (double)first.nnz_short / (double)first.rows_short : 0.0;
-        // (rows of up to 128 bytes; at 256 bytes it changes nothing, at 1 KiB the adds of 256 floats per piece lose 4 %)
-        if ((int64_t)tmp.n_items > 0 && (int64_t)tmp.n_items < 4096 && !getenv("SDDMM_FUSED_SEG") &&
-            (size_t)c->K * elem_size(c->dtype) <= 128) {
-            int shorter = (int)std::min<int64_t>(seg, ((item_entries / 8192 + WAVE - 1) / WAVE) * WAVE);
-            shorter = std::max(shorter, 256);
-            if (shorter < seg) {
-                seg = shorter;
-                rc = count();
-                if (rc) return rc;
-            }
+        // A wavefront walks its item chunk by chunk and the launch waits for the longest one: the long rows are
+        // cut so that there are about 3 072 pieces, none shorter than 256 entries (graph of 50 k rows, 256-byte
+        // rows: 2048 132 us, 512 59 us, 256 50 us; 200 k rows of 512 bytes: 2048 329, 1024 254, 512 246; 1 M rows
+        // of 128 bytes: 2048 306, 1024 293, 512 320, 256 407, the atomic adds of a piece cost what the cut
+        // returns).  Rows that are all about that long stay whole: 3 000 rows of 554 entries of 1 KiB 264 us, in
+        // pieces of 512 280.
+        int best_seg = seg;
+        if (!getenv("SDDMM_FUSED_SEG")) {
+            const int64_t even = ((item_entries / 3072 + WAVE - 1) / WAVE) * WAVE;
+            const int shorter = (int)std::max<int64_t>(256, std::min<int64_t>(seg, even));
+            if ((int64_t)first.max_len > 2 * (int64_t)shorter) best_seg = shorter;
+        }
+        // Where most of the short rows are very short, one of 17 .. 32 entries among them holds up the rows of
+        // its wavefront: those become items too (graphs of 2.8 entries per short row: 5 .. 15 % on 30 k .. 2.6 M
+        // rows, K = 8 .. 256; rows of 5 .. 20 entries lose 20 %, 32 -> 40 us, rows of 17 .. 23 half: 10.6 -> 20 us).
+        const int best_row_max = first.rows_short && c->fused_short_avg < 4.0 ? FUSED_ROW_MAX / 2 : FUSED_ROW_MAX;
+        if (best_seg != seg || best_row_max != row_max) {
+            seg = best_seg;
+            row_max = best_row_max;
+            rc = count();
+            if (rc) return rc;
         }
         c->n_fused_items = (int64_t)tmp.n_items;
         if (c->n_fused_items > c->fused_items_cap) {
@@ -1390,10 +1398,11 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
         }
         if (c->n_fused_items > 0) {
             SDDMM_LAUNCH(c, k_classify_write, nb, SCAN_BLOCK, c->d_rowptr,
-                               panel_owner, c->sM, FUSED_ROW_MAX + 1, seg, c->d_block_sums, c->d_fused_items, 2);
+                               panel_owner, c->sM, row_max + 1, seg, c->d_block_sums, c->d_fused_items, 2);
             LAUNCH_CHECK(c);
         }
     }
+    c->fused_row_max = row_max;
     c->fused_items_valid = true;
     c->fused_items_panels = panel_owner != nullptr;
     return SDDMM_OK;

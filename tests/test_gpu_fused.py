@@ -399,3 +399,33 @@ def test_fused_row_panels_keep_non_finite_b_rows_in_their_own_entries(engine_fac
     np.testing.assert_allclose(got_o[:8], ref_o[:8], rtol=1e-4, atol=1e-5)
     assert np.array_equal(np.isfinite(got_o), np.isfinite(ref_o))
     e.close()
+
+
+@pytest.mark.parametrize("K,dtype", [(8, capi.F32), (32, capi.F32), (64, capi.F16), (128, capi.F32)])
+@pytest.mark.parametrize("M,lens", [
+    (700, [15, 16, 17, 31, 32, 33, 34]),                                     # one row per lane group up to 32 entries
+    (1500, [0, 1, 1, 2, 2, 3]),                                              # up to 16
+    (400_003, [0, 1, 1, 2, 2, 3]),                                           # rows dealt out by entry count
+])
+def test_fused_row_and_item_edges(engine_factory, M, lens, K, dtype):
+    """Row lengths on either side of those that make a row an item and an item several pieces."""
+    rng = np.random.default_rng(M + K)
+    N = 6007
+    n = rng.choice(lens, M)
+    edges = [15, 16, 17, 31, 32, 33, 255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 2049, 6000]
+    n[rng.choice(M, len(edges), replace=False)] = edges
+    n[-1] = 257
+    rowptr = np.concatenate([[0], np.cumsum(n)]).astype(np.int32)
+    first = rng.integers(0, N, M)                                            # ascending runs of every third column, wrapped
+    col = ((np.repeat(first, n) + 3 * (np.arange(rowptr[-1]) - np.repeat(rowptr[:-1], n))) % N).astype(np.int32)
+    val = rng.uniform(-1, 1, len(col)).astype(f32)
+    A = rng.uniform(-1, 1, (M, K)).astype(f32)
+    B = rng.uniform(-1, 1, (N, K)).astype(f32)
+    if dtype == capi.F16:
+        A, B = capi.from_f16(capi.to_f16(A)), capi.from_f16(capi.to_f16(B))
+    e = engine_factory()
+    e.set_dense(A if dtype == capi.F32 else capi.to_f16(A), B if dtype == capi.F32 else capi.to_f16(B), dtype)
+    e.set_csr(M, N, rowptr, col, val)
+    print("fused edges", M, K, dtype, flush=True)
+    _check(e, rowptr, col, val, A, B, "%d rows K=%d" % (M, K))
+    e.close()
