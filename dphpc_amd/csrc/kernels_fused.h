@@ -10,7 +10,7 @@
 // bf16 or fp16 (16-byte units of 4 or 8 elements); P and O are fp32.
 //
 // k_fusedmm: one wavefront per work item = entries [start,end) of one row (rows longer
-// than fused_row_max (16 or 32) entries; shorter ones go to k_fusedmm_rows), in the lane layout
+// than fused_row_max (16 or 64) entries; shorter ones go to k_fusedmm_rows), in the lane layout
 // of the gather kernels: groups of LPN lanes, lane j of a group holds units
 // j, j+LPN, ... of the A row, of the entry's B row and of the group's partial output
 // row.  After the last entry the partial rows of the 64/LPN groups are added with

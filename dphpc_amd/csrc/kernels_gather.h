@@ -25,10 +25,7 @@ namespace sddmm {
 
 constexpr int BLOCK = 256;                 // 4 wavefronts
 constexpr int WAVES_PER_BLOCK = BLOCK / WAVE;
-// fused SDDMM + SpMM: rows up to this length take one lane group each.  A lane group walks its row alone, so
-// longer rows hold up their wavefront: at 64 a graph of 200 k rows takes 95 us (128 bytes) and 273 (512), at 32 87
-// and 250, rows of 42 .. 48 entries 91.8 and 86.7; rows of 5 .. 20 entries do not mind
-constexpr int FUSED_ROW_MAX = 32;
+constexpr int FUSED_ROW_MAX = 64;          // fused SDDMM + SpMM: rows up to this length take one lane group each (a quarter of it: plan_fused_items)
 
 // Byte offset of a row: 32-bit when the whole operand is below 4 GiB (one VALU
 // multiply, scalar base + 32-bit vector offset addressing), 64-bit otherwise.

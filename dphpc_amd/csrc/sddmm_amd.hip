@@ -1380,10 +1380,11 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
             const int shorter = (int)std::max<int64_t>(256, std::min<int64_t>(seg, even));
             if ((int64_t)first.max_len > 2 * (int64_t)shorter) best_seg = shorter;
         }
-        // Where most of the short rows are very short, one of 17 .. 32 entries among them holds up the rows of
-        // its wavefront: those become items too (graphs of 2.8 entries per short row: 5 .. 15 % on 30 k .. 2.6 M
-        // rows, K = 8 .. 256; rows of 5 .. 20 entries lose 20 %, 32 -> 40 us, rows of 17 .. 23 half: 10.6 -> 20 us).
-        const int best_row_max = first.rows_short && c->fused_short_avg < 4.0 ? FUSED_ROW_MAX / 2 : FUSED_ROW_MAX;
+        // Where most of the short rows are very short, one of 17 .. 64 entries among them holds up the rows of its
+        // wavefront: those become items too (graphs of 2.8 .. 4 entries per short row, 64 against 16: 200 k rows K=8
+        // 61 -> 44 us, K=64 fp16 95 -> 86 us; 1 M rows K=64 487 -> 442 us; 50 k rows 51 -> 40 us).  Rows of about one
+        // length stay: 42 .. 48 entries each, K=128 54 us, as items 84; 17 .. 23 entries 10.5 and 20 us.
+        const int best_row_max = first.rows_short && c->fused_short_avg < 8.0 ? FUSED_ROW_MAX / 4 : FUSED_ROW_MAX;
         if (best_seg != seg || best_row_max != row_max) {
             seg = best_seg;
             row_max = best_row_max;

@@ -403,7 +403,7 @@ def test_fused_row_panels_keep_non_finite_b_rows_in_their_own_entries(engine_fac
 
 @pytest.mark.parametrize("K,dtype", [(8, capi.F32), (32, capi.F32), (64, capi.F16), (128, capi.F32)])
 @pytest.mark.parametrize("M,lens", [
-    (700, [15, 16, 17, 31, 32, 33, 34]),                                     # one row per lane group up to 32 entries
+    (700, [15, 16, 17, 31, 33, 63, 64, 65]),                                 # one row per lane group up to 64 entries
     (1500, [0, 1, 1, 2, 2, 3]),                                              # up to 16
     (400_003, [0, 1, 1, 2, 2, 3]),                                           # rows dealt out by entry count
 ])
