@@ -15,6 +15,7 @@ _LIB_PATH = os.environ.get("SDDMM_LIB") or os.path.join(_PKG, "lib", "libsddmm_a
 AUTO, FLAT, ROW_WAVE, SHORT_ROWS, LDS_TILED, MFMA_TILE, EXACT = range(7)
 STRATEGY_NAMES = ["AUTO", "FLAT", "ROW_WAVE", "SHORT_ROWS", "LDS_TILED", "MFMA_TILE", "EXACT"]
 F32, BF16, F16 = 0, 1, 2
+FLAT_SLICES, FLAT_BLOCKS, FLAT_SORTED = 1, 2, 4
 
 OK, ERR_INVALID, ERR_NULL, ERR_STATE, ERR_ALLOC, ERR_HIP, ERR_UNSUPPORTED, ERR_NO_DEVICE, ERR_PATTERN = (
     0, -1, -2, -3, -4, -5, -6, -7, -8)
@@ -29,7 +30,7 @@ EXPORTS = [
     "sddmm_launch", "sddmm_synchronize", "sddmm_time_runs", "sddmm_time_region", "sddmm_run_fused",
     "sddmm_get_fused", "sddmm_get_fused_device", "sddmm_get_values",
     "sddmm_get_values_device", "sddmm_last_stats", "sddmm_partition_rows", "sddmm_version",
-    "sddmm_launch_noalloc",
+    "sddmm_launch_noalloc", "sddmm_flat_variant",
 ]
 
 
@@ -100,6 +101,7 @@ def load_library():
     L.sddmm_get_values.argtypes = [vp, vp]
     L.sddmm_get_values_device.argtypes = [vp, C.POINTER(vp)]
     L.sddmm_last_stats.argtypes = [vp, C.POINTER(Stats)]
+    L.sddmm_flat_variant.argtypes = [vp, C.POINTER(i32)]
     L.sddmm_partition_rows.argtypes = [i32, vp, i32, i32, vp]
     L.sddmm_version.restype = C.c_char_p
     L.sddmm_launch_noalloc.argtypes = [i32, i32, i32, i64, vp, vp, vp, vp, vp, vp, vp]
@@ -258,6 +260,12 @@ class Engine:
         s = Stats()
         self._chk(self.L.sddmm_last_stats(self.h, C.byref(s)))
         return s
+
+    def flat_variant(self):
+        """FLAT_* bits of the current plan (0: the plain flat kernel, or another strategy)."""
+        v = C.c_int(0)
+        self._chk(self.L.sddmm_flat_variant(self.h, C.byref(v)))
+        return v.value
 
 
 def sddmm_csr(rowptr, col, sval, A, B, N=None, strategy=AUTO, dtype=F32, device=0):

@@ -212,6 +212,17 @@ inline int env_int(const char *name, int fallback) {
     return e && *e ? atoi(e) : fallback;
 }
 
+// Memory that a plan can do without: nullptr where the device has none left, or where the array is larger than
+// SDDMM_SPARE_BYTES allows (no limit by default).  The plan then takes the kernels that need no such array.
+inline void *spare_alloc(size_t bytes) {
+    const char *limit = getenv("SDDMM_SPARE_BYTES");
+    if (limit && *limit && bytes > (size_t)strtoull(limit, nullptr, 10)) return nullptr;
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes ? bytes : 16) == hipSuccess && p) return p;
+    (void)hipGetLastError();                               // the failed allocation is not an error of the plan
+    return nullptr;
+}
+
 // ---- kernel dispatch over the (unit type, lanes per entry, units per lane) layouts ----
 struct Shape {
     int unit;    // 0: fp32 x4, 1: fp32 x1 (K < 4), 2: bf16 x8, 3: fp16 x8, 4: fp32 x4 in rows of no whole number of units
@@ -313,7 +324,7 @@ inline int panel_mfma_steps(const sddmm_ctx *c) {
 
 // ---- launchers, one translation unit per family of kernels ----
 void launch_flat(sddmm_ctx *c);                                                  // launch_flat.hip
-void launch_flat_blocks(sddmm_ctx *c);
+int launch_flat_blocks(sddmm_ctx *c);                                            // number of launches
 void launch_unsort(sddmm_ctx *c);
 bool blocks_pay(const sddmm_ctx *c);
 bool order_pays(const sddmm_ctx *c);

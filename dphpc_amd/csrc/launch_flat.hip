@@ -16,13 +16,15 @@ void launch_flat(sddmm_ctx *c) {
     });
 }
 
-void launch_flat_blocks(sddmm_ctx *c) {
+// 0: no kernel for this row layout
+int launch_flat_blocks(sddmm_ctx *c) {
     const Shape s = shape_of(c);
     auto eighth = [](int64_t items) {                      // workgroups per XCD, rounded up twice
         const int64_t blocks = (items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
         return (blocks + NUM_XCD - 1) / NUM_XCD;
     };
     const int64_t grid = NUM_XCD * (eighth(c->block_segments_max) + eighth(c->block_gaps_max));
+    int launches = 0;
     with_layout(s, [&](auto L) {
         using LT = decltype(L);
         if constexpr (!LT::LONG) {
@@ -30,11 +32,13 @@ void launch_flat_blocks(sddmm_ctx *c) {
                 SDDMM_LAUNCH(c, kernel, grid, BLOCK, (const void *)c->dA, (const void *)c->dB, s.len, entry_rows(c),
                              entry_cols(c), (const float *)c->d_sval, out, (const RowItem *)c->d_block_segments,
                              (const RowItem *)c->d_block_gaps, (const unsigned long long *)c->d_block_totals);
+                ++launches;
             };
             if (c->use_order) launch(k_flat_blocks<LT, false>, c->d_order_dots);
             else launch(k_flat_blocks<LT, true>, c->dP);
         }
     });
+    return launches;
 }
 
 void launch_unsort(sddmm_ctx *c) {

@@ -246,14 +246,9 @@ int classify_rows_items(sddmm_ctx *c) {
         if (c->use_short_list && c->n_short_list > c->short_list_cap) {
             dfree(c->d_short_list);
             c->short_list_cap = 0;
-            void *p = nullptr;
-            if (hipMalloc(&p, (size_t)c->n_short_list * sizeof(int2)) == hipSuccess && p) {
-                c->d_short_list = static_cast<decltype(c->d_short_list)>(p);
-                c->short_list_cap = c->n_short_list;
-            } else {
-                (void)hipGetLastError();                       // the failed allocation is not an error of the plan
-                c->use_short_list = false;
-            }
+            c->d_short_list = static_cast<int2 *>(spare_alloc((size_t)c->n_short_list * sizeof(int2)));
+            if (c->d_short_list) c->short_list_cap = c->n_short_list;
+            else c->use_short_list = false;
         }
         if (!c->use_short_list) c->n_short_list = 0;
     }
@@ -623,12 +618,8 @@ int plan_blocks(sddmm_ctx *c, bool cut_long_rows) {
     if (at > c->blocks_bytes) {
         dfree(c->d_blocks);
         c->blocks_bytes = 0;
-        void *p = nullptr;
-        if (hipMalloc(&p, at) != hipSuccess || !p) {
-            (void)hipGetLastError();                       // the failed allocation is not an error of the plan
-            return SDDMM_OK;
-        }
-        c->d_blocks = static_cast<char *>(p);
+        c->d_blocks = static_cast<char *>(spare_alloc(at));
+        if (!c->d_blocks) return SDDMM_OK;
         c->blocks_bytes = at;
     }
     char *b = c->d_blocks;
@@ -670,15 +661,9 @@ bool ensure_slice_workspace(sddmm_ctx *c) {
     const int64_t need = slice_workspace_floats(c);
     if (need <= c->part_floats) return true;
     dfree(c->d_part);
-    c->part_floats = 0;
-    void *p = nullptr;
-    if (hipMalloc(&p, (size_t)need * sizeof(float)) != hipSuccess || !p) {
-        (void)hipGetLastError();                           // the failed allocation is not an error of the plan
-        return false;
-    }
-    c->d_part = static_cast<float *>(p);
-    c->part_floats = need;
-    return true;
+    c->d_part = static_cast<float *>(spare_alloc((size_t)need * sizeof(float)));
+    c->part_floats = c->d_part ? need : 0;
+    return c->d_part != nullptr;
 }
 
 // Entries in no order: sort them by row and column block and plan the flat launch over that order.  Leaves use_order
@@ -701,22 +686,16 @@ int sort_order(sddmm_ctx *c, bool *done) {
     if (at > c->sort_tmp_bytes) {
         dfree(c->d_sort_tmp);
         c->sort_tmp_bytes = 0;
-        if (hipMalloc(&c->d_sort_tmp, at) != hipSuccess) {
-            (void)hipGetLastError();                       // the failed allocation is not an error of the plan
-            c->d_sort_tmp = nullptr;
-            return SDDMM_OK;
-        }
+        c->d_sort_tmp = spare_alloc(at);
+        if (!c->d_sort_tmp) return SDDMM_OK;
         c->sort_tmp_bytes = at;
     }
     if (c->nnz > c->order_cap) {
         const size_t column = (n * 4 + 255) & ~(size_t)255;
         dfree(c->d_order);
         c->order_cap = 0;
-        if (hipMalloc((void **)&c->d_order, 4 * column) != hipSuccess) {
-            (void)hipGetLastError();
-            c->d_order = nullptr;
-            return SDDMM_OK;
-        }
+        c->d_order = static_cast<int32_t *>(spare_alloc(4 * column));
+        if (!c->d_order) return SDDMM_OK;
         c->order_cap = c->nnz;
         c->d_order_row = c->d_order;
         c->d_order_col = c->d_order + column / 4;
@@ -761,8 +740,11 @@ int plan_order(sddmm_ctx *c) {
     c->use_order = true;
     c->use_slices = slices_pay(c, avg_len) && ensure_slice_workspace(c);
     if (!c->use_slices) {
-        rc = plan_blocks(c, blocks_pay(c));
-        if (rc) return rc;
+        // (rows beyond the register layout came here for the slices alone: without their workspace, the plain kernel)
+        if (shape_of(c).LPN != 0) {
+            rc = plan_blocks(c, blocks_pay(c));
+            if (rc) return rc;
+        }
         c->use_order = c->use_blocks;
     }
     return SDDMM_OK;
@@ -822,8 +804,9 @@ int enqueue_run(sddmm_ctx *c) {
         }
         case SDDMM_FLAT:
             if (c->use_slices) c->launches = launch_flat_sliced(c);
-            else if (c->use_blocks) launch_flat_blocks(c);
-            else launch_flat(c);
+            else if (c->use_blocks) {
+                if (launch_flat_blocks(c) == 0) return fail(c, SDDMM_ERR_UNSUPPORTED, "internal: no column blocks for this row layout");
+            } else launch_flat(c);
             if (c->use_order) { launch_unsort(c); ++c->launches; }
             break;
         case SDDMM_ROW_WAVE: launch_row_wave(c, nullptr, c->sM); break;
@@ -1568,6 +1551,14 @@ int sddmm_get_values_device(sddmm_ctx *c, const float **dP) {
 int sddmm_last_stats(const sddmm_ctx *c, sddmm_stats *out) {
     if (!c || !out) return SDDMM_ERR_NULL;
     *out = c->stats;
+    return SDDMM_OK;
+}
+
+int sddmm_flat_variant(const sddmm_ctx *c, int *variant) {
+    if (!c || !variant) return SDDMM_ERR_NULL;
+    const bool flat = c->planned && c->strategy == SDDMM_FLAT;
+    *variant = !flat ? 0 : (c->use_slices ? SDDMM_FLAT_SLICES : 0) | (c->use_blocks ? SDDMM_FLAT_BLOCKS : 0) |
+                               (c->use_order ? SDDMM_FLAT_SORTED : 0);
     return SDDMM_OK;
 }
 

@@ -243,6 +243,14 @@ int sddmm_get_values(sddmm_ctx *ctx, float *P_values);
 /* Device address of P (nnz floats), valid until the next sddmm_set_* / destroy. */
 int sddmm_get_values_device(sddmm_ctx *ctx, const float **dP);
 int sddmm_last_stats(const sddmm_ctx *ctx, sddmm_stats *out);
+/* How the current plan runs the flat strategy that AUTO resolved to: a sum of the values below, 0
+ * for the plain kernel (always so when FLAT was asked for by name) and for other strategies. */
+enum sddmm_flat_variants {
+    SDDMM_FLAT_SLICES = 1,    /* one 128-byte line of every row per pass                    */
+    SDDMM_FLAT_BLOCKS = 2,    /* work items of the plan; long rows cut into column blocks   */
+    SDDMM_FLAT_SORTED = 4     /* entries in no order, sorted by the plan                    */
+};
+int sddmm_flat_variant(const sddmm_ctx *ctx, int *variant);
 
 /* ---- host helpers -------------------------------------------------------- */
 /* nnz-balanced contiguous row partition into `parts` ranges of whole `stride`-row
