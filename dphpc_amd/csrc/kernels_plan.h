@@ -522,16 +522,17 @@ static __global__ __launch_bounds__(256) void k_panel_items(const int32_t *__res
 // ---------------------------------------------------------------------------
 // Column blocks for the long rows of a flat matrix (kernels_flat.h, k_flat_blocks).
 //
-// Rows of more than `seg` entries, in row order (block_offsets: exclusive scan of the long_sums of
-// k_classify_count).
-static __global__ __launch_bounds__(SCAN_BLOCK) void k_long_rows(const int32_t *__restrict__ rowptr, int M, int seg,
+// Rows of several work items, in row order (block_offsets: exclusive scan of the long_sums of
+// k_classify_count, so a row is long here exactly when it is there: rows below `ts` never are).
+static __global__ __launch_bounds__(SCAN_BLOCK) void k_long_rows(const int32_t *__restrict__ rowptr, int M, int ts, int seg,
                                                                  const unsigned int *__restrict__ block_offsets,
                                                                  int32_t *__restrict__ long_rows) {
     const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
     unsigned int mine = 0, is_long = 0;
     for (int q = 0; q < SCAN_ITEMS; ++q) {
         const int64_t i = base + q;
-        const bool l = i < M && rowptr[i + 1] - rowptr[i] > seg;
+        unsigned int len;
+        const bool l = row_item_count(rowptr, nullptr, i, M, ts, seg, &len) > 1;
         is_long |= (l ? 1u : 0u) << q;
         mine += l ? 1u : 0u;
     }

@@ -630,7 +630,7 @@ int plan_blocks(sddmm_ctx *c, bool cut_long_rows) {
     unsigned int *seg_items = (unsigned int *)(b + o_seg[1]), *seg_off = (unsigned int *)(b + o_seg[2]);
     unsigned int *gap_items = (unsigned int *)(b + o_gap[1]), *gap_off = (unsigned int *)(b + o_gap[2]);
     if (n_long > 0) {
-        SDDMM_LAUNCH(c, k_long_rows, nb, SCAN_BLOCK, c->d_rowptr, c->sM, c->seg, (const unsigned int *)c->d_long_sums, rows);
+        SDDMM_LAUNCH(c, k_long_rows, nb, SCAN_BLOCK, c->d_rowptr, c->sM, c->ts, c->seg, (const unsigned int *)c->d_long_sums, rows);
         SDDMM_LAUNCH(c, k_long_segments, grid_for(n_seg, 256), 256, c->d_rowptr, entry_cols(c), c->sN, (const int32_t *)rows,
                      (int)n_long, (int)piece, seg_start, seg_items);
     }

@@ -70,3 +70,26 @@ def test_column_blocks(engine_factory, monkeypatch, K, dtype, kind):
         # a pattern without a long row after one with: the plain kernel again
         M, rowptr, col, val = _matrix(rng, short, N, kind)
         _check(e, M, N, rowptr, col, val, A_all[:M], B, dtype, "no long row")
+
+
+@pytest.mark.parametrize("ts", [1, 257, 258, 600, 100000])
+def test_rows_between_the_segment_length_and_the_short_row_limit(engine_factory, monkeypatch, ts):
+    """SDDMM_TS above SDDMM_SEG: the rows in between are no long rows anywhere, neither in the count that sizes the
+    list of the long rows nor in the list."""
+    monkeypatch.setenv("SDDMM_COLUMN_BLOCKS", "1")
+    monkeypatch.setenv("SDDMM_SLICES", "0")
+    monkeypatch.setenv("SDDMM_TS", str(ts))
+    N, K = 7001, 32
+    rng = np.random.default_rng(ts)
+    short = rng.integers(0, 9, 9000)                              # three blocks of the row scan
+    lens = np.concatenate([[256, 257, 258], short[:2000], rng.integers(255, 602, 60), short[2000:], [599, 600, 601, 2500]])
+    A = rng.uniform(-1, 1, (len(lens), K)).astype(f32)
+    B = rng.uniform(-1, 1, (N, K)).astype(f32)
+    with engine_factory() as e:
+        print("between", ts, flush=True)
+        M, rowptr, col, val = _matrix(rng, lens, N)
+        e.set_dense(A, B)
+        e.set_csr(M, N, rowptr, col, val)
+        e.plan(capi.AUTO)
+        assert e.flat_variant() == (capi.FLAT_BLOCKS if ts <= 2500 else 0)
+        _check(e, M, N, rowptr, col, val, A, B, capi.F32, "ts=%d" % ts)
