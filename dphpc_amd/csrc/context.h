@@ -326,6 +326,7 @@ inline int panel_mfma_steps(const sddmm_ctx *c) {
 void launch_flat(sddmm_ctx *c);                                                  // launch_flat.hip
 int launch_flat_blocks(sddmm_ctx *c);                                            // number of launches
 void launch_unsort(sddmm_ctx *c);
+void block_items_max(const sddmm_ctx *c, bool cut_long_rows, int64_t *segments, int64_t *gaps);
 bool blocks_pay(const sddmm_ctx *c);
 bool order_pays(const sddmm_ctx *c);
 bool slices_pay(const sddmm_ctx *c, double entries_per_row);

@@ -16,14 +16,30 @@ void launch_flat(sddmm_ctx *c) {
     });
 }
 
-// 0: no kernel for this row layout
-int launch_flat_blocks(sddmm_ctx *c) {
-    const Shape s = shape_of(c);
+namespace {
+
+// workgroups of a launch over at most `segments` and `gaps` work items: an eighth of either kind per XCD
+int64_t blocks_grid(int64_t segments, int64_t gaps) {
     auto eighth = [](int64_t items) {                      // workgroups per XCD, rounded up twice
         const int64_t blocks = (items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
         return (blocks + NUM_XCD - 1) / NUM_XCD;
     };
-    const int64_t grid = NUM_XCD * (eighth(c->block_segments_max) + eighth(c->block_gaps_max));
+    return NUM_XCD * (eighth(segments) + eighth(gaps));
+}
+
+}  // namespace
+
+// the most work items there can be, from the counts of the row classes
+void block_items_max(const sddmm_ctx *c, bool cut_long_rows, int64_t *segments, int64_t *gaps) {
+    const int64_t n_long = cut_long_rows ? (int64_t)c->pc.rows_long : 0, nnz_long = cut_long_rows ? (int64_t)c->pc.nnz_long : 0;
+    *segments = nnz_long / c->seg + n_long * COL_BLOCKS;
+    *gaps = (c->nnz - nnz_long) / WAVE + n_long + 1;
+}
+
+// 0: no kernel for this row layout
+int launch_flat_blocks(sddmm_ctx *c) {
+    const Shape s = shape_of(c);
+    const int64_t grid = blocks_grid(c->block_segments_max, c->block_gaps_max);
     int launches = 0;
     with_layout(s, [&](auto L) {
         using LT = decltype(L);
@@ -53,6 +69,9 @@ void launch_unsort(sddmm_ctx *c) {
 bool blocks_pay(const sddmm_ctx *c) {
     const int mode = env_int("SDDMM_COLUMN_BLOCKS", -1);            // -1: decide here, 0: never, 1: wherever there are long rows
     if (shape_of(c).LPN == 0 || c->pc.rows_long == 0) return false;
+    int64_t segments, gaps;                                         // (a launch takes fewer than 2^32 threads)
+    block_items_max(c, true, &segments, &gaps);
+    if (blocks_grid(segments, gaps) * BLOCK >= (int64_t)1 << 32) return false;
     if (mode >= 0) return mode != 0;
     const double b_bytes = (double)c->N * (double)c->K * (double)elem_size(c->dtype);
     return b_bytes >= 12.0 * (1 << 20) && c->nnz >= (1 << 20) && (double)c->pc.nnz_long >= 0.25 * (double)c->nnz;

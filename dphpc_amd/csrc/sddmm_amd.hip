@@ -597,13 +597,11 @@ int ensure_rowidx(sddmm_ctx *c) {
 // need no cutting).
 int plan_blocks(sddmm_ctx *c, bool cut_long_rows) {
     const int64_t n_long = cut_long_rows ? (int64_t)c->pc.rows_long : 0, nb = ((int64_t)c->sM + SCAN_TILE - 1) / SCAN_TILE;
-    const int64_t nnz_long = cut_long_rows ? (int64_t)c->pc.nnz_long : 0;
     if (cut_long_rows && (int64_t)c->raw.long_scanned != n_long)
         return fail(c, SDDMM_ERR_HIP, "internal: scan of the long rows disagrees with their number");
     const int64_t n_seg = n_long * COL_BLOCKS, n_gap = n_long + 1;
     const int64_t piece = c->seg, gap_piece = WAVE;
-    c->block_segments_max = nnz_long / piece + n_seg;
-    c->block_gaps_max = (c->nnz - nnz_long) / gap_piece + n_gap;
+    block_items_max(c, cut_long_rows, &c->block_segments_max, &c->block_gaps_max);
     size_t at = 0;
     auto take = [&](size_t bytes) {
         const size_t here = at;
