@@ -322,6 +322,20 @@ inline int panel_mfma_steps(const sddmm_ctx *c) {
     return (steps == 1 || steps == 2 || steps == 4 || steps == 8 || steps == 16) ? steps : 0;
 }
 
+// The device code of a translation unit is loaded when something first asks for one of its kernels: 3 .. 13 ms, once per
+// process.  A plan asks for the families that its launches take (load_*, one per launch_*.hip), so that no launch has to:
+// launches may be captured, and they are what callers time.
+inline hipError_t load_code(const void *kernel) {
+    hipFuncAttributes a;
+    return hipFuncGetAttributes(&a, kernel);
+}
+hipError_t load_flat();
+hipError_t load_rows();
+hipError_t load_auto();
+hipError_t load_tiles();
+hipError_t load_panels();
+hipError_t load_fused();
+
 // ---- launchers, one translation unit per family of kernels ----
 void launch_flat(sddmm_ctx *c);                                                  // launch_flat.hip
 int launch_flat_blocks(sddmm_ctx *c);                                            // number of launches

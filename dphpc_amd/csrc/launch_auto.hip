@@ -16,3 +16,5 @@ void launch_auto(sddmm_ctx *c) {
                            (const int2 *)(c->use_short_list ? c->d_short_list : nullptr), c->n_short_list);
     });
 }
+
+hipError_t load_auto() { return load_code(reinterpret_cast<const void *>(k_auto<Layout<UnitF32x1, 4, 1, false, false>>)); }

@@ -171,3 +171,5 @@ int launch_flat_sliced(sddmm_ctx *c) {
     if (c->dtype == SDDMM_F16) return launch_slices_u<UnitF16x8>(c);
     return launch_slices_u<UnitF32x4>(c);
 }
+
+hipError_t load_flat() { return load_code(reinterpret_cast<const void *>(k_unsort)); }

@@ -48,3 +48,5 @@ int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
     });
     return launches;
 }
+
+hipError_t load_fused() { return load_code(reinterpret_cast<const void *>(k_fusedmm<Layout<UnitF32x4, 8, 1, true, false>>)); }

@@ -70,3 +70,5 @@ void launch_panels_fused(sddmm_ctx *c) {
         else launch_panel_fused_t<DT_F16, 4>(c);
     }
 }
+
+hipError_t load_panels() { return load_code(reinterpret_cast<const void *>(k_panel_mfma<DT_F32, 2>)); }

@@ -23,3 +23,5 @@ void launch_short_rows(sddmm_ctx *c, int ts, int rpw) {
                            c->sM, ts, rpw, nblocks);
     });
 }
+
+hipError_t load_rows() { return load_code(reinterpret_cast<const void *>(k_row_wave<Layout<UnitF32x1, 4, 1, false, false>>)); }

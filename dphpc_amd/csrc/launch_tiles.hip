@@ -81,3 +81,5 @@ void launch_tiles(sddmm_ctx *c) {
     else if (c->dtype == SDDMM_F16) launch_tile_steps<DT_F16>(c);
     else launch_tile_steps<DT_F32>(c);
 }
+
+hipError_t load_tiles() { return load_code(reinterpret_cast<const void *>(k_tile<DT_F32, 1>)); }

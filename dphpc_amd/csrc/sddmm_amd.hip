@@ -966,6 +966,21 @@ int do_plan(sddmm_ctx *c, int strategy) {
     return SDDMM_OK;
 }
 
+// Device code of every kernel that enqueue_run may launch under this plan.
+int load_planned(sddmm_ctx *c) {
+    switch (c->strategy) {
+        case SDDMM_FLAT: HIP_TRY(c, load_flat()); break;
+        case SDDMM_ROW_WAVE:
+        case SDDMM_SHORT_ROWS: HIP_TRY(c, load_rows()); break;
+        case SDDMM_EXACT: break;                           // (k_exact comes with the plan kernels)
+        default:
+            if (c->tiles_active && c->n_tiles > 0) HIP_TRY(c, load_tiles());
+            if (c->n_panel_items > 0) HIP_TRY(c, load_panels());
+            if (c->rows_short > 0 || c->n_items > 0) HIP_TRY(c, load_auto());
+    }
+    return SDDMM_OK;
+}
+
 void fill_model(sddmm_ctx *c) {
     sddmm_stats &s = c->stats;
     s.strategy_used = c->strategy;
@@ -1269,7 +1284,11 @@ int sddmm_plan(sddmm_ctx *c, int strategy) {
     c->stats = sddmm_stats{};
     c->stats.plan_ms = ms;
     fill_model(c);
-    return SDDMM_OK;
+    if (c->nnz > 0) {
+        rc = load_planned(c);
+        if (rc) c->planned = false;
+    }
+    return rc;
 }
 
 int sddmm_launch(sddmm_ctx *c) {
@@ -1420,6 +1439,10 @@ int sddmm_run_fused(sddmm_ctx *c) {
         c->o_cap = 0;
         ALLOC_TRY(c, c->dO, o_bytes);
         c->o_cap = o_bytes;
+    }
+    if (c->nnz > 0) {
+        HIP_TRY(c, load_fused());
+        if (panels) HIP_TRY(c, load_panels());
     }
     HIP_TRY(c, hipEventRecord(c->ev0, c->stream));
     // (when the panels own every row that has entries, O is complete after a memset and the panel kernel;
@@ -1575,7 +1598,7 @@ constexpr int NOALLOC_MAX_DEVICES = 64;
 int32_t *g_scratch_ptr[NOALLOC_MAX_DEVICES] = {nullptr};   // device address of `scratch`, per device
 std::mutex g_scratch_mu;
 
-// Device address of the current device's copy of `scratch` (looked up once per device).
+// Device address of the current device's copy of `scratch` (looked up once per device, when the flat kernels are loaded too).
 int scratch_of_current_device(int *device, int32_t **ptr) {
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0) return SDDMM_ERR_NO_DEVICE;
@@ -1584,7 +1607,7 @@ int scratch_of_current_device(int *device, int32_t **ptr) {
     if (!g_scratch_ptr[dev]) {
         void *p = nullptr;
         const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (e != hipSuccess || !p) return SDDMM_ERR_HIP;
+        if (e != hipSuccess || !p || load_flat() != hipSuccess) return SDDMM_ERR_HIP;
         g_scratch_ptr[dev] = static_cast<int32_t *>(p);
     }
     *device = dev;

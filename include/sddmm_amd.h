@@ -174,7 +174,9 @@ int sddmm_plan(sddmm_ctx *ctx, int strategy);
 int sddmm_run(sddmm_ctx *ctx);
 /* Enqueue on the context's stream without waiting / wait for it.  On a planned
  * context sddmm_launch only enqueues kernels (no allocation, copy, fill or wait), so
- * it may be recorded into a HIP graph on a lent stream under capture. */
+ * it may be recorded into a HIP graph on a lent stream under capture.  The plan also
+ * loads the device code of those kernels (the first plan of a process that takes a
+ * family of kernels is 3 to 13 ms longer; stats.plan_ms does not include it). */
 int sddmm_launch(sddmm_ctx *ctx);
 int sddmm_synchronize(sddmm_ctx *ctx);
 /* warmup untimed launches, then reps launches each bracketed by HIP events on the
@@ -198,7 +200,8 @@ int sddmm_time_region(sddmm_ctx *ctx, int reps, int include_plan, float *total_m
  * (SDDMM_NOALLOC_MAX_NNZ int32 = 64 MiB per device, held until the process ends) instead
  * of an allocated buffer.  It calls no hipMalloc, hipFree or other allocating routine and
  * waits for nothing.  The first call on a device looks up that device's copy of the
- * array (hipGetSymbolAddress): make it outside a graph capture (nnz = 0 will do).
+ * array (hipGetSymbolAddress) and loads the kernels: make it outside a graph capture
+ * (nnz = 0 will do).
  *   - dA [M x K], dB [N x K] row-major fp32, 16-byte aligned; d_rowptr[M+1], d_col[nnz],
  *     d_sval[nnz], dP[nnz]; P is complete when `stream` has executed the call;
  *   - the structure is NOT validated here (that needs a read-back): pass arrays that
