@@ -141,6 +141,9 @@ struct sddmm_ctx {
     bool fused_items_panels = false; // the fused items leave out the rows that the panel kernel owns
     double fused_short_avg = 0.0;    // entries per non-empty row of at most FUSED_ROW_MAX entries (panel rows apart)
     int fused_row_max = FUSED_ROW_MAX;   // rows beyond it are work items of their own
+    int fused_seg = 0;               // of at most so many entries
+    float *d_fused_parts = nullptr;  // partial output rows of the pieces of the rows cut into several items
+    int64_t n_fused_pieces = 0, fused_part_floats = 0;
     float *dO = nullptr;
     size_t o_cap = 0;
     bool have_fused = false;

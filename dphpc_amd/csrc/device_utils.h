@@ -101,7 +101,7 @@ struct RowItem {
     int32_t row;
     int32_t start;
     int32_t end;
-    int32_t pad;
+    int32_t extra;     // panels: where the first row starts; fused items: place of a cut row's piece (k_piece_places)
 };
 
 // ---- units of the K dimension ----------------------------------------------

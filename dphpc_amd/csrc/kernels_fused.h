@@ -14,20 +14,84 @@
 // of the gather kernels: groups of LPN lanes, lane j of a group holds units
 // j, j+LPN, ... of the A row, of the entry's B row and of the group's partial output
 // row.  After the last entry the partial rows of the 64/LPN groups are added with
-// lane permutes; group 0 writes the output row, or adds it atomically when the row
-// was split into several items (O is cleared before the launch).
+// lane permutes; group 0 writes the output row, or, when the row was cut into several
+// items, the partial row of its piece.  The kernel of the short rows, launched after it,
+// adds the pieces of a row in order (add_pieces): O is the same in every run.
 #pragma once
 #include "kernels_gather.h"
 
 namespace sddmm {
+
+// The output row of a row that k_fusedmm cut into n pieces, by the whole wavefront: lane group g adds pieces g, g + G,
+// .. and the groups are added with lane permutes, the same order in every run.  Until then the row of O holds the place of
+// its first piece.
+template <class L>
+__device__ __forceinline__ void add_pieces(const float *__restrict__ parts, float *__restrict__ O, int KU, int64_t row,
+                                           int n, int lane) {
+    using U = typename L::U;
+    constexpr int E = U::ELEMS, LPN = L::LPN, UPL = L::UPL, G = WAVE / LPN;
+    using C = Chunk<U, L::LPN, L::UPL, L::FULLK, false, L::WIDE>;
+    const int g = lane / LPN, j = lane & (LPN - 1);
+    const int64_t K = (int64_t)KU * E;
+    float *orow = O + row * K;
+    const float *part = parts + (int64_t)__float_as_int(*orow) * K;
+    float acc[UPL][E];
+#pragma unroll
+    for (int i = 0; i < UPL; ++i)
+#pragma unroll
+        for (int e = 0; e < E; ++e) acc[i][e] = 0.f;
+#pragma unroll 4
+    for (int p = g; p < n; p += G) {
+#pragma unroll
+        for (int i = 0; i < UPL; ++i) {
+            const int u = C::unit_on(j, i, KU) ? j + i * LPN : 0;      // (a lane without a unit adds one it does not write)
+#pragma unroll
+            for (int e = 0; e < E; e += 4) {
+                const float4 v = *reinterpret_cast<const float4 *>(part + p * K + E * u + e);
+                acc[i][e] += v.x; acc[i][e + 1] += v.y; acc[i][e + 2] += v.z; acc[i][e + 3] += v.w;
+            }
+        }
+    }
+#pragma unroll
+    for (int off = LPN; off < WAVE; off <<= 1) {
+#pragma unroll
+        for (int i = 0; i < UPL; ++i)
+#pragma unroll
+            for (int e = 0; e < E; ++e) acc[i][e] += __shfl_xor(acc[i][e], off, WAVE);
+    }
+    if (g == 0) {
+#pragma unroll
+        for (int i = 0; i < UPL; ++i) {
+            const int u = j + i * LPN;
+            if (!C::unit_on(j, i, KU)) continue;
+#pragma unroll
+            for (int e = 0; e < E; e += 4)
+                *reinterpret_cast<float4 *>(orow + E * u + e) =
+                    make_float4(acc[i][e], acc[i][e + 1], acc[i][e + 2], acc[i][e + 3]);
+        }
+    }
+}
+
+// the cut rows among those of a wavefront, one after the other (cut: the lane's row was cut, of `len` entries)
+template <class L>
+__device__ __forceinline__ void add_cut_rows(const float *__restrict__ parts, float *__restrict__ O, int KU, bool cut,
+                                             int64_t row, int len, int seg, int lane) {
+    unsigned long long todo = __ballot(cut);
+    while (todo) {                                    // wave-uniform
+        const int src = __ffsll((long long)todo) - 1;
+        todo &= todo - 1;
+        const int n = (int)(((unsigned int)__shfl(len, src, WAVE) + (unsigned int)seg - 1u) / (unsigned int)seg);
+        add_pieces<L>(parts, O, KU, (int64_t)shfl_off<uint64_t>((uint64_t)row, src), n, lane);
+    }
+}
 
 template <class L>
 __global__ __launch_bounds__(BLOCK) void k_fusedmm(const void *__restrict__ A, const void *__restrict__ B, int KU,
                                                    const int32_t *__restrict__ rowptr,
                                                    const int32_t *__restrict__ col,
                                                    const float *__restrict__ sval, float *__restrict__ P,
-                                                   float *__restrict__ O, const RowItem *__restrict__ items,
-                                                   int64_t n_items, int64_t nblocks) {
+                                                   float *__restrict__ O, float *__restrict__ parts,
+                                                   const RowItem *__restrict__ items, int64_t n_items, int64_t nblocks) {
     using U = typename L::U;
     using T = typename U::T;                          // 16 bytes: 4 fp32 or 8 bf16 / fp16
     constexpr int E = U::ELEMS;
@@ -163,21 +227,18 @@ __global__ __launch_bounds__(BLOCK) void k_fusedmm(const void *__restrict__ A, c
             for (int e = 0; e < E; ++e) acc[i][e] += __shfl_xor(acc[i][e], off, WAVE);
     }
     if (g == 0) {
-        const bool whole_row = start == rowptr[row] && end == rowptr[row + 1];
-        float *orow = O + (int64_t)row * KU * E;
+        const int rs = rowptr[row];
+        const bool whole_row = start == rs && end == rowptr[row + 1];
+        float *orow = (whole_row ? O + (int64_t)row * KU * E : parts + (int64_t)it.extra * KU * E);
+        if (!whole_row && start == rs && lane == 0) O[(int64_t)row * KU * E] = __int_as_float(it.extra);
 #pragma unroll
         for (int i = 0; i < UPL; ++i) {
             const int u = j + i * LPN;
             if (!C::unit_on(j, i, KU)) continue;
-            if (whole_row) {
 #pragma unroll
-                for (int e = 0; e < E; e += 4)
-                    *reinterpret_cast<float4 *>(orow + E * u + e) =
-                        make_float4(acc[i][e], acc[i][e + 1], acc[i][e + 2], acc[i][e + 3]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < E; ++e) atomicAdd(orow + E * u + e, acc[i][e]);
-            }
+            for (int e = 0; e < E; e += 4)
+                *reinterpret_cast<float4 *>(orow + E * u + e) =
+                    make_float4(acc[i][e], acc[i][e + 1], acc[i][e + 2], acc[i][e + 3]);
         }
     }
 }
@@ -186,16 +247,18 @@ __global__ __launch_bounds__(BLOCK) void k_fusedmm(const void *__restrict__ A, c
 // consecutive rows, group g walks row r0+g.  Lane j of a group reads column index and
 // S value of entry t0+j, so LPN entries of each row are gathered back to back; the
 // P value of entry t0+j ends up in lane j, and the output row needs no reduction
-// across groups.  Longer rows are left to k_fusedmm and the rows of 8-row panels
-// (panel_owner[row] == 2, when the array is given) to the panel kernel: those rows count
-// as empty here and get a row of zeros, which the kernels launched after this one add to.
-// Every row below M gets its output row written, so O needs no clearing before the launch.
+// across groups.  Longer rows are left to k_fusedmm, launched before, and only their pieces
+// are added here (rows of more than seg entries).  The rows of 8-row panels (panel_owner[row]
+// == 2, when the array is given) are left to the panel kernel: they count as empty and get a
+// row of zeros, which that kernel, launched after this one, adds to.  Every row below M has
+// its output row written by one or the other, so O needs no clearing before the launches.
 template <class L>
 __global__ __launch_bounds__(BLOCK) void k_fusedmm_rows(const void *__restrict__ A, const void *__restrict__ B, int KU,
                                                         const int32_t *__restrict__ rowptr,
                                                         const int32_t *__restrict__ col,
                                                         const float *__restrict__ sval, float *__restrict__ P,
-                                                        float *__restrict__ O, int M, int max_len, int64_t nblocks,
+                                                        float *__restrict__ O, const float *__restrict__ parts, int M,
+                                                        int max_len, int seg, int64_t nblocks,
                                                         const unsigned char *__restrict__ panel_owner) {
     using U = typename L::U;
     using T = typename U::T;
@@ -212,13 +275,15 @@ __global__ __launch_bounds__(BLOCK) void k_fusedmm_rows(const void *__restrict__
     const int g = lane / LPN, j = lane & (LPN - 1);
     const int64_t row = r0 + g;
     int rs = 0, len = 0;
-    bool mine = false;
+    bool panel = false, is_long = false;              // the panel kernel takes the row, k_fusedmm took it
     if (row < M) {
         rs = rowptr[row];
         len = rowptr[row + 1] - rs;
-        mine = len <= max_len && !(panel_owner && panel_owner[row] == 2);
-        if (!mine) len = 0;
+        panel = panel_owner && panel_owner[row] == 2;
+        is_long = len > max_len && !panel;
     }
+    add_cut_rows<L>(parts, O, KU, j == 0 && is_long && len > seg, row, len, seg, lane);
+    if (panel || is_long) len = 0;
     int longest = len;
     for (int off = LPN; off < WAVE; off <<= 1) {
         const int o = __shfl_xor(longest, off, WAVE);
@@ -321,7 +386,7 @@ __global__ __launch_bounds__(BLOCK) void k_fusedmm_rows(const void *__restrict__
         cur = nxt;
         nxt = after;
     }
-    if (row < M) {                                    // (the accumulators of a row left to other kernels are zero)
+    if (row < M && !is_long) {                        // (the accumulators of a panel's row are zero)
         float *orow = O + row * KU * E;
 #pragma unroll
         for (int i = 0; i < UPL; ++i) {
@@ -345,14 +410,14 @@ __global__ __launch_bounds__(BLOCK) void k_fusedmm_rows(const void *__restrict__
 // value; step q then takes entry q with all lanes of the group, gathers the entry's A row with
 // its B row (the rows change inside a group, as in the flat kernel), and the group's partial
 // output row is written whenever the row changes.  Rows without entries of their own (empty,
-// left to other kernels) get zeros, as in k_fusedmm_rows.
+// left to the panel kernel) get zeros and the pieces of cut rows are added, as in k_fusedmm_rows.
 template <class L>
 __global__ __launch_bounds__(BLOCK) void k_fusedmm_rows_balanced(const void *__restrict__ A, const void *__restrict__ B,
                                                                  int KU, const int32_t *__restrict__ rowptr,
                                                                  const int32_t *__restrict__ col,
                                                                  const float *__restrict__ sval, float *__restrict__ P,
-                                                                 float *__restrict__ O, int M, int max_len,
-                                                                 int64_t nblocks,
+                                                                 float *__restrict__ O, const float *__restrict__ parts,
+                                                                 int M, int max_len, int seg, int64_t nblocks,
                                                                  const unsigned char *__restrict__ panel_owner) {
     using U = typename L::U;
     using T = typename U::T;
@@ -372,11 +437,15 @@ __global__ __launch_bounds__(BLOCK) void k_fusedmm_rows_balanced(const void *__r
     // lane l: row r0 + l
     const bool inside = r0 + lane < M;
     int rs = 0, len = 0;
+    bool panel = false, is_long = false;              // the panel kernel takes the row, k_fusedmm took it
     if (inside) {
         rs = rowptr[r0 + lane];
         len = rowptr[r0 + lane + 1] - rs;
-        if (len > max_len || (panel_owner && panel_owner[r0 + lane] == 2)) len = 0;
+        panel = panel_owner && panel_owner[r0 + lane] == 2;
+        is_long = len > max_len && !panel;
     }
+    add_cut_rows<L>(parts, O, KU, is_long && len > seg, r0 + lane, len, seg, lane);
+    if (panel || is_long) len = 0;
     int incl = len;
 #pragma unroll
     for (int o = 1; o < WAVE; o <<= 1) {
@@ -407,7 +476,7 @@ __global__ __launch_bounds__(BLOCK) void k_fusedmm_rows_balanced(const void *__r
     const Off_t rb = (Off_t)KU * (Off_t)sizeof(T);
     // rows with nothing of their own: zeros (lane group g takes rows g, g + G, ..)
     {
-        const unsigned long long empty = __ballot(inside && len == 0);
+        const unsigned long long empty = __ballot(inside && len == 0 && !is_long);
 #pragma unroll
         for (int k = 0; k < WAVE / G; ++k) {
             const int rr = k * G + g;

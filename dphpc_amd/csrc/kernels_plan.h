@@ -39,6 +39,7 @@ struct DevCounters {
     unsigned long long n_candidates;                                 // rows offered to the gathered strips
     unsigned long long utiles_scanned, short_scanned;                // scan totals: union strips, entries of the short rows
     unsigned long long long_scanned;                                 // scan total: rows of more than one item
+    unsigned long long fused_pieces;                                 // places given to the pieces of cut rows
     unsigned int max_len[SPREAD];
     unsigned long long k[K_KINDS][SPREAD];
 };
@@ -444,10 +445,36 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_write(const int3
         const int32_t s = rowptr[row], e = rowptr[row + 1];
         for (unsigned int k = 0; k < cnt[q]; ++k) {
             const int32_t a = s + (int32_t)k * seg;
-            const int32_t b = a + seg < e ? a + seg : e;
+            const int32_t b = e - a > seg ? a + seg : e;
             items[at++] = RowItem{row, a, b, 0};
         }
     }
+}
+
+// Places for the partial output rows of the fused call's pieces (kernels_fused.h): the pieces of a row that was cut
+// into several items lie next to each other, in order; which row comes first does not matter.  One thread per item,
+// the first item of a cut row writes the places of them all (they follow it in the list); one atomic per wavefront
+// that holds such an item.
+static __global__ __launch_bounds__(256) void k_piece_places(const int32_t *__restrict__ rowptr, RowItem *__restrict__ items,
+                                                             int64_t n_items, DevCounters *pc) {
+    const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    unsigned int n = 0;
+    if (w < n_items) {
+        const int row = items[w].row, start = items[w].start, end = items[w].end;
+        const int rs = rowptr[row], re = rowptr[row + 1];
+        if (start == rs && end != re) n = ((unsigned int)(re - rs) + (unsigned int)(end - start) - 1u) / (unsigned int)(end - start);
+    }
+    if (!__ballot(n != 0)) return;
+    const int lane = lane_id();
+    unsigned int incl = n;
+    for (int o = 1; o < WAVE; o <<= 1) {
+        const unsigned int up = __shfl_up(incl, o, WAVE);
+        if (lane >= o) incl += up;
+    }
+    unsigned int first = 0;
+    if (lane == WAVE - 1) first = (unsigned int)atomicAdd(&pc->fused_pieces, (unsigned long long)incl);
+    first = __shfl(first, WAVE - 1, WAVE) + incl - n;
+    for (unsigned int k = 0; k < n; ++k) items[w + k].extra = (int32_t)(first + k);
 }
 
 // ---------------------------------------------------------------------------

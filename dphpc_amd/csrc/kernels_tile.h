@@ -1872,7 +1872,7 @@ __global__ __launch_bounds__(panel_mfma_waves(STEPS) * WAVE, panel_mfma_min_wave
     // fp32 rows of 128 bytes and more: 4x4 blocks, every multiply-add useful (see above)
     constexpr bool BLOCKS = DT == DT_F32 && STEPS % 2 == 0;
     // the 8 rows of a panel have one length and follow each other in the CSR arrays
-    const int rs0 = __builtin_amdgcn_readfirstlane(it.pad);
+    const int rs0 = __builtin_amdgcn_readfirstlane(it.extra);
     const int row_len = __builtin_amdgcn_readfirstlane(rowptr[row0 + 1]) - rs0;
     const int64_t out_row = (int64_t)rs0 + (int64_t)prow * row_len;   // this lane's S/P row starts here
     // ROTATE: the S/P window of a row lags the compute window by `rot` 16-byte units, chosen so

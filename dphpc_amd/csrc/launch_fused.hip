@@ -2,7 +2,7 @@
 #include "context.h"
 #include "kernels_fused.h"
 
-// Rows of at most fused_row_max entries, then the work items of the longer ones; 0: no kernel for this row layout.
+// The work items of the rows of more than fused_row_max entries, then the other rows; 0: no kernel for this row layout.
 int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
     const Shape s = shape_of(c);
     // Short rows of fewer entries, on average, than half of what a lane group takes per step (a power-law
@@ -24,26 +24,28 @@ int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
             const int64_t rows_per_wave = WAVE / LT::LPN;
             const int64_t waves = ((int64_t)c->sM + rows_per_wave - 1) / rows_per_wave;
             const int64_t rblocks = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+            if (c->n_fused_items > 0) {
+                const int64_t nblocks = (c->n_fused_items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+                SDDMM_LAUNCH(c, (k_fusedmm<LT>), xcd_grid(nblocks), BLOCK,
+                                   (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col,
+                                   c->d_sval, c->dP, c->dO, c->d_fused_parts, (const RowItem *)c->d_fused_items,
+                                   c->n_fused_items, nblocks);
+                ++launches;
+            }
             if (balanced) {
                 const int64_t bwaves = ((int64_t)c->sM + WAVE - 1) / WAVE;
                 const int64_t bblocks = (bwaves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
                 SDDMM_LAUNCH(c, (k_fusedmm_rows_balanced<LT>), xcd_grid(bblocks), BLOCK,
                                    (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col, c->d_sval,
-                                   c->dP, c->dO, c->sM, c->fused_row_max, bblocks, panel_owner);
+                                   c->dP, c->dO, (const float *)c->d_fused_parts, c->sM, c->fused_row_max,
+                                   c->fused_seg, bblocks, panel_owner);
             } else {
                 SDDMM_LAUNCH(c, (k_fusedmm_rows<LT>), xcd_grid(rblocks), BLOCK,
                                    (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col, c->d_sval,
-                                   c->dP, c->dO, c->sM, c->fused_row_max, rblocks, panel_owner);
+                                   c->dP, c->dO, (const float *)c->d_fused_parts, c->sM, c->fused_row_max,
+                                   c->fused_seg, rblocks, panel_owner);
             }
             ++launches;
-            if (c->n_fused_items > 0) {
-                const int64_t nblocks = (c->n_fused_items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-                SDDMM_LAUNCH(c, (k_fusedmm<LT>), xcd_grid(nblocks), BLOCK,
-                                   (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col,
-                                   c->d_sval, c->dP, c->dO, (const RowItem *)c->d_fused_items, c->n_fused_items,
-                                   nblocks);
-                ++launches;
-            }
         }
     });
     return launches;

@@ -118,6 +118,8 @@ void release_sparse(sddmm_ctx *c) {
     c->use_order = false;
     dfree(c->d_fused_items);
     c->n_fused_items = c->fused_items_cap = 0;
+    dfree(c->d_fused_parts);
+    c->n_fused_pieces = c->fused_part_floats = 0;
     c->fused_items_valid = c->have_fused = false;
     c->owner_cap = c->panels_cap = c->panel_items_cap = 0;
     c->n_panel_items = c->n_panels = c->nnz_panels = 0;
@@ -1334,21 +1336,30 @@ int sddmm_run(sddmm_ctx *c) {
     return SDDMM_OK;
 }
 
+// Room for the partial output rows of the pieces (K floats each); false when the device does not have it.
+static bool fused_parts(sddmm_ctx *c) {
+    const int64_t need = c->n_fused_pieces * c->K;
+    if (need <= c->fused_part_floats) return true;
+    dfree(c->d_fused_parts);
+    c->d_fused_parts = static_cast<float *>(spare_alloc((size_t)need * sizeof(float)));
+    c->fused_part_floats = c->d_fused_parts ? need : 0;
+    return c->d_fused_parts != nullptr;
+}
+
 // items of the fused kernel: the rows of more than fused_row_max entries, cut into segments of
-// SDDMM_FUSED_SEG entries (default 1024, shortened below when there are few entries; a knob of its own,
-// apart from SDDMM_SEG of the plain SDDMM, because the pieces of a row add to O atomically: the segment
-// length decides which rows are summed in an order that may differ from run to run)
+// SDDMM_FUSED_SEG entries (default 1024, shortened below when there are few entries)
 static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
-    if (c->fused_items_valid && c->fused_items_panels == (panel_owner != nullptr)) return SDDMM_OK;
+    if (c->fused_items_valid && c->fused_items_panels == (panel_owner != nullptr) && fused_parts(c)) return SDDMM_OK;
     int seg = std::max(WAVE, env_int("SDDMM_FUSED_SEG", 1024));
     const int64_t nb = ((int64_t)c->sM + SCAN_TILE - 1) / SCAN_TILE;
     int row_max = FUSED_ROW_MAX;
     const int arc = ensure_arena(c);
     if (arc) return arc;
     ARENA_HOLDS(c, nb, c->block_sums_cap, "block sums");
-    c->n_fused_items = 0;
+    c->n_fused_items = c->n_fused_pieces = 0;
     if (nb > 0) {
         DevCounters tmp;
+        PlanCounters counted;
         auto count = [&]() -> int {
             HIP_TRY(c, hipMemsetAsync(&c->d_pc->k[K_ROWS_SHORT][0], 0,
                                       sizeof(unsigned long long) * SPREAD * (K_NNZ_LONG - K_ROWS_SHORT + 1), c->stream));
@@ -1361,18 +1372,18 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
             LAUNCH_CHECK(c);
             HIP_TRY(c, hipMemcpyAsync(&tmp, c->d_pc, sizeof(DevCounters), hipMemcpyDeviceToHost, c->stream));
             HIP_TRY(c, hipStreamSynchronize(c->stream));
+            counted = summarize(tmp);
             return SDDMM_OK;
         };
         int rc = count();
         if (rc) return rc;
-        const PlanCounters first = summarize(tmp);
+        const PlanCounters first = counted;
         const int64_t item_entries = (int64_t)(first.nnz_medium + first.nnz_long);
         c->fused_short_avg = first.rows_short ? (double)first.nnz_short / (double)first.rows_short : 0.0;
         // A wavefront walks its item chunk by chunk and the launch waits for the longest one: the long rows are
         // cut so that there are about 3 072 pieces, none shorter than 256 entries (graph of 50 k rows, 256-byte
         // rows: 2048 132 us, 512 59 us, 256 50 us; 200 k rows of 512 bytes: 2048 329, 1024 254, 512 246; 1 M rows
-        // of 128 bytes: 2048 306, 1024 293, 512 320, 256 407, the atomic adds of a piece cost what the cut
-        // returns).  Rows that are all about that long stay whole: 3 000 rows of 554 entries of 1 KiB 264 us, in
+        // of 128 bytes: 2048 306, 1024 293, 512 320, 256 407, where a piece costs what the cut returns).  Rows that are all about that long stay whole: 3 000 rows of 554 entries of 1 KiB 264 us, in
         // pieces of 512 280.
         int best_seg = seg;
         if (!getenv("SDDMM_FUSED_SEG")) {
@@ -1391,6 +1402,14 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
             rc = count();
             if (rc) return rc;
         }
+        // the pieces of the rows that are cut, at the most; without room for them every row stays whole
+        c->n_fused_pieces = (int64_t)counted.rows_long + (int64_t)counted.nnz_long / seg;
+        if (!fused_parts(c)) {
+            c->n_fused_pieces = 0;
+            seg = INT_MAX;
+            rc = count();
+            if (rc) return rc;
+        }
         c->n_fused_items = (int64_t)tmp.n_items;
         if (c->n_fused_items > c->fused_items_cap) {
             dfree(c->d_fused_items);
@@ -1400,10 +1419,16 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
         if (c->n_fused_items > 0) {
             SDDMM_LAUNCH(c, k_classify_write, nb, SCAN_BLOCK, c->d_rowptr,
                                panel_owner, c->sM, row_max + 1, seg, c->d_block_sums, c->d_fused_items, 2);
+            if (c->n_fused_pieces > 0) {
+                HIP_TRY(c, hipMemsetAsync(&c->d_pc->fused_pieces, 0, sizeof(unsigned long long), c->stream));
+                SDDMM_LAUNCH(c, k_piece_places, grid_for(c->n_fused_items, 256), 256, (const int32_t *)c->d_rowptr,
+                             c->d_fused_items, c->n_fused_items, c->d_pc);
+            }
             LAUNCH_CHECK(c);
         }
     }
     c->fused_row_max = row_max;
+    c->fused_seg = seg;
     c->fused_items_valid = true;
     c->fused_items_panels = panel_owner != nullptr;
     return SDDMM_OK;
@@ -1446,9 +1471,8 @@ int sddmm_run_fused(sddmm_ctx *c) {
     }
     HIP_TRY(c, hipEventRecord(c->ev0, c->stream));
     // (when the panels own every row that has entries, O is complete after a memset and the panel kernel;
-    // otherwise the kernel of the short rows, first in the stream, writes every row of O below sM, zeros
-
-    // for the rows that the kernels after it add to, and only the rows of A beyond S are cleared here)
+    // otherwise the kernels of the other rows write every row of O below sM, zeros for the panels' rows,
+    // and only the rows of A beyond S are cleared here)
     const bool others = c->sM > 0 && c->nnz > 0 && (!panels || c->n_tiles > 0 || c->rows_short > 0 || c->n_items > 0);
     if (o_bytes) {
         const size_t written = others ? (size_t)c->sM * (size_t)c->K * sizeof(float) : 0;

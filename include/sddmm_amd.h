@@ -227,13 +227,12 @@ int sddmm_launch_noalloc(int M, int N, int K, int64_t nnz, const float *dA, cons
  * (src/competitors/cpu/cpu_basic.hpp:18-51).  O is M x K fp32 row-major, owned by the
  * context.  Needs K <= 256, a multiple of 4 (fp32 operands) or 8 (bf16, fp16), and
  * row-sorted entries (CSR, or COO with non-decreasing rows); SDDMM_ERR_UNSUPPORTED otherwise.
- * Rows cut into several work items (longer than 2048 entries; longer than 256 where a
- * matrix of rows of up to 128 bytes has only a few thousand such rows) are accumulated
- * with atomic adds, so their last bits may differ from run to run.
+ * Long rows are cut into work items whose partial rows are added in a fixed order: O is the
+ * same, bit for bit, in every run of one plan, apart from the panels' rows:
  * K = 32, 64 or 128 (fp32, bf16 or fp16 operands): the rows that the current plan (SDDMM_AUTO
  * is planned if there is none) runs as 8-row panels take a matrix-core kernel that shares
  * every gathered B row between the 8 rows and between both products; the output rows of a
- * panel are accumulated with atomic adds as above.  The other rows take the gather kernels.
+ * panel are accumulated with atomic adds, so their last bits may differ from run to run.  The other rows take the gather kernels.
  * In either kernel a B row is read only for entries that are stored: a non-finite value in B
  * reaches the output rows that have an entry in its column and no others. */
 int sddmm_run_fused(sddmm_ctx *ctx);

@@ -1,0 +1,77 @@
+"""The fused call where rows are cut into several work items: O is the same bit for bit in every run, whatever the
+length at which rows are cut, with and without room for the pieces.  All GPU.  Same bar as test_gpu_fused.py."""
+import numpy as np
+import pytest
+
+from dphpc_amd import capi
+from oracle import oracle as O
+from test_gpu_fused import _check, _rounded
+
+pytestmark = pytest.mark.gpu
+f32 = np.float32
+
+
+def _matrix(rng, N, lens):
+    rows = [np.sort(rng.choice(N, int(n), replace=False)) for n in lens]
+    rowptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    return rowptr, np.concatenate(rows).astype(np.int32), rng.uniform(-1, 1, rowptr[-1]).astype(f32)
+
+
+def _operands(rng, M, N, K, dtype):
+    A, B = rng.uniform(-1, 1, (M, K)).astype(f32), rng.uniform(-1, 1, (N, K)).astype(f32)
+    return (A, A, B, B) if dtype == capi.F32 else _rounded(A, dtype) + _rounded(B, dtype)
+
+
+# one, two, three, four, six and eight units per lane, 1 .. 8 lanes per entry
+@pytest.mark.parametrize("K,dtype", [(4, capi.F32), (12, capi.F32), (32, capi.F32), (64, capi.F16), (96, capi.F32),
+                                     (128, capi.F32), (160, capi.F32), (192, capi.BF16), (256, capi.F32)])
+@pytest.mark.parametrize("env", [{}, {"SDDMM_FUSED_SEG": "64"}, {"SDDMM_FUSED_BALANCED": "1"}])
+def test_cut_rows_repeat(engine_factory, monkeypatch, K, dtype, env):
+    """Rows around the default cuts (256, 512, 1024) and of many pieces, in the first and the last wavefront."""
+    for name, value in env.items():
+        monkeypatch.setenv(name, value)
+    rng = np.random.default_rng(K)
+    N = 6000
+    lens = np.concatenate([[2048, 256, 257, 3], rng.integers(0, 9, 300), [511, 512, 513, 1024, 1025, 5600, 64, 65, 0],
+                           rng.integers(0, 9, 40), [1700, 1]])
+    M = len(lens)
+    rowptr, col, val = _matrix(rng, N, lens)
+    Ah, A, Bh, B = _operands(rng, M + 2, N, K, dtype)
+    print("cut rows", K, dtype, env, flush=True)
+    with engine_factory() as e:
+        e.set_dense(Ah, Bh, dtype)
+        e.set_csr(M, N, rowptr, col, val)
+        first = _check(e, rowptr, col, val, A, B, "K=%d %s" % (K, env))
+        for _ in range(20):
+            np.testing.assert_array_equal(e.run_fused(), first)
+
+
+def test_longer_rows_of_the_operands_under_the_same_items(engine_factory):
+    """The pattern stays, K grows: the pieces need more room."""
+    rng = np.random.default_rng(2)
+    N, lens = 3000, [900, 0, 7, 2900, 300]
+    rowptr, col, val = _matrix(rng, N, lens)
+    with engine_factory() as e:
+        A, _, B, _ = _operands(rng, 5, N, 8, capi.F32)
+        e.set_dense(A, B)
+        e.set_csr(5, N, rowptr, col, val)
+        for K in (8, 200, 16):
+            A, _, B, _ = _operands(rng, 5, N, K, capi.F32)
+            e.set_dense(A, B)
+            _check(e, rowptr, col, val, A, B, "K=%d" % K)
+
+
+def test_without_room_for_the_pieces(engine_factory, monkeypatch):
+    rng = np.random.default_rng(3)
+    N, lens = 6000, np.concatenate([[5000, 2], rng.integers(0, 20, 200), [600, 257, 70]])
+    rowptr, col, val = _matrix(rng, N, lens)
+    A, _, B, _ = _operands(rng, len(lens), N, 64, capi.F32)
+    monkeypatch.setenv("SDDMM_SPARE_BYTES", "0")
+    with engine_factory() as e:
+        e.set_dense(A, B)
+        e.set_csr(len(lens), N, rowptr, col, val)
+        first = _check(e, rowptr, col, val, A, B, "no room")
+        np.testing.assert_array_equal(e.run_fused(), first)
+        monkeypatch.delenv("SDDMM_SPARE_BYTES")
+        e.set_csr(len(lens), N, rowptr, col, val)
+        _check(e, rowptr, col, val, A, B, "room again")
