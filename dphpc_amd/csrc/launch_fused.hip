@@ -25,7 +25,7 @@ int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
             const int64_t waves = ((int64_t)c->sM + rows_per_wave - 1) / rows_per_wave;
             const int64_t rblocks = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
             if (c->n_fused_items > 0) {
-                const int64_t nblocks = (c->n_fused_items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+                const int64_t nblocks = fused_item_blocks(c->n_fused_items);
                 SDDMM_LAUNCH(c, (k_fusedmm<LT>), xcd_grid(nblocks), BLOCK,
                                    (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col,
                                    c->d_sval, c->dP, c->dO, c->d_fused_parts, (const RowItem *)c->d_fused_items,

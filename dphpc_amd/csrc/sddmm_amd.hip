@@ -1401,6 +1401,12 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
             row_max = best_row_max;
             rc = count();
             if (rc) return rc;
+            // (a launch takes fewer than 2^32 threads: 2^26 items, which rows of more than 64 entries cannot reach)
+            if (row_max != FUSED_ROW_MAX && xcd_grid(fused_item_blocks((int64_t)tmp.n_items)) * BLOCK >= (int64_t)1 << 32) {
+                row_max = FUSED_ROW_MAX;
+                rc = count();
+                if (rc) return rc;
+            }
         }
         // the pieces of the rows that are cut, at the most; without room for them every row stays whole
         c->n_fused_pieces = (int64_t)counted.rows_long + (int64_t)counted.nnz_long / seg;

@@ -69,3 +69,34 @@ def test_column_blocks_of_too_many_long_rows(engine_factory, monkeypatch):
         e.close()
         del A, B, S, rowptr, col, lens
         torch.cuda.empty_cache()
+
+
+def test_fused_call_with_too_many_rows_of_17_entries(engine_factory):
+    """69 M rows of 17 entries among shorter ones would be work items of the fused call, a wavefront each: beyond
+    2^26 of them they stay with the short rows."""
+    import torch
+    M, N, K = 161_000_000, 1_000_003, 4
+    lens = torch.where(torch.arange(M, device="cuda").remainder_(7) < 3, 17, 1).int()
+    assert int((lens == 17).sum()) > 1 << 26
+    rowptr, col, nnz = _matrix(torch, lens, N)
+    assert nnz < 8 * M                                                # mostly very short rows: 17 entries are long
+    A, B = _operands(torch, M, N, K)
+    S = torch.ones(nnz, device="cuda")
+    squares = torch.zeros(nnz + 1, dtype=torch.int64, device="cuda")
+    squares[1:] = torch.cumsum(col.remainder(128).long().square_(), 0)
+    want = (squares[rowptr[1:].long()] - squares[rowptr[:-1].long()]).float()
+    del squares, lens
+    torch.cuda.synchronize()
+    print("fused rows of 17", M, nnz, flush=True)
+    e = engine_factory()
+    try:
+        e._chk(e.L.sddmm_set_dense_device(e.h, M, N, K, A.data_ptr(), B.data_ptr(), capi.F32))
+        e._chk(e.L.sddmm_set_csr_device(e.h, M, N, nnz, rowptr.data_ptr(), col.data_ptr(), S.data_ptr()))
+        e.run_fused(fetch=False)
+        _check_p(_device_array(torch, e, e.L.sddmm_get_values_device, (nnz,)), col)
+        out = _device_array(torch, e, e.L.sddmm_get_fused_device, (M, K))
+        assert bool((out[:, 0] == want).all()) and not bool(out[:, 1:].any())
+    finally:
+        e.close()
+        del A, B, S, rowptr, col, want
+        torch.cuda.empty_cache()
