@@ -658,15 +658,16 @@ static __global__ __launch_bounds__(256) void k_order_keys(const int32_t *__rest
     keys[n] = (Key)row[n] * COL_BLOCKS + (Key)((int64_t)col[n] * COL_BLOCKS / N);
     at[n] = (int32_t)n;
 }
+// (32-bit keys lie in row_out, `at` lies in col_out: a thread reads its element of either before it writes there)
 template <class Key>
-static __global__ __launch_bounds__(256) void k_order_entries(const Key *__restrict__ keys, const int32_t *__restrict__ at,
+static __global__ __launch_bounds__(256) void k_order_entries(const Key *keys, const int32_t *at,
                                                               const int32_t *__restrict__ col, int64_t nnz,
-                                                              int32_t *__restrict__ row_out, int32_t *__restrict__ col_out,
+                                                              int32_t *row_out, int32_t *col_out,
                                                               int32_t *__restrict__ place) {
     const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= nnz) return;
-    const int32_t q = at[n];
-    row_out[n] = (int32_t)(keys[n] / COL_BLOCKS);
+    const int32_t q = at[n], row = (int32_t)(keys[n] / COL_BLOCKS);
+    row_out[n] = row;
     col_out[n] = col[q];
     place[q] = (int32_t)n;
 }

@@ -670,46 +670,45 @@ bool ensure_slice_workspace(sddmm_ctx *c) {
 // false when the device has no room.
 template <class Key>
 int sort_order(sddmm_ctx *c, bool *done) {
-    const size_t n = (size_t)c->nnz;
+    const size_t n = (size_t)c->nnz, column = (n * 4 + 255) & ~(size_t)255;
     int bits = 1;
     while (bits < 36 && ((int64_t)c->sM * COL_BLOCKS - 1) >> bits) ++bits;
-    // (the first buffers of either array hold the unsorted ones)
-    size_t at = 0, need = 0;
-    auto take = [&](size_t bytes) {
-        const size_t here = at;
-        at += (bytes + 255) & ~(size_t)255;
-        return here;
-    };
-    HIP_TRY(c, rocprim::radix_sort_pairs(nullptr, need, (Key *)nullptr, (Key *)nullptr, (int32_t *)nullptr, (int32_t *)nullptr, n,
-                                         0, bits, c->stream));
-    const size_t o_keys = take(n * sizeof(Key)), o_sorted = take(n * sizeof(Key)), o_from = take(n * 4), o_at = take(n * 4), o_tmp = take(need);
-    if (at > c->sort_tmp_bytes) {
-        dfree(c->d_sort_tmp);
-        c->sort_tmp_bytes = 0;
-        c->d_sort_tmp = spare_alloc(at);
-        if (!c->d_sort_tmp) return SDDMM_OK;
-        c->sort_tmp_bytes = at;
-    }
     if (c->nnz > c->order_cap) {
-        const size_t column = (n * 4 + 255) & ~(size_t)255;
         dfree(c->d_order);
         c->order_cap = 0;
         c->d_order = static_cast<int32_t *>(spare_alloc(4 * column));
         if (!c->d_order) return SDDMM_OK;
         c->order_cap = c->nnz;
-        c->d_order_row = c->d_order;
-        c->d_order_col = c->d_order + column / 4;
-        c->d_order_place = c->d_order + 2 * (column / 4);
-        c->d_order_dots = (float *)(c->d_order + 3 * (column / 4));
+    }
+    int32_t *part[4];
+    for (int i = 0; i < 4; ++i) part[i] = c->d_order + i * (column / 4);
+    // The sort works in the arrays of the order itself, 16 bytes per entry: the keys it ends with are overwritten by the
+    // rows, its values by the columns, the other buffer of either takes the places and the dot products.  64-bit keys
+    // (2^28 rows and more) have buffers of their own.
+    const size_t key_bytes = sizeof(Key) == 4 ? 0 : (n * sizeof(Key) + 255) & ~(size_t)255;
+    rocprim::double_buffer<Key> keys((Key *)part[0], (Key *)part[2]);
+    rocprim::double_buffer<int32_t> from(part[1], part[3]);
+    size_t need = 0;
+    HIP_TRY(c, rocprim::radix_sort_pairs(nullptr, need, keys, from, n, 0, bits, c->stream));
+    if (2 * key_bytes + need > c->sort_tmp_bytes) {
+        dfree(c->d_sort_tmp);
+        c->sort_tmp_bytes = 0;
+        c->d_sort_tmp = spare_alloc(2 * key_bytes + need);
+        if (!c->d_sort_tmp) return SDDMM_OK;
+        c->sort_tmp_bytes = 2 * key_bytes + need;
     }
     char *b = (char *)c->d_sort_tmp;
-    Key *keys = (Key *)(b + o_keys), *sorted = (Key *)(b + o_sorted);
-    int32_t *from = (int32_t *)(b + o_from), *sorted_from = (int32_t *)(b + o_at);
+    if (key_bytes) keys = rocprim::double_buffer<Key>((Key *)b, (Key *)(b + key_bytes));
     const int64_t grid = (c->nnz + 255) / 256;
-    SDDMM_LAUNCH(c, k_order_keys<Key>, grid, 256, (const int32_t *)c->d_rowidx, (const int32_t *)c->d_col, c->nnz, c->sN, keys, from);
+    SDDMM_LAUNCH(c, k_order_keys<Key>, grid, 256, (const int32_t *)c->d_rowidx, (const int32_t *)c->d_col, c->nnz, c->sN,
+                 keys.current(), from.current());
     LAUNCH_CHECK(c);
-    HIP_TRY(c, rocprim::radix_sort_pairs(b + o_tmp, need, keys, sorted, from, sorted_from, n, 0, bits, c->stream));
-    SDDMM_LAUNCH(c, k_order_entries<Key>, grid, 256, (const Key *)sorted, (const int32_t *)sorted_from,
+    HIP_TRY(c, rocprim::radix_sort_pairs(b + 2 * key_bytes, need, keys, from, n, 0, bits, c->stream));
+    c->d_order_row = key_bytes ? part[0] : (int32_t *)keys.current();
+    c->d_order_place = key_bytes ? part[2] : (int32_t *)keys.alternate();
+    c->d_order_col = from.current();
+    c->d_order_dots = (float *)from.alternate();
+    SDDMM_LAUNCH(c, k_order_entries<Key>, grid, 256, (const Key *)keys.current(), (const int32_t *)from.current(),
                  (const int32_t *)c->d_col, c->nnz, c->d_order_row, c->d_order_col, c->d_order_place);
     SDDMM_LAUNCH(c, k_rowptr_from_sorted_coo, grid_for(c->nnz + 1, 256), 256, (const int32_t *)c->d_order_row, c->nnz, c->sM,
                  c->d_rowptr);
@@ -733,6 +732,10 @@ int plan_order(sddmm_ctx *c) {
     rc = classify_rows_count(c);
     if (rc) return rc;
     rc = fetch_counters(c);
+    if (c->sort_tmp_bytes > ((size_t)16 << 20)) {          // (64-bit keys; the device is done with them)
+        dfree(c->d_sort_tmp);
+        c->sort_tmp_bytes = 0;
+    }
     if (rc) return rc;
     if (c->pc.bad_pattern) return fail(c, SDDMM_ERR_HIP, "internal: row pointer built from sorted entries is inconsistent");
     const double avg_len = c->pc.rows_nonempty ? (double)c->nnz / (double)c->pc.rows_nonempty : 0.0;

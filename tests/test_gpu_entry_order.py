@@ -135,3 +135,25 @@ def test_when_the_plan_sorts(engine_factory):
             st = e.stats()
             assert (st.strategy_used, st.kernels_launched) == (capi.FLAT, launches), name
             _check(e.values(), rr, cc, vv, a, b, name)
+
+
+def test_sorted_by_64_bit_keys(engine_factory, monkeypatch):
+    """2^28 rows and more: row and column block no longer fit 32 bits."""
+    monkeypatch.setenv("SDDMM_ORDER", "1")
+    rng = np.random.default_rng(28)
+    M, N = (1 << 28) + 100, 50
+    r = np.concatenate([rng.integers(0, M, 3000), np.arange(M - 60, M), [0, 0, 5], np.full(400, M - 7)])
+    r = rng.permutation(r).astype(np.int32)
+    c, v = rng.integers(0, N, len(r)).astype(np.int32), rng.uniform(-1, 1, len(r)).astype(f32)
+    A, B = np.zeros((M, 1), f32), rng.uniform(-1, 1, (N, 1)).astype(f32)
+    A[r, 0] = rng.uniform(-1, 1, len(r)).astype(f32)
+    print("2^28 rows", flush=True)
+    with engine_factory() as e:
+        e.set_dense(A, B)
+        e.set_coo(M, N, r, c, v)
+        e.plan(capi.AUTO)
+        assert e.flat_variant() == capi.FLAT_SORTED | capi.FLAT_BLOCKS
+        for _ in range(2):
+            e.run()
+            np.testing.assert_array_equal(e.values(), A[r, 0] * B[c, 0] * v)    # one product and its scaling: no sum
+            e.plan(capi.AUTO)

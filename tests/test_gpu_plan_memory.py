@@ -1,5 +1,7 @@
 """Arrays that a plan can do without, refused (SDDMM_SPARE_BYTES): the plan falls back to kernels that need none,
 with the oracle's values.  All GPU.  Same bar as test_gpu_parity.py."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -79,3 +81,33 @@ def test_csr(engine_factory, monkeypatch, K, env, variant):
             assert e.flat_variant() == (variant if limit is None else 0)
             e.run()
             _check(e.values(), r, c, v, A, B, "K=%d %s limit=%s" % (K, env, limit))
+
+
+def test_the_work_arrays_of_the_sort_are_given_back(engine_factory):
+    """A plan that sorts the entries keeps the sorted order, 16 bytes per entry, and not what the sort worked in."""
+    rng = np.random.default_rng(17)
+    rows, nnz, K = 40000, 3000000, 64
+    r, c = rng.integers(0, rows, nnz).astype(np.int32), rng.integers(0, rows, nnz).astype(np.int32)
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipMemGetInfo.argtypes = [C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]
+
+    def free():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+    with engine_factory() as e:
+        e.set_dense(rng.uniform(-1, 1, (rows, K)).astype(f32), rng.uniform(-1, 1, (rows, K)).astype(f32))
+        e.set_coo(rows, rows, r[:nnz // 2], c[:nnz // 2], np.ones(nnz // 2, f32))
+        e.plan(capi.AUTO)                                 # what a process pays for once
+        assert e.flat_variant() & capi.FLAT_SORTED
+        e.set_coo(rows, rows, r, c, np.ones(nnz, f32))
+        e.plan(capi.FLAT)
+        before = free()
+        e.plan(capi.AUTO)
+        assert e.flat_variant() == capi.FLAT_SORTED | capi.FLAT_BLOCKS
+        kept = before - free()
+        print("kept", kept / nnz, "bytes per entry", flush=True)
+        # 16 bytes and 0.3 for the work items; the arrays by rows and what the allocator rounds up to
+        assert kept < 17 * nnz + (8 << 20)
+        e.plan(capi.AUTO)                                 # planned again: the same
+        assert before - free() < 17 * nnz + (8 << 20)
