@@ -1,6 +1,8 @@
 """The flat kernel with the long rows cut into column blocks, forced on (small matrices): row lengths around
 the length that makes a row long, around whole pieces, long rows at either end and next to each other,
 columns in one block only, unsorted rows; against the oracle.  All GPU.  Same bar as test_gpu_parity.py."""
+import os
+
 import numpy as np
 import pytest
 
@@ -16,6 +18,8 @@ def _check(e, M, N, rowptr, col, val, A, B, dtype, what):
     e.set_csr(M, N, rowptr, col, val)
     e.plan(capi.AUTO)
     assert e.stats().strategy_used == capi.FLAT, what
+    longest, ts = int(np.diff(rowptr).max()), int(os.environ.get("SDDMM_TS", "24"))
+    assert e.flat_variant() == (capi.FLAT_BLOCKS if longest > 256 and longest >= ts else 0), what
     e.run()
     ref = O.sddmm_csr(rowptr, col, val, A, B, threads=0)
     _, mag = O.sddmm_csr_f64(rowptr, col, val, A, B)
@@ -93,3 +97,35 @@ def test_rows_between_the_segment_length_and_the_short_row_limit(engine_factory,
         e.plan(capi.AUTO)
         assert e.flat_variant() == (capi.FLAT_BLOCKS if ts <= 2500 else 0)
         _check(e, M, N, rowptr, col, val, A, B, capi.F32, "ts=%d" % ts)
+
+
+def test_when_the_plan_cuts_long_rows(engine_factory):
+    """The rule by itself, on either side of each of its lines: 12 MB of B, 2^20 entries, a quarter of them in rows of
+    more than 256."""
+    rng = np.random.default_rng(11)
+    N = 100000
+    lens = np.concatenate([np.full(1400, 300), np.full(80000, 8)])
+    rng.shuffle(lens)
+    fewer, shorter = lens.copy(), lens.copy()
+    fewer[np.flatnonzero(lens == 8)[:2000]] = 0                   # 1 044 000 entries
+    shorter[np.flatnonzero(lens == 300)[:600]] = 256              # 240 000 of 1 033 600 in long rows ..
+    shorter[np.flatnonzero(lens == 8)[:8000]] = 20                # .. of 1 129 600
+    cases = [("all three", lens, 32, capi.FLAT_BLOCKS), ("11.2 MB", lens, 28, 0), ("few entries", fewer, 32, 0),
+             ("few in long rows", shorter, 32, 0)]
+    with engine_factory() as e:
+        for name, lens_, K, variant in cases:
+            print(name, flush=True)
+            rowptr = np.concatenate([[0], np.cumsum(lens_)]).astype(np.int32)
+            nnz, M = int(rowptr[-1]), len(lens_)
+            assert (nnz >= 1 << 20) == (name != "few entries")
+            col = rng.integers(0, N, nnz).astype(np.int32)
+            A, B = rng.uniform(-1, 1, (M, K)).astype(f32), rng.uniform(-1, 1, (N, K)).astype(f32)
+            e.set_dense(A, B)
+            e.set_csr(M, N, rowptr, col, np.ones(nnz, f32))
+            e.plan(capi.AUTO)
+            assert (e.stats().strategy_used, e.flat_variant()) == (capi.FLAT, variant), name
+            e.run()
+            val = np.ones(nnz, f32)
+            ref = O.sddmm_csr(rowptr, col, val, A, B, threads=0)
+            ok, worst, i = O.check_values(e.values(), ref, mag=O.sddmm_csr_f64(rowptr, col, val, A, B)[1])
+            assert ok, "%s: entry %d (%.2f x tolerance)" % (name, i, worst)

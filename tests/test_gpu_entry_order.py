@@ -69,6 +69,13 @@ def test_sorted_order(engine_factory, monkeypatch, K, dtype, blocks):
                 got = e.values()
                 what = "%s K=%d slices=%s" % (name, K, slices)
                 assert st.strategy_used == capi.FLAT, what
+                size = 4 if dtype == capi.F32 else 2
+                sliced, in_registers = slices == "1" and K * size > 128, K * size <= 2048
+                variant = capi.FLAT_SLICES if sliced else 0
+                if (np.diff(r) < 0).any() and (sliced or in_registers):
+                    variant |= capi.FLAT_SORTED | (0 if sliced else capi.FLAT_BLOCKS)
+                assert e.flat_variant() == variant, what
+                assert st.kernels_launched == (2 if sliced else 1) + (1 if variant & capi.FLAT_SORTED else 0), what
                 _check(got, r, c, v, A, B, what)
                 if slices == "0":                        # the same arithmetic per entry as the plain kernel
                     e.set_coo(M, N, r, c, v)

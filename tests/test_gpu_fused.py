@@ -52,7 +52,7 @@ def test_fused_random(engine_factory, K):
 
 
 def test_fused_rows_split_into_segments(engine_factory, monkeypatch):
-    """Rows longer than a segment are accumulated by several wavefronts (atomic adds)."""
+    """Rows longer than a segment are cut into pieces for several wavefronts."""
     monkeypatch.setenv("SDDMM_FUSED_SEG", "128")
     rng = np.random.default_rng(31)
     M, N, K = 40, 3000, 32
