@@ -142,20 +142,46 @@ int launch_slices_u(sddmm_ctx *c) {
 
 }  // namespace
 
-// Measured on uniform random matrices of about 1 M entries, N = 1 000 .. 100 000, K = 64 .. 1 000 in fp32, 6 .. 60 entries
-// per row, against the better of k_flat and k_auto.  Slices gain where B exceeds the L2s (1.2 .. 2.2 times from 8 MB on;
-// 0.6 .. 1.1 times below 5 MB), as long as one slice of it comes near to fitting (N = 65 536 is 8 MB: 1.2; 100 000: 1.0) and
-// rows are several lines (256 bytes: 0.8 .. 1.1; 400 bytes: 1.0 .. 1.3).  Very short rows have their A rows gathered
-// per entry, which only pays while the slice fits (6 entries per row: 1.2 at N = 20 000, 0.8 .. 1.1 at 40 000).  Rows
-// beyond the register layout of the gather kernels (2 KB) gain everywhere: 1.3 times at the least.
+// Measured on uniform random matrices, against the better of the other kernels; in a loop / after a flush of the caches.
+// What slices gain is that a line of B is found in the L2 again, so it follows the size of B, the entries per column,
+// and the length of a row, which decides how well the other kernels do:
+//   up to 1 KB   entries per column:    4            8            12           24           48
+//     B of  9 MB (400 B rows)                   0.88 / 0.91   0.96 / 0.99   1.09 / 1.08   1.19 / 1.14
+//     B of 11 MB (600 B)           0.73 / 0.79  0.85 / 0.95   0.89 / 0.96   1.11 / 1.15   1.17 / 1.22   (first column: 6)
+//     B of 15 MB (400 B)           0.91 / 0.92  0.98 / 1.00   1.04 / 1.07   1.08 / 1.10   1.10 / 1.11
+//     B of 20 MB (1 KB)            1.11 / 0.87  1.27 / 0.94   1.39 / 1.05   1.65 / 1.25   1.70 / 1.32
+//     B of 39 MB (1 KB)            1.17 / 0.88  1.33 / 1.03   1.41 / 1.15   1.47 / 1.24   1.43 / 1.30
+//   (0.5 .. 2 per column: 0.5 .. 1.1 / 0.75 .. 1.2); hence 12 entries per column, 20 below 12 MB of B.
+//   1.25 .. 2 KB: 1.0 .. 2.3 / 1.0 .. 2.4 at 0.5 .. 48 entries per column; lowest 0.93 / 0.98 (1 per column, 122 MB of B).
+//   beyond 2 KB (no register layout): 1.4 times at the least.
+// From 32 entries per row on, the other kernel is the row split, which reads an A row once:
+//     entries per column:               2            6            12           24           48
+//     B of  9 MB (1 KB rows)        0.53 / 0.68  0.80 / 0.70  0.88 / 0.73  1.05 / 0.83  1.12 / 0.95
+//     B of 11 MB (600 B)            0.46 / 0.69  0.70 / 0.68  0.79 / 0.78  0.95 / 0.92  1.03 / 1.02
+//     B of 15 MB (400 B)            0.65 / 0.75  1.00 / 0.92  1.14 / 1.06  1.26 / 1.20  1.32 / 1.26
+//     B of 20 MB (1 KB)             0.74 / 0.63  1.05 / 0.73  1.22 / 0.93  1.46 / 1.15  1.67 / 1.32
+//     B of 24 MB (1.25 KB)          1.11 / 0.93  1.18 / 0.88  1.55 / 1.15  1.84 / 1.40  2.07 / 1.60
+//     B of 73 MB (1.9 KB)           1.03 / 0.83  1.46 / 1.19  1.68 / 1.43  1.85 / 1.65  1.85 / 1.77
+// hence 48 below 12 MB of B, 12 from there on, 8 with rows beyond 1 KB.
+// B has to exceed the L2s (0.6 .. 1.1 times below 5 MB) and one slice of it to come near to fitting (N = 65 536 is 8 MB:
+// 1.05 .. 1.25; 100 000: 1.0); rows of 256 bytes 0.8 .. 1.1.  Rows of fewer than 12 entries have their A rows gathered per
+// entry, which pays while the slice fits (6 entries per row: 40 000 columns 0.8 .. 1.1) and, up to 1 KB, with rows that are
+// long and columns of many entries only (6 .. 11 per row, 24 per column: 1 KB rows 1.24 / 0.94, 600 bytes 0.98 / 1.03).
 bool slices_pay(const sddmm_ctx *c, double entries_per_row) {
     const int64_t row_bytes = (int64_t)c->K * (int64_t)elem_size(c->dtype);
     const int mode = env_int("SDDMM_SLICES", -1);                   // -1: decide here, 0: never, 1: wherever the kernel can
     if (mode >= 0) return mode != 0 && row_bytes > SLICE_BYTES && row_bytes < (1 << 30);
     if (row_bytes > 2048) return row_bytes < (1 << 30);
-    const int64_t MB = 1 << 20;
-    return row_bytes >= 400 && (int64_t)c->N * row_bytes >= 8 * MB &&
-           (int64_t)c->N * SLICE_BYTES <= (entries_per_row >= 12.0 ? 8 * MB : 3 * MB);
+    const int64_t MB = 1 << 20, b_bytes = (int64_t)c->N * row_bytes;
+    const bool small_b = b_bytes < 12 * MB;
+    if (row_bytes < 400 || b_bytes < 8 * MB || (int64_t)c->N * SLICE_BYTES > (entries_per_row >= 12.0 ? 8 * MB : 3 * MB)) return false;
+    int per_column;
+    if (entries_per_row >= 32.0) per_column = small_b ? 48 : row_bytes > 1024 ? 8 : 12;
+    else if (row_bytes > 1024) return true;
+    else if (entries_per_row >= 12.0) per_column = small_b ? 20 : 12;
+    else if (row_bytes >= 1000) per_column = 24;
+    else return false;
+    return c->nnz >= per_column * (int64_t)c->sN;
 }
 
 // The partial products of all entries where they fit SLICE_WORKSPACE, of a range of entries at a time otherwise.

@@ -741,7 +741,8 @@ int plan_order(sddmm_ctx *c) {
     const double avg_len = c->pc.rows_nonempty ? (double)c->nnz / (double)c->pc.rows_nonempty : 0.0;
     c->pc.rows_nonempty = 0;                               // (reported as unknown without a row pointer of the caller's order)
     c->use_order = true;
-    c->use_slices = slices_pay(c, avg_len) && ensure_slice_workspace(c);
+    // (the other kernel here is the flat one, whatever the rows hold)
+    c->use_slices = slices_pay(c, std::min(avg_len, 31.0)) && ensure_slice_workspace(c);
     if (!c->use_slices) {
         // (rows beyond the register layout came here for the slices alone: without their workspace, the plain kernel)
         if (shape_of(c).LPN != 0) {

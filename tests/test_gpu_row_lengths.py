@@ -191,3 +191,38 @@ def test_operand_beyond_4gib(engine_factory, monkeypatch, K, slices):
     finally:
         e.close()
         hip.free_all()
+
+
+@pytest.mark.parametrize("K,N,per_row,fewer,enough", [
+    (256, 20000, 24, 11, 13),                             # 20 MB of B
+    (256, 9000, 24, 19, 21),                              # 9 MB
+    (100, 40000, 13, 11, 13),                             # 15 MB
+    (256, 20000, 6, 23, 25),                              # rows of few entries
+    (200, 20000, 6, 25, None),                            # and of 800 bytes
+    (300, 9000, 6, None, 1),                              # rows beyond 1 KB: whatever the columns hold
+    (256, 20000, 40, 11, 13),                             # against the row split: 20 MB of B
+    (300, 20000, 40, 7, 9),                               # rows beyond 1 KB
+    (256, 9000, 40, 47, 49),                              # 9 MB
+])
+def test_slices_where_the_columns_hold_enough_entries(engine_factory, monkeypatch, K, N, per_row, fewer, enough):
+    """The rule by itself: a line of B has to be found in the L2 often enough."""
+    rng = np.random.default_rng(K + N + per_row)
+    for per_column, variant in ((fewer, 0), (enough, capi.FLAT_SLICES)):
+        if per_column is None:
+            continue
+        M = N * per_column // per_row + 1
+        print("reuse", K, N, per_row, per_column, flush=True)
+        rowptr = (np.arange(M + 1) * per_row).astype(np.int32)
+        col = rng.integers(0, N, M * per_row).astype(np.int32)
+        val = np.ones(len(col), f32)
+        A, B = rng.uniform(-1, 1, (M, K)).astype(f32), rng.uniform(-1, 1, (N, K)).astype(f32)
+        with engine_factory() as e:
+            e.set_dense(A, B)
+            e.set_csr(M, N, rowptr, col, val)
+            e.plan(capi.AUTO)
+            assert e.flat_variant() == variant
+            assert e.stats().strategy_used == (capi.FLAT if variant or per_row < 32 else capi.AUTO)
+            e.run()
+            ref = O.sddmm_csr(rowptr, col, val, A, B, threads=0)
+            ok, worst, i = O.check_values(e.values(), ref, mag=O.sddmm_csr_f64(rowptr, col, val, A, B)[1])
+            assert ok, "%d per column: entry %d (%.2f x tolerance)" % (per_column, i, worst)
