@@ -17,7 +17,8 @@
 //
 // Per-entry arithmetic depends on K only (FMA chain over the lane's units in k
 // order, then the fixed tree of group_sum), so all strategies built from these
-// kernels return bit-identical values.
+// kernels return bit-identical values (k_slice_dots of kernels_flat.h does not: it
+// sums line by line of the B row).
 #pragma once
 #include "device_utils.h"
 

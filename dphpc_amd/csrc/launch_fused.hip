@@ -8,11 +8,11 @@ int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
     // Short rows of fewer entries, on average, than half of what a lane group takes per step (a power-law
     // graph: 2.8 against 8 lanes per entry) leave most lanes of a group idle in one row per lane group: the
     // wavefronts deal whole rows out to their groups by entry count instead.  That takes 64 rows per wavefront,
-    // so it needs enough rows to fill the chip: graphs of 2.6 M rows, 128 bytes 944 -> 787 us, 1 M rows,
-    // 256 bytes 442 -> 414 us, 500 k rows 147 -> 132 us; 200 k rows 86 -> 86 us (128 bytes), 215 -> 235 us
-    // (512 bytes); 50 k rows 40 -> 44 us, 8 k rows 14.5 -> 20 us.  With longer rows, or fewer lanes per entry,
-    // the extra gathers of the A rows and the longer walks cost more than the idle lanes (12.5 entries per
-    // short row: 33 -> 65 us; 1 M rows of 64 bytes 206 -> 239 us).
+    // so it needs enough rows to fill the chip: graphs of 2.6 M rows, 128 bytes 935 -> 781 us, 1 M rows 337 -> 287 us
+    // (256 bytes 593 -> 569), 500 k rows 169 -> 152 us; 200 k rows 66 -> 63 us (128 bytes), 217 -> 235 us (512
+    // bytes); 50 k rows 25 -> 32 us, 8 k rows 14 -> 23 us.  With longer rows, or fewer lanes per entry, the extra
+    // gathers of the A rows and the longer walks cost more than the idle lanes (12.5 entries per short row: 31 -> 64 us;
+    // 1 M rows of 64 bytes 249 -> 281 us).
     const int balanced_env = env_int("SDDMM_FUSED_BALANCED", -1);
     const bool balanced = balanced_env >= 0 ? balanced_env != 0
                                             : (c->sM >= 400000 && c->fused_short_avg > 0.0 &&

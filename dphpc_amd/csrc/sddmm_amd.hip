@@ -1385,9 +1385,10 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
         const int64_t item_entries = (int64_t)(first.nnz_medium + first.nnz_long);
         c->fused_short_avg = first.rows_short ? (double)first.nnz_short / (double)first.rows_short : 0.0;
         // A wavefront walks its item chunk by chunk and the launch waits for the longest one: the long rows are
-        // cut so that there are about 3 072 pieces, none shorter than 256 entries (graph of 50 k rows, 256-byte
-        // rows: 2048 132 us, 512 59 us, 256 50 us; 200 k rows of 512 bytes: 2048 329, 1024 254, 512 246; 1 M rows
-        // of 128 bytes: 2048 306, 1024 293, 512 320, 256 407, where a piece costs what the cut returns).  Rows that are all about that long stay whole: 3 000 rows of 554 entries of 1 KiB 264 us, in
+        // cut so that there are about 3 072 pieces, none shorter than 256 entries (pieces of 2048 / 1024 / 512 / 256:
+        // graph of 50 k rows, 256-byte rows, 124 / 74 / 47 / 35 us; 200 k rows of 512 bytes 269 / 220 / 214 / 202; 1 M
+        // rows of 128 bytes 301 / 287 / 278 / 274; 2.6 M rows 795 / 776 / 776 / 778, where a piece costs what the cut
+        // returns).  Rows that are all about that long stay whole: 3 000 rows of 554 entries of 1 KiB 264 us, in
         // pieces of 512 280.
         int best_seg = seg;
         if (!getenv("SDDMM_FUSED_SEG")) {
@@ -1396,9 +1397,10 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
             if ((int64_t)first.max_len > 2 * (int64_t)shorter) best_seg = shorter;
         }
         // Where most of the short rows are very short, one of 17 .. 64 entries among them holds up the rows of its
-        // wavefront: those become items too (graphs of 2.8 .. 4 entries per short row, 64 against 16: 200 k rows K=8
-        // 61 -> 44 us, K=64 fp16 95 -> 86 us; 1 M rows K=64 487 -> 442 us; 50 k rows 51 -> 40 us).  Rows of about one
-        // length stay: 42 .. 48 entries each, K=128 54 us, as items 84; 17 .. 23 entries 10.5 and 20 us.
+        // wavefront: those become items too (graphs of 2.8 .. 4 entries per short row, 64 against 16: 50 k rows K=64
+        // 46 -> 35 us; 200 k rows K=8 60 -> 44 us, K=64 fp16 92 -> 77, K=128 251 -> 218; 1 M rows K=64 606 -> 566;
+        // 2.6 M rows K=32 868 -> 780).  Rows of about one length stay: 42 .. 48 entries each, K=128 54 us, as items 84;
+        // 17 .. 23 entries 10.5 and 20 us.
         const int best_row_max = first.rows_short && c->fused_short_avg < 8.0 ? FUSED_ROW_MAX / 4 : FUSED_ROW_MAX;
         if (best_seg != seg || best_row_max != row_max) {
             seg = best_seg;
