@@ -356,5 +356,5 @@ bool launch_auto_with_tiles(sddmm_ctx *c);                                      
 void launch_tiles(sddmm_ctx *c);
 void launch_panels(sddmm_ctx *c);                                                // launch_panels.hip
 void launch_panels_fused(sddmm_ctx *c);
-inline int64_t fused_item_blocks(int64_t n_items) { return (n_items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK; }
+inline int64_t fused_item_blocks(int64_t n_items) { return (n_items + ITEM_WAVES - 1) / ITEM_WAVES; }
 int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner);           // launch_fused.hip: number of launches

@@ -26,6 +26,15 @@ namespace sddmm {
 
 constexpr int BLOCK = 256;                 // 4 wavefronts
 constexpr int WAVES_PER_BLOCK = BLOCK / WAVE;
+// Kernels of many short work items of different lengths take workgroups of one wavefront: a workgroup keeps its place on
+// the CU until its last wavefront ends, and with four items each the places are half empty (4.9 of 6 wavefronts per SIMD
+// on average in k_flat_blocks).  Against workgroups of four: graph of 2.6 M rows, K = 32, 554 -> 527 us; 200 000 rows
+// K = 32 30.3 -> 28.0, K = 64 56.7 -> 54.9; k_auto, 20 000 columns, 40 entries per row, K = 64 23.7 -> 21.0, 35 per row
+// K = 40 22.2 -> 18.5; the fused call 0 .. 4 %.  Kernels whose wavefronts all take the same work keep four (k_flat
+// K = 64 15.1 -> 16.2, k_slice_dots 204 -> 205 with one), and so do k_flat_blocks' rows of more than 512 bytes
+// (K = 256: 251 -> 255).
+constexpr int ITEM_WAVES = 1;
+constexpr int block_item_waves(int units_per_lane) { return units_per_lane <= 4 ? ITEM_WAVES : WAVES_PER_BLOCK; }
 constexpr int FUSED_ROW_MAX = 64;          // fused SDDMM + SpMM: rows up to this length take one lane group each (a quarter of it: plan_fused_items)
 
 // Byte offset of a row: 32-bit when the whole operand is below 4 GiB (one VALU
@@ -422,15 +431,16 @@ __device__ __forceinline__ void entry_list_body(const void *__restrict__ A, cons
 // totals[0], totals[1]: work items of either kind (the grid is sized for an upper bound)
 //
 template <class L, bool SCALED>
-__global__ __launch_bounds__(BLOCK) void k_flat_blocks(const void *__restrict__ A, const void *__restrict__ B, int KU,
+__global__ __launch_bounds__(block_item_waves(L::UPL) * WAVE) void k_flat_blocks(const void *__restrict__ A, const void *__restrict__ B, int KU,
                                                        const int32_t *__restrict__ rowidx,
                                                        const int32_t *__restrict__ col,
                                                        const float *__restrict__ sval, float *__restrict__ P,
                                                        const RowItem *__restrict__ segments,
                                                        const RowItem *__restrict__ gaps,
                                                        const unsigned long long *__restrict__ totals) {
+    constexpr int WAVES = block_item_waves(L::UPL);
     const int64_t n_seg = (int64_t)totals[0], n_gap = (int64_t)totals[1];
-    const int64_t sb = (n_seg + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK, gb = (n_gap + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+    const int64_t sb = (n_seg + WAVES - 1) / WAVES, gb = (n_gap + WAVES - 1) / WAVES;
     // every XCD its contiguous eighth of each kind
     const int x = (int)(blockIdx.x % NUM_XCD);
     int64_t j = blockIdx.x / NUM_XCD;
@@ -439,7 +449,7 @@ __global__ __launch_bounds__(BLOCK) void k_flat_blocks(const void *__restrict__ 
     const bool segment = j < s_n;
     if (!segment) j -= s_n;
     if (!segment && j >= g_n) return;
-    const int64_t w = (segment ? s_lo + j : g_lo + j) * WAVES_PER_BLOCK + wave_in_block();
+    const int64_t w = (segment ? s_lo + j : g_lo + j) * WAVES + wave_in_block();
     if (w >= (segment ? n_seg : n_gap)) return;
     const RowItem it = segment ? segments[w] : gaps[w];
     const int row = __builtin_amdgcn_readfirstlane(it.row);
@@ -500,7 +510,7 @@ __global__ __launch_bounds__(BLOCK) void k_short_rows(const void *__restrict__ A
 // blocks after them run one segment item per wavefront.  The item blocks come
 // last in the XCD-contiguous order, after the short-row work of the same XCD.
 template <class L>
-__global__ __launch_bounds__(BLOCK) void k_auto(const void *__restrict__ A, const void *__restrict__ B, int KU,
+__global__ __launch_bounds__(ITEM_WAVES * WAVE) void k_auto(const void *__restrict__ A, const void *__restrict__ B, int KU,
                                                 const int32_t *__restrict__ rowptr,
                                                 const unsigned char *__restrict__ owner,
                                                 const int32_t *__restrict__ col,
@@ -517,7 +527,7 @@ __global__ __launch_bounds__(BLOCK) void k_auto(const void *__restrict__ A, cons
     const int64_t items_before = blk * item_blocks / nblocks;
     const bool is_item = ((blk + 1) * item_blocks / nblocks) != items_before;
     if (is_item) {
-        const int64_t w = items_before * WAVES_PER_BLOCK + wave_in_block();
+        const int64_t w = items_before * ITEM_WAVES + wave_in_block();
         if (w >= n_items) return;
         const RowItem it = items[w];
         const int row = __builtin_amdgcn_readfirstlane(it.row);
@@ -527,11 +537,11 @@ __global__ __launch_bounds__(BLOCK) void k_auto(const void *__restrict__ A, cons
     } else {
         const int64_t sb = blk - items_before;
         if (short_list) {
-            entry_list_body<L>(A, B, KU, short_list, n_short_list, col, sval, P, sb * WAVES_PER_BLOCK + wave_in_block(),
+            entry_list_body<L>(A, B, KU, short_list, n_short_list, col, sval, P, sb * ITEM_WAVES + wave_in_block(),
                                lane_id());
             return;
         }
-        const int64_t r0 = (sb * WAVES_PER_BLOCK + wave_in_block()) * rpw;
+        const int64_t r0 = (sb * ITEM_WAVES + wave_in_block()) * rpw;
         if (r0 >= M) return;
         short_rows_body<L>(A, B, KU, rowptr, owner, col, sval, P, M, ts, r0, rpw, lane_id());
     }

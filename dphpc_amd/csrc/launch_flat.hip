@@ -19,9 +19,9 @@ void launch_flat(sddmm_ctx *c) {
 namespace {
 
 // workgroups of a launch over at most `segments` and `gaps` work items: an eighth of either kind per XCD
-int64_t blocks_grid(int64_t segments, int64_t gaps) {
-    auto eighth = [](int64_t items) {                      // workgroups per XCD, rounded up twice
-        const int64_t blocks = (items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+int64_t blocks_grid(int64_t segments, int64_t gaps, int waves) {
+    auto eighth = [waves](int64_t items) {                 // workgroups per XCD, rounded up twice
+        const int64_t blocks = (items + waves - 1) / waves;
         return (blocks + NUM_XCD - 1) / NUM_XCD;
     };
     return NUM_XCD * (eighth(segments) + eighth(gaps));
@@ -39,13 +39,14 @@ void block_items_max(const sddmm_ctx *c, bool cut_long_rows, int64_t *segments, 
 // 0: no kernel for this row layout
 int launch_flat_blocks(sddmm_ctx *c) {
     const Shape s = shape_of(c);
-    const int64_t grid = blocks_grid(c->block_segments_max, c->block_gaps_max);
+    const int waves = block_item_waves(s.UPL);
+    const int64_t grid = blocks_grid(c->block_segments_max, c->block_gaps_max, waves);
     int launches = 0;
     with_layout(s, [&](auto L) {
         using LT = decltype(L);
         if constexpr (!LT::LONG) {
             auto launch = [&](auto kernel, float *out) {
-                SDDMM_LAUNCH(c, kernel, grid, BLOCK, (const void *)c->dA, (const void *)c->dB, s.len, entry_rows(c),
+                SDDMM_LAUNCH(c, kernel, grid, waves * WAVE, (const void *)c->dA, (const void *)c->dB, s.len, entry_rows(c),
                              entry_cols(c), (const float *)c->d_sval, out, (const RowItem *)c->d_block_segments,
                              (const RowItem *)c->d_block_gaps, (const unsigned long long *)c->d_block_totals);
                 ++launches;
@@ -71,7 +72,8 @@ bool blocks_pay(const sddmm_ctx *c) {
     if (shape_of(c).LPN == 0 || c->pc.rows_long == 0) return false;
     int64_t segments, gaps;                                         // (a launch takes fewer than 2^32 threads)
     block_items_max(c, true, &segments, &gaps);
-    if (blocks_grid(segments, gaps) * BLOCK >= (int64_t)1 << 32) return false;
+    const int waves = block_item_waves(shape_of(c).UPL);
+    if (blocks_grid(segments, gaps, waves) * waves * WAVE >= (int64_t)1 << 32) return false;
     if (mode >= 0) return mode != 0;
     const double b_bytes = (double)c->N * (double)c->K * (double)elem_size(c->dtype);
     return b_bytes >= 12.0 * (1 << 20) && c->nnz >= (1 << 20) && (double)c->pc.nnz_long >= 0.25 * (double)c->nnz;

@@ -1408,7 +1408,7 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
             rc = count();
             if (rc) return rc;
             // (a launch takes fewer than 2^32 threads: 2^26 items, which rows of more than 64 entries cannot reach)
-            if (row_max != FUSED_ROW_MAX && xcd_grid(fused_item_blocks((int64_t)tmp.n_items)) * BLOCK >= (int64_t)1 << 32) {
+            if (row_max != FUSED_ROW_MAX && xcd_grid(fused_item_blocks((int64_t)tmp.n_items)) * ITEM_WAVES * WAVE >= (int64_t)1 << 32) {
                 row_max = FUSED_ROW_MAX;
                 rc = count();
                 if (rc) return rc;
