@@ -118,20 +118,22 @@ __global__ __launch_bounds__(ITEM_WAVES * WAVE) void k_fusedmm(const void *__res
 #pragma unroll
         for (int e = 0; e < E; ++e) acc[i][e] = 0.f;
     const int last = end - 1;
-    struct Ent { int n, c; float s; bool valid; };
+    struct Ent { int base, n, c; float s; bool valid; };
     auto entry = [&](int base) {                      // entry base + lane of the item (clamped past its end)
         Ent x;
+        x.base = base;
         x.n = base + lane;
         x.valid = x.n < end;
-        x.c = col[x.n < last ? x.n : last];
-        x.s = x.valid ? sval[x.n] : 0.f;              // entries past the end contribute p = 0
+        const int at = x.n < last ? x.n : last;
+        x.c = col[at];
+        x.s = sval[at];
         return x;
     };
-    // steps t0 .. t0+NB-1 of a chunk: group g gathers the B rows of entries t*G+g
-    auto gather = [&](const Ent &x, int t0, T (&bf)[NB][UPL]) {
+    // steps t0 .. t0+N-1 of a chunk: group g gathers the B rows of entries t*G+g
+    auto gather = [&](const Ent &x, int t0, auto &bf) {
         const Off_t boff = (Off_t)x.c * rb;
 #pragma unroll
-        for (int q = 0; q < NB; ++q) {
+        for (int q = 0; q < (int)(sizeof(bf) / sizeof(bf[0])); ++q) {
             const int src = ((t0 + q) * G + g) & (WAVE - 1);
             const Off_t bo = shfl_off<Off_t>(boff, src);
 #pragma unroll
@@ -141,83 +143,105 @@ __global__ __launch_bounds__(ITEM_WAVES * WAVE) void k_fusedmm(const void *__res
             }
         }
     };
-    auto consume = [&](const Ent &x, int t0, int steps, const T (&bf)[NB][UPL], float &out) {
+    // FULL: all N steps hold entries of the item.  The steps are independent of each other up to the sums into acc: no
+    // branch between them, so that their lane exchanges overlap (a branch and a mask per step: graph of 200 000 rows,
+    // K = 64 in fp16, 47 us for this kernel, now 37; the whole call 89 -> 83 us; near-dense rows K = 64 46 -> 39 us).
+    auto consume = [&](auto full_tag, const Ent &x, int t0, const auto &bf, float &out) {
+        constexpr bool FULL = decltype(full_tag)::value;
+        constexpr int N = sizeof(bf) / sizeof(bf[0]);
+        float p[N];
+        bool live[N];
 #pragma unroll
-        for (int q = 0; q < NB; ++q) {
-            if (t0 + q >= steps) break;               // wave-uniform
+        for (int q = 0; q < N; ++q) {
             const int src = ((t0 + q) * G + g) & (WAVE - 1);
-            float p = 0.f;
+            float d = 0.f;
 #pragma unroll
             for (int i = 0; i < UPL; ++i) {
-                const float d = U::dot(a.u[i], bf[q][i], p);
-                p = C::unit_on(j, i, KU) ? d : p;
+                const float e = U::dot(a.u[i], bf[q][i], d);
+                d = C::unit_on(j, i, KU) ? e : d;
             }
+            p[q] = group_sum<LPN>(d) * __shfl(x.s, src, WAVE);
             // a step past the end of the row works on a clamped position: it must leave the
             // output row alone whatever that position's B row holds (0 * inf is not 0)
-            const bool live = __shfl((int)x.valid, src, WAVE) != 0;
-            p = group_sum<LPN>(p) * __shfl(x.s, src, WAVE);   // every lane takes part in the lane exchange
-            p = live ? p : 0.f;
+            if constexpr (!FULL) {
+                live[q] = x.base + src < end;
+                p[q] = live[q] ? p[q] : 0.f;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
 #pragma unroll
             for (int i = 0; i < UPL; ++i) {
                 float next[E];
 #pragma unroll
                 for (int e = 0; e < E; ++e) next[e] = acc[i][e];
-                U::axpy(p, bf[q][i], next);
+                U::axpy(p[q], bf[q][i], next);
 #pragma unroll
-                for (int e = 0; e < E; ++e) acc[i][e] = live ? next[e] : acc[i][e];
+                for (int e = 0; e < E; ++e) acc[i][e] = FULL || live[q] ? next[e] : acc[i][e];
             }
-            if (j == t0 + q) out = p;
+            if (j == t0 + q) out = p[q];
         }
-    };
-    auto steps_of = [&](int base) {
-        const int count = end - base < WAVE ? end - base : WAVE;
-        const int st = (count + G - 1) / G;
-        return st < LPN ? st : LPN;
     };
     // entry l = t*G+g was kept by lane g*LPN+t
     auto store_p = [&](const Ent &x, float out) {
         const float res = __shfl(out, (lane % G) * LPN + lane / G, WAVE);
         if (x.valid) P[x.n] = res;
     };
-    // Batches of NB steps, LPN / NB of them per chunk of 64 entries: the gathers of the next batch (of
-    // the next chunk after a chunk's last) and the indices of the chunk after the next are in flight
-    // while a batch is multiplied, one round trip per batch instead of one per batch and one per chunk.
-    constexpr int BPC = LPN / NB;
-    static_assert(LPN % NB == 0, "whole batches per chunk");
+    static_assert(LPN % NB == 0, "whole batches per chunk of 64 entries");
+    const std::true_type whole;
+    const std::false_type part;
+    // the last chunk: whole, half or quarter batches, rounded up
+    auto tail = [&](const Ent &x) {
+        constexpr int HALF = NB > 1 ? NB / 2 : 1, QUARTER = NB > 3 ? NB / 4 : 1;
+        const int steps = (end - x.base + G - 1) / G;
+        float out = 0.f;
+        for (int t0 = 0; t0 < steps; t0 += NB) {              // wave-uniform
+            auto batch = [&](auto n_tag) {
+                T bf[decltype(n_tag)::value][UPL];
+                gather(x, t0, bf);
+                consume(part, x, t0, bf, out);
+            };
+            const int left = steps - t0;
+            if (left > HALF) batch(std::integral_constant<int, NB>{});
+            else if (left > QUARTER) batch(std::integral_constant<int, HALF>{});
+            else batch(std::integral_constant<int, QUARTER>{});
+        }
+        store_p(x, out);
+    };
+    // Whole chunks: the gathers of the next chunk and the indices of the one after it are in flight while a chunk is
+    // multiplied, one round trip per chunk.
     // (Rows of more than one unit per lane keep one batch in flight: the second buffer costs them a
     // third of their wavefronts per SIMD, 171 against 153 us on banded rows of 256 bytes.)
-    constexpr bool AHEAD = UPL == 1;
+    constexpr bool AHEAD = UPL == 1 && NB == LPN;
     Ent cur = entry(start);
-    T bcur[NB][UPL];
-    if constexpr (AHEAD) gather(cur, 0, bcur);
-    Ent nxt = entry(start + WAVE);
-    for (int base = start; base < end; base += WAVE) {
-        const int steps = steps_of(base);
-        const bool more = base + WAVE < end;
-        const Ent after = entry(base + 2 * WAVE);
-        float out = 0.f;
-#pragma unroll
-        for (int bq = 0; bq < BPC; ++bq) {
-            const int t0 = bq * NB;
-            if (t0 >= steps) break;                           // wave-uniform
+    if (end - start >= WAVE) {
+        T bcur[NB][UPL];
+        if constexpr (AHEAD) gather(cur, 0, bcur);
+        Ent nxt = entry(start + WAVE);
+        for (int base = start; base + WAVE <= end; base += WAVE) {
+            const Ent after = entry(base + 2 * WAVE);
+            float out = 0.f;
             if constexpr (AHEAD) {
                 T bnxt[NB][UPL];
-                if (bq + 1 < BPC && t0 + NB < steps) gather(cur, t0 + NB, bnxt);
-                else if (more) gather(nxt, 0, bnxt);
-                consume(cur, t0, steps, bcur, out);
+                if (base + 2 * WAVE <= end) gather(nxt, 0, bnxt);
+                consume(whole, cur, 0, bcur, out);
 #pragma unroll
                 for (int q = 0; q < NB; ++q)
 #pragma unroll
                     for (int i = 0; i < UPL; ++i) bcur[q][i] = bnxt[q][i];
             } else {
-                gather(cur, t0, bcur);
-                consume(cur, t0, steps, bcur, out);
+#pragma unroll 1                                              // (unrolled, the gathers of all batches move to the front)
+                for (int t0 = 0; t0 < LPN; t0 += NB) {
+                    gather(cur, t0, bcur);
+                    consume(whole, cur, t0, bcur, out);
+                }
             }
+            store_p(cur, out);
+            cur = nxt;
+            nxt = after;
         }
-        store_p(cur, out);
-        cur = nxt;
-        nxt = after;
     }
+    if (cur.base < end) tail(cur);
     // add the partial output rows of the G groups: lanes with the same j
 #pragma unroll
     for (int off = LPN; off < WAVE; off <<= 1) {
