@@ -1351,7 +1351,7 @@ static bool fused_parts(sddmm_ctx *c) {
 }
 
 // items of the fused kernel: the rows of more than fused_row_max entries, cut into segments of
-// SDDMM_FUSED_SEG entries (default 1024, shortened below when there are few entries)
+// SDDMM_FUSED_SEG entries (by default 256, or 1024 where the rows are all about as long)
 static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
     if (c->fused_items_valid && c->fused_items_panels == (panel_owner != nullptr) && fused_parts(c)) return SDDMM_OK;
     int seg = std::max(WAVE, env_int("SDDMM_FUSED_SEG", 1024));
@@ -1384,17 +1384,15 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
         const PlanCounters first = counted;
         const int64_t item_entries = (int64_t)(first.nnz_medium + first.nnz_long);
         c->fused_short_avg = first.rows_short ? (double)first.nnz_short / (double)first.rows_short : 0.0;
-        // A wavefront walks its item chunk by chunk and the launch waits for the longest one: the long rows are
-        // cut so that there are about 3 072 pieces, none shorter than 256 entries (pieces of 2048 / 1024 / 512 / 256:
-        // graph of 50 k rows, 256-byte rows, 124 / 74 / 47 / 35 us; 200 k rows of 512 bytes 269 / 220 / 214 / 202; 1 M
-        // rows of 128 bytes 301 / 287 / 278 / 274; 2.6 M rows 795 / 776 / 776 / 778, where a piece costs what the cut
-        // returns).  Rows that are all about that long stay whole: 3 000 rows of 554 entries of 1 KiB 264 us, in
+        // A wavefront walks its item chunk by chunk and the launch waits for the longest one: the long rows are cut into
+        // pieces of 256 entries (1024 / 512 / 256: 200 k rows, 128 bytes 85.3 / 84.3 / 81.2 us, 256 bytes 122 / 119 / 116,
+        // 512 bytes 228 / 223 / 218; 1 M rows of 128 bytes 289 / 284 / 281; 2.6 M rows 800 / 793 / 787).  Rows that are all
+        // about as long as what 3 072 wavefronts would take stay whole: 3 000 rows of 554 entries of 1 KiB 264 us, in
         // pieces of 512 280.
         int best_seg = seg;
         if (!getenv("SDDMM_FUSED_SEG")) {
             const int64_t even = ((item_entries / 3072 + WAVE - 1) / WAVE) * WAVE;
-            const int shorter = (int)std::max<int64_t>(256, std::min<int64_t>(seg, even));
-            if ((int64_t)first.max_len > 2 * (int64_t)shorter) best_seg = shorter;
+            if ((int64_t)first.max_len > 2 * std::max<int64_t>(256, std::min<int64_t>(seg, even))) best_seg = 256;
         }
         // Where most of the short rows are very short, one of 17 .. 64 entries among them holds up the rows of its
         // wavefront: those become items too (graphs of 2.8 .. 4 entries per short row, 64 against 16: 50 k rows K=64
