@@ -30,7 +30,7 @@ EXPORTS = [
     "sddmm_launch", "sddmm_synchronize", "sddmm_time_runs", "sddmm_time_region", "sddmm_run_fused",
     "sddmm_get_fused", "sddmm_get_fused_device", "sddmm_get_values",
     "sddmm_get_values_device", "sddmm_last_stats", "sddmm_partition_rows", "sddmm_version",
-    "sddmm_launch_noalloc", "sddmm_flat_variant",
+    "sddmm_launch_noalloc", "sddmm_flat_variant", "sddmm_trim",
 ]
 
 

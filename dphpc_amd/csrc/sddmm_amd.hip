@@ -8,15 +8,20 @@
 
 namespace {
 
+// Gives a block back; it waits for the device first, as hipFree does, unless the caller has.
 template <class T>
-void dfree(T *&p) {
-    if (p) (void)hipFree((void *)p);
+void dfree(T *&p, bool idle = false) {
+    pool_free((void *)p, idle);
     p = nullptr;
 }
 
+// Nothing that uses a block may be in flight when the block is handed on: waits for the whole device, since a caller may
+// read the results on a stream of its own.
+bool wait_for_device() { return hipDeviceSynchronize() == hipSuccess; }
+
 // Views into the plan arena: nothing here is freed on its own.
-void release_arena(sddmm_ctx *c) {
-    dfree(c->d_arena);
+void release_arena(sddmm_ctx *c, bool idle = false) {
+    dfree(c->d_arena, idle);
     c->arena_rows = -1;
     c->d_owner = nullptr;
     c->d_strip_ntiles = c->d_strip_off = c->d_ustrip_ntiles = c->d_ustrip_off = nullptr;
@@ -80,7 +85,8 @@ int ensure_arena(sddmm_ctx *c) {
     } while (0)
 
 void release_dense(sddmm_ctx *c) {
-    if (c->own_dense) { dfree(c->dA); dfree(c->dB); }
+    const bool idle = c->own_dense && wait_for_device();
+    if (c->own_dense) { dfree(c->dA, idle); dfree(c->dB, idle); }
     c->dA = c->dB = nullptr;
     c->have_fused = false;
     c->own_dense = false;
@@ -89,36 +95,38 @@ void release_dense(sddmm_ctx *c) {
 }
 
 void release_sparse(sddmm_ctx *c) {
-    if (c->own_sparse) { dfree(c->d_col); dfree(c->d_sval); }
-    if (c->own_rowptr) dfree(c->d_rowptr);
-    if (c->own_rowidx) dfree(c->d_rowidx);
-    dfree(c->dP);
-    dfree(c->d_items);
-    dfree(c->d_tiles);
-    dfree(c->d_tile_cols);
-    dfree(c->d_windows);
-    dfree(c->d_win_order);
-    dfree(c->d_win_bins);
+    // (every pattern has its array of results, a context without one nothing to give back)
+    const bool idle = c->dP && wait_for_device();
+    if (c->own_sparse) { dfree(c->d_col, idle); dfree(c->d_sval, idle); }
+    if (c->own_rowptr) dfree(c->d_rowptr, idle);
+    if (c->own_rowidx) dfree(c->d_rowidx, idle);
+    dfree(c->dP, idle);
+    dfree(c->d_items, idle);
+    dfree(c->d_tiles, idle);
+    dfree(c->d_tile_cols, idle);
+    dfree(c->d_windows, idle);
+    dfree(c->d_win_order, idle);
+    dfree(c->d_win_bins, idle);
     c->win_order_cap = 0;
     c->use_win_order = false;
     c->n_windows = c->windows_cap = 0;
     c->ustrips_cap = 0;
-    dfree(c->d_sort_tmp);
-    release_arena(c);
+    dfree(c->d_sort_tmp, idle);
+    release_arena(c, idle);
     c->sort_tmp_bytes = 0;
     c->cand_cap = c->vstrips_cap = c->n_cand = c->n_vstrips = 0;
-    dfree(c->d_panel_items);
-    dfree(c->d_short_list);
+    dfree(c->d_panel_items, idle);
+    dfree(c->d_short_list, idle);
     c->short_list_cap = c->n_short_list = 0;
     c->use_short_list = false;
-    dfree(c->d_order);
+    dfree(c->d_order, idle);
     c->d_order_row = c->d_order_col = c->d_order_place = nullptr;
     c->d_order_dots = nullptr;
     c->order_cap = 0;
     c->use_order = false;
-    dfree(c->d_fused_items);
+    dfree(c->d_fused_items, idle);
     c->n_fused_items = c->fused_items_cap = 0;
-    dfree(c->d_fused_parts);
+    dfree(c->d_fused_parts, idle);
     c->n_fused_pieces = c->fused_part_floats = 0;
     c->fused_items_valid = c->have_fused = false;
     c->owner_cap = c->panels_cap = c->panel_items_cap = 0;
@@ -1045,13 +1053,14 @@ int sddmm_create(sddmm_ctx **out, int device) {
     sddmm_ctx *c = new (std::nothrow) sddmm_ctx();
     if (!c) return SDDMM_ERR_ALLOC;
     c->device = device;
-    if (hipStreamCreate(&c->own_stream) != hipSuccess || hipEventCreate(&c->ev0) != hipSuccess ||
-        hipEventCreate(&c->ev1) != hipSuccess || hipMalloc((void **)&c->d_pc, sizeof(DevCounters)) != hipSuccess ||
-        hipHostMalloc((void **)&c->h_pc, sizeof(DevCounters), hipHostMallocDefault) != hipSuccess) {
-        sddmm_destroy(c);
+    if (take_parts(&c->parts, device, sizeof(DevCounters)) != hipSuccess) {
+        delete c;
         return SDDMM_ERR_HIP;
     }
-    c->stream = c->own_stream;
+    c->stream = c->own_stream = c->parts.stream;
+    c->ev0 = c->parts.ev0; c->ev1 = c->parts.ev1;
+    c->d_pc = (DevCounters *)c->parts.counters;
+    c->h_pc = (DevCounters *)c->parts.host_counters;
     *out = c;
     return SDDMM_OK;
 }
@@ -1075,18 +1084,20 @@ int sddmm_get_stream(const sddmm_ctx *c, void **stream) {
 void sddmm_destroy(sddmm_ctx *c) {
     if (!c) return;
     (void)hipSetDevice(c->device);
-    if (c->own_stream) (void)hipStreamSynchronize(c->stream);
+    (void)hipStreamSynchronize(c->stream);
+    const bool idle = wait_for_device();
     release_dense(c);
     release_sparse(c);
-    dfree(c->dO);
-    dfree(c->d_part);
-    dfree(c->d_blocks);
-    dfree(c->d_pc);
-    if (c->h_pc) (void)hipHostFree(c->h_pc);
-    if (c->ev0) (void)hipEventDestroy(c->ev0);
-    if (c->ev1) (void)hipEventDestroy(c->ev1);
-    if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
+    dfree(c->dO, idle);
+    dfree(c->d_part, idle);
+    dfree(c->d_blocks, idle);
+    give_parts(c->parts, idle);
     delete c;
+}
+
+int sddmm_trim(void) {
+    pool_trim();
+    return SDDMM_OK;
 }
 
 static int set_dense_common(sddmm_ctx *c, int M, int N, int K, const void *A, const void *B, int dtype,

@@ -114,6 +114,10 @@ typedef struct sddmm_stats {
 /* ---- life cycle --------------------------------------------------------- */
 int sddmm_create(sddmm_ctx **out, int device);
 void sddmm_destroy(sddmm_ctx *ctx);
+/* Device memory of patterns that were replaced and of contexts that were destroyed is kept for the next ones: at most
+ * 128 MiB per device, none of it in blocks of more than 32 MiB, and the streams and events of up to 8 contexts.  Gives
+ * what is not in use back to the driver (as an allocation that fails does first).  Any thread, any time. */
+int sddmm_trim(void);
 const char *sddmm_strerror(int code);
 /* Text of the last failure on this context ("" if none); owned by the context. */
 const char *sddmm_last_error(const sddmm_ctx *ctx);
