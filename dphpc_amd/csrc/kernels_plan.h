@@ -108,6 +108,21 @@ static __global__ __launch_bounds__(256) void k_plan_reset(unsigned char *__rest
     }
 }
 
+// What a new pattern starts from, in one launch (as fills of the runtime 14 us): no entry of P computed, no counter counted.
+// P is 16-byte aligned.
+static __global__ __launch_bounds__(256) void k_clear_pattern(float *__restrict__ P, int64_t nnz, unsigned int *__restrict__ pc) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = t * 4; i < nnz; i += stride * 4) {
+        if (i + 4 <= nnz) *reinterpret_cast<float4 *>(P + i) = make_float4(0.f, 0.f, 0.f, 0.f);
+        else for (int64_t q = i; q < nnz; ++q) P[q] = 0.f;
+    }
+    if (blockIdx.x == 0)
+        for (int q = (int)threadIdx.x; q < (int)(sizeof(DevCounters) / sizeof(unsigned int)); q += 256) pc[q] = 0u;
+}
+
+// bits of DevCounters::bad_pattern
+constexpr unsigned int BAD_POINTER = 1, BAD_INDEX = 2;
+
 // rowptr[0]==0, rowptr[M]==nnz, non-decreasing; also counts non-empty rows and the
 // longest row.  One lane per row, one set of atomics per workgroup.
 static __global__ __launch_bounds__(256) void k_check_rowptr(const int32_t *__restrict__ rowptr, int M,
@@ -135,20 +150,22 @@ static __global__ __launch_bounds__(256) void k_check_rowptr(const int32_t *__re
     if (threadIdx.x == 0) {
         spread_add(pc, K_ROWS_NONEMPTY, sh_ne);
         if (sh_mx) atomicMax(&pc->max_len[blockIdx.x & (SPREAD - 1)], sh_mx);
-        if (sh_bad) atomicOr(&pc->bad_pattern, 1u);
+        if (sh_bad) atomicOr(&pc->bad_pattern, BAD_POINTER);
     }
 }
 
-// every column index in [0,N)
+// every column index in [0,N).  Does nothing after a launch of k_check_rowptr that found the row pointer malformed: the
+// array need not hold n values then (the host reads both verdicts at once: one wait for the device, 20 us, instead of two).
 static __global__ __launch_bounds__(256) void k_check_index(const int32_t *__restrict__ idx, int64_t n,
                                                      int bound, DevCounters *pc) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    if (pc->bad_pattern & BAD_POINTER) return;              // (this kernel sets the other bit only)
     unsigned int bad = 0;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
         const int32_t c = idx[i];
         bad |= (c < 0 || c >= bound) ? 1u : 0u;
     }
-    if (__ballot(bad != 0) && lane_id() == 0) atomicOr(&pc->bad_pattern, 1u);
+    if (__ballot(bad != 0) && lane_id() == 0) atomicOr(&pc->bad_pattern, BAD_INDEX);
 }
 
 // rowptr -> row index per stored entry (what the flat kernels read).  A wavefront

@@ -762,25 +762,27 @@ int plan_order(sddmm_ctx *c) {
     return SDDMM_OK;
 }
 
+// Clears P and the counters of a new pattern.
+int clear_pattern(sddmm_ctx *c, int64_t nnz) {
+    SDDMM_LAUNCH(c, k_clear_pattern, grid_capped(nnz, 1024, 4096), 256, c->dP, nnz, (unsigned int *)c->d_pc);
+    LAUNCH_CHECK(c);
+    return SDDMM_OK;
+}
+
 // Validate the device-resident CSR and gather row statistics.
 int validate_csr(sddmm_ctx *c) {
-    HIP_TRY(c, hipMemsetAsync(c->d_pc, 0, sizeof(DevCounters), c->stream));
     if (c->sM > 0)
         SDDMM_LAUNCH(c, k_check_rowptr, grid_for(c->sM, 256), 256, c->d_rowptr, c->sM,
                            c->nnz, c->d_pc);
-    LAUNCH_CHECK(c);
-    int rc = fetch_counters(c);
-    if (rc) return rc;
-    if (c->pc.bad_pattern) return fail(c, SDDMM_ERR_PATTERN, "rowptr is not a valid CSR row pointer array");
-    // only now is it safe to walk col[0..nnz)
-    if (c->nnz > 0) {
+    // (walks col[0..nnz) only behind a valid row pointer)
+    if (c->nnz > 0)
         SDDMM_LAUNCH(c, k_check_index, grid_capped(c->nnz, 256), 256, c->d_col, c->nnz,
                            c->sN, c->d_pc);
-        LAUNCH_CHECK(c);
-        rc = fetch_counters(c);
-        if (rc) return rc;
-        if (c->pc.bad_pattern) return fail(c, SDDMM_ERR_PATTERN, "column index outside [0,N)");
-    }
+    LAUNCH_CHECK(c);
+    const int rc = fetch_counters(c);
+    if (rc) return rc;
+    if (c->pc.bad_pattern & BAD_POINTER) return fail(c, SDDMM_ERR_PATTERN, "rowptr is not a valid CSR row pointer array");
+    if (c->pc.bad_pattern) return fail(c, SDDMM_ERR_PATTERN, "column index outside [0,N)");
     return SDDMM_OK;
 }
 
@@ -1158,8 +1160,9 @@ int sddmm_set_csr(sddmm_ctx *c, int M, int N, int64_t nnz, const int32_t *rowptr
     if (nnz) {
         HIP_TRY(c, hipMemcpyAsync(c->d_col, col, (size_t)nnz * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
         HIP_TRY(c, hipMemcpyAsync(c->d_sval, sval, (size_t)nnz * sizeof(float), hipMemcpyHostToDevice, c->stream));
-        HIP_TRY(c, hipMemsetAsync(c->dP, 0, (size_t)nnz * sizeof(float), c->stream));
     }
+    rc = clear_pattern(c, nnz);
+    if (rc) return rc;
     c->sM = M; c->sN = N; c->nnz = nnz;
     rc = validate_csr(c);
     if (rc) { release_sparse(c); return rc; }
@@ -1180,7 +1183,8 @@ int sddmm_set_csr_device(sddmm_ctx *c, int M, int N, int64_t nnz, const int32_t 
     c->d_col = const_cast<int32_t *>(d_col);
     c->d_sval = const_cast<float *>(d_sval);
     ALLOC_TRY(c, c->dP, (size_t)nnz * sizeof(float));
-    if (nnz) HIP_TRY(c, hipMemsetAsync(c->dP, 0, (size_t)nnz * sizeof(float), c->stream));
+    rc = clear_pattern(c, nnz);
+    if (rc) return rc;
     c->sM = M; c->sN = N; c->nnz = nnz;
     rc = validate_csr(c);
     if (rc) { release_sparse(c); return rc; }
@@ -1211,14 +1215,14 @@ static int set_coo_common(sddmm_ctx *c, int M, int N, int64_t nnz, const int32_t
     ALLOC_TRY(c, c->dP, (size_t)nnz * sizeof(float));
     ALLOC_TRY(c, c->d_rowptr, (size_t)(M + 1) * sizeof(int32_t));
     c->sM = M; c->sN = N; c->nnz = nnz;
-    HIP_TRY(c, hipMemsetAsync(c->d_pc, 0, sizeof(DevCounters), c->stream));
+    rc = clear_pattern(c, nnz);
+    if (rc) return rc;
     if (nnz) {
         if (!on_device) {
             HIP_TRY(c, hipMemcpyAsync(c->d_rowidx, row, (size_t)nnz * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
             HIP_TRY(c, hipMemcpyAsync(c->d_col, col, (size_t)nnz * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
             HIP_TRY(c, hipMemcpyAsync(c->d_sval, sval, (size_t)nnz * sizeof(float), hipMemcpyHostToDevice, c->stream));
         }
-        HIP_TRY(c, hipMemsetAsync(c->dP, 0, (size_t)nnz * sizeof(float), c->stream));
         const int g = grid_capped(nnz, 256);
         SDDMM_LAUNCH(c, k_check_index, g, 256, c->d_rowidx, nnz, M, c->d_pc);
         SDDMM_LAUNCH(c, k_check_index, g, 256, c->d_col, nnz, N, c->d_pc);
