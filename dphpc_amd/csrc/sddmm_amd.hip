@@ -1427,11 +1427,11 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
                 if (rc) return rc;
             }
         }
-        // the pieces of the rows that are cut, at the most; without room for them every row stays whole
-        c->n_fused_pieces = (int64_t)counted.rows_long + (int64_t)counted.nnz_long / seg;
-        if (!fused_parts(c)) {
-            c->n_fused_pieces = 0;
-            seg = INT_MAX;
+        // the pieces of the rows that are cut, at the most; without room for them fewer and longer ones, and at last every
+        // row stays whole
+        const auto pieces = [&]() { return c->n_fused_pieces = (int64_t)counted.rows_long + (int64_t)counted.nnz_long / seg; };
+        for (pieces(); !fused_parts(c); pieces()) {
+            seg = seg < 1024 ? 1024 : INT_MAX;
             rc = count();
             if (rc) return rc;
         }

@@ -75,3 +75,20 @@ def test_without_room_for_the_pieces(engine_factory, monkeypatch):
         monkeypatch.delenv("SDDMM_SPARE_BYTES")
         e.set_csr(len(lens), N, rowptr, col, val)
         _check(e, rowptr, col, val, A, B, "room again")
+
+
+def test_room_for_fewer_pieces_only(engine_factory, monkeypatch):
+    """25 pieces of 256 entries take 6 400 bytes, 5 of 1 024 take 1 280: the sums are then those of the longer pieces."""
+    rng = np.random.default_rng(4)
+    N, lens = 6000, np.concatenate([[5000, 2], rng.integers(0, 20, 200), [600, 257, 70]])
+    rowptr, col, val = _matrix(rng, N, lens)
+    A, _, B, _ = _operands(rng, len(lens), N, 64, capi.F32)
+    got = []
+    for name, value in (("SDDMM_SPARE_BYTES", "4000"), ("SDDMM_FUSED_SEG", "1024"), ("SDDMM_FUSED_SEG", "256")):
+        with monkeypatch.context() as m, engine_factory() as e:
+            m.setenv(name, value)
+            e.set_dense(A, B)
+            e.set_csr(len(lens), N, rowptr, col, val)
+            got.append(_check(e, rowptr, col, val, A, B, name))
+    np.testing.assert_array_equal(got[0], got[1])
+    assert (got[0] != got[2]).any()
