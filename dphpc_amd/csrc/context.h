@@ -144,6 +144,7 @@ struct sddmm_ctx {
     double fused_short_avg = 0.0;    // entries per non-empty row of at most FUSED_ROW_MAX entries (panel rows apart)
     int fused_row_max = FUSED_ROW_MAX;   // rows beyond it are work items of their own
     int fused_seg = 0;               // of at most so many entries
+    int fused_block_waves = WAVES_PER_BLOCK;   // wavefronts per workgroup of the fused gather kernels
     float *d_fused_parts = nullptr;  // partial output rows of the pieces of the rows cut into several items
     int64_t n_fused_pieces = 0, fused_part_floats = 0;
     float *dO = nullptr;
@@ -358,5 +359,5 @@ bool launch_auto_with_tiles(sddmm_ctx *c);                                      
 void launch_tiles(sddmm_ctx *c);
 void launch_panels(sddmm_ctx *c);                                                // launch_panels.hip
 void launch_panels_fused(sddmm_ctx *c);
-inline int64_t fused_item_blocks(int64_t n_items) { return (n_items + ITEM_WAVES - 1) / ITEM_WAVES; }
+inline int64_t blocks_of(int64_t waves, int per_block) { return (waves + per_block - 1) / per_block; }
 int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner);           // launch_fused.hip: number of launches

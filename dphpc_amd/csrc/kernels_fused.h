@@ -86,7 +86,7 @@ __device__ __forceinline__ void add_cut_rows(const float *__restrict__ parts, fl
 }
 
 template <class L>
-__global__ __launch_bounds__(ITEM_WAVES * WAVE) void k_fusedmm(const void *__restrict__ A, const void *__restrict__ B, int KU,
+__global__ __launch_bounds__(BLOCK) void k_fusedmm(const void *__restrict__ A, const void *__restrict__ B, int KU,
                                                    const int32_t *__restrict__ rowptr,
                                                    const int32_t *__restrict__ col,
                                                    const float *__restrict__ sval, float *__restrict__ P,
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(ITEM_WAVES * WAVE) void k_fusedmm(const void *__res
     constexpr int NB = C::BIG;                        // steps whose gathers are in flight together
     const int64_t blk = xcd_remap(blockIdx.x, nblocks);
     if (blk < 0) return;
-    const int64_t w = blk * ITEM_WAVES + wave_in_block();
+    const int64_t w = blk * waves_in_block() + wave_in_block();
     if (w >= n_items) return;
     const RowItem it = items[w];
     const int row = __builtin_amdgcn_readfirstlane(it.row);
@@ -277,7 +277,7 @@ __global__ __launch_bounds__(ITEM_WAVES * WAVE) void k_fusedmm(const void *__res
 // row of zeros, which that kernel, launched after this one, adds to.  Every row below M has
 // its output row written by one or the other, so O needs no clearing before the launches.
 template <class L>
-__global__ __launch_bounds__(ITEM_WAVES * WAVE) void k_fusedmm_rows(const void *__restrict__ A, const void *__restrict__ B, int KU,
+__global__ __launch_bounds__(BLOCK) void k_fusedmm_rows(const void *__restrict__ A, const void *__restrict__ B, int KU,
                                                         const int32_t *__restrict__ rowptr,
                                                         const int32_t *__restrict__ col,
                                                         const float *__restrict__ sval, float *__restrict__ P,
@@ -293,7 +293,7 @@ __global__ __launch_bounds__(ITEM_WAVES * WAVE) void k_fusedmm_rows(const void *
     constexpr int NB = C::BIG;
     const int64_t blk = xcd_remap(blockIdx.x, nblocks);
     if (blk < 0) return;
-    const int64_t r0 = (blk * ITEM_WAVES + wave_in_block()) * G;
+    const int64_t r0 = (blk * waves_in_block() + wave_in_block()) * G;
     if (r0 >= M) return;
     const int lane = lane_id();
     const int g = lane / LPN, j = lane & (LPN - 1);
@@ -436,7 +436,7 @@ __global__ __launch_bounds__(ITEM_WAVES * WAVE) void k_fusedmm_rows(const void *
 // output row is written whenever the row changes.  Rows without entries of their own (empty,
 // left to the panel kernel) get zeros and the pieces of cut rows are added, as in k_fusedmm_rows.
 template <class L>
-__global__ __launch_bounds__(ITEM_WAVES * WAVE) void k_fusedmm_rows_balanced(const void *__restrict__ A, const void *__restrict__ B,
+__global__ __launch_bounds__(BLOCK) void k_fusedmm_rows_balanced(const void *__restrict__ A, const void *__restrict__ B,
                                                                  int KU, const int32_t *__restrict__ rowptr,
                                                                  const int32_t *__restrict__ col,
                                                                  const float *__restrict__ sval, float *__restrict__ P,
@@ -450,10 +450,10 @@ __global__ __launch_bounds__(ITEM_WAVES * WAVE) void k_fusedmm_rows_balanced(con
     using Off_t = typename C::O;
     constexpr int LPN = L::LPN, UPL = L::UPL, G = WAVE / LPN;
     constexpr int NB = C::BIG > 4 ? 4 : C::BIG;       // A and B rows of a batch of steps in flight together
-    __shared__ int pre_all[ITEM_WAVES][WAVE], pos_all[ITEM_WAVES][WAVE];
+    __shared__ int pre_all[WAVES_PER_BLOCK][WAVE], pos_all[WAVES_PER_BLOCK][WAVE];
     const int64_t blk = xcd_remap(blockIdx.x, nblocks);
     if (blk < 0) return;
-    const int64_t r0 = (blk * ITEM_WAVES + wave_in_block()) * WAVE;
+    const int64_t r0 = (blk * waves_in_block() + wave_in_block()) * WAVE;
     if (r0 >= M) return;
     const int lane = lane_id();
     const int g = lane / LPN, j = lane & (LPN - 1);

@@ -26,15 +26,15 @@ namespace sddmm {
 
 constexpr int BLOCK = 256;                 // 4 wavefronts
 constexpr int WAVES_PER_BLOCK = BLOCK / WAVE;
-// Kernels of many short work items of different lengths take workgroups of one wavefront: a workgroup keeps its place on
-// the CU until its last wavefront ends, and with four items each the places are half empty (4.9 of 6 wavefronts per SIMD
-// on average in k_flat_blocks).  Against workgroups of four: graph of 2.6 M rows, K = 32, 554 -> 527 us; 200 000 rows
-// K = 32 30.3 -> 28.0, K = 64 56.7 -> 54.9; k_auto, 20 000 columns, 40 entries per row, K = 64 23.7 -> 21.0, 35 per row
-// K = 40 22.2 -> 18.5; the fused call 0 .. 4 %.  Kernels whose wavefronts all take the same work keep four (k_flat
-// K = 64 15.1 -> 16.2, k_slice_dots 204 -> 205 with one), and so do k_flat_blocks' rows of more than 512 bytes
-// (K = 256: 251 -> 255).
-constexpr int ITEM_WAVES = 1;
-constexpr int block_item_waves(int units_per_lane) { return units_per_lane <= 4 ? ITEM_WAVES : WAVES_PER_BLOCK; }
+// Work items of different lengths over columns that neighbours do not share take workgroups of one wavefront: a workgroup
+// keeps its place on the CU until its last wavefront ends, and with four items each the places are half empty (4.9 of 6
+// wavefronts per SIMD on average in k_flat_blocks).  Against workgroups of four: graph of 2.6 M rows, K = 32, 554 -> 527 us;
+// 200 000 rows K = 32 30.3 -> 28.0, K = 64 56.7 -> 54.9; rows of more than 512 bytes keep four (K = 256: 251 -> 255 with
+// one).  Kernels whose wavefronts all take the same work keep four (k_flat K = 64 15.1 -> 16.2, k_slice_dots 204 -> 205
+// with one), and so does k_auto: with one, rows of 20 000 random columns gain (K = 64 23.7 -> 21.0), but rows whose
+// neighbours hold the same columns lose what they find in the CU's L1 (banded blocks K = 42 59 -> 92, dense tiles K = 120
+// bf16 30 -> 35) and items of a few bytes wait for their dispatch (45 entries per row, K = 8 bf16, 20 -> 36).
+constexpr int block_item_waves(int units_per_lane) { return units_per_lane <= 4 ? 1 : WAVES_PER_BLOCK; }
 constexpr int FUSED_ROW_MAX = 64;          // fused SDDMM + SpMM: rows up to this length take one lane group each (a quarter of it: plan_fused_items)
 
 // Byte offset of a row: 32-bit when the whole operand is below 4 GiB (one VALU
@@ -510,7 +510,7 @@ __global__ __launch_bounds__(BLOCK) void k_short_rows(const void *__restrict__ A
 // blocks after them run one segment item per wavefront.  The item blocks come
 // last in the XCD-contiguous order, after the short-row work of the same XCD.
 template <class L>
-__global__ __launch_bounds__(ITEM_WAVES * WAVE) void k_auto(const void *__restrict__ A, const void *__restrict__ B, int KU,
+__global__ __launch_bounds__(BLOCK) void k_auto(const void *__restrict__ A, const void *__restrict__ B, int KU,
                                                 const int32_t *__restrict__ rowptr,
                                                 const unsigned char *__restrict__ owner,
                                                 const int32_t *__restrict__ col,
@@ -527,7 +527,7 @@ __global__ __launch_bounds__(ITEM_WAVES * WAVE) void k_auto(const void *__restri
     const int64_t items_before = blk * item_blocks / nblocks;
     const bool is_item = ((blk + 1) * item_blocks / nblocks) != items_before;
     if (is_item) {
-        const int64_t w = items_before * ITEM_WAVES + wave_in_block();
+        const int64_t w = items_before * WAVES_PER_BLOCK + wave_in_block();
         if (w >= n_items) return;
         const RowItem it = items[w];
         const int row = __builtin_amdgcn_readfirstlane(it.row);
@@ -537,11 +537,11 @@ __global__ __launch_bounds__(ITEM_WAVES * WAVE) void k_auto(const void *__restri
     } else {
         const int64_t sb = blk - items_before;
         if (short_list) {
-            entry_list_body<L>(A, B, KU, short_list, n_short_list, col, sval, P, sb * ITEM_WAVES + wave_in_block(),
+            entry_list_body<L>(A, B, KU, short_list, n_short_list, col, sval, P, sb * WAVES_PER_BLOCK + wave_in_block(),
                                lane_id());
             return;
         }
-        const int64_t r0 = (sb * ITEM_WAVES + wave_in_block()) * rpw;
+        const int64_t r0 = (sb * WAVES_PER_BLOCK + wave_in_block()) * rpw;
         if (r0 >= M) return;
         short_rows_body<L>(A, B, KU, rowptr, owner, col, sval, P, M, ts, r0, rpw, lane_id());
     }

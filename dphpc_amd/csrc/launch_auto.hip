@@ -4,12 +4,12 @@
 void launch_auto(sddmm_ctx *c) {
     const Shape s = shape_of(c);
     const int64_t waves = short_row_waves(c);
-    const int64_t short_blocks = (waves + ITEM_WAVES - 1) / ITEM_WAVES;
-    const int64_t item_blocks = (c->n_items + ITEM_WAVES - 1) / ITEM_WAVES;
+    const int64_t short_blocks = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
+    const int64_t item_blocks = (c->n_items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
     const int64_t nblocks = short_blocks + item_blocks;
     with_layout(s, [&](auto L) {
         using LT = decltype(L);
-        SDDMM_LAUNCH(c, (k_auto<LT>), xcd_grid(nblocks), ITEM_WAVES * WAVE,
+        SDDMM_LAUNCH(c, (k_auto<LT>), xcd_grid(nblocks), BLOCK,
                            (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr,
                            (const unsigned char *)(c->owner_active ? c->d_owner : nullptr), c->d_col, c->d_sval,
                            c->dP, c->sM, c->ts, c->rpw, short_blocks, c->d_items, c->n_items, nblocks,

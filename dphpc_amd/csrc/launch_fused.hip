@@ -23,10 +23,10 @@ int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
         if constexpr (!LT::LONG && LT::LPN <= 8 && LT::U::ELEMS > 1 && LT::U::WHOLE && LT::UPL * LT::U::ELEMS <= 32) {
             const int64_t rows_per_wave = WAVE / LT::LPN;
             const int64_t waves = ((int64_t)c->sM + rows_per_wave - 1) / rows_per_wave;
-            const int64_t rblocks = (waves + ITEM_WAVES - 1) / ITEM_WAVES;
+            const int64_t rblocks = blocks_of(waves, c->fused_block_waves);
             if (c->n_fused_items > 0) {
-                const int64_t nblocks = fused_item_blocks(c->n_fused_items);
-                SDDMM_LAUNCH(c, (k_fusedmm<LT>), xcd_grid(nblocks), ITEM_WAVES * WAVE,
+                const int64_t nblocks = blocks_of(c->n_fused_items, c->fused_block_waves);
+                SDDMM_LAUNCH(c, (k_fusedmm<LT>), xcd_grid(nblocks), c->fused_block_waves * WAVE,
                                    (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col,
                                    c->d_sval, c->dP, c->dO, c->d_fused_parts, (const RowItem *)c->d_fused_items,
                                    c->n_fused_items, nblocks);
@@ -34,13 +34,13 @@ int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
             }
             if (balanced) {
                 const int64_t bwaves = ((int64_t)c->sM + WAVE - 1) / WAVE;
-                const int64_t bblocks = (bwaves + ITEM_WAVES - 1) / ITEM_WAVES;
-                SDDMM_LAUNCH(c, (k_fusedmm_rows_balanced<LT>), xcd_grid(bblocks), ITEM_WAVES * WAVE,
+                const int64_t bblocks = blocks_of(bwaves, c->fused_block_waves);
+                SDDMM_LAUNCH(c, (k_fusedmm_rows_balanced<LT>), xcd_grid(bblocks), c->fused_block_waves * WAVE,
                                    (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col, c->d_sval,
                                    c->dP, c->dO, (const float *)c->d_fused_parts, c->sM, c->fused_row_max,
                                    c->fused_seg, bblocks, panel_owner);
             } else {
-                SDDMM_LAUNCH(c, (k_fusedmm_rows<LT>), xcd_grid(rblocks), ITEM_WAVES * WAVE,
+                SDDMM_LAUNCH(c, (k_fusedmm_rows<LT>), xcd_grid(rblocks), c->fused_block_waves * WAVE,
                                    (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col, c->d_sval,
                                    c->dP, c->dO, (const float *)c->d_fused_parts, c->sM, c->fused_row_max,
                                    c->fused_seg, rblocks, panel_owner);

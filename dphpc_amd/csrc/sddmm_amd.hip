@@ -1404,11 +1404,14 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
         // 512 bytes 228 / 223 / 218; 1 M rows of 128 bytes 289 / 284 / 281; 2.6 M rows 800 / 793 / 787).  Rows that are all
         // about as long as what 3 072 wavefronts would take stay whole: 3 000 rows of 554 entries of 1 KiB 264 us, in
         // pieces of 512 280.
-        int best_seg = seg;
-        if (!getenv("SDDMM_FUSED_SEG")) {
-            const int64_t even = ((item_entries / 3072 + WAVE - 1) / WAVE) * WAVE;
-            if ((int64_t)first.max_len > 2 * std::max<int64_t>(256, std::min<int64_t>(seg, even))) best_seg = 256;
-        }
+        const int64_t even = ((item_entries / 3072 + WAVE - 1) / WAVE) * WAVE;
+        const bool uneven = (int64_t)first.max_len > 2 * std::max<int64_t>(256, std::min<int64_t>(seg, even));
+        const int best_seg = uneven && !getenv("SDDMM_FUSED_SEG") ? 256 : seg;
+        // Workgroups of one wavefront only where lengths differ: the place on the CU is then free as soon as an item ends
+        // (four / one: graphs of 200 k rows, K=64 fp16 78.3 / 74.3 us, K=8 bf16 54.6 / 51.4, K=16 42.6 / 40.5).  Rows of about
+        // one length end together, and neighbours share B rows in the vector L1 (banded blocks of 36 k rows K=256 499 / 522,
+        // K=16 67.7 / 71.0; uniform rows of 45 entries K=8 bf16 222 / 232).
+        c->fused_block_waves = uneven ? 1 : WAVES_PER_BLOCK;
         // Where most of the short rows are very short, one of 17 .. 64 entries among them holds up the rows of its
         // wavefront: those become items too (graphs of 2.8 .. 4 entries per short row, 64 against 16: 50 k rows K=64
         // 46 -> 35 us; 200 k rows K=8 60 -> 44 us, K=64 fp16 92 -> 77, K=128 251 -> 218; 1 M rows K=64 606 -> 566;
@@ -1421,7 +1424,7 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
             rc = count();
             if (rc) return rc;
             // (a launch takes fewer than 2^32 threads: 2^26 items, which rows of more than 64 entries cannot reach)
-            if (row_max != FUSED_ROW_MAX && xcd_grid(fused_item_blocks((int64_t)tmp.n_items)) * ITEM_WAVES * WAVE >= (int64_t)1 << 32) {
+            if (row_max != FUSED_ROW_MAX && xcd_grid(blocks_of((int64_t)tmp.n_items, c->fused_block_waves)) * c->fused_block_waves * WAVE >= (int64_t)1 << 32) {
                 row_max = FUSED_ROW_MAX;
                 rc = count();
                 if (rc) return rc;
