@@ -303,7 +303,10 @@ __device__ __forceinline__ void row_segment_body(const void *__restrict__ A, con
             int cn = 0;
             float sn = 1.f;
             auto prefetch = [&]() {
-                if (left <= WAVE) return;                   // (wave-uniform)
+                // Nothing to load ahead of the last chunk; with one unit per lane the branch costs more than the loads (with /
+                // without it: mixed rows K = 21 13.9 / 13.2 us, banded K = 20 17.2 / 16.0, K = 40 bf16 20.1 / 18.1), with two
+                // it returns more (35 entries per row K = 40 35.6 / 38.4, graph of 200 000 rows K = 100 107.7 / 111.2).
+                if (L::UPL > 1 && left <= WAVE) return;     // (wave-uniform)
                 const int pn = n + WAVE < last ? n + WAVE : last;
                 cn = ld_stream(col + pn);
                 if constexpr (SCALED) sn = ld_stream(sval + pn);
