@@ -148,21 +148,25 @@ inline hipError_t take_parts(ContextParts *out, int device, size_t counter_bytes
             }
     }
     ContextParts c;
-    c.device = device;
-    hipError_t e = hipStreamCreate(&c.stream);
-    if (e == hipSuccess) e = hipEventCreate(&c.ev0);
-    if (e == hipSuccess) e = hipEventCreate(&c.ev1);
-    if (e == hipSuccess) e = hipMalloc(&c.counters, counter_bytes);
-    if (e == hipErrorOutOfMemory) {                          // (free blocks are given back first, as in pool_alloc)
+    auto make = [&]() {
+        c.device = device;
+        hipError_t e = hipStreamCreate(&c.stream);
+        if (e == hipSuccess) e = hipEventCreate(&c.ev0);
+        if (e == hipSuccess) e = hipEventCreate(&c.ev1);
+        if (e == hipSuccess) e = hipMalloc(&c.counters, counter_bytes);
+        if (e == hipSuccess) e = hipHostMalloc(&c.host_counters, counter_bytes, hipHostMallocDefault);
+        if (e != hipSuccess) destroy_parts(c);
+        return e;
+    };
+    hipError_t e = make();
+    if (e == hipErrorOutOfMemory) {                          // the whole set again, once the free blocks are given back
         (void)hipGetLastError();
         {
             const std::lock_guard<std::mutex> hold(device_pool.lock);
             pool_trim_locked(device_pool, device);
         }
-        e = hipMalloc(&c.counters, counter_bytes);
+        e = make();
     }
-    if (e == hipSuccess) e = hipHostMalloc(&c.host_counters, counter_bytes, hipHostMallocDefault);
-    if (e != hipSuccess) destroy_parts(c);
     *out = c;
     return e;
 }
