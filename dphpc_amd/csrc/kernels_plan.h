@@ -19,6 +19,7 @@ struct PlanCounters {
     unsigned long long n_tiles, nnz_tiles, tiles_scanned;     // dense-tile path: 16-row and gathered strips
     unsigned long long n_utiles, nnz_utiles, utiles_scanned;  // dense-tile path: union strips
     unsigned long long n_panels, nnz_panels, panel_items;     // row-panel path
+    unsigned int fused_longest;    // fused call: longest row that its gather kernels take
 };
 
 // The same counters on the device.  Sums that thousands of workgroups contribute to
@@ -35,7 +36,8 @@ enum CounterKind {
 };
 struct DevCounters {
     unsigned int bad_pattern, coo_unsorted, pad0, pad1;
-    unsigned long long n_items, tiles_scanned, panel_items;          // scan totals, one writer each
+    unsigned long long n_items, fused_longest;                       // (one fill clears both; PlanCounters)
+    unsigned long long tiles_scanned, panel_items;                   // scan totals, one writer each, as is n_items
     unsigned long long n_candidates;                                 // rows offered to the gathered strips
     unsigned long long utiles_scanned, short_scanned;                // scan totals: union strips, entries of the short rows
     unsigned long long long_scanned;                                 // scan total: rows of more than one item
@@ -64,6 +66,7 @@ inline PlanCounters summarize(const DevCounters &d) {
     p.n_tiles = sum[K_TILES]; p.nnz_tiles = sum[K_NNZ_TILES];
     p.n_utiles = sum[K_UTILES]; p.nnz_utiles = sum[K_NNZ_UTILES]; p.utiles_scanned = d.utiles_scanned;
     p.n_panels = sum[K_PANELS]; p.nnz_panels = sum[K_NNZ_PANELS];
+    p.fused_longest = (unsigned int)d.fused_longest;
     p.n_items = d.n_items; p.tiles_scanned = d.tiles_scanned; p.panel_items = d.panel_items;
     return p;
 }
@@ -299,12 +302,13 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int3
                                                                unsigned int *__restrict__ short_sums,
                                                                unsigned int *__restrict__ long_sums) {
     const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
-    unsigned int items = 0;
+    unsigned int items = 0, longest = 0;
     unsigned long long r_short = 0, r_med = 0, r_long = 0, n_short = 0, n_med = 0, n_long = 0;
     for (int q = 0; q < SCAN_ITEMS; ++q) {
         unsigned int len;
         const unsigned int cnt = row_item_count(rowptr, owner, base + q, M, ts, seg, &len, only);
         items += cnt;
+        longest = len > longest ? len : longest;
         if (len == 0) continue;
         if (cnt == 0) { ++r_short; n_short += len; }
         else if (cnt == 1) { ++r_med; n_med += len; }
@@ -329,6 +333,10 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int3
     }
     __syncthreads();
     if (threadIdx.x < 6) spread_add(pc, K_ROWS_SHORT + (int)threadIdx.x, sh[threadIdx.x]);
+    if (only) {                                       // the fused call (most workgroups find a longer row there already)
+        longest = wave_max_u32(longest);
+        if (lane_id() == 0 && longest > pc->fused_longest) atomicMax(&pc->fused_longest, (unsigned long long)longest);
+    }
     // entries of this block's short rows, for the entry list (k_short_list_write)
     if (short_sums && threadIdx.x == 0) short_sums[blockIdx.x] = (unsigned int)sh[3];
     // and its rows of more than one item, for the list of the long rows (k_long_rows)

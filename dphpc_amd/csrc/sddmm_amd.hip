@@ -1366,7 +1366,7 @@ static bool fused_parts(sddmm_ctx *c) {
 }
 
 // items of the fused kernel: the rows of more than fused_row_max entries, cut into segments of
-// SDDMM_FUSED_SEG entries (by default 256, or 1024 where the rows are all about as long)
+// SDDMM_FUSED_SEG entries (by default 256, and up to 1024 where most rows are about as long)
 static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
     if (c->fused_items_valid && c->fused_items_panels == (panel_owner != nullptr) && fused_parts(c)) return SDDMM_OK;
     int seg = std::max(WAVE, env_int("SDDMM_FUSED_SEG", 1024));
@@ -1382,7 +1382,7 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
         auto count = [&]() -> int {
             HIP_TRY(c, hipMemsetAsync(&c->d_pc->k[K_ROWS_SHORT][0], 0,
                                       sizeof(unsigned long long) * SPREAD * (K_NNZ_LONG - K_ROWS_SHORT + 1), c->stream));
-            HIP_TRY(c, hipMemsetAsync(&c->d_pc->n_items, 0, sizeof(unsigned long long), c->stream));
+            HIP_TRY(c, hipMemsetAsync(&c->d_pc->n_items, 0, 2 * sizeof(unsigned long long), c->stream));
             SDDMM_LAUNCH(c, k_classify_count, nb, SCAN_BLOCK, c->d_rowptr,
                                panel_owner, c->sM, row_max + 1, seg, c->d_block_sums, c->d_pc, 2,
                                (unsigned int *)nullptr, (unsigned int *)nullptr);
@@ -1405,13 +1405,10 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
         // about as long as what 3 072 wavefronts would take stay whole: 3 000 rows of 554 entries of 1 KiB 264 us, in
         // pieces of 512 280.
         const int64_t even = ((item_entries / 3072 + WAVE - 1) / WAVE) * WAVE;
-        const bool uneven = (int64_t)first.max_len > 2 * std::max<int64_t>(256, std::min<int64_t>(seg, even));
-        const int best_seg = uneven && !getenv("SDDMM_FUSED_SEG") ? 256 : seg;
-        // Workgroups of one wavefront only where lengths differ: the place on the CU is then free as soon as an item ends
-        // (four / one: graphs of 200 k rows, K=64 fp16 78.3 / 74.3 us, K=8 bf16 54.6 / 51.4, K=16 42.6 / 40.5).  Rows of about
-        // one length end together, and neighbours share B rows in the vector L1 (banded blocks of 36 k rows K=256 499 / 522,
-        // K=16 67.7 / 71.0; uniform rows of 45 entries K=8 bf16 222 / 232).
-        c->fused_block_waves = uneven ? 1 : WAVES_PER_BLOCK;
+        const int longer = (int)std::max<int64_t>(256, std::min<int64_t>(seg, even));
+        bool uneven = (int64_t)first.fused_longest > 2 * (int64_t)longer;
+        const bool choose_seg = uneven && !getenv("SDDMM_FUSED_SEG");
+        const int best_seg = choose_seg ? 256 : seg;
         // Where most of the short rows are very short, one of 17 .. 64 entries among them holds up the rows of its
         // wavefront: those become items too (graphs of 2.8 .. 4 entries per short row, 64 against 16: 50 k rows K=64
         // 46 -> 35 us; 200 k rows K=8 60 -> 44 us, K=64 fp16 92 -> 77, K=128 251 -> 218; 1 M rows K=64 606 -> 566;
@@ -1423,8 +1420,25 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
             row_max = best_row_max;
             rc = count();
             if (rc) return rc;
+            // Where that would cut more than a third of the items, most rows are about one length and a few are longer: only
+            // those are cut.  (The share is a fifth to a quarter in graphs.  256 / this rule: 36 000 rows of 392 entries and
+            // one of 3 365, K=256 766 / 552 us, K=16 92 / 65; 20 000 rows of 390 and 500 of 4 000, K=64 245 / 243, K=16 85 / 78;
+            // no row cut that stays whole now, 20 000 rows of 100 and 100 of 4 000: K=64 78 us with 256, 93 without.)
+            if (choose_seg && longer > seg && 3 * (counted.rows_long - first.rows_long) > first.rows_medium + first.rows_long) {
+                uneven = false;
+                seg = longer;
+                rc = count();
+                if (rc) return rc;
+            }
+        }
+        // Workgroups of one wavefront only where lengths differ: the place on the CU is then free as soon as an item ends
+        // (four / one: graphs of 200 k rows, K=64 fp16 78.3 / 74.3 us, K=8 bf16 54.6 / 51.4, K=16 42.6 / 40.5).  Rows of about
+        // one length end together, and neighbours share B rows in the vector L1 (banded blocks of 36 k rows K=256 499 / 522,
+        // K=16 67.7 / 71.0; uniform rows of 45 entries K=8 bf16 222 / 232).
+        c->fused_block_waves = uneven ? 1 : WAVES_PER_BLOCK;
+        if (row_max != FUSED_ROW_MAX) {
             // (a launch takes fewer than 2^32 threads: 2^26 items, which rows of more than 64 entries cannot reach)
-            if (row_max != FUSED_ROW_MAX && xcd_grid(blocks_of((int64_t)tmp.n_items, c->fused_block_waves)) * c->fused_block_waves * WAVE >= (int64_t)1 << 32) {
+            if (xcd_grid(blocks_of((int64_t)tmp.n_items, c->fused_block_waves)) * c->fused_block_waves * WAVE >= (int64_t)1 << 32) {
                 row_max = FUSED_ROW_MAX;
                 rc = count();
                 if (rc) return rc;

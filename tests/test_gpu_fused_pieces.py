@@ -92,3 +92,33 @@ def test_room_for_fewer_pieces_only(engine_factory, monkeypatch):
             got.append(_check(e, rowptr, col, val, A, B, name))
     np.testing.assert_array_equal(got[0], got[1])
     assert (got[0] != got[2]).any()
+
+
+@pytest.mark.parametrize("panel_rows,longer", [(0, 3), (0, 1100), (256, 0)])
+def test_a_few_longer_rows_do_not_cut_the_others(engine_factory, monkeypatch, panel_rows, longer):
+    """3 600 rows of about 380 entries stay whole beside 3 rows of 2 000, and beside 256 rows of 1 100 that the panel
+    kernel takes; beside 1 100 rows of 2 000 too (they are three quarters of the items).  The sums of a row tell whether
+    it was cut."""
+    rng = np.random.default_rng(5)
+    N, bulk, K = 3000, 3600, 32
+    lens = np.concatenate([np.full(panel_rows, 1100), rng.integers(375, 386, bulk), np.full(longer, 2000)]).astype(np.int64)
+    rowptr, col, val = _matrix(rng, N, lens)
+    for r in range(panel_rows):                                # eight rows on the columns of the first
+        a = rowptr[r // 8 * 8]
+        col[rowptr[r]:rowptr[r + 1]] = col[a:a + 1100]
+    M = len(lens)
+    A, _, B, _ = _operands(rng, M, N, K, capi.F32)
+    got = {}
+    for seg in (None, "4096", "256"):                          # by rule, every row whole, every row cut
+        with monkeypatch.context() as m, engine_factory() as e:
+            if seg:
+                m.setenv("SDDMM_FUSED_SEG", seg)
+            e.set_dense(A, B)
+            e.set_csr(M, N, rowptr, col, val)
+            got[seg] = _check(e, rowptr, col, val, A, B, str(seg))
+            assert e.stats().kernels_launched == (3 if panel_rows else 2)
+    rows = slice(panel_rows, panel_rows + bulk)
+    np.testing.assert_array_equal(got[None][rows], got["4096"][rows])
+    assert (got["256"][rows] != got["4096"][rows]).any()
+    if longer:
+        assert (got[None][panel_rows + bulk:] != got["4096"][panel_rows + bulk:]).any()
