@@ -144,6 +144,7 @@ struct sddmm_ctx {
     double fused_short_avg = 0.0;    // entries per non-empty row of at most FUSED_ROW_MAX entries (panel rows apart)
     int fused_row_max = FUSED_ROW_MAX;   // rows beyond it are work items of their own
     int fused_seg = 0;               // of at most so many entries
+    bool fused_rows_alike = false;   // most rows beyond fused_row_max look like the row after them (banded blocks, dense tiles)
     int fused_block_waves = WAVES_PER_BLOCK;   // wavefronts per workgroup of the fused gather kernels
     float *d_fused_parts = nullptr;  // partial output rows of the pieces of the rows cut into several items
     int64_t n_fused_pieces = 0, fused_part_floats = 0;

@@ -85,7 +85,15 @@ __device__ __forceinline__ void add_cut_rows(const float *__restrict__ parts, fl
     }
 }
 
-template <class L>
+// STEPS: one step after the other, and no more of them than the item has, instead of whole batches of steps (the sums are
+// the same bit for bit).  The batches hold the values of several steps and both products in registers (a lane with two fp32
+// units 82 instead of 53, with four bf16 units 170 instead of 127): a wavefront is faster and the chip holds fewer of them.
+// What that gives and costs (steps / batches): near-dense rows, fewer of them than there are places, K = 128 fp16 75 / 68
+// us; dense tiles K = 256 fp16 194 / 151; 3 000 rows of 300 .. 700 entries K = 64 50 / 38; graphs of 50 000 rows K = 64
+// 43 / 37.7; 36 000 banded rows that share their columns with their neighbours K = 256 fp16 379 / 310; but 20 000 rows of
+// 390 random columns out of 40 000, where the wavefronts in flight walk B together from one end to the other, K = 64
+// 120 / 186, K = 192 fp16 246 / 287, and 30 000 rows of 65 .. 127 entries K = 128 bf16 92 / 102 (fused_in_steps: the rule).
+template <class L, bool STEPS>
 __global__ __launch_bounds__(BLOCK) void k_fusedmm(const void *__restrict__ A, const void *__restrict__ B, int KU,
                                                    const int32_t *__restrict__ rowptr,
                                                    const int32_t *__restrict__ col,
@@ -151,8 +159,7 @@ __global__ __launch_bounds__(BLOCK) void k_fusedmm(const void *__restrict__ A, c
         constexpr int N = sizeof(bf) / sizeof(bf[0]);
         float p[N];
         bool live[N];
-#pragma unroll
-        for (int q = 0; q < N; ++q) {
+        auto product = [&](int q) {
             const int src = ((t0 + q) * G + g) & (WAVE - 1);
             float d = 0.f;
 #pragma unroll
@@ -167,9 +174,8 @@ __global__ __launch_bounds__(BLOCK) void k_fusedmm(const void *__restrict__ A, c
                 live[q] = x.base + src < end;
                 p[q] = live[q] ? p[q] : 0.f;
             }
-        }
-#pragma unroll
-        for (int q = 0; q < N; ++q) {
+        };
+        auto update = [&](int q) {
 #pragma unroll
             for (int i = 0; i < UPL; ++i) {
                 float next[E];
@@ -180,6 +186,20 @@ __global__ __launch_bounds__(BLOCK) void k_fusedmm(const void *__restrict__ A, c
                 for (int e = 0; e < E; ++e) acc[i][e] = FULL || live[q] ? next[e] : acc[i][e];
             }
             if (j == t0 + q) out = p[q];
+        };
+        if constexpr (STEPS) {
+            const int steps = (end - x.base + G - 1) / G;
+#pragma unroll
+            for (int q = 0; q < N; ++q) {
+                if (t0 + q >= steps) break;                   // wave-uniform
+                product(q);
+                update(q);
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < N; ++q) product(q);
+#pragma unroll
+            for (int q = 0; q < N; ++q) update(q);
         }
     };
     // entry l = t*G+g was kept by lane g*LPN+t
@@ -214,7 +234,24 @@ __global__ __launch_bounds__(BLOCK) void k_fusedmm(const void *__restrict__ A, c
     // third of their wavefronts per SIMD, 171 against 153 us on banded rows of 256 bytes.)
     constexpr bool AHEAD = UPL == 1 && NB == LPN;
     Ent cur = entry(start);
-    if (end - start >= WAVE) {
+    if constexpr (STEPS) {
+        Ent nxt = entry(start + WAVE);
+        for (int base = start; base < end; base += WAVE) {
+            const Ent after = entry(base + 2 * WAVE);
+            const int steps = (end - base + G - 1) / G;
+            float out = 0.f;
+#pragma unroll
+            for (int t0 = 0; t0 < LPN; t0 += NB) {
+                if (t0 >= steps) break;                       // wave-uniform
+                T bf[NB][UPL];
+                gather(cur, t0, bf);
+                consume(part, cur, t0, bf, out);
+            }
+            store_p(cur, out);
+            cur = nxt;
+            nxt = after;
+        }
+    } else if (end - start >= WAVE) {
         T bcur[NB][UPL];
         if constexpr (AHEAD) gather(cur, 0, bcur);
         Ent nxt = entry(start + WAVE);
@@ -241,7 +278,9 @@ __global__ __launch_bounds__(BLOCK) void k_fusedmm(const void *__restrict__ A, c
             nxt = after;
         }
     }
-    if (cur.base < end) tail(cur);
+    if constexpr (!STEPS) {
+        if (cur.base < end) tail(cur);
+    }
     // add the partial output rows of the G groups: lanes with the same j
 #pragma unroll
     for (int off = LPN; off < WAVE; off <<= 1) {

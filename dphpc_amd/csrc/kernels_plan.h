@@ -20,6 +20,7 @@ struct PlanCounters {
     unsigned long long n_utiles, nnz_utiles, utiles_scanned;  // dense-tile path: union strips
     unsigned long long n_panels, nnz_panels, panel_items;     // row-panel path
     unsigned int fused_longest;    // fused call: longest row that its gather kernels take
+    unsigned long long rows_alike; // fused call: work-item rows that look like the next row (its length, its first column)
 };
 
 // The same counters on the device.  Sums that thousands of workgroups contribute to
@@ -30,6 +31,7 @@ constexpr int SPREAD = 64;
 enum CounterKind {
     K_ROWS_NONEMPTY = 0,
     K_ROWS_SHORT, K_ROWS_MEDIUM, K_ROWS_LONG, K_NNZ_SHORT, K_NNZ_MEDIUM, K_NNZ_LONG,   // row classifier
+    K_ROWS_ALIKE,                                                                      // and for the fused call
     K_TILES, K_NNZ_TILES, K_UTILES, K_NNZ_UTILES, K_PANELS, K_NNZ_PANELS,              // ownership classifiers
     K_COO_JUMPS,                                                                       // validation of COO entries
     K_KINDS
@@ -61,6 +63,7 @@ inline PlanCounters summarize(const DevCounters &d) {
     }
     p.rows_nonempty = sum[K_ROWS_NONEMPTY];
     p.coo_jumps = sum[K_COO_JUMPS];
+    p.rows_alike = sum[K_ROWS_ALIKE];
     p.rows_short = sum[K_ROWS_SHORT]; p.rows_medium = sum[K_ROWS_MEDIUM]; p.rows_long = sum[K_ROWS_LONG];
     p.nnz_short = sum[K_NNZ_SHORT]; p.nnz_medium = sum[K_NNZ_MEDIUM]; p.nnz_long = sum[K_NNZ_LONG];
     p.n_tiles = sum[K_TILES]; p.nnz_tiles = sum[K_NNZ_TILES];
@@ -300,16 +303,21 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int3
                                                                int ts, int seg, unsigned int *__restrict__ block_sums,
                                                                DevCounters *pc, int only,
                                                                unsigned int *__restrict__ short_sums,
-                                                               unsigned int *__restrict__ long_sums) {
+                                                               unsigned int *__restrict__ long_sums,
+                                                               const int32_t *__restrict__ col) {
     const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
     unsigned int items = 0, longest = 0;
-    unsigned long long r_short = 0, r_med = 0, r_long = 0, n_short = 0, n_med = 0, n_long = 0;
+    unsigned long long r_alike = 0, r_short = 0, r_med = 0, r_long = 0, n_short = 0, n_med = 0, n_long = 0;
     for (int q = 0; q < SCAN_ITEMS; ++q) {
         unsigned int len;
         const unsigned int cnt = row_item_count(rowptr, owner, base + q, M, ts, seg, &len, only);
         items += cnt;
         longest = len > longest ? len : longest;
         if (len == 0) continue;
+        if (only && cnt > 0 && base + q + 1 < M) {
+            const int32_t a = rowptr[base + q], b = rowptr[base + q + 1];
+            if ((unsigned int)(rowptr[base + q + 2] - b) == len && col[a] == col[b]) ++r_alike;
+        }
         if (cnt == 0) { ++r_short; n_short += len; }
         else if (cnt == 1) { ++r_med; n_med += len; }
         else { ++r_long; n_long += len; }
@@ -335,6 +343,8 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int3
     if (threadIdx.x < 6) spread_add(pc, K_ROWS_SHORT + (int)threadIdx.x, sh[threadIdx.x]);
     if (only) {                                       // the fused call (most workgroups find a longer row there already)
         longest = wave_max_u32(longest);
+        r_alike = wave_sum_u64(r_alike);
+        if (lane_id() == 0 && r_alike) spread_add(pc, K_ROWS_ALIKE, r_alike);
         if (lane_id() == 0 && longest > pc->fused_longest) atomicMax(&pc->fused_longest, (unsigned long long)longest);
     }
     // entries of this block's short rows, for the entry list (k_short_list_write)

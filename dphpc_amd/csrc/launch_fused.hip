@@ -2,6 +2,19 @@
 #include "context.h"
 #include "kernels_fused.h"
 
+// k_fusedmm in steps (its comment has both sides): items of about one length (they were not cut to 256 entries), more of
+// them than the chip holds wavefronts (256 CUs x 32), and neighbouring rows do not share their columns.  Lanes with four
+// bf16 units lose half of their places to the batches: steps whatever the number and the columns (steps / batches: 3 000
+// rows of 300 .. 700 entries 77 / 88 us, near-dense rows 141 / 147, banded rows 390 / 405), batches in graphs (73 / 71).
+// SDDMM_FUSED_STEPS 0 / 1 overrides it.
+template <class L>
+bool fused_in_steps(const sddmm_ctx *c) {
+    const int mode = env_int("SDDMM_FUSED_STEPS", -1);
+    if (mode >= 0) return mode != 0;
+    if (c->fused_block_waves == 1) return false;
+    return (L::U::DT == DT_BF16 && L::UPL >= 4) || (c->n_fused_items > 256 * 32 && !c->fused_rows_alike);
+}
+
 // The work items of the rows of more than fused_row_max entries, then the other rows; 0: no kernel for this row layout.
 int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
     const Shape s = shape_of(c);
@@ -26,10 +39,15 @@ int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
             const int64_t rblocks = blocks_of(waves, c->fused_block_waves);
             if (c->n_fused_items > 0) {
                 const int64_t nblocks = blocks_of(c->n_fused_items, c->fused_block_waves);
-                SDDMM_LAUNCH(c, (k_fusedmm<LT>), xcd_grid(nblocks), c->fused_block_waves * WAVE,
-                                   (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col,
-                                   c->d_sval, c->dP, c->dO, c->d_fused_parts, (const RowItem *)c->d_fused_items,
-                                   c->n_fused_items, nblocks);
+                auto launch = [&](auto kernel) {
+                    SDDMM_LAUNCH(c, kernel, xcd_grid(nblocks), c->fused_block_waves * WAVE,
+                                       (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col,
+                                       c->d_sval, c->dP, c->dO, c->d_fused_parts, (const RowItem *)c->d_fused_items,
+                                       c->n_fused_items, nblocks);
+                };
+                if constexpr (LT::UPL == 1) launch(k_fusedmm<LT, false>);
+                else if (fused_in_steps<LT>(c)) launch(k_fusedmm<LT, true>);
+                else launch(k_fusedmm<LT, false>);
                 ++launches;
             }
             if (balanced) {
@@ -51,4 +69,4 @@ int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
     return launches;
 }
 
-hipError_t load_fused() { return load_code(reinterpret_cast<const void *>(k_fusedmm<Layout<UnitF32x4, 8, 1, true, false>>)); }
+hipError_t load_fused() { return load_code(reinterpret_cast<const void *>(k_fusedmm<Layout<UnitF32x4, 8, 1, true, false>, false>)); }

@@ -202,7 +202,8 @@ int classify_rows_count(sddmm_ctx *c, bool again = false) {
     if (nb > 0) {
         const unsigned char *owner = c->owner_active ? c->d_owner : nullptr;
         SDDMM_LAUNCH(c, k_classify_count, nb, SCAN_BLOCK, c->d_rowptr, owner,
-                           c->sM, c->ts, c->seg, c->d_block_sums, c->d_pc, 0, c->d_short_sums, c->d_long_sums);
+                           c->sM, c->ts, c->seg, c->d_block_sums, c->d_pc, 0, c->d_short_sums, c->d_long_sums,
+                           (const int32_t *)nullptr);
         LAUNCH_CHECK(c);
         if (nb <= SCAN_SMALL_MAX) {
             int rc = queue_scan(c, c->d_block_sums, c->d_block_sums, nb, &c->d_pc->n_items);
@@ -1381,11 +1382,11 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
         PlanCounters counted;
         auto count = [&]() -> int {
             HIP_TRY(c, hipMemsetAsync(&c->d_pc->k[K_ROWS_SHORT][0], 0,
-                                      sizeof(unsigned long long) * SPREAD * (K_NNZ_LONG - K_ROWS_SHORT + 1), c->stream));
+                                      sizeof(unsigned long long) * SPREAD * (K_ROWS_ALIKE - K_ROWS_SHORT + 1), c->stream));
             HIP_TRY(c, hipMemsetAsync(&c->d_pc->n_items, 0, 2 * sizeof(unsigned long long), c->stream));
             SDDMM_LAUNCH(c, k_classify_count, nb, SCAN_BLOCK, c->d_rowptr,
                                panel_owner, c->sM, row_max + 1, seg, c->d_block_sums, c->d_pc, 2,
-                               (unsigned int *)nullptr, (unsigned int *)nullptr);
+                               (unsigned int *)nullptr, (unsigned int *)nullptr, (const int32_t *)c->d_col);
             SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, c->d_block_sums, (int)nb,
                                &c->d_pc->n_items);
             LAUNCH_CHECK(c);
@@ -1398,6 +1399,7 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
         if (rc) return rc;
         const PlanCounters first = counted;
         const int64_t item_entries = (int64_t)(first.nnz_medium + first.nnz_long);
+        c->fused_rows_alike = 2 * first.rows_alike >= first.rows_medium + first.rows_long;
         c->fused_short_avg = first.rows_short ? (double)first.nnz_short / (double)first.rows_short : 0.0;
         // A wavefront walks its item chunk by chunk and the launch waits for the longest one: the long rows are cut into
         // pieces of 256 entries (1024 / 512 / 256: 200 k rows, 128 bytes 85.3 / 84.3 / 81.2 us, 256 bytes 122 / 119 / 116,

@@ -122,3 +122,31 @@ def test_a_few_longer_rows_do_not_cut_the_others(engine_factory, monkeypatch, pa
     assert (got["256"][rows] != got["4096"][rows]).any()
     if longer:
         assert (got[None][panel_rows + bulk:] != got["4096"][panel_rows + bulk:]).any()
+
+
+@pytest.mark.parametrize("K,dtype", [(16, capi.F32), (64, capi.F32), (96, capi.F32), (100, capi.F32), (128, capi.BF16), (136, capi.F16),
+                                     (192, capi.BF16), (192, capi.F32), (256, capi.F32), (256, capi.F16), (256, capi.BF16)])
+def test_steps_and_batches_give_the_same(engine_factory, monkeypatch, K, dtype):
+    """Both forms of the kernel add in the same order.  Rows around its chunks of 64 entries and their halves and quarters;
+    an infinite row of B that no entry names and one that a single row names."""
+    rng = np.random.default_rng(K + dtype)
+    N = 400
+    lens = np.concatenate([np.arange(60, 140), [191, 192, 193, 255, 256, 257, 319, 320, 321, 398, 1]])
+    rowptr, col, val = _matrix(rng, N - 2, lens)
+    Ah, A, Bh, B = _operands(rng, len(lens), N, K, dtype)
+    got = {}
+    for steps in ("0", "1"):
+        monkeypatch.setenv("SDDMM_FUSED_STEPS", steps)
+        with engine_factory() as e:
+            e.set_dense(Ah, Bh, dtype)
+            e.set_csr(len(lens), N, rowptr, col, val)
+            o = _check(e, rowptr, col, val, A, B, "steps " + steps)
+            got[steps] = (o, e.values())
+            wild = Bh.copy()
+            wild[N - 1] = wild[col[-1]] = {capi.F32: np.inf, capi.BF16: 0x7F80, capi.F16: 0x7C00}[dtype]
+            e.set_dense(Ah, wild, dtype)
+            named = np.array([col[-1] in col[rowptr[r]:rowptr[r + 1]] for r in range(len(lens))])
+            o = e.run_fused()
+            assert np.isfinite(o[~named]).all() and not np.isfinite(o[named]).all(axis=1).any()
+    for a, b in zip(got["0"], got["1"]):
+        np.testing.assert_array_equal(a, b)
