@@ -146,6 +146,8 @@ struct sddmm_ctx {
     int fused_seg = 0;               // of at most so many entries
     bool fused_rows_alike = false;   // most rows beyond fused_row_max look like the row after them (banded blocks, dense tiles)
     int fused_block_waves = WAVES_PER_BLOCK;   // wavefronts per workgroup of the fused gather kernels
+    int64_t n_fused_cut = 0;         // rows that k_add_cut_rows completes, listed behind the items (0: the kernel of the short rows does)
+    int fused_add_block = 0;         // its workgroup size
     float *d_fused_parts = nullptr;  // partial output rows of the pieces of the rows cut into several items
     int64_t n_fused_pieces = 0, fused_part_floats = 0;
     float *dO = nullptr;
@@ -360,5 +362,10 @@ bool launch_auto_with_tiles(sddmm_ctx *c);                                      
 void launch_tiles(sddmm_ctx *c);
 void launch_panels(sddmm_ctx *c);                                                // launch_panels.hip
 void launch_panels_fused(sddmm_ctx *c);
+// the list of the rows for k_add_cut_rows
+inline int32_t *fused_cut_rows(const sddmm_ctx *c) {
+    return c->n_fused_cut > 0 ? reinterpret_cast<int32_t *>(c->d_fused_items + c->n_fused_items) : nullptr;
+}
 inline int64_t blocks_of(int64_t waves, int per_block) { return (waves + per_block - 1) / per_block; }
+bool fused_balanced(const sddmm_ctx *c);                                           // which kernel takes the short rows
 int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner);           // launch_fused.hip: number of launches

@@ -16,7 +16,7 @@
 // row.  After the last entry the partial rows of the 64/LPN groups are added with
 // lane permutes; group 0 writes the output row, or, when the row was cut into several
 // items, the partial row of its piece.  The kernel of the short rows, launched after it,
-// adds the pieces of a row in order (add_pieces): O is the same in every run.
+// adds the pieces of a row in order (add_pieces; k_add_cut_rows where they are many): O is the same in every run.
 #pragma once
 #include "kernels_gather.h"
 
@@ -83,6 +83,46 @@ __device__ __forceinline__ void add_cut_rows(const float *__restrict__ parts, fl
         const int n = (int)(((unsigned int)__shfl(len, src, WAVE) + (unsigned int)seg - 1u) / (unsigned int)seg);
         add_pieces<L>(parts, O, KU, (int64_t)shfl_off<uint64_t>((uint64_t)row, src), n, lane);
     }
+}
+
+// The output rows of the cut rows, a workgroup per row: where one wavefront of the kernel of the short rows would add more
+// than FUSED_APART_PIECES pieces, of one very long row or of neighbouring long rows (a graph whose rows are sorted by
+// length), and the launch would wait for it: 10 .. 20 ns a piece.  That costs a launch, 3 .. 4 us.  There / here: 1 M rows,
+// the first 64 of 50 000 entries, K = 32 478 / 223 us; one row of 2.6 M entries K = 64 253 / 171, K = 256 3 468 / 650; 2.6 M
+// rows of a graph sorted by length 1 031 / 984; at the line, one row of 300 000 entries 74.9 / 74.5; below it, 200 000
+// sorted rows K = 64 fp16 79.7 / 83.7.
+// Thread t takes component group t mod Q, Q the power of two that holds a row, and pieces t/Q, t/Q + threads/Q, ..; the
+// sums are added in halves: the same order in every run.
+static __global__ __launch_bounds__(FUSED_APART_BLOCK) void k_add_cut_rows(const float *__restrict__ parts, float *__restrict__ O,
+                                                                       int K, int seg, const int32_t *__restrict__ rowptr,
+                                                                       const int32_t *__restrict__ cut_rows) {
+    __shared__ float4 sum[FUSED_APART_BLOCK];
+    const int64_t row = cut_rows[blockIdx.x];
+    const int quads = K / 4, t = (int)threadIdx.x, threads = (int)blockDim.x;      // (K is a multiple of 4, at most 256)
+    int q = 1;
+    while (q < quads) q *= 2;
+    const int n = (int)(((unsigned int)(rowptr[row + 1] - rowptr[row]) + (unsigned int)seg - 1u) / (unsigned int)seg);
+    float4 *orow = reinterpret_cast<float4 *>(O + row * K);
+    const float4 *part = reinterpret_cast<const float4 *>(parts + (int64_t)__float_as_int(O[row * K]) * K);
+    const int u = t & (q - 1);
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (u < quads) {
+#pragma unroll 4
+        for (int p = t / q; p < n; p += threads / q) {
+            const float4 v = part[(int64_t)p * quads + u];
+            acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
+        }
+    }
+    sum[t] = acc;
+    for (int half = threads / 2; half >= q; half /= 2) {
+        __syncthreads();
+        if (t < half) {
+            const float4 v = sum[t + half];
+            acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
+            sum[t] = acc;
+        }
+    }
+    if (t < quads) orow[t] = acc;                     // (every thread has read the place in it before the first barrier)
 }
 
 // STEPS: one step after the other, and no more of them than the item has, instead of whole batches of steps (the sums are

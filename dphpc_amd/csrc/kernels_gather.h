@@ -35,6 +35,8 @@ constexpr int WAVES_PER_BLOCK = BLOCK / WAVE;
 // neighbours hold the same columns lose what they find in the CU's L1 (banded blocks K = 42 59 -> 92, dense tiles K = 120
 // bf16 30 -> 35) and items of a few bytes wait for their dispatch (45 entries per row, K = 8 bf16, 20 -> 36).
 constexpr int block_item_waves(int units_per_lane) { return units_per_lane <= 4 ? 1 : WAVES_PER_BLOCK; }
+constexpr int FUSED_APART_PIECES = 1024;   // more pieces than that for one wavefront of the kernel of the short rows: k_add_cut_rows
+constexpr int FUSED_APART_BLOCK = 1024;
 constexpr int FUSED_ROW_MAX = 64;          // fused SDDMM + SpMM: rows up to this length take one lane group each (a quarter of it: plan_fused_items)
 
 // Byte offset of a row: 32-bit when the whole operand is below 4 GiB (one VALU

@@ -20,6 +20,7 @@ struct PlanCounters {
     unsigned long long n_utiles, nnz_utiles, utiles_scanned;  // dense-tile path: union strips
     unsigned long long n_panels, nnz_panels, panel_items;     // row-panel path
     unsigned int fused_longest;    // fused call: longest row that its gather kernels take
+    unsigned long long fused_window;   // fused call: most pieces of cut rows among the rows of a wavefront
     unsigned long long rows_alike; // fused call: work-item rows that look like the next row (its length, its first column)
 };
 
@@ -38,12 +39,12 @@ enum CounterKind {
 };
 struct DevCounters {
     unsigned int bad_pattern, coo_unsorted, pad0, pad1;
-    unsigned long long n_items, fused_longest;                       // (one fill clears both; PlanCounters)
+    unsigned long long n_items, fused_longest, fused_window;         // (one fill clears them; PlanCounters)
     unsigned long long tiles_scanned, panel_items;                   // scan totals, one writer each, as is n_items
     unsigned long long n_candidates;                                 // rows offered to the gathered strips
     unsigned long long utiles_scanned, short_scanned;                // scan totals: union strips, entries of the short rows
     unsigned long long long_scanned;                                 // scan total: rows of more than one item
-    unsigned long long fused_pieces;                                 // places given to the pieces of cut rows
+    unsigned long long fused_pieces, fused_cut;                      // places given to the pieces of cut rows, to those rows
     unsigned int max_len[SPREAD];
     unsigned long long k[K_KINDS][SPREAD];
 };
@@ -70,6 +71,7 @@ inline PlanCounters summarize(const DevCounters &d) {
     p.n_utiles = sum[K_UTILES]; p.nnz_utiles = sum[K_NNZ_UTILES]; p.utiles_scanned = d.utiles_scanned;
     p.n_panels = sum[K_PANELS]; p.nnz_panels = sum[K_NNZ_PANELS];
     p.fused_longest = (unsigned int)d.fused_longest;
+    p.fused_window = d.fused_window;
     p.n_items = d.n_items; p.tiles_scanned = d.tiles_scanned; p.panel_items = d.panel_items;
     return p;
 }
@@ -304,15 +306,16 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int3
                                                                DevCounters *pc, int only,
                                                                unsigned int *__restrict__ short_sums,
                                                                unsigned int *__restrict__ long_sums,
-                                                               const int32_t *__restrict__ col) {
+                                                               const int32_t *__restrict__ col, int window) {
     const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
-    unsigned int items = 0, longest = 0;
+    unsigned int items = 0, longest = 0, pieces = 0;
     unsigned long long r_alike = 0, r_short = 0, r_med = 0, r_long = 0, n_short = 0, n_med = 0, n_long = 0;
     for (int q = 0; q < SCAN_ITEMS; ++q) {
         unsigned int len;
         const unsigned int cnt = row_item_count(rowptr, owner, base + q, M, ts, seg, &len, only);
         items += cnt;
         longest = len > longest ? len : longest;
+        pieces += cnt > 1 ? cnt : 0;
         if (len == 0) continue;
         if (only && cnt > 0 && base + q + 1 < M) {
             const int32_t a = rowptr[base + q], b = rowptr[base + q + 1];
@@ -341,8 +344,11 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int3
     }
     __syncthreads();
     if (threadIdx.x < 6) spread_add(pc, K_ROWS_SHORT + (int)threadIdx.x, sh[threadIdx.x]);
-    if (only) {                                       // the fused call (most workgroups find a longer row there already)
+    if (only) {                                       // the fused call (most workgroups find as much there already)
         longest = wave_max_u32(longest);
+        for (int o = 1; o < window / SCAN_ITEMS; o <<= 1) pieces += __shfl_xor(pieces, o, WAVE);
+        pieces = wave_max_u32(pieces);
+        if (lane_id() == 0 && pieces > pc->fused_window) atomicMax(&pc->fused_window, (unsigned long long)pieces);
         r_alike = wave_sum_u64(r_alike);
         if (lane_id() == 0 && r_alike) spread_add(pc, K_ROWS_ALIKE, r_alike);
         if (lane_id() == 0 && longest > pc->fused_longest) atomicMax(&pc->fused_longest, (unsigned long long)longest);
@@ -489,13 +495,15 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_write(const int3
 // Places for the partial output rows of the fused call's pieces (kernels_fused.h): the pieces of a row that was cut
 // into several items lie next to each other, in order; which row comes first does not matter.  One thread per item,
 // the first item of a cut row writes the places of them all (they follow it in the list); one atomic per wavefront
-// that holds such an item.
+// that holds such an item.  cut_rows (if given): the cut rows, in any order.
 static __global__ __launch_bounds__(256) void k_piece_places(const int32_t *__restrict__ rowptr, RowItem *__restrict__ items,
-                                                             int64_t n_items, DevCounters *pc) {
+                                                             int64_t n_items, int32_t *__restrict__ cut_rows, DevCounters *pc) {
     const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     unsigned int n = 0;
+    int row = 0;
     if (w < n_items) {
-        const int row = items[w].row, start = items[w].start, end = items[w].end;
+        row = items[w].row;
+        const int start = items[w].start, end = items[w].end;
         const int rs = rowptr[row], re = rowptr[row + 1];
         if (start == rs && end != re) n = ((unsigned int)(re - rs) + (unsigned int)(end - start) - 1u) / (unsigned int)(end - start);
     }
@@ -510,6 +518,12 @@ static __global__ __launch_bounds__(256) void k_piece_places(const int32_t *__re
     if (lane == WAVE - 1) first = (unsigned int)atomicAdd(&pc->fused_pieces, (unsigned long long)incl);
     first = __shfl(first, WAVE - 1, WAVE) + incl - n;
     for (unsigned int k = 0; k < n; ++k) items[w + k].extra = (int32_t)(first + k);
+    if (!cut_rows) return;
+    const unsigned long long cut = __ballot(n != 0);
+    unsigned int at = 0;
+    if (lane == 0) at = (unsigned int)atomicAdd(&pc->fused_cut, (unsigned long long)__popcll(cut));
+    at = __shfl(at, 0, WAVE) + (unsigned int)__popcll(cut & ((1ull << lane) - 1ull));
+    if (n != 0) cut_rows[at] = row;
 }
 
 // ---------------------------------------------------------------------------

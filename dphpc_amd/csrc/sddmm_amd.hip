@@ -125,7 +125,7 @@ void release_sparse(sddmm_ctx *c) {
     c->order_cap = 0;
     c->use_order = false;
     dfree(c->d_fused_items, idle);
-    c->n_fused_items = c->fused_items_cap = 0;
+    c->n_fused_items = c->n_fused_cut = c->fused_items_cap = 0;
     dfree(c->d_fused_parts, idle);
     c->n_fused_pieces = c->fused_part_floats = 0;
     c->fused_items_valid = c->have_fused = false;
@@ -203,7 +203,7 @@ int classify_rows_count(sddmm_ctx *c, bool again = false) {
         const unsigned char *owner = c->owner_active ? c->d_owner : nullptr;
         SDDMM_LAUNCH(c, k_classify_count, nb, SCAN_BLOCK, c->d_rowptr, owner,
                            c->sM, c->ts, c->seg, c->d_block_sums, c->d_pc, 0, c->d_short_sums, c->d_long_sums,
-                           (const int32_t *)nullptr);
+                           (const int32_t *)nullptr, 0);
         LAUNCH_CHECK(c);
         if (nb <= SCAN_SMALL_MAX) {
             int rc = queue_scan(c, c->d_block_sums, c->d_block_sums, nb, &c->d_pc->n_items);
@@ -1376,17 +1376,19 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
     const int arc = ensure_arena(c);
     if (arc) return arc;
     ARENA_HOLDS(c, nb, c->block_sums_cap, "block sums");
-    c->n_fused_items = c->n_fused_pieces = 0;
+    c->n_fused_items = c->n_fused_pieces = c->n_fused_cut = 0;
     if (nb > 0) {
         DevCounters tmp;
         PlanCounters counted;
+        int window = WAVE / shape_of(c).LPN;               // rows of a wavefront of the kernel of the short rows
         auto count = [&]() -> int {
             HIP_TRY(c, hipMemsetAsync(&c->d_pc->k[K_ROWS_SHORT][0], 0,
                                       sizeof(unsigned long long) * SPREAD * (K_ROWS_ALIKE - K_ROWS_SHORT + 1), c->stream));
-            HIP_TRY(c, hipMemsetAsync(&c->d_pc->n_items, 0, 2 * sizeof(unsigned long long), c->stream));
+            HIP_TRY(c, hipMemsetAsync(&c->d_pc->n_items, 0, 3 * sizeof(unsigned long long), c->stream));
             SDDMM_LAUNCH(c, k_classify_count, nb, SCAN_BLOCK, c->d_rowptr,
                                panel_owner, c->sM, row_max + 1, seg, c->d_block_sums, c->d_pc, 2,
-                               (unsigned int *)nullptr, (unsigned int *)nullptr, (const int32_t *)c->d_col);
+                               (unsigned int *)nullptr, (unsigned int *)nullptr, (const int32_t *)c->d_col,
+                               window);
             SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, c->d_block_sums, (int)nb,
                                &c->d_pc->n_items);
             LAUNCH_CHECK(c);
@@ -1401,6 +1403,7 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
         const int64_t item_entries = (int64_t)(first.nnz_medium + first.nnz_long);
         c->fused_rows_alike = 2 * first.rows_alike >= first.rows_medium + first.rows_long;
         c->fused_short_avg = first.rows_short ? (double)first.nnz_short / (double)first.rows_short : 0.0;
+        if (fused_balanced(c)) window = WAVE;              // (those rows are so short that they are counted again, below)
         // A wavefront walks its item chunk by chunk and the launch waits for the longest one: the long rows are cut into
         // pieces of 256 entries (1024 / 512 / 256: 200 k rows, 128 bytes 85.3 / 84.3 / 81.2 us, 256 bytes 122 / 119 / 116,
         // 512 bytes 228 / 223 / 218; 1 M rows of 128 bytes 289 / 284 / 281; 2.6 M rows 800 / 793 / 787).  Rows that are all
@@ -1455,18 +1458,24 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
             if (rc) return rc;
         }
         c->n_fused_items = (int64_t)tmp.n_items;
-        if (c->n_fused_items > c->fused_items_cap) {
+        const int apart = env_int("SDDMM_FUSED_ADD_APART", -1);
+        if (apart >= 0 ? apart != 0 : counted.fused_window > FUSED_APART_PIECES) c->n_fused_cut = (int64_t)counted.rows_long;
+        // (a launch takes fewer than 2^32 threads)
+        c->fused_add_block = counted.fused_longest / (unsigned int)seg > 512 && c->n_fused_cut < 65536 ? FUSED_APART_BLOCK : 256;
+        const int64_t room = c->n_fused_items + (c->n_fused_cut + 3) / 4;           // a list of rows behind the items
+        if (room > c->fused_items_cap) {
             dfree(c->d_fused_items);
-            ALLOC_TRY(c, c->d_fused_items, (size_t)c->n_fused_items * sizeof(RowItem));
-            c->fused_items_cap = c->n_fused_items;
+            c->fused_items_cap = 0;
+            ALLOC_TRY(c, c->d_fused_items, (size_t)room * sizeof(RowItem));
+            c->fused_items_cap = room;
         }
         if (c->n_fused_items > 0) {
             SDDMM_LAUNCH(c, k_classify_write, nb, SCAN_BLOCK, c->d_rowptr,
                                panel_owner, c->sM, row_max + 1, seg, c->d_block_sums, c->d_fused_items, 2);
             if (c->n_fused_pieces > 0) {
-                HIP_TRY(c, hipMemsetAsync(&c->d_pc->fused_pieces, 0, sizeof(unsigned long long), c->stream));
+                HIP_TRY(c, hipMemsetAsync(&c->d_pc->fused_pieces, 0, 2 * sizeof(unsigned long long), c->stream));
                 SDDMM_LAUNCH(c, k_piece_places, grid_for(c->n_fused_items, 256), 256, (const int32_t *)c->d_rowptr,
-                             c->d_fused_items, c->n_fused_items, c->d_pc);
+                             c->d_fused_items, c->n_fused_items, fused_cut_rows(c), c->d_pc);
             }
             LAUNCH_CHECK(c);
         }

@@ -150,3 +150,43 @@ def test_steps_and_batches_give_the_same(engine_factory, monkeypatch, K, dtype):
             assert np.isfinite(o[~named]).all() and not np.isfinite(o[named]).all(axis=1).any()
     for a, b in zip(got["0"], got["1"]):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("K,dtype", [(4, capi.F32), (12, capi.F32), (64, capi.F16), (100, capi.F32), (160, capi.BF16), (256, capi.F32)])
+@pytest.mark.parametrize("env", [{}, {"SDDMM_FUSED_SEG": "64"}, {"SDDMM_FUSED_BALANCED": "1"}])
+def test_pieces_added_by_a_kernel_of_their_own(engine_factory, monkeypatch, K, dtype, env):
+    monkeypatch.setenv("SDDMM_FUSED_ADD_APART", "1")
+    for name, value in env.items():
+        monkeypatch.setenv(name, value)
+    rng = np.random.default_rng(K)
+    N, M = 6000, 350
+    lens = rng.integers(0, 9, M)
+    lens[[0, 1, 2, 63, 64, 65, 200, M - 1]] = [2048, 256, 257, 513, 5900, 1025, 64, 700]
+    rowptr, col, val = _matrix(rng, N, lens)
+    Ah, A, Bh, B = _operands(rng, M + 2, N, K, dtype)
+    with engine_factory() as e:
+        e.set_dense(Ah, Bh, dtype)
+        for _ in range(2):                                     # a new pattern in the same blocks
+            e.set_csr(M, N, rowptr, col, val)
+            first = _check(e, rowptr, col, val, A, B, "K=%d %s" % (K, env))
+            assert e.stats().kernels_launched == 3
+            for _ in range(5):
+                np.testing.assert_array_equal(e.run_fused(), first)
+
+
+@pytest.mark.parametrize("hubs,length,balanced,apart", [(64, 5000, "1", True), (64, 5000, "0", False), (1, 262144, "0", False),
+                                                        (1, 262145, "0", True), (1, 600000, "0", True), (0, 0, "0", False)])
+def test_which_kernel_adds_the_pieces(engine_factory, monkeypatch, hubs, length, balanced, apart):
+    """More than 1 024 pieces of 256 entries for one wavefront of the kernel of the short rows: it takes 64 rows, or 16 at K = 16."""
+    monkeypatch.setenv("SDDMM_FUSED_BALANCED", balanced)
+    rng = np.random.default_rng(hubs + 1)
+    N = max(6000, length + 10)
+    lens = np.concatenate([rng.integers(1, 5, 640), np.full(hubs, length)]).astype(np.int64)
+    rowptr, col, val = _matrix(rng, N, lens)
+    A, _, B, _ = _operands(rng, len(lens), N, 16, capi.F32)
+    with engine_factory() as e:
+        e.set_dense(A, B)
+        e.set_csr(len(lens), N, rowptr, col, val)
+        first = _check(e, rowptr, col, val, A, B, "hubs")
+        assert e.stats().kernels_launched == (3 if apart else 2 if hubs else 1)
+        np.testing.assert_array_equal(e.run_fused(), first)
