@@ -1356,9 +1356,13 @@ int sddmm_run(sddmm_ctx *c) {
     return SDDMM_OK;
 }
 
-// Room for the partial output rows of the pieces (K floats each); false when the device does not have it.
-static bool fused_parts(sddmm_ctx *c) {
+// Room for the partial output rows of the pieces of at most seg entries (K floats each); false when the device does not
+// have it.  256 entries a piece can take K / 64 bytes per stored entry: beyond SDDMM_FUSED_PARTS_MAX MiB (1 024 by default)
+// they have to be longer.
+static bool fused_parts(sddmm_ctx *c, int seg) {
     const int64_t need = c->n_fused_pieces * c->K;
+    const int64_t most = ((int64_t)env_int("SDDMM_FUSED_PARTS_MAX", 1024) << 20) / (int64_t)sizeof(float);
+    if (seg < 1024 && need > most && !getenv("SDDMM_FUSED_SEG")) return false;
     if (need <= c->fused_part_floats) return true;
     dfree(c->d_fused_parts);
     c->d_fused_parts = static_cast<float *>(spare_alloc((size_t)need * sizeof(float)));
@@ -1369,7 +1373,7 @@ static bool fused_parts(sddmm_ctx *c) {
 // items of the fused kernel: the rows of more than fused_row_max entries, cut into segments of
 // SDDMM_FUSED_SEG entries (by default 256, and up to 1024 where most rows are about as long)
 static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
-    if (c->fused_items_valid && c->fused_items_panels == (panel_owner != nullptr) && fused_parts(c)) return SDDMM_OK;
+    if (c->fused_items_valid && c->fused_items_panels == (panel_owner != nullptr) && fused_parts(c, c->fused_seg)) return SDDMM_OK;
     int seg = std::max(WAVE, env_int("SDDMM_FUSED_SEG", 1024));
     const int64_t nb = ((int64_t)c->sM + SCAN_TILE - 1) / SCAN_TILE;
     int row_max = FUSED_ROW_MAX;
@@ -1452,7 +1456,7 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
         // the pieces of the rows that are cut, at the most; without room for them fewer and longer ones, and at last every
         // row stays whole
         const auto pieces = [&]() { return c->n_fused_pieces = (int64_t)counted.rows_long + (int64_t)counted.nnz_long / seg; };
-        for (pieces(); !fused_parts(c); pieces()) {
+        for (pieces(); !fused_parts(c, seg); pieces()) {
             seg = seg < 1024 ? 1024 : INT_MAX;
             rc = count();
             if (rc) return rc;

@@ -84,7 +84,8 @@ def test_room_for_fewer_pieces_only(engine_factory, monkeypatch):
     rowptr, col, val = _matrix(rng, N, lens)
     A, _, B, _ = _operands(rng, len(lens), N, 64, capi.F32)
     got = []
-    for name, value in (("SDDMM_SPARE_BYTES", "4000"), ("SDDMM_FUSED_SEG", "1024"), ("SDDMM_FUSED_SEG", "256")):
+    for name, value in (("SDDMM_SPARE_BYTES", "4000"), ("SDDMM_FUSED_SEG", "1024"), ("SDDMM_FUSED_SEG", "256"),
+                        ("SDDMM_FUSED_PARTS_MAX", "0"), ("SDDMM_FUSED_PARTS_MAX", "1")):
         with monkeypatch.context() as m, engine_factory() as e:
             m.setenv(name, value)
             e.set_dense(A, B)
@@ -92,6 +93,31 @@ def test_room_for_fewer_pieces_only(engine_factory, monkeypatch):
             got.append(_check(e, rowptr, col, val, A, B, name))
     np.testing.assert_array_equal(got[0], got[1])
     assert (got[0] != got[2]).any()
+    np.testing.assert_array_equal(got[0], got[3])              # more than 0 MiB is too much, the pieces of 256 fit 1
+    np.testing.assert_array_equal(got[2], got[4])
+
+
+def test_room_after_the_operands_grew(engine_factory, monkeypatch):
+    """400 rows of 2 000 entries, planned at K = 8 (100 KiB of pieces), then K = 256 (3.2 MB): above 1 MiB pieces of 1 024."""
+    monkeypatch.setenv("SDDMM_FUSED_PARTS_MAX", "1")
+    rng = np.random.default_rng(6)
+    N, lens = 3000, np.full(400, 2000)
+    rowptr, col, val = _matrix(rng, N, lens)
+    got = []
+    for grow in (True, False):
+        with engine_factory() as e:
+            if grow:
+                e.set_dense(*[np.ones((n, 8), f32) for n in (400, N)])
+                e.set_csr(400, N, rowptr, col, val)
+                e.run_fused()
+            else:
+                monkeypatch.setenv("SDDMM_FUSED_SEG", "1024")
+            A, _, B, _ = _operands(np.random.default_rng(7), 400, N, 256, capi.F32)
+            e.set_dense(A, B)
+            if not grow:
+                e.set_csr(400, N, rowptr, col, val)
+            got.append(_check(e, rowptr, col, val, A, B, str(grow)))
+    np.testing.assert_array_equal(got[0], got[1])
 
 
 @pytest.mark.parametrize("panel_rows,longer", [(0, 3), (0, 1100), (256, 0)])
