@@ -20,8 +20,8 @@ struct PlanCounters {
     unsigned long long n_utiles, nnz_utiles, utiles_scanned;  // dense-tile path: union strips
     unsigned long long n_panels, nnz_panels, panel_items;     // row-panel path
     unsigned int fused_longest;    // fused call: longest row that its gather kernels take
-    unsigned long long fused_window;   // fused call: most pieces of cut rows among the rows of a wavefront
-    unsigned long long rows_alike; // fused call: work-item rows that look like the next row (its length, its first column)
+    unsigned int fused_window;     // fused call: most pieces of cut rows among the rows of a wavefront
+    unsigned long long rows_alike; // fused call, every fourth row: work-item rows like the next row (its length, its first column)
 };
 
 // The same counters on the device.  Sums that thousands of workgroups contribute to
@@ -32,15 +32,14 @@ constexpr int SPREAD = 64;
 enum CounterKind {
     K_ROWS_NONEMPTY = 0,
     K_ROWS_SHORT, K_ROWS_MEDIUM, K_ROWS_LONG, K_NNZ_SHORT, K_NNZ_MEDIUM, K_NNZ_LONG,   // row classifier
-    K_ROWS_ALIKE,                                                                      // and for the fused call
+    K_ROWS_ALIKE, K_LONGEST, K_WINDOW,                                                 // and for the fused call (two maxima)
     K_TILES, K_NNZ_TILES, K_UTILES, K_NNZ_UTILES, K_PANELS, K_NNZ_PANELS,              // ownership classifiers
     K_COO_JUMPS,                                                                       // validation of COO entries
     K_KINDS
 };
 struct DevCounters {
     unsigned int bad_pattern, coo_unsorted, pad0, pad1;
-    unsigned long long n_items, fused_longest, fused_window;         // (one fill clears them; PlanCounters)
-    unsigned long long tiles_scanned, panel_items;                   // scan totals, one writer each, as is n_items
+    unsigned long long n_items, tiles_scanned, panel_items;          // scan totals, one writer each
     unsigned long long n_candidates;                                 // rows offered to the gathered strips
     unsigned long long utiles_scanned, short_scanned;                // scan totals: union strips, entries of the short rows
     unsigned long long long_scanned;                                 // scan total: rows of more than one item
@@ -70,8 +69,10 @@ inline PlanCounters summarize(const DevCounters &d) {
     p.n_tiles = sum[K_TILES]; p.nnz_tiles = sum[K_NNZ_TILES];
     p.n_utiles = sum[K_UTILES]; p.nnz_utiles = sum[K_NNZ_UTILES]; p.utiles_scanned = d.utiles_scanned;
     p.n_panels = sum[K_PANELS]; p.nnz_panels = sum[K_NNZ_PANELS];
-    p.fused_longest = (unsigned int)d.fused_longest;
-    p.fused_window = d.fused_window;
+    for (int s = 0; s < SPREAD; ++s) {
+        p.fused_longest = std::max(p.fused_longest, (unsigned int)d.k[K_LONGEST][s]);
+        p.fused_window = std::max(p.fused_window, (unsigned int)d.k[K_WINDOW][s]);
+    }
     p.n_items = d.n_items; p.tiles_scanned = d.tiles_scanned; p.panel_items = d.panel_items;
     return p;
 }
@@ -309,7 +310,8 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int3
                                                                const int32_t *__restrict__ col, int window) {
     const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
     unsigned int items = 0, longest = 0, pieces = 0;
-    unsigned long long r_alike = 0, r_short = 0, r_med = 0, r_long = 0, n_short = 0, n_med = 0, n_long = 0;
+    unsigned int r_alike = 0;
+    unsigned long long r_short = 0, r_med = 0, r_long = 0, n_short = 0, n_med = 0, n_long = 0;
     for (int q = 0; q < SCAN_ITEMS; ++q) {
         unsigned int len;
         const unsigned int cnt = row_item_count(rowptr, owner, base + q, M, ts, seg, &len, only);
@@ -317,9 +319,9 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int3
         longest = len > longest ? len : longest;
         pieces += cnt > 1 ? cnt : 0;
         if (len == 0) continue;
-        if (only && cnt > 0 && base + q + 1 < M) {
-            const int32_t a = rowptr[base + q], b = rowptr[base + q + 1];
-            if ((unsigned int)(rowptr[base + q + 2] - b) == len && col[a] == col[b]) ++r_alike;
+        if (q == 0 && col && cnt > 0 && base + 1 < M) {         // (a sample: the chain of loads of every row takes 5 us)
+            const int32_t a = rowptr[base], b = rowptr[base + 1];
+            if ((unsigned int)(rowptr[base + 2] - b) == len && col[a] == col[b]) r_alike = 1;
         }
         if (cnt == 0) { ++r_short; n_short += len; }
         else if (cnt == 1) { ++r_med; n_med += len; }
@@ -344,14 +346,26 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int3
     }
     __syncthreads();
     if (threadIdx.x < 6) spread_add(pc, K_ROWS_SHORT + (int)threadIdx.x, sh[threadIdx.x]);
-    if (only) {                                       // the fused call (most workgroups find as much there already)
-        longest = wave_max_u32(longest);
+    if (only) {                                       // the fused call
+        __shared__ unsigned int most[3];
+        if (threadIdx.x < 3) most[threadIdx.x] = 0;
+        __syncthreads();
         for (int o = 1; o < window / SCAN_ITEMS; o <<= 1) pieces += __shfl_xor(pieces, o, WAVE);
         pieces = wave_max_u32(pieces);
-        if (lane_id() == 0 && pieces > pc->fused_window) atomicMax(&pc->fused_window, (unsigned long long)pieces);
-        r_alike = wave_sum_u64(r_alike);
-        if (lane_id() == 0 && r_alike) spread_add(pc, K_ROWS_ALIKE, r_alike);
-        if (lane_id() == 0 && longest > pc->fused_longest) atomicMax(&pc->fused_longest, (unsigned long long)longest);
+        longest = wave_max_u32(longest);
+        const unsigned int alike = (unsigned int)__popcll(__ballot(r_alike != 0));
+        if (lane_id() == 0) {
+            atomicMax(&most[0], longest);
+            atomicMax(&most[1], pieces);
+            atomicAdd(&most[2], alike);
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const int slot = blockIdx.x & (SPREAD - 1);
+            atomicMax(&pc->k[K_LONGEST][slot], (unsigned long long)most[0]);
+            if (most[1]) atomicMax(&pc->k[K_WINDOW][slot], (unsigned long long)most[1]);
+            spread_add(pc, K_ROWS_ALIKE, most[2]);
+        }
     }
     // entries of this block's short rows, for the entry list (k_short_list_write)
     if (short_sums && threadIdx.x == 0) short_sums[blockIdx.x] = (unsigned int)sh[3];

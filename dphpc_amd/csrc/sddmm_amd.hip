@@ -1385,14 +1385,14 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
         DevCounters tmp;
         PlanCounters counted;
         int window = WAVE / shape_of(c).LPN;               // rows of a wavefront of the kernel of the short rows
+        const int32_t *look_at = c->d_col;                 // (which rows are alike: the first count tells)
         auto count = [&]() -> int {
             HIP_TRY(c, hipMemsetAsync(&c->d_pc->k[K_ROWS_SHORT][0], 0,
-                                      sizeof(unsigned long long) * SPREAD * (K_ROWS_ALIKE - K_ROWS_SHORT + 1), c->stream));
-            HIP_TRY(c, hipMemsetAsync(&c->d_pc->n_items, 0, 3 * sizeof(unsigned long long), c->stream));
+                                      sizeof(unsigned long long) * SPREAD * (K_WINDOW - K_ROWS_SHORT + 1), c->stream));
+            HIP_TRY(c, hipMemsetAsync(&c->d_pc->n_items, 0, sizeof(unsigned long long), c->stream));
             SDDMM_LAUNCH(c, k_classify_count, nb, SCAN_BLOCK, c->d_rowptr,
                                panel_owner, c->sM, row_max + 1, seg, c->d_block_sums, c->d_pc, 2,
-                               (unsigned int *)nullptr, (unsigned int *)nullptr, (const int32_t *)c->d_col,
-                               window);
+                               (unsigned int *)nullptr, (unsigned int *)nullptr, look_at, window);
             SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, c->d_block_sums, (int)nb,
                                &c->d_pc->n_items);
             LAUNCH_CHECK(c);
@@ -1404,8 +1404,9 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
         int rc = count();
         if (rc) return rc;
         const PlanCounters first = counted;
+        look_at = nullptr;
         const int64_t item_entries = (int64_t)(first.nnz_medium + first.nnz_long);
-        c->fused_rows_alike = 2 * first.rows_alike >= first.rows_medium + first.rows_long;
+        c->fused_rows_alike = 2 * SCAN_ITEMS * first.rows_alike >= first.rows_medium + first.rows_long;
         c->fused_short_avg = first.rows_short ? (double)first.nnz_short / (double)first.rows_short : 0.0;
         if (fused_balanced(c)) window = WAVE;              // (those rows are so short that they are counted again, below)
         // A wavefront walks its item chunk by chunk and the launch waits for the longest one: the long rows are cut into
