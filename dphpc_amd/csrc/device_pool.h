@@ -6,11 +6,13 @@
 // of 783 k entries paid 50 .. 90 us for creating its context and 125 .. 170 for destroying it (2 and 2 now): 1095 -> 840 us.
 //
 //   bound   POOL_BYTES of free blocks per device, the oldest go first; no block beyond POOL_BLOCK_MAX is kept;
-//           POOL_CONTEXTS sets of parts.  sddmm_trim gives all of it back, and so does an allocation that fails.
+//           POOL_CONTEXTS sets of parts.  sddmm_trim gives all of it back; an allocation that fails gives the free blocks of
+//           its device back and is tried once more.
 //   safety  A block that is given back may be handed to any context of the device, so it is given back when the device is
 //           idle (release_*: one hipDeviceSynchronize for all blocks of a pattern, which is what every hipFree did).
 //           One mutex guards the tables.  They have fixed sizes: nothing here allocates host memory or throws; a block
 //           that finds no place in them is a plain hipMalloc / hipFree.
+//   reset   hipDeviceReset takes back what is kept; the next context finds that out and starts afresh.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -21,7 +23,8 @@
 namespace sddmm {
 
 constexpr size_t POOL_BYTES = (size_t)128 << 20, POOL_BLOCK_MAX = (size_t)32 << 20;
-constexpr int POOL_BLOCKS = 512, POOL_CONTEXTS = 8;
+constexpr int POOL_BLOCKS = 512, POOL_CONTEXTS = 8, POOL_DEVICES = 16;
+constexpr size_t POOL_WITNESS = 19 * 4096 - 16;              // bytes that hardly any other allocation asks for
 
 // what is asked for, rounded up to eighths of its power of two: patterns of about one size share their blocks
 inline size_t pool_round(size_t bytes) {
@@ -32,9 +35,19 @@ inline size_t pool_round(size_t bytes) {
 
 struct ContextParts {
     int device = -1;
+    unsigned int life = 0;                                   // of the device (PoolDevice) that they were made in
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     void *counters = nullptr, *host_counters = nullptr;      // device block, pinned landing place
+};
+
+// A device that the pool keeps something of.  hipDeviceReset takes all of it back without a word: the witness, a block that
+// only the pool knows, is then gone as well (pool_look_after).
+struct PoolDevice {
+    int device = -1;
+    unsigned int life = 0;                                   // resets seen so far
+    void *witness = nullptr;
+    size_t bytes = 0;                                        // its size, as the runtime tells it
 };
 
 struct DevicePool {
@@ -50,6 +63,8 @@ struct DevicePool {
     uint64_t clock = 0;
     ContextParts parts[POOL_CONTEXTS];
     int n_parts = 0;
+    PoolDevice devices[POOL_DEVICES];
+    int n_devices = 0;
 };
 inline DevicePool device_pool;
 
@@ -63,6 +78,42 @@ inline void pool_trim_locked(DevicePool &d, int device) {
             (void)hipFree(d.block[i].p);
             pool_drop(d, i);
         }
+}
+
+inline PoolDevice *pool_device(DevicePool &d, int device) {
+    for (int i = 0; i < d.n_devices; ++i)
+        if (d.devices[i].device == device) return &d.devices[i];
+    return nullptr;
+}
+
+// (the lock is held) forgets what a reset of the device took back
+inline void pool_look_after(DevicePool &d, PoolDevice &v) {
+    size_t bytes = 0;
+    if (!v.witness || (hipMemPtrGetInfo(v.witness, &bytes) == hipSuccess && bytes == v.bytes)) return;
+    (void)hipGetLastError();
+    for (int i = d.n - 1; i >= 0; --i)
+        if (d.block[i].device == v.device) pool_drop(d, i);
+    for (int i = d.n_parts - 1; i >= 0; --i)
+        if (d.parts[i].device == v.device) d.parts[i] = d.parts[--d.n_parts];
+    v.witness = nullptr;
+    ++v.life;
+}
+
+// (the lock is held; device is the current one) Before a new context.  nullptr, or no witness: nothing of this device is kept.
+inline PoolDevice *pool_open(DevicePool &d, int device) {
+    PoolDevice *v = pool_device(d, device);
+    if (!v && d.n_devices < POOL_DEVICES) {
+        v = &d.devices[d.n_devices++];
+        v->device = device;
+    }
+    if (!v) return nullptr;
+    pool_look_after(d, *v);
+    if (!v->witness && (hipMalloc(&v->witness, POOL_WITNESS) != hipSuccess || hipMemPtrGetInfo(v->witness, &v->bytes) != hipSuccess)) {
+        (void)hipGetLastError();
+        if (v->witness) (void)hipFree(v->witness);
+        v->witness = nullptr;
+    }
+    return v;
 }
 
 // memory of the current device
@@ -92,7 +143,8 @@ inline hipError_t pool_alloc(void **out, size_t bytes) {
         e = hipMalloc(out, bytes);
     }
     if (e != hipSuccess) { *out = nullptr; return e; }
-    if (bytes <= POOL_BLOCK_MAX && d.n < POOL_BLOCKS) d.block[d.n++] = DevicePool::Block{*out, bytes, 0, device};
+    const PoolDevice *v = pool_device(d, device);
+    if (bytes <= POOL_BLOCK_MAX && d.n < POOL_BLOCKS && v && v->witness) d.block[d.n++] = DevicePool::Block{*out, bytes, 0, device};
     return hipSuccess;
 }
 
@@ -136,10 +188,14 @@ inline void destroy_parts(ContextParts &c) {
     c = ContextParts{};
 }
 
+// device is the current one
 inline hipError_t take_parts(ContextParts *out, int device, size_t counter_bytes) {
+    unsigned int life = 0;
     {
         DevicePool &d = device_pool;
         const std::lock_guard<std::mutex> hold(d.lock);
+        const PoolDevice *v = pool_open(d, device);
+        if (v) life = v->life;
         for (int i = d.n_parts - 1; i >= 0; --i)
             if (d.parts[i].device == device) {
                 *out = d.parts[i];
@@ -150,6 +206,7 @@ inline hipError_t take_parts(ContextParts *out, int device, size_t counter_bytes
     ContextParts c;
     auto make = [&]() {
         c.device = device;
+        c.life = life;
         hipError_t e = hipStreamCreate(&c.stream);
         if (e == hipSuccess) e = hipEventCreate(&c.ev0);
         if (e == hipSuccess) e = hipEventCreate(&c.ev1);
@@ -176,7 +233,9 @@ inline void give_parts(ContextParts c, bool idle) {
     DevicePool &d = device_pool;
     if (idle) {
         const std::lock_guard<std::mutex> hold(d.lock);
-        if (d.n_parts < POOL_CONTEXTS) {
+        const PoolDevice *v = pool_device(d, c.device);
+        if (v && v->life != c.life) return;                  // a reset took them back
+        if (v && v->witness && d.n_parts < POOL_CONTEXTS) {
             d.parts[d.n_parts++] = c;
             return;
         }
@@ -187,8 +246,17 @@ inline void give_parts(ContextParts c, bool idle) {
 inline void pool_trim() {
     DevicePool &d = device_pool;
     const std::lock_guard<std::mutex> hold(d.lock);
+    for (int i = 0; i < d.n_devices; ++i) pool_look_after(d, d.devices[i]);
     pool_trim_locked(d, -1);
     while (d.n_parts > 0) destroy_parts(d.parts[--d.n_parts]);
+    for (int i = 0; i < d.n_devices; ++i) {
+        PoolDevice &v = d.devices[i];
+        bool used = false;
+        for (int k = 0; k < d.n; ++k) used = used || d.block[k].device == v.device;
+        if (used || !v.witness) continue;                    // (stays as long as a context has blocks of the table)
+        (void)hipFree(v.witness);
+        v.witness = nullptr;
+    }
 }
 
 }  // namespace sddmm

@@ -116,7 +116,9 @@ int sddmm_create(sddmm_ctx **out, int device);
 void sddmm_destroy(sddmm_ctx *ctx);
 /* Device memory of patterns that were replaced and of contexts that were destroyed is kept for the next ones: at most
  * 128 MiB per device, none of it in blocks of more than 32 MiB, and the streams and events of up to 8 contexts.  Gives
- * what is not in use back to the driver (as an allocation that fails does first).  Any thread, any time. */
+ * what is not in use back to the driver (an allocation that fails does so first with the free memory of its device).  Any
+ * thread, any time.  After a hipDeviceReset the next sddmm_create or sddmm_trim finds that what was kept is gone; contexts
+ * that were open over the reset can only be destroyed. */
 int sddmm_trim(void);
 const char *sddmm_strerror(int code);
 /* Text of the last failure on this context ("" if none); owned by the context. */
