@@ -8,8 +8,8 @@
 //   bound   POOL_BYTES of free blocks per device, the oldest go first; no block beyond POOL_BLOCK_MAX is kept;
 //           POOL_CONTEXTS sets of parts.  sddmm_trim gives all of it back; an allocation that fails gives the free blocks of
 //           its device back and is tried once more.
-//   safety  A block that is given back may be handed to any context of the device, so it is given back when the device is
-//           idle (release_*: one hipDeviceSynchronize for all blocks of a pattern, which is what every hipFree did).
+//   safety  A block that is given back may be handed to any context of the device, so it is kept only when the device is
+//           idle (release_*: one wait for all blocks of a pattern, pool_wait); otherwise it goes to hipFree, which waits.
 //           One mutex guards the tables.  They have fixed sizes: nothing here allocates host memory or throws; a block
 //           that finds no place in them is a plain hipMalloc / hipFree.
 //   reset   hipDeviceReset takes back what is kept; the next context finds that out and starts afresh.
@@ -19,6 +19,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <mutex>
+#include <utility>
 
 namespace sddmm {
 
@@ -48,6 +49,7 @@ struct PoolDevice {
     unsigned int life = 0;                                   // resets seen so far
     void *witness = nullptr;
     size_t bytes = 0;                                        // its size, as the runtime tells it
+    void *to_free = nullptr;                                 // by the next pool_wait
 };
 
 struct DevicePool {
@@ -95,7 +97,7 @@ inline void pool_look_after(DevicePool &d, PoolDevice &v) {
         if (d.block[i].device == v.device) pool_drop(d, i);
     for (int i = d.n_parts - 1; i >= 0; --i)
         if (d.parts[i].device == v.device) d.parts[i] = d.parts[--d.n_parts];
-    v.witness = nullptr;
+    v.witness = v.to_free = nullptr;
     ++v.life;
 }
 
@@ -148,11 +150,34 @@ inline hipError_t pool_alloc(void **out, size_t bytes) {
     return hipSuccess;
 }
 
+// Waits for all work of the current device, on whatever stream: false if it could not.  As hipFree does it, by freeing
+// something: hipDeviceSynchronize breaks every capture in progress, those of other threads and of relaxed mode too.  A new
+// pattern 218 us with it, 213 with hipDeviceSynchronize; 30 .. 80 us more once, after a program's other work.
+inline bool pool_wait() {
+    DevicePool &d = device_pool;
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess) return false;
+    void *p = nullptr;
+    {
+        const std::lock_guard<std::mutex> hold(d.lock);
+        PoolDevice *v = pool_device(d, device);
+        if (v) std::swap(p, v->to_free);
+    }
+    const bool waited = (p || hipMalloc(&p, 16) == hipSuccess) && hipFree(p) == hipSuccess;
+    if (waited && hipMalloc(&p, 16) == hipSuccess) {         // the next one, where the last one was: a new place costs 40 us
+        const std::lock_guard<std::mutex> hold(d.lock);
+        PoolDevice *v = pool_device(d, device);
+        if (v && v->witness && !v->to_free) std::swap(p, v->to_free);
+        else (void)hipFree(p);
+    }
+    (void)hipGetLastError();
+    return waited;
+}
+
 // idle: the caller knows that no work which uses the block is in flight
 inline void pool_free(void *p, bool idle) {
     if (!p) return;
     DevicePool &d = device_pool;
-    if (!idle) idle = hipDeviceSynchronize() == hipSuccess;
     const std::lock_guard<std::mutex> hold(d.lock);
     int at = -1;
     for (int i = 0; i < d.n && at < 0; ++i)
@@ -255,7 +280,8 @@ inline void pool_trim() {
         for (int k = 0; k < d.n; ++k) used = used || d.block[k].device == v.device;
         if (used || !v.witness) continue;                    // (stays as long as a context has blocks of the table)
         (void)hipFree(v.witness);
-        v.witness = nullptr;
+        if (v.to_free) (void)hipFree(v.to_free);
+        v.witness = v.to_free = nullptr;
     }
 }
 

@@ -8,16 +8,12 @@
 
 namespace {
 
-// Gives a block back; it waits for the device first, as hipFree does, unless the caller has.
+// Gives a block back: to the pool if the caller has waited for the device, otherwise to hipFree.
 template <class T>
 void dfree(T *&p, bool idle = false) {
     pool_free((void *)p, idle);
     p = nullptr;
 }
-
-// Nothing that uses a block may be in flight when the block is handed on: waits for the whole device, since a caller may
-// read the results on a stream of its own.
-bool wait_for_device() { return hipDeviceSynchronize() == hipSuccess; }
 
 // Views into the plan arena: nothing here is freed on its own.
 void release_arena(sddmm_ctx *c, bool idle = false) {
@@ -84,8 +80,10 @@ int ensure_arena(sddmm_ctx *c) {
                         (long long)(need), (long long)(cap));                                       \
     } while (0)
 
-void release_dense(sddmm_ctx *c) {
-    const bool idle = c->own_dense && wait_for_device();
+// Nothing that uses a block may be in flight when the block is handed on: release_* wait for the whole device (unless the
+// caller has), since a caller may read the results on a stream of its own.
+void release_dense(sddmm_ctx *c, bool idle = false) {
+    idle = idle || (c->own_dense && pool_wait());
     if (c->own_dense) { dfree(c->dA, idle); dfree(c->dB, idle); }
     c->dA = c->dB = nullptr;
     c->have_fused = false;
@@ -94,9 +92,9 @@ void release_dense(sddmm_ctx *c) {
     c->planned = false;
 }
 
-void release_sparse(sddmm_ctx *c) {
+void release_sparse(sddmm_ctx *c, bool idle = false) {
     // (every pattern has its array of results, a context without one nothing to give back)
-    const bool idle = c->dP && wait_for_device();
+    idle = idle || (c->dP && pool_wait());
     if (c->own_sparse) { dfree(c->d_col, idle); dfree(c->d_sval, idle); }
     if (c->own_rowptr) dfree(c->d_rowptr, idle);
     if (c->own_rowidx) dfree(c->d_rowidx, idle);
@@ -1088,9 +1086,9 @@ void sddmm_destroy(sddmm_ctx *c) {
     if (!c) return;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
-    const bool idle = wait_for_device();
-    release_dense(c);
-    release_sparse(c);
+    const bool idle = pool_wait();
+    release_dense(c, idle);
+    release_sparse(c, idle);
     dfree(c->dO, idle);
     dfree(c->d_part, idle);
     dfree(c->d_blocks, idle);

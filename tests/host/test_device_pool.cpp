@@ -26,6 +26,7 @@ std::map<void *, size_t> sizes;
 int calls = 0;                         // of those that create something
 int fail_from = -1, fail_count = 0;    // calls [fail_from, fail_from + fail_count) fail
 hipError_t fail_with = hipErrorOutOfMemory;
+int frees = 0;                         // calls of hipFree: each waits for the device
 int bad_destroys = 0;                  // of something that is not there
 
 hipError_t create(void **out, size_t bytes) {
@@ -59,9 +60,8 @@ void fail(int from, int count, hipError_t with = hipErrorOutOfMemory) {
 extern "C" {
 hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
 hipError_t hipGetLastError(void) { return hipSuccess; }
-hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
 hipError_t hipMalloc(void **p, size_t bytes) { return rt::create(p, bytes); }
-hipError_t hipFree(void *p) { return rt::destroy(p); }
+hipError_t hipFree(void *p) { ++rt::frees; return rt::destroy(p); }
 hipError_t hipMemPtrGetInfo(void *p, size_t *bytes) { return (*bytes = rt::size_of(p)) ? hipSuccess : hipErrorInvalidValue; }
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned int) { return rt::create(p, bytes); }
 hipError_t hipHostFree(void *p) { return rt::destroy(p); }
@@ -190,8 +190,36 @@ static void kept_and_bounded() {
     CHECK(rt::bad_destroys == 0, "%d things destroyed that were not there", rt::bad_destroys);
 }
 
+// The wait is a hipFree of something that is there, whatever fails; without one it says that it could not wait.
+static void wait_for_the_device() {
+    ContextParts c;
+    rt::fail(-1, 0);
+    CHECK(take_parts(&c, 0, 64) == hipSuccess, "parts");
+    for (int fails : {0, 1000, 1, 0}) {
+        rt::fail(fails ? 0 : -1, fails);
+        const int before = rt::frees;
+        const bool waited = pool_wait();
+        CHECK(waited == (rt::frees > before), "waited %d, %d frees", waited, rt::frees - before);
+        CHECK(waited || fails, "could not wait");
+    }
+    rt::fail(-1, 0);
+    give_parts(c, true);
+    pool_trim();
+    CHECK(pool_wait(), "with nothing kept");
+    CHECK(rt::live.empty(), "%zu left behind", rt::live.size());
+    CHECK(rt::bad_destroys == 0, "%d things destroyed that were not there", rt::bad_destroys);
+    // after a reset that no context has noticed yet
+    CHECK(take_parts(&c, 0, 64) == hipSuccess && pool_wait(), "parts");
+    rt::reset();
+    CHECK(!pool_wait() || rt::live.empty(), "what a reset took back was freed for a wait");
+    rt::bad_destroys = 0;
+    pool_trim();
+    CHECK(rt::live.empty() && rt::bad_destroys == 0, "after a reset");
+}
+
 int main() {
     parts_that_fail();
+    wait_for_the_device();
     reset_of_the_device();
     kept_and_bounded();
     std::printf("%d failed\n", failures);
