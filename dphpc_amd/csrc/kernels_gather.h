@@ -211,9 +211,9 @@ __device__ __forceinline__ void flat_body(const void *__restrict__ A, const void
                                           const float *__restrict__ sval, float *__restrict__ P, int64_t base,
                                           int64_t stop, int lane) {
     using U = typename L::U;
-    // Index loads are unconditional (clamped to the last entry of the range): lanes
-    // past the end then hold a valid row/column whose result is never stored, and
-    // the loads need no branch, which keeps the wait counts of the gathers exact.
+    // Index loads are clamped to the last entry of the range: lanes past the end then
+    // hold a valid row/column whose result is never stored, and the loads need no
+    // branch per lane.
     const int64_t last = stop - 1;
     const int64_t n0 = base + lane < last ? base + lane : last;
     int c = ld_stream(col + n0), r = ld_stream(rowidx + n0);
@@ -227,7 +227,12 @@ __device__ __forceinline__ void flat_body(const void *__restrict__ A, const void
         int cn = 0, rn = 0;
         float sn = 1.f;
         auto prefetch = [&]() {
-            if (left <= WAVE) return;                       // (wave-uniform)
+            // Nothing to load ahead of the last chunk.  Eight lanes of one bf16 unit do without the branch: with it the kernel
+            // holds two batches of rows (97 .. 122 registers instead of 76 .. 101; 100 000 rows of 20 entries K = 64 21.0 us with
+            // it, 19.5 without, graph of 1 M rows 158 / 150).  Elsewhere it returns a little or nothing (K = 8 18.4 / 19.1,
+            // K = 24 bf16 25.9 / 26.8, K = 32 18.9 / 18.5, banded rows K = 21 110 / 118).
+            constexpr bool BRANCH = !(L::UPL == 1 && L::LPN == 8 && U::DT == DT_BF16);
+            if (BRANCH && left <= WAVE) return;             // (wave-uniform)
             const int64_t pn = n + WAVE < last ? n + WAVE : last;
             cn = ld_stream(col + pn); rn = ld_stream(rowidx + pn);
             if constexpr (SCALED) sn = ld_stream(sval + pn);
@@ -290,9 +295,9 @@ __device__ __forceinline__ void row_segment_body(const void *__restrict__ A, con
         using O = typename C::O;
         const O rb = (O)U::row_bytes(KU);
         const typename C::Areg a = C::load_a(A, (O)row * rb, lane & (L::LPN - 1), KU);
-        // Index loads are unconditional (clamped to the last entry of the range): lanes
-        // past the end then hold a valid column whose result is never stored, and the
-        // loads need no branch, which keeps the wait counts of the gathers exact.
+        // Index loads are clamped to the last entry of the range: lanes past the end then
+        // hold a valid column whose result is never stored, and the loads need no branch
+        // per lane.
         const int last = end - 1;
         const int n0 = start + lane < last ? start + lane : last;
         int c = ld_stream(col + n0);
@@ -372,7 +377,11 @@ __device__ __forceinline__ void short_rows_body(const void *__restrict__ A, cons
         int nn = n, rown = row, cn = 0;
         float sn = 0.f;
         auto prefetch = [&]() {
-            if (left <= WAVE) return;                       // (wave-uniform)
+            // (with eight lanes of one unit the branch costs k_auto a third of its wavefronts, 95 registers instead of 64:
+            // 20 000 rows of 40 entries K = 32 10.8 us with it, 9.8 without, banded rows K = 21 83 / 73, dense tiles K = 21
+            // 31.6 / 28.2)
+            constexpr bool BRANCH = !(L::UPL == 1 && L::LPN == 8);
+            if (BRANCH && left <= WAVE) return;             // (wave-uniform)
             locate(base + WAVE + lane, nn, rown);
             cn = ld_stream(col + nn); sn = ld_stream(sval + nn);
         };
