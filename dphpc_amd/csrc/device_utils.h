@@ -43,8 +43,8 @@ __device__ __forceinline__ float group_sum(float v) {
 }
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (WAVE - 1); }
-// index of the wavefront inside its workgroup, as a scalar
 __device__ __forceinline__ int waves_in_block() { return (int)(blockDim.x >> 6); }
+// index of the wavefront inside its workgroup, as a scalar
 __device__ __forceinline__ int wave_in_block() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
 // LDS that only one wavefront touches: its LDS operations execute in program order, so a

@@ -27,10 +27,9 @@ namespace sddmm {
 constexpr int BLOCK = 256;                 // 4 wavefronts
 constexpr int WAVES_PER_BLOCK = BLOCK / WAVE;
 // Work items of different lengths over columns that neighbours do not share take workgroups of one wavefront: a workgroup
-// keeps its place on the CU until its last wavefront ends, and with four items each the places are half empty (4.9 of 6
-// wavefronts per SIMD on average in k_flat_blocks).  Against workgroups of four: graph of 2.6 M rows, K = 32, 554 -> 527 us;
-// 200 000 rows K = 32 30.3 -> 28.0, K = 64 56.7 -> 54.9; rows of more than 512 bytes keep four (K = 256: 251 -> 255 with
-// one).  Kernels whose wavefronts all take the same work keep four (k_flat K = 64 15.1 -> 16.2, k_slice_dots 204 -> 205
+// keeps its place on the CU until its last wavefront ends.  Against workgroups of four: graph of 2.6 M rows, K = 32, 554 ->
+// 527 us; 200 000 rows K = 32 30.3 -> 28.0, K = 64 56.7 -> 54.9; rows of more than 512 bytes keep four (K = 256: 251 -> 255
+// with one).  Kernels whose wavefronts all take the same work keep four (k_flat K = 64 15.1 -> 16.2, k_slice_dots 204 -> 205
 // with one), and so does k_auto: with one, rows of 20 000 random columns gain (K = 64 23.7 -> 21.0), but rows whose
 // neighbours hold the same columns lose what they find in the CU's L1 (banded blocks K = 42 59 -> 92, dense tiles K = 120
 // bf16 30 -> 35) and items of a few bytes wait for their dispatch (45 entries per row, K = 8 bf16, 20 -> 36).
@@ -137,7 +136,7 @@ struct Chunk {
     }
 
     // boff / aoff: byte offset of this lane's entry's B row / A row (a valid row in
-    // every lane, row 0 past the end of the chunk); count = entries in the chunk.
+    // every lane, the last entry's past the end of the chunk); count = entries in the chunk.
     // `prefetch` is called once, right after the first gathers have been issued:
     // the place to start the index loads of the next chunk, so that they travel
     // while this chunk computes (loads return in issue order, so anything issued
@@ -440,8 +439,9 @@ __device__ __forceinline__ void entry_list_body(const void *__restrict__ A, cons
 // segments of one column block each are taken block by block, an XCD two of the COL_BLOCKS blocks, so
 // that its L2 sees an eighth of B from them (two thirds of the entries: 518 us).  A segment is a work
 // item of one row, its A row stays in registers.  The entries between the long rows are taken 64 at a
-// time in storage order (64: 524 us, 256: 538, 512: 541), after the segments on every XCD (before
-// them: the same; dealt out evenly: 542 us).
+// time in storage order (64 / 128 / 256, with workgroups of one wavefront: 2.6 M rows 427 / 450 / 460 us, 1 M rows 150 /
+// 159 / 160, 200 000 rows K = 100 in the same order), after the segments on every XCD (before
+// them: the same; dealt out evenly: 542 against 524 us with workgroups of four).
 // totals[0], totals[1]: work items of either kind (the grid is sized for an upper bound)
 //
 template <class L, bool SCALED>
