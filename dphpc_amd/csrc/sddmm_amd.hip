@@ -1461,9 +1461,10 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
             if (rc) return rc;
         }
         c->n_fused_items = (int64_t)tmp.n_items;
+        // (a launch takes fewer than 2^32 threads, a workgroup per cut row)
         const int apart = env_int("SDDMM_FUSED_ADD_APART", -1);
-        if (apart >= 0 ? apart != 0 : counted.fused_window > FUSED_APART_PIECES) c->n_fused_cut = (int64_t)counted.rows_long;
-        // (a launch takes fewer than 2^32 threads)
+        if ((apart >= 0 ? apart != 0 : counted.fused_window > FUSED_APART_PIECES) && counted.rows_long < (1u << 24))
+            c->n_fused_cut = (int64_t)counted.rows_long;
         c->fused_add_block = counted.fused_longest / (unsigned int)seg > 512 && c->n_fused_cut < 65536 ? FUSED_APART_BLOCK : 256;
         const int64_t room = c->n_fused_items + (c->n_fused_cut + 3) / 4;           // a list of rows behind the items
         if (room > c->fused_items_cap) {
