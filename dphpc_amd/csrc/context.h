@@ -124,8 +124,7 @@ struct sddmm_ctx {
     char *d_blocks = nullptr;        // one allocation: lists and scans of the plan, item counts, items
     size_t blocks_bytes = 0;
     RowItem *d_block_segments = nullptr, *d_block_gaps = nullptr;
-    unsigned long long *d_block_totals = nullptr;
-    int64_t block_segments_max = 0, block_gaps_max = 0;
+    int64_t block_segments_max = 0, block_gaps_max = 0;      // as the launch sizes its grid: the true numbers where the host has them
     bool use_blocks = false;         // set by a plan of SDDMM_AUTO
     unsigned int *d_long_sums = nullptr;    // arena view: long rows per block of the row scan
     // entries that came in no order, sorted by row and column block: row and column of each, the place every entry
@@ -349,6 +348,7 @@ hipError_t load_fused();
 void launch_flat(sddmm_ctx *c);                                                  // launch_flat.hip
 int launch_flat_blocks(sddmm_ctx *c);                                            // number of launches
 void launch_unsort(sddmm_ctx *c);
+int column_blocks_most(const sddmm_ctx *c);
 void block_items_max(const sddmm_ctx *c, bool cut_long_rows, int64_t *segments, int64_t *gaps);
 bool blocks_pay(const sddmm_ctx *c);
 bool order_pays(const sddmm_ctx *c);

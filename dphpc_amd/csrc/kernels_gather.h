@@ -436,8 +436,8 @@ __device__ __forceinline__ void entry_list_body(const void *__restrict__ A, cons
 // FLAT with the long rows cut into column blocks.  The lines of B that a flat launch gathers come from
 // the last-level cache (7.3 TB/s, the bound on a graph: 633 us for 36 M entries over 333 MB of B), since
 // every XCD touches all of B.  Much of a power-law graph lies in rows of hundreds of entries: their
-// segments of one column block each are taken block by block, an XCD two of the COL_BLOCKS blocks, so
-// that its L2 sees an eighth of B from them (two thirds of the entries: 518 us).  A segment is a work
+// segments of one column block each (8 to 64 blocks, row_blocks) are taken block by block, an XCD an eighth of
+// them, so that its L2 sees an eighth of B from them, a few MB at a time (two thirds of the entries: 515 us).  A segment is a work
 // item of one row, its A row stays in registers.  The entries between the long rows are taken 64 at a
 // time in storage order (64 / 128 / 256, with workgroups of one wavefront: 2.6 M rows 427 / 450 / 460 us, 1 M rows 150 /
 // 159 / 160, 200 000 rows K = 100 in the same order), after the segments on every XCD (before

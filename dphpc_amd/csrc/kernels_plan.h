@@ -44,6 +44,7 @@ struct DevCounters {
     unsigned long long utiles_scanned, short_scanned;                // scan totals: union strips, entries of the short rows
     unsigned long long long_scanned;                                 // scan total: rows of more than one item
     unsigned long long fused_pieces, fused_cut;                      // places given to the pieces of cut rows, to those rows
+    unsigned long long block_items[2];                               // work items of k_flat_blocks: segments, gaps
     unsigned int max_len[SPREAD];
     unsigned long long k[K_KINDS][SPREAD];
 };
@@ -632,43 +633,59 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_long_rows(const int32_t *
         if ((is_long >> q) & 1u) long_rows[at++] = (int32_t)(base + q);
 }
 
-// 16 lanes per long row: lane b finds where the row's columns of block b start (columns ascend inside a
+// Column blocks of a long row: a power of two, 8 to `most`, such that its segments hold COL_BLOCK_ENTRIES entries or more
+// on average (from 16 blocks on).  More blocks find more lines of B in an XCD's L2, short segments leave lanes idle and are
+// work items more.  16 blocks for every row / 8 .. 64 with 32, 64, 96 entries, all with the exact grid (launch_flat_blocks):
+// graph of 2.6 M rows K = 32 521 us / 524, 515, 513; 1.5 M rows K = 64 bf16 229 / 230, 225, 223; 800 000 rows K = 64
+// 253 / 251, 249, 249; 200 000 rows K = 32 27.7 / 28.2, 27.3, 26.9, K = 100 116.4 / 114.6, 114.8, 115.5, K = 256 244 / 238,
+// 241, 243.  From 4 blocks on: 532, 226, 259, 27.1, 118, 265.
+constexpr int COL_BLOCKS_MIN = 8, COL_BLOCKS_MAX = WAVE, COL_BLOCK_ENTRIES = 64;
+constexpr int COL_BLOCKS_ORDER = 16;           // that the sort of COO entries knows
+__host__ __device__ inline int row_blocks(int len, int most) {
+    int n = COL_BLOCKS_MIN;
+    while (n < most && len >= 2 * n * COL_BLOCK_ENTRIES) n *= 2;
+    return n;
+}
+
+// `most` lanes per long row: lane b finds where the row's columns of block b start (columns ascend inside a
 // row: its entries of a block are consecutive; in a row that is not sorted the cuts fall anywhere, every
-// entry still lands in exactly one segment).  Segment (b, i): block b of long row i, block-major.
-constexpr int COL_BLOCKS = 16;
+// entry still lands in exactly one segment).  Segment (b, i): block b of long row i, block-major; a row of fewer blocks
+// has its segments at the first of the blocks that each of them covers.
 static __global__ __launch_bounds__(256) void k_long_segments(const int32_t *__restrict__ rowptr,
                                                               const int32_t *__restrict__ col, int N,
                                                               const int32_t *__restrict__ long_rows, int n_long, int piece,
+                                                              int most,
                                                               int32_t *__restrict__ seg_start,
                                                               unsigned int *__restrict__ seg_items) {
     const int64_t slot = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int i = (int)(slot / COL_BLOCKS), b = (int)(slot % COL_BLOCKS);
+    const int i = (int)(slot / most), b = (int)(slot % most);
     const bool on = i < n_long;
-    int lo = 0, end = 0;
+    int lo = 0, end = 0, every = most;
     if (on) {
         const int row = long_rows[i];
         lo = rowptr[row];
         end = rowptr[row + 1];
-        const int first = (int)(((int64_t)N * b + COL_BLOCKS - 1) / COL_BLOCKS);     // (of block b, as in k_order_keys)
+        every = most / row_blocks(end - lo, most);
+        const int first = (int)(((int64_t)N * b + most - 1) / most);     // (of block b, as in k_order_keys)
         int hi = end;
-        if (b == 0) hi = lo;
+        if (b % every != 0 || b == 0) hi = lo;
         while (lo < hi) {
             const int mid = lo + ((hi - lo) >> 1);
             if (col[mid] < first) lo = mid + 1; else hi = mid;
         }
     }
-    // the cuts of a row must ascend whatever its columns do: running maximum over the 16 lanes
-#pragma unroll
-    for (int o = 1; o < COL_BLOCKS; o <<= 1) {
+    // the cuts of a row must ascend whatever its columns do: running maximum over its lanes
+    for (int o = 1; o < most; o <<= 1) {
         const int up = __shfl_up(lo, o, WAVE);
         if (b >= o) lo = up > lo ? up : lo;
     }
-    int next = __shfl_down(lo, 1, WAVE);
-    if (b == COL_BLOCKS - 1) next = end;
+    const int lane = lane_id(), ahead = (every - b % every) % every;         // to the next block that starts a segment
+    const int after = __shfl(lo, (lane + ahead) & (WAVE - 1), WAVE), next_after = __shfl(lo, (lane + every) & (WAVE - 1), WAVE);
     if (!on) return;
-    const int len = next - lo;
-    seg_start[(int64_t)b * n_long + i] = lo;
-    seg_items[(int64_t)b * n_long + i] = (unsigned int)((len + piece - 1) / piece);
+    const int start = b + ahead < most ? after : end;
+    const int next = b % every != 0 ? start : b + every < most ? next_after : end;
+    seg_start[(int64_t)b * n_long + i] = start;
+    seg_items[(int64_t)b * n_long + i] = (unsigned int)((next - start + piece - 1) / piece);
 }
 
 // the entries between long rows: gap i lies before long row i, the last one after all of them
@@ -718,7 +735,7 @@ static __global__ __launch_bounds__(256) void k_order_keys(const int32_t *__rest
                                                            int32_t *__restrict__ at) {
     const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= nnz) return;
-    keys[n] = (Key)row[n] * COL_BLOCKS + (Key)((int64_t)col[n] * COL_BLOCKS / N);
+    keys[n] = (Key)row[n] * COL_BLOCKS_ORDER + (Key)((int64_t)col[n] * COL_BLOCKS_ORDER / N);
     at[n] = (int32_t)n;
 }
 // (32-bit keys lie in row_out, `at` lies in col_out: a thread reads its element of either before it writes there)
@@ -729,7 +746,7 @@ static __global__ __launch_bounds__(256) void k_order_entries(const Key *keys, c
                                                               int32_t *__restrict__ place) {
     const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= nnz) return;
-    const int32_t q = at[n], row = (int32_t)(keys[n] / COL_BLOCKS);
+    const int32_t q = at[n], row = (int32_t)(keys[n] / COL_BLOCKS_ORDER);
     row_out[n] = row;
     col_out[n] = col[q];
     place[q] = (int32_t)n;

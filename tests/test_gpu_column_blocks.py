@@ -76,6 +76,31 @@ def test_column_blocks(engine_factory, monkeypatch, K, dtype, kind):
         _check(e, M, N, rowptr, col, val, A_all[:M], B, dtype, "no long row")
 
 
+@pytest.mark.parametrize("kind", ["spread", "one block", "unsorted"])
+@pytest.mark.parametrize("longest", [257, 1023, 1024, 2048, 4095, 4096, 9000])
+def test_rows_around_the_numbers_of_blocks(engine_factory, monkeypatch, longest, kind):
+    """8, 16, 32 and 64 blocks (from 1 024, 2 048 and 4 096 entries on), rows of every number in one matrix whose longest
+    row sets the most there are; with the grid of a plan that the host has waited for and with that of one it has not."""
+    monkeypatch.setenv("SDDMM_COLUMN_BLOCKS", "1")
+    monkeypatch.setenv("SDDMM_SLICES", "0")
+    N, K = 16 * 10000 if kind == "one block" else 12001, 8
+    rng = np.random.default_rng(longest)
+    edges = [257, 1023, 1024, 1025, 2047, 2048, 4095, 4096, 4097, 9000]
+    lens = np.concatenate([[l for l in edges if l <= longest], rng.integers(0, 9, 4000), [l for l in edges if l <= longest], [3]])
+    A = rng.uniform(-1, 1, (len(lens), K)).astype(f32)
+    B = rng.uniform(-1, 1, (N, K)).astype(f32)
+    with engine_factory() as e:
+        print("numbers of blocks", longest, kind, flush=True)
+        M, rowptr, col, val = _matrix(rng, lens, N, kind)
+        _check(e, M, N, rowptr, col, val, A, B, capi.F32, "longest %d %s" % (longest, kind))
+        want = e.values()
+        e.set_csr(M, N, rowptr, col, val)
+        e.plan(capi.AUTO)
+        e.time_runs(0, 1, include_plan=True)
+        assert e.flat_variant() == capi.FLAT_BLOCKS
+        np.testing.assert_array_equal(e.values(), want)
+
+
 @pytest.mark.parametrize("ts", [1, 257, 258, 600, 100000])
 def test_rows_between_the_segment_length_and_the_short_row_limit(engine_factory, monkeypatch, ts):
     """SDDMM_TS above SDDMM_SEG: the rows in between are no long rows anywhere, neither in the count that sizes the
