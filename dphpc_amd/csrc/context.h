@@ -71,6 +71,7 @@ struct sddmm_ctx {
     TileDesc *d_tiles = nullptr;
     int64_t n_tiles = 0, tiles_cap = 0, nnz_tiles = 0;
     int tile_steps = 0;
+    bool ragged = false;             // tiles and panels of the plan are of ragged rows (ragged_steps)
     bool tiles_active = false;       // d_tiles describes the current pattern
     int32_t *d_win_order = nullptr;  // order in which the launch takes the windows (null: storage order)
     unsigned int *d_win_bins = nullptr;
@@ -330,6 +331,14 @@ inline int panel_mfma_steps(const sddmm_ctx *c) {
     return (steps == 1 || steps == 2 || steps == 4 || steps == 8 || steps == 16) ? steps : 0;
 }
 
+// Steps of 64 bytes that the tile and panel kernels take for rows of no whole power of two of them: as many as the row
+// layout of the gather kernels holds; 0: no such kernel.
+inline int ragged_steps(const sddmm_ctx *c) {
+    const Shape s = shape_of(c);
+    if (s.unit == 1 || s.wide || (s.LPN != 4 && s.LPN != 8) || panel_mfma_steps(c) != 0) return 0;
+    return s.LPN * s.UPL / 4;
+}
+
 // The device code of a translation unit is loaded when something first asks for one of its kernels: 3 .. 13 ms, once per
 // process.  A plan asks for the families that its launches take (load_*, one per launch_*.hip), so that no launch has to:
 // launches may be captured, and they are what callers time.
@@ -340,8 +349,10 @@ inline hipError_t load_code(const void *kernel) {
 hipError_t load_flat();
 hipError_t load_rows();
 hipError_t load_auto();
-hipError_t load_tiles();
-hipError_t load_panels();
+hipError_t load_tiles(bool ragged);
+hipError_t load_ragged_tiles();
+hipError_t load_panels(bool ragged);
+hipError_t load_ragged_panels();
 hipError_t load_fused();
 
 // ---- launchers, one translation unit per family of kernels ----
@@ -360,7 +371,10 @@ void launch_short_rows(sddmm_ctx *c, int ts, int rpw);
 void launch_auto(sddmm_ctx *c);                                                  // launch_auto.hip
 bool launch_auto_with_tiles(sddmm_ctx *c);                                       // launch_tiles.hip
 void launch_tiles(sddmm_ctx *c);
+bool launch_ragged_auto_with_tiles(sddmm_ctx *c);                                // launch_tiles_ragged.hip
+void launch_ragged_tiles(sddmm_ctx *c);
 void launch_panels(sddmm_ctx *c);                                                // launch_panels.hip
+void launch_ragged_panels(sddmm_ctx *c);                                         // launch_panels_ragged.hip
 void launch_panels_fused(sddmm_ctx *c);
 // the list of the rows for k_add_cut_rows
 inline int32_t *fused_cut_rows(const sddmm_ctx *c) {

@@ -847,6 +847,102 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_apply(const unsigned
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 
+// ---- rows as the tile and panel kernels read them ---------------------------------------
+// Step s of these kernels takes the units (16 bytes) 4s .. 4s+3 of a row.  WholeRows: rows of STEPS * 64 bytes.
+// RaggedRows: rows of any other length up to that (more than ragged_whole_steps).  A unit past the end
+// of the row is the last one loaded again, and is zeroed (trim) once it has arrived, in both operands: what a product
+// adds there is 0 * 0 whatever the rows hold.  fp32 rows of no whole number of units are read as the gather kernels
+// read them (UnitF32x4u).
+constexpr int ragged_whole_steps(int steps) {
+    return steps <= 1 ? 0 : steps == 2 ? 1 : steps == 4 ? 2 : steps == 6 ? 4 : steps == 8 ? 6 : steps == 12 ? 8 : 12;
+}
+
+template <int STEPS>
+struct WholeRows {
+    static constexpr bool RAGGED = false;
+    using Row = const uint4 *;
+    explicit __device__ __forceinline__ WholeRows(int) {}
+    __device__ __forceinline__ Row row(const void *base, int64_t r) const { return (const uint4 *)base + r * (STEPS * 4); }
+    __device__ __forceinline__ uint4 unit(const void *, Row row, int u, int) const { return row[u]; }
+    __device__ __forceinline__ uint4 trim(const uint4 &v, int, int) const { return v; }
+};
+
+template <class U_, int STEPS>
+struct RaggedRows {
+    using U = U_;
+    static constexpr bool RAGGED = true;
+    static constexpr int WHOLE_STEPS = ragged_whole_steps(STEPS);
+    using Row = uint32_t;                                     // byte offset: operands below 4 GiB
+    int len, last;                                            // length as U takes it, last unit
+    explicit __device__ __forceinline__ RaggedRows(int len_) : len(len_), last(U::units(len_) - 1) {}
+    __device__ __forceinline__ Row row(const void *, int64_t r) const { return (uint32_t)r * U::row_bytes(len); }
+    // unit u of a row; step: the step it belongs to as far as the compiler knows it (STEPS: any)
+    __device__ __forceinline__ uint4 unit(const void *base, Row row, int u, int step) const {
+        const uint32_t at = step < WHOLE_STEPS ? (uint32_t)u * 16u : U::unit_off(u < last ? u : last, len);
+        return __builtin_bit_cast(uint4, load_unit<U, uint32_t>(base, row + at));
+    }
+    __device__ __forceinline__ uint4 trim(const uint4 &v, int u, int step) const {
+        if (step < WHOLE_STEPS) return v;
+        const uint4 t = __builtin_bit_cast(uint4, U::trim(__builtin_bit_cast(typename U::T, v), u, len));
+        const bool in = u <= last;
+        return make_uint4(in ? t.x : 0u, in ? t.y : 0u, in ? t.z : 0u, in ? t.w : 0u);
+    }
+};
+
+// acc += the products of one unit of 16 rows with one of 16 columns.  Where CHAINS is 4 the four components of an fp32
+// unit have an accumulator each.
+template <int DT, int CHAINS>
+__device__ __forceinline__ void mfma_unit(const uint4 &a, const uint4 &b, f32x4_t (&acc)[CHAINS]) {
+    if constexpr (DT == DT_BF16) {
+        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b),
+                                                         acc[0], 0, 0, 0);
+    } else if constexpr (DT == DT_F16) {
+        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b),
+                                                        acc[0], 0, 0, 0);
+    } else {
+        auto part = [&](uint32_t x, uint32_t y, f32x4_t &c) {
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, x), __builtin_bit_cast(float, y), c, 0, 0, 0);
+        };
+        part(a.x, b.x, acc[0]);
+        part(a.y, b.y, acc[1 % CHAINS]);
+        part(a.z, b.z, acc[2 % CHAINS]);
+        part(a.w, b.w, acc[3 % CHAINS]);
+    }
+}
+
+// f(S0) + ... + f(S0 + N - 1), added in pairs
+template <int S0, int N, class F>
+__device__ __forceinline__ auto pairwise(F &&f) {
+    if constexpr (N == 1) return f(std::integral_constant<int, S0>{});
+    else return pairwise<S0, (N + 1) / 2>(f) + pairwise<S0 + (N + 1) / 2, N / 2>(f);
+}
+
+// The 16x16 products of N steps; b(s): the column operand of step s.  Whole rows: one accumulator.
+// The gather kernels, which took ragged rows before, add up chains of an eighth of a row; one accumulator over all of it is
+// further from the exact sum (fp32 K = 250 1.5e-7 of the result's norm against 1.2e-7, bf16 K = 456 1.0e-7 against 0.7e-7),
+// so every step starts from zero and the steps are added in pairs (0.9e-7 and 0.7e-7).
+template <int DT, class R, int N, class F>
+__device__ __forceinline__ f32x4_t mfma_steps(const uint4 (&a)[N], F &&b) {
+    if constexpr (R::RAGGED) {
+        return pairwise<0, N>([&](auto s) {
+            constexpr int CHAINS = DT == DT_F32 ? 4 : 1;
+            f32x4_t acc[CHAINS] = {};
+            mfma_unit<DT, CHAINS>(a[(int)s], b((int)s), acc);
+            if constexpr (CHAINS == 4) {
+                const f32x4_t sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+                // (steps that overlap take sixteen registers each: near-dense rows K = 33 23 -> 52 us without this, in spills)
+                __builtin_amdgcn_sched_barrier(0);
+                return sum;
+            } else return acc[0];
+        });
+    } else {
+        f32x4_t acc[1] = {};
+#pragma unroll
+        for (int s = 0; s < N; ++s) mfma_unit<DT, 1>(a[s], b(s), acc);
+        return acc[0];
+    }
+}
+
 // One wavefront computes `tiles_per_wave` consecutive tiles.  Operand layout of
 // both MFMA shapes used: lane l supplies row (l & 15) of its operand and the k
 // positions selected by (l >> 4); the result register i of lane l is row
@@ -867,8 +963,8 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 // The A panel of the current strip stays in registers and is reloaded only when
 // the strip changes (a wave-uniform branch placed before the iteration's loads).
 // tiles [w*tiles_per_wave, (w+1)*tiles_per_wave) on the calling wavefront
-template <int DT, int STEPS>
-__device__ __forceinline__ void tile_wave(const void *__restrict__ A, const void *__restrict__ B, int M, int N,
+template <int DT, int STEPS, class R>
+__device__ __forceinline__ void tile_wave(const R &rows, const void *__restrict__ A, const void *__restrict__ B, int M, int N,
                                           const int32_t *__restrict__ vrows, const int32_t *__restrict__ tile_cols,
                                           const TileDesc *__restrict__ tiles, int64_t n_tiles, int tiles_per_wave,
                                           const float *__restrict__ sval, float *__restrict__ P, int64_t w) {
@@ -881,17 +977,14 @@ __device__ __forceinline__ void tile_wave(const void *__restrict__ A, const void
     const int r16 = lane & 15, q = lane >> 4;        // operand / result layout
     const int lrow = lane >> 2, lunit = lane & 3;    // memory layout: four neighbouring lanes on 64 bytes of a row
     const int to_operand_from = (4 * r16 + q) << 2;  // ds_bpermute address: operand lane (r16,q) <- memory lane 4*r16+q
-    constexpr uint32_t ROW_UNITS = STEPS * 4;
-    const uint4 *__restrict__ Au = (const uint4 *)A;
-    const uint4 *__restrict__ Bu = (const uint4 *)B;
     const unsigned int below = (1u << r16) - 1u;
-    auto to_operand = [&](const uint4 &v) {
+    auto to_operand = [&](const uint4 &v, int s) {     // unit 4s + q of the lane's row
         uint4 r;
         r.x = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.x);
         r.y = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.y);
         r.z = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.z);
         r.w = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.w);
-        return r;
+        return rows.trim(r, 4 * s + q, s);
     };
 
     struct Desc {
@@ -919,9 +1012,9 @@ __device__ __forceinline__ void tile_wave(const void *__restrict__ A, const void
         Oper o;
         int64_t brow = d.bcol;
         brow = brow < N ? brow : N - 1;   // columns past N (and the filler of a short union tile) are never in a mask
-        const uint4 *src = Bu + brow * ROW_UNITS + lunit;
+        const typename R::Row src = rows.row(B, brow);
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) o.b[s] = src[s * 4];
+        for (int s = 0; s < STEPS; ++s) o.b[s] = rows.unit(B, src, 4 * s + lunit, s);
         const int offs[4] = {d.off.x, d.off.y, d.off.z, d.off.w};
         const unsigned int masks[4] = {d.mask.x & 0xFFFFu, d.mask.x >> 16, d.mask.y & 0xFFFFu, d.mask.y >> 16};
         o.act = 0;
@@ -948,37 +1041,17 @@ __device__ __forceinline__ void tile_wave(const void *__restrict__ A, const void
             int64_t arow = strip >= GATHERED_BASE ? (int64_t)vrows[(int64_t)(strip - GATHERED_BASE) * 16 + lrow]
                                                   : (int64_t)strip * 16 + lrow;
             arow = arow < 0 ? 0 : (arow < M ? arow : M - 1);   // missing rows are never in a mask
-            const uint4 *src = Au + arow * ROW_UNITS + lunit;
+            const typename R::Row src = rows.row(A, arow);
 #pragma unroll
-            for (int s = 0; s < STEPS; ++s) a[s] = to_operand(src[s * 4]);
+            for (int s = 0; s < STEPS; ++s) a[s] = to_operand(rows.unit(A, src, 4 * s + lunit, s), s);
         }
         const Oper o_nxt = load_oper(d_nxt);
         const Desc d_nn = load_desc(t + 2);
-        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < STEPS; ++s) {
-            const uint4 b = to_operand(o_cur.b[s]);
-            if constexpr (DT == DT_BF16) {
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[s]),
-                                                              __builtin_bit_cast(bf16x8_t, b), acc, 0, 0, 0);
-            } else if constexpr (DT == DT_F16) {
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a[s]),
-                                                             __builtin_bit_cast(half8_t, b), acc, 0, 0, 0);
-            } else {
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a[s].x),
-                                                           __builtin_bit_cast(float, b.x), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a[s].y),
-                                                           __builtin_bit_cast(float, b.y), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a[s].z),
-                                                           __builtin_bit_cast(float, b.z), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a[s].w),
-                                                           __builtin_bit_cast(float, b.w), acc, 0, 0, 0);
-            }
-        }
+        const f32x4_t sum = mfma_steps<DT, R>(a, [&](int s) { return to_operand(o_cur.b[s], s); });
         // scale by S and scatter: result register i is row 4*q+i, column r16
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            if ((o_cur.act >> i) & 1u) P[o_cur.pos[i]] = acc[i] * o_cur.s[i];
+            if ((o_cur.act >> i) & 1u) P[o_cur.pos[i]] = sum[i] * o_cur.s[i];
         o_cur = o_nxt;
         d_cur = d_nxt;
         d_nxt = d_nn;
@@ -1069,8 +1142,8 @@ static __global__ __launch_bounds__(256) void k_tile_windows(const int32_t *__re
 }
 
 // window w on the calling wavefront; lds: WIN_LDS_FLOATS floats of its own
-template <int DT, int STEPS>
-__device__ __forceinline__ void tile_window_wave(const void *__restrict__ A, const void *__restrict__ B, int M, int N,
+template <int DT, int STEPS, class R>
+__device__ __forceinline__ void tile_window_wave(const R &rows, const void *__restrict__ A, const void *__restrict__ B, int M, int N,
                                                  const int32_t *__restrict__ vrows,
                                                  const int32_t *__restrict__ tile_cols,
                                                  const TileDesc *__restrict__ tiles, int64_t n_tiles,
@@ -1082,13 +1155,13 @@ __device__ __forceinline__ void tile_window_wave(const void *__restrict__ A, con
     if (order) w = order[w];                              // the plan's order of the windows (k_window_order)
     const int lane = lane_id();
     if (win == nullptr) {                                 // the plan chose the tile-by-tile walk for this matrix
-        tile_wave<DT, STEPS>(A, B, M, N, vrows, tile_cols, tiles, n_tiles, TILE_WINDOW, sval, P, w);
+        tile_wave<DT, STEPS>(rows, A, B, M, N, vrows, tile_cols, tiles, n_tiles, TILE_WINDOW, sval, P, w);
         return;
     }
     const int32_t *rec = reinterpret_cast<const int32_t *>(win + w);
     const int dw = rec[lane < 48 ? lane : 47];
     if (__builtin_amdgcn_readlane(dw, 44) != 0) {
-        tile_wave<DT, STEPS>(A, B, M, N, vrows, tile_cols, tiles, n_tiles, TILE_WINDOW, sval, P, w);
+        tile_wave<DT, STEPS>(rows, A, B, M, N, vrows, tile_cols, tiles, n_tiles, TILE_WINDOW, sval, P, w);
         return;
     }
     const int maxcnt = __builtin_amdgcn_readlane(dw, 45);
@@ -1096,16 +1169,13 @@ __device__ __forceinline__ void tile_window_wave(const void *__restrict__ A, con
     const int r16 = lane & 15, q = lane >> 4;        // operand / result layout
     const int lrow = lane >> 2, lunit = lane & 3;    // memory layout: four neighbouring lanes on 64 bytes of a row
     const int to_operand_from = (4 * r16 + q) << 2;
-    constexpr uint32_t ROW_UNITS = STEPS * 4;
-    const uint4 *__restrict__ Au = (const uint4 *)A;
-    const uint4 *__restrict__ Bu = (const uint4 *)B;
-    auto to_operand = [&](const uint4 &v) {
+    auto to_operand = [&](const uint4 &v, int s) {     // unit 4s + q of the lane's row
         uint4 r;
         r.x = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.x);
         r.y = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.y);
         r.z = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.z);
         r.w = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.w);
-        return r;
+        return rows.trim(r, 4 * s + q, s);
     };
     int tj[TILE_WINDOW];
 #pragma unroll
@@ -1125,16 +1195,16 @@ __device__ __forceinline__ void tile_window_wave(const void *__restrict__ A, con
     // ---- second round trip: everything at once ----------------------------------------
     uint4 a_mem[STEPS];
     {
-        const uint4 *src = Au + arow * ROW_UNITS + lunit;
+        const typename R::Row src = rows.row(A, arow);
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) a_mem[s] = src[s * 4];
+        for (int s = 0; s < STEPS; ++s) a_mem[s] = rows.unit(A, src, 4 * s + lunit, s);
     }
     auto load_b = [&](int k, uint4 (&dst)[STEPS]) {
         int64_t brow = (int64_t)(tj[k] < 0 ? 0 : tj[k]) * 16 + lrow;
         brow = brow < N ? brow : N - 1;                   // columns past N are in no row's entries
-        const uint4 *src = Bu + brow * ROW_UNITS + lunit;
+        const typename R::Row src = rows.row(B, brow);
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) dst[s] = src[s * 4];
+        for (int s = 0; s < STEPS; ++s) dst[s] = rows.unit(B, src, 4 * s + lunit, s);
     };
     // rows of up to 128 bytes: the B rows of all four tiles in flight; longer rows two tiles at a time (at 256
     // bytes four in flight cost 13 registers and a wave per SIMD of the launch that also runs rows: 22.0 -> 21.2 us)
@@ -1158,31 +1228,11 @@ __device__ __forceinline__ void tile_window_wave(const void *__restrict__ A, con
     // ---- products of every tile into LDS ------------------------------------------------
     uint4 a[STEPS];
 #pragma unroll
-    for (int s = 0; s < STEPS; ++s) a[s] = to_operand(a_mem[s]);
+    for (int s = 0; s < STEPS; ++s) a[s] = to_operand(a_mem[s], s);
     auto product = [&](const uint4 (&bt)[STEPS], int k) {
-        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < STEPS; ++s) {
-            const uint4 bo = to_operand(bt[s]);
-            if constexpr (DT == DT_BF16) {
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[s]),
-                                                              __builtin_bit_cast(bf16x8_t, bo), acc, 0, 0, 0);
-            } else if constexpr (DT == DT_F16) {
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a[s]),
-                                                             __builtin_bit_cast(half8_t, bo), acc, 0, 0, 0);
-            } else {
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a[s].x),
-                                                           __builtin_bit_cast(float, bo.x), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a[s].y),
-                                                           __builtin_bit_cast(float, bo.y), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a[s].z),
-                                                           __builtin_bit_cast(float, bo.z), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a[s].w),
-                                                           __builtin_bit_cast(float, bo.w), acc, 0, 0, 0);
-            }
-        }
+        const f32x4_t sum = mfma_steps<DT, R>(a, [&](int s) { return to_operand(bt[s], s); });
         // result register i of lane (r16, q) is row 4q+i, column r16 of tile k
-        *reinterpret_cast<f32x4_t *>(lds + (k * 16 + r16) * WIN_PITCH + 4 * q) = acc;
+        *reinterpret_cast<f32x4_t *>(lds + (k * 16 + r16) * WIN_PITCH + 4 * q) = sum;
     };
     if constexpr (ALL_B) {
 #pragma unroll
@@ -1225,12 +1275,14 @@ __device__ __forceinline__ void tile_window_wave(const void *__restrict__ A, con
 }
 
 constexpr int PAIR_MAX_STEPS = 4;             // row bytes / 64 up to which pairs of windows share a wavefront
+// (not with ragged fp32 rows, whose sums take more registers: near-dense rows K = 48 39 us in pairs, 23 without)
+constexpr bool tile_pairs(bool ragged, bool f32, int steps) { return steps <= PAIR_MAX_STEPS && !(ragged && f32); }
 // Windows wa and wa+1 of a pair of gathered strips on the calling wavefront: the same four tile
 // columns for 2 x 16 rows.  Every B tile is loaded and moved into operand layout once and
 // multiplied with both A panels; the products of the second strip wait in registers while the
 // entries of the first are picked out of the LDS buffer (one buffer, as for a single window).
-template <int DT, int STEPS>
-__device__ __forceinline__ void tile_window_pair_wave(const void *__restrict__ A, const void *__restrict__ B, int M, int N,
+template <int DT, int STEPS, class R>
+__device__ __forceinline__ void tile_window_pair_wave(const R &rows, const void *__restrict__ A, const void *__restrict__ B, int M, int N,
                                                       const int32_t *__restrict__ vrows,
                                                       const int32_t *__restrict__ tile_cols,
                                                       const TileDesc *__restrict__ tiles, int64_t n_tiles,
@@ -1252,7 +1304,7 @@ __device__ __forceinline__ void tile_window_pair_wave(const void *__restrict__ A
     }
     if (!plain) {                                         // wave-uniform: one window after the other
         for (int64_t w = wa; w < wa + 2; ++w)
-            tile_window_wave<DT, STEPS>(A, B, M, N, vrows, tile_cols, tiles, n_tiles, win, n_win, col, sval, P, nnz, w, lds);
+            tile_window_wave<DT, STEPS>(rows, A, B, M, N, vrows, tile_cols, tiles, n_tiles, win, n_win, col, sval, P, nnz, w, lds);
         return;
     }
     const int maxcnt0 = __builtin_amdgcn_readlane(dw0, 45), maxcnt1 = __builtin_amdgcn_readlane(dw1, 45);
@@ -1260,16 +1312,13 @@ __device__ __forceinline__ void tile_window_pair_wave(const void *__restrict__ A
     const int r16 = lane & 15, q = lane >> 4;        // operand / result layout
     const int lrow = lane >> 2, lunit = lane & 3;    // memory layout: four neighbouring lanes on 64 bytes of a row
     const int to_operand_from = (4 * r16 + q) << 2;
-    constexpr uint32_t ROW_UNITS = STEPS * 4;
-    const uint4 *__restrict__ Au = (const uint4 *)A;
-    const uint4 *__restrict__ Bu = (const uint4 *)B;
-    auto to_operand = [&](const uint4 &v) {
+    auto to_operand = [&](const uint4 &v, int s) {     // unit 4s + q of the lane's row
         uint4 r;
         r.x = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.x);
         r.y = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.y);
         r.z = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.z);
         r.w = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.w);
-        return r;
+        return rows.trim(r, 4 * s + q, s);
     };
     // S/P accesses of this lane in either strip: strip row lane>>2, its entries 4(lane&3)+16m.. of the window
     struct Rows { int p0, cnt; };
@@ -1292,16 +1341,19 @@ __device__ __forceinline__ void tile_window_pair_wave(const void *__restrict__ A
     uint4 a0[STEPS], a1[STEPS];
     {
         const int64_t ar0 = __shfl(dw0, lrow, WAVE), ar1 = __shfl(dw1, lrow, WAVE);
-        const uint4 *s0 = Au + ar0 * ROW_UNITS + lunit, *s1 = Au + ar1 * ROW_UNITS + lunit;
+        const typename R::Row s0 = rows.row(A, ar0), s1 = rows.row(A, ar1);
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) { a0[s] = s0[s * 4]; a1[s] = s1[s * 4]; }
+        for (int s = 0; s < STEPS; ++s) {
+            a0[s] = rows.unit(A, s0, 4 * s + lunit, s);
+            a1[s] = rows.unit(A, s1, 4 * s + lunit, s);
+        }
     }
     auto load_b = [&](int k, uint4 (&dst)[STEPS]) {
         int64_t brow = (int64_t)(tj[k] < 0 ? 0 : tj[k]) * 16 + lrow;
         brow = brow < N ? brow : N - 1;                   // columns past N are in no row's entries
-        const uint4 *src = Bu + brow * ROW_UNITS + lunit;
+        const typename R::Row src = rows.row(B, brow);
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) dst[s] = src[s * 4];
+        for (int s = 0; s < STEPS; ++s) dst[s] = rows.unit(B, src, 4 * s + lunit, s);
     };
     uint4 b[2][STEPS];                                    // two B tiles in flight
     load_b(0, b[0]);
@@ -1321,45 +1373,35 @@ __device__ __forceinline__ void tile_window_pair_wave(const void *__restrict__ A
     const Pre pre0 = prefetch(rows0, iters0);
     // ---- products: strip 0's into LDS, strip 1's kept ----------------------------------------------
 #pragma unroll
-    for (int s = 0; s < STEPS; ++s) { a0[s] = to_operand(a0[s]); a1[s] = to_operand(a1[s]); }
+    for (int s = 0; s < STEPS; ++s) { a0[s] = to_operand(a0[s], s); a1[s] = to_operand(a1[s], s); }
     f32x4_t keep[TILE_WINDOW];
 #pragma unroll
     for (int k = 0; k < TILE_WINDOW; ++k) {
         keep[k] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         if (tj[k] < 0) continue;                          // wave-uniform
-        f32x4_t acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+        f32x4_t sum0, sum1;
+        if constexpr (R::RAGGED) {
+            uint4 bo[STEPS];
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) {
-            const uint4 bo = to_operand(b[k & 1][s]);
-            if constexpr (DT == DT_BF16) {
-                acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a0[s]),
-                                                               __builtin_bit_cast(bf16x8_t, bo), acc0, 0, 0, 0);
-                acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a1[s]),
-                                                               __builtin_bit_cast(bf16x8_t, bo), acc1, 0, 0, 0);
-            } else if constexpr (DT == DT_F16) {
-                acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a0[s]),
-                                                              __builtin_bit_cast(half8_t, bo), acc0, 0, 0, 0);
-                acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a1[s]),
-                                                              __builtin_bit_cast(half8_t, bo), acc1, 0, 0, 0);
-            } else {
-                const float bf[4] = {__builtin_bit_cast(float, bo.x), __builtin_bit_cast(float, bo.y),
-                                     __builtin_bit_cast(float, bo.z), __builtin_bit_cast(float, bo.w)};
-                const float f0[4] = {__builtin_bit_cast(float, a0[s].x), __builtin_bit_cast(float, a0[s].y),
-                                     __builtin_bit_cast(float, a0[s].z), __builtin_bit_cast(float, a0[s].w)};
-                const float f1[4] = {__builtin_bit_cast(float, a1[s].x), __builtin_bit_cast(float, a1[s].y),
-                                     __builtin_bit_cast(float, a1[s].z), __builtin_bit_cast(float, a1[s].w)};
+            for (int s = 0; s < STEPS; ++s) bo[s] = to_operand(b[k & 1][s], s);
+            sum0 = mfma_steps<DT, R>(a0, [&](int s) { return bo[s]; });
+            sum1 = mfma_steps<DT, R>(a1, [&](int s) { return bo[s]; });
+        } else {
+            f32x4_t acc0[1] = {}, acc1[1] = {};
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(f0[i], bf[i], acc0, 0, 0, 0);
-                    acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(f1[i], bf[i], acc1, 0, 0, 0);
-                }
+            for (int s = 0; s < STEPS; ++s) {
+                const uint4 bo = to_operand(b[k & 1][s], s);
+                mfma_unit<DT, 1>(a0[s], bo, acc0);
+                mfma_unit<DT, 1>(a1[s], bo, acc1);
             }
+            sum0 = acc0[0];
+            sum1 = acc1[0];
         }
         // the registers of this B tile are free: the tile after the next one
         if (k + 2 < TILE_WINDOW && tj[k + 2 < TILE_WINDOW ? k + 2 : k] >= 0) load_b(k + 2, b[k & 1]);
         // result register i of lane (r16, q) is row 4q+i, column r16 of tile k
-        *reinterpret_cast<f32x4_t *>(lds + (k * 16 + r16) * WIN_PITCH + 4 * q) = acc0;
-        keep[k] = acc1;
+        *reinterpret_cast<f32x4_t *>(lds + (k * 16 + r16) * WIN_PITCH + 4 * q) = sum0;
+        keep[k] = sum1;
     }
     wave_lds_order();
     const Pre pre1 = prefetch(rows1, iters1);             // lands while strip 0's entries are written
@@ -1401,8 +1443,8 @@ __device__ __forceinline__ void tile_window_pair_wave(const void *__restrict__ A
 
 // Wavefront `unit` of a tile launch: windows [0, n_single) one per wavefront, the windows after them (pairs of
 // gathered strips) two per wavefront.
-template <int DT, int STEPS>
-__device__ __forceinline__ void tile_unit_wave(const void *__restrict__ A, const void *__restrict__ B, int M, int N,
+template <int DT, int STEPS, class R>
+__device__ __forceinline__ void tile_unit_wave(const R &rows, const void *__restrict__ A, const void *__restrict__ B, int M, int N,
                                                const int32_t *__restrict__ vrows, const int32_t *__restrict__ tile_cols,
                                                const TileDesc *__restrict__ tiles, int64_t n_tiles,
                                                const TileWindow *__restrict__ win, int64_t n_win, int64_t n_single,
@@ -1411,18 +1453,19 @@ __device__ __forceinline__ void tile_unit_wave(const void *__restrict__ A, const
                                                const int32_t *__restrict__ order) {
     // (rows beyond 256 bytes: the second A panel and the kept products do not fit the registers, the
     // plan gives such launches one wavefront per window throughout)
-    if (STEPS > PAIR_MAX_STEPS || win == nullptr || unit < n_single) {     // wave-uniform
-        tile_window_wave<DT, STEPS>(A, B, M, N, vrows, tile_cols, tiles, n_tiles, win, n_win, col, sval, P, nnz, unit, lds,
+    constexpr bool PAIRS = tile_pairs(R::RAGGED, DT == DT_F32, STEPS);
+    if (!PAIRS || win == nullptr || unit < n_single) {     // wave-uniform
+        tile_window_wave<DT, STEPS>(rows, A, B, M, N, vrows, tile_cols, tiles, n_tiles, win, n_win, col, sval, P, nnz, unit, lds,
                                     order);
         return;
     }
-    if constexpr (STEPS <= PAIR_MAX_STEPS)
-        tile_window_pair_wave<DT, STEPS>(A, B, M, N, vrows, tile_cols, tiles, n_tiles, win, n_win, col, sval, P, nnz,
+    if constexpr (PAIRS)
+        tile_window_pair_wave<DT, STEPS>(rows, A, B, M, N, vrows, tile_cols, tiles, n_tiles, win, n_win, col, sval, P, nnz,
                                          n_single + 2 * (unit - n_single), lds);
 }
 
-template <int DT, int STEPS>
-__global__ __launch_bounds__(BLOCK) void k_tile(const void *__restrict__ A, const void *__restrict__ B, int M, int N,
+template <int DT, int STEPS, class R>
+__global__ __launch_bounds__(BLOCK) void k_tile(const void *__restrict__ A, const void *__restrict__ B, int len, int M, int N,
                                                 const int32_t *__restrict__ vrows,
                                                 const int32_t *__restrict__ tile_cols,
                                                 const TileDesc *__restrict__ tiles, int64_t n_tiles,
@@ -1433,7 +1476,7 @@ __global__ __launch_bounds__(BLOCK) void k_tile(const void *__restrict__ A, cons
     __shared__ __attribute__((aligned(16))) float win_lds[WAVES_PER_BLOCK][WIN_LDS_FLOATS];
     const int64_t blk = xcd_remap(blockIdx.x, nblocks);
     if (blk < 0) return;
-    tile_unit_wave<DT, STEPS>(A, B, M, N, vrows, tile_cols, tiles, n_tiles, win, n_win, n_single, col, sval, P, nnz,
+    tile_unit_wave<DT, STEPS>(R(len), A, B, M, N, vrows, tile_cols, tiles, n_tiles, win, n_win, n_single, col, sval, P, nnz,
                               blk * WAVES_PER_BLOCK + wave_in_block(), win_lds[wave_in_block()], order);
 }
 
@@ -1449,8 +1492,8 @@ constexpr int KSPLIT = WAVES_PER_BLOCK;
 static_assert(KSPLIT == 4 && TILE_WINDOW == 4, "one finishing wave per tile of a window");
 constexpr int KSPLIT_LDS_FLOATS = TILE_WINDOW * KSPLIT * 256;
 
-template <int DT, int STEPS>
-__global__ __launch_bounds__(BLOCK) void k_tile_ksplit(const void *__restrict__ A, const void *__restrict__ B, int M, int N,
+template <int DT, int STEPS, class R>
+__global__ __launch_bounds__(BLOCK) void k_tile_ksplit(const void *__restrict__ A, const void *__restrict__ B, int len, int M, int N,
                                                        const int32_t *__restrict__ vrows,
                                                        const int32_t *__restrict__ tile_cols,
                                                        const TileDesc *__restrict__ tiles, int64_t n_tiles,
@@ -1470,16 +1513,15 @@ __global__ __launch_bounds__(BLOCK) void k_tile_ksplit(const void *__restrict__ 
     const int r16 = lane & 15, q = lane >> 4;        // operand / result layout
     const int lrow = lane >> 2, lunit = lane & 3;    // memory layout: four neighbouring lanes on 64 bytes of a row
     const int to_operand_from = (4 * r16 + q) << 2;
-    constexpr uint32_t ROW_UNITS = STEPS * 4;
-    const uint4 *__restrict__ Au = (const uint4 *)A + (uint32_t)(j * SW * 4);    // this wave's quarter of every row
-    const uint4 *__restrict__ Bu = (const uint4 *)B + (uint32_t)(j * SW * 4);
-    auto to_operand = [&](const uint4 &v) {
+    const R rows(len);
+    const int u0 = j * SW * 4;                            // this wave's quarter of every row
+    auto to_operand = [&](const uint4 &v, int s) {
         uint4 r;
         r.x = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.x);
         r.y = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.y);
         r.z = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.z);
         r.w = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.w);
-        return r;
+        return rows.trim(r, u0 + 4 * s + q, STEPS);
     };
     // first round trip: strip and B rows of every tile, the per-row fields of this wave's own tile
     // (one load each: lane u of every quad asks for tile u, the values are dealt out inside the quad)
@@ -1500,22 +1542,22 @@ __global__ __launch_bounds__(BLOCK) void k_tile_ksplit(const void *__restrict__ 
         int64_t arow = st >= GATHERED_BASE ? (int64_t)vrows[(int64_t)(st - GATHERED_BASE) * 16 + lrow]
                                            : (int64_t)st * 16 + lrow;
         arow = arow < 0 ? 0 : (arow < M ? arow : M - 1);      // missing rows are never in a mask
-        return Au + arow * ROW_UNITS + lunit;
+        return rows.row(A, arow);
     };
     // second round trip: this wave's quarter of the A panel and of all B tiles, the S values of its own tile
     uint4 a[SW], b[TILE_WINDOW][SW];
     {
-        const uint4 *src = a_rows(strip[0]);
+        const typename R::Row src = a_rows(strip[0]);
 #pragma unroll
-        for (int s = 0; s < SW; ++s) a[s] = src[s * 4];
+        for (int s = 0; s < SW; ++s) a[s] = rows.unit(A, src, u0 + 4 * s + lunit, STEPS);
     }
 #pragma unroll
     for (int k = 0; k < TILE_WINDOW; ++k) {
         int64_t brow = bcol[k];
         brow = brow < N ? brow : N - 1;                   // columns past N (and the filler of a short union tile) are in no mask
-        const uint4 *src = Bu + brow * ROW_UNITS + lunit;
+        const typename R::Row src = rows.row(B, brow);
 #pragma unroll
-        for (int s = 0; s < SW; ++s) b[k][s] = src[s * 4];
+        for (int s = 0; s < SW; ++s) b[k][s] = rows.unit(B, src, u0 + 4 * s + lunit, STEPS);
     }
     const unsigned int below = (1u << r16) - 1u;
     const int offs[4] = {off4.x, off4.y, off4.z, off4.w};
@@ -1531,37 +1573,17 @@ __global__ __launch_bounds__(BLOCK) void k_tile_ksplit(const void *__restrict__ 
         sv[i] = sval[pos[i]];
     }
 #pragma unroll
-    for (int s = 0; s < SW; ++s) a[s] = to_operand(a[s]);
+    for (int s = 0; s < SW; ++s) a[s] = to_operand(a[s], s);
 #pragma unroll
     for (int k = 0; k < TILE_WINDOW; ++k) {
         if (k >= n) break;                                // workgroup-uniform
         if (k > 0 && strip[k] != strip[k - 1]) {          // workgroup-uniform: the window reaches into the next strip
-            const uint4 *src = a_rows(strip[k]);
+            const typename R::Row src = a_rows(strip[k]);
 #pragma unroll
-            for (int s = 0; s < SW; ++s) a[s] = to_operand(src[s * 4]);
+            for (int s = 0; s < SW; ++s) a[s] = to_operand(rows.unit(A, src, u0 + 4 * s + lunit, STEPS), s);
         }
-        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < SW; ++s) {
-            const uint4 bo = to_operand(b[k][s]);
-            if constexpr (DT == DT_BF16) {
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[s]),
-                                                              __builtin_bit_cast(bf16x8_t, bo), acc, 0, 0, 0);
-            } else if constexpr (DT == DT_F16) {
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a[s]),
-                                                             __builtin_bit_cast(half8_t, bo), acc, 0, 0, 0);
-            } else {
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a[s].x),
-                                                           __builtin_bit_cast(float, bo.x), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a[s].y),
-                                                           __builtin_bit_cast(float, bo.y), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a[s].z),
-                                                           __builtin_bit_cast(float, bo.z), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, a[s].w),
-                                                           __builtin_bit_cast(float, bo.w), acc, 0, 0, 0);
-            }
-        }
-        *reinterpret_cast<f32x4_t *>(part + (k * KSPLIT + j) * 256 + lane * 4) = acc;
+        *reinterpret_cast<f32x4_t *>(part + (k * KSPLIT + j) * 256 + lane * 4) =
+            mfma_steps<DT, R>(a, [&](int s) { return to_operand(b[k][s], s); });
     }
     __syncthreads();
     if (j < n) {
@@ -1627,7 +1649,7 @@ static __global__ __launch_bounds__(256) void k_window_scatter(const TileDesc *_
 // evenly between tile blocks (tile_wave), segment-item blocks and short-row blocks,
 // so that every XCD gets its share of each.  Kernels of one stream run one after
 // the other; two short launches leave the chip half idle twice, one launch does not.
-// L must be the full-K, 32-bit-offset layout of a row of STEPS * 64 bytes.
+// L: a 32-bit-offset layout of 4 * STEPS units, full-K for rows of STEPS * 64 bytes.
 #ifndef SDDMM_FUSED_WAVES
 #define SDDMM_FUSED_WAVES 5
 #endif
@@ -1678,7 +1700,11 @@ __global__ __launch_bounds__(BLOCK, STEPS <= 2 ? SDDMM_FUSED_WAVES : STEPS == 4 
         }
     }
     if (tile_block >= 0) {
-        tile_unit_wave<L::U::DT, STEPS>(A, B, M, N, vrows, tile_cols, tiles, n_tiles, win, n_win, n_single, col, sval, P,
+        // (a ragged fp32 row is read element-wise at its end, whatever the unit of the row kernels)
+        constexpr bool F32 = L::U::DT == DT_F32;
+        using R = std::conditional_t<L::FULLK, WholeRows<STEPS>,
+                                     RaggedRows<std::conditional_t<F32, UnitF32x4u, typename L::U>, STEPS>>;
+        tile_unit_wave<L::U::DT, STEPS>(R(F32 && L::U::WHOLE ? 4 * KU : KU), A, B, M, N, vrows, tile_cols, tiles, n_tiles, win, n_win, n_single, col, sval, P,
                                         nnz, tile_block * WAVES_PER_BLOCK + wave_in_block(),
                                         win_lds[wave_in_block()], order);
         return;
@@ -1843,13 +1869,14 @@ constexpr int panel_mfma_min_waves(int steps, bool fused, bool half_width = fals
     return fused ? (k <= 32 ? 3 : k == 64 ? 2 : 1) : steps == 8 ? 4 : 1;
 }
 
-template <int DT, int STEPS, bool FUSED = false>
-__global__ __launch_bounds__(panel_mfma_waves(STEPS) * WAVE, panel_mfma_min_waves(STEPS, FUSED, DT != DT_F32)) void k_panel_mfma(const void *__restrict__ A, const void *__restrict__ B,
+template <int DT, int STEPS, bool FUSED = false, class R = WholeRows<STEPS>>
+__global__ __launch_bounds__(panel_mfma_waves(STEPS) * WAVE, panel_mfma_min_waves(STEPS, FUSED, DT != DT_F32)) void k_panel_mfma(const void *__restrict__ A, const void *__restrict__ B, int len,
                                                       const int32_t *__restrict__ rowptr,
                                                       const int32_t *__restrict__ col,
                                                       const float *__restrict__ sval, float *__restrict__ P,
                                                       const RowItem *__restrict__ items, int64_t n_items,
                                                       int64_t nblocks, float *__restrict__ O) {
+    static_assert(!FUSED || !R::RAGGED, "fused panels: whole rows");
     static_assert(!FUSED || (DT == DT_F32 ? (STEPS == 2 || STEPS == 4 || STEPS == 8) : (STEPS == 1 || STEPS == 2 || STEPS == 4)),
                   "fused panels: 32, 64 or 128 components per row");
     __shared__ __attribute__((aligned(16))) float p_tiles[FUSED ? panel_mfma_waves(STEPS) : 1][FUSED ? PANEL_ROWS * PANEL_TILE_PITCH : 4];
@@ -1893,24 +1920,24 @@ __global__ __launch_bounds__(panel_mfma_waves(STEPS) * WAVE, panel_mfma_min_wave
     const int to_memory_from =
         (BLOCKS ? 32 * (prow >> 2) + 16 * (src_unit >> 2) + 4 * (src_unit & 3) + (prow & 3)
                 : 16 * (src_unit & 3) + prow + 8 * (src_unit >> 2)) << 2;
-    constexpr int ROW_UNITS = STEPS * 4;
     // groups of 16 columns in flight; rows of 512 bytes and more leave registers for two
     constexpr int GROUPS = STEPS >= 8 ? 2 : 4;
-    const uint4 *__restrict__ Au = (const uint4 *)A;
-    const uint4 *__restrict__ Bu = (const uint4 *)B;
+    const R rows(len);
     constexpr int A_REGS = BLOCKS ? STEPS / 2 : STEPS;
     uint4 a[A_REGS];
     if constexpr (BLOCKS) {
         // block cg of every k quarter: rows 4(cg&1).. of the units 4(2s'+(cg>>1))+q
         const int cg = (lane >> 2) & 3, t = lane & 3;
-        const uint4 *src = Au + (int64_t)(row0 + 4 * (cg & 1) + t) * ROW_UNITS + 4 * (cg >> 1) + q;
+        const typename R::Row src = rows.row(A, row0 + 4 * (cg & 1) + t);
+        const int u0 = 4 * (cg >> 1) + q;
 #pragma unroll
-        for (int s2 = 0; s2 < A_REGS; ++s2) a[s2] = src[s2 * 8];
+        for (int s2 = 0; s2 < A_REGS; ++s2)
+            a[s2] = rows.trim(rows.unit(A, src, 8 * s2 + u0, 2 * s2 + 1), 8 * s2 + u0, 2 * s2 + 1);
     } else {
         // panel rows: lanes 8..15 of every 16 repeat rows 0..7, their results are not stored
-        const uint4 *src = Au + (int64_t)(row0 + (n & 7)) * ROW_UNITS + q;
+        const typename R::Row src = rows.row(A, row0 + (n & 7));
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) a[s] = src[s * 4];
+        for (int s = 0; s < STEPS; ++s) a[s] = rows.trim(rows.unit(A, src, 4 * s + q, s), 4 * s + q, s);
     }
     const int last = end - 1;
     auto cols_of_chunk = [&](int base) {                        // column of entry base + lane (clamped)
@@ -1923,9 +1950,9 @@ __global__ __launch_bounds__(panel_mfma_waves(STEPS) * WAVE, panel_mfma_min_wave
     auto load_oper = [&](int cc, int u) {                       // group u of the chunk whose columns are in cc
         Oper o;
         const int c = __shfl(cc, u * 16 + lrow, WAVE);
-        const uint4 *src = Bu + (int64_t)c * ROW_UNITS + lunit;
+        const typename R::Row src = rows.row(B, c);
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) o.b[s] = src[s * 4];
+        for (int s = 0; s < STEPS; ++s) o.b[s] = rows.unit(B, src, 4 * s + lunit, s);
         return o;
     };
     // The S values of entries g0+4*(punit-rot) .. +3 of this lane's row: one access for the pair of
@@ -1948,22 +1975,40 @@ __global__ __launch_bounds__(panel_mfma_waves(STEPS) * WAVE, panel_mfma_min_wave
         r.w = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)w_);
         return r;
     };
+    auto b_operand = [&](const Oper &o, int s) {
+        return rows.trim(permute4(to_operand_from, o.b[s].x, o.b[s].y, o.b[s].z, o.b[s].w), 4 * s + q, s);
+    };
     // 4x4 blocks: both row halves of 16 columns, partial over the k quarters
     auto compute_blocks = [&](const Oper &o, f32x4_t &lo, f32x4_t &hi) {
         lo = f32x4_t{0.f, 0.f, 0.f, 0.f};
         hi = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        if constexpr (BLOCKS) {
+        if constexpr (BLOCKS && R::RAGGED) {                     // (added as in mfma_steps)
+            struct Halves {
+                f32x4_t lo, hi;
+                __device__ __forceinline__ Halves operator+(const Halves &x) const { return {lo + x.lo, hi + x.hi}; }
+            };
+            const Halves sum = pairwise<0, STEPS>([&](auto step) {
+                constexpr int s = decltype(step)::value;
+                const uint4 b = b_operand(o, s);
+                Halves r{};
+                mfma_blocks_unit<2 * (s % 2)>(a[s / 2], b, r.lo, r.hi);
+                __builtin_amdgcn_sched_group_barrier(0x080, 4, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+                return r;
+            });
+            lo = sum.lo;
+            hi = sum.hi;
+        } else if constexpr (BLOCKS) {
 #pragma unroll
             for (int s2 = 0; s2 < A_REGS; ++s2) {
                 {
-                    const uint4 b = permute4(to_operand_from, o.b[2 * s2].x, o.b[2 * s2].y, o.b[2 * s2].z, o.b[2 * s2].w);
+                    const uint4 b = b_operand(o, 2 * s2);
                     mfma_blocks_unit<0>(a[s2], b, lo, hi);
                     __builtin_amdgcn_sched_group_barrier(0x080, 4, 0);
                     __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
                 }
                 {
-                    const uint4 b = permute4(to_operand_from, o.b[2 * s2 + 1].x, o.b[2 * s2 + 1].y, o.b[2 * s2 + 1].z,
-                                             o.b[2 * s2 + 1].w);
+                    const uint4 b = b_operand(o, 2 * s2 + 1);
                     mfma_blocks_unit<2>(a[s2], b, lo, hi);
                     __builtin_amdgcn_sched_group_barrier(0x080, 4, 0);
                     __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
@@ -1972,25 +2017,18 @@ __global__ __launch_bounds__(panel_mfma_waves(STEPS) * WAVE, panel_mfma_min_wave
         }
     };
     auto compute = [&](const Oper &o) {
-        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (BLOCKS) return f32x4_t{0.f, 0.f, 0.f, 0.f};
+        else if constexpr (R::RAGGED || DT != DT_F32) {
+            // (the gathered rows are the "row" operand)
+            uint4 b[STEPS];
 #pragma unroll
-        for (int s = 0; s < (BLOCKS ? 0 : STEPS); ++s) {
-            const uint4 b = permute4(to_operand_from, o.b[s].x, o.b[s].y, o.b[s].z, o.b[s].w);
-            if constexpr (DT == DT_BF16) {
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, b),
-                                                              __builtin_bit_cast(bf16x8_t, a[s]), acc, 0, 0, 0);
-            } else if constexpr (DT == DT_F16) {
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, b),
-                                                             __builtin_bit_cast(half8_t, a[s]), acc, 0, 0, 0);
-            } else {
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, b.x),
-                                                           __builtin_bit_cast(float, a[s].x), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, b.y),
-                                                           __builtin_bit_cast(float, a[s].y), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, b.z),
-                                                           __builtin_bit_cast(float, a[s].z), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, b.w),
-                                                           __builtin_bit_cast(float, a[s].w), acc, 0, 0, 0);
+            for (int s = 0; s < STEPS; ++s) b[s] = b_operand(o, s);
+            return mfma_steps<DT, R>(b, [&](int s) { return a[s]; });
+        } else {
+            f32x4_t acc[1] = {};
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s) {
+                mfma_unit<DT, 1>(b_operand(o, s), a[s], acc);
                 // Order of issue: the four permutes of a step, then its four MFMAs.  Left alone the
                 // compiler pairs every MFMA with one permute and a wait for it (16 LDS round trips
                 // per 16 columns in the wave's dependency chain instead of 4); whole groups of 8 or
@@ -1998,8 +2036,8 @@ __global__ __launch_bounds__(panel_mfma_waves(STEPS) * WAVE, panel_mfma_min_wave
                 __builtin_amdgcn_sched_group_barrier(0x080, 4, 0);
                 __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
             }
+            return acc[0];
         }
-        return acc;
     };
     // FUSED: accumulator (h, s, comp) of the output rows, see above
     constexpr int COMPS = DT == DT_F32 ? 4 : 8;                 // components of a 16-byte unit

@@ -78,6 +78,8 @@ bool blocks_pay(const sddmm_ctx *c) {
     if (shape_of(c).LPN == 0 || c->pc.rows_long == 0) return false;
     int64_t segments, gaps;                                         // (a launch takes fewer than 2^32 threads)
     block_items_max(c, true, &segments, &gaps);
+    // (sixteen blocks a row, whatever its length: what a launch refuses does not hang on the lengths)
+    segments = std::max(segments, (int64_t)(c->pc.nnz_long / c->seg + c->pc.rows_long * 16));
     const int waves = block_item_waves(shape_of(c).UPL);
     if (blocks_grid(segments, gaps, waves) * waves * WAVE >= (int64_t)1 << 32) return false;
     if (mode >= 0) return mode != 0;

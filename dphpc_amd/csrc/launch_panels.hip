@@ -1,5 +1,5 @@
 // Launches of the row-panel kernels.
-#include "context.h"
+#include "launch_panels.h"
 
 template <class U, int UPL>
 void launch_panel_t(sddmm_ctx *c, int KU) {
@@ -14,35 +14,31 @@ void launch_panel_u(sddmm_ctx *c, const Shape &s) {
     if (s.UPL == 1) launch_panel_t<U, 1>(c, s.KU);
     else launch_panel_t<U, 2>(c, s.KU);
 }
-template <int DT, int STEPS>
-void launch_panel_mfma_t(sddmm_ctx *c) {
-    constexpr int PW = panel_mfma_waves(STEPS);
-    const int64_t nblocks = (c->n_panel_items + PW - 1) / PW;
-    SDDMM_LAUNCH(c, (k_panel_mfma<DT, STEPS>), xcd_grid(nblocks), PW * WAVE,
-                       (const void *)c->dA, (const void *)c->dB, c->d_rowptr, c->d_col, (const float *)c->d_sval,
-                       c->dP, (const RowItem *)c->d_panel_items, c->n_panel_items, nblocks, (float *)nullptr);
-}
 // the panels of the fused SDDMM+SpMM: P and the panels' part of O
 template <int DT, int STEPS>
 void launch_panel_fused_t(sddmm_ctx *c) {
     constexpr int PW = panel_mfma_waves(STEPS);
     const int64_t nblocks = (c->n_panel_items + PW - 1) / PW;
     SDDMM_LAUNCH(c, (k_panel_mfma<DT, STEPS, true>), xcd_grid(nblocks), PW * WAVE,
-                       (const void *)c->dA, (const void *)c->dB, c->d_rowptr, c->d_col, (const float *)c->d_sval,
+                       (const void *)c->dA, (const void *)c->dB, 0, c->d_rowptr, c->d_col, (const float *)c->d_sval,
                        c->dP, (const RowItem *)c->d_panel_items, c->n_panel_items, nblocks, c->dO);
 }
 template <int DT>
 void launch_panel_mfma_steps(sddmm_ctx *c) {
     switch (panel_mfma_steps(c)) {
-        case 1: launch_panel_mfma_t<DT, 1>(c); break;
-        case 2: launch_panel_mfma_t<DT, 2>(c); break;
-        case 4: launch_panel_mfma_t<DT, 4>(c); break;
-        case 8: launch_panel_mfma_t<DT, 8>(c); break;
-        default: launch_panel_mfma_t<DT, 16>(c); break;
+        case 1: launch_panel_mfma_t<DT, 1, WholeRows<1>>(c, 0); break;
+        case 2: launch_panel_mfma_t<DT, 2, WholeRows<2>>(c, 0); break;
+        case 4: launch_panel_mfma_t<DT, 4, WholeRows<4>>(c, 0); break;
+        case 8: launch_panel_mfma_t<DT, 8, WholeRows<8>>(c, 0); break;
+        default: launch_panel_mfma_t<DT, 16, WholeRows<16>>(c, 0); break;
     }
 }
 
 void launch_panels(sddmm_ctx *c) {
+    if (c->panel_mfma && c->ragged) {
+        launch_ragged_panels(c);
+        return;
+    }
     if (c->panel_mfma) {
         if (c->dtype == SDDMM_BF16) launch_panel_mfma_steps<DT_BF16>(c);
         else if (c->dtype == SDDMM_F16) launch_panel_mfma_steps<DT_F16>(c);
@@ -71,4 +67,6 @@ void launch_panels_fused(sddmm_ctx *c) {
     }
 }
 
-hipError_t load_panels() { return load_code(reinterpret_cast<const void *>(k_panel_mfma<DT_F32, 2>)); }
+hipError_t load_panels(bool ragged) {
+    return ragged ? load_ragged_panels() : load_code(reinterpret_cast<const void *>(k_panel_mfma<DT_F32, 2>));
+}

@@ -1,85 +1,27 @@
-// Launches of the dense-tile kernels, alone and together with the rows.
-#include "context.h"
+// Launches of the dense-tile kernels: rows of whole steps of 64 bytes.
+#include "launch_tiles.h"
 
-// Tiles and rows in one launch (k_auto_tiles); measured faster than two launches at
-// every row size the tile path takes (mixed-density shape: 23 -> 20 us at 128-byte
-// rows, 107 -> 92 us at 1 KiB rows).  Returns false when the layout has no fused
-// kernel; the caller then launches the two kernels in turn.
-bool launch_auto_with_tiles(sddmm_ctx *c) {
-    const Shape s = shape_of(c);
-    if (c->tile_steps < 1 || c->tile_steps > env_int("SDDMM_FUSE_STEPS", 16) || !s.fullk || s.wide || !s.whole() || s.KU != 4 * c->tile_steps)
-        return false;
-    const int64_t waves = short_row_waves(c);
-    const int64_t short_blocks = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    const int64_t item_blocks = (c->n_items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    const int64_t tile_blocks = (c->n_tile_units + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    const int64_t nblocks = short_blocks + item_blocks + tile_blocks;
-    // Order of the blocks on every XCD.  Rows of up to 256 bytes: the tile windows (the wavefronts that
-    // live longest) start first, then the items, then the chunks of the entry list -- measured
-    // 14.7 -> 13.5 us on the mixed-density shape at 128 bytes, 21.3 -> 21.1 us (cold 29.7 -> 27.8) at
-    // 256; at 1 KiB, where the gathers of the short rows are the longer half, the even deal is 3 % faster.
-    const int longest_first = env_int("SDDMM_LONGEST_FIRST", c->tile_steps <= 4 ? 1 : 0);
-    auto eighth = [](int64_t n) { return (n + NUM_XCD - 1) / NUM_XCD; };
-    const int64_t grid = longest_first ? NUM_XCD * (eighth(short_blocks) + eighth(item_blocks) + eighth(tile_blocks))
-                                       : xcd_grid(nblocks);
-    bool launched = false;
-    with_layout(s, [&](auto L) {
-        using LT = decltype(L);
-        constexpr int KU_ = LT::LPN * LT::UPL;
-        if constexpr (!LT::LONG && LT::FULLK && !LT::WIDE && LT::U::ELEMS > 1 && LT::U::WHOLE && (KU_ == 4 || KU_ == 8 || KU_ == 16 || KU_ == 32 || KU_ == 64)) {
-            SDDMM_LAUNCH(c, (k_auto_tiles<LT, KU_ / 4>), grid, BLOCK,
-                               (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr,
-                               (const unsigned char *)(c->owner_active ? c->d_owner : nullptr), c->d_col, c->d_sval,
-                               c->dP, c->sM, c->N, c->ts, c->rpw, short_blocks, c->d_items, c->n_items,
-                               (const int32_t *)c->d_vrows, (const int32_t *)c->d_tile_cols,
-                               (const TileDesc *)c->d_tiles, c->n_tiles,
-                               (const TileWindow *)(c->use_windows ? c->d_windows : nullptr), c->n_windows, c->nnz,
-                               tile_blocks, nblocks, (const int2 *)(c->use_short_list ? c->d_short_list : nullptr),
-                               c->n_short_list, longest_first,
-                               (const int32_t *)(c->use_win_order ? c->d_win_order : nullptr), c->n_win_single);
-            launched = true;
-        }
-    });
-    return launched;
-}
-
-template <int DT, int STEPS>
-void launch_tile_t(sddmm_ctx *c) {
-    // Well-filled tiles (walked from the descriptors' masks) of rows of 256 bytes and more, fewer
-    // windows than keep the chip busy on their own: one workgroup per window, K in four parts.
-    if constexpr (STEPS % KSPLIT == 0) {
-        if (!c->use_windows && c->n_windows <= (int64_t)env_int("SDDMM_KSPLIT_MAX", 32768) && env_int("SDDMM_KSPLIT", 1) != 0) {
-            const int64_t nb = c->n_windows;
-            SDDMM_LAUNCH(c, (k_tile_ksplit<DT, STEPS>), xcd_grid(nb), BLOCK,
-                               (const void *)c->dA, (const void *)c->dB, c->M, c->N, (const int32_t *)c->d_vrows,
-                               (const int32_t *)c->d_tile_cols, (const TileDesc *)c->d_tiles, c->n_tiles,
-                               (const float *)c->d_sval, c->dP, nb,
-                               (const int32_t *)(c->use_win_order ? c->d_win_order : nullptr));
-            return;
-        }
-    }
-    const int64_t nblocks = (c->n_tile_units + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    SDDMM_LAUNCH(c, (k_tile<DT, STEPS>), xcd_grid(nblocks), BLOCK,
-                       (const void *)c->dA, (const void *)c->dB, c->M, c->N, (const int32_t *)c->d_vrows,
-                       (const int32_t *)c->d_tile_cols, (const TileDesc *)c->d_tiles, c->n_tiles,
-                       (const TileWindow *)(c->use_windows ? c->d_windows : nullptr), c->n_windows,
-                       (const int32_t *)c->d_col, (const float *)c->d_sval, c->dP, c->nnz, nblocks,
-                       (const int32_t *)(c->use_win_order ? c->d_win_order : nullptr), c->n_win_single);
-}
 template <int DT>
 void launch_tile_steps(sddmm_ctx *c) {
     switch (c->tile_steps) {
-        case 1: launch_tile_t<DT, 1>(c); break;
-        case 2: launch_tile_t<DT, 2>(c); break;
-        case 4: launch_tile_t<DT, 4>(c); break;
-        case 8: launch_tile_t<DT, 8>(c); break;
-        default: launch_tile_t<DT, 16>(c); break;
+        case 1: launch_tile_t<DT, 1, WholeRows<1>>(c, 0); break;
+        case 2: launch_tile_t<DT, 2, WholeRows<2>>(c, 0); break;
+        case 4: launch_tile_t<DT, 4, WholeRows<4>>(c, 0); break;
+        case 8: launch_tile_t<DT, 8, WholeRows<8>>(c, 0); break;
+        default: launch_tile_t<DT, 16, WholeRows<16>>(c, 0); break;
     }
 }
+
+bool launch_auto_with_tiles(sddmm_ctx *c) {
+    return c->ragged ? launch_ragged_auto_with_tiles(c) : launch_auto_with_tiles_t<false>(c);
+}
 void launch_tiles(sddmm_ctx *c) {
-    if (c->dtype == SDDMM_BF16) launch_tile_steps<DT_BF16>(c);
+    if (c->ragged) launch_ragged_tiles(c);
+    else if (c->dtype == SDDMM_BF16) launch_tile_steps<DT_BF16>(c);
     else if (c->dtype == SDDMM_F16) launch_tile_steps<DT_F16>(c);
     else launch_tile_steps<DT_F32>(c);
 }
 
-hipError_t load_tiles() { return load_code(reinterpret_cast<const void *>(k_tile<DT_F32, 1>)); }
+hipError_t load_tiles(bool ragged) {
+    return ragged ? load_ragged_tiles() : load_code(reinterpret_cast<const void *>(k_tile<DT_F32, 1, WholeRows<1>>));
+}

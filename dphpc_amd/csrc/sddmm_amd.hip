@@ -314,12 +314,19 @@ int begin_ownership(sddmm_ctx *c) {
 bool tile_path_applies(sddmm_ctx *c) {
     c->tile_steps = 0;
     if (c->nnz == 0) return false;
-    const size_t row_bytes = (size_t)c->K * elem_size(c->dtype);
-    if (row_bytes % 64) return false;
-    const int steps = (int)(row_bytes / 64);
-    if (steps != 1 && steps != 2 && steps != 4 && steps != 8 && steps != 16) return false;
-    c->tile_steps = steps;
-    return true;
+    c->tile_steps = c->ragged ? ragged_steps(c) : panel_mfma_steps(c);
+    return c->tile_steps != 0;
+}
+
+// Ragged rows on the tile and panel kernels instead of the gather kernels.  Measured: banded blocks of 2 000 .. 36 000 rows,
+// dense tiles of 100 k .. 2.5 M entries, near-dense rows, K = 9 .. 250 in fp32 and 24 .. 456 in 16 bits: 36 000 banded rows
+// K = 21 69 -> 29 us, K = 100 407 -> 74, K = 120 bf16 137 -> 39; dense tiles K = 100 48.7 -> 14.7, K = 200 bf16 53 -> 10;
+// near-dense rows K = 75 70 -> 36, K = 120 bf16 49 -> 21.  Few entries: a launch of a few microseconds either way, and the
+// plan has more to look at (100 k entries in dense tiles K = 21 4.3 us without, 5.3 with; K = 100 6.8 and 4.6).
+bool ragged_pays(const sddmm_ctx *c) {
+    const int steps = ragged_steps(c), mode = env_int("SDDMM_RAGGED", -1);       // -1: decide here, 0: never, 1: wherever it can
+    if (mode >= 0) return mode != 0 && steps != 0;
+    return steps != 0 && c->nnz >= (steps <= 2 ? 1 << 18 : 1 << 16);
 }
 
 int plan_tiles_count(sddmm_ctx *c, int min_fill) {
@@ -380,7 +387,9 @@ int plan_gathered_count(sddmm_ctx *c, int min_fill, bool *launched) {
     *launched = false;
     if (c->tile_steps == 0 || c->sM < 2) return SDDMM_OK;
     c->n_cand = (int64_t)c->raw.n_candidates;
-    if (c->n_cand < 2) { c->n_cand = 0; return SDDMM_OK; }
+    // ragged rows: fewer tiles than the chip holds wavefronts do not pay (800 of 8 000 rows near-dense, 280 / 120 entries
+    // each: fp32 K = 100 13.6 us without, 15.8 with them / 8.6 and 13.0, bf16 K = 72 9.8 and 7.3 / 6.0 and 7.3)
+    if (c->n_cand < (c->ragged ? 1024 : 2)) { c->n_cand = 0; return SDDMM_OK; }
     int rc;
     // candidates ordered by (first column, row): a few thousand by their ranks in one launch (4 us against 23 us
     // for the radix sort on 3 000 keys), more by the library's radix sort
@@ -524,7 +533,7 @@ int plan_tiles_fill(sddmm_ctx *c) {
     // (their descriptors come last and fill whole windows, an even number of them)
     c->n_win_single = c->n_windows;
     // (rows of up to 256 bytes: beyond that the second A panel and the kept products do not fit the registers)
-    if (c->use_windows && c->n_tiles > gathered_lo && c->tile_steps <= PAIR_MAX_STEPS && env_int("SDDMM_PAIRS", 1) != 0)
+    if (c->use_windows && c->n_tiles > gathered_lo && tile_pairs(c->ragged, c->dtype == SDDMM_F32, c->tile_steps) && env_int("SDDMM_PAIRS", 1) != 0)
         c->n_win_single = gathered_lo / TILE_WINDOW;
     c->n_tile_units = c->n_win_single + (c->n_windows - c->n_win_single + 1) / 2;
     if (!c->use_windows) {
@@ -556,7 +565,7 @@ bool panel_valu_applicable(const sddmm_ctx *c) {
 int plan_panels_flags(sddmm_ctx *c, int min_len, int pseg) {
     c->panels_flagged = false;
     if (c->nnz == 0) return SDDMM_OK;
-    c->panel_mfma = panel_mfma_steps(c) != 0 && env_int("SDDMM_PANEL_MFMA", 1) != 0;
+    c->panel_mfma = (c->ragged || panel_mfma_steps(c) != 0) && env_int("SDDMM_PANEL_MFMA", 1) != 0;
     if (!c->panel_mfma && !panel_valu_applicable(c)) return SDDMM_OK;
     if (c->panel_mfma) min_len = std::max(min_len, 4);   // 16-byte S/P accesses stay inside a row
     const int64_t n_panels = (int64_t)c->sM / 8;
@@ -871,15 +880,23 @@ int do_plan(sddmm_ctx *c, int strategy) {
             // and 512 bytes; 64-byte rows keep the older, conservative figure
             const size_t row_bytes = (size_t)c->K * elem_size(c->dtype);
             const int tile_fill = std::max(1, env_int("SDDMM_TILE_FILL", row_bytes <= 64 ? 96 : row_bytes <= 128 ? 80 : 56));
-            const int pseg = std::max(WAVE, env_int("SDDMM_PANEL_SEG", 512));
-            const bool gathered = resolved == SDDMM_AUTO && env_int("SDDMM_GATHERED", 1) != 0;
+            // panel items of 512 columns, fewer where the panels are too few for the chip (3 072 items if all entries are in
+            // panels: 4 000 banded rows of 158 entries K = 100 18.9 -> 16.2 us, of 8 000 K = 32 9.9 -> 7.6)
+            const int64_t even = (c->nnz / PANEL_ROWS / 3072 + WAVE - 1) / WAVE * WAVE;
+            const int pseg = std::max(WAVE, env_int("SDDMM_PANEL_SEG", (int)std::min<int64_t>(512, even)));
             c->tile_steps = 0;
+            c->ragged = resolved == SDDMM_AUTO && ragged_pays(c);
+            // (ragged fp32 rows of more than twelve steps: a wavefront per SIMD; near-dense rows K = 200 108 us without, 155 with)
+            const bool gathered = resolved == SDDMM_AUTO && env_int("SDDMM_GATHERED", 1) != 0 &&
+                                  !(c->ragged && c->dtype == SDDMM_F32 && ragged_steps(c) > 12);
             // the classifiers are launched back to back; their totals come back together
             if (resolved != SDDMM_LDS_TILED) {
                 // 16-row strips are looked at before the row panels and must not take what the
                 // panel kernel does better (8x8-block rows reach ~80 entries per tile); the
-                // strips gathered after the panels use the measured break-even
-                rc = plan_tiles_count(c, resolved == SDDMM_MFMA_TILE ? 1 : std::max(96, tile_fill));
+                // strips gathered after the panels use the measured break-even.  Ragged rows: banded
+                // blocks in narrow bands reach 140 (4 000 rows, panels / tiles: K = 48 7.6 / 17.2 us, K = 24 bf16 3.9 / 8.1),
+                // and strips that are no panels come back as union strips
+                rc = plan_tiles_count(c, resolved == SDDMM_MFMA_TILE ? 1 : std::max(c->ragged ? 160 : 96, tile_fill));
                 if (rc) return rc;
             }
             if (resolved != SDDMM_MFMA_TILE) {
@@ -989,8 +1006,8 @@ int load_planned(sddmm_ctx *c) {
         case SDDMM_SHORT_ROWS: HIP_TRY(c, load_rows()); break;
         case SDDMM_EXACT: break;                           // (k_exact comes with the plan kernels)
         default:
-            if (c->tiles_active && c->n_tiles > 0) HIP_TRY(c, load_tiles());
-            if (c->n_panel_items > 0) HIP_TRY(c, load_panels());
+            if (c->tiles_active && c->n_tiles > 0) HIP_TRY(c, load_tiles(c->ragged));
+            if (c->n_panel_items > 0) HIP_TRY(c, load_panels(c->ragged));
             if (c->rows_short > 0 || c->n_items > 0) HIP_TRY(c, load_auto());
     }
     return SDDMM_OK;
@@ -1532,7 +1549,7 @@ int sddmm_run_fused(sddmm_ctx *c) {
     }
     if (c->nnz > 0) {
         HIP_TRY(c, load_fused());
-        if (panels) HIP_TRY(c, load_panels());
+        if (panels) HIP_TRY(c, load_panels(false));
     }
     HIP_TRY(c, hipEventRecord(c->ev0, c->stream));
     // (when the panels own every row that has entries, O is complete after a memset and the panel kernel;
