@@ -33,11 +33,9 @@ constexpr int SLICE_ENTRIES = SLICE_CHUNKS * WAVE;
 
 // MISALIGNED: some B row does not start on a line; UNALIGNED: rows are only 4-byte aligned (K % 4 in fp32)
 template <class U, bool MISALIGNED, bool UNALIGNED, bool WIDE>
-__global__ __launch_bounds__(BLOCK, 4) void k_slice_dots(const void *__restrict__ A, const void *__restrict__ B,
-                                                         int row_bytes, const int32_t *__restrict__ rowidx,
-                                                         const int32_t *__restrict__ col, float *__restrict__ part,
-                                                         int64_t nnz, int64_t stride, int64_t blocks_per_slice,
-                                                         int64_t nblocks) {
+__global__ __launch_bounds__(BLOCK, 4) void k_slice_dots(int64_t nblocks, int64_t blocks_per_slice, int64_t nnz,
+    const int32_t *__restrict__ rowidx, const int32_t *__restrict__ col, const void *__restrict__ A,
+    const void *__restrict__ B, int row_bytes, float *__restrict__ part, int64_t stride) {
     static_assert(MISALIGNED || !UNALIGNED, "rows of no whole number of units are misaligned");
     using T = typename U::T;
     using O = typename Off<WIDE>::T;

@@ -134,12 +134,9 @@ static __global__ __launch_bounds__(FUSED_APART_BLOCK) void k_add_cut_rows(const
 // 390 random columns out of 40 000, where the wavefronts in flight walk B together from one end to the other, K = 64
 // 120 / 186, K = 192 fp16 246 / 287, and 30 000 rows of 65 .. 127 entries K = 128 bf16 92 / 102 (fused_in_steps: the rule).
 template <class L, bool STEPS>
-__global__ __launch_bounds__(BLOCK) void k_fusedmm(const void *__restrict__ A, const void *__restrict__ B, int KU,
-                                                   const int32_t *__restrict__ rowptr,
-                                                   const int32_t *__restrict__ col,
-                                                   const float *__restrict__ sval, float *__restrict__ P,
-                                                   float *__restrict__ O, float *__restrict__ parts,
-                                                   const RowItem *__restrict__ items, int64_t n_items, int64_t nblocks) {
+__global__ __launch_bounds__(BLOCK) void k_fusedmm(int64_t nblocks, int64_t n_items, const RowItem *__restrict__ items,
+    const int32_t *__restrict__ col, const float *__restrict__ sval, const void *__restrict__ A, const void *__restrict__ B,
+    int KU, const int32_t *__restrict__ rowptr, float *__restrict__ P, float *__restrict__ O, float *__restrict__ parts) {
     using U = typename L::U;
     using T = typename U::T;                          // 16 bytes: 4 fp32 or 8 bf16 / fp16
     constexpr int E = U::ELEMS;
@@ -356,13 +353,10 @@ __global__ __launch_bounds__(BLOCK) void k_fusedmm(const void *__restrict__ A, c
 // row of zeros, which that kernel, launched after this one, adds to.  Every row below M has
 // its output row written by one or the other, so O needs no clearing before the launches.
 template <class L>
-__global__ __launch_bounds__(BLOCK) void k_fusedmm_rows(const void *__restrict__ A, const void *__restrict__ B, int KU,
-                                                        const int32_t *__restrict__ rowptr,
-                                                        const int32_t *__restrict__ col,
-                                                        const float *__restrict__ sval, float *__restrict__ P,
-                                                        float *__restrict__ O, const float *__restrict__ parts, int M,
-                                                        int max_len, int seg, int64_t nblocks,
-                                                        const unsigned char *__restrict__ panel_owner) {
+__global__ __launch_bounds__(BLOCK) void k_fusedmm_rows(int64_t nblocks, const int32_t *__restrict__ rowptr,
+    const unsigned char *__restrict__ panel_owner, const int32_t *__restrict__ col, const float *__restrict__ sval,
+    const void *__restrict__ A, const void *__restrict__ B, int KU, float *__restrict__ P, float *__restrict__ O,
+    const float *__restrict__ parts, int M, int max_len, int seg) {
     using U = typename L::U;
     using T = typename U::T;
     constexpr int E = U::ELEMS;
@@ -515,13 +509,10 @@ __global__ __launch_bounds__(BLOCK) void k_fusedmm_rows(const void *__restrict__
 // output row is written whenever the row changes.  Rows without entries of their own (empty,
 // left to the panel kernel) get zeros and the pieces of cut rows are added, as in k_fusedmm_rows.
 template <class L>
-__global__ __launch_bounds__(BLOCK) void k_fusedmm_rows_balanced(const void *__restrict__ A, const void *__restrict__ B,
-                                                                 int KU, const int32_t *__restrict__ rowptr,
-                                                                 const int32_t *__restrict__ col,
-                                                                 const float *__restrict__ sval, float *__restrict__ P,
-                                                                 float *__restrict__ O, const float *__restrict__ parts,
-                                                                 int M, int max_len, int seg, int64_t nblocks,
-                                                                 const unsigned char *__restrict__ panel_owner) {
+__global__ __launch_bounds__(BLOCK) void k_fusedmm_rows_balanced(int64_t nblocks, const int32_t *__restrict__ rowptr,
+    const unsigned char *__restrict__ panel_owner, const int32_t *__restrict__ col, const float *__restrict__ sval,
+    const void *__restrict__ A, const void *__restrict__ B, int KU, float *__restrict__ P, float *__restrict__ O,
+    const float *__restrict__ parts, int M, int max_len, int seg) {
     using U = typename L::U;
     using T = typename U::T;
     constexpr int E = U::ELEMS;

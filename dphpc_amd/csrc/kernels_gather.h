@@ -1,5 +1,7 @@
 // Gather kernels: every stored entry (i,j) of S reads row i of A and row j of B.
 //
+// Arguments of the kernels: what a wavefront needs for its first loads comes first (the first 14 words are preloaded).
+//
 // Lane layout (all kernels below).  A wavefront works on a "chunk" of up to 64
 // consecutive stored entries.  Lane l loads the column index / S value of entry
 // l of the chunk and finally stores its P value: plain coalesced 64-wide
@@ -253,12 +255,9 @@ __device__ __forceinline__ void flat_body(const void *__restrict__ A, const void
 }
 
 template <class L>
-__global__ __launch_bounds__(BLOCK) void k_flat(const void *__restrict__ A, const void *__restrict__ B, int KU,
-                                                const int32_t *__restrict__ rowidx,
-                                                const int32_t *__restrict__ col,
-                                                const float *__restrict__ sval,
-                                                float *__restrict__ P, int64_t nnz,
-                                                int chunks_per_wave, int64_t nblocks) {
+__global__ __launch_bounds__(BLOCK) void k_flat(int64_t nblocks, int64_t nnz, int chunks_per_wave, int KU,
+    const int32_t *__restrict__ rowidx, const int32_t *__restrict__ col, const void *__restrict__ A,
+    const void *__restrict__ B, const float *__restrict__ sval, float *__restrict__ P) {
     const int64_t blk = xcd_remap(blockIdx.x, nblocks);
     if (blk < 0) return;
     const int64_t base = (blk * WAVES_PER_BLOCK + wave_in_block()) * (int64_t)chunks_per_wave * WAVE;
@@ -445,13 +444,11 @@ __device__ __forceinline__ void entry_list_body(const void *__restrict__ A, cons
 // totals[0], totals[1]: work items of either kind (the grid is sized for an upper bound)
 //
 template <class L, bool SCALED>
-__global__ __launch_bounds__(block_item_waves(L::UPL) * WAVE) void k_flat_blocks(const void *__restrict__ A, const void *__restrict__ B, int KU,
-                                                       const int32_t *__restrict__ rowidx,
-                                                       const int32_t *__restrict__ col,
-                                                       const float *__restrict__ sval, float *__restrict__ P,
-                                                       const RowItem *__restrict__ segments,
-                                                       const RowItem *__restrict__ gaps,
-                                                       const unsigned long long *__restrict__ totals) {
+__global__ __launch_bounds__(block_item_waves(L::UPL) * WAVE)
+void k_flat_blocks(const unsigned long long *__restrict__ totals, const RowItem *__restrict__ segments,
+                   const RowItem *__restrict__ gaps, const int32_t *__restrict__ col, const float *__restrict__ sval,
+                   const void *__restrict__ A, const void *__restrict__ B, int KU, const int32_t *__restrict__ rowidx,
+                   float *__restrict__ P) {
     constexpr int WAVES = block_item_waves(L::UPL);
     const int64_t n_seg = (int64_t)totals[0], n_gap = (int64_t)totals[1];
     const int64_t sb = (n_seg + WAVES - 1) / WAVES, gb = (n_gap + WAVES - 1) / WAVES;
@@ -477,13 +474,9 @@ __global__ __launch_bounds__(block_item_waves(L::UPL) * WAVE) void k_flat_blocks
 // ROW_WAVE: one wavefront per work item.  With items == nullptr item w is the
 // whole row w.
 template <class L>
-__global__ __launch_bounds__(BLOCK) void k_row_wave(const void *__restrict__ A, const void *__restrict__ B,
-                                                    int KU, const int32_t *__restrict__ rowptr,
-                                                    const int32_t *__restrict__ col,
-                                                    const float *__restrict__ sval,
-                                                    float *__restrict__ P,
-                                                    const RowItem *__restrict__ items,
-                                                    int64_t n_items, int64_t nblocks) {
+__global__ __launch_bounds__(BLOCK) void k_row_wave(int64_t nblocks, int64_t n_items, const RowItem *__restrict__ items,
+    const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, const void *__restrict__ A,
+    const void *__restrict__ B, int KU, const float *__restrict__ sval, float *__restrict__ P) {
     const int64_t blk = xcd_remap(blockIdx.x, nblocks);
     if (blk < 0) return;
     const int64_t w = blk * WAVES_PER_BLOCK + wave_in_block();
@@ -524,15 +517,10 @@ __global__ __launch_bounds__(BLOCK) void k_short_rows(const void *__restrict__ A
 // blocks after them run one segment item per wavefront.  The item blocks come
 // last in the XCD-contiguous order, after the short-row work of the same XCD.
 template <class L>
-__global__ __launch_bounds__(BLOCK) void k_auto(const void *__restrict__ A, const void *__restrict__ B, int KU,
-                                                const int32_t *__restrict__ rowptr,
-                                                const unsigned char *__restrict__ owner,
-                                                const int32_t *__restrict__ col,
-                                                const float *__restrict__ sval, float *__restrict__ P, int M,
-                                                int ts, int rpw, int64_t short_blocks,
-                                                const RowItem *__restrict__ items, int64_t n_items,
-                                                int64_t nblocks, const int2 *__restrict__ short_list,
-                                                int64_t n_short_list) {
+__global__ __launch_bounds__(BLOCK) void k_auto(int64_t nblocks, int64_t short_blocks, const RowItem *__restrict__ items,
+    int64_t n_items, const int2 *__restrict__ short_list, const void *__restrict__ A, const void *__restrict__ B, int KU,
+    const int32_t *__restrict__ rowptr, const unsigned char *__restrict__ owner, const int32_t *__restrict__ col,
+    const float *__restrict__ sval, float *__restrict__ P, int M, int ts, int rpw, int64_t n_short_list) {
     const int64_t blk = xcd_remap(blockIdx.x, nblocks);
     if (blk < 0) return;
     // interleave: the item blocks of a long-row-heavy matrix start early instead

@@ -1465,14 +1465,11 @@ __device__ __forceinline__ void tile_unit_wave(const R &rows, const void *__rest
 }
 
 template <int DT, int STEPS, class R>
-__global__ __launch_bounds__(BLOCK) void k_tile(const void *__restrict__ A, const void *__restrict__ B, int len, int M, int N,
-                                                const int32_t *__restrict__ vrows,
-                                                const int32_t *__restrict__ tile_cols,
-                                                const TileDesc *__restrict__ tiles, int64_t n_tiles,
-                                                const TileWindow *__restrict__ win, int64_t n_win,
-                                                const int32_t *__restrict__ col, const float *__restrict__ sval,
-                                                float *__restrict__ P, int64_t nnz, int64_t nblocks,
-                                                const int32_t *__restrict__ order, int64_t n_single) {
+__global__ __launch_bounds__(BLOCK) void k_tile(int64_t nblocks, const TileWindow *__restrict__ win, int64_t n_win,
+    int64_t n_single, const int32_t *__restrict__ order, const void *__restrict__ A, const void *__restrict__ B, int len,
+    int M, int N, const int32_t *__restrict__ vrows, const int32_t *__restrict__ tile_cols,
+    const TileDesc *__restrict__ tiles, int64_t n_tiles, const int32_t *__restrict__ col, const float *__restrict__ sval,
+    float *__restrict__ P, int64_t nnz) {
     __shared__ __attribute__((aligned(16))) float win_lds[WAVES_PER_BLOCK][WIN_LDS_FLOATS];
     const int64_t blk = xcd_remap(blockIdx.x, nblocks);
     if (blk < 0) return;
@@ -1493,12 +1490,10 @@ static_assert(KSPLIT == 4 && TILE_WINDOW == 4, "one finishing wave per tile of a
 constexpr int KSPLIT_LDS_FLOATS = TILE_WINDOW * KSPLIT * 256;
 
 template <int DT, int STEPS, class R>
-__global__ __launch_bounds__(BLOCK) void k_tile_ksplit(const void *__restrict__ A, const void *__restrict__ B, int len, int M, int N,
-                                                       const int32_t *__restrict__ vrows,
-                                                       const int32_t *__restrict__ tile_cols,
-                                                       const TileDesc *__restrict__ tiles, int64_t n_tiles,
-                                                       const float *__restrict__ sval, float *__restrict__ P,
-                                                       int64_t nblocks, const int32_t *__restrict__ order) {
+__global__ __launch_bounds__(BLOCK) void k_tile_ksplit(int64_t nblocks, const int32_t *__restrict__ order,
+    const TileDesc *__restrict__ tiles, int64_t n_tiles, const int32_t *__restrict__ tile_cols, const void *__restrict__ A,
+    const void *__restrict__ B, int len, int M, int N, const int32_t *__restrict__ vrows, const float *__restrict__ sval,
+    float *__restrict__ P) {
     static_assert(STEPS % KSPLIT == 0, "K in four equal parts of whole 64-byte steps");
     constexpr int SW = STEPS / KSPLIT;                    // steps of this wave
     __shared__ __attribute__((aligned(16))) float part[KSPLIT_LDS_FLOATS];
@@ -1514,7 +1509,10 @@ __global__ __launch_bounds__(BLOCK) void k_tile_ksplit(const void *__restrict__ 
     const int lrow = lane >> 2, lunit = lane & 3;    // memory layout: four neighbouring lanes on 64 bytes of a row
     const int to_operand_from = (4 * r16 + q) << 2;
     const R rows(len);
-    const int u0 = j * SW * 4;                            // this wave's quarter of every row
+    const int quarter = j * SW * 4;                       // this wave's quarter of every row: whole rows have it in the base
+    const void *Aq = R::RAGGED ? A : (const void *)((const uint4 *)A + (uint32_t)quarter);
+    const void *Bq = R::RAGGED ? B : (const void *)((const uint4 *)B + (uint32_t)quarter);
+    const int u0 = R::RAGGED ? quarter : 0;
     auto to_operand = [&](const uint4 &v, int s) {
         uint4 r;
         r.x = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.x);
@@ -1542,22 +1540,22 @@ __global__ __launch_bounds__(BLOCK) void k_tile_ksplit(const void *__restrict__ 
         int64_t arow = st >= GATHERED_BASE ? (int64_t)vrows[(int64_t)(st - GATHERED_BASE) * 16 + lrow]
                                            : (int64_t)st * 16 + lrow;
         arow = arow < 0 ? 0 : (arow < M ? arow : M - 1);      // missing rows are never in a mask
-        return rows.row(A, arow);
+        return rows.row(Aq, arow);
     };
     // second round trip: this wave's quarter of the A panel and of all B tiles, the S values of its own tile
     uint4 a[SW], b[TILE_WINDOW][SW];
     {
         const typename R::Row src = a_rows(strip[0]);
 #pragma unroll
-        for (int s = 0; s < SW; ++s) a[s] = rows.unit(A, src, u0 + 4 * s + lunit, STEPS);
+        for (int s = 0; s < SW; ++s) a[s] = rows.unit(Aq, src, u0 + 4 * s + lunit, STEPS);
     }
 #pragma unroll
     for (int k = 0; k < TILE_WINDOW; ++k) {
         int64_t brow = bcol[k];
         brow = brow < N ? brow : N - 1;                   // columns past N (and the filler of a short union tile) are in no mask
-        const typename R::Row src = rows.row(B, brow);
+        const typename R::Row src = rows.row(Bq, brow);
 #pragma unroll
-        for (int s = 0; s < SW; ++s) b[k][s] = rows.unit(B, src, u0 + 4 * s + lunit, STEPS);
+        for (int s = 0; s < SW; ++s) b[k][s] = rows.unit(Bq, src, u0 + 4 * s + lunit, STEPS);
     }
     const unsigned int below = (1u << r16) - 1u;
     const int offs[4] = {off4.x, off4.y, off4.z, off4.w};
@@ -1580,7 +1578,7 @@ __global__ __launch_bounds__(BLOCK) void k_tile_ksplit(const void *__restrict__ 
         if (k > 0 && strip[k] != strip[k - 1]) {          // workgroup-uniform: the window reaches into the next strip
             const typename R::Row src = a_rows(strip[k]);
 #pragma unroll
-            for (int s = 0; s < SW; ++s) a[s] = to_operand(rows.unit(A, src, u0 + 4 * s + lunit, STEPS), s);
+            for (int s = 0; s < SW; ++s) a[s] = to_operand(rows.unit(Aq, src, u0 + 4 * s + lunit, STEPS), s);
         }
         *reinterpret_cast<f32x4_t *>(part + (k * KSPLIT + j) * 256 + lane * 4) =
             mfma_steps<DT, R>(a, [&](int s) { return to_operand(b[k][s], s); });
@@ -1654,33 +1652,28 @@ static __global__ __launch_bounds__(256) void k_window_scatter(const TileDesc *_
 #define SDDMM_FUSED_WAVES 5
 #endif
 template <class L, int STEPS>
-__global__ __launch_bounds__(BLOCK, STEPS <= 2 ? SDDMM_FUSED_WAVES : STEPS == 4 ? 4 : 1) void k_auto_tiles(const void *__restrict__ A, const void *__restrict__ B, int KU,
-                                                      const int32_t *__restrict__ rowptr,
-                                                      const unsigned char *__restrict__ owner,
-                                                      const int32_t *__restrict__ col,
-                                                      const float *__restrict__ sval, float *__restrict__ P, int M,
-                                                      int N, int ts, int rpw, int64_t short_blocks,
-                                                      const RowItem *__restrict__ items, int64_t n_items,
-                                                      const int32_t *__restrict__ vrows,
-                                                      const int32_t *__restrict__ tile_cols,
-                                                      const TileDesc *__restrict__ tiles, int64_t n_tiles,
-                                                      const TileWindow *__restrict__ win, int64_t n_win, int64_t nnz,
-                                                      int64_t tile_blocks, int64_t nblocks,
-                                                      const int2 *__restrict__ short_list, int64_t n_short_list,
-                                                      int longest_first, const int32_t *__restrict__ order,
-                                                      int64_t n_single) {
+__global__ __launch_bounds__(BLOCK, STEPS <= 2 ? SDDMM_FUSED_WAVES : STEPS == 4 ? 4 : 1)
+void k_auto_tiles(int tile_blocks, int nblocks, int short_blocks, int longest_first, int n_win, int n_single,
+                  const TileWindow *__restrict__ win, const int2 *__restrict__ short_list, const void *__restrict__ A,
+                  const void *__restrict__ B, const int32_t *__restrict__ col, const float *__restrict__ sval,
+                  float *__restrict__ P, int64_t nnz, int M, int N, int KU, int ts, int rpw,
+                  const int32_t *__restrict__ rowptr, const unsigned char *__restrict__ owner,
+                  const RowItem *__restrict__ items, int64_t n_items, const int32_t *__restrict__ vrows,
+                  const int32_t *__restrict__ tile_cols, const TileDesc *__restrict__ tiles, int64_t n_tiles,
+                  int64_t n_short_list, const int32_t *__restrict__ order) {
     __shared__ __attribute__((aligned(16))) float win_lds[WAVES_PER_BLOCK][WIN_LDS_FLOATS];
     int64_t tile_block = -1, item_block = -1, short_block = -1;
     if (longest_first) {
         // Workgroups start in the order of their ids, round-robin over the XCDs: on every XCD the
         // tile windows first (the longest wavefronts), then the segment items, then the chunks of
         // the entry list, each XCD with its contiguous eighth of each kind.
+        // (a launch has fewer than 2^24 workgroups: eight times that is an int)
         const int x = (int)(blockIdx.x % NUM_XCD);
-        int64_t j = blockIdx.x / NUM_XCD;
-        const int64_t item_blocks = nblocks - tile_blocks - short_blocks;
-        const int64_t t_lo = x * tile_blocks / NUM_XCD, t_n = (x + 1) * tile_blocks / NUM_XCD - t_lo;
-        const int64_t i_lo = x * item_blocks / NUM_XCD, i_n = (x + 1) * item_blocks / NUM_XCD - i_lo;
-        const int64_t s_lo = x * short_blocks / NUM_XCD, s_n = (x + 1) * short_blocks / NUM_XCD - s_lo;
+        int j = (int)(blockIdx.x / NUM_XCD);
+        const int item_blocks = nblocks - tile_blocks - short_blocks;
+        const int t_lo = x * tile_blocks / NUM_XCD, t_n = (x + 1) * tile_blocks / NUM_XCD - t_lo;
+        const int i_lo = x * item_blocks / NUM_XCD, i_n = (x + 1) * item_blocks / NUM_XCD - i_lo;
+        const int s_lo = x * short_blocks / NUM_XCD, s_n = (x + 1) * short_blocks / NUM_XCD - s_lo;
         if (j < t_n) tile_block = t_lo + j;
         else if ((j -= t_n) < i_n) item_block = i_lo + j;
         else if ((j -= i_n) < s_n) short_block = s_lo + j;
@@ -1870,12 +1863,10 @@ constexpr int panel_mfma_min_waves(int steps, bool fused, bool half_width = fals
 }
 
 template <int DT, int STEPS, bool FUSED = false, class R = WholeRows<STEPS>>
-__global__ __launch_bounds__(panel_mfma_waves(STEPS) * WAVE, panel_mfma_min_waves(STEPS, FUSED, DT != DT_F32)) void k_panel_mfma(const void *__restrict__ A, const void *__restrict__ B, int len,
-                                                      const int32_t *__restrict__ rowptr,
-                                                      const int32_t *__restrict__ col,
-                                                      const float *__restrict__ sval, float *__restrict__ P,
-                                                      const RowItem *__restrict__ items, int64_t n_items,
-                                                      int64_t nblocks, float *__restrict__ O) {
+__global__ __launch_bounds__(panel_mfma_waves(STEPS) * WAVE, panel_mfma_min_waves(STEPS, FUSED, DT != DT_F32))
+void k_panel_mfma(const RowItem *__restrict__ items, int64_t n_items, int64_t nblocks, const int32_t *__restrict__ rowptr,
+                  const int32_t *__restrict__ col, const void *__restrict__ A, const void *__restrict__ B, int len,
+                  const float *__restrict__ sval, float *__restrict__ P, float *__restrict__ O) {
     static_assert(!FUSED || !R::RAGGED, "fused panels: whole rows");
     static_assert(!FUSED || (DT == DT_F32 ? (STEPS == 2 || STEPS == 4 || STEPS == 8) : (STEPS == 1 || STEPS == 2 || STEPS == 4)),
                   "fused panels: 32, 64 or 128 components per row");

@@ -9,11 +9,10 @@ void launch_auto(sddmm_ctx *c) {
     const int64_t nblocks = short_blocks + item_blocks;
     with_layout(s, [&](auto L) {
         using LT = decltype(L);
-        SDDMM_LAUNCH(c, (k_auto<LT>), xcd_grid(nblocks), BLOCK,
-                           (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr,
-                           (const unsigned char *)(c->owner_active ? c->d_owner : nullptr), c->d_col, c->d_sval,
-                           c->dP, c->sM, c->ts, c->rpw, short_blocks, c->d_items, c->n_items, nblocks,
-                           (const int2 *)(c->use_short_list ? c->d_short_list : nullptr), c->n_short_list);
+        SDDMM_LAUNCH(c, (k_auto<LT>), xcd_grid(nblocks), BLOCK, nblocks, short_blocks, c->d_items, c->n_items,
+                     (const int2 *)(c->use_short_list ? c->d_short_list : nullptr), (const void *)c->dA, (const void *)c->dB,
+                     s.len, c->d_rowptr, (const unsigned char *)(c->owner_active ? c->d_owner : nullptr), c->d_col, c->d_sval,
+                     c->dP, c->sM, c->ts, c->rpw, c->n_short_list);
     });
 }
 

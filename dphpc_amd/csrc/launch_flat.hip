@@ -10,9 +10,8 @@ void launch_flat(sddmm_ctx *c) {
     const int64_t nblocks = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
     with_layout(s, [&](auto L) {
         using LT = decltype(L);
-        SDDMM_LAUNCH(c, (k_flat<LT>), xcd_grid(nblocks), BLOCK,
-                           (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowidx, c->d_col, c->d_sval, c->dP,
-                           c->nnz, cpw, nblocks);
+        SDDMM_LAUNCH(c, (k_flat<LT>), xcd_grid(nblocks), BLOCK, nblocks, c->nnz, cpw, s.len, c->d_rowidx, c->d_col,
+                     (const void *)c->dA, (const void *)c->dB, c->d_sval, c->dP);
     });
 }
 
@@ -52,9 +51,9 @@ int launch_flat_blocks(sddmm_ctx *c) {
         using LT = decltype(L);
         if constexpr (!LT::LONG) {
             auto launch = [&](auto kernel, float *out) {
-                SDDMM_LAUNCH(c, kernel, grid, waves * WAVE, (const void *)c->dA, (const void *)c->dB, s.len, entry_rows(c),
-                             entry_cols(c), (const float *)c->d_sval, out, (const RowItem *)c->d_block_segments,
-                             (const RowItem *)c->d_block_gaps, (const unsigned long long *)c->d_pc->block_items);
+                SDDMM_LAUNCH(c, kernel, grid, waves * WAVE, (const unsigned long long *)c->d_pc->block_items,
+                             (const RowItem *)c->d_block_segments, (const RowItem *)c->d_block_gaps, entry_cols(c),
+                             (const float *)c->d_sval, (const void *)c->dA, (const void *)c->dB, s.len, entry_rows(c), out);
                 ++launches;
             };
             if (c->use_order) launch(k_flat_blocks<LT, false>, c->d_order_dots);
@@ -125,9 +124,9 @@ int launch_slices_t(sddmm_ctx *c, int slices) {
         const int64_t stride = (n + WAVE - 1) / WAVE * WAVE;
         const int64_t waves = (n + SLICE_ENTRIES - 1) / SLICE_ENTRIES;
         const int64_t per_slice = (waves + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK, nblocks = per_slice * slices;
-        SDDMM_LAUNCH(c, (k_slice_dots<U, MISALIGNED, UNALIGNED, WIDE>), xcd_grid(nblocks), BLOCK, (const void *)c->dA,
-                     (const void *)c->dB, row_bytes, entry_rows(c) + e0, entry_cols(c) + e0,
-                     c->d_part, n, stride, per_slice, nblocks);
+        SDDMM_LAUNCH(c, (k_slice_dots<U, MISALIGNED, UNALIGNED, WIDE>), xcd_grid(nblocks), BLOCK, nblocks, per_slice, n,
+                     entry_rows(c) + e0, entry_cols(c) + e0, (const void *)c->dA, (const void *)c->dB, row_bytes, c->d_part,
+                     stride);
         SDDMM_LAUNCH(c, k_slice_sum, (n + 4 * BLOCK - 1) / (4 * BLOCK), BLOCK, (const float *)c->d_part, slices, stride,
                      (const float *)(c->use_order ? nullptr : c->d_sval + e0),
                      c->use_order ? c->d_order_dots + e0 : c->dP + e0, n);

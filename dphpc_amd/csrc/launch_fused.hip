@@ -43,10 +43,9 @@ int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
             if (c->n_fused_items > 0) {
                 const int64_t nblocks = blocks_of(c->n_fused_items, c->fused_block_waves);
                 auto launch = [&](auto kernel) {
-                    SDDMM_LAUNCH(c, kernel, xcd_grid(nblocks), c->fused_block_waves * WAVE,
-                                       (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col,
-                                       c->d_sval, c->dP, c->dO, c->d_fused_parts, (const RowItem *)c->d_fused_items,
-                                       c->n_fused_items, nblocks);
+                    SDDMM_LAUNCH(c, kernel, xcd_grid(nblocks), c->fused_block_waves * WAVE, nblocks, c->n_fused_items,
+                                 (const RowItem *)c->d_fused_items, c->d_col, c->d_sval, (const void *)c->dA,
+                                 (const void *)c->dB, s.len, c->d_rowptr, c->dP, c->dO, c->d_fused_parts);
                 };
                 if constexpr (LT::UPL == 1) launch(k_fusedmm<LT, false>);
                 else if (fused_in_steps<LT>(c)) launch(k_fusedmm<LT, true>);
@@ -62,15 +61,13 @@ int launch_fused_rows(sddmm_ctx *c, const unsigned char *panel_owner) {
             if (balanced) {
                 const int64_t bwaves = ((int64_t)c->sM + WAVE - 1) / WAVE;
                 const int64_t bblocks = blocks_of(bwaves, c->fused_block_waves);
-                SDDMM_LAUNCH(c, (k_fusedmm_rows_balanced<LT>), xcd_grid(bblocks), c->fused_block_waves * WAVE,
-                                   (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col, c->d_sval,
-                                   c->dP, c->dO, (const float *)c->d_fused_parts, c->sM, c->fused_row_max,
-                                   seg, bblocks, panel_owner);
+                SDDMM_LAUNCH(c, (k_fusedmm_rows_balanced<LT>), xcd_grid(bblocks), c->fused_block_waves * WAVE, bblocks,
+                             c->d_rowptr, panel_owner, c->d_col, c->d_sval, (const void *)c->dA, (const void *)c->dB, s.len,
+                             c->dP, c->dO, (const float *)c->d_fused_parts, c->sM, c->fused_row_max, seg);
             } else {
-                SDDMM_LAUNCH(c, (k_fusedmm_rows<LT>), xcd_grid(rblocks), c->fused_block_waves * WAVE,
-                                   (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col, c->d_sval,
-                                   c->dP, c->dO, (const float *)c->d_fused_parts, c->sM, c->fused_row_max,
-                                   seg, rblocks, panel_owner);
+                SDDMM_LAUNCH(c, (k_fusedmm_rows<LT>), xcd_grid(rblocks), c->fused_block_waves * WAVE, rblocks, c->d_rowptr,
+                             panel_owner, c->d_col, c->d_sval, (const void *)c->dA, (const void *)c->dB, s.len, c->dP, c->dO,
+                             (const float *)c->d_fused_parts, c->sM, c->fused_row_max, seg);
             }
             ++launches;
         }

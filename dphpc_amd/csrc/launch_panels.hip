@@ -20,8 +20,8 @@ void launch_panel_fused_t(sddmm_ctx *c) {
     constexpr int PW = panel_mfma_waves(STEPS);
     const int64_t nblocks = (c->n_panel_items + PW - 1) / PW;
     SDDMM_LAUNCH(c, (k_panel_mfma<DT, STEPS, true>), xcd_grid(nblocks), PW * WAVE,
-                       (const void *)c->dA, (const void *)c->dB, 0, c->d_rowptr, c->d_col, (const float *)c->d_sval,
-                       c->dP, (const RowItem *)c->d_panel_items, c->n_panel_items, nblocks, c->dO);
+                 (const RowItem *)c->d_panel_items, c->n_panel_items, nblocks, c->d_rowptr, c->d_col, (const void *)c->dA,
+                 (const void *)c->dB, 0, (const float *)c->d_sval, c->dP, c->dO);
 }
 template <int DT>
 void launch_panel_mfma_steps(sddmm_ctx *c) {

@@ -6,9 +6,8 @@ void launch_row_wave(sddmm_ctx *c, const RowItem *items, int64_t n_items) {
     const int64_t nblocks = (n_items + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
     with_layout(s, [&](auto L) {
         using LT = decltype(L);
-        SDDMM_LAUNCH(c, (k_row_wave<LT>), xcd_grid(nblocks), BLOCK,
-                           (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr, c->d_col, c->d_sval, c->dP,
-                           items, n_items, nblocks);
+        SDDMM_LAUNCH(c, (k_row_wave<LT>), xcd_grid(nblocks), BLOCK, nblocks, n_items, items, c->d_rowptr, c->d_col,
+                     (const void *)c->dA, (const void *)c->dB, s.len, c->d_sval, c->dP);
     });
 }
 

@@ -31,16 +31,14 @@ bool launch_auto_with_tiles_t(sddmm_ctx *c) {
         constexpr int KU_ = LT::LPN * LT::UPL;
         if constexpr (!LT::LONG && LT::FULLK != RAGGED && !LT::WIDE && LT::U::ELEMS > 1 && (LT::LPN == 4 || LT::LPN == 8) &&
                       (RAGGED || (LT::U::WHOLE && LT::UPL != 3 && LT::UPL != 6))) {
-            SDDMM_LAUNCH(c, (k_auto_tiles<LT, KU_ / 4>), grid, BLOCK,
-                               (const void *)c->dA, (const void *)c->dB, s.len, c->d_rowptr,
-                               (const unsigned char *)(c->owner_active ? c->d_owner : nullptr), c->d_col, c->d_sval,
-                               c->dP, c->sM, c->N, c->ts, c->rpw, short_blocks, c->d_items, c->n_items,
-                               (const int32_t *)c->d_vrows, (const int32_t *)c->d_tile_cols,
-                               (const TileDesc *)c->d_tiles, c->n_tiles,
-                               (const TileWindow *)(c->use_windows ? c->d_windows : nullptr), c->n_windows, c->nnz,
-                               tile_blocks, nblocks, (const int2 *)(c->use_short_list ? c->d_short_list : nullptr),
-                               c->n_short_list, longest_first,
-                               (const int32_t *)(c->use_win_order ? c->d_win_order : nullptr), c->n_win_single);
+            SDDMM_LAUNCH(c, (k_auto_tiles<LT, KU_ / 4>), grid, BLOCK, (int)tile_blocks, (int)nblocks, (int)short_blocks,
+                         longest_first, (int)c->n_windows, (int)c->n_win_single,
+                         (const TileWindow *)(c->use_windows ? c->d_windows : nullptr),
+                         (const int2 *)(c->use_short_list ? c->d_short_list : nullptr), (const void *)c->dA,
+                         (const void *)c->dB, c->d_col, c->d_sval, c->dP, c->nnz, c->sM, c->N, s.len, c->ts, c->rpw,
+                         c->d_rowptr, (const unsigned char *)(c->owner_active ? c->d_owner : nullptr), c->d_items, c->n_items,
+                         (const int32_t *)c->d_vrows, (const int32_t *)c->d_tile_cols, (const TileDesc *)c->d_tiles,
+                         c->n_tiles, c->n_short_list, (const int32_t *)(c->use_win_order ? c->d_win_order : nullptr));
             launched = true;
         }
     });
@@ -55,19 +53,17 @@ void launch_tile_t(sddmm_ctx *c, int len) {
     if constexpr (KSTEPS % KSPLIT == 0) {
         if (!c->use_windows && c->n_windows <= (int64_t)env_int("SDDMM_KSPLIT_MAX", 32768) && env_int("SDDMM_KSPLIT", 1) != 0) {
             const int64_t nb = c->n_windows;
-            SDDMM_LAUNCH(c, (k_tile_ksplit<DT, KSTEPS, KR>), xcd_grid(nb), BLOCK,
-                               (const void *)c->dA, (const void *)c->dB, len, c->M, c->N, (const int32_t *)c->d_vrows,
-                               (const int32_t *)c->d_tile_cols, (const TileDesc *)c->d_tiles, c->n_tiles,
-                               (const float *)c->d_sval, c->dP, nb,
-                               (const int32_t *)(c->use_win_order ? c->d_win_order : nullptr));
+            SDDMM_LAUNCH(c, (k_tile_ksplit<DT, KSTEPS, KR>), xcd_grid(nb), BLOCK, nb,
+                         (const int32_t *)(c->use_win_order ? c->d_win_order : nullptr), (const TileDesc *)c->d_tiles,
+                         c->n_tiles, (const int32_t *)c->d_tile_cols, (const void *)c->dA, (const void *)c->dB, len, c->M,
+                         c->N, (const int32_t *)c->d_vrows, (const float *)c->d_sval, c->dP);
             return;
         }
     }
     const int64_t nblocks = (c->n_tile_units + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK;
-    SDDMM_LAUNCH(c, (k_tile<DT, STEPS, R>), xcd_grid(nblocks), BLOCK,
-                       (const void *)c->dA, (const void *)c->dB, len, c->M, c->N, (const int32_t *)c->d_vrows,
-                       (const int32_t *)c->d_tile_cols, (const TileDesc *)c->d_tiles, c->n_tiles,
-                       (const TileWindow *)(c->use_windows ? c->d_windows : nullptr), c->n_windows,
-                       (const int32_t *)c->d_col, (const float *)c->d_sval, c->dP, c->nnz, nblocks,
-                       (const int32_t *)(c->use_win_order ? c->d_win_order : nullptr), c->n_win_single);
+    SDDMM_LAUNCH(c, (k_tile<DT, STEPS, R>), xcd_grid(nblocks), BLOCK, nblocks,
+                 (const TileWindow *)(c->use_windows ? c->d_windows : nullptr), c->n_windows, c->n_win_single,
+                 (const int32_t *)(c->use_win_order ? c->d_win_order : nullptr), (const void *)c->dA, (const void *)c->dB,
+                 len, c->M, c->N, (const int32_t *)c->d_vrows, (const int32_t *)c->d_tile_cols, (const TileDesc *)c->d_tiles,
+                 c->n_tiles, (const int32_t *)c->d_col, (const float *)c->d_sval, c->dP, c->nnz);
 }
