@@ -61,8 +61,9 @@ struct sddmm_ctx {
     int ts = 0, seg = 0, rpw = 64;
     RowItem *d_items = nullptr;
     int64_t n_items = 0, items_cap = 0;
-    unsigned int *d_block_sums = nullptr;
-    int64_t block_sums_cap = 0;
+    unsigned int *d_block_sums = nullptr, *d_block_off = nullptr;     // items per block of the row scan, their exclusive scan
+    unsigned int *d_scan_sums = nullptr;    // block sums of a long scan (device_scan)
+    int64_t block_sums_cap = 0, scan_sums_cap = 0;
     int64_t rows_short = 0;
     int launches = 0;
     // dense-tile (MFMA) path
@@ -95,6 +96,7 @@ struct sddmm_ctx {
     void *d_sort_tmp = nullptr;
     size_t sort_tmp_bytes = 0;
     int64_t cand_cap = 0, vstrips_cap = 0, n_cand = 0, n_vstrips = 0;
+    int gathered_stride = 0;         // words of a pair's kept bitmap (k_gathered_count), 0: not kept
     unsigned int *d_vstrip_ntiles = nullptr, *d_vstrip_off = nullptr;
     // row ownership (one byte per row: 0 row kernels, 1 dense tiles, 2 row panels, 3 gathered strips, 4 union strips)
     unsigned char *d_owner = nullptr;
@@ -112,7 +114,7 @@ struct sddmm_ctx {
     ScanJobs scan_jobs{};            // short scans waiting for the next read-back of the counters
     int n_scan_jobs = 0;
     bool use_short_list = false;
-    unsigned int *d_short_sums = nullptr;   // arena view: entries of short rows per block of the row scan
+    unsigned int *d_short_sums = nullptr, *d_short_off = nullptr;     // arena views: entries of short rows per block of the row scan
     RowItem *d_panel_items = nullptr;
     int64_t n_panel_items = 0, panel_items_cap = 0, n_panels = 0, nnz_panels = 0;
     bool panel_mfma = false;         // panels run on k_panel_mfma (else on k_panel)
@@ -127,7 +129,7 @@ struct sddmm_ctx {
     RowItem *d_block_segments = nullptr, *d_block_gaps = nullptr;
     int64_t block_segments_max = 0, block_gaps_max = 0;      // as the launch sizes its grid: the true numbers where the host has them
     bool use_blocks = false;         // set by a plan of SDDMM_AUTO
-    unsigned int *d_long_sums = nullptr;    // arena view: long rows per block of the row scan
+    unsigned int *d_long_sums = nullptr, *d_long_off = nullptr;       // arena views: long rows per block of the row scan
     // entries that came in no order, sorted by row and column block: row and column of each, the place every entry
     // went to, and the dot products in that order
     int32_t *d_order = nullptr;      // one allocation, kept until the sparse operand goes

@@ -92,28 +92,22 @@ __device__ __forceinline__ unsigned int wave_max_u32(unsigned int v) {
 
 // What a plan clears before its classifiers run, in one launch (a fill through the
 // runtime is a launch of its own for every region): the row-ownership bytes and every
-// counter except what validation measured (non-empty rows, longest row).  rows_only: just
-// the row classes and the item total, for the second count after the gathered strips.
+// counter except what validation measured (non-empty rows, longest row).
 static __global__ __launch_bounds__(256) void k_plan_reset(unsigned char *__restrict__ owner, int64_t owner_bytes,
-                                                    DevCounters *pc, int rows_only) {
+                                                    DevCounters *pc) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (!rows_only) {
-        // 16 bytes per thread (the array is 256-byte aligned and padded to 64 bytes past the rows)
-        const int64_t at = i * 16;
-        if (at + 16 <= owner_bytes) *reinterpret_cast<uint4 *>(owner + at) = make_uint4(0u, 0u, 0u, 0u);
-        else for (int64_t q = at; q < owner_bytes; ++q) owner[q] = 0;
-    }
+    // 16 bytes per thread (the array is 256-byte aligned and padded to 64 bytes past the rows)
+    const int64_t at = i * 16;
+    if (at + 16 <= owner_bytes) *reinterpret_cast<uint4 *>(owner + at) = make_uint4(0u, 0u, 0u, 0u);
+    else for (int64_t q = at; q < owner_bytes; ++q) owner[q] = 0;
     if (blockIdx.x == 0) {
-        const int first = K_ROWS_SHORT, last = rows_only ? K_NNZ_LONG : K_NNZ_PANELS;
-        for (int k = first; k <= last; ++k)
+        for (int k = K_ROWS_SHORT; k <= K_NNZ_PANELS; ++k)
             for (int sl = threadIdx.x; sl < SPREAD; sl += blockDim.x) pc->k[k][sl] = 0ull;
         if (threadIdx.x == 0) {
             pc->n_items = 0ull;
             pc->short_scanned = 0ull;
             pc->long_scanned = 0ull;
-            if (!rows_only) {
-                pc->tiles_scanned = 0ull; pc->panel_items = 0ull; pc->n_candidates = 0ull; pc->utiles_scanned = 0ull;
-            }
+            pc->tiles_scanned = 0ull; pc->panel_items = 0ull; pc->n_candidates = 0ull; pc->utiles_scanned = 0ull;
         }
     }
 }
@@ -269,13 +263,33 @@ constexpr int SCAN_TILE = SCAN_BLOCK * SCAN_ITEMS;  // rows per block
 // 16-row strip, 3: a strip of rows gathered by column window) or the row-panel path
 // (2) computes the row; such rows count as empty here
 // (only != 0: just the rows of that owner count as empty)
-__device__ __forceinline__ unsigned int row_item_count(const int32_t *__restrict__ rowptr,
-                                                       const unsigned char *__restrict__ owner, int64_t i,
-                                                       int M, int ts, int seg, unsigned int *len_out, int only = 0) {
-    if (i >= M || (owner && (only ? owner[i] == only : owner[i] != 0))) { *len_out = 0; return 0; }
-    const unsigned int len = (unsigned int)(rowptr[i + 1] - rowptr[i]);
-    *len_out = len;
+__device__ __forceinline__ unsigned int row_item_count(unsigned int len, int ts, int seg) {
     return len >= (unsigned int)ts ? (len + seg - 1) / seg : 0u;
+}
+
+// lengths of the SCAN_ITEMS rows from `base` on, 0 for those that do not exist or have an owner (as row_item_count)
+__device__ __forceinline__ void row_lengths(const int32_t *__restrict__ rowptr, const unsigned char *__restrict__ owner,
+                                            int64_t base, int M, unsigned int (&len)[SCAN_ITEMS], int only = 0) {
+    static_assert(SCAN_ITEMS == 4, "one 16-byte load of the row pointer");
+    if (base + SCAN_ITEMS <= M) {                              // one round trip instead of one per row
+        const I4u p = *reinterpret_cast<const I4u *>(rowptr + base);
+        const int last = rowptr[base + SCAN_ITEMS];
+        uint32_t own = 0;
+        if (owner) own = *reinterpret_cast<const uint32_t *>(owner + base);
+        const int at[SCAN_ITEMS + 1] = {p.x, p.y, p.z, p.w, last};
+#pragma unroll
+        for (int q = 0; q < SCAN_ITEMS; ++q) {
+            const uint32_t o = (own >> (8 * q)) & 0xFFu;
+            len[q] = (only ? o == (uint32_t)only : o != 0u) ? 0u : (unsigned int)(at[q + 1] - at[q]);
+        }
+        return;
+    }
+#pragma unroll
+    for (int q = 0; q < SCAN_ITEMS; ++q) {
+        const int64_t i = base + q;
+        const bool on = i < M && !(owner && (only ? owner[i] == only : owner[i] != 0));
+        len[q] = on ? (unsigned int)(rowptr[i + 1] - rowptr[i]) : 0u;
+    }
 }
 
 // block-wide exclusive scan of one value per thread (SCAN_BLOCK threads); returns
@@ -313,9 +327,10 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int3
     unsigned int items = 0, longest = 0, pieces = 0;
     unsigned int r_alike = 0;
     unsigned long long r_short = 0, r_med = 0, r_long = 0, n_short = 0, n_med = 0, n_long = 0;
+    unsigned int lens[SCAN_ITEMS];
+    row_lengths(rowptr, owner, base, M, lens, only);
     for (int q = 0; q < SCAN_ITEMS; ++q) {
-        unsigned int len;
-        const unsigned int cnt = row_item_count(rowptr, owner, base + q, M, ts, seg, &len, only);
+        const unsigned int len = lens[q], cnt = row_item_count(len, ts, seg);
         items += cnt;
         longest = len > longest ? len : longest;
         pieces += cnt > 1 ? cnt : 0;
@@ -374,16 +389,16 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_count(const int3
     if (long_sums && threadIdx.x == 0) long_sums[blockIdx.x] = (unsigned int)sh[2];
 }
 
-// pass 2: exclusive scan of the block sums in place (one workgroup), total -> *total_out
-static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_block_sums(unsigned int *__restrict__ block_sums, int n,
+// pass 2: exclusive scan of the block sums (one workgroup; in == out is allowed), total -> *total_out
+static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_block_sums(const unsigned int *in, unsigned int *out, int n,
                                                                 unsigned long long *__restrict__ total_out) {
     unsigned int carry = 0;
     for (int base = 0; base < n; base += SCAN_BLOCK) {
         const int i = base + (int)threadIdx.x;
-        const unsigned int v = i < n ? block_sums[i] : 0u;
+        const unsigned int v = i < n ? in[i] : 0u;
         unsigned int total;
         const unsigned int ex = block_exclusive_scan(v, &total);
-        if (i < n) block_sums[i] = carry + ex;
+        if (i < n) out[i] = carry + ex;
         carry += total;
     }
     if (threadIdx.x == 0) *total_out = carry;
@@ -453,31 +468,43 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_jobs(ScanJobs jobs) 
 // The entry list of the short rows: {position, row} of every stored entry of the rows that
 // have fewer than ts entries and no owner, in storage order.  The kernels take it 64 entries
 // per wavefront, whatever the lengths of the rows (block_offsets: exclusive scan of the
-// short_sums of k_classify_count).
+// short_sums of k_classify_count).  SHORT_LIST_SPLIT workgroups share a block of the row scan, each writes the entries
+// of its part of the rows, two threads per row (one workgroup, a thread per four rows: 9.2 us for 27 000 rows of 12
+// entries, 30 workgroups on 256 CUs; split 4.9).
+constexpr int SHORT_LIST_SPLIT = 8, SHORT_LIST_ROWS = SCAN_TILE / SHORT_LIST_SPLIT;
 static __global__ __launch_bounds__(SCAN_BLOCK) void k_short_list_write(const int32_t *__restrict__ rowptr,
                                                                  const unsigned char *__restrict__ owner, int M,
                                                                  int ts, const unsigned int *__restrict__ block_offsets,
                                                                  int2 *__restrict__ list) {
-    const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
+    static_assert(2 * SHORT_LIST_ROWS == SCAN_BLOCK && SHORT_LIST_ROWS % SCAN_ITEMS == 0, "two threads per row of the part");
+    __shared__ unsigned int at_of[SHORT_LIST_ROWS], len_of[SHORT_LIST_ROWS];
+    const int64_t block = blockIdx.x / SHORT_LIST_SPLIT;
+    const int part = (int)(blockIdx.x % SHORT_LIST_SPLIT), tid = (int)threadIdx.x;
     unsigned int len[SCAN_ITEMS], mine = 0;
+    row_lengths(rowptr, owner, block * SCAN_TILE + (int64_t)tid * SCAN_ITEMS, M, len);
+#pragma unroll
     for (int q = 0; q < SCAN_ITEMS; ++q) {
-        const int64_t i = base + q;
-        unsigned int l = 0;
-        if (i < M && !(owner && owner[i] != 0)) {
-            l = (unsigned int)(rowptr[i + 1] - rowptr[i]);
-            if (l >= (unsigned int)ts) l = 0;
-        }
-        len[q] = l;
-        mine += l;
+        if (len[q] >= (unsigned int)ts) len[q] = 0;
+        mine += len[q];
     }
     unsigned int total;
-    unsigned int at = block_offsets[blockIdx.x] + block_exclusive_scan(mine, &total);
-    for (int q = 0; q < SCAN_ITEMS; ++q) {
-        if (len[q] == 0) continue;
-        const int32_t row = (int32_t)(base + q);
-        const int32_t rs = rowptr[row];
-        for (unsigned int e = 0; e < len[q]; ++e) list[at++] = make_int2(rs + (int32_t)e, row);
+    unsigned int at = block_offsets[block] + block_exclusive_scan(mine, &total);
+    const int first = tid * SCAN_ITEMS - part * SHORT_LIST_ROWS;            // row of the part
+    if (first >= 0 && first < SHORT_LIST_ROWS) {
+#pragma unroll
+        for (int q = 0; q < SCAN_ITEMS; ++q) {
+            at_of[first + q] = at;
+            len_of[first + q] = len[q];
+            at += len[q];
+        }
     }
+    __syncthreads();
+    const int r = tid >> 1;
+    const unsigned int n = len_of[r], to = at_of[r];
+    if (n == 0) return;                                                     // (rows past the last one have none)
+    const int32_t row = (int32_t)(block * SCAN_TILE + part * SHORT_LIST_ROWS + r);
+    const int32_t rs = rowptr[row];
+    for (unsigned int e = tid & 1; e < n; e += 2) list[to + e] = make_int2(rs + (int32_t)e, row);
 }
 
 // pass 3: write the items
@@ -487,10 +514,10 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_classify_write(const int3
                                                                const unsigned int *__restrict__ block_offsets,
                                                                RowItem *__restrict__ items, int only) {
     const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
-    unsigned int cnt[SCAN_ITEMS], mine = 0;
+    unsigned int cnt[SCAN_ITEMS], lens[SCAN_ITEMS], mine = 0;
+    row_lengths(rowptr, owner, base, M, lens, only);
     for (int q = 0; q < SCAN_ITEMS; ++q) {
-        unsigned int len;
-        cnt[q] = row_item_count(rowptr, owner, base + q, M, ts, seg, &len, only);
+        cnt[q] = row_item_count(lens[q], ts, seg);
         mine += cnt[q];
     }
     unsigned int total;
@@ -619,11 +646,10 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_long_rows(const int32_t *
                                                                  const unsigned int *__restrict__ block_offsets,
                                                                  int32_t *__restrict__ long_rows) {
     const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
-    unsigned int mine = 0, is_long = 0;
+    unsigned int mine = 0, is_long = 0, lens[SCAN_ITEMS];
+    row_lengths(rowptr, nullptr, base, M, lens);
     for (int q = 0; q < SCAN_ITEMS; ++q) {
-        const int64_t i = base + q;
-        unsigned int len;
-        const bool l = row_item_count(rowptr, nullptr, i, M, ts, seg, &len) > 1;
+        const bool l = row_item_count(lens[q], ts, seg) > 1;
         is_long |= (l ? 1u : 0u) << q;
         mine += l ? 1u : 0u;
     }

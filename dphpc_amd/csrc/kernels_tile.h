@@ -645,13 +645,42 @@ __device__ __forceinline__ bool gathered_mark(const int32_t *__restrict__ col, c
     return *unsorted_flag == 0;
 }
 
+// The row classes as k_classify_count left them.
+struct RowClasses {
+    unsigned int *items, *short_entries, *long_rows;           // per block of the row scan
+    int ts, seg;
+};
+// The 64 lanes' rows (len 0: none) leave the classes, for they have found an owner.
+__device__ __forceinline__ void leave_classes(const RowClasses &c, DevCounters *pc, int row, unsigned int len) {
+    const unsigned int cnt = row_item_count(len, c.ts, c.seg);
+    const int64_t block = row / SCAN_TILE;
+    if (cnt) atomicSub(&c.items[block], cnt);
+    else if (len) atomicSub(&c.short_entries[block], len);
+    if (cnt > 1) atomicSub(&c.long_rows[block], 1u);
+    const unsigned long long rows[3] = {(unsigned long long)__popcll(__ballot(len != 0 && cnt == 0)),
+                                        (unsigned long long)__popcll(__ballot(cnt == 1)),
+                                        (unsigned long long)__popcll(__ballot(cnt > 1))};
+    const unsigned long long entries[3] = {wave_sum_u64(cnt == 0 ? len : 0u), wave_sum_u64(cnt == 1 ? len : 0u),
+                                           wave_sum_u64(cnt > 1 ? len : 0u)};
+    if (lane_id() == 0) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {                          // (the sums wrap around: the slots add up to the difference)
+            spread_add(pc, K_ROWS_SHORT + k, 0ull - rows[k]);
+            spread_add(pc, K_NNZ_SHORT + k, 0ull - entries[k]);
+        }
+    }
+}
+
 // pass 1 of the gathered strips: descriptors per strip of the pair (0: not taken; the same for
-// both strips), the strips' row table, ownership of the rows of a taken pair.
+// both strips), the strips' row table, ownership of the rows of a taken pair, which leave the row classes (counting
+// all rows again was a launch of 6 us and one that cleared the counters).  The bitmap of a taken pair is kept for pass 2
+// where there is room (stride words per pair: first tile column, span, bitmap; 0: no room).
 static __global__ __launch_bounds__(GATHERED_BLOCK) void k_gathered_count(
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col,
     const unsigned long long *__restrict__ sorted_keys,
     int64_t n_cand, int64_t n_vpairs, int min_fill, unsigned int *__restrict__ vstrip_ntiles,
-    int32_t *__restrict__ vrows, unsigned char *__restrict__ owner, DevCounters *pc) {
+    int32_t *__restrict__ vrows, unsigned char *__restrict__ owner, DevCounters *pc, RowClasses classes,
+    unsigned int *__restrict__ kept, int stride) {
     __shared__ unsigned int bm[STRIP_BM_WORDS];
     __shared__ int unsorted_flag, tile_total;
     const int64_t vp = blockIdx.x;
@@ -676,7 +705,13 @@ static __global__ __launch_bounds__(GATHERED_BLOCK) void k_gathered_count(
         take = sorted && tiles > 0 && h.entries >= (int64_t)min_fill * tiles * h.halves;
     }
     const int padded = (tiles + TILE_WINDOW - 1) / TILE_WINDOW * TILE_WINDOW;
+    if (take && stride) {                                      // (the span of a taken pair fits the bitmap and stays below N)
+        unsigned int *to = kept + vp * stride;
+        for (int w = (int)threadIdx.x; w < (h.span + 31) >> 5; w += GATHERED_BLOCK) to[2 + w] = bm[w];
+        if (threadIdx.x == 0) { to[0] = (unsigned int)h.lo; to[1] = (unsigned int)h.span; }
+    }
     if (first) {
+        if (take) leave_classes(classes, pc, h.row, h.row >= 0 ? (unsigned int)(h.e - h.s) : 0u);
         if (take && h.row >= 0) owner[h.row] = 3;
         if (lane == 0) {
             vstrip_ntiles[2 * vp] = take ? (unsigned int)padded : 0u;
@@ -708,19 +743,50 @@ static __global__ __launch_bounds__(GATHERED_BLOCK) void k_gathered_tiles(
     const unsigned long long *__restrict__ sorted_keys,
     int64_t n_cand, int64_t n_vpairs, const unsigned int *__restrict__ vstrip_ntiles,
     const unsigned int *__restrict__ vstrip_off, TileDesc *__restrict__ tiles, int32_t *__restrict__ tile_cols,
-    int lead) {
+    int lead, const unsigned int *__restrict__ kept, int stride) {
     __shared__ unsigned int bm[STRIP_BM_WORDS];
-    __shared__ int unsorted_flag;
+    __shared__ int before[STRIP_BM_WORDS];                     // tile columns in the words before
+    __shared__ int unsorted_flag, totals[GATHERED_BLOCK / WAVE], highest;
     const int64_t vp = blockIdx.x;
     // (strip -1 is nobody's: the window that holds them is walked tile by tile, and they write nothing)
     if (vp == 0 && (int)threadIdx.x < lead) write_empty_desc(tiles, tile_cols, -(int64_t)lead + threadIdx.x, -1, 0);
     const unsigned int per_strip = vstrip_ntiles[2 * vp];
     if (per_strip == 0) return;                      // workgroup-uniform
     const int lane = lane_id();
-    const GatheredHead h = gathered_head(rowptr, col, sorted_keys, n_cand, vp);
-    (void)gathered_mark(col, h, bm, &unsorted_flag);
-    if (wave_in_block() != 0) return;                // the first wave writes the descriptors in column order
-    const int words = (h.span + 31) >> 5;
+    int lo, words;
+    if (stride) {
+        const unsigned int *from = kept + vp * stride;
+        lo = (int)from[0];
+        words = ((int)from[1] + 31) >> 5;
+        for (int w = (int)threadIdx.x; w < words; w += GATHERED_BLOCK) bm[w] = from[2 + w];
+    } else {
+        const GatheredHead h = gathered_head(rowptr, col, sorted_keys, n_cand, vp);
+        (void)gathered_mark(col, h, bm, &unsorted_flag);
+        lo = h.lo;
+        words = (h.span + 31) >> 5;
+    }
+    __syncthreads();
+    // one thread per word: tile columns in the words before it
+    static_assert(STRIP_BM_WORDS <= GATHERED_BLOCK, "one word per thread");
+    const int t = (int)threadIdx.x;
+    const unsigned int mine = t < words ? bm[t] : 0u;
+    const int n = __builtin_popcount(mine);
+    int incl = n;
+    for (int o = 1; o < WAVE; o <<= 1) {
+        const int up = __shfl_up(incl, o, WAVE);
+        if (lane >= o) incl += up;
+    }
+    if (lane == WAVE - 1) totals[wave_in_block()] = incl;
+    if (t == 0) highest = -1;
+    __syncthreads();
+    int run = incl - n, all = 0;
+    for (int w = 0; w < GATHERED_BLOCK / WAVE; ++w) {
+        run += w < wave_in_block() ? totals[w] : 0;
+        all += totals[w];
+    }
+    if (t < words) before[t] = run;
+    if (mine) atomicMax(&highest, t * 32 + 31 - __builtin_clz(mine));
+    __syncthreads();
     const int64_t base = vstrip_off[2 * vp];
     const int strip0 = GATHERED_BASE + (int)(2 * vp);
     auto put = [&](int rank, int tj) {
@@ -730,35 +796,15 @@ static __global__ __launch_bounds__(GATHERED_BLOCK) void k_gathered_tiles(
         *reinterpret_cast<int4 *>(tiles + at + TILE_WINDOW) = make_int4(strip0 + 1, tj, 0, 0);
         write_aligned_cols(tile_cols, at + TILE_WINDOW, tj);
     };
-    int run = 0, top = -1;
-    for (int wb = 0; wb < words; wb += WAVE) {
-        const int w = wb + lane;
-        unsigned int x = w < words ? bm[w] : 0u;
-        const int n = __builtin_popcount(x);
-        int incl = n;
-        for (int o = 1; o < WAVE; o <<= 1) {
-            const int up = __shfl_up(incl, o, WAVE);
-            if (lane >= o) incl += up;
-        }
-        int rank = run + (incl - n);
-        while (x) {
-            const int b = __builtin_ctz(x);
-            x &= x - 1;
-            const int tj = h.lo + w * 32 + b;
-            put(rank, tj);
-            top = tj;                                 // ascending inside a lane and from lane to lane
-            ++rank;
-        }
-        run += __builtin_amdgcn_readlane(incl, WAVE - 1);
+    // one thread per tile column of the span
+    for (int b = t; b < words * 32; b += GATHERED_BLOCK) {
+        const unsigned int x = bm[b >> 5], bit = 1u << (b & 31);
+        if (x & bit) put(before[b >> 5] + __builtin_popcount(x & (bit - 1u)), lo + b);
     }
     // the padding: tile columns beyond the pair's last one, which no row of the pair has
-    for (int o = WAVE / 2; o > 0; o >>= 1) {
-        const int other = __shfl_xor(top, o, WAVE);
-        top = other > top ? other : top;
-    }
     // (k_tile_rows gives them their per-row positions like any other descriptor: the masks come out
     // empty, the positions say where a row's entries before that column end)
-    if (run + lane < (int)per_strip) put(run + lane, top + 1 + lane);
+    if (all + t < (int)per_strip) put(all + t, lo + highest + 1 + t);
 }
 
 // pass 3: one thread per (descriptor, row): CSR position of the row's first entry
@@ -769,7 +815,7 @@ static __global__ __launch_bounds__(256) void k_tile_rows(const int32_t *__restr
                                                    const int32_t *__restrict__ col, int M,
                                                    const int32_t *__restrict__ vrows,
                                                    const int32_t *__restrict__ tile_cols,
-                                                   TileDesc *__restrict__ tiles, int64_t n_tiles) {
+                                                   TileDesc *__restrict__ tiles, int64_t n_tiles, int64_t nnz) {
     const int64_t slot = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t t = slot >> 4;
     const int sub = (int)(slot & 15);
@@ -803,8 +849,18 @@ static __global__ __launch_bounds__(256) void k_tile_rows(const int32_t *__restr
     if (a < end) {
         const int last = end - 1;
         int cs[16];
+        if (a + 16 <= nnz) {
+            // sixteen entries in four loads (as sixteen loads: 16.0 us for 20 000 tiles, four: 9.5; a load whose 64 lanes
+            // touch as many lines takes the address unit 64 cycles whatever its width)
 #pragma unroll
-        for (int j = 0; j < 16; ++j) cs[j] = col[a + j < last ? a + j : last];
+            for (int j = 0; j < 16; j += 4) {
+                const I4u v = *reinterpret_cast<const I4u *>(col + a + j);
+                cs[j] = v.x; cs[j + 1] = v.y; cs[j + 2] = v.z; cs[j + 3] = v.w;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) cs[j] = col[a + j < last ? a + j : last];
+        }
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
             if (a + j <= last && cs[j] <= top) {

@@ -25,6 +25,7 @@ void release_arena(sddmm_ctx *c, bool idle = false) {
     c->d_cand_keys = c->d_sorted_keys = nullptr;
     c->d_vrows = nullptr;
     c->d_block_sums = c->d_short_sums = c->d_long_sums = nullptr;
+    c->d_block_off = c->d_short_off = c->d_long_off = c->d_scan_sums = nullptr;
     c->owner_cap = c->strips_cap = c->ustrips_cap = c->panels_cap = c->cand_cap = c->vstrips_cap = 0;
     c->block_sums_cap = 0;
 }
@@ -49,7 +50,9 @@ int ensure_arena(sddmm_ctx *c) {
     const size_t o_vrows = take((size_t)(n_strips + 2) * 16 * 4);
     const size_t o_panel_n = take((size_t)n_panels * 4), o_panel_o = take((size_t)n_panels * 4);
     const size_t o_keys = take((size_t)(M + 1) * 8), o_sorted = take((size_t)(M + 1) * 8);
-    const size_t o_sums = take((size_t)n_sums * 4), o_short_sums = take((size_t)n_sums * 4), o_long_sums = take((size_t)n_sums * 4);
+    const size_t n_blocks = (size_t)((M + SCAN_TILE - 1) / SCAN_TILE);
+    const size_t o_scan = take((size_t)n_sums * 4), o_sums = take(n_blocks * 4), o_short_sums = take(n_blocks * 4), o_long_sums = take(n_blocks * 4);
+    const size_t o_off = take(n_blocks * 4), o_short_off = take(n_blocks * 4), o_long_off = take(n_blocks * 4);
     ALLOC_TRY(c, c->d_arena, at);
     char *b = c->d_arena;
     c->d_owner = (unsigned char *)(b + o_owner);
@@ -62,12 +65,17 @@ int ensure_arena(sddmm_ctx *c) {
     c->d_block_sums = (unsigned int *)(b + o_sums);
     c->d_short_sums = (unsigned int *)(b + o_short_sums);
     c->d_long_sums = (unsigned int *)(b + o_long_sums);
+    c->d_block_off = (unsigned int *)(b + o_off);
+    c->d_short_off = (unsigned int *)(b + o_short_off);
+    c->d_long_off = (unsigned int *)(b + o_long_off);
+    c->d_scan_sums = (unsigned int *)(b + o_scan);
     c->owner_cap = M + 64;
     c->strips_cap = c->ustrips_cap = n_strips;
     c->vstrips_cap = n_strips + 2;
     c->panels_cap = n_panels;
     c->cand_cap = M + 1;
-    c->block_sums_cap = n_sums;
+    c->scan_sums_cap = n_sums;
+    c->block_sums_cap = (int64_t)n_blocks;
     c->arena_rows = M;
     return SDDMM_OK;
 }
@@ -187,40 +195,37 @@ int rows_per_wave(double avg_short_len) {
 
 // Row classifier: statistics, then the item list of the wave-per-segment kernel.
 // Row classes and work items of the rows nobody owns, in two halves around a read-back of the
-// counters: the count (launch only; it may be launched again after more rows found an owner) ...
-int classify_rows_count(sddmm_ctx *c, bool again = false) {
+// counters: the count (launch only; it finds its counters cleared, begin_ownership), the scans of its sums (k_gathered_count
+// takes the rows of the gathered strips out of the sums, which are then scanned once more) ...
+int classify_rows_scan(sddmm_ctx *c) {
+    const int64_t nb = ((int64_t)c->sM + SCAN_TILE - 1) / SCAN_TILE;
+    if (nb == 0) return SDDMM_OK;
+    if (nb <= SCAN_SMALL_MAX) {
+        int rc = queue_scan(c, c->d_block_sums, c->d_block_off, nb, &c->d_pc->n_items);
+        if (rc) return rc;
+        rc = queue_scan(c, c->d_short_sums, c->d_short_off, nb, &c->d_pc->short_scanned);
+        if (rc) return rc;
+        return queue_scan(c, c->d_long_sums, c->d_long_off, nb, &c->d_pc->long_scanned);
+    }
+    SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, (const unsigned int *)c->d_block_sums, c->d_block_off, (int)nb, &c->d_pc->n_items);
+    SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, (const unsigned int *)c->d_short_sums, c->d_short_off, (int)nb,
+                 &c->d_pc->short_scanned);
+    SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, (const unsigned int *)c->d_long_sums, c->d_long_off, (int)nb,
+                 &c->d_pc->long_scanned);
+    LAUNCH_CHECK(c);
+    return SDDMM_OK;
+}
+int classify_rows_count(sddmm_ctx *c) {
     const int64_t nb = ((int64_t)c->sM + SCAN_TILE - 1) / SCAN_TILE;
     ARENA_HOLDS(c, nb, c->block_sums_cap, "block sums");
-    // the first count of a plan finds its counters cleared (begin_ownership); a second one keeps what
-    // validation and the ownership classifiers measured and clears the row classes
-    if (again) {
-        SDDMM_LAUNCH(c, k_plan_reset, 1, 256, c->d_owner, (int64_t)0, c->d_pc, 1);
-        LAUNCH_CHECK(c);
-    }
     if (nb > 0) {
         const unsigned char *owner = c->owner_active ? c->d_owner : nullptr;
         SDDMM_LAUNCH(c, k_classify_count, nb, SCAN_BLOCK, c->d_rowptr, owner,
                            c->sM, c->ts, c->seg, c->d_block_sums, c->d_pc, 0, c->d_short_sums, c->d_long_sums,
                            (const int32_t *)nullptr, 0);
         LAUNCH_CHECK(c);
-        if (nb <= SCAN_SMALL_MAX) {
-            int rc = queue_scan(c, c->d_block_sums, c->d_block_sums, nb, &c->d_pc->n_items);
-            if (rc) return rc;
-            rc = queue_scan(c, c->d_short_sums, c->d_short_sums, nb, &c->d_pc->short_scanned);
-            if (rc) return rc;
-            rc = queue_scan(c, c->d_long_sums, c->d_long_sums, nb, &c->d_pc->long_scanned);
-            if (rc) return rc;
-        } else {
-            SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, c->d_block_sums, (int)nb,
-                               &c->d_pc->n_items);
-            SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, c->d_short_sums, (int)nb,
-                               &c->d_pc->short_scanned);
-            SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, c->d_long_sums, (int)nb,
-                               &c->d_pc->long_scanned);
-            LAUNCH_CHECK(c);
-        }
     }
-    return SDDMM_OK;
+    return classify_rows_scan(c);
 }
 // ... and the items, once the counters are on the host (nothing may use the block sums in between)
 int classify_rows_items(sddmm_ctx *c) {
@@ -237,7 +242,7 @@ int classify_rows_items(sddmm_ctx *c) {
     if (c->n_items > 0) {
         SDDMM_LAUNCH(c, k_classify_write, nb, SCAN_BLOCK, c->d_rowptr,
                            (const unsigned char *)(c->owner_active ? c->d_owner : nullptr), c->sM, c->ts, c->seg,
-                           c->d_block_sums, c->d_items, 0);
+                           (const unsigned int *)c->d_block_off, c->d_items, 0);
         LAUNCH_CHECK(c);
     }
     // the entries of the short rows as a list, taken 64 at a time (entry_list_body)
@@ -262,9 +267,9 @@ int classify_rows_items(sddmm_ctx *c) {
         if (!c->use_short_list) c->n_short_list = 0;
     }
     if (c->use_short_list) {
-        SDDMM_LAUNCH(c, k_short_list_write, nb, SCAN_BLOCK, c->d_rowptr,
+        SDDMM_LAUNCH(c, k_short_list_write, nb * SHORT_LIST_SPLIT, SCAN_BLOCK, c->d_rowptr,
                            (const unsigned char *)(c->owner_active ? c->d_owner : nullptr), c->sM, c->ts,
-                           (const unsigned int *)c->d_short_sums, c->d_short_list);
+                           (const unsigned int *)c->d_short_off, c->d_short_list);
         LAUNCH_CHECK(c);
     }
     return SDDMM_OK;
@@ -273,16 +278,12 @@ int classify_rows_items(sddmm_ctx *c) {
 // Exclusive scan of n unsigned ints on the device (in != out), total to *d_total.
 int device_scan(sddmm_ctx *c, const unsigned int *in, unsigned int *out, int64_t n, unsigned long long *d_total) {
     if (n <= SCAN_SMALL_MAX) return queue_scan(c, in, out, n, d_total);
-    {
-        const int rc = flush_scans(c);             // (the long scan borrows the block sums)
-        if (rc) return rc;
-    }
     const int64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
-    ARENA_HOLDS(c, nb, c->block_sums_cap, "block sums");
-    SDDMM_LAUNCH(c, k_scan_sums, nb, SCAN_BLOCK, in, n, c->d_block_sums);
-    SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, c->d_block_sums, (int)nb, d_total);
+    ARENA_HOLDS(c, nb, c->scan_sums_cap, "block sums");
+    SDDMM_LAUNCH(c, k_scan_sums, nb, SCAN_BLOCK, in, n, c->d_scan_sums);
+    SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, (const unsigned int *)c->d_scan_sums, c->d_scan_sums, (int)nb, d_total);
     SDDMM_LAUNCH(c, k_scan_apply, nb, SCAN_BLOCK, in, n,
-                       (const unsigned int *)c->d_block_sums, out);
+                       (const unsigned int *)c->d_scan_sums, out);
     LAUNCH_CHECK(c);
     return SDDMM_OK;
 }
@@ -294,7 +295,7 @@ int begin_ownership(sddmm_ctx *c) {
     if (arc) return arc;
     ARENA_HOLDS(c, bytes, c->owner_cap, "row owners");
     // one launch clears the owners and every counter of the classifiers, the row classes included
-    SDDMM_LAUNCH(c, k_plan_reset, grid_for((bytes + 15) / 16, 256), 256, c->d_owner, bytes, c->d_pc, 0);
+    SDDMM_LAUNCH(c, k_plan_reset, grid_for((bytes + 15) / 16, 256), 256, c->d_owner, bytes, c->d_pc);
     LAUNCH_CHECK(c);
     c->owner_active = true;
     c->tiles_active = false;
@@ -411,12 +412,17 @@ int plan_gathered_count(sddmm_ctx *c, int min_fill, bool *launched) {
                                             c->stream));
     }
     // pairs of strips: 32 consecutive candidates share one list of tile columns
+    const int64_t M = c->sM;
     const int64_t n_vpairs = (c->n_cand + 31) / 32;
     c->n_vstrips = 2 * n_vpairs;
     ARENA_HOLDS(c, c->n_vstrips, c->vstrips_cap, "gathered strips");
+    // the bitmaps of the pairs wait for k_gathered_tiles where the unsorted keys were, if they fit there
+    c->gathered_stride = 2 + std::min(STRIP_BM_WORDS, (c->sN + 511) / 512);
+    if (n_vpairs * c->gathered_stride * (int64_t)sizeof(unsigned int) > (M + 1) * (int64_t)sizeof(unsigned long long)) c->gathered_stride = 0;
+    const RowClasses rows{c->d_block_sums, c->d_short_sums, c->d_long_sums, c->ts, c->seg};
     SDDMM_LAUNCH(c, k_gathered_count, n_vpairs, GATHERED_BLOCK, c->d_rowptr, c->d_col,
                        (const unsigned long long *)c->d_sorted_keys, c->n_cand, n_vpairs, min_fill, c->d_vstrip_ntiles,
-                       c->d_vrows, c->d_owner, c->d_pc);
+                       c->d_vrows, c->d_owner, c->d_pc, rows, (unsigned int *)c->d_cand_keys, c->gathered_stride);
     LAUNCH_CHECK(c);
     rc = device_scan(c, c->d_vstrip_ntiles, c->d_vstrip_off, c->n_vstrips, &c->d_pc->tiles_scanned);
     if (rc) return rc;
@@ -512,12 +518,13 @@ int plan_tiles_fill(sddmm_ctx *c) {
         SDDMM_LAUNCH(c, k_gathered_tiles, c->n_vstrips / 2, GATHERED_BLOCK, c->d_rowptr,
                            c->d_col, (const unsigned long long *)c->d_sorted_keys, c->n_cand, c->n_vstrips / 2,
                            c->d_vstrip_ntiles, c->d_vstrip_off, c->d_tiles + gathered_lo,
-                           c->d_tile_cols + gathered_lo * 16, (int)c->n_tiles_lead);
+                           c->d_tile_cols + gathered_lo * 16, (int)c->n_tiles_lead, (const unsigned int *)c->d_cand_keys,
+                           c->gathered_stride);
         LAUNCH_CHECK(c);
     }
     SDDMM_LAUNCH(c, k_tile_rows, ((c->n_tiles * 16 + 255) / 256), 256,
                        c->d_rowptr, c->d_col, c->sM, (const int32_t *)c->d_vrows, (const int32_t *)c->d_tile_cols,
-                       c->d_tiles, c->n_tiles);
+                       c->d_tiles, c->n_tiles, c->nnz);
     LAUNCH_CHECK(c);
     // windows of TILE_WINDOW descriptors: what a wavefront of the tile kernels takes.  As a batch
     // (one access per run of a row's entries, which costs reading the column indices) where the
@@ -646,7 +653,7 @@ int plan_blocks(sddmm_ctx *c, bool cut_long_rows) {
     unsigned int *seg_items = (unsigned int *)(b + o_seg[1]), *seg_off = (unsigned int *)(b + o_seg[2]);
     unsigned int *gap_items = (unsigned int *)(b + o_gap[1]), *gap_off = (unsigned int *)(b + o_gap[2]);
     if (n_long > 0) {
-        SDDMM_LAUNCH(c, k_long_rows, nb, SCAN_BLOCK, c->d_rowptr, c->sM, c->ts, c->seg, (const unsigned int *)c->d_long_sums, rows);
+        SDDMM_LAUNCH(c, k_long_rows, nb, SCAN_BLOCK, c->d_rowptr, c->sM, c->ts, c->seg, (const unsigned int *)c->d_long_off, rows);
         SDDMM_LAUNCH(c, k_long_segments, grid_for(n_seg, 256), 256, c->d_rowptr, entry_cols(c), c->sN, (const int32_t *)rows,
                      (int)n_long, (int)piece, most, seg_start, seg_items);
     }
@@ -936,8 +943,8 @@ int do_plan(sddmm_ctx *c, int strategy) {
                 rc = plan_gathered_count(c, std::max(1, env_int("SDDMM_GATHERED_FILL", tile_fill * 3 / 4)), &launched);
                 if (rc) return rc;
                 if (launched) {
-                    // gathered strips may have taken rows: classify again, one more read-back
-                    rc = classify_rows_count(c, true);
+                    // gathered strips may have taken rows: the row classes without them, one more read-back
+                    rc = classify_rows_scan(c);
                     if (rc) return rc;
                     rc = fetch_counters(c);
                     if (rc) return rc;
@@ -1416,7 +1423,7 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
             SDDMM_LAUNCH(c, k_classify_count, nb, SCAN_BLOCK, c->d_rowptr,
                                panel_owner, c->sM, row_max + 1, seg, c->d_block_sums, c->d_pc, 2,
                                (unsigned int *)nullptr, (unsigned int *)nullptr, look_at, window);
-            SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, c->d_block_sums, (int)nb,
+            SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, (const unsigned int *)c->d_block_sums, c->d_block_off, (int)nb,
                                &c->d_pc->n_items);
             LAUNCH_CHECK(c);
             HIP_TRY(c, hipMemcpyAsync(&tmp, c->d_pc, sizeof(DevCounters), hipMemcpyDeviceToHost, c->stream));
@@ -1500,7 +1507,7 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
         }
         if (c->n_fused_items > 0) {
             SDDMM_LAUNCH(c, k_classify_write, nb, SCAN_BLOCK, c->d_rowptr,
-                               panel_owner, c->sM, row_max + 1, seg, c->d_block_sums, c->d_fused_items, 2);
+                               panel_owner, c->sM, row_max + 1, seg, (const unsigned int *)c->d_block_off, c->d_fused_items, 2);
             if (c->n_fused_pieces > 0) {
                 HIP_TRY(c, hipMemsetAsync(&c->d_pc->fused_pieces, 0, 2 * sizeof(unsigned long long), c->stream));
                 SDDMM_LAUNCH(c, k_piece_places, grid_for(c->n_fused_items, 256), 256, (const int32_t *)c->d_rowptr,
