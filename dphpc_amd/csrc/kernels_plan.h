@@ -91,11 +91,12 @@ __device__ __forceinline__ unsigned int wave_max_u32(unsigned int v) {
 }
 
 // What a plan clears before its classifiers run, in one launch (a fill through the
-// runtime is a launch of its own for every region): the row-ownership bytes and every
-// counter except what validation measured (non-empty rows, longest row).
+// runtime is a launch of its own for every region): the row-ownership bytes (owner_bytes 0: k_own_rows writes them all),
+// the sums of the row classes (n_sums words) and every counter except what validation measured (non-empty rows, longest row).
 static __global__ __launch_bounds__(256) void k_plan_reset(unsigned char *__restrict__ owner, int64_t owner_bytes,
-                                                    DevCounters *pc) {
+                                                    unsigned int *__restrict__ sums, int64_t n_sums, DevCounters *pc) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n_sums) sums[i] = 0u;
     // 16 bytes per thread (the array is 256-byte aligned and padded to 64 bytes past the rows)
     const int64_t at = i * 16;
     if (at + 16 <= owner_bytes) *reinterpret_cast<uint4 *>(owner + at) = make_uint4(0u, 0u, 0u, 0u);
@@ -566,52 +567,6 @@ static __global__ __launch_bounds__(256) void k_piece_places(const int32_t *__re
     if (lane == 0) at = (unsigned int)atomicAdd(&pc->fused_cut, (unsigned long long)__popcll(cut));
     at = __shfl(at, 0, WAVE) + (unsigned int)__popcll(cut & ((1ull << lane) - 1ull));
     if (n != 0) cut_rows[at] = row;
-}
-
-// ---------------------------------------------------------------------------
-// Row-panel detector: panel p = rows [8p, 8p+8).  It qualifies when all 8 rows
-// exist, are not owned by the dense-tile path, have the same length >= min_len and
-// the same column list.  One wavefront per panel; lanes stride over the list.
-// counts[p] = work items of the panel (ceil(len/pseg)) or 0; owner = 2 on its rows when taken.
-static __global__ __launch_bounds__(256) void k_panel_flags(const int32_t *__restrict__ rowptr,
-                                                     const int32_t *__restrict__ col, int M, int64_t n_panels,
-                                                     int min_len, int pseg, unsigned char *__restrict__ owner,
-                                                     unsigned int *__restrict__ counts, DevCounters *pc) {
-    const int64_t p = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    if (p >= n_panels) return;
-    const int lane = lane_id();
-    const int64_t row0 = p * 8;
-    bool ok = row0 + 8 <= M && owner[row0] == 0;   // strips own aligned groups of 16 rows
-    int s0 = 0, len = 0;
-    if (ok) {
-        s0 = rowptr[row0];
-        len = rowptr[row0 + 1] - s0;
-        ok = len >= min_len;
-        for (int r = 1; ok && r < 8; ++r) ok = rowptr[row0 + r + 1] - rowptr[row0 + r] == len;
-    }
-    // ok is the same in every lane here.  Equal lengths make the 8 rows equally spaced
-    // in the CSR arrays (row r starts at s0 + r*len), so the 7 comparisons of one
-    // position are independent loads.
-    if (ok) {
-        bool differ = false;
-        for (int e = lane; e < len; e += WAVE) {
-            const int32_t *pc0 = col + s0 + e;
-            const int c0 = pc0[0];
-            int d = 0;
-#pragma unroll
-            for (int r = 1; r < 8; ++r) d |= pc0[(int64_t)r * len] ^ c0;
-            differ |= d != 0;
-        }
-        ok = __ballot(differ) == 0;
-    }
-    if (ok && lane < 8) owner[row0 + lane] = 2;
-    if (lane == 0) {
-        counts[p] = ok ? (unsigned int)((len + pseg - 1) / pseg) : 0u;
-        if (ok) {
-            spread_add(pc, K_PANELS, 1ull);
-            spread_add(pc, K_NNZ_PANELS, (unsigned long long)len * 8ull);
-        }
-    }
 }
 
 // items of the taken panels: {first row, [start,end) inside the shared list}

@@ -4,7 +4,7 @@
 //
 //   * a strip is rows [16*ti, 16*ti+16); a tile is the strip's entries whose
 //     column lies in [16*tj, 16*tj+16);
-//   * the classifier (k_strip_count / k_strip_tiles / k_tile_rows, plan phase,
+//   * the classifier (k_own_rows / k_strip_tiles / k_tile_rows, plan phase,
 //     device only) finds the non-empty tiles of every strip and emits one TileDesc
 //     per tile: for every row the CSR position of its first entry inside the tile
 //     and a 16-bit mask of the columns present;
@@ -257,19 +257,11 @@ __device__ __forceinline__ void strip_bounds(const int32_t *__restrict__ col, in
     *boundary_descents = __popcll(__ballot(has && first_col <= before));
 }
 
-// pass 1: strip_ntiles[s] = number of tiles of a strip that goes to the tile path
-// (sorted rows, at least min_fill entries per tile on average), else 0.
-static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_strip_count(
-    const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int M, int64_t n_strips, int min_fill,
-    unsigned int *__restrict__ strip_ntiles, unsigned char *__restrict__ owner, DevCounters *pc) {
-    __shared__ unsigned int bm_all[STRIPS_PER_BLOCK][STRIP_BM_WORDS];
-    const int64_t strip = (int64_t)blockIdx.x * STRIPS_PER_BLOCK + wave_in_block();
-    if (strip >= n_strips) return;            // whole waves leave
-    unsigned int *bm = bm_all[wave_in_block()];
+// Number of tiles of a strip that goes to the tile path (sorted rows, at least min_fill entries per tile on average), else 0.
+// bm: STRIP_BM_WORDS words of the wave's own.
+__device__ __forceinline__ int strip_tiles_of(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int M,
+                                              int64_t strip, int lane_rp, int e0, int e1, int min_fill, unsigned int *bm) {
     const int lane = lane_id();
-    const int64_t r = strip * 16 + lane;
-    const int lane_rp = rowptr[r < M ? r : M];
-    const int e0 = __builtin_amdgcn_readlane(lane_rp, 0), e1 = __builtin_amdgcn_readlane(lane_rp, 16);
     const int64_t entries = (int64_t)e1 - (int64_t)e0;
     const int64_t max_tiles = entries / min_fill;
     // changes >= (row, tile) pairs - 15 and tiles >= pairs / 16
@@ -326,14 +318,7 @@ static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_strip_count(
         }
         take = tiles > 0 && tiles <= max_tiles && entries >= (int64_t)min_fill * tiles;
     }
-    if (take && lane < 16 && strip * 16 + lane < M) owner[strip * 16 + lane] = 1;
-    if (lane == 0) {
-        strip_ntiles[strip] = take ? (unsigned int)tiles : 0u;
-        if (take) {
-            spread_add(pc, K_TILES, (unsigned long long)tiles);
-            spread_add(pc, K_NNZ_TILES, (unsigned long long)entries);
-        }
-    }
+    return take ? (int)tiles : 0;
 }
 
 // pass 2 (after the exclusive scan of strip_ntiles into strip_off): strip and tile
@@ -412,54 +397,6 @@ constexpr int UNION_BM_WORDS = 4096;          // a column span of 131072 per str
 
 __device__ __forceinline__ int max16(int v) { return -min16(-v); }
 
-static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_union_count(
-    const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int M, int64_t n_strips, int min_fill,
-    unsigned char *__restrict__ owner, unsigned int *__restrict__ ustrip_ntiles, DevCounters *pc) {
-    __shared__ unsigned int bm_all[STRIPS_PER_BLOCK][UNION_BM_WORDS];
-    const int64_t strip = (int64_t)blockIdx.x * STRIPS_PER_BLOCK + wave_in_block();
-    if (strip >= n_strips) return;
-    unsigned int *bm = bm_all[wave_in_block()];
-    const int lane = lane_id();
-    const int64_t r = strip * 16 + lane;
-    const int lane_rp = rowptr[r < M ? r : M];
-    const int e0 = __builtin_amdgcn_readlane(lane_rp, 0), e1 = __builtin_amdgcn_readlane(lane_rp, 16);
-    const int64_t entries = (int64_t)e1 - (int64_t)e0;
-    // the strip must be free as a whole, and even its longest row alone must not need
-    // more tiles than the threshold allows
-    const bool owned = lane < 16 && r < M && owner[r] != 0;
-    const int next_rp = __shfl_down(lane_rp, 1, WAVE);          // every lane takes part in the permute
-    const int len = lane < 16 ? next_rp - lane_rp : 0;
-    const int longest = __builtin_amdgcn_readfirstlane(max16(lane < 16 ? len : 0));
-    int64_t tiles = 0;
-    bool take = false;
-    if (__ballot(owned) == 0ull && entries >= (int64_t)min_fill * ((longest + 15) / 16) && entries >= min_fill) {
-        int lo, span, allowed;
-        strip_bounds<0>(col, lane_rp, e0, &lo, &span, &allowed);
-        if (span > 0 && span <= UNION_BM_WORDS * 32) {
-            const int words = (span + 31) >> 5;
-            for (int w = lane; w < words; w += WAVE) bm[w] = 0u;
-            wave_lds_order();
-            int64_t descents = 0;
-            (void)strip_scan<2>(col, e0, e1, INT64_MAX, lo, span, bm, &descents);
-            wave_lds_order();
-            if (descents == allowed) {
-                int t = 0;
-                for (int w = lane; w < words; w += WAVE) t += __builtin_popcount(bm[w]);
-                tiles = (wave_sum_i32(t) + 15) / 16;
-                take = tiles > 0 && entries >= (int64_t)min_fill * tiles;
-            }
-        }
-    }
-    if (take && lane < 16 && r < M) owner[r] = 4;
-    if (lane == 0) {
-        ustrip_ntiles[strip] = take ? (unsigned int)tiles : 0u;
-        if (take) {
-            spread_add(pc, K_UTILES, (unsigned long long)tiles);
-            spread_add(pc, K_NNZ_UTILES, (unsigned long long)entries);
-        }
-    }
-}
-
 // descriptors of the union strips: header and the 16 union columns of every tile
 static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_union_tiles(
     const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int M, int64_t n_strips,
@@ -524,33 +461,194 @@ static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_union_tiles(
 constexpr int GATHERED_BASE = 1 << 30;
 constexpr int TILE_WINDOW = 4;                  // descriptors per window (what a wavefront of the tile kernels takes)
 
-static __global__ __launch_bounds__(256) void k_gather_candidates(const int32_t *__restrict__ rowptr,
-                                                           const int32_t *__restrict__ col, int M,
-                                                           const unsigned char *__restrict__ owner, int min_len,
-                                                           unsigned long long *__restrict__ keys,
-                                                           unsigned long long *__restrict__ count) {
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    bool cand = false;
-    int first = 0;
-    if (r < M && owner[r] == 0) {
-        const int s = rowptr[r], e = rowptr[r + 1];
-        if (e - s >= min_len) {
-            first = col[s];
-            const int64_t span = (int64_t)col[e - 1] - first + 1;
-            cand = span > 0 && (int64_t)(e - s) * 4 >= span;
-        }
+// ---- who owns a row -----------------------------------------------------------------------
+// The classifiers of a plan in one launch: a wavefront looks at a 16-row strip (dense tiles), then at its two 8-row panels;
+// the workgroup looks together at those of its four strips that could be union strips (their bitmap takes the LDS of all
+// four); the first wavefront then offers the rows that are left to the gathered strips and classifies them.  As five
+// launches they read the row pointer five times and waited for each other: OWN_FIGURES
+struct OwnRules {
+    int strip_fill, panel_min, union_fill, cand_min;     // 0: not looked for
+    int pseg;                                             // entries of a panel's work items
+    int ts, seg;                                          // row classes (k_classify_count)
+};
+struct OwnArrays {
+    unsigned char *owner;                                 // 1: strip, 2: panel, 4: union strip, 0: nobody
+    unsigned int *strip_ntiles, *panel_counts, *ustrip_ntiles;
+    unsigned long long *cand_keys;
+    unsigned int *items, *short_entries, *long_rows;      // per block of the row scan, cleared
+};
+
+// 8 rows from row0 on with one column list?  (Equal lengths make them equally spaced in the CSR arrays: row r starts at
+// s0 + r * len, so the 7 comparisons of one position are independent loads.)
+__device__ __forceinline__ bool same_lists(const int32_t *__restrict__ col, int s0, int len) {
+    bool differ = false;
+    for (int e = lane_id(); e < len; e += WAVE) {
+        const int32_t *at = col + s0 + e;
+        const int c0 = at[0];
+        int d = 0;
+#pragma unroll
+        for (int r = 1; r < 8; ++r) d |= at[(int64_t)r * len] ^ c0;
+        differ |= d != 0;
     }
-    // one append per wave
-    const unsigned long long m = __ballot(cand);
-    if (m == 0ull) return;
-    const int lane = lane_id();
-    unsigned long long base = 0;
-    if (lane == 0) base = atomicAdd(count, (unsigned long long)__popcll(m));
-    base = ((unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)(base >> 32)) << 32) |
-           (unsigned int)__builtin_amdgcn_readfirstlane((int)base);
-    if (cand) {
-        const unsigned long long at = base + (unsigned long long)__popcll(m & ((1ull << lane) - 1ull));
-        keys[at] = ((unsigned long long)(unsigned int)first << 32) | (unsigned long long)(unsigned int)r;
+    return __ballot(differ) == 0;
+}
+
+static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_own_rows(const int32_t *__restrict__ rowptr,
+                                                                            const int32_t *__restrict__ col, int M,
+                                                                            int64_t n_strips, int strips_per_wave,
+                                                                            OwnRules rules, OwnArrays out, DevCounters *pc) {
+    static_assert(STRIPS_PER_BLOCK == 4 && STRIPS_PER_BLOCK * STRIP_BM_WORDS == UNION_BM_WORDS, "one buffer for both bitmaps");
+    __shared__ unsigned int bm_all[UNION_BM_WORDS];
+    __shared__ int rp_of[STRIPS_PER_BLOCK][17], own_of[STRIPS_PER_BLOCK][16];
+    __shared__ int lo_of[STRIPS_PER_BLOCK], span_of[STRIPS_PER_BLOCK], allowed_of[STRIPS_PER_BLOCK];   // span 0: no union strip
+    __shared__ int found, descents_found;
+    const int lane = lane_id(), wv = wave_in_block(), tid = (int)threadIdx.x;
+    unsigned int rows_sum[3] = {0, 0, 0}, entries_sum[3] = {0, 0, 0};      // wave 0: short, medium, long
+    for (int g = 0; g < strips_per_wave; ++g) {
+        const int64_t first = ((int64_t)blockIdx.x * strips_per_wave + g) * STRIPS_PER_BLOCK;
+        if (first >= n_strips) break;                                     // workgroup-uniform
+        const int64_t strip = first + wv, r = strip * 16 + lane;
+        const int lane_rp = rowptr[r < M ? r : M];                        // (a strip past the last one has no entries)
+        const int e0 = __builtin_amdgcn_readlane(lane_rp, 0), e1 = __builtin_amdgcn_readlane(lane_rp, 16);
+        const int next_rp = __shfl_down(lane_rp, 1, WAVE);
+        const int len = lane < 16 ? next_rp - lane_rp : 0;
+        int owned = 0;                                                    // lane < 16: owner of its row
+        int tiles = 0, items[2] = {0, 0};
+        if (rules.strip_fill) tiles = strip_tiles_of(rowptr, col, M, strip, lane_rp, e0, e1, rules.strip_fill, bm_all + wv * STRIP_BM_WORDS);
+        if (tiles) owned = 1;
+        else if (rules.panel_min) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int s0 = __builtin_amdgcn_readlane(lane_rp, 8 * h), l0 = __builtin_amdgcn_readlane(len, 8 * h);
+                const bool alike = (__ballot(len == l0) >> (8 * h) & 0xFFull) == 0xFFull;
+                if (strip * 16 + 8 * h + 8 <= M && l0 >= rules.panel_min && alike && same_lists(col, s0, l0)) {
+                    items[h] = (l0 + rules.pseg - 1) / rules.pseg;
+                    if (lane >> 3 == h) owned = 2;
+                    if (lane == 0) {
+                        spread_add(pc, K_PANELS, 1ull);
+                        spread_add(pc, K_NNZ_PANELS, (unsigned long long)l0 * 8ull);
+                    }
+                }
+            }
+        }
+        int lo = 0, span = 0, allowed = 0;
+        if (rules.union_fill) {
+            // the strip must be free as a whole, and even its longest row alone must not need
+            // more tiles than the threshold allows
+            const int64_t entries = (int64_t)e1 - (int64_t)e0;
+            const int longest = __builtin_amdgcn_readfirstlane(max16(len));
+            if (!tiles && !items[0] && !items[1] && entries >= (int64_t)rules.union_fill * ((longest + 15) / 16) && entries >= rules.union_fill) {
+                strip_bounds<0>(col, lane_rp, e0, &lo, &span, &allowed);
+                if (span > UNION_BM_WORDS * 32) span = 0;
+            }
+        }
+        if (strip < n_strips && lane == 0) {
+            if (rules.strip_fill) {
+                out.strip_ntiles[strip] = (unsigned int)tiles;
+                if (tiles) {
+                    spread_add(pc, K_TILES, (unsigned long long)tiles);
+                    spread_add(pc, K_NNZ_TILES, (unsigned long long)(e1 - e0));
+                }
+            }
+            if (rules.panel_min) {
+                if (2 * strip < M / 8) out.panel_counts[2 * strip] = (unsigned int)items[0];
+                if (2 * strip + 1 < M / 8) out.panel_counts[2 * strip + 1] = (unsigned int)items[1];
+            }
+        }
+        if (lane < 17) rp_of[wv][lane] = lane_rp;
+        if (lane < 16) own_of[wv][lane] = owned;
+        if (lane == 0) { lo_of[wv] = lo; span_of[wv] = span > 0 ? span : 0; allowed_of[wv] = allowed; }
+        __syncthreads();
+        if (rules.union_fill) {
+            for (int w = 0; w < STRIPS_PER_BLOCK; ++w) {
+                const int u_span = span_of[w];
+                int u_tiles = 0;
+                const int u0 = rp_of[w][0], u1 = rp_of[w][16];
+                if (u_span > 0) {                                         // workgroup-uniform
+                    const int words = (u_span + 31) >> 5;
+                    for (int k = tid; k < words; k += WAVE * STRIPS_PER_BLOCK) bm_all[k] = 0u;
+                    if (tid == 0) { found = 0; descents_found = 0; }
+                    __syncthreads();
+                    // a quarter of the entries each
+                    const int64_t n = (int64_t)u1 - u0;
+                    const int a = u0 + (int)(n * wv / STRIPS_PER_BLOCK), b = u0 + (int)(n * (wv + 1) / STRIPS_PER_BLOCK);
+                    if (b > a) {
+                        int64_t descents = 0;
+                        (void)strip_scan<2>(col, a, b, INT64_MAX, lo_of[w], u_span, bm_all, &descents);
+                        const int over = a > u0 && col[a] <= col[a - 1] ? 1 : 0;   // (the scan does not see the entry before its first)
+                        if (lane == 0) atomicAdd(&descents_found, (int)descents + over);
+                    }
+                    __syncthreads();
+                    int t = 0;
+                    for (int k = tid; k < words; k += WAVE * STRIPS_PER_BLOCK) t += __builtin_popcount(bm_all[k]);
+                    t = wave_sum_i32(t);
+                    if (lane == 0 && t) atomicAdd(&found, t);
+                    __syncthreads();
+                    u_tiles = (found + 15) / 16;
+                    if (descents_found != allowed_of[w] || u_tiles == 0 || n < (int64_t)rules.union_fill * u_tiles) u_tiles = 0;
+                    if (u_tiles && tid < 16) own_of[w][tid] = 4;
+                    if (u_tiles && tid == 0) {
+                        spread_add(pc, K_UTILES, (unsigned long long)u_tiles);
+                        spread_add(pc, K_NNZ_UTILES, (unsigned long long)n);
+                    }
+                    __syncthreads();                                      // (the next strip's bitmap; own_of)
+                }
+                if (tid == 0 && first + w < n_strips) out.ustrip_ntiles[first + w] = (unsigned int)u_tiles;
+            }
+        }
+        if (wv == 0) {
+            // one row per lane
+            const int64_t row = first * 16 + lane;
+            const int s = rp_of[lane >> 4][lane & 15], n = rp_of[lane >> 4][(lane & 15) + 1] - s;
+            const int who = own_of[lane >> 4][lane & 15];
+            if (row < M) out.owner[row] = (unsigned char)who;
+            const unsigned int l = row < M && who == 0 ? (unsigned int)n : 0u;
+            if (rules.cand_min) {
+                bool cand = l >= (unsigned int)rules.cand_min;
+                int at0 = 0;
+                if (cand) {
+                    at0 = col[s];
+                    const int64_t width = (int64_t)col[s + n - 1] - at0 + 1;
+                    cand = width > 0 && (int64_t)n * 4 >= width;
+                }
+                const unsigned long long m = __ballot(cand);
+                if (m) {                                                  // one append per wave
+                    unsigned long long base = 0;
+                    if (lane == 0) base = atomicAdd(&pc->n_candidates, (unsigned long long)__popcll(m));
+                    base = ((unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)(base >> 32)) << 32) |
+                           (unsigned int)__builtin_amdgcn_readfirstlane((int)base);
+                    if (cand)
+                        out.cand_keys[base + (unsigned long long)__popcll(m & ((1ull << lane) - 1ull))] =
+                            ((unsigned long long)(unsigned int)at0 << 32) | (unsigned long long)(unsigned int)row;
+                }
+            }
+            // (sums of entries stay below the number of entries, which is an int)
+            const unsigned int cnt = row_item_count(l, rules.ts, rules.seg);
+            const int kind = cnt == 0 ? 0 : cnt == 1 ? 1 : 2;
+            const int n_items = wave_sum_i32((int)cnt);
+            unsigned int part[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                rows_sum[k] += (unsigned int)__popcll(__ballot(l != 0 && kind == k));
+                part[k] = (unsigned int)wave_sum_i32(kind == k ? (int)l : 0);
+                entries_sum[k] += part[k];
+            }
+            const unsigned int n_long = (unsigned int)__popcll(__ballot(l != 0 && kind == 2));
+            if (lane == 0) {
+                const int64_t block = first * 16 / SCAN_TILE;
+                if (n_items) atomicAdd(&out.items[block], (unsigned int)n_items);
+                if (part[0]) atomicAdd(&out.short_entries[block], part[0]);
+                if (n_long) atomicAdd(&out.long_rows[block], n_long);
+            }
+        }
+        __syncthreads();                                                  // (the next group's bitmaps and rows)
+    }
+    if (tid == 0) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            spread_add(pc, K_ROWS_SHORT + k, rows_sum[k]);
+            spread_add(pc, K_NNZ_SHORT + k, entries_sum[k]);
+        }
     }
 }
 
@@ -1781,7 +1879,7 @@ void k_auto_tiles(int tile_blocks, int nblocks, int short_blocks, int longest_fi
 
 // ---------------------------------------------------------------------------
 // ROW PANEL on the matrix cores: 8 consecutive rows with one column list (see
-// k_panel_flags).  One wavefront per work item = entries [start,end) of the shared
+// k_own_rows).  One wavefront per work item = entries [start,end) of the shared
 // list, 16 columns per MFMA accumulator:
 //
 //     D[c][r] = sum_k B[col_c][k] * A[row0+r][k]      c = 0..15, r = 0..7 (8..15 unused)

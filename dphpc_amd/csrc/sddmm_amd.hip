@@ -288,14 +288,16 @@ int device_scan(sddmm_ctx *c, const unsigned int *in, unsigned int *out, int64_t
     return SDDMM_OK;
 }
 
-// Clears the row-ownership bytes and the tile / panel counters before the classifiers run.
-int begin_ownership(sddmm_ctx *c) {
+// Clears the row-ownership bytes (owners false: k_own_rows writes them all), the sums of the row classes and the counters
+// before the classifiers run.
+int begin_ownership(sddmm_ctx *c, bool owners) {
     const int64_t bytes = (int64_t)c->sM + 64;
     const int arc = ensure_arena(c);
     if (arc) return arc;
     ARENA_HOLDS(c, bytes, c->owner_cap, "row owners");
-    // one launch clears the owners and every counter of the classifiers, the row classes included
-    SDDMM_LAUNCH(c, k_plan_reset, grid_for((bytes + 15) / 16, 256), 256, c->d_owner, bytes, c->d_pc);
+    const int64_t n_sums = c->d_block_off - c->d_block_sums;              // (the three arrays of sums lie next to each other)
+    const int64_t threads = std::max(n_sums, owners ? (bytes + 15) / 16 : 0);
+    SDDMM_LAUNCH(c, k_plan_reset, grid_for(threads, 256), 256, c->d_owner, owners ? bytes : (int64_t)0, c->d_block_sums, n_sums, c->d_pc);
     LAUNCH_CHECK(c);
     c->owner_active = true;
     c->tiles_active = false;
@@ -307,11 +309,7 @@ int begin_ownership(sddmm_ctx *c) {
     return SDDMM_OK;
 }
 
-// Dense-tile classifier, in three steps so that the row panels can be looked for in
-// between: (1) 16-row strips, (2) strips of rows gathered by column window among the
-// rows nobody owns yet, (3) descriptors of both.  min_fill = average stored entries
-// per 16x16 tile a strip needs to be taken.  tile_steps stays 0 when the path does not
-// apply (row size not a multiple of 64 bytes).
+// tile_steps stays 0 when the tile path does not apply (row length).
 bool tile_path_applies(sddmm_ctx *c) {
     c->tile_steps = 0;
     if (c->nnz == 0) return false;
@@ -330,18 +328,33 @@ bool ragged_pays(const sddmm_ctx *c) {
     return steps != 0 && c->nnz >= (steps <= 2 ? 1 << 18 : 1 << 16);
 }
 
-int plan_tiles_count(sddmm_ctx *c, int min_fill) {
-    if (!tile_path_applies(c)) return SDDMM_OK;
-    const int64_t n_strips = ((int64_t)c->sM + 15) / 16;
+// The rows' owners and, of the rows that are left, the candidates of the gathered strips and the row classes (launches
+// only; fetch_counters brings the totals).  Rules that do not apply have been taken out.
+int plan_owners(sddmm_ctx *c, const OwnRules &rules) {
+    const int64_t M = c->sM, n_strips = (M + 15) / 16;
     ARENA_HOLDS(c, n_strips, c->strips_cap, "strips");
-    const unsigned strip_grid = (unsigned)((n_strips + STRIPS_PER_BLOCK - 1) / STRIPS_PER_BLOCK);
-    SDDMM_LAUNCH(c, k_strip_count, strip_grid, WAVE * STRIPS_PER_BLOCK, c->d_rowptr,
-                       c->d_col, c->sM, n_strips, min_fill, c->d_strip_ntiles, c->d_owner, c->d_pc);
+    ARENA_HOLDS(c, n_strips, c->ustrips_cap, "union strips");
+    ARENA_HOLDS(c, M / 8, c->panels_cap, "panels");
+    ARENA_HOLDS(c, M, c->cand_cap, "candidate rows");
+    ARENA_HOLDS(c, (M + SCAN_TILE - 1) / SCAN_TILE, c->block_sums_cap, "block sums");
+    const OwnArrays out{c->d_owner, c->d_strip_ntiles, c->d_panel_counts, c->d_ustrip_ntiles, c->d_cand_keys,
+                        c->d_block_sums, c->d_short_sums, c->d_long_sums};
+    // a group of four strips per workgroup, several one after the other where there are more than the chip holds
+    const int64_t groups = (n_strips + STRIPS_PER_BLOCK - 1) / STRIPS_PER_BLOCK;
+    const int each = (int)std::min<int64_t>(16, std::max<int64_t>(1, groups / 4096));
+    SDDMM_LAUNCH(c, k_own_rows, (groups + each - 1) / each, WAVE * STRIPS_PER_BLOCK, c->d_rowptr, c->d_col, c->sM, n_strips, each,
+                 rules, out, c->d_pc);
     LAUNCH_CHECK(c);
-    return device_scan(c, c->d_strip_ntiles, c->d_strip_off, n_strips, &c->d_pc->tiles_scanned);
+    c->panels_flagged = rules.panel_min != 0;
+    c->union_counted = rules.union_fill != 0;
+    int rc = SDDMM_OK;
+    if (rules.strip_fill) rc = device_scan(c, c->d_strip_ntiles, c->d_strip_off, n_strips, &c->d_pc->tiles_scanned);
+    if (!rc && rules.panel_min) rc = device_scan(c, c->d_panel_counts, c->d_panel_off, M / 8, &c->d_pc->panel_items);
+    if (!rc && rules.union_fill) rc = device_scan(c, c->d_ustrip_ntiles, c->d_ustrip_off, n_strips, &c->d_pc->utiles_scanned);
+    return rc ? rc : classify_rows_scan(c);
 }
 
-// after a fetch_counters that follows plan_tiles_count (and precedes the gathered strips)
+// after a fetch_counters that follows plan_owners (and precedes the gathered strips)
 int take_tile_counts(sddmm_ctx *c) {
     c->n_tiles = c->n_tiles_natural = (int64_t)c->pc.n_tiles;
     c->nnz_tiles = (int64_t)c->pc.nnz_tiles;
@@ -356,34 +369,7 @@ int take_tile_counts(sddmm_ctx *c) {
     return SDDMM_OK;
 }
 
-// Union strips among the 16-row strips nobody owns yet (launch only; after the panel
-// detector, before the candidates of the gathered strips).
-int plan_union_count(sddmm_ctx *c, int min_fill) {
-    if (c->tile_steps == 0) return SDDMM_OK;
-    const int64_t n_strips = ((int64_t)c->sM + 15) / 16;
-    ARENA_HOLDS(c, n_strips, c->ustrips_cap, "union strips");
-    const unsigned strip_grid = (unsigned)((n_strips + STRIPS_PER_BLOCK - 1) / STRIPS_PER_BLOCK);
-    SDDMM_LAUNCH(c, k_union_count, strip_grid, WAVE * STRIPS_PER_BLOCK, c->d_rowptr,
-                       c->d_col, c->sM, n_strips, min_fill, c->d_owner, c->d_ustrip_ntiles, c->d_pc);
-    LAUNCH_CHECK(c);
-    c->union_counted = true;
-    return device_scan(c, c->d_ustrip_ntiles, c->d_ustrip_off, n_strips, &c->d_pc->utiles_scanned);
-}
-
-// Candidates of the gathered strips (launch only; the count arrives with the next
-// fetch_counters).
-int plan_gathered_candidates(sddmm_ctx *c, int min_len) {
-    if (c->tile_steps == 0 || c->sM < 2) return SDDMM_OK;
-    const int64_t M = c->sM;
-    ARENA_HOLDS(c, M, c->cand_cap, "candidate rows");
-    SDDMM_LAUNCH(c, k_gather_candidates, ((M + 255) / 256), 256, c->d_rowptr,
-                       c->d_col, c->sM, (const unsigned char *)c->d_owner, min_len, c->d_cand_keys,
-                       &c->d_pc->n_candidates);
-    LAUNCH_CHECK(c);
-    return SDDMM_OK;
-}
-
-// after the fetch_counters that follows plan_gathered_candidates
+// after the fetch_counters that follows plan_owners
 int plan_gathered_count(sddmm_ctx *c, int min_fill, bool *launched) {
     *launched = false;
     if (c->tile_steps == 0 || c->sM < 2) return SDDMM_OK;
@@ -568,23 +554,14 @@ bool panel_valu_applicable(const sddmm_ctx *c) {
     return s.unit == 0 ? s.UPL <= 2 : s.UPL == 1;
 }
 
-// panel detector (launch only) / panel items (after the next fetch_counters)
-int plan_panels_flags(sddmm_ctx *c, int min_len, int pseg) {
-    c->panels_flagged = false;
-    if (c->nnz == 0) return SDDMM_OK;
+// whether the 8-row panels are looked for, and by which kernel they would be computed
+bool panel_path_applies(sddmm_ctx *c) {
+    if (c->nnz == 0 || c->sM < PANEL_ROWS) return false;
     c->panel_mfma = (c->ragged || panel_mfma_steps(c) != 0) && env_int("SDDMM_PANEL_MFMA", 1) != 0;
-    if (!c->panel_mfma && !panel_valu_applicable(c)) return SDDMM_OK;
-    if (c->panel_mfma) min_len = std::max(min_len, 4);   // 16-byte S/P accesses stay inside a row
-    const int64_t n_panels = (int64_t)c->sM / 8;
-    if (n_panels == 0) return SDDMM_OK;
-    ARENA_HOLDS(c, n_panels, c->panels_cap, "panels");
-    SDDMM_LAUNCH(c, k_panel_flags, ((n_panels * WAVE + 255) / 256), 256,
-                       c->d_rowptr, c->d_col, c->sM, n_panels, min_len, pseg, c->d_owner, c->d_panel_counts, c->d_pc);
-    LAUNCH_CHECK(c);
-    c->panels_flagged = true;
-    return device_scan(c, c->d_panel_counts, c->d_panel_off, n_panels, &c->d_pc->panel_items);
+    return c->panel_mfma || panel_valu_applicable(c);
 }
 
+// after the fetch_counters that follows plan_owners
 int plan_panels_items(sddmm_ctx *c, int pseg) {
     if (!c->panels_flagged) return SDDMM_OK;
     const int64_t n_panels = (int64_t)c->sM / 8;
@@ -744,7 +721,7 @@ int plan_order(sddmm_ctx *c) {
     bool done = false;
     int rc = (int64_t)c->sM * COL_BLOCKS_ORDER <= ((int64_t)1 << 32) ? sort_order<uint32_t>(c, &done) : sort_order<uint64_t>(c, &done);
     if (rc || !done) return rc;
-    rc = begin_ownership(c);
+    rc = begin_ownership(c, true);
     if (rc) return rc;
     // row statistics of the sorted entries; no row has another owner
     c->ts = std::max(1, env_int("SDDMM_TS", 24));
@@ -880,8 +857,6 @@ int do_plan(sddmm_ctx *c, int strategy) {
             // rest is split by length.  MFMA_TILE takes every sorted strip and no panel,
             // LDS_TILED every panel and no strip; AUTO applies the thresholds.
             if (!csr_ok) return fail(c, SDDMM_ERR_UNSUPPORTED, "strategy %d needs row-sorted entries", resolved);
-            int rc = begin_ownership(c);
-            if (rc) return rc;
             // entries per 16x16 tile from which the tile kernel beats the gather kernels,
             // measured on banded matrices of varying fill: 74 at 128-byte rows, 50 at 256
             // and 512 bytes; 64-byte rows keep the older, conservative figure
@@ -896,39 +871,35 @@ int do_plan(sddmm_ctx *c, int strategy) {
             // (ragged fp32 rows of more than twelve steps: a wavefront per SIMD; near-dense rows K = 200 108 us without, 155 with)
             const bool gathered = resolved == SDDMM_AUTO && env_int("SDDMM_GATHERED", 1) != 0 &&
                                   !(c->ragged && c->dtype == SDDMM_F32 && ragged_steps(c) > 12);
-            // the classifiers are launched back to back; their totals come back together
-            if (resolved != SDDMM_LDS_TILED) {
-                // 16-row strips are looked at before the row panels and must not take what the
-                // panel kernel does better (8x8-block rows reach ~80 entries per tile); the
-                // strips gathered after the panels use the measured break-even.  Ragged rows: banded
-                // blocks in narrow bands reach 140 (4 000 rows, panels / tiles: K = 48 7.6 / 17.2 us, K = 24 bf16 3.9 / 8.1),
-                // and strips that are no panels come back as union strips
-                rc = plan_tiles_count(c, resolved == SDDMM_MFMA_TILE ? 1 : std::max(c->ragged ? 160 : 96, tile_fill));
-                if (rc) return rc;
+            const bool tiles = resolved != SDDMM_LDS_TILED && tile_path_applies(c);
+            OwnRules rules{};
+            // 16-row strips are looked at before the row panels and must not take what the
+            // panel kernel does better (8x8-block rows reach ~80 entries per tile); the
+            // strips gathered after the panels use the measured break-even.  Ragged rows: banded
+            // blocks in narrow bands reach 140 (4 000 rows, panels / tiles: K = 48 7.6 / 17.2 us, K = 24 bf16 3.9 / 8.1),
+            // and strips that are no panels come back as union strips
+            if (tiles) rules.strip_fill = resolved == SDDMM_MFMA_TILE ? 1 : std::max(c->ragged ? 160 : 96, tile_fill);
+            if (resolved != SDDMM_MFMA_TILE && panel_path_applies(c)) {
+                rules.panel_min = resolved == SDDMM_LDS_TILED ? 1 : std::max(1, env_int("SDDMM_PANEL_MIN", 16));
+                if (c->panel_mfma) rules.panel_min = std::max(rules.panel_min, 4);       // 16-byte S/P accesses stay inside a row
             }
-            if (resolved != SDDMM_MFMA_TILE) {
-                rc = plan_panels_flags(c, resolved == SDDMM_LDS_TILED ? 1 : std::max(1, env_int("SDDMM_PANEL_MIN", 16)), pseg);
-                if (rc) return rc;
-            } else {
-                c->panels_flagged = false;
-            }
-            if (resolved == SDDMM_AUTO && env_int("SDDMM_UNION", 1) != 0) {
-                rc = plan_union_count(c, std::max(1, env_int("SDDMM_UNION_FILL", tile_fill)));
-                if (rc) return rc;
-            }
-            if (gathered) {
-                rc = plan_gathered_candidates(c, std::max(16, env_int("SDDMM_GATHERED_MIN", 64)));
-                if (rc) return rc;
-            }
-            // the rows nobody owns so far are classified in the same batch: most matrices have
+            if (tiles && resolved == SDDMM_AUTO && env_int("SDDMM_UNION", 1) != 0)
+                rules.union_fill = std::max(1, env_int("SDDMM_UNION_FILL", tile_fill));
+            if (tiles && gathered && c->sM >= 2) rules.cand_min = std::max(16, env_int("SDDMM_GATHERED_MIN", 64));
+            rules.pseg = pseg;
+            // the rows nobody owns so far are classified in the same launch: most matrices have
             // no gathered strips, and their plan then waits for the device once
-            c->ts = std::max(1, env_int("SDDMM_TS", 24));
+            c->ts = rules.ts = std::max(1, env_int("SDDMM_TS", 24));
             // segment items of 256 entries: a wavefront walks its item chunk by chunk, one dependent
             // round trip each, so a few long items set the duration of a short launch (eight rows of
             // 554 entries as single items: 17.5 us on the mixed-density shape, 14.6 us in pieces of
             // 256); on a matrix of 36 M entries pieces of 128..2048 differ by 3 %
-            c->seg = std::max(WAVE, env_int("SDDMM_SEG", 256));
-            rc = classify_rows_count(c);
+            c->seg = rules.seg = std::max(WAVE, env_int("SDDMM_SEG", 256));
+            const bool looked = c->sM > 0 && (rules.strip_fill || rules.panel_min || rules.union_fill || rules.cand_min);
+            int rc = begin_ownership(c, !looked);
+            if (rc) return rc;
+            c->panels_flagged = false;
+            rc = looked ? plan_owners(c, rules) : classify_rows_count(c);
             if (rc) return rc;
             rc = fetch_counters(c);
             if (rc) return rc;
