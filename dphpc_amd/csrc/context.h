@@ -137,6 +137,7 @@ struct sddmm_ctx {
     float *d_order_dots = nullptr;
     int64_t order_cap = 0;
     int64_t coo_jumps = 0;           // entries that share neither row nor column with the one before them
+    double col_near = 1.0;           // share of the entries that lie in the same 16 columns as the one before them (a sample)
     bool use_order = false;          // set by a plan of SDDMM_AUTO
     // fused SDDMM + SpMM: items covering every non-empty row, output M x K
     RowItem *d_fused_items = nullptr;

@@ -321,11 +321,13 @@ bool tile_path_applies(sddmm_ctx *c) {
 // dense tiles of 100 k .. 2.5 M entries, near-dense rows, K = 9 .. 250 in fp32 and 24 .. 456 in 16 bits: 36 000 banded rows
 // K = 21 69 -> 29 us, K = 100 407 -> 74, K = 120 bf16 137 -> 39; dense tiles K = 100 48.7 -> 14.7, K = 200 bf16 53 -> 10;
 // near-dense rows K = 75 70 -> 36, K = 120 bf16 49 -> 21.  Few entries: a launch of a few microseconds either way, and the
-// plan has more to look at (100 k entries in dense tiles K = 21 4.3 us without, 5.3 with; K = 100 6.8 and 4.6).
+// plan has more to look at (100 k entries in dense tiles K = 21 4.3 us without, 5.3 with; K = 100 6.8 and 4.6).  Entries
+// that hardly ever share 16 columns with their neighbour fill no tile and no near-dense row: the plan need not look
+// (0.02 .. 0.06 in graphs and uniform rows, 0.7 .. 0.95 in the shapes above; 20 000 uniform rows 13 us of a new pattern).
 bool ragged_pays(const sddmm_ctx *c) {
     const int steps = ragged_steps(c), mode = env_int("SDDMM_RAGGED", -1);       // -1: decide here, 0: never, 1: wherever it can
     if (mode >= 0) return mode != 0 && steps != 0;
-    return steps != 0 && c->nnz >= (steps <= 2 ? 1 << 18 : 1 << 16);
+    return steps != 0 && c->nnz >= (steps <= 2 ? 1 << 18 : 1 << 16) && c->col_near >= 0.25;
 }
 
 // The rows' owners and, of the rows that are left, the candidates of the gathered strips and the row classes (launches
@@ -508,10 +510,12 @@ int plan_tiles_fill(sddmm_ctx *c) {
                            c->gathered_stride);
         LAUNCH_CHECK(c);
     }
-    SDDMM_LAUNCH(c, k_tile_rows, ((c->n_tiles * 16 + 255) / 256), 256,
-                       c->d_rowptr, c->d_col, c->sM, (const int32_t *)c->d_vrows, (const int32_t *)c->d_tile_cols,
-                       c->d_tiles, c->n_tiles, c->nnz);
-    LAUNCH_CHECK(c);
+    const int64_t of_strips = c->n_tiles_natural + c->n_tiles_union;       // (the others are complete)
+    if (of_strips > 0) {
+        SDDMM_LAUNCH(c, k_tile_rows, ((of_strips * 16 + 255) / 256), 256, c->d_rowptr, c->d_col, c->sM,
+                     (const int32_t *)c->d_tile_cols, c->d_tiles, of_strips, c->nnz);
+        LAUNCH_CHECK(c);
+    }
     // windows of TILE_WINDOW descriptors: what a wavefront of the tile kernels takes.  As a batch
     // (one access per run of a row's entries, which costs reading the column indices) where the
     // tiles are sparsely filled; tile by tile from the descriptors' masks where they are nearly
@@ -768,13 +772,14 @@ int validate_csr(sddmm_ctx *c) {
                            c->nnz, c->d_pc);
     // (walks col[0..nnz) only behind a valid row pointer)
     if (c->nnz > 0)
-        SDDMM_LAUNCH(c, k_check_index, grid_capped(c->nnz, 256), 256, c->d_col, c->nnz,
+        SDDMM_LAUNCH(c, k_check_index, grid_capped((c->nnz + 3) / 4, 256, 4096), 256, c->d_col, c->nnz,
                            c->sN, c->d_pc);
     LAUNCH_CHECK(c);
     const int rc = fetch_counters(c);
     if (rc) return rc;
     if (c->pc.bad_pattern & BAD_POINTER) return fail(c, SDDMM_ERR_PATTERN, "rowptr is not a valid CSR row pointer array");
     if (c->pc.bad_pattern) return fail(c, SDDMM_ERR_PATTERN, "column index outside [0,N)");
+    c->col_near = c->pc.col_pairs ? (double)c->pc.col_near / (double)c->pc.col_pairs : 1.0;
     return SDDMM_OK;
 }
 
@@ -1232,6 +1237,7 @@ static int set_coo_common(sddmm_ctx *c, int M, int N, int64_t nnz, const int32_t
     }
     const bool sorted = c->pc.coo_unsorted == 0;
     c->coo_jumps = (int64_t)c->pc.coo_jumps;
+    c->col_near = 1.0;                                     // (not measured)
     if (sorted) {
         SDDMM_LAUNCH(c, k_rowptr_from_sorted_coo, grid_for(nnz + 1, 256), 256,
                            c->d_rowidx, nnz, M, c->d_rowptr);
