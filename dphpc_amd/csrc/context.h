@@ -73,6 +73,7 @@ struct sddmm_ctx {
     int64_t n_tiles = 0, tiles_cap = 0, nnz_tiles = 0;
     int tile_steps = 0;
     bool ragged = false;             // tiles and panels of the plan are of ragged rows (ragged_steps)
+    bool long_rows = false;          // and of more than 1 KiB each (rows_are_long)
     bool tiles_active = false;       // d_tiles describes the current pattern
     int32_t *d_win_order = nullptr;  // order in which the launch takes the windows (null: storage order)
     unsigned int *d_win_bins = nullptr;
@@ -342,6 +343,14 @@ inline int ragged_steps(const sddmm_ctx *c) {
     return s.LPN * s.UPL / 4;
 }
 
+// Rows of more than 1 KiB, which the tile and panel kernels take LONG_STEPS at a time.  (As in ragged rows the length need
+// be no whole number of units.)
+constexpr int LONG_STEPS = 8;
+inline bool rows_are_long(const sddmm_ctx *c) {
+    const Shape s = shape_of(c);
+    return s.unit != 1 && !s.wide && (size_t)c->K * elem_size(c->dtype) > 1024;
+}
+
 // The device code of a translation unit is loaded when something first asks for one of its kernels: 3 .. 13 ms, once per
 // process.  A plan asks for the families that its launches take (load_*, one per launch_*.hip), so that no launch has to:
 // launches may be captured, and they are what callers time.
@@ -376,8 +385,10 @@ bool launch_auto_with_tiles(sddmm_ctx *c);                                      
 void launch_tiles(sddmm_ctx *c);
 bool launch_ragged_auto_with_tiles(sddmm_ctx *c);                                // launch_tiles_ragged.hip
 void launch_ragged_tiles(sddmm_ctx *c);
+void launch_long_tiles(sddmm_ctx *c);
 void launch_panels(sddmm_ctx *c);                                                // launch_panels.hip
 void launch_ragged_panels(sddmm_ctx *c);                                         // launch_panels_ragged.hip
+int launch_long_panels(sddmm_ctx *c);                                            // number of launches
 void launch_panels_fused(sddmm_ctx *c);
 // the list of the rows for k_add_cut_rows
 inline int32_t *fused_cut_rows(const sddmm_ctx *c) {

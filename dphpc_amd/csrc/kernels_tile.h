@@ -1075,6 +1075,7 @@ struct WholeRows {
     __device__ __forceinline__ Row row(const void *base, int64_t r) const { return (const uint4 *)base + r * (STEPS * 4); }
     __device__ __forceinline__ uint4 unit(const void *, Row row, int u, int) const { return row[u]; }
     __device__ __forceinline__ uint4 trim(const uint4 &v, int, int) const { return v; }
+    __device__ __forceinline__ int last_unit() const { return STEPS * 4 - 1; }
 };
 
 template <class U_, int STEPS>
@@ -1084,6 +1085,7 @@ struct RaggedRows {
     static constexpr int WHOLE_STEPS = ragged_whole_steps(STEPS);
     using Row = uint32_t;                                     // byte offset: operands below 4 GiB
     int len, last;                                            // length as U takes it, last unit
+    __device__ __forceinline__ int last_unit() const { return last; }
     explicit __device__ __forceinline__ RaggedRows(int len_) : len(len_), last(U::units(len_) - 1) {}
     __device__ __forceinline__ Row row(const void *, int64_t r) const { return (uint32_t)r * U::row_bytes(len); }
     // unit u of a row; step: the step it belongs to as far as the compiler knows it (STEPS: any)
@@ -1699,12 +1701,14 @@ constexpr int KSPLIT = WAVES_PER_BLOCK;
 static_assert(KSPLIT == 4 && TILE_WINDOW == 4, "one finishing wave per tile of a window");
 constexpr int KSPLIT_LDS_FLOATS = TILE_WINDOW * KSPLIT * 256;
 
-template <int DT, int STEPS, class R>
+// LONG: rows of any length (RaggedRows), STEPS of them at a time.
+template <int DT, int STEPS, class R, bool LONG = false>
 __global__ __launch_bounds__(BLOCK) void k_tile_ksplit(int64_t nblocks, const int32_t *__restrict__ order,
     const TileDesc *__restrict__ tiles, int64_t n_tiles, const int32_t *__restrict__ tile_cols, const void *__restrict__ A,
     const void *__restrict__ B, int len, int M, int N, const int32_t *__restrict__ vrows, const float *__restrict__ sval,
     float *__restrict__ P) {
     static_assert(STEPS % KSPLIT == 0, "K in four equal parts of whole 64-byte steps");
+    static_assert(!LONG || R::RAGGED, "rows of any length are ragged ones");
     constexpr int SW = STEPS / KSPLIT;                    // steps of this wave
     __shared__ __attribute__((aligned(16))) float part[KSPLIT_LDS_FLOATS];
     int64_t w = xcd_remap(blockIdx.x, nblocks);
@@ -1722,7 +1726,7 @@ __global__ __launch_bounds__(BLOCK) void k_tile_ksplit(int64_t nblocks, const in
     const int quarter = j * SW * 4;                       // this wave's quarter of every row: whole rows have it in the base
     const void *Aq = R::RAGGED ? A : (const void *)((const uint4 *)A + (uint32_t)quarter);
     const void *Bq = R::RAGGED ? B : (const void *)((const uint4 *)B + (uint32_t)quarter);
-    const int u0 = R::RAGGED ? quarter : 0;
+    int u0 = R::RAGGED ? quarter : 0;
     auto to_operand = [&](const uint4 &v, int s) {
         uint4 r;
         r.x = (uint32_t)__builtin_amdgcn_ds_bpermute(to_operand_from, (int)v.x);
@@ -1754,19 +1758,20 @@ __global__ __launch_bounds__(BLOCK) void k_tile_ksplit(int64_t nblocks, const in
     };
     // second round trip: this wave's quarter of the A panel and of all B tiles, the S values of its own tile
     uint4 a[SW], b[TILE_WINDOW][SW];
-    {
+    auto load = [&]() {
         const typename R::Row src = a_rows(strip[0]);
 #pragma unroll
         for (int s = 0; s < SW; ++s) a[s] = rows.unit(Aq, src, u0 + 4 * s + lunit, STEPS);
-    }
 #pragma unroll
-    for (int k = 0; k < TILE_WINDOW; ++k) {
-        int64_t brow = bcol[k];
-        brow = brow < N ? brow : N - 1;                   // columns past N (and the filler of a short union tile) are in no mask
-        const typename R::Row src = rows.row(Bq, brow);
+        for (int k = 0; k < TILE_WINDOW; ++k) {
+            int64_t brow = bcol[k];
+            brow = brow < N ? brow : N - 1;               // columns past N (and the filler of a short union tile) are in no mask
+            const typename R::Row src_b = rows.row(Bq, brow);
 #pragma unroll
-        for (int s = 0; s < SW; ++s) b[k][s] = rows.unit(Bq, src, u0 + 4 * s + lunit, STEPS);
-    }
+            for (int s = 0; s < SW; ++s) b[k][s] = rows.unit(Bq, src_b, u0 + 4 * s + lunit, STEPS);
+        }
+    };
+    load();
     const unsigned int below = (1u << r16) - 1u;
     const int offs[4] = {off4.x, off4.y, off4.z, off4.w};
     const unsigned int masks[4] = {mask2.x & 0xFFFFu, mask2.x >> 16, mask2.y & 0xFFFFu, mask2.y >> 16};
@@ -1780,18 +1785,33 @@ __global__ __launch_bounds__(BLOCK) void k_tile_ksplit(int64_t nblocks, const in
         pos[i] = on ? offs[i] + __builtin_popcount(masks[i] & below) : 0;   // (row 4q+i, column r16); entry 0 when absent
         sv[i] = sval[pos[i]];
     }
+    auto products = [&](auto &&take) {                    // take(k, the sums of tile k)
 #pragma unroll
-    for (int s = 0; s < SW; ++s) a[s] = to_operand(a[s], s);
+        for (int s = 0; s < SW; ++s) a[s] = to_operand(a[s], s);
 #pragma unroll
-    for (int k = 0; k < TILE_WINDOW; ++k) {
-        if (k >= n) break;                                // workgroup-uniform
-        if (k > 0 && strip[k] != strip[k - 1]) {          // workgroup-uniform: the window reaches into the next strip
-            const typename R::Row src = a_rows(strip[k]);
+        for (int k = 0; k < TILE_WINDOW; ++k) {
+            if (k >= n) break;                            // workgroup-uniform
+            if (k > 0 && strip[k] != strip[k - 1]) {      // workgroup-uniform: the window reaches into the next strip
+                const typename R::Row src = a_rows(strip[k]);
 #pragma unroll
-            for (int s = 0; s < SW; ++s) a[s] = to_operand(rows.unit(Aq, src, u0 + 4 * s + lunit, STEPS), s);
+                for (int s = 0; s < SW; ++s) a[s] = to_operand(rows.unit(Aq, src, u0 + 4 * s + lunit, STEPS), s);
+            }
+            take(k, mfma_steps<DT, R>(a, [&](int s) { return to_operand(b[k][s], s); }));
         }
-        *reinterpret_cast<f32x4_t *>(part + (k * KSPLIT + j) * 256 + lane * 4) =
-            mfma_steps<DT, R>(a, [&](int s) { return to_operand(b[k][s], s); });
+    };
+    auto keep = [&](int k, const f32x4_t &sum) { *reinterpret_cast<f32x4_t *>(part + (k * KSPLIT + j) * 256 + lane * 4) = sum; };
+    if constexpr (LONG) {
+        f32x4_t total[TILE_WINDOW] = {};
+        for (;;) {                                        // (the same number of turns in every wave)
+            products([&](int k, const f32x4_t &sum) { total[k] += sum; });
+            u0 += 4 * STEPS;
+            if (u0 - quarter > rows.last) break;
+            load();
+        }
+#pragma unroll
+        for (int k = 0; k < TILE_WINDOW; ++k) keep(k, total[k]);
+    } else {
+        products(keep);
     }
     __syncthreads();
     if (j < n) {
@@ -2072,11 +2092,14 @@ constexpr int panel_mfma_min_waves(int steps, bool fused, bool half_width = fals
     return fused ? (k <= 32 ? 3 : k == 64 ? 2 : 1) : steps == 8 ? 4 : 1;
 }
 
-template <int DT, int STEPS, bool FUSED = false, class R = WholeRows<STEPS>>
+// SLICED: rows of any length, STEPS of them per launch from unit0 on; the launches add their sums to P in turn, the last one
+// multiplies by S.
+template <int DT, int STEPS, bool FUSED = false, class R = WholeRows<STEPS>, bool SLICED = false>
 __global__ __launch_bounds__(panel_mfma_waves(STEPS) * WAVE, panel_mfma_min_waves(STEPS, FUSED, DT != DT_F32))
 void k_panel_mfma(const RowItem *__restrict__ items, int64_t n_items, int64_t nblocks, const int32_t *__restrict__ rowptr,
                   const int32_t *__restrict__ col, const void *__restrict__ A, const void *__restrict__ B, int len,
-                  const float *__restrict__ sval, float *__restrict__ P, float *__restrict__ O) {
+                  const float *__restrict__ sval, float *__restrict__ P, float *__restrict__ O, int unit0) {
+    static_assert(!SLICED || R::RAGGED, "rows of any length are ragged ones");
     static_assert(!FUSED || !R::RAGGED, "fused panels: whole rows");
     static_assert(!FUSED || (DT == DT_F32 ? (STEPS == 2 || STEPS == 4 || STEPS == 8) : (STEPS == 1 || STEPS == 2 || STEPS == 4)),
                   "fused panels: 32, 64 or 128 components per row");
@@ -2124,21 +2147,24 @@ void k_panel_mfma(const RowItem *__restrict__ items, int64_t n_items, int64_t nb
     // groups of 16 columns in flight; rows of 512 bytes and more leave registers for two
     constexpr int GROUPS = STEPS >= 8 ? 2 : 4;
     const R rows(len);
+    const int first_unit = SLICED ? unit0 : 0;
+    const bool add = SLICED && unit0 > 0, scale = !SLICED || unit0 + 4 * STEPS > rows.last_unit();
+    auto step_of = [](int s) { return SLICED ? STEPS : s; };   // (any step can hold the end of a row)
     constexpr int A_REGS = BLOCKS ? STEPS / 2 : STEPS;
     uint4 a[A_REGS];
     if constexpr (BLOCKS) {
         // block cg of every k quarter: rows 4(cg&1).. of the units 4(2s'+(cg>>1))+q
         const int cg = (lane >> 2) & 3, t = lane & 3;
         const typename R::Row src = rows.row(A, row0 + 4 * (cg & 1) + t);
-        const int u0 = 4 * (cg >> 1) + q;
+        const int u0 = first_unit + 4 * (cg >> 1) + q;
 #pragma unroll
         for (int s2 = 0; s2 < A_REGS; ++s2)
-            a[s2] = rows.trim(rows.unit(A, src, 8 * s2 + u0, 2 * s2 + 1), 8 * s2 + u0, 2 * s2 + 1);
+            a[s2] = rows.trim(rows.unit(A, src, 8 * s2 + u0, step_of(2 * s2 + 1)), 8 * s2 + u0, step_of(2 * s2 + 1));
     } else {
         // panel rows: lanes 8..15 of every 16 repeat rows 0..7, their results are not stored
         const typename R::Row src = rows.row(A, row0 + (n & 7));
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) a[s] = rows.trim(rows.unit(A, src, 4 * s + q, s), 4 * s + q, s);
+        for (int s = 0; s < STEPS; ++s) a[s] = rows.trim(rows.unit(A, src, first_unit + 4 * s + q, step_of(s)), first_unit + 4 * s + q, step_of(s));
     }
     const int last = end - 1;
     auto cols_of_chunk = [&](int base) {                        // column of entry base + lane (clamped)
@@ -2153,7 +2179,7 @@ void k_panel_mfma(const RowItem *__restrict__ items, int64_t n_items, int64_t nb
         const int c = __shfl(cc, u * 16 + lrow, WAVE);
         const typename R::Row src = rows.row(B, c);
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) o.b[s] = rows.unit(B, src, 4 * s + lunit, s);
+        for (int s = 0; s < STEPS; ++s) o.b[s] = rows.unit(B, src, first_unit + 4 * s + lunit, step_of(s));
         return o;
     };
     // The S values of entries g0+4*(punit-rot) .. +3 of this lane's row: one access for the pair of
@@ -2162,11 +2188,17 @@ void k_panel_mfma(const RowItem *__restrict__ items, int64_t n_items, int64_t nb
     // inside the item fetch their S values again.  (Requested one chunk ahead of its products;
     // two chunks ahead was measured slower, in a loop 34 against 30 us and cold 53 against 48 us
     // at 128-byte rows: a request that waits for HBM holds its place in the vector memory queue.)
+    struct Window {
+        F4u s, p;                                                // SLICED: and the sums so far
+    };
     auto load_s = [&](int g0) {
         int e = g0 + 4 * (punit - rot);
         e = e < row_len - 4 ? e : row_len - 4;
         e = e > 0 ? e : 0;
-        return *reinterpret_cast<const F4u *>(sval + out_row + e);
+        Window w{F4u{1.f, 1.f, 1.f, 1.f}, F4u{0.f, 0.f, 0.f, 0.f}};
+        if (scale) w.s = *reinterpret_cast<const F4u *>(sval + out_row + e);          // (wave-uniform)
+        if (add) w.p = *reinterpret_cast<const F4u *>(P + out_row + e);
+        return w;
     };
     auto permute4 = [&](int from, uint32_t x, uint32_t y, uint32_t z, uint32_t w_) {
         uint4 r;
@@ -2177,7 +2209,7 @@ void k_panel_mfma(const RowItem *__restrict__ items, int64_t n_items, int64_t nb
         return r;
     };
     auto b_operand = [&](const Oper &o, int s) {
-        return rows.trim(permute4(to_operand_from, o.b[s].x, o.b[s].y, o.b[s].z, o.b[s].w), 4 * s + q, s);
+        return rows.trim(permute4(to_operand_from, o.b[s].x, o.b[s].y, o.b[s].z, o.b[s].w), first_unit + 4 * s + q, step_of(s));
     };
     // 4x4 blocks: both row halves of 16 columns, partial over the k quarters
     auto compute_blocks = [&](const Oper &o, f32x4_t &lo, f32x4_t &hi) {
@@ -2275,7 +2307,7 @@ void k_panel_mfma(const RowItem *__restrict__ items, int64_t n_items, int64_t nb
     };
     // groups o0 (entries g0..g0+15) and o1 (g0+16..g0+31) of the shared column list
     float held[4] = {0.f, 0.f, 0.f, 0.f};                        // ROTATE: the unit taken from the previous pair
-    auto compute_store_pair = [&](const Oper &o0, const Oper &o1, const F4u &sw, int g0) {
+    auto compute_store_pair = [&](const Oper &o0, const Oper &o1, const Window &win, int g0) {
         if (g0 >= end + (any_rot ? 32 : 0)) return;              // wave-uniform
         const bool past = g0 >= end;                             // the store-only step after the last pair
         float r0 = 0.f, r1 = 0.f, r2 = 0.f, r3 = 0.f;
@@ -2326,6 +2358,8 @@ void k_panel_mfma(const RowItem *__restrict__ items, int64_t n_items, int64_t nb
             // ROTATE, first pair: these lanes' first unit comes with the next pair
         } else if (e + 4 <= end) {
             // four consecutive entries inside the item (so the S window was not clamped)
+            const F4u sw = win.s;
+            if constexpr (SLICED) { d0 += win.p.x; d1 += win.p.y; d2 += win.p.z; d3 += win.p.w; }
             F4u out{d0 * sw.x, d1 * sw.y, d2 * sw.z, d3 * sw.w};
             *reinterpret_cast<F4u *>(P + out_row + e) = out;
             p[0] = out.x; p[1] = out.y; p[2] = out.z; p[3] = out.w;
@@ -2335,7 +2369,9 @@ void k_panel_mfma(const RowItem *__restrict__ items, int64_t n_items, int64_t nb
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 if (e + i < end) {
-                    p[i] = d[i] * sval[out_row + e + i];
+                    float sum = d[i];
+                    if constexpr (SLICED) sum += add ? P[out_row + e + i] : 0.f;
+                    p[i] = scale ? sum * sval[out_row + e + i] : sum;
                     P[out_row + e + i] = p[i];
                 }
         }
@@ -2361,7 +2397,7 @@ void k_panel_mfma(const RowItem *__restrict__ items, int64_t n_items, int64_t nb
     // this prologue too, so the prologue issues its loads in the order the loop does
     // (both column loads first, then the groups in the order they are consumed);
     // otherwise the loop would wait for almost everything it has just requested.
-    F4u s_cur[GROUPS / 2];
+    Window s_cur[GROUPS / 2];
     const int cc0 = cols_of_chunk(start);
     int cc_nxt = cols_of_chunk(start + CHUNK);                  // columns of the next chunk
     __builtin_amdgcn_sched_barrier(0);

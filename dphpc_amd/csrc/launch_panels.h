@@ -9,5 +9,5 @@ void launch_panel_mfma_t(sddmm_ctx *c, int len) {
     const int64_t nblocks = (c->n_panel_items + PW - 1) / PW;
     SDDMM_LAUNCH(c, (k_panel_mfma<DT, STEPS, false, R>), xcd_grid(nblocks), PW * WAVE,
                  (const RowItem *)c->d_panel_items, c->n_panel_items, nblocks, c->d_rowptr, c->d_col, (const void *)c->dA,
-                 (const void *)c->dB, len, (const float *)c->d_sval, c->dP, (float *)nullptr);
+                 (const void *)c->dB, len, (const float *)c->d_sval, c->dP, (float *)nullptr, 0);
 }

@@ -21,7 +21,7 @@ void launch_panel_fused_t(sddmm_ctx *c) {
     const int64_t nblocks = (c->n_panel_items + PW - 1) / PW;
     SDDMM_LAUNCH(c, (k_panel_mfma<DT, STEPS, true>), xcd_grid(nblocks), PW * WAVE,
                  (const RowItem *)c->d_panel_items, c->n_panel_items, nblocks, c->d_rowptr, c->d_col, (const void *)c->dA,
-                 (const void *)c->dB, 0, (const float *)c->d_sval, c->dP, c->dO);
+                 (const void *)c->dB, 0, (const float *)c->d_sval, c->dP, c->dO, 0);
 }
 template <int DT>
 void launch_panel_mfma_steps(sddmm_ctx *c) {

@@ -14,6 +14,25 @@ void launch_ragged_panel_steps(sddmm_ctx *c, int len) {
     }
 }
 
+// rows of more than 1 KiB: LONG_STEPS at a time
+template <int DT, class U>
+int launch_long_panel_steps(sddmm_ctx *c, int len, int units) {
+    constexpr int PW = panel_mfma_waves(LONG_STEPS);
+    const int64_t nblocks = (c->n_panel_items + PW - 1) / PW;
+    int launches = 0;
+    for (int unit0 = 0; unit0 < units; unit0 += 4 * LONG_STEPS, ++launches)
+        SDDMM_LAUNCH(c, (k_panel_mfma<DT, LONG_STEPS, false, RaggedRows<U, LONG_STEPS>, true>), xcd_grid(nblocks), PW * WAVE,
+                     (const RowItem *)c->d_panel_items, c->n_panel_items, nblocks, c->d_rowptr, c->d_col, (const void *)c->dA,
+                     (const void *)c->dB, len, (const float *)c->d_sval, c->dP, (float *)nullptr, unit0);
+    return launches;
+}
+
+int launch_long_panels(sddmm_ctx *c) {
+    if (c->dtype == SDDMM_BF16) return launch_long_panel_steps<DT_BF16, UnitBF16x8>(c, c->K / 8, c->K / 8);
+    if (c->dtype == SDDMM_F16) return launch_long_panel_steps<DT_F16, UnitF16x8>(c, c->K / 8, c->K / 8);
+    return launch_long_panel_steps<DT_F32, UnitF32x4u>(c, c->K, (c->K + 3) / 4);
+}
+
 void launch_ragged_panels(sddmm_ctx *c) {
     if (c->dtype == SDDMM_BF16) launch_ragged_panel_steps<DT_BF16, UnitBF16x8>(c, c->K / 8);
     else if (c->dtype == SDDMM_F16) launch_ragged_panel_steps<DT_F16, UnitF16x8>(c, c->K / 8);

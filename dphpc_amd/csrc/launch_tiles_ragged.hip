@@ -14,6 +14,20 @@ void launch_ragged_tile_steps(sddmm_ctx *c, int len) {
     }
 }
 
+// rows of more than 1 KiB: LONG_STEPS at a time
+template <int DT, class U>
+void launch_long_tile_steps(sddmm_ctx *c, int len) {
+    SDDMM_LAUNCH(c, (k_tile_ksplit<DT, LONG_STEPS, RaggedRows<U, LONG_STEPS>, true>), xcd_grid(c->n_windows), BLOCK, c->n_windows,
+                 (const int32_t *)(c->use_win_order ? c->d_win_order : nullptr), (const TileDesc *)c->d_tiles, c->n_tiles,
+                 (const int32_t *)c->d_tile_cols, (const void *)c->dA, (const void *)c->dB, len, c->M, c->N,
+                 (const int32_t *)c->d_vrows, (const float *)c->d_sval, c->dP);
+}
+void launch_long_tiles(sddmm_ctx *c) {
+    if (c->dtype == SDDMM_BF16) launch_long_tile_steps<DT_BF16, UnitBF16x8>(c, c->K / 8);
+    else if (c->dtype == SDDMM_F16) launch_long_tile_steps<DT_F16, UnitF16x8>(c, c->K / 8);
+    else launch_long_tile_steps<DT_F32, UnitF32x4u>(c, c->K);
+}
+
 bool launch_ragged_auto_with_tiles(sddmm_ctx *c) { return launch_auto_with_tiles_t<true>(c); }
 void launch_ragged_tiles(sddmm_ctx *c) {
     if (c->dtype == SDDMM_BF16) launch_ragged_tile_steps<DT_BF16, UnitBF16x8>(c, c->K / 8);

@@ -313,7 +313,7 @@ int begin_ownership(sddmm_ctx *c, bool owners) {
 bool tile_path_applies(sddmm_ctx *c) {
     c->tile_steps = 0;
     if (c->nnz == 0) return false;
-    c->tile_steps = c->ragged ? ragged_steps(c) : panel_mfma_steps(c);
+    c->tile_steps = c->long_rows ? LONG_STEPS : c->ragged ? ragged_steps(c) : panel_mfma_steps(c);
     return c->tile_steps != 0;
 }
 
@@ -328,6 +328,13 @@ bool ragged_pays(const sddmm_ctx *c) {
     const int steps = ragged_steps(c), mode = env_int("SDDMM_RAGGED", -1);       // -1: decide here, 0: never, 1: wherever it can
     if (mode >= 0) return mode != 0 && steps != 0;
     return steps != 0 && c->nnz >= (steps <= 2 ? 1 << 18 : 1 << 16) && c->col_near >= 0.25;
+}
+
+// Rows of more than 1 KiB on the tile and panel kernels, if they own nearly all of the entries.
+bool long_pays(const sddmm_ctx *c) {
+    const int mode = env_int("SDDMM_LONG_TILES", -1);              // -1: decide here, 0: never, 1: wherever it can
+    if (!rows_are_long(c) || mode == 0) return false;
+    return mode > 0 || (c->nnz >= 1 << 18 && c->col_near >= 0.5);
 }
 
 // The rows' owners and, of the rows that are left, the candidates of the gathered strips and the row classes (launches
@@ -525,7 +532,7 @@ int plan_tiles_fill(sddmm_ctx *c) {
         const int rc = plan_window_order(c);
         if (rc) return rc;
     }
-    c->use_windows = c->nnz_tiles < (int64_t)env_int("SDDMM_WINDOW_FILL", 176) * c->n_tiles;
+    c->use_windows = !c->long_rows && c->nnz_tiles < (int64_t)env_int("SDDMM_WINDOW_FILL", 176) * c->n_tiles;
     // wavefronts of a tile launch: one per window, and one per two windows of a pair of gathered strips
     // (their descriptors come last and fill whole windows, an even number of them)
     c->n_win_single = c->n_windows;
@@ -806,10 +813,17 @@ int enqueue_run(sddmm_ctx *c) {
             c->launches = 0;
             const bool tiles = c->tiles_active && c->n_tiles > 0, rows = c->rows_short > 0 || c->n_items > 0;
             bool fused = false;
-            if (tiles && rows && env_int("SDDMM_FUSE", 1) != 0) fused = launch_auto_with_tiles(c);
+            if (tiles && rows && !c->long_rows && env_int("SDDMM_FUSE", 1) != 0) fused = launch_auto_with_tiles(c);
             if (fused) ++c->launches;
-            if (tiles && !fused) { launch_tiles(c); ++c->launches; }
-            if (c->n_panel_items > 0) { launch_panels(c); ++c->launches; }
+            if (tiles && !fused) {
+                if (c->long_rows) launch_long_tiles(c);
+                else launch_tiles(c);
+                ++c->launches;
+            }
+            if (c->n_panel_items > 0) {
+                if (c->long_rows) c->launches += launch_long_panels(c);
+                else { launch_panels(c); ++c->launches; }
+            }
             if (rows && !fused) { launch_auto(c); ++c->launches; }
             break;
         }
@@ -872,10 +886,11 @@ int do_plan(sddmm_ctx *c, int strategy) {
             const int64_t even = (c->nnz / PANEL_ROWS / 3072 + WAVE - 1) / WAVE * WAVE;
             const int pseg = std::max(WAVE, env_int("SDDMM_PANEL_SEG", (int)std::min<int64_t>(512, even)));
             c->tile_steps = 0;
-            c->ragged = resolved == SDDMM_AUTO && ragged_pays(c);
+            c->long_rows = resolved == SDDMM_AUTO && long_pays(c);
+            c->ragged = c->long_rows || (resolved == SDDMM_AUTO && ragged_pays(c));
             // (ragged fp32 rows of more than twelve steps: a wavefront per SIMD; near-dense rows K = 200 108 us without, 155 with)
             const bool gathered = resolved == SDDMM_AUTO && env_int("SDDMM_GATHERED", 1) != 0 &&
-                                  !(c->ragged && c->dtype == SDDMM_F32 && ragged_steps(c) > 12);
+                                  !c->long_rows && !(c->ragged && c->dtype == SDDMM_F32 && ragged_steps(c) > 12);
             const bool tiles = resolved != SDDMM_LDS_TILED && tile_path_applies(c);
             OwnRules rules{};
             // 16-row strips are looked at before the row panels and must not take what the
@@ -910,6 +925,16 @@ int do_plan(sddmm_ctx *c, int strategy) {
             if (rc) return rc;
             rc = take_tile_counts(c);
             if (rc) return rc;
+            // The kernels of the other rows take a row of more than 1 KiB an entry at a time: the matrix goes in slices as a
+            // whole where strips and panels do not own nearly all of it.
+            if (c->long_rows && (int64_t)(c->pc.nnz_tiles + c->pc.nnz_utiles + c->pc.nnz_panels) < c->nnz - c->nnz / 16) {
+                c->ragged = c->long_rows = c->panels_flagged = false;
+                c->tile_steps = 0;
+                rc = begin_ownership(c, true);
+                if (!rc) rc = classify_rows_count(c);
+                if (!rc) rc = fetch_counters(c);
+                if (rc) return rc;
+            }
             rc = plan_panels_items(c, pseg);
             if (rc) return rc;
             if (gathered) {

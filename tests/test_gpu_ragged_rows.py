@@ -113,6 +113,55 @@ def test_ragged_rows_keep_infinities_to_themselves(engine_factory, monkeypatch, 
     np.testing.assert_array_equal(np.isnan(out[1]), np.isnan(out[0]))
 
 
+LONG = [(K, capi.F32) for K in (257, 260, 300, 384, 511, 512, 516, 640, 1000, 1025)]
+LONG += [(K, d) for d in (capi.BF16, capi.F16) for K in (520, 600, 768, 1024, 1032)]
+
+
+@pytest.mark.parametrize("K,dtype", LONG)
+def test_rows_beyond_1_kib(engine_factory, monkeypatch, K, dtype):
+    """Tiles and panels of rows that the kernels take in several turns or launches; the rows that nobody owns stay with the
+    gather kernels, and a matrix with many of them does as a whole."""
+    M, N, rowptr, col, val, rng = _structured(K, near_dense=0)
+    Ad, Bd, A, B = _operands(rng, M, N, K, dtype)
+    ref = O.sddmm_csr(rowptr, col, val, A, B)
+    _, mag = O.sddmm_csr_f64(rowptr, col, val, A, B)
+    monkeypatch.setenv("SDDMM_LONG_TILES", "1")
+    e = engine_factory()
+    got, st = _run(e, M, N, rowptr, col, val, Ad, Bd, dtype)
+    assert st.mfma_tiles > 0 and st.panels >= 4 and st.strategy_used == capi.AUTO
+    ok, worst, i = O.check_values(got, ref, mag=mag)
+    assert ok, (K, dtype, i, got[i], ref[i], worst)
+    e.run()                                                      # P is built up anew
+    np.testing.assert_array_equal(e.values(), got)
+    monkeypatch.setenv("SDDMM_PANEL_SEG", "67")
+    got, _ = _run(e, M, N, rowptr, col, val, Ad, Bd, dtype)
+    assert O.check_values(got, ref, mag=mag)[0]
+    # non-finite values at the start and the end of a row, and of a turn
+    for k in (0, 127, 128, 255, K - 1):
+        if k < K:
+            A[int(rng.integers(0, M)), k] = np.inf
+            B[int(rng.integers(0, N)), k] = np.nan
+    Ad, Bd = (A, B) if dtype == capi.F32 else [(capi.to_bf16 if dtype == capi.BF16 else capi.to_f16)(x).reshape(x.shape) for x in (A, B)]
+    a, _ = _run(e, M, N, rowptr, col, val, Ad, Bd, dtype)
+    monkeypatch.setenv("SDDMM_LONG_TILES", "0")
+    b, st = _run(e, M, N, rowptr, col, val, Ad, Bd, dtype)
+    assert st.mfma_tiles == 0 and st.panels == 0
+    np.testing.assert_array_equal(np.isnan(a), np.isnan(b))
+    np.testing.assert_array_equal(np.isfinite(a), np.isfinite(b))
+
+
+def test_rows_beyond_1_kib_among_others(engine_factory, monkeypatch):
+    M, N, rowptr, col, val, rng = _structured(5)                 # most entries in rows that nobody owns
+    K = 300
+    Ad, Bd, A, B = _operands(rng, M, N, K, capi.F32)
+    monkeypatch.setenv("SDDMM_LONG_TILES", "1")
+    got, st = _run(engine_factory(), M, N, rowptr, col, val, Ad, Bd, capi.F32)
+    assert st.mfma_tiles == 0 and st.panels == 0
+    ref = O.sddmm_csr(rowptr, col, val, A, B)
+    _, mag = O.sddmm_csr_f64(rowptr, col, val, A, B)
+    assert O.check_values(got, ref, mag=mag)[0]
+
+
 def test_ragged_rows_need_entries(engine_factory):
     """Few entries stay on the gather kernels, whatever their structure; rows beyond 1 KiB do too."""
     M, N, rowptr, col, val, rng = _structured(7, near_dense=20)
