@@ -20,6 +20,7 @@ struct PlanCounters {
     unsigned long long n_tiles, nnz_tiles, tiles_scanned;     // dense-tile path: 16-row and gathered strips
     unsigned long long n_utiles, nnz_utiles, utiles_scanned;  // dense-tile path: union strips
     unsigned long long n_panels, nnz_panels, panel_items;     // row-panel path
+    unsigned long long either_tiles, nnz_either_strip, nnz_either_panels;      // strips of two panels: tiles, entries of either choice
     unsigned int fused_longest;    // fused call: longest row that its gather kernels take
     unsigned int fused_window;     // fused call: most pieces of cut rows among the rows of a wavefront
     unsigned long long rows_alike; // fused call, every fourth row: work-item rows like the next row (its length, its first column)
@@ -34,7 +35,8 @@ enum CounterKind {
     K_ROWS_NONEMPTY = 0,
     K_ROWS_SHORT, K_ROWS_MEDIUM, K_ROWS_LONG, K_NNZ_SHORT, K_NNZ_MEDIUM, K_NNZ_LONG,   // row classifier
     K_ROWS_ALIKE, K_LONGEST, K_WINDOW,                                                 // and for the fused call (two maxima)
-    K_TILES, K_NNZ_TILES, K_UTILES, K_NNZ_UTILES, K_PANELS, K_NNZ_PANELS,              // ownership classifiers
+    K_TILES, K_NNZ_TILES, K_UTILES, K_NNZ_UTILES,                                      // ownership classifiers
+    K_EITHER_TILES, K_NNZ_EITHER_STRIP, K_NNZ_EITHER_PANELS, K_PANELS, K_NNZ_PANELS,
     K_COO_JUMPS,                                                                       // validation of COO entries
     K_COL_PAIRS, K_COL_NEAR,                                                           // and of column indices (a sample)
     K_KINDS
@@ -73,6 +75,8 @@ inline PlanCounters summarize(const DevCounters &d) {
     p.n_tiles = sum[K_TILES]; p.nnz_tiles = sum[K_NNZ_TILES];
     p.n_utiles = sum[K_UTILES]; p.nnz_utiles = sum[K_NNZ_UTILES]; p.utiles_scanned = d.utiles_scanned;
     p.n_panels = sum[K_PANELS]; p.nnz_panels = sum[K_NNZ_PANELS];
+    p.either_tiles = sum[K_EITHER_TILES];
+    p.nnz_either_strip = sum[K_NNZ_EITHER_STRIP]; p.nnz_either_panels = sum[K_NNZ_EITHER_PANELS];
     for (int s = 0; s < SPREAD; ++s) {
         p.fused_longest = std::max(p.fused_longest, (unsigned int)d.k[K_LONGEST][s]);
         p.fused_window = std::max(p.fused_window, (unsigned int)d.k[K_WINDOW][s]);

@@ -465,9 +465,11 @@ constexpr int TILE_WINDOW = 4;                  // descriptors per window (what 
 // The classifiers of a plan in one launch: a wavefront looks at a 16-row strip (dense tiles), then at its two 8-row panels;
 // the workgroup looks together at those of its four strips that could be union strips (their bitmap takes the LDS of all
 // four); the first wavefront then offers the rows that are left to the gathered strips and classifies them.  As five
-// launches they read the row pointer five times and waited for each other: OWN_FIGURES
+// launches they read the row pointer five times and waited for each other (new pattern
+// with every call: 36 000 banded rows 226 -> 188 us, 30 000 near-dense and short rows 199 -> 180).
 struct OwnRules {
     int strip_fill, panel_min, union_fill, cand_min;     // 0: not looked for
+    int panels_below;                                     // entries per tile from which a strip of two panels stays a strip
     int pseg;                                             // entries of a panel's work items
     int ts, seg;                                          // row classes (k_classify_count)
 };
@@ -515,22 +517,38 @@ static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_own_rows(con
         int owned = 0;                                                    // lane < 16: owner of its row
         int tiles = 0, items[2] = {0, 0};
         if (rules.strip_fill) tiles = strip_tiles_of(rowptr, col, M, strip, lane_rp, e0, e1, rules.strip_fill, bm_all + wv * STRIP_BM_WORDS);
-        if (tiles) owned = 1;
-        else if (rules.panel_min) {
+        // A strip of two panels stays a strip where its tiles are well filled.
+        if (rules.panel_min) {
+            int list[2];
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int s0 = __builtin_amdgcn_readlane(lane_rp, 8 * h), l0 = __builtin_amdgcn_readlane(len, 8 * h);
                 const bool alike = (__ballot(len == l0) >> (8 * h) & 0xFFull) == 0xFFull;
-                if (strip * 16 + 8 * h + 8 <= M && l0 >= rules.panel_min && alike && same_lists(col, s0, l0)) {
-                    items[h] = (l0 + rules.pseg - 1) / rules.pseg;
-                    if (lane >> 3 == h) owned = 2;
-                    if (lane == 0) {
-                        spread_add(pc, K_PANELS, 1ull);
-                        spread_add(pc, K_NNZ_PANELS, (unsigned long long)l0 * 8ull);
-                    }
+                const bool panel = !(tiles && h && !items[0]) && strip * 16 + 8 * h + 8 <= M && l0 >= rules.panel_min && alike &&
+                                   same_lists(col, s0, l0);
+                items[h] = panel ? (l0 + rules.pseg - 1) / rules.pseg : 0;
+                list[h] = l0;
+            }
+            if (tiles && items[0] && items[1]) {
+                const bool panels = (int64_t)e1 - e0 < (int64_t)rules.panels_below * tiles;
+                if (lane == 0) {
+                    spread_add(pc, K_EITHER_TILES, (unsigned long long)tiles);
+                    spread_add(pc, panels ? K_NNZ_EITHER_PANELS : K_NNZ_EITHER_STRIP, (unsigned long long)(e1 - e0));
+                }
+                if (panels) tiles = 0;
+                else items[0] = items[1] = 0;
+            } else if (tiles) items[0] = items[1] = 0;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                if (!items[h]) continue;
+                if (lane >> 3 == h) owned = 2;
+                if (lane == 0) {
+                    spread_add(pc, K_PANELS, 1ull);
+                    spread_add(pc, K_NNZ_PANELS, (unsigned long long)list[h] * 8ull);
                 }
             }
         }
+        if (tiles) owned = 1;
         int lo = 0, span = 0, allowed = 0;
         if (rules.union_fill) {
             // the strip must be free as a whole, and even its longest row alone must not need
@@ -2251,7 +2269,7 @@ void k_panel_mfma(const RowItem *__restrict__ items, int64_t n_items, int64_t nb
     };
     auto compute = [&](const Oper &o) {
         if constexpr (BLOCKS) return f32x4_t{0.f, 0.f, 0.f, 0.f};
-        else if constexpr (R::RAGGED || DT != DT_F32) {
+        else if constexpr (R::RAGGED) {
             // (the gathered rows are the "row" operand)
             uint4 b[STEPS];
 #pragma unroll
@@ -2266,8 +2284,10 @@ void k_panel_mfma(const RowItem *__restrict__ items, int64_t n_items, int64_t nb
                 // compiler pairs every MFMA with one permute and a wait for it (16 LDS round trips
                 // per 16 columns in the wave's dependency chain instead of 4); whole groups of 8 or
                 // 16 permutes ahead of their MFMAs were measured slower than either.
-                __builtin_amdgcn_sched_group_barrier(0x080, 4, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+                if constexpr (DT == DT_F32) {
+                    __builtin_amdgcn_sched_group_barrier(0x080, 4, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+                }
             }
             return acc[0];
         }

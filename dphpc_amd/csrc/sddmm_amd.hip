@@ -565,6 +565,24 @@ bool panel_valu_applicable(const sddmm_ctx *c) {
     return s.unit == 0 ? s.UPL <= 2 : s.UPL == 1;
 }
 
+int panel_steps(const sddmm_ctx *c) { return c->long_rows ? LONG_STEPS : c->ragged ? ragged_steps(c) : panel_mfma_steps(c); }
+
+// Columns per work item of a panel: 512, fewer where an item per panel would leave half of the chip's wavefronts idle.  (The
+// kernel's registers hold 5 wavefronts per SIMD at 128-byte rows, 4 up to 512 bytes, 2 beyond.  512 / this rule: 1 000 panels
+// of 96 columns K = 32 4.9 / 4.0 us, K = 256 13.5 / 11.6; 1 500 of 200 K = 128 20.9 / 17.6, K = 64 12.4 / 12.3; 2 000 of 240
+// K = 32 11.3 / 10.6, K = 256 in halves 42 / 48.)  16-bit rows beyond 128 bytes only where there are very few panels: 1 000
+// of 96 columns K = 128 bf16 5.0 / 5.4, 2 000 of 240 13.7 / 14.8.
+int panel_item_columns(const sddmm_ctx *c) {
+    const int steps = panel_steps(c);
+    const int64_t wavefronts = 1024 * (steps <= 2 ? 5 : steps <= 8 ? 4 : 2), panels = std::max<int64_t>(1, c->sM / PANEL_ROWS);
+    int64_t columns = 512;
+    if ((c->dtype != SDDMM_F32 && steps > 2 ? 8 : 2) * panels <= wavefronts) {
+        const int64_t pieces = wavefronts / panels;                       // of a row of average length
+        columns = std::min<int64_t>(512, (c->nnz / std::max(1, c->sM) / pieces + WAVE - 1) / WAVE * WAVE);
+    }
+    return std::max<int>(WAVE, env_int("SDDMM_PANEL_SEG", (int)columns));
+}
+
 // whether the 8-row panels are looked for, and by which kernel they would be computed
 bool panel_path_applies(sddmm_ctx *c) {
     if (c->nnz == 0 || c->sM < PANEL_ROWS) return false;
@@ -881,10 +899,6 @@ int do_plan(sddmm_ctx *c, int strategy) {
             // and 512 bytes; 64-byte rows keep the older, conservative figure
             const size_t row_bytes = (size_t)c->K * elem_size(c->dtype);
             const int tile_fill = std::max(1, env_int("SDDMM_TILE_FILL", row_bytes <= 64 ? 96 : row_bytes <= 128 ? 80 : 56));
-            // panel items of 512 columns, fewer where the panels are too few for the chip (3 072 items if all entries are in
-            // panels: 4 000 banded rows of 158 entries K = 100 18.9 -> 16.2 us, of 8 000 K = 32 9.9 -> 7.6)
-            const int64_t even = (c->nnz / PANEL_ROWS / 3072 + WAVE - 1) / WAVE * WAVE;
-            const int pseg = std::max(WAVE, env_int("SDDMM_PANEL_SEG", (int)std::min<int64_t>(512, even)));
             c->tile_steps = 0;
             c->long_rows = resolved == SDDMM_AUTO && long_pays(c);
             c->ragged = c->long_rows || (resolved == SDDMM_AUTO && ragged_pays(c));
@@ -893,12 +907,9 @@ int do_plan(sddmm_ctx *c, int strategy) {
                                   !c->long_rows && !(c->ragged && c->dtype == SDDMM_F32 && ragged_steps(c) > 12);
             const bool tiles = resolved != SDDMM_LDS_TILED && tile_path_applies(c);
             OwnRules rules{};
-            // 16-row strips are looked at before the row panels and must not take what the
-            // panel kernel does better (8x8-block rows reach ~80 entries per tile); the
-            // strips gathered after the panels use the measured break-even.  Ragged rows: banded
-            // blocks in narrow bands reach 140 (4 000 rows, panels / tiles: K = 48 7.6 / 17.2 us, K = 24 bf16 3.9 / 8.1),
-            // and strips that are no panels come back as union strips
-            if (tiles) rules.strip_fill = resolved == SDDMM_MFMA_TILE ? 1 : std::max(c->ragged ? 160 : 96, tile_fill);
+            // 16-row strips must not take what the panel kernel does better (8x8-block rows reach ~80 entries per tile, in
+            // narrow bands 190); the strips gathered after the panels use the measured break-even
+            if (tiles) rules.strip_fill = resolved == SDDMM_MFMA_TILE ? 1 : std::max(96, tile_fill);
             if (resolved != SDDMM_MFMA_TILE && panel_path_applies(c)) {
                 rules.panel_min = resolved == SDDMM_LDS_TILED ? 1 : std::max(1, env_int("SDDMM_PANEL_MIN", 16));
                 if (c->panel_mfma) rules.panel_min = std::max(rules.panel_min, 4);       // 16-byte S/P accesses stay inside a row
@@ -906,7 +917,9 @@ int do_plan(sddmm_ctx *c, int strategy) {
             if (tiles && resolved == SDDMM_AUTO && env_int("SDDMM_UNION", 1) != 0)
                 rules.union_fill = std::max(1, env_int("SDDMM_UNION_FILL", tile_fill));
             if (tiles && gathered && c->sM >= 2) rules.cand_min = std::max(16, env_int("SDDMM_GATHERED_MIN", 64));
+            const int pseg = panel_item_columns(c);
             rules.pseg = pseg;
+            rules.panels_below = 192;
             // the rows nobody owns so far are classified in the same launch: most matrices have
             // no gathered strips, and their plan then waits for the device once
             c->ts = rules.ts = std::max(1, env_int("SDDMM_TS", 24));
@@ -923,6 +936,19 @@ int do_plan(sddmm_ctx *c, int strategy) {
             if (rc) return rc;
             rc = fetch_counters(c);
             if (rc) return rc;
+            // Strips that are two panels each, some above the line and some below it: tiles and panels are two launches, so all
+            // of them go the way that their average says.  (Launch us, all strips / mixed / all panels: 2 000 rows in a band,
+            // 155 entries per tile, K = 32 5.2 / 8.6 / 4.2, K = 512 bf16 8.9 / 13.9 / 10.4; 16 000 rows, 174 entries, K = 64
+            // 21.7 / 23.5, K = 256 53 / 58; below the line altogether, 120 entries, 4 000 rows, K = 32 13.3 with a few panels
+            // among strips, 5.0 as panels, K = 512 bf16 37.7 and 15.6.)
+            if (c->pc.nnz_either_strip && c->pc.nnz_either_panels) {
+                const unsigned long long line = (panel_steps(c) >= 12 ? 144ull : 160ull) * c->pc.either_tiles;
+                rules.panels_below = c->pc.nnz_either_strip + c->pc.nnz_either_panels >= line ? 0 : INT_MAX;
+                rc = begin_ownership(c, false);
+                if (!rc) rc = plan_owners(c, rules);
+                if (!rc) rc = fetch_counters(c);
+                if (rc) return rc;
+            }
             rc = take_tile_counts(c);
             if (rc) return rc;
             // The kernels of the other rows take a row of more than 1 KiB an entry at a time: the matrix goes in slices as a

@@ -1,0 +1,109 @@
+"""Who owns a row where the rules of a plan meet: strips that are two panels, panel lists cut for the chip's wavefronts,
+gathered pairs wider than the masks in LDS, classifiers of more rows than one pass, columns too far apart for ragged tiles."""
+import numpy as np
+import pytest
+
+from dphpc_amd import capi
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+f32 = np.float32
+
+
+def _csr(rows):
+    rowptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    return rowptr, np.concatenate(rows).astype(np.int32)
+
+
+def _check(engine_factory, rows, N, K, rng, **counts):
+    M = len(rows)
+    rowptr, col = _csr(rows)
+    val = rng.uniform(-1, 1, len(col)).astype(f32)
+    A, B = rng.uniform(-1, 1, (M, K)).astype(f32), rng.uniform(-1, 1, (N, K)).astype(f32)
+    e = engine_factory()
+    e.set_dense(A, B)
+    e.set_csr(M, N, rowptr, col, val)
+    e.plan(capi.AUTO)
+    st = e.stats()
+    e.run()
+    ref = O.sddmm_csr(rowptr, col, val, A, B, threads=0)
+    _, mag = O.sddmm_csr_f64(rowptr, col, val, A, B)
+    ok, worst, i = O.check_values(e.values(), ref, mag=mag)
+    assert ok, (i, worst)
+    assert st.nnz_mfma + st.nnz_panel + st.nnz_short + st.nnz_medium + st.nnz_long == len(col)
+    for name, want in counts.items():
+        assert getattr(st, name) == want, (name, getattr(st, name), want)
+    e.close()
+    return st
+
+
+@pytest.mark.parametrize("K", [16, 32, 100, 256])
+@pytest.mark.parametrize("full,loose,panels", [(9, 0, False), (0, 9, True), (7, 2, False), (1, 8, True), (1, 0, False),
+                                               (0, 1, True)])
+def test_strips_of_two_panels_go_one_way(engine_factory, monkeypatch, K, full, loose, panels):
+    """full strips fill 80 % of their tiles, loose ones 49 %: tiles or panels, whichever suits the average, never both."""
+    monkeypatch.setenv("SDDMM_RAGGED", "1")
+    rng = np.random.default_rng(100 * full + loose)
+    N, rows = 640, []
+    for k in rng.permutation(full + loose):
+        lo = 16 * int(rng.integers(0, 30))
+        for _ in range(2):
+            inside = np.sort(rng.choice(160, 128 if k < full else 78, replace=False))
+            inside[[0, -1]] = 0, 159
+            rows += [lo + np.unique(inside)] * 8
+    _check(engine_factory, rows, N, K, rng, panels=2 * (full + loose) if panels else 0,
+           mfma_tiles=0 if panels else 10 * (full + loose))
+
+
+@pytest.mark.parametrize("K,groups", [(32, 3), (32, 700), (256, 40)])
+def test_panel_lists_cut_for_the_chip(engine_factory, K, groups):
+    """Lists of 1 .. 1 300 columns in as many panels as leave the chip idle, nearly fill it, or do."""
+    rng = np.random.default_rng(groups)
+    N, rows = 5000, []
+    for length in rng.choice([16, 17, 63, 64, 65, 127, 129, 200, 511, 513, 1300] if groups < 100 else [40, 65, 130], groups):
+        rows += [np.sort(rng.choice(N, int(length), replace=False))] * 8
+    _check(engine_factory, rows, N, K, rng, panels=groups)
+
+
+@pytest.mark.parametrize("N,width", [(60000, 7000), (60000, 6144), (9000, 7000)])
+def test_gathered_pairs_wider_than_the_masks(engine_factory, N, width):
+    """Near-dense rows over more tile columns than k_gathered_tiles has masks for; N = 60 000 leaves no room for the kept
+    bitmaps of the pairs, N = 9 000 does."""
+    rng = np.random.default_rng(width + N)
+    rows = []
+    for i in range(100):
+        rows.append(1000 + np.unique(np.concatenate([[0, width - 1], np.flatnonzero(rng.random(width) < 0.62)])))
+        rows.append(np.sort(rng.choice(N, int(rng.integers(0, 9)), replace=False)))
+    st = _check(engine_factory, rows, N, 32, rng)
+    assert st.mfma_tiles >= 6 * ((width + 15) // 16) and st.panels == 0
+
+
+def test_classifiers_of_many_rows(engine_factory):
+    """More 16-row strips than workgroups of the classifiers: tiles, panels, near-dense and short rows among empty ones."""
+    rng = np.random.default_rng(3)
+    M, N = 1_100_007, 2000
+    empty = np.zeros(0, np.int64)
+    rows = [empty] * M
+    for s in rng.choice(M // 16, 300, replace=False):
+        lo, kind = 16 * int(rng.integers(0, 100)), int(rng.integers(0, 3))
+        own = [lo + np.arange(48)] * 16 if kind == 0 else [np.sort(rng.choice(N, 60, replace=False))] * 8 + [empty] * 8
+        if kind == 2:
+            own = [lo + np.flatnonzero(rng.random(200) < 0.6)] + [rng.choice(N, 3, replace=False) for _ in range(15)]
+            own = [np.sort(r) for r in own]
+        rows[16 * s:16 * s + 16] = own
+    rows[M - 7:] = [np.arange(100, 148)] * 7
+    st = _check(engine_factory, rows, N, 16, rng)
+    assert st.mfma_tiles >= 150 and st.panels >= 50 and st.nnz_short > 0
+
+
+@pytest.mark.parametrize("near", [False, True])
+def test_ragged_tiles_where_columns_are_near(engine_factory, near):
+    """Rows of no whole number of 64-byte steps: looked at for tiles only where neighbours tend to share a tile."""
+    rng = np.random.default_rng(11)
+    N, rows = 40000, []
+    for i in range(4000):
+        lo = 16 * int(rng.integers(0, N // 16 - 8))
+        rows.append(lo + np.arange(80) if near else np.sort(rng.choice(N, 80, replace=False)))
+    rows[:64] = [np.arange(256)] * 64
+    st = _check(engine_factory, rows, N, 75, rng)
+    assert (st.mfma_tiles > 0) == near
