@@ -47,6 +47,44 @@ __device__ __forceinline__ int waves_in_block() { return (int)(blockDim.x >> 6);
 // index of the wavefront inside its workgroup, as a scalar
 __device__ __forceinline__ int wave_in_block() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
+// ---- 16-lane helpers (a strip is walked by 16 neighbouring lanes) -------------
+template <int CTRL>
+__device__ __forceinline__ int dpp_i32(int v) {
+    return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, false);
+}
+__device__ __forceinline__ int min16(int v) {
+    int o;
+    o = dpp_i32<DPP_QUAD_XOR1>(v); v = o < v ? o : v;
+    o = dpp_i32<DPP_QUAD_XOR2>(v); v = o < v ? o : v;
+    o = dpp_i32<DPP_ROW_HALF_MIRROR>(v); v = o < v ? o : v;
+    o = dpp_i32<DPP_ROW_MIRROR>(v); v = o < v ? o : v;
+    return v;
+}
+__device__ __forceinline__ int sum16(int v) {
+    v += dpp_i32<DPP_QUAD_XOR1>(v);
+    v += dpp_i32<DPP_QUAD_XOR2>(v);
+    v += dpp_i32<DPP_ROW_HALF_MIRROR>(v);
+    v += dpp_i32<DPP_ROW_MIRROR>(v);
+    return v;
+}
+
+// Sums over a wavefront in the vector unit, all 64 lanes active.  (As six __shfl steps through the LDS crossbar: k_own_rows of
+// 29 000 rows 18.2 us, so 16.5; k_scan_jobs 5.8 and 5.2.)
+__device__ __forceinline__ int wave_sum_i32(int v) {
+    v = sum16(v);
+    return (__builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16)) +
+           (__builtin_amdgcn_readlane(v, 32) + __builtin_amdgcn_readlane(v, 48));
+}
+__device__ __forceinline__ int wave_inclusive_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);       // row_shr:1, 2, 4, 8: within 16 lanes
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);       // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);       // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 // LDS that only one wavefront touches: its LDS operations execute in program order, so a
 // write followed by a read of another lane's slot needs no workgroup barrier, only that the
 // compiler keeps the order.

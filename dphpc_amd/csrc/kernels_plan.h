@@ -189,7 +189,8 @@ static __global__ __launch_bounds__(256) void k_check_index(const int32_t *__res
     // atomics: 14 M entries 13 us, 24 with 1 700 of them)
     const unsigned int each = gridDim.x > SPREAD ? gridDim.x / SPREAD : 1u;
     if (blockIdx.x % each == 0) {
-        for (int o = 1; o < WAVE; o <<= 1) { pairs += __shfl_xor(pairs, o, WAVE); near += __shfl_xor(near, o, WAVE); }
+        pairs = wave_sum_i32(pairs);
+        near = wave_sum_i32(near);
         if (lane_id() == 0) {
             atomicAdd(&pc->k[K_COL_PAIRS][(blockIdx.x / each) & (SPREAD - 1)], (unsigned long long)pairs);
             atomicAdd(&pc->k[K_COL_NEAR][(blockIdx.x / each) & (SPREAD - 1)], (unsigned long long)near);
@@ -322,11 +323,7 @@ __device__ __forceinline__ void row_lengths(const int32_t *__restrict__ rowptr, 
 __device__ __forceinline__ unsigned int block_exclusive_scan(unsigned int v, unsigned int *total) {
     __shared__ unsigned int wave_sums[SCAN_BLOCK / WAVE];
     const int lane = lane_id(), wid = threadIdx.x >> 6;
-    unsigned int incl = v;
-    for (int o = 1; o < WAVE; o <<= 1) {
-        const unsigned int up = __shfl_up(incl, o, WAVE);
-        if (lane >= o) incl += up;
-    }
+    const unsigned int incl = (unsigned int)wave_inclusive_sum((int)v);
     if (lane == WAVE - 1) wave_sums[wid] = incl;
     __syncthreads();
     unsigned int before = 0, all = 0;
@@ -576,11 +573,7 @@ static __global__ __launch_bounds__(256) void k_piece_places(const int32_t *__re
     }
     if (!__ballot(n != 0)) return;
     const int lane = lane_id();
-    unsigned int incl = n;
-    for (int o = 1; o < WAVE; o <<= 1) {
-        const unsigned int up = __shfl_up(incl, o, WAVE);
-        if (lane >= o) incl += up;
-    }
+    const unsigned int incl = (unsigned int)wave_inclusive_sum((int)n);
     unsigned int first = 0;
     if (lane == WAVE - 1) first = (unsigned int)atomicAdd(&pc->fused_pieces, (unsigned long long)incl);
     first = __shfl(first, WAVE - 1, WAVE) + incl - n;

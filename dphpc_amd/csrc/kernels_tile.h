@@ -35,27 +35,6 @@ struct alignas(16) TileDesc {
 };
 static_assert(sizeof(TileDesc) == 112, "TileDesc layout");
 
-// ---- 16-lane helpers (a strip is walked by 16 neighbouring lanes) -------------
-template <int CTRL>
-__device__ __forceinline__ int dpp_i32(int v) {
-    return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, false);
-}
-__device__ __forceinline__ int min16(int v) {
-    int o;
-    o = dpp_i32<DPP_QUAD_XOR1>(v); v = o < v ? o : v;
-    o = dpp_i32<DPP_QUAD_XOR2>(v); v = o < v ? o : v;
-    o = dpp_i32<DPP_ROW_HALF_MIRROR>(v); v = o < v ? o : v;
-    o = dpp_i32<DPP_ROW_MIRROR>(v); v = o < v ? o : v;
-    return v;
-}
-__device__ __forceinline__ int sum16(int v) {
-    v += dpp_i32<DPP_QUAD_XOR1>(v);
-    v += dpp_i32<DPP_QUAD_XOR2>(v);
-    v += dpp_i32<DPP_ROW_HALF_MIRROR>(v);
-    v += dpp_i32<DPP_ROW_MIRROR>(v);
-    return v;
-}
-
 // Walks the tiles of one strip in increasing tile column.  All 16 lanes of the
 // strip call on_tile(tj, first, mask) together; `first` / `mask` are this lane's
 // row's first position and column mask in the tile (mask 0: row absent).  The walk
@@ -155,9 +134,24 @@ constexpr int STRIP_BM_WORDS = 1024;          // 32768 tile columns: a span of 5
 constexpr int STRIP_UNROLL = 4;               // loads of 256 entries per batch, two batches in flight
 constexpr int STRIPS_PER_BLOCK = 4;
 
-__device__ __forceinline__ int wave_sum_i32(int v) {
-    for (int o = WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-    return v;
+// N * 256 entries from base on, four per lane and load; past e1 the last one, or anything in whole loads past it.
+constexpr int PER_LOAD = WAVE * 4;
+template <int N>
+__device__ __forceinline__ void load_entries(const int32_t *__restrict__ col, int base, int e1, I4u (&c)[N]) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        const int b = base + u * PER_LOAD, i0 = b + 4 * lane_id(), last = e1 - 1;
+        if (b + PER_LOAD <= e1) {                                 // wave-uniform: every lane's four entries exist
+            c[u] = *reinterpret_cast<const I4u *>(col + i0);
+        } else if (b < e1 || u == 0) {                            // the last load: clamped, entry by entry
+            c[u].x = col[i0 < last ? i0 : last];
+            c[u].y = col[i0 + 1 < last ? i0 + 1 : last];
+            c[u].z = col[i0 + 2 < last ? i0 + 2 : last];
+            c[u].w = col[i0 + 3 < last ? i0 + 3 : last];
+        } else {
+            c[u] = I4u{0, 0, 0, 0};
+        }
+    }
 }
 
 // Streams entries [e0, e1).  Returns the number of tile-column changes, or -1 as
@@ -173,27 +167,9 @@ template <int BITS>
 __device__ __forceinline__ int64_t strip_scan(const int32_t *__restrict__ col, int e0, int e1, int64_t budget,
                                               int lo, int span, unsigned int *bm, int64_t *descents) {
     const int lane = lane_id();
-    constexpr int PER_LOAD = WAVE * 4;
     constexpr int BATCH = PER_LOAD * STRIP_UNROLL;
     int64_t changes = 0, desc = 0;
     int carry = -1;                           // column before the batch; -1: entry e0 counts as a change
-    auto load = [&](int base, I4u (&c)[STRIP_UNROLL]) {
-#pragma unroll
-        for (int u = 0; u < STRIP_UNROLL; ++u) {
-            const int b = base + u * PER_LOAD;
-            if (b + PER_LOAD <= e1) {                             // wave-uniform: every lane's four entries exist
-                c[u] = *reinterpret_cast<const I4u *>(col + b + 4 * lane);
-            } else if (b < e1 || u == 0) {                        // the last load of the strip: clamped, entry by entry
-                const int last = e1 - 1, i0 = b + 4 * lane;
-                c[u].x = col[i0 < last ? i0 : last];
-                c[u].y = col[i0 + 1 < last ? i0 + 1 : last];
-                c[u].z = col[i0 + 2 < last ? i0 + 2 : last];
-                c[u].w = col[i0 + 3 < last ? i0 + 3 : last];
-            } else {
-                c[u] = I4u{0, 0, 0, 0};
-            }
-        }
-    };
     auto mark = [&](bool on, int column) {
         if constexpr (BITS == 1) {
             const int t = (column >> 4) - lo;
@@ -204,9 +180,9 @@ __device__ __forceinline__ int64_t strip_scan(const int32_t *__restrict__ col, i
         }
     };
     I4u cur[STRIP_UNROLL], nxt[STRIP_UNROLL];
-    load(e0, cur);
+    load_entries(col, e0, e1, cur);
     for (int base = e0; base < e1; base += BATCH) {
-        load(base + BATCH, nxt);
+        load_entries(col, base + BATCH, e1, nxt);
         int my_changes = 0, my_desc = 0;
 #pragma unroll
         for (int u = 0; u < STRIP_UNROLL; ++u) {
@@ -321,6 +297,59 @@ __device__ __forceinline__ int strip_tiles_of(const int32_t *__restrict__ rowptr
     return take ? (int)tiles : 0;
 }
 
+// The same by a workgroup of 16 wavefronts, a row each (every wavefront must call it; each answers for the whole strip).
+// bm and flags (0, 0) are the workgroup's.
+constexpr int WIDE_BLOCK = 16 * WAVE;
+__device__ __forceinline__ int strip_tiles_of_wide(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int M,
+                                                   int64_t strip, int lane_rp, int e0, int e1, int min_fill, unsigned int *bm,
+                                                   int *flags) {
+    const int lane = lane_id(), wv = wave_in_block();
+    const int64_t entries = (int64_t)e1 - (int64_t)e0, max_tiles = entries / min_fill, budget = 16 * max_tiles;
+    if (max_tiles <= 0) return 0;
+    int64_t descents = 0;
+    int lo, span, allowed;
+    strip_bounds(col, lane_rp, e0, &lo, &span, &allowed);
+    if (span <= 0) return 0;
+    if (span > STRIP_BM_WORDS * 32) {
+        if (wv == 0) {
+            const int tiles = strip_tiles_of(rowptr, col, M, strip, lane_rp, e0, e1, min_fill, bm);
+            if (lane == 0) flags[1] = tiles;
+        }
+        __syncthreads();
+        return flags[1];
+    }
+    const int words = (span + 31) >> 5;
+    for (int w = (int)threadIdx.x; w < words; w += WIDE_BLOCK) bm[w] = 0u;
+    __syncthreads();
+    // (a row's tile columns change at most as often as the strip's, and its first entry has none before it)
+    const int s = __builtin_amdgcn_readlane(lane_rp, wv), e = __builtin_amdgcn_readlane(lane_rp, wv + 1);
+    if (e > s && (strip_scan<1>(col, s, e, budget, lo, span, bm, &descents) < 0 || descents != 0) && lane == 0) atomicOr(&flags[0], 1);
+    __syncthreads();
+    int t = 0;
+    for (int w = (int)threadIdx.x; w < words; w += WIDE_BLOCK) t += __builtin_popcount(bm[w]);
+    t = wave_sum_i32(t);
+    if (lane == 0 && t) atomicAdd(&flags[1], t);
+    __syncthreads();
+    const int tiles = flags[1];
+    return flags[0] == 0 && tiles <= max_tiles && entries >= (int64_t)min_fill * tiles ? tiles : 0;
+}
+
+// The descriptors of a strip too wide for a bitmap, by the merging walk in a wavefront's first 16 lanes.
+__device__ __forceinline__ void walk_descriptors(const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int M, int64_t strip,
+                                                 int64_t at, TileDesc *__restrict__ tiles, int32_t *__restrict__ tile_cols) {
+    const int lane = lane_id();
+    if (lane >= 16) return;
+    (void)walk_strip(rowptr, col, M, strip, lane, [&](int tj, int first, unsigned int mask) {
+        TileDesc *d = tiles + at;
+        d->off[lane] = first;
+        d->mask[lane] = (uint16_t)mask;
+        if (lane == 0) { d->strip = (int32_t)strip; d->tj = tj; d->pad[0] = 1; d->pad[1] = 0; }
+        tile_cols[at * 16 + lane] = tj * 16 + lane;
+        ++at;
+        return true;
+    });
+}
+
 // pass 2 (after the exclusive scan of strip_ntiles into strip_off): strip and tile
 // column of every descriptor, in increasing tile column.  Descriptors of a strip
 // that needs the merging walk are written completely here (pad[0] = 1); the others
@@ -342,18 +371,7 @@ static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_strip_tiles(
     strip_bounds(col, lane_rp, e0, &lo, &span, &allowed);
     const int64_t first_desc = strip_off[strip];
     if (span > STRIP_BM_WORDS * 32) {
-        if (lane < 16) {
-            int64_t at = first_desc;
-            (void)walk_strip(rowptr, col, M, strip, lane, [&](int tj, int first, unsigned int mask) {
-                TileDesc *d = tiles + at;
-                d->off[lane] = first;
-                d->mask[lane] = (uint16_t)mask;
-                if (lane == 0) { d->strip = (int32_t)strip; d->tj = tj; d->pad[0] = 1; d->pad[1] = 0; }
-                tile_cols[at * 16 + lane] = tj * 16 + lane;
-                ++at;
-                return true;
-            });
-        }
+        walk_descriptors(rowptr, col, M, strip, first_desc, tiles, tile_cols);
         return;
     }
     const int words = (span + 31) >> 5;
@@ -367,11 +385,7 @@ static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_strip_tiles(
         const int w = wb + lane;
         unsigned int x = w < words ? bm[w] : 0u;
         const int n = __builtin_popcount(x);
-        int incl = n;
-        for (int o = 1; o < WAVE; o <<= 1) {
-            const int up = __shfl_up(incl, o, WAVE);
-            if (lane >= o) incl += up;
-        }
+        const int incl = wave_inclusive_sum(n);
         int64_t at = run + (incl - n);
         while (x) {
             const int b = __builtin_ctz(x);
@@ -426,11 +440,7 @@ static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_union_tiles(
         const int w = wb + lane;
         unsigned int x = w < words ? bm[w] : 0u;
         const int n = __builtin_popcount(x);
-        int incl = n;
-        for (int o = 1; o < WAVE; o <<= 1) {
-            const int up = __shfl_up(incl, o, WAVE);
-            if (lane >= o) incl += up;
-        }
+        const int incl = wave_inclusive_sum(n);
         int64_t rank = run + (incl - n);
         while (x) {
             const int b = __builtin_ctz(x);
@@ -478,13 +488,14 @@ struct OwnArrays {
     unsigned int *strip_ntiles, *panel_counts, *ustrip_ntiles;
     unsigned long long *cand_keys;
     unsigned int *items, *short_entries, *long_rows;      // per block of the row scan, cleared
+    unsigned int *either;                                 // tiles of a strip that is two panels as well, else 0
 };
 
 // 8 rows from row0 on with one column list?  (Equal lengths make them equally spaced in the CSR arrays: row r starts at
-// s0 + r * len, so the 7 comparisons of one position are independent loads.)
-__device__ __forceinline__ bool same_lists(const int32_t *__restrict__ col, int s0, int len) {
+// s0 + r * len, so the 7 comparisons of one position are independent loads.)  Every parts-th 64 columns of it.
+__device__ __forceinline__ bool same_lists(const int32_t *__restrict__ col, int s0, int len, int part = 0, int parts = 1) {
     bool differ = false;
-    for (int e = lane_id(); e < len; e += WAVE) {
+    for (int e = part * WAVE + lane_id(); e < len; e += parts * WAVE) {
         const int32_t *at = col + s0 + e;
         const int c0 = at[0];
         int d = 0;
@@ -495,28 +506,41 @@ __device__ __forceinline__ bool same_lists(const int32_t *__restrict__ col, int 
     return __ballot(differ) == 0;
 }
 
-static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_own_rows(const int32_t *__restrict__ rowptr,
-                                                                            const int32_t *__restrict__ col, int M,
-                                                                            int64_t n_strips, int strips_per_wave,
-                                                                            OwnRules rules, OwnArrays out, DevCounters *pc) {
+// WIDE: a workgroup of 16 wavefronts per strip, where the strips are long and too few for the chip's wavefronts.  (A
+// wavefront reads 1 024 entries per round trip: 35 strips of 33 000 entries 79 us, so 17.)
+template <bool WIDE>
+static __global__ __launch_bounds__(WIDE ? WIDE_BLOCK : WAVE * STRIPS_PER_BLOCK) void k_own_rows(
+    const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int M, int64_t n_strips, int strips_per_wave,
+    OwnRules rules, OwnArrays out, DevCounters *pc) {
     static_assert(STRIPS_PER_BLOCK == 4 && STRIPS_PER_BLOCK * STRIP_BM_WORDS == UNION_BM_WORDS, "one buffer for both bitmaps");
+    constexpr int STRIPS = WIDE ? 1 : STRIPS_PER_BLOCK, WAVES = WIDE ? 16 : STRIPS_PER_BLOCK;
     __shared__ unsigned int bm_all[UNION_BM_WORDS];
-    __shared__ int rp_of[STRIPS_PER_BLOCK][17], own_of[STRIPS_PER_BLOCK][16];
-    __shared__ int lo_of[STRIPS_PER_BLOCK], span_of[STRIPS_PER_BLOCK], allowed_of[STRIPS_PER_BLOCK];   // span 0: no union strip
+    __shared__ int rp_of[STRIPS][17], own_of[STRIPS][16];
+    __shared__ int lo_of[STRIPS], span_of[STRIPS], allowed_of[STRIPS];   // span 0: no union strip
     __shared__ int found, descents_found;
+    __shared__ int flags[4];                                              // WIDE: strip_tiles_of_wide; lists of a half that differ
     const int lane = lane_id(), wv = wave_in_block(), tid = (int)threadIdx.x;
+    const bool speaks = lane == 0 && (!WIDE || wv == 0);                  // for its strip
+    if (WIDE) {
+        if (tid < 4) flags[tid] = 0;
+        __syncthreads();
+    }
     unsigned int rows_sum[3] = {0, 0, 0}, entries_sum[3] = {0, 0, 0};      // wave 0: short, medium, long
     for (int g = 0; g < strips_per_wave; ++g) {
-        const int64_t first = ((int64_t)blockIdx.x * strips_per_wave + g) * STRIPS_PER_BLOCK;
+        const int64_t first = ((int64_t)blockIdx.x * strips_per_wave + g) * STRIPS;
         if (first >= n_strips) break;                                     // workgroup-uniform
-        const int64_t strip = first + wv, r = strip * 16 + lane;
+        const int64_t strip = first + (WIDE ? 0 : wv), r = strip * 16 + lane;
         const int lane_rp = rowptr[r < M ? r : M];                        // (a strip past the last one has no entries)
         const int e0 = __builtin_amdgcn_readlane(lane_rp, 0), e1 = __builtin_amdgcn_readlane(lane_rp, 16);
         const int next_rp = __shfl_down(lane_rp, 1, WAVE);
         const int len = lane < 16 ? next_rp - lane_rp : 0;
         int owned = 0;                                                    // lane < 16: owner of its row
         int tiles = 0, items[2] = {0, 0};
-        if (rules.strip_fill) tiles = strip_tiles_of(rowptr, col, M, strip, lane_rp, e0, e1, rules.strip_fill, bm_all + wv * STRIP_BM_WORDS);
+        if (rules.strip_fill)
+            tiles = WIDE ? strip_tiles_of_wide(rowptr, col, M, strip, lane_rp, e0, e1, rules.strip_fill, bm_all, flags)
+                         : strip_tiles_of(rowptr, col, M, strip, lane_rp, e0, e1, rules.strip_fill, bm_all + (WIDE ? 0 : wv) * STRIP_BM_WORDS);
+        const unsigned int strip_tiles = (unsigned int)tiles;
+        bool either = false;
         // A strip of two panels stays a strip where its tiles are well filled.
         if (rules.panel_min) {
             int list[2];
@@ -524,14 +548,27 @@ static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_own_rows(con
             for (int h = 0; h < 2; ++h) {
                 const int s0 = __builtin_amdgcn_readlane(lane_rp, 8 * h), l0 = __builtin_amdgcn_readlane(len, 8 * h);
                 const bool alike = (__ballot(len == l0) >> (8 * h) & 0xFFull) == 0xFFull;
-                const bool panel = !(tiles && h && !items[0]) && strip * 16 + 8 * h + 8 <= M && l0 >= rules.panel_min && alike &&
-                                   same_lists(col, s0, l0);
-                items[h] = panel ? (l0 + rules.pseg - 1) / rules.pseg : 0;
+                const bool panel = (WIDE || !(tiles && h && !items[0])) && strip * 16 + 8 * h + 8 <= M && l0 >= rules.panel_min && alike;
+                if (WIDE) {
+                    if (panel && !same_lists(col, s0, l0, wv, WAVES) && lane == 0) atomicOr(&flags[2 + h], 1);
+                    items[h] = panel;
+                } else {
+                    items[h] = panel && same_lists(col, s0, l0);
+                }
                 list[h] = l0;
             }
-            if (tiles && items[0] && items[1]) {
+            if (WIDE) {
+                __syncthreads();
+                items[0] = items[0] && !flags[2];
+                items[1] = items[1] && !flags[3];
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h) items[h] = items[h] ? (list[h] + rules.pseg - 1) / rules.pseg : 0;
+            // (or of one, where the matrix ends after 8 rows)
+            either = tiles && items[0] && (items[1] || strip * 16 + 8 == M);
+            if (either) {
                 const bool panels = (int64_t)e1 - e0 < (int64_t)rules.panels_below * tiles;
-                if (lane == 0) {
+                if (speaks) {
                     spread_add(pc, K_EITHER_TILES, (unsigned long long)tiles);
                     spread_add(pc, panels ? K_NNZ_EITHER_PANELS : K_NNZ_EITHER_STRIP, (unsigned long long)(e1 - e0));
                 }
@@ -542,7 +579,7 @@ static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_own_rows(con
             for (int h = 0; h < 2; ++h) {
                 if (!items[h]) continue;
                 if (lane >> 3 == h) owned = 2;
-                if (lane == 0) {
+                if (speaks) {
                     spread_add(pc, K_PANELS, 1ull);
                     spread_add(pc, K_NNZ_PANELS, (unsigned long long)list[h] * 8ull);
                 }
@@ -560,7 +597,8 @@ static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_own_rows(con
                 if (span > UNION_BM_WORDS * 32) span = 0;
             }
         }
-        if (strip < n_strips && lane == 0) {
+        if (strip < n_strips && speaks) {
+            if (rules.strip_fill && rules.panel_min) out.either[strip] = either ? strip_tiles : 0u;
             if (rules.strip_fill) {
                 out.strip_ntiles[strip] = (unsigned int)tiles;
                 if (tiles) {
@@ -573,23 +611,26 @@ static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_own_rows(con
                 if (2 * strip + 1 < M / 8) out.panel_counts[2 * strip + 1] = (unsigned int)items[1];
             }
         }
-        if (lane < 17) rp_of[wv][lane] = lane_rp;
-        if (lane < 16) own_of[wv][lane] = owned;
-        if (lane == 0) { lo_of[wv] = lo; span_of[wv] = span > 0 ? span : 0; allowed_of[wv] = allowed; }
+        if (!WIDE || wv == 0) {
+            const int at = WIDE ? 0 : wv;
+            if (lane < 17) rp_of[at][lane] = lane_rp;
+            if (lane < 16) own_of[at][lane] = owned;
+            if (lane == 0) { lo_of[at] = lo; span_of[at] = span > 0 ? span : 0; allowed_of[at] = allowed; }
+        }
         __syncthreads();
         if (rules.union_fill) {
-            for (int w = 0; w < STRIPS_PER_BLOCK; ++w) {
+            for (int w = 0; w < STRIPS; ++w) {
                 const int u_span = span_of[w];
                 int u_tiles = 0;
                 const int u0 = rp_of[w][0], u1 = rp_of[w][16];
                 if (u_span > 0) {                                         // workgroup-uniform
                     const int words = (u_span + 31) >> 5;
-                    for (int k = tid; k < words; k += WAVE * STRIPS_PER_BLOCK) bm_all[k] = 0u;
+                    for (int k = tid; k < words; k += WAVE * WAVES) bm_all[k] = 0u;
                     if (tid == 0) { found = 0; descents_found = 0; }
                     __syncthreads();
-                    // a quarter of the entries each
+                    // as many entries each
                     const int64_t n = (int64_t)u1 - u0;
-                    const int a = u0 + (int)(n * wv / STRIPS_PER_BLOCK), b = u0 + (int)(n * (wv + 1) / STRIPS_PER_BLOCK);
+                    const int a = u0 + (int)(n * wv / WAVES), b = u0 + (int)(n * (wv + 1) / WAVES);
                     if (b > a) {
                         int64_t descents = 0;
                         (void)strip_scan<2>(col, a, b, INT64_MAX, lo_of[w], u_span, bm_all, &descents);
@@ -598,7 +639,7 @@ static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_own_rows(con
                     }
                     __syncthreads();
                     int t = 0;
-                    for (int k = tid; k < words; k += WAVE * STRIPS_PER_BLOCK) t += __builtin_popcount(bm_all[k]);
+                    for (int k = tid; k < words; k += WAVE * WAVES) t += __builtin_popcount(bm_all[k]);
                     t = wave_sum_i32(t);
                     if (lane == 0 && t) atomicAdd(&found, t);
                     __syncthreads();
@@ -617,10 +658,11 @@ static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_own_rows(con
         if (wv == 0) {
             // one row per lane
             const int64_t row = first * 16 + lane;
-            const int s = rp_of[lane >> 4][lane & 15], n = rp_of[lane >> 4][(lane & 15) + 1] - s;
-            const int who = own_of[lane >> 4][lane & 15];
-            if (row < M) out.owner[row] = (unsigned char)who;
-            const unsigned int l = row < M && who == 0 ? (unsigned int)n : 0u;
+            const bool mine = row < M && lane < 16 * STRIPS;
+            const int at = WIDE ? 0 : lane >> 4, s = rp_of[at][lane & 15], n = rp_of[at][(lane & 15) + 1] - s;
+            const int who = own_of[at][lane & 15];
+            if (mine) out.owner[row] = (unsigned char)who;
+            const unsigned int l = mine && who == 0 ? (unsigned int)n : 0u;
             if (rules.cand_min) {
                 bool cand = l >= (unsigned int)rules.cand_min;
                 int at0 = 0;
@@ -667,6 +709,34 @@ static __global__ __launch_bounds__(WAVE * STRIPS_PER_BLOCK) void k_own_rows(con
             spread_add(pc, K_ROWS_SHORT + k, rows_sum[k]);
             spread_add(pc, K_NNZ_SHORT + k, entries_sum[k]);
         }
+    }
+}
+
+// Strips of two panels that k_own_rows sent either way all go one way, a strip per thread.
+static __global__ __launch_bounds__(256) void k_settle_owners(const int32_t *__restrict__ rowptr, int M, int64_t n_strips,
+                                                              int to_panels, int pseg, OwnArrays out, DevCounters *pc) {
+    const int64_t strip = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const unsigned int tiles = strip < n_strips ? out.either[strip] : 0u;
+    const bool moves = tiles != 0u && (out.strip_ntiles[strip] != 0u) == (to_panels != 0);
+    int entries = 0;
+    int panels = 0;
+    if (moves) {                                               // (two panels, or one at the end of the matrix)
+        out.strip_ntiles[strip] = to_panels ? 0u : tiles;
+        for (; panels < 2 && strip * 16 + 8 * panels + 8 <= M; ++panels) {
+            const int n = rowptr[strip * 16 + 8 * panels + 8] - rowptr[strip * 16 + 8 * panels];
+            entries += n;
+            out.panel_counts[2 * strip + panels] = to_panels ? (unsigned int)((n / 8 + pseg - 1) / pseg) : 0u;
+            for (int r = 0; r < 8; ++r) out.owner[strip * 16 + 8 * panels + r] = to_panels ? 2 : 1;
+        }
+    }
+    if (!__ballot(moves)) return;
+    const unsigned long long all = (unsigned long long)wave_sum_i32(panels);
+    const unsigned long long t = (unsigned long long)wave_sum_i32(moves ? (int)tiles : 0), n = (unsigned long long)wave_sum_i32(entries);
+    if (lane_id() == 0) {                                      // (the sums wrap around: the slots add up to the difference)
+        spread_add(pc, K_TILES, to_panels ? 0ull - t : t);
+        spread_add(pc, K_NNZ_TILES, to_panels ? 0ull - n : n);
+        spread_add(pc, K_PANELS, to_panels ? all : 0ull - all);
+        spread_add(pc, K_NNZ_PANELS, to_panels ? n : 0ull - n);
     }
 }
 
@@ -849,114 +919,91 @@ __device__ __forceinline__ void write_empty_desc(TileDesc *__restrict__ tiles, i
     write_aligned_cols(tile_cols, at, tj);
 }
 
-// pass 2 of the gathered strips: the descriptors, window by window
-// (descriptor 8k + 4h + j of the pair: strip h, the (4k+j)-th tile column).  `tiles` / `tile_cols`
-// point at the first gathered descriptor; the `lead` descriptors before it (fewer than
-// TILE_WINDOW) fill the last window of the strips that precede the gathered ones.
+// The descriptors of a strip, or of a pair of gathered strips window by window (descriptor 8k + 4h + j of the pair: strip h,
+// the (4k+j)-th tile column), from base on, by a workgroup of 16 wavefronts; lds.bm holds the tile columns from lo on.
 // Wave i writes what the descriptors say of rows i and 16+i: it walks the row, marks every entry in the mask of its tile
 // (LDS), and the entries in the masks before a tile tell where the row enters it.  (As a binary search per tile and row
 // afterwards, k_tile_rows: 13.8 us for 20 000 tiles.)
-constexpr int GATHERED_MASKS = 384;                            // tile columns of a pair whose masks fit the LDS
-static __global__ __launch_bounds__(GATHERED_BLOCK) void k_gathered_tiles(
-    const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col,
-    const unsigned long long *__restrict__ sorted_keys,
-    int64_t n_cand, int64_t n_vpairs, const unsigned int *__restrict__ vstrip_ntiles,
-    const unsigned int *__restrict__ vstrip_off, TileDesc *__restrict__ tiles, int32_t *__restrict__ tile_cols,
-    int lead, const unsigned int *__restrict__ kept, int stride) {
-    __shared__ unsigned int bm[STRIP_BM_WORDS];
-    __shared__ int before[STRIP_BM_WORDS];                     // tile columns in the words before
-    __shared__ int unsorted_flag, totals[GATHERED_BLOCK / WAVE], highest;
-    __shared__ unsigned int masks[GATHERED_BLOCK / WAVE][GATHERED_MASKS];
-    const int64_t vp = blockIdx.x;
-    // (strip -1 is nobody's: the window that holds them is walked tile by tile, and they write nothing)
-    if (vp == 0 && (int)threadIdx.x < lead) write_empty_desc(tiles, tile_cols, -(int64_t)lead + threadIdx.x, -1, 0);
-    const unsigned int per_strip = vstrip_ntiles[2 * vp];
-    if (per_strip == 0) return;                      // workgroup-uniform
-    const int lane = lane_id(), wv = wave_in_block();
-    int lo, words, row_s, row_e;                               // lanes 0..31: a row of the pair each
-    if (stride) {
-        const unsigned int *from = kept + vp * stride;
-        lo = (int)from[0];
-        words = ((int)from[1] + 31) >> 5;
-        const int64_t idx = vp * 32 + lane;
-        const int row = lane < 32 && idx < n_cand ? (int)(unsigned int)sorted_keys[idx] : -1;
-        for (int w = (int)threadIdx.x; w < words; w += GATHERED_BLOCK) bm[w] = from[2 + w];
-        row_s = row >= 0 ? rowptr[row] : 0;
-        row_e = row >= 0 ? rowptr[row + 1] : 0;
-    } else {
-        const GatheredHead h = gathered_head(rowptr, col, sorted_keys, n_cand, vp);
-        (void)gathered_mark(col, h, bm, &unsorted_flag);
-        lo = h.lo;
-        words = (h.span + 31) >> 5;
-        row_s = h.s;
-        row_e = h.e;
-    }
+constexpr int GATHERED_MASKS = 384;                            // tile columns whose masks fit the LDS
+struct DescriptorLds {
+    unsigned int bm[STRIP_BM_WORDS];
+    int before[STRIP_BM_WORDS];                                // tile columns in the words before
+    int totals[16], highest, unsorted;
+    unsigned int masks[16][GATHERED_MASKS];
+};
+template <bool PAIR>
+__device__ __forceinline__ void write_descriptors(const int32_t *__restrict__ col, int row_s, int row_e, int lo, int words, int per_strip,
+                                                  int strip0, int64_t base, TileDesc *__restrict__ tiles,
+                                                  int32_t *__restrict__ tile_cols, DescriptorLds &lds) {
     __syncthreads();
     // one thread per word: tile columns in the words before it
     static_assert(STRIP_BM_WORDS <= GATHERED_BLOCK, "one word per thread");
-    const int t = (int)threadIdx.x;
-    const unsigned int mine = t < words ? bm[t] : 0u;
+    const int t = (int)threadIdx.x, lane = lane_id(), wv = wave_in_block();
+    const unsigned int mine = t < words ? lds.bm[t] : 0u;
     const int n = __builtin_popcount(mine);
-    int incl = n;
-    for (int o = 1; o < WAVE; o <<= 1) {
-        const int up = __shfl_up(incl, o, WAVE);
-        if (lane >= o) incl += up;
-    }
-    if (lane == WAVE - 1) totals[wv] = incl;
-    if (t == 0) highest = -1;
+    const int incl = wave_inclusive_sum(n);
+    if (lane == WAVE - 1) lds.totals[wv] = incl;
+    if (t == 0) lds.highest = -1;
     __syncthreads();
     int run = incl - n, all = 0;
     for (int w = 0; w < GATHERED_BLOCK / WAVE; ++w) {
-        run += w < wv ? totals[w] : 0;
-        all += totals[w];
+        run += w < wv ? lds.totals[w] : 0;
+        all += lds.totals[w];
     }
-    if (t < words) before[t] = run;
-    if (mine) atomicMax(&highest, t * 32 + 31 - __builtin_clz(mine));
+    if (t < words) lds.before[t] = run;
+    if (mine) atomicMax(&lds.highest, t * 32 + 31 - __builtin_clz(mine));
     __syncthreads();
-    const int64_t base = vstrip_off[2 * vp];
-    const int strip0 = GATHERED_BASE + (int)(2 * vp);
-    auto place = [&](int rank) { return base + 2 * TILE_WINDOW * (rank / TILE_WINDOW) + (rank % TILE_WINDOW); };
+    auto place = [&](int rank) { return PAIR ? base + 2 * TILE_WINDOW * (rank / TILE_WINDOW) + (rank % TILE_WINDOW) : base + rank; };
     auto put = [&](int rank, int tj) {
         const int64_t at = place(rank);
         *reinterpret_cast<int4 *>(tiles + at) = make_int4(strip0, tj, 1, 0);
         write_aligned_cols(tile_cols, at, tj);
-        *reinterpret_cast<int4 *>(tiles + at + TILE_WINDOW) = make_int4(strip0 + 1, tj, 1, 0);
-        write_aligned_cols(tile_cols, at + TILE_WINDOW, tj);
+        if (PAIR) {
+            *reinterpret_cast<int4 *>(tiles + at + TILE_WINDOW) = make_int4(strip0 + 1, tj, 1, 0);
+            write_aligned_cols(tile_cols, at + TILE_WINDOW, tj);
+        }
     };
     // one thread per tile column of the span
     for (int b = t; b < words * 32; b += GATHERED_BLOCK) {
-        const unsigned int x = bm[b >> 5], bit = 1u << (b & 31);
-        if (x & bit) put(before[b >> 5] + __builtin_popcount(x & (bit - 1u)), lo + b);
+        const unsigned int x = lds.bm[b >> 5], bit = 1u << (b & 31);
+        if (x & bit) put(lds.before[b >> 5] + __builtin_popcount(x & (bit - 1u)), lo + b);
     }
     // the padding: tile columns beyond the pair's last one, which no row of the pair has (the masks come out empty, the
     // positions say where the row ends)
-    if (all + t < (int)per_strip) put(all + t, lo + highest + 1 + t);
+    if (all + t < per_strip) put(all + t, lo + lds.highest + 1 + t);
     // the rows' part of the descriptors
     auto rank_of = [&](int c) {
         const int b = (c >> 4) - lo;
-        return before[b >> 5] + __builtin_popcount(bm[b >> 5] & ((1u << (b & 31)) - 1u));
+        return lds.before[b >> 5] + __builtin_popcount(lds.bm[b >> 5] & ((1u << (b & 31)) - 1u));
     };
-    unsigned int *mk = masks[wv];
-    for (int half = 0; half < 2; ++half) {
+    unsigned int *mk = lds.masks[wv];
+    for (int half = 0; half < (PAIR ? 2 : 1); ++half) {
         const int s = __builtin_amdgcn_readlane(row_s, (wv & 15) + 16 * half), e = __builtin_amdgcn_readlane(row_e, (wv & 15) + 16 * half);
         int at = s;                                            // where the row enters the next tile
         // (a pair of more tile columns than there is room for: some of them at a time)
-        for (int r0 = 0; r0 < (int)per_strip; r0 += GATHERED_MASKS) {
-            const int n_here = (int)per_strip - r0 < GATHERED_MASKS ? (int)per_strip - r0 : GATHERED_MASKS;
+        for (int r0 = 0; r0 < per_strip; r0 += GATHERED_MASKS) {
+            const int n_here = per_strip - r0 < GATHERED_MASKS ? per_strip - r0 : GATHERED_MASKS;
             for (int k = lane; k < n_here; k += WAVE) mk[k] = 0u;
             wave_lds_order();
-            constexpr int AHEAD = 10;
-            for (int p = s; p < e; p += AHEAD * WAVE) {
-                int c[AHEAD];
+            // (the entries of a tile that one lane holds as one: neighbours in one word of LDS wait for each other)
+            constexpr int AHEAD = 4;
+            for (int p = s; p < e; p += AHEAD * PER_LOAD) {
+                I4u c[AHEAD];
+                load_entries(col, p, e, c);
 #pragma unroll
                 for (int u = 0; u < AHEAD; ++u) {
-                    const int q = p + u * WAVE + lane;
-                    c[u] = col[q < e ? q : e - 1];
-                }
+                    const int i0 = p + u * PER_LOAD + 4 * lane;
+                    const int q[4] = {c[u].x, c[u].y, c[u].z, c[u].w};
+                    unsigned int m = 0;
 #pragma unroll
-                for (int u = 0; u < AHEAD; ++u) {
-                    const int k = rank_of(c[u]) - r0;
-                    if (p + u * WAVE + lane < e && (unsigned int)k < (unsigned int)n_here) atomicOr(&mk[k], 1u << (c[u] & 15));
+                    for (int j = 0; j < 4; ++j) {
+                        m |= 1u << (q[j] & 15);
+                        if (i0 + j < e && (j == 3 || i0 + j + 1 >= e || (q[j < 3 ? j + 1 : 3] >> 4) != (q[j] >> 4))) {
+                            const int k = rank_of(q[j]) - r0;
+                            if ((unsigned int)k < (unsigned int)n_here) atomicOr(&mk[k], m);
+                            m = 0;
+                        }
+                    }
                 }
             }
             wave_lds_order();
@@ -964,11 +1011,7 @@ static __global__ __launch_bounds__(GATHERED_BLOCK) void k_gathered_tiles(
                 const int k = k0 + lane;
                 const unsigned int m = k < n_here ? mk[k] : 0u;
                 const int n_in = __builtin_popcount(m);
-                int upto = n_in;
-                for (int o = 1; o < WAVE; o <<= 1) {
-                    const int up = __shfl_up(upto, o, WAVE);
-                    if (lane >= o) upto += up;
-                }
+                const int upto = wave_inclusive_sum(n_in);
                 if (k < n_here) {
                     TileDesc *d = tiles + place(r0 + k) + half * TILE_WINDOW;
                     d->off[wv & 15] = at + upto - n_in;
@@ -979,6 +1022,70 @@ static __global__ __launch_bounds__(GATHERED_BLOCK) void k_gathered_tiles(
             wave_lds_order();                                  // (the masks of the next columns or row)
         }
     }
+}
+
+// pass 2 of the strips where there are few of them: a workgroup per strip, complete descriptors.
+static __global__ __launch_bounds__(WIDE_BLOCK) void k_strip_tiles_wide(
+    const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col, int M,
+    const unsigned int *__restrict__ strip_ntiles, const unsigned int *__restrict__ strip_off,
+    TileDesc *__restrict__ tiles, int32_t *__restrict__ tile_cols) {
+    __shared__ DescriptorLds lds;
+    const int64_t strip = blockIdx.x;
+    const int per_strip = (int)strip_ntiles[strip];
+    if (per_strip == 0) return;                                // workgroup-uniform
+    const int lane = lane_id(), wv = wave_in_block();
+    const int64_t r = strip * 16 + lane;
+    const int row_s = rowptr[r < M ? r : M], row_e = __shfl_down(row_s, 1, WAVE);
+    int lo, span, allowed;
+    strip_bounds(col, row_s, __builtin_amdgcn_readlane(row_s, 0), &lo, &span, &allowed);
+    if (span > STRIP_BM_WORDS * 32) {
+        if (wv == 0) walk_descriptors(rowptr, col, M, strip, strip_off[strip], tiles, tile_cols);
+        return;
+    }
+    const int words = (span + 31) >> 5;
+    for (int w = (int)threadIdx.x; w < words; w += WIDE_BLOCK) lds.bm[w] = 0u;
+    __syncthreads();
+    const int s = __builtin_amdgcn_readlane(row_s, wv), e = __builtin_amdgcn_readlane(row_e, wv);
+    int64_t descents;
+    if (e > s) (void)strip_scan<1>(col, s, e, INT64_MAX, lo, span, lds.bm, &descents);
+    write_descriptors<false>(col, row_s, row_e, lo, words, per_strip, (int)strip, strip_off[strip], tiles, tile_cols, lds);
+}
+
+// pass 2 of the gathered strips.  `tiles` / `tile_cols`
+// point at the first gathered descriptor; the `lead` descriptors before it (fewer than
+// TILE_WINDOW) fill the last window of the strips that precede the gathered ones.
+static __global__ __launch_bounds__(GATHERED_BLOCK) void k_gathered_tiles(
+    const int32_t *__restrict__ rowptr, const int32_t *__restrict__ col,
+    const unsigned long long *__restrict__ sorted_keys,
+    int64_t n_cand, int64_t n_vpairs, const unsigned int *__restrict__ vstrip_ntiles,
+    const unsigned int *__restrict__ vstrip_off, TileDesc *__restrict__ tiles, int32_t *__restrict__ tile_cols,
+    int lead, const unsigned int *__restrict__ kept, int stride) {
+    __shared__ DescriptorLds lds;
+    const int64_t vp = blockIdx.x;
+    // (strip -1 is nobody's: the window that holds them is walked tile by tile, and they write nothing)
+    if (vp == 0 && (int)threadIdx.x < lead) write_empty_desc(tiles, tile_cols, -(int64_t)lead + threadIdx.x, -1, 0);
+    const unsigned int per_strip = vstrip_ntiles[2 * vp];
+    if (per_strip == 0) return;                      // workgroup-uniform
+    const int lane = lane_id();
+    int lo, words, row_s, row_e;                               // lanes 0..31: a row of the pair each
+    if (stride) {
+        const unsigned int *from = kept + vp * stride;
+        lo = (int)from[0];
+        words = ((int)from[1] + 31) >> 5;
+        const int64_t idx = vp * 32 + lane;
+        const int row = lane < 32 && idx < n_cand ? (int)(unsigned int)sorted_keys[idx] : -1;
+        for (int w = (int)threadIdx.x; w < words; w += GATHERED_BLOCK) lds.bm[w] = from[2 + w];
+        row_s = row >= 0 ? rowptr[row] : 0;
+        row_e = row >= 0 ? rowptr[row + 1] : 0;
+    } else {
+        const GatheredHead h = gathered_head(rowptr, col, sorted_keys, n_cand, vp);
+        (void)gathered_mark(col, h, lds.bm, &lds.unsorted);
+        lo = h.lo;
+        words = (h.span + 31) >> 5;
+        row_s = h.s;
+        row_e = h.e;
+    }
+    write_descriptors<true>(col, row_s, row_e, lo, words, (int)per_strip, GATHERED_BASE + (int)(2 * vp), vstrip_off[2 * vp], tiles, tile_cols, lds);
 }
 
 // pass 3 (strips and union strips): one thread per (descriptor, row): CSR position of the row's first entry
@@ -1889,6 +1996,38 @@ static __global__ __launch_bounds__(256) void k_window_scatter(const TileDesc *_
     if (w >= n_win) return;
     const unsigned int at = atomicAdd(&cursors[window_bin(tiles, w, strip_span, tile_col_span, RB, CB)], 1u);
     order[at] = (int32_t)w;
+}
+
+// The same by one workgroup where there are few windows (the four launches and their gaps
+// 35 us of a plan more, 340 to 3 000 windows).
+constexpr int WINDOW_ORDER_BLOCK = 1024, WINDOW_ORDER_EACH = 8;
+static __global__ __launch_bounds__(WINDOW_ORDER_BLOCK) void k_window_order(const TileDesc *__restrict__ tiles, int n_win,
+                                                                            int64_t strip_span, int64_t tile_col_span, int RB, int CB,
+                                                                            int32_t *__restrict__ order) {
+    static_assert(WINDOW_BINS <= WINDOW_ORDER_BLOCK, "a bin per thread");
+    __shared__ unsigned int count[WINDOW_BINS], cursor[WINDOW_BINS];
+    const int tid = (int)threadIdx.x;
+    if (tid < WINDOW_BINS) count[tid] = 0u;
+    __syncthreads();
+    int bin[WINDOW_ORDER_EACH];
+#pragma unroll
+    for (int k = 0; k < WINDOW_ORDER_EACH; ++k) {
+        const int w = k * WINDOW_ORDER_BLOCK + tid;
+        bin[k] = w < n_win ? window_bin(tiles, w, strip_span, tile_col_span, RB, CB) : -1;
+    }
+#pragma unroll
+    for (int k = 0; k < WINDOW_ORDER_EACH; ++k)
+        if (bin[k] >= 0) atomicAdd(&count[bin[k]], 1u);
+    __syncthreads();
+    if (tid < WINDOW_BINS) {
+        unsigned int before = 0;
+        for (int i = 0; i < tid; ++i) before += count[i];
+        cursor[tid] = before;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < WINDOW_ORDER_EACH; ++k)
+        if (bin[k] >= 0) order[atomicAdd(&cursor[bin[k]], 1u)] = k * WINDOW_ORDER_BLOCK + tid;
 }
 
 // AUTO in one launch when a matrix has tiles and rows: logical blocks are dealt out

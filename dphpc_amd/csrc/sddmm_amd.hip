@@ -324,17 +324,40 @@ bool tile_path_applies(sddmm_ctx *c) {
 // plan has more to look at (100 k entries in dense tiles K = 21 4.3 us without, 5.3 with; K = 100 6.8 and 4.6).  Entries
 // that hardly ever share 16 columns with their neighbour fill no tile and no near-dense row: the plan need not look
 // (0.02 .. 0.06 in graphs and uniform rows, 0.7 .. 0.95 in the shapes above; 20 000 uniform rows 13 us of a new pattern).
+// Few entries in long fp32 rows: dense tiles only (0.94 and more: 72 k entries K = 171 9.2 -> 6.1 us), panels are too few for
+// a kernel of one or two wavefronts per SIMD (117 of 224 columns K = 200 10.8 us on the gather kernels, 12.7 as panels).
 bool ragged_pays(const sddmm_ctx *c) {
     const int steps = ragged_steps(c), mode = env_int("SDDMM_RAGGED", -1);       // -1: decide here, 0: never, 1: wherever it can
     if (mode >= 0) return mode != 0 && steps != 0;
-    return steps != 0 && c->nnz >= (steps <= 2 ? 1 << 18 : 1 << 16) && c->col_near >= 0.25;
+    const bool few_panels = c->dtype == SDDMM_F32 && steps > 8 && c->nnz < 1 << 18;
+    return steps != 0 && c->nnz >= (steps <= 1 ? 1 << 19 : steps <= 2 ? 1 << 18 : 1 << 16) && c->col_near >= (few_panels ? 0.92 : 0.25);
 }
 
-// Rows of more than 1 KiB on the tile and panel kernels, if they own nearly all of the entries.
+// Gathered strips of ragged rows?  They cost 55 us of a plan more.  Not for little work (a launch without / with them, 64-byte
+// steps times entries: 1 .. 2.3 M 7.2 / 6.6 .. 13.7 / 10.7 us; 6.5 M 40.8 / 25.0; 14 M 85.8 / 30.7; of nine fp32 steps 4.7 M
+// 31.2 / 33.0), not for fp32 rows of more than twelve (a wavefront per SIMD; near-dense rows K = 200 108 us without, 155 with).
+bool ragged_gathers(const sddmm_ctx *c) {
+    const int steps = ragged_steps(c);
+    if (c->long_rows || (c->dtype == SDDMM_F32 && steps > 12)) return false;
+    return env_int("SDDMM_RAGGED", -1) > 0 || c->nnz * steps >= (c->dtype == SDDMM_F32 && steps > 8 ? 1 << 24 : 1 << 22);
+}
+
+// Rows of more than 1 KiB on the tile and panel kernels, if they own nearly all of the entries.  (Slices / panels, which are a
+// launch per 512 bytes: fp32 265 k entries K = 512 22.7 / 33.6 us, 509 k K = 390 36.7 / 42.7, 793 k K = 858 167 / 71; bf16
+// 573 k K = 752 49.3 / 38.3.  Dense tiles, whose entries nearly all have neighbours: 303 k K = 452 30.9 / 14.7.)
 bool long_pays(const sddmm_ctx *c) {
     const int mode = env_int("SDDMM_LONG_TILES", -1);              // -1: decide here, 0: never, 1: wherever it can
     if (!rows_are_long(c) || mode == 0) return false;
-    return mode > 0 || (c->nnz >= 1 << 18 && c->col_near >= 0.5);
+    if (mode > 0) return true;
+    return c->nnz >= (c->col_near >= 0.92 ? 1 << 18 : c->dtype == SDDMM_F32 ? 3 << 18 : 1 << 19) && c->col_near >= 0.5;
+}
+
+// A workgroup of 16 wavefronts per strip, not four strips to a workgroup of four wavefronts: where the chip holds them all at
+// once and a strip is more than two round trips of a wavefront.  (k_own_rows four to a workgroup / one: 66 strips of 6 300
+// entries 22.1 / 14.2 us, 130 of 4 000 22.0 / 16.7, 1 037 of 5 200 25.7 / 65.6.)
+bool strips_are_wide(const sddmm_ctx *c) {
+    const int64_t n_strips = ((int64_t)c->sM + 15) / 16;
+    return n_strips <= 512 && c->nnz >= 2048 * n_strips;
 }
 
 // The rows' owners and, of the rows that are left, the candidates of the gathered strips and the row classes (launches
@@ -347,12 +370,15 @@ int plan_owners(sddmm_ctx *c, const OwnRules &rules) {
     ARENA_HOLDS(c, M, c->cand_cap, "candidate rows");
     ARENA_HOLDS(c, (M + SCAN_TILE - 1) / SCAN_TILE, c->block_sums_cap, "block sums");
     const OwnArrays out{c->d_owner, c->d_strip_ntiles, c->d_panel_counts, c->d_ustrip_ntiles, c->d_cand_keys,
-                        c->d_block_sums, c->d_short_sums, c->d_long_sums};
+                        c->d_block_sums, c->d_short_sums, c->d_long_sums, c->d_vstrip_ntiles};
     // a group of four strips per workgroup, several one after the other where there are more than the chip holds
     const int64_t groups = (n_strips + STRIPS_PER_BLOCK - 1) / STRIPS_PER_BLOCK;
     const int each = (int)std::min<int64_t>(16, std::max<int64_t>(1, groups / 4096));
-    SDDMM_LAUNCH(c, k_own_rows, (groups + each - 1) / each, WAVE * STRIPS_PER_BLOCK, c->d_rowptr, c->d_col, c->sM, n_strips, each,
-                 rules, out, c->d_pc);
+    if (strips_are_wide(c))
+        SDDMM_LAUNCH(c, k_own_rows<true>, n_strips, WIDE_BLOCK, c->d_rowptr, c->d_col, c->sM, n_strips, 1, rules, out, c->d_pc);
+    else
+        SDDMM_LAUNCH(c, k_own_rows<false>, (groups + each - 1) / each, WAVE * STRIPS_PER_BLOCK, c->d_rowptr, c->d_col, c->sM, n_strips,
+                     each, rules, out, c->d_pc);
     LAUNCH_CHECK(c);
     c->panels_flagged = rules.panel_min != 0;
     c->union_counted = rules.union_fill != 0;
@@ -361,6 +387,17 @@ int plan_owners(sddmm_ctx *c, const OwnRules &rules) {
     if (!rc && rules.panel_min) rc = device_scan(c, c->d_panel_counts, c->d_panel_off, M / 8, &c->d_pc->panel_items);
     if (!rc && rules.union_fill) rc = device_scan(c, c->d_ustrip_ntiles, c->d_ustrip_off, n_strips, &c->d_pc->utiles_scanned);
     return rc ? rc : classify_rows_scan(c);
+}
+
+// Strips of two panels that plan_owners sent either way go one way (launches only).
+int settle_owners(sddmm_ctx *c, bool to_panels, int pseg) {
+    const int64_t M = c->sM, n_strips = (M + 15) / 16;
+    const OwnArrays out{c->d_owner, c->d_strip_ntiles, c->d_panel_counts, c->d_ustrip_ntiles, c->d_cand_keys,
+                        c->d_block_sums, c->d_short_sums, c->d_long_sums, c->d_vstrip_ntiles};
+    SDDMM_LAUNCH(c, k_settle_owners, (n_strips + 255) / 256, 256, c->d_rowptr, c->sM, n_strips, (int)to_panels, pseg, out, c->d_pc);
+    LAUNCH_CHECK(c);
+    const int rc = device_scan(c, c->d_strip_ntiles, c->d_strip_off, n_strips, &c->d_pc->tiles_scanned);
+    return rc ? rc : device_scan(c, c->d_panel_counts, c->d_panel_off, M / 8, &c->d_pc->panel_items);
 }
 
 // after a fetch_counters that follows plan_owners (and precedes the gathered strips)
@@ -468,10 +505,17 @@ int plan_window_order(sddmm_ctx *c) {
         ALLOC_TRY(c, c->d_win_order, (size_t)c->n_windows * sizeof(int32_t));
         c->win_order_cap = c->n_windows;
     }
-    if (!c->d_win_bins) ALLOC_TRY(c, c->d_win_bins, (size_t)WINDOW_BINS * sizeof(unsigned int));
-    HIP_TRY(c, hipMemsetAsync(c->d_win_bins, 0, (size_t)WINDOW_BINS * sizeof(unsigned int), c->stream));
     const int64_t strip_span = std::max<int64_t>(1, std::max(((int64_t)c->sM + 15) / 16, c->n_vstrips));
     const int64_t tile_col_span = std::max<int64_t>(1, ((int64_t)c->N + 15) / 16);
+    if (c->n_windows <= WINDOW_ORDER_BLOCK * WINDOW_ORDER_EACH) {
+        SDDMM_LAUNCH(c, k_window_order, 1, WINDOW_ORDER_BLOCK, (const TileDesc *)c->d_tiles, (int)c->n_windows, strip_span, tile_col_span,
+                     RB, CB, c->d_win_order);
+        LAUNCH_CHECK(c);
+        c->use_win_order = true;
+        return SDDMM_OK;
+    }
+    if (!c->d_win_bins) ALLOC_TRY(c, c->d_win_bins, (size_t)WINDOW_BINS * sizeof(unsigned int));
+    HIP_TRY(c, hipMemsetAsync(c->d_win_bins, 0, (size_t)WINDOW_BINS * sizeof(unsigned int), c->stream));
     const unsigned grid = (unsigned)((c->n_windows + 255) / 256);
     SDDMM_LAUNCH(c, k_window_histogram, grid, 256, (const TileDesc *)c->d_tiles, c->n_windows, strip_span, tile_col_span,
                        RB, CB, c->d_win_bins);
@@ -493,11 +537,18 @@ int plan_tiles_fill(sddmm_ctx *c) {
         ALLOC_TRY(c, c->d_tile_cols, (size_t)c->n_tiles * 16 * sizeof(int32_t));
         c->tiles_cap = c->n_tiles;
     }
+    // (1 037 strips, 33 000 tiles: k_strip_tiles and k_tile_rows 40 us, k_strip_tiles_wide 29; 35 strips 48 and 16.5.  Many more
+    // strips than tiles: a workgroup that finds nothing costs 16 wavefronts)
+    const bool strips_complete = ((int64_t)c->sM + 15) / 16 <= 8192;
     if (c->n_tiles_natural > 0) {
         const int64_t n_strips = ((int64_t)c->sM + 15) / 16;
         const unsigned strip_grid = (unsigned)((n_strips + STRIPS_PER_BLOCK - 1) / STRIPS_PER_BLOCK);
-        SDDMM_LAUNCH(c, k_strip_tiles, strip_grid, WAVE * STRIPS_PER_BLOCK, c->d_rowptr,
-                           c->d_col, c->sM, n_strips, c->d_strip_ntiles, c->d_strip_off, c->d_tiles, c->d_tile_cols);
+        if (strips_complete)
+            SDDMM_LAUNCH(c, k_strip_tiles_wide, n_strips, WIDE_BLOCK, c->d_rowptr, c->d_col, c->sM, c->d_strip_ntiles, c->d_strip_off,
+                         c->d_tiles, c->d_tile_cols);
+        else
+            SDDMM_LAUNCH(c, k_strip_tiles, strip_grid, WAVE * STRIPS_PER_BLOCK, c->d_rowptr, c->d_col, c->sM, n_strips,
+                         c->d_strip_ntiles, c->d_strip_off, c->d_tiles, c->d_tile_cols);
         LAUNCH_CHECK(c);
     }
     if (c->n_tiles_union > 0) {
@@ -517,10 +568,11 @@ int plan_tiles_fill(sddmm_ctx *c) {
                            c->gathered_stride);
         LAUNCH_CHECK(c);
     }
-    const int64_t of_strips = c->n_tiles_natural + c->n_tiles_union;       // (the others are complete)
+    const int64_t complete = strips_complete ? c->n_tiles_natural : 0;     // (and the gathered ones)
+    const int64_t of_strips = c->n_tiles_natural + c->n_tiles_union - complete;
     if (of_strips > 0) {
         SDDMM_LAUNCH(c, k_tile_rows, ((of_strips * 16 + 255) / 256), 256, c->d_rowptr, c->d_col, c->sM,
-                     (const int32_t *)c->d_tile_cols, c->d_tiles, of_strips, c->nnz);
+                     (const int32_t *)(c->d_tile_cols + complete * 16), c->d_tiles + complete, of_strips, c->nnz);
         LAUNCH_CHECK(c);
     }
     // windows of TILE_WINDOW descriptors: what a wavefront of the tile kernels takes.  As a batch
@@ -902,9 +954,7 @@ int do_plan(sddmm_ctx *c, int strategy) {
             c->tile_steps = 0;
             c->long_rows = resolved == SDDMM_AUTO && long_pays(c);
             c->ragged = c->long_rows || (resolved == SDDMM_AUTO && ragged_pays(c));
-            // (ragged fp32 rows of more than twelve steps: a wavefront per SIMD; near-dense rows K = 200 108 us without, 155 with)
-            const bool gathered = resolved == SDDMM_AUTO && env_int("SDDMM_GATHERED", 1) != 0 &&
-                                  !c->long_rows && !(c->ragged && c->dtype == SDDMM_F32 && ragged_steps(c) > 12);
+            const bool gathered = resolved == SDDMM_AUTO && env_int("SDDMM_GATHERED", 1) != 0 && (!c->ragged || ragged_gathers(c));
             const bool tiles = resolved != SDDMM_LDS_TILED && tile_path_applies(c);
             OwnRules rules{};
             // 16-row strips must not take what the panel kernel does better (8x8-block rows reach ~80 entries per tile, in
@@ -943,9 +993,7 @@ int do_plan(sddmm_ctx *c, int strategy) {
             // among strips, 5.0 as panels, K = 512 bf16 37.7 and 15.6.)
             if (c->pc.nnz_either_strip && c->pc.nnz_either_panels) {
                 const unsigned long long line = (panel_steps(c) >= 12 ? 144ull : 160ull) * c->pc.either_tiles;
-                rules.panels_below = c->pc.nnz_either_strip + c->pc.nnz_either_panels >= line ? 0 : INT_MAX;
-                rc = begin_ownership(c, false);
-                if (!rc) rc = plan_owners(c, rules);
+                rc = settle_owners(c, c->pc.nnz_either_strip + c->pc.nnz_either_panels < line, pseg);
                 if (!rc) rc = fetch_counters(c);
                 if (rc) return rc;
             }
@@ -956,10 +1004,12 @@ int do_plan(sddmm_ctx *c, int strategy) {
             if (c->long_rows && (int64_t)(c->pc.nnz_tiles + c->pc.nnz_utiles + c->pc.nnz_panels) < c->nnz - c->nnz / 16) {
                 c->ragged = c->long_rows = c->panels_flagged = false;
                 c->tile_steps = 0;
-                rc = begin_ownership(c, true);
-                if (!rc) rc = classify_rows_count(c);
-                if (!rc) rc = fetch_counters(c);
-                if (rc) return rc;
+                if (c->pc.nnz_tiles + c->pc.nnz_utiles + c->pc.nnz_panels) {        // (else the rows are classified as if not looked at)
+                    rc = begin_ownership(c, true);
+                    if (!rc) rc = classify_rows_count(c);
+                    if (!rc) rc = fetch_counters(c);
+                    if (rc) return rc;
+                }
             }
             rc = plan_panels_items(c, pseg);
             if (rc) return rc;

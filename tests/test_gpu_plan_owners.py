@@ -107,3 +107,30 @@ def test_ragged_tiles_where_columns_are_near(engine_factory, near):
     rows[:64] = [np.arange(256)] * 64
     st = _check(engine_factory, rows, N, 75, rng)
     assert (st.mfma_tiles > 0) == near
+
+
+@pytest.mark.parametrize("strips,per_strip", [(64, 1), (255, 128), (257, 128), (600, 64)])
+def test_window_order_by_one_workgroup_and_by_many(engine_factory, monkeypatch, strips, per_strip):
+    """The order of the windows over strips and tile columns: up to 8 192 windows one workgroup sorts, above four launches."""
+    monkeypatch.setenv("SDDMM_WINDOW_ORDER", "1")
+    rng = np.random.default_rng(strips)
+    N, rows = 16 * 2 * per_strip, []
+    for _ in range(strips):
+        tc = np.sort(rng.choice(N // 16, per_strip, replace=False))
+        c = (tc[:, None] * 16 + np.arange(16)[None, :]).ravel()
+        rows += [c[(np.arange(len(c)) + r) % 2 == 0] for r in range(16)]
+    _check(engine_factory, rows, N, 32, rng, mfma_tiles=strips * per_strip)
+
+
+@pytest.mark.parametrize("M", [8, 24, 25, 40])
+def test_a_matrix_that_ends_with_half_a_strip_of_a_panel(engine_factory, M):
+    """8 rows after the last whole strip: they go the way of the strips that are two panels, unless more rows follow."""
+    rng = np.random.default_rng(M)
+    N, rows = 640, []
+    for _ in range((M + 7) // 8):
+        rows += [np.sort(rng.choice(160, 90, replace=False))] * 8
+    rows = rows[:M]
+    st = _check(engine_factory, rows, N, 32, rng)
+    assert st.nnz_panel + st.nnz_mfma >= 90 * (M - 1)
+    if M % 16 == 8:
+        assert st.mfma_tiles == 0 and st.panels == M // 8
