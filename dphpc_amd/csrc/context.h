@@ -52,8 +52,8 @@ struct sddmm_ctx {
     int strategy = SDDMM_AUTO;       // resolved
     int requested = SDDMM_AUTO;
     DevCounters *d_pc = nullptr;     // device counters
-    DevCounters raw{};               // host copy of the device block
-    DevCounters *h_pc = nullptr;     // pinned landing place of the read-back (no staging copy)
+    DevTotals raw{};                 // what the device reported last
+    DevCounters *h_pc = nullptr;     // pinned landing place of the reports and of copies
     PlanCounters pc{};               // its summary
     sddmm_stats stats{};
     // AUTO: rows shorter than ts go to the many-rows-per-wave kernel, the others

@@ -43,6 +43,7 @@ enum CounterKind {
 };
 struct DevCounters {
     unsigned int bad_pattern, coo_unsorted, pad0, pad1;
+    // (from here on in the order of DevTotals)
     unsigned long long n_items, tiles_scanned, panel_items;          // scan totals, one writer each
     unsigned long long n_candidates;                                 // rows offered to the gathered strips
     unsigned long long utiles_scanned, short_scanned;                // scan totals: union strips, entries of the short rows
@@ -57,30 +58,35 @@ __device__ __forceinline__ void spread_add(DevCounters *dc, int kind, unsigned l
     if (v) atomicAdd(&dc->k[kind][blockIdx.x & (SPREAD - 1)], v);
 }
 
-inline PlanCounters summarize(const DevCounters &d) {
+// What the host reads: the scan totals (in the order of DevCounters) and the sums, or maxima, over the slots.  The last launch
+// before the host waits writes it to pinned memory (k_scan_jobs).  (A copy of the slots was a launch and a gap more, and their
+// sum work of the host: new pattern with every call, 30 000 near-dense and short rows 170 us, so 167; graph of 200 000 rows 242
+// and 234.)
+struct DevTotals {
+    unsigned int bad_pattern, coo_unsorted, max_len, pad;
+    unsigned long long n_items, tiles_scanned, panel_items, n_candidates, utiles_scanned, short_scanned, long_scanned;
+    unsigned long long k[K_KINDS];
+};
+constexpr int SCAN_TOTALS = 7;
+
+inline PlanCounters summarize(const DevTotals &d) {
     PlanCounters p{};
     p.bad_pattern = d.bad_pattern;
     p.coo_unsorted = d.coo_unsorted;
-    unsigned long long sum[K_KINDS] = {0};
-    for (int s = 0; s < SPREAD; ++s) {
-        p.max_len = d.max_len[s] > p.max_len ? d.max_len[s] : p.max_len;
-        for (int k = 0; k < K_KINDS; ++k) sum[k] += d.k[k][s];
-    }
-    p.rows_nonempty = sum[K_ROWS_NONEMPTY];
-    p.coo_jumps = sum[K_COO_JUMPS];
-    p.col_pairs = sum[K_COL_PAIRS]; p.col_near = sum[K_COL_NEAR];
-    p.rows_alike = sum[K_ROWS_ALIKE];
-    p.rows_short = sum[K_ROWS_SHORT]; p.rows_medium = sum[K_ROWS_MEDIUM]; p.rows_long = sum[K_ROWS_LONG];
-    p.nnz_short = sum[K_NNZ_SHORT]; p.nnz_medium = sum[K_NNZ_MEDIUM]; p.nnz_long = sum[K_NNZ_LONG];
-    p.n_tiles = sum[K_TILES]; p.nnz_tiles = sum[K_NNZ_TILES];
-    p.n_utiles = sum[K_UTILES]; p.nnz_utiles = sum[K_NNZ_UTILES]; p.utiles_scanned = d.utiles_scanned;
-    p.n_panels = sum[K_PANELS]; p.nnz_panels = sum[K_NNZ_PANELS];
-    p.either_tiles = sum[K_EITHER_TILES];
-    p.nnz_either_strip = sum[K_NNZ_EITHER_STRIP]; p.nnz_either_panels = sum[K_NNZ_EITHER_PANELS];
-    for (int s = 0; s < SPREAD; ++s) {
-        p.fused_longest = std::max(p.fused_longest, (unsigned int)d.k[K_LONGEST][s]);
-        p.fused_window = std::max(p.fused_window, (unsigned int)d.k[K_WINDOW][s]);
-    }
+    p.max_len = d.max_len;
+    p.rows_nonempty = d.k[K_ROWS_NONEMPTY];
+    p.coo_jumps = d.k[K_COO_JUMPS];
+    p.col_pairs = d.k[K_COL_PAIRS]; p.col_near = d.k[K_COL_NEAR];
+    p.rows_alike = d.k[K_ROWS_ALIKE];
+    p.rows_short = d.k[K_ROWS_SHORT]; p.rows_medium = d.k[K_ROWS_MEDIUM]; p.rows_long = d.k[K_ROWS_LONG];
+    p.nnz_short = d.k[K_NNZ_SHORT]; p.nnz_medium = d.k[K_NNZ_MEDIUM]; p.nnz_long = d.k[K_NNZ_LONG];
+    p.n_tiles = d.k[K_TILES]; p.nnz_tiles = d.k[K_NNZ_TILES];
+    p.n_utiles = d.k[K_UTILES]; p.nnz_utiles = d.k[K_NNZ_UTILES]; p.utiles_scanned = d.utiles_scanned;
+    p.n_panels = d.k[K_PANELS]; p.nnz_panels = d.k[K_NNZ_PANELS];
+    p.either_tiles = d.k[K_EITHER_TILES];
+    p.nnz_either_strip = d.k[K_NNZ_EITHER_STRIP]; p.nnz_either_panels = d.k[K_NNZ_EITHER_PANELS];
+    p.fused_longest = (unsigned int)d.k[K_LONGEST];
+    p.fused_window = (unsigned int)d.k[K_WINDOW];
     p.n_items = d.n_items; p.tiles_scanned = d.tiles_scanned; p.panel_items = d.panel_items;
     return p;
 }
@@ -89,12 +95,13 @@ __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
     return v;
 }
+// (values below 2^31)
 __device__ __forceinline__ unsigned int wave_max_u32(unsigned int v) {
-    for (int o = 32; o > 0; o >>= 1) {
-        unsigned int x = __shfl_xor(v, o, WAVE);
-        v = x > v ? x : v;
-    }
-    return v;
+    const int m = min16(-(int)v);
+    const int a = __builtin_amdgcn_readlane(m, 0), b = __builtin_amdgcn_readlane(m, 16);
+    const int c = __builtin_amdgcn_readlane(m, 32), e = __builtin_amdgcn_readlane(m, 48);
+    const int x = a < b ? a : b, y = c < e ? c : e;
+    return (unsigned int)-(x < y ? x : y);
 }
 
 // What a plan clears before its classifiers run, in one launch (a fill through the
@@ -454,7 +461,8 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_small(const unsigned
 }
 
 // Several short scans in one launch: workgroup j takes job j (in == out is allowed: a thread
-// writes only the positions it has read).
+// writes only the positions it has read).  With a place for the totals in host memory, whose jobs' totals are among the
+// first SCAN_TOTALS of DevCounters, one more workgroup reports the counters.
 constexpr int SCAN_JOBS_MAX = 8;
 struct ScanJob {
     const unsigned int *in;
@@ -464,7 +472,44 @@ struct ScanJob {
     int pad;
 };
 struct ScanJobs { ScanJob job[SCAN_JOBS_MAX]; };
-static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_jobs(ScanJobs jobs) {
+// The workgroup after the last job: the counters, but for the totals of this launch's own jobs, which those write.
+__device__ __forceinline__ void report_totals(const ScanJobs &jobs, int n_jobs, const DevCounters *pc,
+                                              DevTotals *__restrict__ totals) {
+    constexpr int WAVES = SCAN_BLOCK / WAVE, EACH = (K_KINDS + WAVES - 1) / WAVES;
+    const int lane = lane_id(), wv = wave_in_block(), tid = (int)threadIdx.x;
+    unsigned long long v[EACH];
+#pragma unroll
+    for (int q = 0; q < EACH; ++q) v[q] = wv + q * WAVES < K_KINDS ? pc->k[wv + q * WAVES][lane] : 0ull;
+    const unsigned int longest = wave_max_u32(pc->max_len[lane]);
+#pragma unroll
+    for (int q = 0; q < EACH; ++q) {
+        const int kind = wv + q * WAVES;
+        if (kind >= K_KINDS) break;
+        // (64 numbers of 24 bits stay below 2^31; what wraps around, as the slots of a difference do, comes out right)
+        unsigned long long sum = (unsigned long long)wave_sum_i32((int)(v[q] & 0xFFFFFF)) +
+                                 ((unsigned long long)wave_sum_i32((int)(v[q] >> 24 & 0xFFFFFF)) << 24) +
+                                 ((unsigned long long)wave_sum_i32((int)(v[q] >> 48)) << 48);
+        if (kind == K_LONGEST || kind == K_WINDOW) sum = wave_max_u32((unsigned int)v[q]);
+        if (lane == 0) totals->k[kind] = sum;
+    }
+    if (tid == 0) {
+        totals->bad_pattern = pc->bad_pattern;
+        totals->coo_unsorted = pc->coo_unsorted;
+        totals->max_len = longest;
+    }
+    if (tid < SCAN_TOTALS) {
+        bool of_a_job = false;
+        for (int j = 0; j < n_jobs; ++j) of_a_job |= jobs.job[j].total == &pc->n_items + tid;
+        if (!of_a_job) (&totals->n_items)[tid] = (&pc->n_items)[tid];
+    }
+}
+
+static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_jobs(ScanJobs jobs, int n_jobs, const DevCounters *pc,
+                                                                 DevTotals *__restrict__ totals) {
+    if ((int)blockIdx.x == n_jobs) {
+        report_totals(jobs, n_jobs, pc, totals);
+        return;
+    }
     const ScanJob jb = jobs.job[blockIdx.x];
     unsigned int carry = 0;
     for (int base = 0; base < jb.n; base += SCAN_BLOCK * SCAN_SMALL_ITEMS) {
@@ -484,7 +529,10 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_jobs(ScanJobs jobs) 
         }
         carry += total;
     }
-    if (threadIdx.x == 0) *jb.total = carry;
+    if (threadIdx.x == 0) {
+        *jb.total = carry;
+        if (totals) (&totals->n_items)[jb.total - &pc->n_items] = carry;
+    }
 }
 
 // The entry list of the short rows: {position, row} of every stored entry of the rows that

@@ -159,7 +159,7 @@ int grid_capped(int64_t n, int block, int cap = 16384) {
 // there instead of one launch each behind its producer.
 int flush_scans(sddmm_ctx *c) {
     if (c->n_scan_jobs == 0) return SDDMM_OK;
-    SDDMM_LAUNCH(c, k_scan_jobs, c->n_scan_jobs, SCAN_BLOCK, c->scan_jobs);
+    SDDMM_LAUNCH(c, k_scan_jobs, c->n_scan_jobs, SCAN_BLOCK, c->scan_jobs, c->n_scan_jobs, (const DevCounters *)c->d_pc, (DevTotals *)nullptr);
     c->n_scan_jobs = 0;
     LAUNCH_CHECK(c);
     return SDDMM_OK;
@@ -173,14 +173,20 @@ int queue_scan(sddmm_ctx *c, const unsigned int *in, unsigned int *out, int64_t 
     return SDDMM_OK;
 }
 
-int fetch_counters(sddmm_ctx *c) {
-    {
-        const int rc = flush_scans(c);
-        if (rc) return rc;
-    }
-    HIP_TRY(c, hipMemcpyAsync(c->h_pc, c->d_pc, sizeof(DevCounters), hipMemcpyDeviceToHost, c->stream));
+// The scans that wait and a report of the counters; waits for it.
+int read_totals(sddmm_ctx *c, DevTotals *out) {
+    static_assert(sizeof(DevTotals) <= sizeof(DevCounters::k), "the slots' place in the pinned block");
+    DevTotals *const totals = reinterpret_cast<DevTotals *>(&c->h_pc->k[0][0]);
+    SDDMM_LAUNCH(c, k_scan_jobs, c->n_scan_jobs + 1, SCAN_BLOCK, c->scan_jobs, c->n_scan_jobs, (const DevCounters *)c->d_pc, totals);
+    c->n_scan_jobs = 0;
+    LAUNCH_CHECK(c);
     HIP_TRY(c, hipStreamSynchronize(c->stream));
-    c->raw = *c->h_pc;
+    *out = *totals;
+    return SDDMM_OK;
+}
+int fetch_counters(sddmm_ctx *c) {
+    const int rc = read_totals(c, &c->raw);
+    if (rc) return rc;
     c->pc = summarize(c->raw);
     return SDDMM_OK;
 }
@@ -1490,7 +1496,7 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
     ARENA_HOLDS(c, nb, c->block_sums_cap, "block sums");
     c->n_fused_items = c->n_fused_pieces = c->n_fused_cut = 0;
     if (nb > 0) {
-        DevCounters tmp;
+        DevTotals tmp;
         PlanCounters counted;
         int window = WAVE / shape_of(c).LPN;               // rows of a wavefront of the kernel of the short rows
         const int32_t *look_at = c->d_col;                 // (which rows are alike: the first count tells)
@@ -1504,10 +1510,9 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
             SDDMM_LAUNCH(c, k_scan_block_sums, 1, SCAN_BLOCK, (const unsigned int *)c->d_block_sums, c->d_block_off, (int)nb,
                                &c->d_pc->n_items);
             LAUNCH_CHECK(c);
-            HIP_TRY(c, hipMemcpyAsync(&tmp, c->d_pc, sizeof(DevCounters), hipMemcpyDeviceToHost, c->stream));
-            HIP_TRY(c, hipStreamSynchronize(c->stream));
+            const int trc = read_totals(c, &tmp);
             counted = summarize(tmp);
-            return SDDMM_OK;
+            return trc;
         };
         int rc = count();
         if (rc) return rc;
