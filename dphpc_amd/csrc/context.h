@@ -324,7 +324,7 @@ inline int64_t short_row_waves(const sddmm_ctx *c) {
 }
 
 // Row-panel detector (8 consecutive rows, 8-aligned, same column list).  Two
-// kernels can run the panels: the MFMA one (row size a multiple of 64 bytes, up to
+// kernels can run the panels: the MFMA one (rows of 36 bytes and more, up to
 // 1 KiB) and the VALU one (8-lanes-per-entry layouts whose 8 A rows fit in
 // registers: fp32 K = 32 or 64, bf16 / fp16 K = 64, 32-bit offsets); the VALU kernel has
 // the per-entry arithmetic of the gather kernels, the MFMA kernel is faster.

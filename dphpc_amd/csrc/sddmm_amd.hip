@@ -377,9 +377,10 @@ int plan_owners(sddmm_ctx *c, const OwnRules &rules) {
     ARENA_HOLDS(c, (M + SCAN_TILE - 1) / SCAN_TILE, c->block_sums_cap, "block sums");
     const OwnArrays out{c->d_owner, c->d_strip_ntiles, c->d_panel_counts, c->d_ustrip_ntiles, c->d_cand_keys,
                         c->d_block_sums, c->d_short_sums, c->d_long_sums, c->d_vstrip_ntiles};
-    // a group of four strips per workgroup, several one after the other where there are more than the chip holds
+    // a group of four strips per workgroup, several one after the other where there are more than the chip holds at a time (five
+    // per CU; a workgroup ends with atomics: graph of 200 000 rows, new pattern with every call 238 us with one group, 222 with two)
     const int64_t groups = (n_strips + STRIPS_PER_BLOCK - 1) / STRIPS_PER_BLOCK;
-    const int each = (int)std::min<int64_t>(16, std::max<int64_t>(1, groups / 4096));
+    const int each = (int)std::min<int64_t>(16, std::max<int64_t>(1, groups / 1280));
     if (strips_are_wide(c))
         SDDMM_LAUNCH(c, k_own_rows<true>, n_strips, WIDE_BLOCK, c->d_rowptr, c->d_col, c->sM, n_strips, 1, rules, out, c->d_pc);
     else
