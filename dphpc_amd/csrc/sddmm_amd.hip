@@ -329,14 +329,12 @@ bool tile_path_applies(sddmm_ctx *c) {
 // near-dense rows K = 75 70 -> 36, K = 120 bf16 49 -> 21.  Few entries: a launch of a few microseconds either way, and the
 // plan has more to look at (100 k entries in dense tiles K = 21 4.3 us without, 5.3 with; K = 100 6.8 and 4.6).  Entries
 // that hardly ever share 16 columns with their neighbour fill no tile and no near-dense row: the plan need not look
-// (0.02 .. 0.06 in graphs and uniform rows, 0.7 .. 0.95 in the shapes above; 20 000 uniform rows 13 us of a new pattern).
-// Few entries in long fp32 rows: dense tiles only (0.94 and more: 72 k entries K = 171 9.2 -> 6.1 us), panels are too few for
-// a kernel of one or two wavefronts per SIMD (117 of 224 columns K = 200 10.8 us on the gather kernels, 12.7 as panels).
+// (0.02 .. 0.06 in graphs and uniform rows, around 0.5 where those have few columns, 0.7 .. 0.95 in the shapes above; 20 000
+// uniform rows 13 us of a new pattern, a graph of 8 600 rows K = 54 85 without, 97 with).
 bool ragged_pays(const sddmm_ctx *c) {
     const int steps = ragged_steps(c), mode = env_int("SDDMM_RAGGED", -1);       // -1: decide here, 0: never, 1: wherever it can
     if (mode >= 0) return mode != 0 && steps != 0;
-    const bool few_panels = c->dtype == SDDMM_F32 && steps > 8 && c->nnz < 1 << 18;
-    return steps != 0 && c->nnz >= (steps <= 1 ? 1 << 19 : steps <= 2 ? 1 << 18 : 1 << 16) && c->col_near >= (few_panels ? 0.92 : 0.25);
+    return steps != 0 && c->nnz >= (steps <= 1 ? 1 << 19 : steps <= 2 ? 1 << 18 : 1 << 16) && c->col_near >= 0.6;
 }
 
 // Gathered strips of ragged rows?  They cost 55 us of a plan more.  Not for little work (a launch without / with them, 64-byte
@@ -348,14 +346,12 @@ bool ragged_gathers(const sddmm_ctx *c) {
     return env_int("SDDMM_RAGGED", -1) > 0 || c->nnz * steps >= (c->dtype == SDDMM_F32 && steps > 8 ? 1 << 24 : 1 << 22);
 }
 
-// Rows of more than 1 KiB on the tile and panel kernels, if they own nearly all of the entries.  (Slices / panels, which are a
-// launch per 512 bytes: fp32 265 k entries K = 512 22.7 / 33.6 us, 509 k K = 390 36.7 / 42.7, 793 k K = 858 167 / 71; bf16
-// 573 k K = 752 49.3 / 38.3.  Dense tiles, whose entries nearly all have neighbours: 303 k K = 452 30.9 / 14.7.)
+// Rows of more than 1 KiB on the tile and panel kernels, if they own nearly all of the entries.  (Slices / dense tiles: 303 k
+// entries K = 452 30.9 / 14.7 us.)
 bool long_pays(const sddmm_ctx *c) {
     const int mode = env_int("SDDMM_LONG_TILES", -1);              // -1: decide here, 0: never, 1: wherever it can
     if (!rows_are_long(c) || mode == 0) return false;
-    if (mode > 0) return true;
-    return c->nnz >= (c->col_near >= 0.92 ? 1 << 18 : c->dtype == SDDMM_F32 ? 3 << 18 : 1 << 19) && c->col_near >= 0.5;
+    return mode > 0 || (c->nnz >= 1 << 18 && c->col_near >= 0.6);
 }
 
 // A workgroup of 16 wavefronts per strip, not four strips to a workgroup of four wavefronts: where the chip holds them all at
@@ -364,6 +360,17 @@ bool long_pays(const sddmm_ctx *c) {
 bool strips_are_wide(const sddmm_ctx *c) {
     const int64_t n_strips = ((int64_t)c->sM + 15) / 16;
     return n_strips <= 512 && c->nnz >= 2048 * n_strips;
+}
+
+// After the classifiers: panels of ragged or long rows, and too few of them for kernels that occupy the chip with one or two
+// wavefronts per SIMD, or that are a launch per 512 bytes.  (Gather kernels / panels: 117 panels of 224 columns, fp32 K = 200
+// 10.8 / 12.7 us, K = 512 309 k entries 24.0 / 33.6, 509 k K = 390 36.7 / 42.7; 577 k K = 196 22.3 / 15.4, 793 k K = 858 167 /
+// 71; bf16 573 k K = 752 49.3 / 38.3.)
+bool too_few_panels(const sddmm_ctx *c) {
+    if (!c->ragged || (int64_t)c->pc.nnz_panels <= c->nnz / 2) return false;
+    const bool f32 = c->dtype == SDDMM_F32;
+    if (c->long_rows) return env_int("SDDMM_LONG_TILES", -1) < 0 && c->nnz < (f32 ? 3 << 18 : 1 << 19);
+    return env_int("SDDMM_RAGGED", -1) < 0 && f32 && ragged_steps(c) > 8 && c->nnz < 1 << 18;
 }
 
 // The rows' owners and, of the rows that are left, the candidates of the gathered strips and the row classes (launches
@@ -1008,7 +1015,7 @@ int do_plan(sddmm_ctx *c, int strategy) {
             if (rc) return rc;
             // The kernels of the other rows take a row of more than 1 KiB an entry at a time: the matrix goes in slices as a
             // whole where strips and panels do not own nearly all of it.
-            if (c->long_rows && (int64_t)(c->pc.nnz_tiles + c->pc.nnz_utiles + c->pc.nnz_panels) < c->nnz - c->nnz / 16) {
+            if ((c->long_rows && (int64_t)(c->pc.nnz_tiles + c->pc.nnz_utiles + c->pc.nnz_panels) < c->nnz - c->nnz / 16) || too_few_panels(c)) {
                 c->ragged = c->long_rows = c->panels_flagged = false;
                 c->tile_steps = 0;
                 if (c->pc.nnz_tiles + c->pc.nnz_utiles + c->pc.nnz_panels) {        // (else the rows are classified as if not looked at)

@@ -134,3 +134,14 @@ def test_a_matrix_that_ends_with_half_a_strip_of_a_panel(engine_factory, M):
     assert st.nnz_panel + st.nnz_mfma >= 90 * (M - 1)
     if M % 16 == 8:
         assert st.mfma_tiles == 0 and st.panels == M // 8
+
+
+@pytest.mark.parametrize("K,groups,panels", [(200, 60, 0), (200, 170, 170), (512, 170, 0), (100, 60, 60)])
+def test_panels_of_long_ragged_rows_need_entries(engine_factory, K, groups, panels):
+    """Too few panels of long fp32 rows stay on the gather kernels, with every row classified anew."""
+    rng = np.random.default_rng(K + groups)
+    N, rows = 4000, []
+    for _ in range(groups):
+        c = 8 * np.sort(rng.choice(N // 8, 25, replace=False))
+        rows += [(c[:, None] + np.arange(8)[None, :]).ravel()] * 8
+    _check(engine_factory, rows, N, K, rng, panels=panels, mfma_tiles=0)
