@@ -282,3 +282,52 @@ def test_launch_is_capturable_into_a_hip_graph(engine_factory):
             assert O.check_values(replayed, ref, mag=mag)[0], (name, rep)
         del graph
         e.close()
+
+
+@pytest.mark.parametrize("name,K", [("fem_banded", 100), ("fem_banded", 57), ("fem_banded", 300), ("fem_banded", 700)])
+def test_launches_of_ragged_and_long_rows_are_capturable(engine_factory, monkeypatch, name, K):
+    """Rows of no whole number of 64-byte steps and rows of several launches: recorded without a launch before, replayed with
+    eager work in between, each replay against the eager result and the oracle."""
+    import torch
+
+    monkeypatch.setenv("SDDMM_RAGGED", "1")
+    monkeypatch.setenv("SDDMM_LONG_TILES", "1")
+    rng = np.random.default_rng(K)
+    dev = torch.device("cuda:0")
+    w = W.make(name, "small", K=K)
+    tA, tB = torch.from_numpy(w.A).to(dev), torch.from_numpy(w.B).to(dev)
+    t_rp, t_col, t_val = (torch.from_numpy(x).to(dev) for x in (w.rowptr, w.col, w.sval))
+    torch.cuda.synchronize()
+    e = engine_factory()
+    stream = torch.cuda.Stream(device=dev)
+    e.set_stream(stream.cuda_stream)
+    e._chk(e.L.sddmm_set_dense_device(e.h, w.M, w.N, K, C.c_void_p(tA.data_ptr()), C.c_void_p(tB.data_ptr()), capi.F32))
+    e._chk(e.L.sddmm_set_csr_device(e.h, w.M, w.N, len(w.col), C.c_void_p(t_rp.data_ptr()),
+                                    C.c_void_p(t_col.data_ptr()), C.c_void_p(t_val.data_ptr())))
+    e.nnz = len(w.col)
+    e.plan(capi.AUTO)
+    st = e.stats()
+    assert st.mfma_tiles + st.panels > 0
+    dP = C.c_void_p()
+    e._chk(e.L.sddmm_get_values_device(e.h, C.byref(dP)))
+    tP = torch.as_tensor(_DeviceArray(dP.value, len(w.col)), device=dev)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        e.launch()
+    for rep in range(3):
+        tA.copy_(torch.from_numpy(rng.uniform(-1, 1, w.A.shape).astype(f32)))
+        tP.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        replayed = tP.cpu().numpy().copy()
+        tP.zero_()
+        torch.cuda.synchronize()
+        e.run()
+        np.testing.assert_array_equal(replayed, e.values(), err_msg="replay %d" % rep)
+        a = tA.cpu().numpy()
+        ref = O.sddmm_csr(w.rowptr, w.col, w.sval, a, w.B)
+        _, mag = O.sddmm_csr_f64(w.rowptr, w.col, w.sval, a, w.B)
+        assert O.check_values(replayed, ref, mag=mag)[0], rep
+    del graph
+    e.close()
