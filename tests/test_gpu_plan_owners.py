@@ -145,3 +145,14 @@ def test_panels_of_long_ragged_rows_need_entries(engine_factory, K, groups, pane
         c = 8 * np.sort(rng.choice(N // 8, 25, replace=False))
         rows += [(c[:, None] + np.arange(8)[None, :]).ravel()] * 8
     _check(engine_factory, rows, N, K, rng, panels=panels, mfma_tiles=0)
+
+
+@pytest.mark.parametrize("strips,tiles", [(2, 140), (40, 130)])
+def test_long_strips_wider_than_the_bitmap(engine_factory, strips, tiles):
+    """A workgroup per strip whose columns span more than the bitmap holds: one wavefront merges its rows."""
+    rng = np.random.default_rng(tiles)
+    N, rows = 600_000, []
+    for _ in range(strips):
+        tc = np.sort(np.concatenate([[0, N // 16 - 1], 1 + rng.choice(N // 16 - 2, tiles - 2, replace=False)]))
+        rows += [(tc[:, None] * 16 + np.arange(16)[None, :]).ravel()[(np.arange(16 * tiles) + r) % 9 != 0] for r in range(16)]
+    _check(engine_factory, rows, N, 16, rng, mfma_tiles=strips * tiles)
