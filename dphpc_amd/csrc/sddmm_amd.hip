@@ -602,8 +602,9 @@ int plan_tiles_fill(sddmm_ctx *c) {
     // wavefronts of a tile launch: one per window, and one per two windows of a pair of gathered strips
     // (their descriptors come last and fill whole windows, an even number of them)
     c->n_win_single = c->n_windows;
-    // (rows of up to 256 bytes: beyond that the second A panel and the kept products do not fit the registers)
-    if (c->use_windows && c->n_tiles > gathered_lo && tile_pairs(c->ragged, c->dtype == SDDMM_F32, c->tile_steps) && env_int("SDDMM_PAIRS", 1) != 0)
+    // (rows of up to 256 bytes: beyond that the second A panel and the kept products do not fit the registers; a launch in
+    // another order than the storage order takes every window alone)
+    if (c->use_windows && !c->use_win_order && c->n_tiles > gathered_lo && tile_pairs(c->ragged, c->dtype == SDDMM_F32, c->tile_steps) && env_int("SDDMM_PAIRS", 1) != 0)
         c->n_win_single = gathered_lo / TILE_WINDOW;
     c->n_tile_units = c->n_win_single + (c->n_windows - c->n_win_single + 1) / 2;
     if (!c->use_windows) {

@@ -156,3 +156,17 @@ def test_long_strips_wider_than_the_bitmap(engine_factory, strips, tiles):
         tc = np.sort(np.concatenate([[0, N // 16 - 1], 1 + rng.choice(N // 16 - 2, tiles - 2, replace=False)]))
         rows += [(tc[:, None] * 16 + np.arange(16)[None, :]).ravel()[(np.arange(16 * tiles) + r) % 9 != 0] for r in range(16)]
     _check(engine_factory, rows, N, 16, rng, mfma_tiles=strips * tiles)
+
+@pytest.mark.parametrize("K", [32, 64, 128])
+def test_window_order_with_gathered_pairs(engine_factory, monkeypatch, K):
+    """An order asked for by name also where two windows of a gathered pair would share a wavefront: every window once."""
+    monkeypatch.setenv("SDDMM_WINDOW_ORDER", "1")
+    rng = np.random.default_rng(K)
+    N, rows = 3000, []
+    for i in range(600):
+        lo = int(rng.integers(0, N - 400))
+        rows.append(lo + np.flatnonzero(rng.random(400) < 0.5))
+        rows += [np.sort(rng.choice(N, 9, replace=False))] * 2
+    rows = [16 * s + np.arange(128) for s in range(40) for _ in range(16)] + rows          # 320 tiles of strips before them
+    st = _check(engine_factory, rows, N, K, rng)
+    assert st.mfma_tiles > 1000
