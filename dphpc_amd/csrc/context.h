@@ -118,6 +118,10 @@ struct sddmm_ctx {
     unsigned int *d_short_sums = nullptr, *d_short_off = nullptr;     // arena views: entries of short rows per block of the row scan
     RowItem *d_panel_items = nullptr;
     int64_t n_panel_items = 0, panel_items_cap = 0, n_panels = 0, nnz_panels = 0;
+    int panel_columns = 0;           // of a work item
+    RowItem *d_fused_panels = nullptr;       // the items of the fused call, where they are cut otherwise
+    int64_t n_fused_panels = 0, fused_panels_cap = 0;
+    bool fused_panels_valid = false;
     bool panel_mfma = false;         // panels run on k_panel_mfma (else on k_panel)
     bool panels_flagged = false;     // the panel detector ran in this plan
     // FLAT in slices of K (kernels_flat.h): partial products of a range of entries, [slice][entry]

@@ -3,6 +3,7 @@
 // device; the host reads back only the small PlanCounters block.
 #pragma once
 #include "device_utils.h"
+#include "plan_rules.h"
 
 namespace sddmm {
 
@@ -659,8 +660,17 @@ static __global__ __launch_bounds__(256) void k_piece_places(const int32_t *__re
     if (n != 0) cut_rows[at] = row;
 }
 
-// items of the taken panels: {first row, [start,end) inside the shared list}
-static __global__ __launch_bounds__(256) void k_panel_items(const int32_t *__restrict__ rowptr, int64_t n_panels, int pseg,
+// Items per taken panel for the fused call, in place of those of the SDDMM (fused_panel_columns).
+static __global__ __launch_bounds__(256) void k_fused_panel_counts(const int32_t *__restrict__ rowptr, int64_t n_panels, int halves_from,
+                                                                   unsigned int *__restrict__ counts) {
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= n_panels || counts[p] == 0) return;
+    const int len = rowptr[p * 8 + 1] - rowptr[p * 8], columns = fused_panel_columns(len, halves_from);
+    counts[p] = (unsigned int)((len + columns - 1) / columns);
+}
+
+// items of the taken panels: {first row, [start,end) inside the shared list}; pseg 0: of the fused call
+static __global__ __launch_bounds__(256) void k_panel_items(const int32_t *__restrict__ rowptr, int64_t n_panels, int pseg, int halves_from,
                                                      const unsigned int *__restrict__ counts,
                                                      const unsigned int *__restrict__ offsets,
                                                      RowItem *__restrict__ items) {
@@ -671,10 +681,11 @@ static __global__ __launch_bounds__(256) void k_panel_items(const int32_t *__res
     const int32_t row0 = (int32_t)(p * 8);
     const int32_t rs0 = rowptr[row0];
     const int32_t len = rowptr[row0 + 1] - rs0;
+    const int columns = pseg ? pseg : fused_panel_columns(len, halves_from);
     unsigned int at = offsets[p];
     for (unsigned int k = 0; k < n; ++k) {
-        const int32_t a = (int32_t)k * pseg;
-        const int32_t b = a + pseg < len ? a + pseg : len;
+        const int32_t a = (int32_t)k * columns;
+        const int32_t b = a + columns < len ? a + columns : len;
         // pad carries the CSR position of the panel's first row: the 8 rows have the same
         // length and follow each other, so row r starts at pad + r*len and a kernel can
         // start reading the column list without first waiting for a row pointer

@@ -18,9 +18,10 @@ void launch_panel_u(sddmm_ctx *c, const Shape &s) {
 template <int DT, int STEPS>
 void launch_panel_fused_t(sddmm_ctx *c) {
     constexpr int PW = panel_mfma_waves(STEPS);
-    const int64_t nblocks = (c->n_panel_items + PW - 1) / PW;
+    const int64_t n_items = c->n_fused_panels ? c->n_fused_panels : c->n_panel_items;
+    const int64_t nblocks = (n_items + PW - 1) / PW;
     SDDMM_LAUNCH(c, (k_panel_mfma<DT, STEPS, true>), xcd_grid(nblocks), PW * WAVE,
-                 (const RowItem *)c->d_panel_items, c->n_panel_items, nblocks, c->d_rowptr, c->d_col, (const void *)c->dA,
+                 (const RowItem *)(c->n_fused_panels ? c->d_fused_panels : c->d_panel_items), n_items, nblocks, c->d_rowptr, c->d_col, (const void *)c->dA,
                  (const void *)c->dB, 0, (const float *)c->d_sval, c->dP, c->dO, 0);
 }
 template <int DT>

@@ -122,6 +122,9 @@ void release_sparse(sddmm_ctx *c, bool idle = false) {
     c->sort_tmp_bytes = 0;
     c->cand_cap = c->vstrips_cap = c->n_cand = c->n_vstrips = 0;
     dfree(c->d_panel_items, idle);
+    dfree(c->d_fused_panels, idle);
+    c->n_fused_panels = c->fused_panels_cap = 0;
+    c->fused_panels_valid = false;
     dfree(c->d_short_list, idle);
     c->short_list_cap = c->n_short_list = 0;
     c->use_short_list = false;
@@ -642,10 +645,10 @@ int panel_steps(const sddmm_ctx *c) { return c->long_rows ? LONG_STEPS : c->ragg
 int panel_item_columns(const sddmm_ctx *c) {
     const int steps = panel_steps(c);
     const int64_t wavefronts = 1024 * (steps <= 2 ? 5 : steps <= 8 ? 4 : 2), panels = std::max<int64_t>(1, c->sM / PANEL_ROWS);
-    int64_t columns = 512;
+    int64_t columns = PANEL_COLUMNS;
     if ((c->dtype != SDDMM_F32 && steps > 2 ? 8 : 2) * panels <= wavefronts) {
         const int64_t pieces = wavefronts / panels;                       // of a row of average length
-        columns = std::min<int64_t>(512, (c->nnz / std::max(1, c->sM) / pieces + WAVE - 1) / WAVE * WAVE);
+        columns = std::min<int64_t>(PANEL_COLUMNS, (c->nnz / std::max(1, c->sM) / pieces + WAVE - 1) / WAVE * WAVE);
     }
     return std::max<int>(WAVE, env_int("SDDMM_PANEL_SEG", (int)columns));
 }
@@ -664,6 +667,7 @@ int plan_panels_items(sddmm_ctx *c, int pseg) {
     c->n_panels = (int64_t)c->pc.n_panels;
     c->nnz_panels = (int64_t)c->pc.nnz_panels;
     c->n_panel_items = (int64_t)c->pc.panel_items;
+    c->panel_columns = pseg;
     if (c->n_panel_items == 0) return SDDMM_OK;
     if (c->n_panel_items > c->panel_items_cap) {
         dfree(c->d_panel_items);
@@ -671,7 +675,7 @@ int plan_panels_items(sddmm_ctx *c, int pseg) {
         c->panel_items_cap = c->n_panel_items;
     }
     SDDMM_LAUNCH(c, k_panel_items, ((n_panels + 255) / 256), 256, c->d_rowptr,
-                       n_panels, pseg, (const unsigned int *)c->d_panel_counts, (const unsigned int *)c->d_panel_off,
+                       n_panels, pseg, 0, (const unsigned int *)c->d_panel_counts, (const unsigned int *)c->d_panel_off,
                        c->d_panel_items);
     LAUNCH_CHECK(c);
     return SDDMM_OK;
@@ -948,6 +952,7 @@ int do_plan(sddmm_ctx *c, int strategy) {
     c->n_scan_jobs = 0;
     c->use_slices = c->use_blocks = c->use_order = false;
     c->fused_items_valid = false;    // they leave out the rows of this plan's panels
+    c->fused_panels_valid = false;
     int resolved = strategy;
     const bool csr_ok = c->have_rowptr;
     // without a row pointer (unsorted COO) only the flat kernels apply
@@ -1615,6 +1620,38 @@ static int plan_fused_items(sddmm_ctx *c, const unsigned char *panel_owner) {
     return SDDMM_OK;
 }
 
+// items of the fused panel kernel: those of the plan, or a list of its own
+static int plan_fused_panels(sddmm_ctx *c) {
+    if (c->fused_panels_valid) return SDDMM_OK;
+    c->n_fused_panels = 0;
+    const bool half_width = c->dtype != SDDMM_F32;
+    const int halves_from = fused_halves_from(c->n_panels, panel_mfma_min_waves(panel_mfma_steps(c), true, half_width), half_width);
+    if (!getenv("SDDMM_PANEL_SEG") && (halves_from || c->panel_columns != PANEL_COLUMNS)) {
+        const int64_t n_panels = (int64_t)c->sM / 8;
+        SDDMM_LAUNCH(c, k_fused_panel_counts, (n_panels + 255) / 256, 256, (const int32_t *)c->d_rowptr, n_panels, halves_from,
+                     c->d_panel_counts);
+        LAUNCH_CHECK(c);
+        int rc = device_scan(c, c->d_panel_counts, c->d_panel_off, n_panels, &c->d_pc->panel_items);
+        if (rc) return rc;
+        DevTotals totals;
+        rc = read_totals(c, &totals);
+        if (rc) return rc;
+        const int64_t n = (int64_t)totals.panel_items;
+        if (n > c->fused_panels_cap) {
+            dfree(c->d_fused_panels);
+            c->fused_panels_cap = 0;
+            ALLOC_TRY(c, c->d_fused_panels, (size_t)n * sizeof(RowItem));
+            c->fused_panels_cap = n;
+        }
+        SDDMM_LAUNCH(c, k_panel_items, (n_panels + 255) / 256, 256, (const int32_t *)c->d_rowptr, n_panels, 0, halves_from,
+                     (const unsigned int *)c->d_panel_counts, (const unsigned int *)c->d_panel_off, c->d_fused_panels);
+        LAUNCH_CHECK(c);
+        c->n_fused_panels = n;
+    }
+    c->fused_panels_valid = true;
+    return SDDMM_OK;
+}
+
 int sddmm_run_fused(sddmm_ctx *c) {
     if (!c) return SDDMM_ERR_NULL;
     HIP_TRY(c, hipSetDevice(c->device));
@@ -1639,6 +1676,10 @@ int sddmm_run_fused(sddmm_ctx *c) {
     const unsigned char *panel_owner = panels ? (const unsigned char *)c->d_owner : nullptr;
     rc = plan_fused_items(c, panel_owner);
     if (rc) return rc;
+    if (panels) {
+        rc = plan_fused_panels(c);
+        if (rc) return rc;
+    }
     const size_t o_bytes = (size_t)c->M * (size_t)c->K * sizeof(float);
     if (o_bytes > c->o_cap) {
         dfree(c->dO);

@@ -429,3 +429,40 @@ def test_fused_row_and_item_edges(engine_factory, M, lens, K, dtype):
     print("fused edges", M, K, dtype, flush=True)
     _check(e, rowptr, col, val, A, B, "%d rows K=%d" % (M, K))
     e.close()
+
+
+@pytest.mark.parametrize("K,dtype", [(32, capi.F32), (64, capi.F32), (128, capi.F32), (32, capi.BF16), (64, capi.F16), (128, capi.BF16)])
+@pytest.mark.parametrize("panels", [3, 100, 700, 1600])
+def test_fused_panels_repeat_bit_for_bit(engine_factory, K, dtype, panels):
+    """Panels of up to 1 024 columns, few enough for two work items each or too many: O is the same in every run, and after
+    plans and launches of the SDDMM in between, whose items are others."""
+    rng = np.random.default_rng(K + panels)
+    N, rows = 1500, []
+    for length in rng.choice([16, 33, 64, 65, 127, 129, 240, 500, 640, 1023, 1024] if panels < 700 else [16, 65, 129, 240, 500], panels):
+        rows += [np.sort(rng.choice(N, int(length), replace=False))] * 8
+    rows += [np.sort(rng.choice(N, 5, replace=False))] * 3
+    M = len(rows)
+    rowptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    col = np.concatenate(rows).astype(np.int32)
+    val = rng.uniform(-1, 1, len(col)).astype(f32)
+    A, B = rng.uniform(-1, 1, (M, K)).astype(f32), rng.uniform(-1, 1, (N, K)).astype(f32)
+    Ad, Bd = A, B
+    if dtype != capi.F32:
+        to, back = (capi.to_bf16, capi.from_bf16) if dtype == capi.BF16 else (capi.to_f16, capi.from_f16)
+        Ad, Bd = to(A).reshape(M, K), to(B).reshape(N, K)
+        A, B = back(Ad).reshape(M, K), back(Bd).reshape(N, K)
+    e = engine_factory()
+    e.set_dense(Ad, Bd, dtype)
+    e.set_csr(M, N, rowptr, col, val)
+    e.plan(capi.AUTO)
+    assert e.stats().panels == panels
+    e.run()
+    p = e.values()
+    out = _check(e, rowptr, col, val, A, B, "panels %d K=%d dtype=%d" % (panels, K, dtype))
+    for i in range(6):
+        np.testing.assert_array_equal(e.run_fused(), out)
+    e.run()
+    np.testing.assert_array_equal(e.values(), p)
+    e.plan(capi.AUTO)
+    np.testing.assert_array_equal(e.run_fused(), out)
+    e.close()
