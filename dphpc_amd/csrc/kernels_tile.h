@@ -1198,7 +1198,7 @@ struct WholeRows {
     using Row = const uint4 *;
     explicit __device__ __forceinline__ WholeRows(int) {}
     __device__ __forceinline__ Row row(const void *base, int64_t r) const { return (const uint4 *)base + r * (STEPS * 4); }
-    __device__ __forceinline__ uint4 unit(const void *, Row row, int u, int) const { return row[u]; }
+    __device__ __forceinline__ const uint4 &unit(const void *, Row row, int u, int) const { return row[u]; }
     __device__ __forceinline__ uint4 trim(const uint4 &v, int, int) const { return v; }
     __device__ __forceinline__ int last_unit() const { return STEPS * 4 - 1; }
 };
