@@ -375,7 +375,6 @@ hipError_t load_fused();
 void launch_flat(sddmm_ctx *c);                                                  // launch_flat.hip
 int launch_flat_blocks(sddmm_ctx *c);                                            // number of launches
 void launch_unsort(sddmm_ctx *c);
-int column_blocks_most(const sddmm_ctx *c);
 void block_items_max(const sddmm_ctx *c, bool cut_long_rows, int64_t *segments, int64_t *gaps);
 bool blocks_pay(const sddmm_ctx *c);
 bool order_pays(const sddmm_ctx *c);

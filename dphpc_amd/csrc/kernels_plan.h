@@ -715,20 +715,6 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_long_rows(const int32_t *
         if ((is_long >> q) & 1u) long_rows[at++] = (int32_t)(base + q);
 }
 
-// Column blocks of a long row: a power of two, 8 to `most`, such that its segments hold COL_BLOCK_ENTRIES entries or more
-// on average (from 16 blocks on).  More blocks find more lines of B in an XCD's L2, short segments leave lanes idle and are
-// work items more.  16 blocks for every row / 8 .. 64 with 32, 64, 96 entries, all with the exact grid (launch_flat_blocks):
-// graph of 2.6 M rows K = 32 521 us / 524, 515, 513; 1.5 M rows K = 64 bf16 229 / 230, 225, 223; 800 000 rows K = 64
-// 253 / 251, 249, 249; 200 000 rows K = 32 27.7 / 28.2, 27.3, 26.9, K = 100 116.4 / 114.6, 114.8, 115.5, K = 256 244 / 238,
-// 241, 243.  From 4 blocks on: 532, 226, 259, 27.1, 118, 265.
-constexpr int COL_BLOCKS_MIN = 8, COL_BLOCKS_MAX = WAVE, COL_BLOCK_ENTRIES = 64;
-constexpr int COL_BLOCKS_ORDER = 16;           // that the sort of COO entries knows
-__host__ __device__ inline int row_blocks(int len, int most) {
-    int n = COL_BLOCKS_MIN;
-    while (n < most && len >= 2 * n * COL_BLOCK_ENTRIES) n *= 2;
-    return n;
-}
-
 // `most` lanes per long row: lane b finds where the row's columns of block b start (columns ascend inside a
 // row: its entries of a block are consecutive; in a row that is not sorted the cuts fall anywhere, every
 // entry still lands in exactly one segment).  Segment (b, i): block b of long row i, block-major; a row of fewer blocks
@@ -736,7 +722,7 @@ __host__ __device__ inline int row_blocks(int len, int most) {
 static __global__ __launch_bounds__(256) void k_long_segments(const int32_t *__restrict__ rowptr,
                                                               const int32_t *__restrict__ col, int N,
                                                               const int32_t *__restrict__ long_rows, int n_long, int piece,
-                                                              int most,
+                                                              int least, int most,
                                                               int32_t *__restrict__ seg_start,
                                                               unsigned int *__restrict__ seg_items) {
     const int64_t slot = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -747,7 +733,7 @@ static __global__ __launch_bounds__(256) void k_long_segments(const int32_t *__r
         const int row = long_rows[i];
         lo = rowptr[row];
         end = rowptr[row + 1];
-        every = most / row_blocks(end - lo, most);
+        every = most / row_blocks(end - lo, least, most);
         const int first = (int)(((int64_t)N * b + most - 1) / most);     // (of block b, as in k_order_keys)
         int hi = end;
         if (b % every != 0 || b == 0) hi = lo;

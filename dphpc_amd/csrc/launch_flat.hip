@@ -28,16 +28,10 @@ int64_t blocks_grid(int64_t segments, int64_t gaps, int waves) {
 
 }  // namespace
 
-// the most column blocks that a row is cut into
-int column_blocks_most(const sddmm_ctx *c) {
-    return c->use_order ? std::min(COL_BLOCKS_ORDER, row_blocks((int)c->pc.max_len, COL_BLOCKS_ORDER))
-                        : row_blocks((int)c->pc.max_len, COL_BLOCKS_MAX);
-}
-
 // the most work items there can be, from the counts of the row classes
 void block_items_max(const sddmm_ctx *c, bool cut_long_rows, int64_t *segments, int64_t *gaps) {
     const int64_t n_long = cut_long_rows ? (int64_t)c->pc.rows_long : 0, nnz_long = cut_long_rows ? (int64_t)c->pc.nnz_long : 0;
-    *segments = nnz_long / c->seg + std::min(n_long * column_blocks_most(c), n_long * COL_BLOCKS_MIN + nnz_long / COL_BLOCK_ENTRIES);
+    *segments = row_block_segments(n_long, nnz_long, c->seg, c->use_order, (int)c->pc.max_len);
     *gaps = (c->nnz - nnz_long) / WAVE + n_long + 1;
 }
 

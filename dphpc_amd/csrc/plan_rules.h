@@ -5,6 +5,34 @@
 
 namespace sddmm {
 
+// ---- column blocks of a long row (kernels_flat.h) ---------------------------------------------
+// A power of two, `least` to `most`, such that the segments hold COL_BLOCK_ENTRIES entries or more on average (beyond `least`
+// blocks).  More blocks find more lines of B in an XCD's L2, short segments leave lanes idle and are work items more.  16 blocks
+// for every row / 8 .. 64 with 32, 64, 96 entries, all with the exact grid (launch_flat_blocks): graph of 2.6 M rows K = 32
+// 521 us / 524, 515, 513; 1.5 M rows K = 64 bf16 229 / 230, 225, 223; 800 000 rows K = 64 253 / 251, 249, 249; 200 000 rows
+// K = 32 27.7 / 28.2, 27.3, 26.9, K = 100 116.4 / 114.6, 114.8, 115.5, K = 256 244 / 238, 241, 243.  From 4 blocks on: 532,
+// 226, 259, 27.1, 118, 265.
+// Entries that came in no order were sorted by row and by 16 blocks, and keep them, whatever the row: 8 and 16 / 16, with the
+// unsorting, 400 000 rows K = 128 310.7 / 304.4 us, K = 200 550 / 540; 1 M rows K = 100 816 / 799, K = 75 703 / 688; 100 000 rows
+// K = 200 108.6 / 106.6, K = 75 50.0 / 50.6, with new inputs in turn 54.8 / 51.6; up to 64 floats a row 1 % the other way.
+constexpr int COL_BLOCKS_MIN = 8, COL_BLOCKS_MAX = 64, COL_BLOCK_ENTRIES = 64;
+constexpr int COL_BLOCKS_ORDER = 16;           // that the sort of COO entries knows
+constexpr int row_blocks(int len, int least, int most) {
+    int n = least;
+    while (n < most && len >= 2 * n * COL_BLOCK_ENTRIES) n *= 2;
+    return n;
+}
+constexpr int row_blocks_least(bool sorted_order) { return sorted_order ? COL_BLOCKS_ORDER : COL_BLOCKS_MIN; }
+constexpr int row_blocks_most(bool sorted_order, int longest_row) {
+    return row_blocks(longest_row, row_blocks_least(sorted_order), sorted_order ? COL_BLOCKS_ORDER : COL_BLOCKS_MAX);
+}
+// the most segments of pieces of `piece` entries that n_long rows of nnz_long entries can have
+constexpr int64_t row_block_segments(int64_t n_long, int64_t nnz_long, int piece, bool sorted_order, int longest_row) {
+    const int64_t most = n_long * row_blocks_most(sorted_order, longest_row);
+    const int64_t by_length = n_long * row_blocks_least(sorted_order) + nnz_long / COL_BLOCK_ENTRIES;
+    return nnz_long / piece + (most < by_length ? most : by_length);
+}
+
 // ---- 8-row panels ---------------------------------------------------------------------------
 constexpr int PANEL_COLUMNS = 512;             // columns of a panel's work item, at the most
 

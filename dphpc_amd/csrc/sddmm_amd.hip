@@ -701,7 +701,7 @@ int plan_blocks(sddmm_ctx *c, bool cut_long_rows) {
     const int64_t n_long = cut_long_rows ? (int64_t)c->pc.rows_long : 0, nb = ((int64_t)c->sM + SCAN_TILE - 1) / SCAN_TILE;
     if (cut_long_rows && (int64_t)c->raw.long_scanned != n_long)
         return fail(c, SDDMM_ERR_HIP, "internal: scan of the long rows disagrees with their number");
-    const int most = column_blocks_most(c);
+    const int least = row_blocks_least(c->use_order), most = row_blocks_most(c->use_order, (int)c->pc.max_len);
     const int64_t n_seg = n_long * most, n_gap = n_long + 1;
     const int64_t piece = c->seg, gap_piece = WAVE;
     block_items_max(c, cut_long_rows, &c->block_segments_max, &c->block_gaps_max);
@@ -732,7 +732,7 @@ int plan_blocks(sddmm_ctx *c, bool cut_long_rows) {
     if (n_long > 0) {
         SDDMM_LAUNCH(c, k_long_rows, nb, SCAN_BLOCK, c->d_rowptr, c->sM, c->ts, c->seg, (const unsigned int *)c->d_long_off, rows);
         SDDMM_LAUNCH(c, k_long_segments, grid_for(n_seg, 256), 256, c->d_rowptr, entry_cols(c), c->sN, (const int32_t *)rows,
-                     (int)n_long, (int)piece, most, seg_start, seg_items);
+                     (int)n_long, (int)piece, least, most, seg_start, seg_items);
     }
     SDDMM_LAUNCH(c, k_long_gaps, grid_for(n_gap, 256), 256, c->d_rowptr, (const int32_t *)rows, (int)n_long, (int)c->nnz,
                  (int)gap_piece, gap_start, gap_items);

@@ -29,7 +29,24 @@ static void fused_panels() {
     CHECK(fused_halves_from(512, 1, true) == 128 && fused_halves_from(513, 1, true) == 0, "one wavefront per SIMD");
 }
 
+// Rows of every length: a power of two that divides `most` (the lanes of a row), the bound that sizes the list of segments.
+static void column_blocks() {
+    for (bool sorted : {false, true})
+        for (int longest : {257, 1023, 1024, 4096, 100000}) {
+            const int least = row_blocks_least(sorted), most = row_blocks_most(sorted, longest);
+            CHECK(most >= least && most <= COL_BLOCKS_MAX && most % least == 0, "%d", longest);
+            for (int len = 257; len <= longest; len += len / 50 + 1) {
+                const int n = row_blocks(len, least, most);
+                CHECK(n >= least && most % n == 0, "%d blocks of a row of %d", n, len);
+                CHECK(n == least || len >= n * COL_BLOCK_ENTRIES, "%d blocks of a row of %d", n, len);
+                CHECK(row_block_segments(7, 7 * (int64_t)len, 256, sorted, longest) >= 7 * (len / 256 + n), "row of %d", len);
+                if (sorted) CHECK(n == 16, "sorted entries, %d blocks of a row of %d", n, len);
+            }
+        }
+}
+
 int main() {
+    column_blocks();
     fused_panels();
     std::printf("%d failed\n", failures);
     return failures != 0;
