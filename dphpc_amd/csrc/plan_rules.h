@@ -36,6 +36,24 @@ constexpr int64_t row_block_segments(int64_t n_long, int64_t nnz_long, int piece
 // ---- 8-row panels ---------------------------------------------------------------------------
 constexpr int PANEL_COLUMNS = 512;             // columns of a panel's work item, at the most
 
+// Columns of a panel's work item, for rows of `steps` 64-byte steps: fewer than 512 where whole panels, of `average` columns,
+// would leave most of the chip's wavefronts idle (the kernel's registers hold 5 per SIMD at 128-byte rows, 4 up to 512 bytes, 2
+// beyond): as many items as half of the wavefronts, but two per panel for up to three eighths of them.
+// 512 / this rule: 250 panels of 240 random columns K = 32 7.2 / 4.8 us, K = 256 30.5 / 13.4; 500 K = 128 16.2 / 10.2; 1 000
+// K = 32 9.8 / 7.3, K = 64 12.7 / 11.0, K = 128 17.6 / 18.8, K = 64 fp16 7.1 / 6.5; 1 000 in 8x8 blocks K = 128 16.4 / 13.9;
+// 1 500 K = 128 21.5 / 18.3, random 25.5 / 25.9.  Items for all of the wavefronts, and for up to half as many panels: 1 000 of
+// 240 random columns K = 128 19.9, K = 64 fp16 7.55; 2 000 of 100 K = 128 19.0 (18.4 uncut), K = 64 fp16 7.3 (6.8); 2 000 of
+// 160 K = 128 22.7 (20.7).  16-bit rows beyond 128 bytes, whose items are shorter in time, only where there are very few
+// panels: 1 000 of 104 columns K = 128 bf16 6.0 / 6.8.
+constexpr int panel_columns(int steps, bool half_width, int64_t panels, int64_t average) {
+    const int64_t wavefronts = 1024 * (steps <= 2 ? 5 : steps <= 8 ? 4 : 2);
+    int64_t pieces = steps <= 8 ? wavefronts / (2 * panels) : wavefronts / panels;
+    if (pieces < 2 && 8 * panels <= 3 * wavefronts) pieces = 2;
+    if (pieces < 2 || (half_width && steps > 2 && 8 * panels > wavefronts)) return PANEL_COLUMNS;
+    const int64_t columns = (average / pieces + 63) / 64 * 64;       // of a panel of average length
+    return columns < 64 ? 64 : columns < PANEL_COLUMNS ? (int)columns : PANEL_COLUMNS;
+}
+
 // Columns of a work item of the fused call: a panel of up to 1 024 columns is one item, or two where that leaves wavefronts
 // of the chip something to do (halves_from: from more columns on; 0: not).  The items of a panel add their part of the
 // output rows atomically to zeros: two sums come out the same in either order, three do not.

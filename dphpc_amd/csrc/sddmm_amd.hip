@@ -637,20 +637,10 @@ bool panel_valu_applicable(const sddmm_ctx *c) {
 
 int panel_steps(const sddmm_ctx *c) { return c->long_rows ? LONG_STEPS : c->ragged ? ragged_steps(c) : panel_mfma_steps(c); }
 
-// Columns per work item of a panel: 512, fewer where an item per panel would leave half of the chip's wavefronts idle.  (The
-// kernel's registers hold 5 wavefronts per SIMD at 128-byte rows, 4 up to 512 bytes, 2 beyond.  512 / this rule: 1 000 panels
-// of 96 columns K = 32 4.9 / 4.0 us, K = 256 13.5 / 11.6; 1 500 of 200 K = 128 20.9 / 17.6, K = 64 12.4 / 12.3; 2 000 of 240
-// K = 32 11.3 / 10.6, K = 256 in halves 42 / 48.)  16-bit rows beyond 128 bytes only where there are very few panels: 1 000
-// of 96 columns K = 128 bf16 5.0 / 5.4, 2 000 of 240 13.7 / 14.8.
 int panel_item_columns(const sddmm_ctx *c) {
-    const int steps = panel_steps(c);
-    const int64_t wavefronts = 1024 * (steps <= 2 ? 5 : steps <= 8 ? 4 : 2), panels = std::max<int64_t>(1, c->sM / PANEL_ROWS);
-    int64_t columns = PANEL_COLUMNS;
-    if ((c->dtype != SDDMM_F32 && steps > 2 ? 8 : 2) * panels <= wavefronts) {
-        const int64_t pieces = wavefronts / panels;                       // of a row of average length
-        columns = std::min<int64_t>(PANEL_COLUMNS, (c->nnz / std::max(1, c->sM) / pieces + WAVE - 1) / WAVE * WAVE);
-    }
-    return std::max<int>(WAVE, env_int("SDDMM_PANEL_SEG", (int)columns));
+    const int64_t M = std::max(1, c->sM);
+    const int columns = panel_columns(panel_steps(c), c->dtype != SDDMM_F32, std::max<int64_t>(1, M / PANEL_ROWS), c->nnz / M);
+    return std::max<int>(WAVE, env_int("SDDMM_PANEL_SEG", columns));
 }
 
 // whether the 8-row panels are looked for, and by which kernel they would be computed

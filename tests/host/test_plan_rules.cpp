@@ -17,6 +17,23 @@ static int failures = 0;
         }                                                                       \
     } while (0)
 
+static void panels() {
+    for (int steps : {1, 2, 4, 6, 8, 12, 16})
+        for (bool half : {false, true})
+            for (int64_t n : {1, 7, 100, 255, 256, 257, 512, 513, 1000, 1024, 1025, 1280, 1281, 1536, 1537, 4500, 1000000})
+                for (int64_t average : {0, 1, 16, 63, 64, 65, 104, 127, 128, 160, 240, 480, 481, 5000}) {
+                    const int columns = panel_columns(steps, half, n, average);
+                    CHECK(columns >= 64 && columns <= PANEL_COLUMNS, "%d columns", columns);
+                    CHECK(columns % 64 == 0, "%d columns", columns);
+                    if (n > 1920) CHECK(columns == PANEL_COLUMNS, "%d panels fill the chip", (int)n);
+                    // no more items than wavefronts
+                    const int64_t items = n * ((average + columns - 1) / columns), whole = n * ((average + PANEL_COLUMNS - 1) / PANEL_COLUMNS);
+                    CHECK(items <= 5120 || items <= whole, "%d items of %d panels of %d columns", (int)items, (int)n, (int)average);
+                }
+    CHECK(panel_columns(8, false, 1000, 240) == 128 && panel_columns(2, true, 1000, 240) == 128, "1 000 panels of 240");
+    for (int steps : {2, 4, 8}) CHECK(panel_columns(steps, false, 2000, 160) == PANEL_COLUMNS, "2 000 panels");
+}
+
 static void fused_panels() {
     for (int from : {0, 64, 128})
         for (int len = 1; len <= 5000; ++len) {
@@ -46,6 +63,7 @@ static void column_blocks() {
 }
 
 int main() {
+    panels();
     column_blocks();
     fused_panels();
     std::printf("%d failed\n", failures);
