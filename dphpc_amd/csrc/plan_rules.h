@@ -54,6 +54,30 @@ constexpr int panel_columns(int steps, bool half_width, int64_t panels, int64_t 
     return columns < 64 ? 64 : columns < PANEL_COLUMNS ? (int)columns : PANEL_COLUMNS;
 }
 
+// Entries per tile below which 16-row strips that are two panels of `panels` (as many as the matrix has groups of 8 rows) go to
+// the panel kernel as panels, and from which they stay strips of dense tiles.  One line for a strip alone and, where some lie
+// above it and some below, for all of them together: tiles and panels are two launches.
+// Time of tiles / time of panels, strips of one fill, 112 .. 208 entries per tile:
+//   rows of up to 128 bytes 0.92 .. 2.0, more with the size: 192, of fewer than 5 M entries 187 (a mixture of 205 and 125
+//   entries that averages that is better as tiles).
+//   256 bytes and more: from 176 entries on the launch splits K over a workgroup, 0.5 .. 1.0; below 0.85 .. 1.8.  Of 5 M entries
+//   and more 176 .. 192 are 1.0 .. 1.4, with 1 KiB 0.8 .. 1.0.
+//   the same, 600 .. 1 000 panels of up to 1.5 M entries, which whole panels do not fill the chip with and more items delay:
+//   fp32 0.85 .. 1.05 from 144 entries on, 0.94 .. 1.14 below; 16 bits 0.62 .. 1.05 at any fill (2 000 panels: 1.0 .. 1.37).
+//   16 bits, up to 1 000 panels: 512 bytes 0.76 .. 1.0 with up to 1.5 M entries, 1.1 .. 1.4 with more; 1 KiB 0.6 .. 1.0 up to 4 M
+//   entries, then 1.0 .. 1.2.
+//   3 000 and 6 000 panels of 28 .. 48 columns, a step of 64 half empty: 0.78 .. 0.96.
+constexpr int panels_below(int steps, bool half_width, int64_t panels, int64_t nnz) {
+    constexpr int never = 0;
+    const bool few = panels <= 1280, some = few && panels > 512;
+    if (panels > 2560 && nnz < 48 * 8 * panels) return never;
+    const bool many = nnz >= (int64_t)5 << 20;
+    if (steps <= 2) return many ? 192 : 187;
+    if (half_width && nnz < (steps > 8 ? (int64_t)1 << 22 : (int64_t)3 << 19) && (steps > 4 ? few : some)) return never;
+    if (!half_width && some && nnz < (int64_t)3 << 19) return 144;
+    return many && steps <= 8 ? 192 : 176;
+}
+
 // Columns of a work item of the fused call: a panel of up to 1 024 columns is one item, or two where that leaves wavefronts
 // of the chip something to do (halves_from: from more columns on; 0: not).  The items of a panel add their part of the
 // output rows atomically to zeros: two sums come out the same in either order, three do not.

@@ -979,7 +979,8 @@ int do_plan(sddmm_ctx *c, int strategy) {
             if (tiles && gathered && c->sM >= 2) rules.cand_min = std::max(16, env_int("SDDMM_GATHERED_MIN", 64));
             const int pseg = panel_item_columns(c);
             rules.pseg = pseg;
-            rules.panels_below = 192;
+            // (long rows take either kernel 512 bytes at a time)
+            rules.panels_below = panels_below(c->long_rows ? 16 : panel_steps(c), c->dtype != SDDMM_F32, c->sM / PANEL_ROWS, c->nnz);
             // the rows nobody owns so far are classified in the same launch: most matrices have
             // no gathered strips, and their plan then waits for the device once
             c->ts = rules.ts = std::max(1, env_int("SDDMM_TS", 24));
@@ -996,14 +997,13 @@ int do_plan(sddmm_ctx *c, int strategy) {
             if (rc) return rc;
             rc = fetch_counters(c);
             if (rc) return rc;
-            // Strips that are two panels each, some above the line and some below it: tiles and panels are two launches, so all
-            // of them go the way that their average says.  (Launch us, all strips / mixed / all panels: 2 000 rows in a band,
-            // 155 entries per tile, K = 32 5.2 / 8.6 / 4.2, K = 512 bf16 8.9 / 13.9 / 10.4; 16 000 rows, 174 entries, K = 64
-            // 21.7 / 23.5, K = 256 53 / 58; below the line altogether, 120 entries, 4 000 rows, K = 32 13.3 with a few panels
-            // among strips, 5.0 as panels, K = 512 bf16 37.7 and 15.6.)
+            // Strips that are two panels each, some above the line and some below it: all of them go the way that their average
+            // says, since tiles and panels are two launches.  (Launch us, all strips / mixed / all panels: 2 000 rows in a band,
+            // 155 entries per tile, K = 32 5.2 / 8.6 / 4.2, K = 512 bf16 8.9 / 13.9 / 10.4; 120 entries, 4 000 rows, K = 32 13.3
+            // with a few panels among strips, 5.0 as panels.)
             if (c->pc.nnz_either_strip && c->pc.nnz_either_panels) {
-                const unsigned long long line = (panel_steps(c) >= 12 ? 144ull : 160ull) * c->pc.either_tiles;
-                rc = settle_owners(c, c->pc.nnz_either_strip + c->pc.nnz_either_panels < line, pseg);
+                const unsigned long long entries = c->pc.nnz_either_strip + c->pc.nnz_either_panels;
+                rc = settle_owners(c, entries < (unsigned long long)rules.panels_below * c->pc.either_tiles, pseg);
                 if (!rc) rc = fetch_counters(c);
                 if (rc) return rc;
             }

@@ -34,6 +34,17 @@ static void panels() {
     for (int steps : {2, 4, 8}) CHECK(panel_columns(steps, false, 2000, 160) == PANEL_COLUMNS, "2 000 panels");
 }
 
+// A matrix whose strips all hold the same number of entries per tile, on either side of the line.
+static void tiles_or_panels() {
+    CHECK(panels_below(4, false, 250, 200000) == 176 && panels_below(16, false, 4000, 11000000) == 176, "split K");
+    CHECK(panels_below(4, false, 4000, 11000000) == 192 && panels_below(2, false, 250, 200000) == 187, "many entries, short rows");
+    CHECK(panels_below(4, false, 1000, 1200000) == 144 && panels_below(4, false, 2000, 1200000) == 176, "a chip that whole panels do not fill");
+    CHECK(panels_below(16, true, 250, 200000) == 0 && panels_below(16, true, 1000, 4100000) == 0, "16 bits, 1 KiB");
+    CHECK(panels_below(16, true, 4000, 11000000) == 176 && panels_below(8, true, 1000, 1200000) == 0, "16 bits");
+    CHECK(panels_below(4, true, 250, 200000) == 176 && panels_below(4, true, 600, 500000) == 0, "16 bits, 256 bytes");
+    CHECK(panels_below(1, false, 6000, 6000 * 8 * 47) == 0 && panels_below(1, false, 6000, 6000 * 8 * 48) == 187, "short lists");
+}
+
 static void fused_panels() {
     for (int from : {0, 64, 128})
         for (int len = 1; len <= 5000; ++len) {
@@ -63,6 +74,7 @@ static void column_blocks() {
 }
 
 int main() {
+    tiles_or_panels();
     panels();
     column_blocks();
     fused_panels();

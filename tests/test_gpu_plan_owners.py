@@ -15,13 +15,18 @@ def _csr(rows):
     return rowptr, np.concatenate(rows).astype(np.int32)
 
 
-def _check(engine_factory, rows, N, K, rng, **counts):
+def _check(engine_factory, rows, N, K, rng, dtype=capi.F32, **counts):
     M = len(rows)
     rowptr, col = _csr(rows)
     val = rng.uniform(-1, 1, len(col)).astype(f32)
     A, B = rng.uniform(-1, 1, (M, K)).astype(f32), rng.uniform(-1, 1, (N, K)).astype(f32)
     e = engine_factory()
-    e.set_dense(A, B)
+    if dtype == capi.BF16:
+        Ab, Bb = capi.to_bf16(A).reshape(M, K), capi.to_bf16(B).reshape(N, K)
+        A, B = capi.from_bf16(Ab).reshape(M, K), capi.from_bf16(Bb).reshape(N, K)
+        e.set_dense(Ab, Bb, dtype)
+    else:
+        e.set_dense(A, B)
     e.set_csr(M, N, rowptr, col, val)
     e.plan(capi.AUTO)
     st = e.stats()
@@ -170,3 +175,18 @@ def test_window_order_with_gathered_pairs(engine_factory, monkeypatch, K):
     rows = [16 * s + np.arange(128) for s in range(40) for _ in range(16)] + rows          # 320 tiles of strips before them
     st = _check(engine_factory, rows, N, K, rng)
     assert st.mfma_tiles > 1000
+
+
+@pytest.mark.parametrize("per_tile,K,dtype,panels", [(160, 64, capi.F32, True), (176, 64, capi.F32, False), (176, 256, capi.F32, False),
+                                                     (160, 256, capi.F32, True), (176, 32, capi.F32, True), (192, 32, capi.F32, False),
+                                                     (160, 512, capi.BF16, False), (112, 512, capi.BF16, False), (112, 32, capi.BF16, True)])
+def test_strips_of_two_panels_without_a_mixture(engine_factory, per_tile, K, dtype, panels):
+    """Every strip holds the same number of entries per tile: the line that decides for a mixture decides here too."""
+    rng = np.random.default_rng(per_tile + K)
+    N, rows = 640, []
+    for _ in range(40):
+        lo = int(rng.integers(0, 30))
+        for _ in range(2):
+            rows += [np.concatenate([16 * (lo + t) + np.sort(rng.choice(16, per_tile // 16, replace=False)) for t in range(10)])] * 8
+    _check(engine_factory, rows, N, K, rng, dtype, panels=80 if panels else 0, mfma_tiles=0 if panels else 400)
+
