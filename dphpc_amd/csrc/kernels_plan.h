@@ -176,8 +176,9 @@ static __global__ __launch_bounds__(256) void k_check_rowptr(const int32_t *__re
 
 // every column index in [0,N).  Does nothing after a launch of k_check_rowptr that found the row pointer malformed: the
 // array need not hold n values then (the host reads both verdicts at once: one wait for the device, 20 us, instead of two).
+// sample: also counts, on some of the entries, how often neighbours lie in the same 16 columns.
 static __global__ __launch_bounds__(256) void k_check_index(const int32_t *__restrict__ idx, int64_t n,
-                                                     int bound, DevCounters *pc) {
+                                                     int bound, int sample, DevCounters *pc) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x * 4;
     if (pc->bad_pattern & BAD_POINTER) return;              // (this kernel sets the other bit only)
     unsigned int bad = 0, pairs = 0, near = 0;
@@ -193,8 +194,8 @@ static __global__ __launch_bounds__(256) void k_check_index(const int32_t *__res
         }
     }
     if (__ballot(bad != 0) && lane_id() == 0) atomicOr(&pc->bad_pattern, BAD_INDEX);
-    // How often neighbours lie in the same 16 columns: 64 to 128 workgroups count (thousands would wait for each other's
-    // atomics: 14 M entries 13 us, 24 with 1 700 of them)
+    if (!sample) return;
+    // 64 to 128 workgroups count (thousands would wait for each other's atomics: 14 M entries 13 us, 24 with 1 700 of them)
     const unsigned int each = gridDim.x > SPREAD ? gridDim.x / SPREAD : 1u;
     if (blockIdx.x % each == 0) {
         pairs = wave_sum_i32(pairs);

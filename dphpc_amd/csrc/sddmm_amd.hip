@@ -851,6 +851,12 @@ int clear_pattern(sddmm_ctx *c, int64_t nnz) {
     return SDDMM_OK;
 }
 
+// Checks the column indices and samples how near neighbours are to each other.
+void check_columns(sddmm_ctx *c) {
+    SDDMM_LAUNCH(c, k_check_index, grid_capped((c->nnz + 3) / 4, 256, 4096), 256, (const int32_t *)c->d_col, c->nnz, c->sN, 1, c->d_pc);
+}
+double columns_near(const PlanCounters &pc) { return pc.col_pairs ? (double)pc.col_near / (double)pc.col_pairs : 1.0; }
+
 // Validate the device-resident CSR and gather row statistics.
 int validate_csr(sddmm_ctx *c) {
     if (c->sM > 0)
@@ -858,14 +864,13 @@ int validate_csr(sddmm_ctx *c) {
                            c->nnz, c->d_pc);
     // (walks col[0..nnz) only behind a valid row pointer)
     if (c->nnz > 0)
-        SDDMM_LAUNCH(c, k_check_index, grid_capped((c->nnz + 3) / 4, 256, 4096), 256, c->d_col, c->nnz,
-                           c->sN, c->d_pc);
+        check_columns(c);
     LAUNCH_CHECK(c);
     const int rc = fetch_counters(c);
     if (rc) return rc;
     if (c->pc.bad_pattern & BAD_POINTER) return fail(c, SDDMM_ERR_PATTERN, "rowptr is not a valid CSR row pointer array");
     if (c->pc.bad_pattern) return fail(c, SDDMM_ERR_PATTERN, "column index outside [0,N)");
-    c->col_near = c->pc.col_pairs ? (double)c->pc.col_near / (double)c->pc.col_pairs : 1.0;
+    c->col_near = columns_near(c->pc);
     return SDDMM_OK;
 }
 
@@ -1333,9 +1338,8 @@ static int set_coo_common(sddmm_ctx *c, int M, int N, int64_t nnz, const int32_t
             HIP_TRY(c, hipMemcpyAsync(c->d_col, col, (size_t)nnz * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
             HIP_TRY(c, hipMemcpyAsync(c->d_sval, sval, (size_t)nnz * sizeof(float), hipMemcpyHostToDevice, c->stream));
         }
-        const int g = grid_capped(nnz, 256);
-        SDDMM_LAUNCH(c, k_check_index, g, 256, c->d_rowidx, nnz, M, c->d_pc);
-        SDDMM_LAUNCH(c, k_check_index, g, 256, c->d_col, nnz, N, c->d_pc);
+        SDDMM_LAUNCH(c, k_check_index, grid_capped((nnz + 3) / 4, 256, 4096), 256, (const int32_t *)c->d_rowidx, nnz, M, 0, c->d_pc);
+        check_columns(c);
         SDDMM_LAUNCH(c, k_check_coo_sorted, grid_capped(nnz, 256, 1024), 256, (const int32_t *)c->d_rowidx,
                            (const int32_t *)c->d_col, nnz, c->d_pc);
         LAUNCH_CHECK(c);
@@ -1348,7 +1352,7 @@ static int set_coo_common(sddmm_ctx *c, int M, int N, int64_t nnz, const int32_t
     }
     const bool sorted = c->pc.coo_unsorted == 0;
     c->coo_jumps = (int64_t)c->pc.coo_jumps;
-    c->col_near = 1.0;                                     // (not measured)
+    c->col_near = columns_near(c->pc);                     // (of entries in no order: of no use, they have no rows to look at)
     if (sorted) {
         SDDMM_LAUNCH(c, k_rowptr_from_sorted_coo, grid_for(nnz + 1, 256), 256,
                            c->d_rowidx, nnz, M, c->d_rowptr);

@@ -15,7 +15,7 @@ def _csr(rows):
     return rowptr, np.concatenate(rows).astype(np.int32)
 
 
-def _check(engine_factory, rows, N, K, rng, dtype=capi.F32, **counts):
+def _check(engine_factory, rows, N, K, rng, dtype=capi.F32, coo=False, **counts):
     M = len(rows)
     rowptr, col = _csr(rows)
     val = rng.uniform(-1, 1, len(col)).astype(f32)
@@ -27,7 +27,10 @@ def _check(engine_factory, rows, N, K, rng, dtype=capi.F32, **counts):
         e.set_dense(Ab, Bb, dtype)
     else:
         e.set_dense(A, B)
-    e.set_csr(M, N, rowptr, col, val)
+    if coo:
+        e.set_coo(M, N, np.repeat(np.arange(M, dtype=np.int32), np.diff(rowptr)), col, val)
+    else:
+        e.set_csr(M, N, rowptr, col, val)
     e.plan(capi.AUTO)
     st = e.stats()
     e.run()
@@ -189,4 +192,19 @@ def test_strips_of_two_panels_without_a_mixture(engine_factory, per_tile, K, dty
         for _ in range(2):
             rows += [np.concatenate([16 * (lo + t) + np.sort(rng.choice(16, per_tile // 16, replace=False)) for t in range(10)])] * 8
     _check(engine_factory, rows, N, K, rng, dtype, panels=80 if panels else 0, mfma_tiles=0 if panels else 400)
+
+
+@pytest.mark.parametrize("K", [75, 90])
+@pytest.mark.parametrize("near", [False, True])
+def test_sorted_coo_entries_are_looked_at_like_csr(engine_factory, near, K):
+    """The same matrix as row-sorted COO: rows of any length go to the tiles only where neighbours tend to share one."""
+    rng = np.random.default_rng(12)
+    N, rows = 40000, []
+    for i in range(4000):
+        lo = 16 * (i // 16)
+        rows.append(lo + np.arange(80) if near else np.sort(rng.choice(N, 80, replace=False)))
+    rows[:64] = [np.arange(256)] * 64
+    both = [_check(engine_factory, rows, N, K, np.random.default_rng(1), coo=coo) for coo in (False, True)]
+    assert (both[0].mfma_tiles, both[0].panels) == (both[1].mfma_tiles, both[1].panels)
+    assert (both[1].mfma_tiles > 0) == near
 
