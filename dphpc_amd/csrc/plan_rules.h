@@ -55,8 +55,10 @@ constexpr int panel_columns(int steps, bool half_width, int64_t panels, int64_t 
 }
 
 // Entries per tile below which 16-row strips that are two panels of `panels` (as many as the matrix has groups of 8 rows) go to
-// the panel kernel as panels, and from which they stay strips of dense tiles.  One line for a strip alone and, where some lie
-// above it and some below, for all of them together: tiles and panels are two launches.
+// the panel kernel as panels, and from which they are strips of dense tiles: all of them together, by their average, since
+// tiles and panels are two launches; for the same reason all of them are panels where others of the matrix are, up to
+// PANELS_AMONG_PANELS entries per tile (4 000 banded rows, 120 entries, a few panels among the strips: K = 32 13.3 us, all panels
+// 5.0, K = 512 bf16 37.7 and 15.6).
 // Time of tiles / time of panels, strips of one fill, 112 .. 208 entries per tile:
 //   rows of up to 128 bytes 0.92 .. 2.0, more with the size: 192, of fewer than 5 M entries 187 (a mixture of 205 and 125
 //   entries that averages that is better as tiles).
@@ -67,6 +69,7 @@ constexpr int panel_columns(int steps, bool half_width, int64_t panels, int64_t 
 //   16 bits, up to 1 000 panels: 512 bytes 0.76 .. 1.0 with up to 1.5 M entries, 1.1 .. 1.4 with more; 1 KiB 0.6 .. 1.0 up to 4 M
 //   entries, then 1.0 .. 1.2.
 //   3 000 and 6 000 panels of 28 .. 48 columns, a step of 64 half empty: 0.78 .. 0.96.
+constexpr int PANELS_AMONG_PANELS = 192;
 constexpr int panels_below(int steps, bool half_width, int64_t panels, int64_t nnz) {
     constexpr int never = 0;
     const bool few = panels <= 1280, some = few && panels > 512;

@@ -984,8 +984,7 @@ int do_plan(sddmm_ctx *c, int strategy) {
             if (tiles && gathered && c->sM >= 2) rules.cand_min = std::max(16, env_int("SDDMM_GATHERED_MIN", 64));
             const int pseg = panel_item_columns(c);
             rules.pseg = pseg;
-            // (long rows take either kernel 512 bytes at a time)
-            rules.panels_below = panels_below(c->long_rows ? 16 : panel_steps(c), c->dtype != SDDMM_F32, c->sM / PANEL_ROWS, c->nnz);
+            rules.panels_below = PANELS_AMONG_PANELS;                // (settled below)
             // the rows nobody owns so far are classified in the same launch: most matrices have
             // no gathered strips, and their plan then waits for the device once
             c->ts = rules.ts = std::max(1, env_int("SDDMM_TS", 24));
@@ -1002,15 +1001,20 @@ int do_plan(sddmm_ctx *c, int strategy) {
             if (rc) return rc;
             rc = fetch_counters(c);
             if (rc) return rc;
-            // Strips that are two panels each, some above the line and some below it: all of them go the way that their average
-            // says, since tiles and panels are two launches.  (Launch us, all strips / mixed / all panels: 2 000 rows in a band,
-            // 155 entries per tile, K = 32 5.2 / 8.6 / 4.2, K = 512 bf16 8.9 / 13.9 / 10.4; 120 entries, 4 000 rows, K = 32 13.3
-            // with a few panels among strips, 5.0 as panels.)
-            if (c->pc.nnz_either_strip && c->pc.nnz_either_panels) {
-                const unsigned long long entries = c->pc.nnz_either_strip + c->pc.nnz_either_panels;
-                rc = settle_owners(c, entries < (unsigned long long)rules.panels_below * c->pc.either_tiles, pseg);
-                if (!rc) rc = fetch_counters(c);
-                if (rc) return rc;
+            // Strips that are two panels each: all of them go the way that their average says.  (Launch us, all strips / some /
+            // all panels: 2 000 rows in a band, 155 entries per tile, K = 32 5.2 / 8.6 / 4.2, K = 512 bf16 8.9 / 13.9 / 10.4.)
+            if (c->pc.either_tiles) {
+                const uint64_t either = c->pc.nnz_either_strip + c->pc.nnz_either_panels;
+                const bool among_panels = c->pc.nnz_panels - c->pc.nnz_either_panels > either / 16;
+                // (long rows take either kernel 512 bytes at a time)
+                const int line = among_panels ? PANELS_AMONG_PANELS
+                                              : panels_below(c->long_rows ? 16 : panel_steps(c), c->dtype != SDDMM_F32, c->sM / PANEL_ROWS, c->nnz);
+                const bool to_panels = either < (uint64_t)line * c->pc.either_tiles;
+                if (to_panels ? c->pc.nnz_either_strip : c->pc.nnz_either_panels) {
+                    rc = settle_owners(c, to_panels, pseg);
+                    if (!rc) rc = fetch_counters(c);
+                    if (rc) return rc;
+                }
             }
             rc = take_tile_counts(c);
             if (rc) return rc;

@@ -208,3 +208,15 @@ def test_sorted_coo_entries_are_looked_at_like_csr(engine_factory, near, K):
     assert (both[0].mfma_tiles, both[0].panels) == (both[1].mfma_tiles, both[1].panels)
     assert (both[1].mfma_tiles > 0) == near
 
+
+@pytest.mark.parametrize("K,dtype", [(512, capi.BF16), (64, capi.F32)])
+def test_strips_among_panels_go_with_them(engine_factory, K, dtype):
+    """Strips that are two panels, which would be tiles by themselves, next to panels that are not: one launch."""
+    rng = np.random.default_rng(K)
+    N, rows = 3000, []
+    for i in range(60):
+        lo = int(rng.integers(0, 160))
+        for _ in range(2):
+            rows += [np.concatenate([16 * (lo + t) + np.sort(rng.choice(16, 11, replace=False)) for t in range(10)])] * 8
+        rows += [np.sort(rng.choice(N, 110, replace=False))] * 8 + [np.sort(rng.choice(N, 110, replace=False))] * 8
+    _check(engine_factory, rows, N, K, rng, dtype, panels=240, mfma_tiles=0)
