@@ -81,6 +81,13 @@ constexpr int panels_below(int steps, bool half_width, int64_t panels, int64_t n
     return many && steps <= 8 ? 192 : 176;
 }
 
+// The same for rows of more than 1 KiB, whose tiles always split K over a workgroup and whose panels take a launch per 512 bytes:
+// 16 bits 0.24 .. 0.76 at 100 .. 224 entries per tile; fp32 0.38 .. 0.89 with 0.2 .. 0.8 M entries, 0.8 .. 1.3 with 0.8 .. 1.8 M (1.0
+// from 144 entries per tile on), 1.2 .. 1.6 with 1.6 .. 2.6 M.
+constexpr int long_panels_below(bool half_width, int64_t nnz) {
+    return half_width || nnz < (int64_t)1 << 20 ? 0 : nnz < (int64_t)3 << 19 ? 144 : PANELS_AMONG_PANELS;
+}
+
 // Columns of a work item of the fused call: a panel of up to 1 024 columns is one item, or two where that leaves wavefronts
 // of the chip something to do (halves_from: from more columns on; 0: not).  The items of a panel add their part of the
 // output rows atomically to zeros: two sums come out the same in either order, three do not.

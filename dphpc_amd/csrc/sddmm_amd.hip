@@ -1006,9 +1006,10 @@ int do_plan(sddmm_ctx *c, int strategy) {
             if (c->pc.either_tiles) {
                 const uint64_t either = c->pc.nnz_either_strip + c->pc.nnz_either_panels;
                 const bool among_panels = c->pc.nnz_panels - c->pc.nnz_either_panels > either / 16;
-                // (long rows take either kernel 512 bytes at a time)
+                const bool half_width = c->dtype != SDDMM_F32;
                 const int line = among_panels ? PANELS_AMONG_PANELS
-                                              : panels_below(c->long_rows ? 16 : panel_steps(c), c->dtype != SDDMM_F32, c->sM / PANEL_ROWS, c->nnz);
+                               : c->long_rows ? long_panels_below(half_width, c->nnz)
+                                              : panels_below(panel_steps(c), half_width, c->sM / PANEL_ROWS, c->nnz);
                 const bool to_panels = either < (uint64_t)line * c->pc.either_tiles;
                 if (to_panels ? c->pc.nnz_either_strip : c->pc.nnz_either_panels) {
                     rc = settle_owners(c, to_panels, pseg);

@@ -42,6 +42,8 @@ static void tiles_or_panels() {
     CHECK(panels_below(16, true, 250, 200000) == 0 && panels_below(16, true, 1000, 4100000) == 0, "16 bits, 1 KiB");
     CHECK(panels_below(16, true, 4000, 11000000) == 176 && panels_below(8, true, 1000, 1200000) == 0, "16 bits");
     CHECK(panels_below(4, true, 250, 200000) == 176 && panels_below(4, true, 600, 500000) == 0, "16 bits, 256 bytes");
+    CHECK(long_panels_below(true, 100000000) == 0 && long_panels_below(false, 700000) == 0, "long rows");
+    CHECK(long_panels_below(false, 1200000) == 144 && long_panels_below(false, 1800000) == 192, "long rows, many entries");
     CHECK(panels_below(1, false, 6000, 6000 * 8 * 47) == 0 && panels_below(1, false, 6000, 6000 * 8 * 48) == 187, "short lists");
 }
 

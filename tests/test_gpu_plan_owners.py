@@ -182,9 +182,11 @@ def test_window_order_with_gathered_pairs(engine_factory, monkeypatch, K):
 
 @pytest.mark.parametrize("per_tile,K,dtype,panels", [(160, 64, capi.F32, True), (176, 64, capi.F32, False), (176, 256, capi.F32, False),
                                                      (160, 256, capi.F32, True), (176, 32, capi.F32, True), (192, 32, capi.F32, False),
-                                                     (160, 512, capi.BF16, False), (112, 512, capi.BF16, False), (112, 32, capi.BF16, True)])
-def test_strips_of_two_panels_without_a_mixture(engine_factory, per_tile, K, dtype, panels):
+                                                     (160, 512, capi.BF16, False), (112, 512, capi.BF16, False), (112, 32, capi.BF16, True),
+                                                     (112, 300, capi.F32, False), (160, 600, capi.BF16, False)])
+def test_strips_of_two_panels_without_a_mixture(engine_factory, monkeypatch, per_tile, K, dtype, panels):
     """Every strip holds the same number of entries per tile: the line that decides for a mixture decides here too."""
+    monkeypatch.setenv("SDDMM_LONG_TILES", "1")
     rng = np.random.default_rng(per_tile + K)
     N, rows = 640, []
     for _ in range(40):
