@@ -33,6 +33,44 @@ constexpr int64_t row_block_segments(int64_t n_long, int64_t nnz_long, int piece
     return nnz_long / piece + (most < by_length ? most : by_length);
 }
 
+// ---- rows of any length on the tile and panel kernels --------------------------------------------
+// Rows of 64 * {1, 2, 4, 8, 16} bytes are always looked at.  For the others the look costs a plan 8 us (1 000 rows) to 40 (4 M
+// entries), where it finds gathered strips 60, and the launch gains what `steps` 64-byte steps times the entries are worth to it.  A
+// caller who plans a pattern once has the cost back soon in any case; a caller with a new pattern for every launch never has
+// unless one launch gains it.  The lines lie where two to four launches do.
+
+// Share of the entries that lie in the same 16 columns as the one before them (a sample, from the check of the columns): 1.0
+// in banded blocks and dense tiles, 0.7 where near-dense rows hold most of the entries, 0.02 .. 0.06 in graphs and uniform
+// rows, 0.5 where those have few columns.
+constexpr double STRUCTURED_NEAR = 0.85, GATHERED_NEAR = 0.6;
+
+// Entries from which structured patterns of `steps` steps are looked at.  Launch without / with, us, and set, plan and launch
+// without / with: dense tiles of 1.2 M entries K = 9 6.6 / 6.2, 83 / 105, K = 33 15.9 / 6.1, 92 / 105, K = 75 21.4 / 8.7, 98 / 108,
+// K = 100 27.8 / 8.7, 103 / 109; 2.4 M K = 15 11.1 / 7.0, 89 / 118; 4 M K = 15 17.2 / 8.8, 96 / 129, K = 21 23.3 / 10.7, 103 /
+// 131, K = 33 43.9 / 13.5, 123 / 134; 0.4 M K = 33 8.9 / 4.3, 83 / 95, K = 75 10.9 / 5.3, 85 / 96; banded blocks of 0.96 M K = 21
+// 7.8 / 6.1, 82 / 96, K = 51 11.7 / 8.1, 86 / 99, K = 100 19.7 / 9.7, 93 / 100; 3.8 M K = 15 16 / 10, 96 / 98, K = 40 bf16 28 / 10,
+// 106 / 98, K = 75 59 / 28, 139 / 113; 14 M K = 21 69 / 29.
+constexpr int64_t ragged_entries(int steps) {
+    return steps <= 1 ? 3 << 20 : steps <= 2 ? 3 << 19 : steps <= 4 ? 3 << 18 : steps <= 6 ? 5 << 16 : 1 << 16;
+}
+
+// Near-dense rows among others: their gathered strips are all there is to find.  Launch without / with, set, plan and launch
+// without / with: 2 M entries K = 33 29.9 / 21.1, 111 / 169, K = 75 70.0 / 36.8, 150 / 184, K = 100 68.8 / 56.2, 151 / 202, K = 133
+// 118.6 / 74.7, 203 / 222, K = 120 bf16 48.5 / 21.5, 129 / 169, K = 200 bf16 90.1 / 32.4, 172 / 178; 0.8 M K = 75 24.4 / 18.4,
+// 104 / 156, K = 200 bf16 31.5 / 15.7, 110 / 153, K = 456 bf16 69.5 / 35.8, 153 / 173.  fp32 rows of more than twelve steps leave a wavefront per SIMD: K = 200
+// 108 / 155.
+constexpr int ragged_gathered_steps(bool half_width) { return half_width ? 16 : 12; }
+constexpr int64_t ragged_gathered_entries(int steps, bool half_width) {
+    return (half_width ? 7 << 20 : steps <= 6 ? 1 << 23 : 1 << 24) / steps;
+}
+
+// Rows of more than 1 KiB, which the tile and panel kernels take 512 bytes at a time.  Launch without / with: 0.27 M entries in
+// 170 panels of 200 columns K = 260 26 / 23, K = 512 26 / 34, K = 1000 63 / 68; 0.48 M in 375 panels K = 300 32 / 26, K = 452 33 /
+// 36, K = 700 77 / 57, K = 1024 bf16 34 / 44; 0.67 M in 300 panels K = 452 47 / 41; 0.96 M in 750 panels K = 512 100 / 53; dense
+// tiles of 0.29 M K = 260 .. 512 28 / 11 .. 14, of 0.4 M K = 452 40 / 16, K = 1024 bf16 45 / 11.  (Rows of 1.5 to 2 KiB, which the
+// gather kernels hold in registers, are four launches of the panel kernel: the only ones that lose.)
+constexpr int64_t long_row_entries(int64_t row_bytes) { return row_bytes <= 1536 ? 1 << 18 : 17 << 14; }
+
 // ---- 8-row panels ---------------------------------------------------------------------------
 constexpr int PANEL_COLUMNS = 512;             // columns of a panel's work item, at the most
 

@@ -326,35 +326,23 @@ bool tile_path_applies(sddmm_ctx *c) {
     return c->tile_steps != 0;
 }
 
-// Ragged rows on the tile and panel kernels instead of the gather kernels.  Measured: banded blocks of 2 000 .. 36 000 rows,
-// dense tiles of 100 k .. 2.5 M entries, near-dense rows, K = 9 .. 250 in fp32 and 24 .. 456 in 16 bits: 36 000 banded rows
-// K = 21 69 -> 29 us, K = 100 407 -> 74, K = 120 bf16 137 -> 39; dense tiles K = 100 48.7 -> 14.7, K = 200 bf16 53 -> 10;
-// near-dense rows K = 75 70 -> 36, K = 120 bf16 49 -> 21.  Few entries: a launch of a few microseconds either way, and the
-// plan has more to look at (100 k entries in dense tiles K = 21 4.3 us without, 5.3 with; K = 100 6.8 and 4.6).  Entries
-// that hardly ever share 16 columns with their neighbour fill no tile and no near-dense row: the plan need not look
-// (0.02 .. 0.06 in graphs and uniform rows, around 0.5 where those have few columns, 0.7 .. 0.95 in the shapes above; 20 000
-// uniform rows 13 us of a new pattern, a graph of 8 600 rows K = 54 85 without, 97 with).
-bool ragged_pays(const sddmm_ctx *c) {
-    const int steps = ragged_steps(c), mode = env_int("SDDMM_RAGGED", -1);       // -1: decide here, 0: never, 1: wherever it can
-    if (mode >= 0) return mode != 0 && steps != 0;
-    return steps != 0 && c->nnz >= (steps <= 1 ? 1 << 19 : steps <= 2 ? 1 << 18 : 1 << 16) && c->col_near >= 0.6;
-}
-
-// Gathered strips of ragged rows?  They cost 55 us of a plan more.  Not for little work (a launch without / with them, 64-byte
-// steps times entries: 1 .. 2.3 M 7.2 / 6.6 .. 13.7 / 10.7 us; 6.5 M 40.8 / 25.0; 14 M 85.8 / 30.7; of nine fp32 steps 4.7 M
-// 31.2 / 33.0), not for fp32 rows of more than twelve (a wavefront per SIMD; near-dense rows K = 200 108 us without, 155 with).
+// Ragged rows on the tile and panel kernels instead of the gather kernels, and their gathered strips?
 bool ragged_gathers(const sddmm_ctx *c) {
-    const int steps = ragged_steps(c);
-    if (c->long_rows || (c->dtype == SDDMM_F32 && steps > 12)) return false;
-    return env_int("SDDMM_RAGGED", -1) > 0 || c->nnz * steps >= (c->dtype == SDDMM_F32 && steps > 8 ? 1 << 24 : 1 << 22);
+    const int steps = ragged_steps(c), mode = env_int("SDDMM_RAGGED", -1);       // -1: decide here, 0: never, 1: wherever it can
+    if (c->long_rows || steps > ragged_gathered_steps(c->dtype != SDDMM_F32)) return false;
+    return mode > 0 || c->nnz >= ragged_gathered_entries(steps, c->dtype != SDDMM_F32);
+}
+bool ragged_pays(const sddmm_ctx *c) {
+    const int steps = ragged_steps(c), mode = env_int("SDDMM_RAGGED", -1);
+    if (steps == 0 || mode >= 0) return steps != 0 && mode != 0;
+    return c->col_near >= STRUCTURED_NEAR ? c->nnz >= ragged_entries(steps) : c->col_near >= GATHERED_NEAR && ragged_gathers(c);
 }
 
-// Rows of more than 1 KiB on the tile and panel kernels, if they own nearly all of the entries.  (Slices / dense tiles: 303 k
-// entries K = 452 30.9 / 14.7 us.)
+// Rows of more than 1 KiB on the tile and panel kernels, if they own nearly all of the entries?
 bool long_pays(const sddmm_ctx *c) {
     const int mode = env_int("SDDMM_LONG_TILES", -1);              // -1: decide here, 0: never, 1: wherever it can
     if (!rows_are_long(c) || mode == 0) return false;
-    return mode > 0 || (c->nnz >= 1 << 18 && c->col_near >= 0.6);
+    return mode > 0 || (c->nnz >= long_row_entries((int64_t)c->K * (int64_t)elem_size(c->dtype)) && c->col_near >= STRUCTURED_NEAR);
 }
 
 // A workgroup of 16 wavefronts per strip, not four strips to a workgroup of four wavefronts: where the chip holds them all at
@@ -365,15 +353,12 @@ bool strips_are_wide(const sddmm_ctx *c) {
     return n_strips <= 512 && c->nnz >= 2048 * n_strips;
 }
 
-// After the classifiers: panels of ragged or long rows, and too few of them for kernels that occupy the chip with one or two
-// wavefronts per SIMD, or that are a launch per 512 bytes.  (Gather kernels / panels: 117 panels of 224 columns, fp32 K = 200
-// 10.8 / 12.7 us, K = 512 309 k entries 24.0 / 33.6, 509 k K = 390 36.7 / 42.7; 577 k K = 196 22.3 / 15.4, 793 k K = 858 167 /
-// 71; bf16 573 k K = 752 49.3 / 38.3.)
+// After the classifiers: panels of ragged fp32 rows of more than 512 bytes, and too few of them for kernels that occupy the chip
+// with one or two wavefronts per SIMD.  (Gather kernels / panels: 117 panels of 224 columns K = 200 10.8 / 12.7 us; 577 k
+// entries K = 196 22.3 / 15.4.)
 bool too_few_panels(const sddmm_ctx *c) {
-    if (!c->ragged || (int64_t)c->pc.nnz_panels <= c->nnz / 2) return false;
-    const bool f32 = c->dtype == SDDMM_F32;
-    if (c->long_rows) return env_int("SDDMM_LONG_TILES", -1) < 0 && c->nnz < (f32 ? 3 << 18 : 1 << 19);
-    return env_int("SDDMM_RAGGED", -1) < 0 && f32 && ragged_steps(c) > 8 && c->nnz < 1 << 18;
+    if (!c->ragged || c->long_rows || (int64_t)c->pc.nnz_panels <= c->nnz / 2) return false;
+    return env_int("SDDMM_RAGGED", -1) < 0 && c->dtype == SDDMM_F32 && ragged_steps(c) > 8 && c->nnz < 1 << 18;
 }
 
 // The rows' owners and, of the rows that are left, the candidates of the gathered strips and the row classes (launches

@@ -59,6 +59,22 @@ static void fused_panels() {
     CHECK(fused_halves_from(512, 1, true) == 128 && fused_halves_from(513, 1, true) == 0, "one wavefront per SIMD");
 }
 
+// A launch of few short steps never pays for a longer plan; longer rows and more entries do.
+static void rows_of_any_length() {
+    int64_t before = INT64_MAX;
+    for (int steps : {1, 2, 4, 6, 8, 12, 16}) {
+        CHECK(ragged_entries(steps) <= before, "%d steps", steps);
+        before = ragged_entries(steps);
+        for (bool half : {false, true}) CHECK(ragged_gathered_entries(steps, half) * steps <= 1 << 24, "%d steps", steps);
+    }
+    CHECK(ragged_entries(1) > 5 << 19 && ragged_entries(2) > 5 << 18 && ragged_entries(4) > 1 << 19, "rows of up to 256 bytes");
+    CHECK(ragged_entries(1) <= 3840000 && ragged_entries(4) <= 960000, "a launch that gains more than the look costs");
+    CHECK(ragged_entries(6) <= 331264 && ragged_entries(8) <= 96000, "longer rows");
+    CHECK(ragged_gathered_entries(6, false) <= 1960000 && ragged_gathered_entries(8, false) > 1960000, "near-dense rows");
+    CHECK(ragged_gathered_entries(4, true) <= 1960000 && ragged_gathered_entries(4, false) > 1960000, "near-dense rows, 16 bits");
+    CHECK(long_row_entries(1200) == 1 << 18 && long_row_entries(2048) > 272000 && long_row_entries(4000) <= 287744, "beyond 1 KiB");
+}
+
 // Rows of every length: a power of two that divides `most` (the lanes of a row), the bound that sizes the list of segments.
 static void column_blocks() {
     for (bool sorted : {false, true})
@@ -76,6 +92,7 @@ static void column_blocks() {
 }
 
 int main() {
+    rows_of_any_length();
     tiles_or_panels();
     panels();
     column_blocks();

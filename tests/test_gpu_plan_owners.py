@@ -211,6 +211,39 @@ def test_sorted_coo_entries_are_looked_at_like_csr(engine_factory, near, K):
     assert (both[1].mfma_tiles > 0) == near
 
 
+@pytest.mark.parametrize("kind,K,looked", [("tiles", 15, False), ("tiles", 33, False), ("tiles", 75, True), ("tiles", 100, True),
+                                           ("panels", 300, True), ("panels", 512, False), ("tiles", 512, True), ("near-dense", 75, False)])
+def test_rows_of_any_length_are_looked_at_where_launches_pay(engine_factory, kind, K, looked):
+    """Structured rows of no whole number of steps: short rows and few entries stay on the gather kernels, since a plan that
+    looks at them costs more than several launches gain; longer rows do not."""
+    rng = np.random.default_rng(K)
+    N, rows = 4000, []
+    if kind == "tiles":                                          # 338 688 entries
+        for _ in range(42):
+            rows += [(16 * np.sort(rng.choice(N // 16, 36, replace=False))[:, None] + np.arange(16)[None, :]).ravel()[:504]] * 16
+    elif kind == "panels":                                       # 272 000
+        for _ in range(170):
+            rows += [(8 * np.sort(rng.choice(N // 8, 25, replace=False))[:, None] + np.arange(8)[None, :]).ravel()] * 8
+    else:                                                        # 0.83 M, most of them in 1 400 near-dense rows
+        for i in range(9400):
+            lo = int(rng.integers(0, N - 1385))
+            rows.append(lo + np.flatnonzero(rng.random(1385) < 0.4) if i % 7 == 0 else np.sort(rng.choice(N, 9, replace=False)))
+    M = len(rows)
+    rowptr, col = _csr(rows)
+    val = rng.uniform(-1, 1, len(col)).astype(f32)
+    A, B = rng.uniform(-1, 1, (M, K)).astype(f32), rng.uniform(-1, 1, (N, K)).astype(f32)
+    e = engine_factory()
+    e.set_dense(A, B)
+    e.set_csr(M, N, rowptr, col, val)
+    e.plan(capi.AUTO)
+    st = e.stats()
+    assert (st.mfma_tiles + st.panels > 0) == looked, (len(col), st.mfma_tiles, st.panels)
+    e.run()
+    ok, worst, i = O.check_values(e.values(), O.sddmm_csr(rowptr, col, val, A, B, threads=0), mag=O.sddmm_csr_f64(rowptr, col, val, A, B)[1])
+    assert ok, (i, worst)
+    e.close()
+
+
 @pytest.mark.parametrize("K,dtype", [(512, capi.BF16), (64, capi.F32)])
 def test_strips_among_panels_go_with_them(engine_factory, K, dtype):
     """Strips that are two panels, which would be tiles by themselves, next to panels that are not: one launch."""
