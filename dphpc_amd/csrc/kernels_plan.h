@@ -463,8 +463,8 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_small(const unsigned
 }
 
 // Several short scans in one launch: workgroup j takes job j (in == out is allowed: a thread
-// writes only the positions it has read).  With a place for the totals in host memory, whose jobs' totals are among the
-// first SCAN_TOTALS of DevCounters, one more workgroup reports the counters.
+// writes only the positions it has read).  With a place for the totals in host memory one more workgroup reports the
+// counters, and every job its total if that is one of the first SCAN_TOTALS of DevCounters.
 constexpr int SCAN_JOBS_MAX = 8;
 struct ScanJob {
     const unsigned int *in;
@@ -558,7 +558,8 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_jobs(ScanJobs jobs, 
     }
     if (threadIdx.x == 0) {
         *jb.total = carry;
-        if (totals) (&totals->n_items)[jb.total - &pc->n_items] = carry;
+        const int slot = scan_total_slot(jb.total, &pc->n_items, SCAN_TOTALS);
+        if (totals && slot >= 0) (&totals->n_items)[slot] = carry;
     }
 }
 

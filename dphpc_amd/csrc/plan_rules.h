@@ -5,6 +5,12 @@
 
 namespace sddmm {
 
+// ---- reports of the counters (k_scan_jobs) -----------------------------------------------------
+// Place of a scan's total among the n that are reported, counted from the first one; -1: not one of them.
+constexpr int scan_total_slot(const unsigned long long *total, const unsigned long long *first, int n) {
+    return total >= first && total < first + n ? (int)(total - first) : -1;
+}
+
 // ---- column blocks of a long row (kernels_flat.h) ---------------------------------------------
 // A power of two, `least` to `most`, such that the segments hold COL_BLOCK_ENTRIES entries or more on average (beyond `least`
 // blocks).  More blocks find more lines of B in an XCD's L2, short segments leave lanes idle and are work items more.  16 blocks

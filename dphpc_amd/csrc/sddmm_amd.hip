@@ -146,6 +146,7 @@ void release_sparse(sddmm_ctx *c, bool idle = false) {
     c->tiles_active = false;
     c->d_col = nullptr; c->d_sval = nullptr; c->d_rowptr = nullptr; c->d_rowidx = nullptr;
     c->own_sparse = c->own_rowptr = c->own_rowidx = false;
+    c->n_scan_jobs = 0;                       // (of a plan that failed: their arrays are gone)
     c->have_sparse = c->have_rowptr = false;
     c->from_coo = false;
     c->planned = false;
