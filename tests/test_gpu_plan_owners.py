@@ -196,8 +196,7 @@ def test_strips_of_two_panels_without_a_mixture(engine_factory, monkeypatch, per
     _check(engine_factory, rows, N, K, rng, dtype, panels=80 if panels else 0, mfma_tiles=0 if panels else 400)
 
 
-@pytest.mark.parametrize("K", [75, 90])
-@pytest.mark.parametrize("near", [False, True])
+@pytest.mark.parametrize("K,near", [(75, False), (75, True), (90, False), (90, True), (300, True)])
 def test_sorted_coo_entries_are_looked_at_like_csr(engine_factory, near, K):
     """The same matrix as row-sorted COO: rows of any length go to the tiles only where neighbours tend to share one."""
     rng = np.random.default_rng(12)

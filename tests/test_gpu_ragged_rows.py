@@ -113,6 +113,38 @@ def test_ragged_rows_keep_infinities_to_themselves(engine_factory, monkeypatch, 
     np.testing.assert_array_equal(np.isnan(out[1]), np.isnan(out[0]))
 
 
+@pytest.mark.parametrize("K,dtype", KS)
+def test_ragged_rows_tile_by_tile(engine_factory, monkeypatch, K, dtype):
+    """The kernels of well-filled tiles, whatever the fill: tiles walked from their masks together with the rows, K split over the
+    waves of a workgroup (from four steps on), a wavefront per window; non-finite values included."""
+    M, N, rowptr, col, val, rng = _structured(2000 + K)
+    Ad, Bd, A, B = _operands(rng, M, N, K, dtype)
+    ref = O.sddmm_csr(rowptr, col, val, A, B)
+    _, mag = O.sddmm_csr_f64(rowptr, col, val, A, B)
+    A, B = A.copy(), B.copy()
+    for k in (0, K - 8 if K > 8 else 1, K - 4, K - 1):
+        A[int(rng.integers(0, M)), k] = np.inf
+        B[int(rng.integers(0, N)), k] = np.nan
+    B[N - 1, K - 1] = -np.inf
+    Ai, Bi = (A, B) if dtype == capi.F32 else [(capi.to_bf16 if dtype == capi.BF16 else capi.to_f16)(x).reshape(x.shape) for x in (A, B)]
+    e = engine_factory()
+    monkeypatch.setenv("SDDMM_RAGGED", "0")
+    plain, _ = _run(e, M, N, rowptr, col, val, Ai, Bi, dtype)
+    assert not np.isfinite(plain).all()
+    monkeypatch.setenv("SDDMM_RAGGED", "1")
+    monkeypatch.setenv("SDDMM_WINDOW_FILL", "0")                 # no windows
+    for fuse, ksplit in (("1", "1"), ("0", "1"), ("0", "0")):
+        monkeypatch.setenv("SDDMM_FUSE", fuse)
+        monkeypatch.setenv("SDDMM_KSPLIT", ksplit)
+        got, st = _run(e, M, N, rowptr, col, val, Ad, Bd, dtype)
+        assert st.mfma_tiles > 0 and st.kernels_launched == (2 if fuse == "1" else 3)
+        ok, worst, i = O.check_values(got, ref, mag=mag)
+        assert ok, (K, dtype, fuse, ksplit, i, got[i], ref[i], worst)
+        got, _ = _run(e, M, N, rowptr, col, val, Ai, Bi, dtype)
+        np.testing.assert_array_equal(np.isfinite(got), np.isfinite(plain))
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(plain))
+
+
 LONG = [(K, capi.F32) for K in (257, 260, 300, 384, 511, 512, 516, 640, 1000, 1025)]
 LONG += [(K, d) for d in (capi.BF16, capi.F16) for K in (520, 600, 768, 1024, 1032)]
 
