@@ -441,8 +441,7 @@ __device__ __forceinline__ void entry_list_body(const void *__restrict__ A, cons
 // time in storage order (64 / 128 / 256, with workgroups of one wavefront: 2.6 M rows 427 / 450 / 460 us, 1 M rows 150 /
 // 159 / 160, 200 000 rows K = 100 in the same order), after the segments on every XCD (before
 // them: the same; dealt out evenly: 542 against 524 us with workgroups of four).
-// totals[0], totals[1]: work items of either kind (the grid is sized for an upper bound)
-//
+// totals[0], totals[1]: work items of either kind (what the grid is sized for, or less: launch_flat_blocks)
 template <class L, bool SCALED>
 __global__ __launch_bounds__(block_item_waves(L::UPL) * WAVE)
 void k_flat_blocks(const unsigned long long *__restrict__ totals, const RowItem *__restrict__ segments,

@@ -29,8 +29,8 @@ struct PlanCounters {
 
 // The same counters on the device.  Sums that thousands of workgroups contribute to
 // are spread over SPREAD slots chosen by workgroup id (same-address atomics were
-// measured at ~10 ns each, which made the counting kernels atomic-bound); the host
-// adds the slots up after the copy.
+// measured at ~10 ns each, which made the counting kernels atomic-bound);
+// report_totals adds the slots up.
 constexpr int SPREAD = 64;
 enum CounterKind {
     K_ROWS_NONEMPTY = 0,
@@ -435,32 +435,8 @@ static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_block_sums(const uns
     if (threadIdx.x == 0) *total_out = carry;
 }
 
-// the whole exclusive scan of a short array in one workgroup (one launch instead of three)
-constexpr int SCAN_SMALL_ITEMS = 8;
+constexpr int SCAN_SMALL_ITEMS = 8;                // words per thread and step of a short scan
 constexpr int SCAN_SMALL_MAX = 16384;
-static __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_small(const unsigned int *__restrict__ in, int n,
-                                                           unsigned int *__restrict__ out,
-                                                           unsigned long long *__restrict__ total_out) {
-    unsigned int carry = 0;
-    for (int base = 0; base < n; base += SCAN_BLOCK * SCAN_SMALL_ITEMS) {
-        const int i0 = base + (int)threadIdx.x * SCAN_SMALL_ITEMS;
-        unsigned int v[SCAN_SMALL_ITEMS], mine = 0;
-#pragma unroll
-        for (int q = 0; q < SCAN_SMALL_ITEMS; ++q) {
-            v[q] = i0 + q < n ? in[i0 + q] : 0u;
-            mine += v[q];
-        }
-        unsigned int total;
-        unsigned int at = carry + block_exclusive_scan(mine, &total);
-#pragma unroll
-        for (int q = 0; q < SCAN_SMALL_ITEMS; ++q) {
-            if (i0 + q < n) out[i0 + q] = at;
-            at += v[q];
-        }
-        carry += total;
-    }
-    if (threadIdx.x == 0) *total_out = carry;
-}
 
 // Several short scans in one launch: workgroup j takes job j (in == out is allowed: a thread
 // writes only the positions it has read).  With a place for the totals in host memory one more workgroup reports the
