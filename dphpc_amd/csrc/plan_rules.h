@@ -20,7 +20,8 @@ constexpr int scan_total_slot(const unsigned long long *total, const unsigned lo
 // 226, 259, 27.1, 118, 265.
 // Entries that came in no order were sorted by row and by 16 blocks, and keep them, whatever the row: 8 and 16 / 16, with the
 // unsorting, 400 000 rows K = 128 310.7 / 304.4 us, K = 200 550 / 540; 1 M rows K = 100 816 / 799, K = 75 703 / 688; 100 000 rows
-// K = 200 108.6 / 106.6, K = 75 50.0 / 50.6, with new inputs in turn 54.8 / 51.6; up to 64 floats a row 1 % the other way.
+// K = 200 108.6 / 106.6, K = 75 50.0 / 50.6, with new inputs in turn 53.5 / 53.2 (the same run twice differs by 2 %); up to 64
+// floats a row 1 % the other way.
 constexpr int COL_BLOCKS_MIN = 8, COL_BLOCKS_MAX = 64, COL_BLOCK_ENTRIES = 64;
 constexpr int COL_BLOCKS_ORDER = 16;           // that the sort of COO entries knows
 constexpr int row_blocks(int len, int least, int most) {
@@ -43,7 +44,9 @@ constexpr int64_t row_block_segments(int64_t n_long, int64_t nnz_long, int piece
 // Rows of 64 * {1, 2, 4, 8, 16} bytes are always looked at.  For the others the look costs a plan 8 us (1 000 rows) to 40 (4 M
 // entries), where it finds gathered strips 60, and the launch gains what `steps` 64-byte steps times the entries are worth to it.  A
 // caller who plans a pattern once has the cost back soon in any case; a caller with a new pattern for every launch never has
-// unless one launch gains it.  The lines lie where two to four launches do.
+// unless one launch gains it.  The lines lie where about three launches of dense tiles do; of banded blocks, which gain less, it
+// takes four to nine there (rows of 3 and 4 steps, 0.72 M entries in bands: 9.2 .. 10.3 / 7.1 us, plan 13 us longer; 0.62 M in tiles 9.8 ..
+// 10.4 / 5.1, 17 us).
 
 // Share of the entries that lie in the same 16 columns as the one before them (a sample, from the check of the columns): 1.0
 // in banded blocks and dense tiles, 0.7 where near-dense rows hold most of the entries, 0.02 .. 0.06 in graphs and uniform
