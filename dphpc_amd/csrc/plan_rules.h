@@ -92,13 +92,29 @@ constexpr int PANEL_COLUMNS = 512;             // columns of a panel's work item
 // 240 random columns K = 128 19.9, K = 64 fp16 7.55; 2 000 of 100 K = 128 19.0 (18.4 uncut), K = 64 fp16 7.3 (6.8); 2 000 of
 // 160 K = 128 22.7 (20.7).  16-bit rows beyond 128 bytes, whose items are shorter in time, only where there are very few
 // panels: 1 000 of 104 columns K = 128 bf16 6.0 / 6.8.
+constexpr int panel_item_of(int64_t average, int64_t pieces) {          // columns, of a panel of average length
+    const int64_t columns = pieces < 2 ? PANEL_COLUMNS : (average / pieces + 63) / 64 * 64;
+    return columns < 64 ? 64 : columns < PANEL_COLUMNS ? (int)columns : PANEL_COLUMNS;
+}
 constexpr int panel_columns(int steps, bool half_width, int64_t panels, int64_t average) {
     const int64_t wavefronts = 1024 * (steps <= 2 ? 5 : steps <= 8 ? 4 : 2);
     int64_t pieces = steps <= 8 ? wavefronts / (2 * panels) : wavefronts / panels;
     if (pieces < 2 && 8 * panels <= 3 * wavefronts) pieces = 2;
-    if (pieces < 2 || (half_width && steps > 2 && 8 * panels > wavefronts)) return PANEL_COLUMNS;
-    const int64_t columns = (average / pieces + 63) / 64 * 64;       // of a panel of average length
-    return columns < 64 ? 64 : columns < PANEL_COLUMNS ? (int)columns : PANEL_COLUMNS;
+    if (half_width && steps > 2 && 8 * panels > wavefronts) pieces = 1;
+    const int columns = panel_item_of(average, pieces);
+    if (half_width || steps > 8) return columns;
+    // fp32: shorter items, for all of the wavefronts, where the steps of 64 columns go into them without a rest (four of five at
+    // the least), of 64 columns only where they do not go into the longer ones; rows beyond 128 bytes only where panels are cut
+    // anyway.  Without / with: 1 333 panels of 360 columns K = 24 14.8 / 11.9 us, K = 32 12.5 / 10.8, K = 64 17.2 / 15.7, K = 100
+    // 27.4 / 24.6, K = 128 24.5 / 23.0, random K = 32 12.9 / 11.5, K = 128 30.2 / 32.7; 1 700 of 360 K = 24 15.9 / 13.9; 1 700 of 160
+    // K = 24 8.5 / 8.0; 2 000 of 240 K = 24 12.9 / 12.1, K = 32 11.3 / 11.1; 2 523 of 288 K = 24 17.3 / 15.7.  (After a copy of 640 MB
+    // K = 32 18.3 .. 26 us, 2 .. 9 % the other way; random columns, 1 700 of 360 K = 128 31.4 / 39.2 where panels are whole.)
+    const int finer = panel_item_of(average, wavefronts / panels);
+    if (finer >= columns || (steps > 2 && columns == PANEL_COLUMNS)) return columns;
+    const int64_t blocks = (average + 63) / 64, per_item = finer / 64, items = (blocks + per_item - 1) / per_item;
+    const bool even = items * per_item == blocks;
+    if (finer == 64) return steps <= 2 && blocks * 64 > columns && blocks % (columns / 64) != 0 ? finer : columns;
+    return even || (steps <= 2 && blocks >= 5 && 6 * blocks >= 5 * items * per_item) ? finer : columns;
 }
 
 // Entries per tile below which 16-row strips that are two panels of `panels` (as many as the matrix has groups of 8 rows) go to

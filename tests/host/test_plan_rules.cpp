@@ -25,13 +25,19 @@ static void panels() {
                     const int columns = panel_columns(steps, half, n, average);
                     CHECK(columns >= 64 && columns <= PANEL_COLUMNS, "%d columns", columns);
                     CHECK(columns % 64 == 0, "%d columns", columns);
-                    if (n > 1920) CHECK(columns == PANEL_COLUMNS, "%d panels fill the chip", (int)n);
+                    if (n > (steps <= 2 && !half ? 2560 : 1920)) CHECK(columns == PANEL_COLUMNS, "%d panels fill the chip", (int)n);
                     // no more items than wavefronts
                     const int64_t items = n * ((average + columns - 1) / columns), whole = n * ((average + PANEL_COLUMNS - 1) / PANEL_COLUMNS);
                     CHECK(items <= 5120 || items <= whole, "%d items of %d panels of %d columns", (int)items, (int)n, (int)average);
                 }
     CHECK(panel_columns(8, false, 1000, 240) == 128 && panel_columns(2, true, 1000, 240) == 128, "1 000 panels of 240");
     for (int steps : {2, 4, 8}) CHECK(panel_columns(steps, false, 2000, 160) == PANEL_COLUMNS, "2 000 panels");
+    // steps of 64 columns that go into the items without a rest
+    for (int steps : {1, 2, 4, 8}) CHECK(panel_columns(steps, false, 1333, 360) == 128, "%d steps, 1 333 panels of 360", steps);
+    CHECK(panel_columns(2, false, 2000, 240) == 128 && panel_columns(8, false, 2000, 240) == PANEL_COLUMNS, "2 000 of 240");
+    CHECK(panel_columns(2, false, 1700, 160) == 64 && panel_columns(2, false, 1000, 240) == 128, "items of 64 columns");
+    CHECK(panel_columns(2, true, 1333, 360) == 192 && panel_columns(12, false, 1333, 360) == PANEL_COLUMNS, "16 bits, long rows");
+    CHECK(panel_columns(2, false, 2523, 288) == 192 && panel_columns(2, false, 1555, 448) == 256, "a rest of one step");
 }
 
 // A matrix whose strips all hold the same number of entries per tile, on either side of the line.
