@@ -44,9 +44,8 @@ constexpr int64_t row_block_segments(int64_t n_long, int64_t nnz_long, int piece
 // Rows of 64 * {1, 2, 4, 8, 16} bytes are always looked at.  For the others the look costs a plan 8 us (1 000 rows) to 40 (4 M
 // entries), where it finds gathered strips 60, and the launch gains what `steps` 64-byte steps times the entries are worth to it.  A
 // caller who plans a pattern once has the cost back soon in any case; a caller with a new pattern for every launch never has
-// unless one launch gains it.  The lines lie where about three launches of dense tiles do; of banded blocks, which gain less, it
-// takes four to nine there (rows of 3 and 4 steps, 0.72 M entries in bands: 9.2 .. 10.3 / 7.1 us, plan 13 us longer; 0.62 M in tiles 9.8 ..
-// 10.4 / 5.1, 17 us).
+// unless one launch gains it.  The lines lie where three to five launches of dense tiles do; of banded blocks, which gain less, it
+// takes eight and more there.
 
 // Share of the entries that lie in the same 16 columns as the one before them (a sample, from the check of the columns): 1.0
 // in banded blocks and dense tiles, 0.7 where near-dense rows hold most of the entries, 0.02 .. 0.06 in graphs and uniform
@@ -58,9 +57,12 @@ constexpr double STRUCTURED_NEAR = 0.85, GATHERED_NEAR = 0.6;
 // K = 100 27.8 / 8.7, 103 / 109; 2.4 M K = 15 11.1 / 7.0, 89 / 118; 4 M K = 15 17.2 / 8.8, 96 / 129, K = 21 23.3 / 10.7, 103 /
 // 131, K = 33 43.9 / 13.5, 123 / 134; 0.4 M K = 33 8.9 / 4.3, 83 / 95, K = 75 10.9 / 5.3, 85 / 96; banded blocks of 0.96 M K = 21
 // 7.8 / 6.1, 82 / 96, K = 51 11.7 / 8.1, 86 / 99, K = 100 19.7 / 9.7, 93 / 100; 3.8 M K = 15 16 / 10, 96 / 98, K = 40 bf16 28 / 10,
-// 106 / 98, K = 75 59 / 28, 139 / 113; 14 M K = 21 69 / 29.
+// 106 / 98, K = 75 59 / 28, 139 / 113; 14 M K = 21 69 / 29.  At the lines of two to four steps, launch without / with and how much longer
+// the plan takes: tiles of 0.38 M K = 40 8.8 / 4.9, 15, K = 60 8.0 / 5.2, 16, K = 72 bf16 9.7 / 4.5, 13; 0.65 M in 548 rows K = 45
+// 9.4 / 4.3; 0.83 M K = 40 bf16 8.9 / 5.2, 19; 1.2 M 11.3 / 5.5, 25, K = 24 9.4 / 6.7, 24; bands of 0.48 M K = 40 8.0 / 6.5, 11, K = 60
+// 7.4 / 6.7, 10, K = 72 bf16 8.9 / 5.2, 11; 0.96 M K = 24 7.7 / 5.6, 16, K = 40 bf16 8.8 / 5.8, 16.
 constexpr int64_t ragged_entries(int steps) {
-    return steps <= 1 ? 3 << 20 : steps <= 2 ? 3 << 19 : steps <= 4 ? 3 << 18 : steps <= 6 ? 5 << 16 : 1 << 16;
+    return steps <= 1 ? 3 << 20 : steps <= 2 ? 1 << 20 : steps <= 4 ? 3 << 17 : steps <= 6 ? 5 << 16 : 1 << 16;
 }
 
 // Near-dense rows among others: their gathered strips are all there is to find.  Launch without / with, set, plan and launch

@@ -73,8 +73,8 @@ static void rows_of_any_length() {
         before = ragged_entries(steps);
         for (bool half : {false, true}) CHECK(ragged_gathered_entries(steps, half) * steps <= 1 << 24, "%d steps", steps);
     }
-    CHECK(ragged_entries(1) > 5 << 19 && ragged_entries(2) > 5 << 18 && ragged_entries(4) > 1 << 19, "rows of up to 256 bytes");
-    CHECK(ragged_entries(1) <= 3840000 && ragged_entries(4) <= 960000, "a launch that gains more than the look costs");
+    CHECK(ragged_entries(1) > 5 << 19 && ragged_entries(2) > 825600 && ragged_entries(4) > 338688, "rows of up to 256 bytes");
+    CHECK(ragged_entries(1) <= 3840000 && ragged_entries(2) <= 1199872 && ragged_entries(4) <= 480000, "where few launches gain what the look costs");
     CHECK(ragged_entries(6) <= 331264 && ragged_entries(8) <= 96000, "longer rows");
     CHECK(ragged_gathered_entries(6, false) <= 1960000 && ragged_gathered_entries(8, false) > 1960000, "near-dense rows");
     CHECK(ragged_gathered_entries(4, true) <= 1960000 && ragged_gathered_entries(4, false) > 1960000, "near-dense rows, 16 bits");
